@@ -14,12 +14,7 @@ constexpr int kPartialWords = 64;      // one lane's partial accumulator: 256 by
 constexpr int kWaveLanes = 64;
 constexpr size_t kSlabSegments = 32768;   // row segments per launch: 512 MiB of partial sums
 
-// Lanes that share a row in the one-wave row-reduction kernel: 8 when rows alone fill the chip (measured
-// best for 4096 rows of 64 partials: 4 lanes +6 %, 16 +33 %, 32 +65 % - idle lanes of the tree steps cost
-// more than shorter chains save), up to a whole wave when rows are few and the chain per lane is
-// what takes the time (one row of 32768 partials: 150 ms with 8 lanes).  With 512 rows and more (a value
-// below 6) a call that waits for its result takes the four-wave kernel instead, which hands partial sums
-// between waves through LDS (tree_row / tree_share below); the value still bounds the column segments of a row.
+// Bounds the column segments of a row (wide_plan): a row leaves at most 128 partial sums per 2^this.
 GRAPE_HD uint32_t reduce_lanes_log2(size_t rows) {
     if (rows >= 2048) return 3;
     if (rows >= 1024) return 4;
@@ -34,15 +29,17 @@ struct WidePlan {
     size_t slab;            // rows per launch
     size_t partial_bytes;   // work buffer of one launch (slab * nseg * 64 lanes * 256 bytes)
 };
-// segments: enough waves to fill the chip (>= 4 per SIMD) but at least 64 columns per lane-sweep, and
-// no more than leaves each reducing lane a chain of 128 partial sums; rows go through in slabs of
-// slab_segments row segments
+// segments: two waves per SIMD (one with fewer than 512 rows: there the additions of the row reduction cost as much as
+// those saved by shorter lane chains - 64 rows of 4096: 159 us in 16 segments, 184 in 32, 252 in 64; 256 rows 284, 292,
+// 339; 512 rows 447, 439, 478; 1024 rows 764, 720, 723), at least 64 columns per lane-sweep, and no more than
+// leaves 128 * 2^lg_lpr partial sums per row; rows go through in slabs of slab_segments row segments
 GRAPE_HD WidePlan wide_plan(size_t size, uint32_t rowlen, size_t slab_segments) {
     WidePlan p;
     p.rows = size / rowlen;
     p.lg_lpr = reduce_lanes_log2(p.rows);
     p.nseg = 1;
-    while (p.rows * p.nseg < 4096 && rowlen / (p.nseg * 2) >= 64 && p.nseg * 2 <= (2u << p.lg_lpr)) p.nseg *= 2;
+    const size_t waves = p.rows < 512 ? 1024 : 2048;
+    while (p.rows * p.nseg < waves && rowlen / (p.nseg * 2) >= 64 && p.nseg * 2 <= (2u << p.lg_lpr)) p.nseg *= 2;
     p.seg = (rowlen + p.nseg - 1) / p.nseg;
     p.slab = slab_segments / (size_t)p.nseg;
     if (p.slab < 1) p.slab = 1;
@@ -72,17 +69,47 @@ GRAPE_HD size_t table_entry(uint32_t w, uint32_t K, uint32_t mag, size_t N, uint
 // 32-bit-word offset of partial accumulator i (i = wave * 64 + lane in the accumulation kernel,
 // row * nparts + j in the reduction kernel)
 GRAPE_HD size_t partial_word(size_t i) { return (size_t)kPartialWords * i; }
-// reduction kernel: row of lane `lane` of workgroup `block`
-GRAPE_HD size_t reduce_row(size_t block, int lane, uint32_t lg_lpr) { return block * (size_t)(kWaveLanes >> lg_lpr) + (size_t)(lane >> lg_lpr); }
-// four-wave reduction kernel: a workgroup of 256 threads takes kTreeRows rows, 32 lanes a row; thread t works
-// on row tree_row(block, t) and starts from partial sums tree_share(t), tree_share(t) + 32, ... of that row
+// row of lane `lane` of wave `wave` when 2^lg_lpr lanes share a row
+GRAPE_HD size_t reduce_row(size_t wave, int lane, uint32_t lg_lpr) { return wave * (size_t)(kWaveLanes >> lg_lpr) + (size_t)(lane >> lg_lpr); }
+// which share of its row the quad of lane `lane` takes
+GRAPE_HD uint32_t quad_share(int lane, uint32_t lg_qpr) { return (uint32_t)(lane >> 2) & ((1u << lg_qpr) - 1u); }
+
+// How a row's nparts partial sums become one (measured with the three kernels of g1_kernels.hip, microseconds):
+//   - more than 8192 rows: lanes first, down to 8 per row, then quads (32768 rows of 64: 540, quads alone 650 to 680);
+//     at 8192 rows quads alone are as fast (209 against 199) and one launch less;
+//   - up to 512 rows of more than 64 partial sums: quads in groups of 64 first, so that the chain stays at 7 additions
+//     (512 rows of 512: 196 against 243; 64 of 4096: 223 against 1430; 1024 rows of 256: 190 against 162, so not there);
+//   - quads per row: as many as a wave holds while rows * quads stays below 2^15, i.e. two waves per SIMD (2048 rows
+//     of 128: 154 with 16, 151 with 8, 232 with 4; 8192 of 64: 285, 225, 209 with 16, 8, 4).
+constexpr uint32_t kQuadsPerWaveLog2 = 4;
+constexpr uint32_t kReduceGroup = 64;      // partial sums of a group
+constexpr uint32_t kReduceKeep = 8;        // partial sums per row that the lane kernel leaves
+struct ReducePlan {
+    bool lanes;             // first stage by commit_reduce_lane_kernel
+    uint32_t left;          // partial sums per row after the first stage (nparts when there is none)
+    uint32_t lg_qpr;        // log2 of the quads per row in the last stage
+};
+GRAPE_HD ReducePlan reduce_plan(size_t rows, uint32_t nparts) {
+    ReducePlan p;
+    p.lanes = rows > 8192 && nparts > kReduceKeep;
+    p.left = p.lanes ? kReduceKeep : (rows <= 512 && nparts > kReduceGroup && nparts % kReduceGroup == 0) ? nparts / kReduceGroup : nparts;
+    p.lg_qpr = 0;
+    while (p.lg_qpr < kQuadsPerWaveLog2 && (2u << p.lg_qpr) <= p.left && (rows << (p.lg_qpr + 1)) <= 32768) p.lg_qpr++;
+    if (p.lanes) p.lg_qpr = 1;
+    return p;
+}
+// accumulators of work space for at most `rows` rows: what the first stage leaves, and the row sums
+GRAPE_HD size_t reduce_tmp_accumulators(size_t rows, uint32_t nparts) {
+    const size_t grouped = (rows < 512 ? rows : 512) * (size_t)(nparts / kReduceGroup), kept = rows > 8192 ? rows * kReduceKeep : 0;
+    return rows + (grouped > kept ? grouped : kept);
+}
+
+// The layout of a four-wave reduction (eight rows a workgroup, 32 lanes a row) that no kernel uses any more; the host
+// walk of the tests still goes through it.
 constexpr int kTreeRows = 8;
 constexpr int kTreeThreads = 256;
 GRAPE_HD size_t tree_row(size_t block, int t) { return block * (size_t)kTreeRows + (size_t)(t & (kTreeRows - 1)); }
 GRAPE_HD uint32_t tree_share(int t) { return (uint32_t)t >> 3; }
-// taken for 512 to 4096 rows: up to 512 workgroups, which the chip holds all at once (two per compute unit) - with more
-// rows the waves that idle at the kernel's barriers keep later workgroups out, and the one-wave kernel is faster
-// (32 768 rows: 0.8 against 1.5 ms)
 GRAPE_HD bool tree_reduction(size_t rows, uint32_t lg_lpr, uint32_t nparts) { return lg_lpr <= 5 && rows <= 4096 && nparts <= 4096; }
 // workgroups of a launch of `threads` threads in groups of `per_block`
 GRAPE_HD size_t blocks_needed(size_t threads, size_t per_block) { return (threads + per_block - 1) / per_block; }

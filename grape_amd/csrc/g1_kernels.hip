@@ -13,6 +13,7 @@
 #include "commit_geometry.hpp"
 #include "fp28.hpp"
 #include "fr26.hpp"
+#include "quad28.hpp"
 
 namespace grape {
 
@@ -802,109 +803,84 @@ __global__ void __launch_bounds__(64) commit_sparse_fr_kernel(uint32_t* partial,
     if (have_row) st_partial28(partial, row * G + sub, acc);
 }
 
-// Row epilogue: 2^lg_lpr lanes per row, each sums its share of the partials serially, then a
-// tree over those lanes; the leader maps the row sum to affine coordinates.  All in the 28-bit form.
-template <bool AFFINE>
-__global__ void __launch_bounds__(64) commit_reduce_kernel(uint32_t* out, const uint32_t* partial, size_t rows, uint32_t nparts,
-                                                           uint32_t lg_lpr) {
-    const int lane = threadIdx.x & 63;
-    const int lpr = 1 << lg_lpr;                       // lanes per row: 8, 16, 32 or 64
-    const int sub = lane & (lpr - 1);
-    const size_t row = geom::reduce_row(blockIdx.x, lane, lg_lpr);
-    Xyzz28 acc = xyzz28_inf();
-    // one addition site serves both the serial part and the tree steps (code size)
-    const uint32_t nserial = (nparts + lpr - 1) >> lg_lpr;
-    for (uint32_t step = 0; step < nserial + lg_lpr; step++) {
-        Xyzz28 q;
-        bool doit;
-        if (step < nserial) {
-            const uint32_t j = sub + (step << lg_lpr);
-            doit = row < rows && j < nparts;
-            q = doit ? ld_partial28(partial, row * nparts + j) : xyzz28_inf();
-        } else {
-            const int off = (lpr >> 1) >> (step - nserial);
-            q = shfl_down_xyzz28(acc, off);
-            doit = sub + off < lpr;
-        }
-        if (doit) padd28(acc, q);
-    }
-    if (row < rows && sub == 0) {
-        if (AFFINE) st_affine(out, row, xyzz28_to_affine(acc));
-        else st_partial28(out, row, acc);        // left as an accumulator (256 bytes) for a later combination
-    }
-}
-
-// Row epilogue for many rows: a workgroup of four waves takes eight rows, 32 lanes a row (thread t: row t & 7,
-// share t >> 3).  Every lane sums its share of the row's partial sums, waves 2 and 3 hand theirs to waves 0 and 1
-// through LDS, wave 1 hands its to wave 0, and wave 0 finishes with three shuffle steps: for 64 partial sums a
-// chain of 6 additions instead of the 10 of eight lanes per row, with every lane of the early steps at work (a
-// tree by shuffles alone would keep all four waves issuing with idle lanes).  Both barriers are reached by all
-// four waves; waves 1 to 3 leave after the second.
-using geom::kTreeRows;
-constexpr int kTreeLdsWords = 4 * L28 + 1;
-__device__ __forceinline__ void st_lds_xyzz28(uint32_t* lds, int slot, const Xyzz28& a) {
+// Row epilogue: the partial sums of a row become one point, the point its affine image.  Three kernels:
+//   commit_reduce_lane_kernel  rows by the ten thousand: one lane per kept partial sum adds its share (107 wave
+//                              instructions per addition, the fewest, but chains of 7 additions at 18 us each)
+//   commit_reduce_quad_kernel  2^lg_qpr quads (quad28.hpp) per row, each adds its share, then a tree of shuffles
+//                              (154 wave instructions per addition, 5.1 us each)
+//   quad_affine_kernel         the map to affine coordinates, a quad per row
+// geom::reduce_plan picks.  Bound: instruction latency - a SIMD issues hardly faster with two of these waves than with
+// one, so what counts is one wave per SIMD (workgroups of four waves spread evenly over a compute unit's
+// SIMDs, one-wave workgroups do not: 139 against 175 us for 4096 rows of 64) and few additions in a chain.
+// The map is a kernel of its own so that every quad of a wave inverts: left to the sum kernel's first quads
+// it took 0.1 ms longer.  Measured, one box, before (one lane per accumulator, shuffle or LDS trees) and now:
+// 4096 rows of 64: 0.291 -> 0.148 ms; 512 of 64: 0.196 -> 0.079; one of 4096: 0.277 -> 0.124; 64 of 256: 0.237 -> 0.093;
+// 32768 of 64: 1.08 -> 0.54.
+__device__ __forceinline__ quad::Acc ld_quad_partial(const uint32_t* base, size_t i) {
+    const uint32_t* p = base + geom::partial_word(i);
+    const uint2* q = reinterpret_cast<const uint2*>(p + (threadIdx.x & 3) * L28);
+    quad::Acc a;
 #pragma unroll
-    for (int k = 0; k < L28; k++) {
-        lds[(0 * L28 + k) * 192 + slot] = (uint32_t)a.x.v[k];
-        lds[(1 * L28 + k) * 192 + slot] = (uint32_t)a.y.v[k];
-        lds[(2 * L28 + k) * 192 + slot] = (uint32_t)a.zz.v[k];
-        lds[(3 * L28 + k) * 192 + slot] = (uint32_t)a.zzz.v[k];
+    for (int k = 0; k < L28 / 2; k++) {
+        const uint2 w = q[k];
+        a.v.v[2 * k] = (int32_t)w.x;
+        a.v.v[2 * k + 1] = (int32_t)w.y;
     }
-    lds[4 * L28 * 192 + slot] = a.inf ? 1u : 0u;
-}
-__device__ __forceinline__ Xyzz28 ld_lds_xyzz28(const uint32_t* lds, int slot) {
-    Xyzz28 a;
-#pragma unroll
-    for (int k = 0; k < L28; k++) {
-        a.x.v[k] = (int32_t)lds[(0 * L28 + k) * 192 + slot];
-        a.y.v[k] = (int32_t)lds[(1 * L28 + k) * 192 + slot];
-        a.zz.v[k] = (int32_t)lds[(2 * L28 + k) * 192 + slot];
-        a.zzz.v[k] = (int32_t)lds[(3 * L28 + k) * 192 + slot];
-    }
-    a.inf = lds[4 * L28 * 192 + slot] != 0;
+    a.inf = p[4 * L28] != 0;
     return a;
 }
-template <bool AFFINE>
-__global__ void __launch_bounds__(geom::kTreeThreads, 2) commit_reduce_tree_kernel(uint32_t* out, const uint32_t* partial, size_t rows, uint32_t nparts) {
-    __shared__ uint32_t lds[kTreeLdsWords * 192];      // slots 0..127: waves 2, 3; slots 128..191: wave 1
-    const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
-    const size_t row = geom::tree_row(blockIdx.x, t);
-    const uint32_t sub = geom::tree_share(t);
+__device__ __forceinline__ void st_quad_partial(uint32_t* base, size_t i, const quad::Acc& a) {
+    uint32_t* p = base + geom::partial_word(i);
+    uint2* q = reinterpret_cast<uint2*>(p + (threadIdx.x & 3) * L28);
+#pragma unroll
+    for (int k = 0; k < L28 / 2; k++) q[k] = make_uint2((uint32_t)a.v.v[2 * k], (uint32_t)a.v.v[2 * k + 1]);
+    if ((threadIdx.x & 3) == 0) p[4 * L28] = a.inf ? 1u : 0u;
+}
+static_assert(L28 % 2 == 0, "a coordinate is moved as 8-byte words");
+__global__ void __launch_bounds__(kBlock) commit_reduce_quad_kernel(uint32_t* out, const uint32_t* partial, size_t rows, uint32_t nparts,
+                                                                    uint32_t lg_qpr) {
+    const int lane = threadIdx.x & 63;
+    const size_t wave = ((size_t)blockIdx.x * kBlock + threadIdx.x) >> 6;
+    const uint32_t qpr = 1u << lg_qpr, sub = geom::quad_share(lane, lg_qpr);
+    const size_t row = geom::reduce_row(wave, lane, lg_qpr + 2);
     const bool have = row < rows;
-    Xyzz28 acc = xyzz28_inf();
-    const uint32_t nserial = (nparts + 31) >> 5;
-    // one addition site serves every step (code size)
-    for (uint32_t step = 0; step < nserial + 5; step++) {
-        Xyzz28 q = xyzz28_inf();
-        bool doit = false;
+    quad::Acc acc = quad::identity(), next = quad::identity();
+    const uint32_t nserial = (nparts + qpr - 1) >> lg_qpr;
+    if (have && sub < nparts) next = ld_quad_partial(partial, row * nparts + sub);
+    // one addition site serves both the serial part and the tree steps (code size); the next partial sum is on its way
+    // while this one is added
+    for (uint32_t step = 0; step < nserial + lg_qpr; step++) {
+        quad::Acc q = next;
+        next = quad::identity();
         if (step < nserial) {
-            const uint32_t j = sub + (step << 5);
-            doit = have && j < nparts;
-            if (doit) q = ld_partial28(partial, row * nparts + j);
-        } else if (step == nserial) {
-            if (wave >= 2) st_lds_xyzz28(lds, t - 128, acc);
-            __syncthreads();
-            if (wave < 2) {
-                q = ld_lds_xyzz28(lds, t);
-                doit = true;
-            }
-        } else if (step == nserial + 1) {
-            if (wave == 1) st_lds_xyzz28(lds, 128 + lane, acc);
-            __syncthreads();
-            if (wave != 0) return;
-            q = ld_lds_xyzz28(lds, 128 + lane);
-            doit = true;
+            const uint32_t j = sub + ((step + 1) << lg_qpr);
+            if (have && j < nparts) next = ld_quad_partial(partial, row * nparts + j);
         } else {
-            const int off = 32 >> (step - nserial - 2);      // 32, 16, 8: the partner holds the same row
-            q = shfl_down_xyzz28(acc, off);
-            doit = lane + off < 64;
+            const uint32_t off = (qpr >> 1) >> (step - nserial);
+#pragma unroll
+            for (int k = 0; k < L28; k++) q.v.v[k] = __shfl_down(acc.v.v[k], 4 * off, 64);
+            q.inf = __shfl_down((int)acc.inf, 4 * off, 64) != 0 || sub + off >= qpr;
         }
-        if (doit) padd28(acc, q);
+        quad::add(acc, q);
     }
-    if (t < kTreeRows && have) {
-        if (AFFINE) st_affine(out, row, xyzz28_to_affine(acc));
-        else st_partial28(out, row, acc);
-    }
+    if (have && sub == 0) st_quad_partial(out, row, acc);      // 256 bytes per row: an accumulator
+}
+__global__ void __launch_bounds__(kBlock) quad_affine_kernel(uint32_t* out, const uint32_t* sums, size_t rows) {
+    const size_t row = ((size_t)blockIdx.x * kBlock + threadIdx.x) >> 2;
+    if (row >= rows) return;
+    const Fp c = quad::to_affine(ld_quad_partial(sums, row));
+    const uint32_t r = threadIdx.x & 3;
+    if (r < 2) st_fp(out + 2 * FW * row + FW * r, c);
+}
+// out[row * keep + k] = the sum of the row's partial sums k, k + keep, ...
+__global__ void __launch_bounds__(kBlock) commit_reduce_lane_kernel(uint32_t* out, const uint32_t* partial, size_t rows, uint32_t nparts, uint32_t keep) {
+    const size_t t = (size_t)blockIdx.x * kBlock + threadIdx.x;
+    if (t >= rows * keep) return;
+    const size_t row = t / keep;
+    const uint32_t sub = (uint32_t)(t - row * keep);
+    Xyzz28 acc = ld_partial28(partial, row * nparts + sub);
+    for (uint32_t j = sub + keep; j < nparts; j += keep) padd28(acc, ld_partial28(partial, row * nparts + j));
+    st_partial28(out, t, acc);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -1020,35 +996,23 @@ using geom::reduce_lanes_log2;
 // largest size the GPU tests run; the host classes split longer tensors by rows.
 constexpr size_t kMaxCommitScalars = (size_t)1 << 28;
 
-// Row reduction of `rows` rows of `nparts` partial sums each.  With few rows the chain of additions of
-// the reducing lanes is what takes the time (one row of 4096 partial sums on 64 lanes: 64 + 6 additions
-// one after the other, 1 ms), so those go through two levels: every 256 partial sums of a row become
-// one (4 + 6 additions, one wave per group), then the groups of a row are folded (`tmp`: one
-// accumulator of 256 bytes per group).
-constexpr uint32_t kReduceGroup = 256;
-static size_t reduce_tmp_bytes(size_t rows, uint32_t nparts) { return rows * (size_t)(nparts / kReduceGroup + 1) * (4 * kPartialWords); }
+// Row reduction of `rows` rows of `nparts` partial sums each (`tmp`: work space of reduce_tmp_bytes): to affine points, or
+// to accumulators of 256 bytes for a later combination.
+static size_t reduce_tmp_bytes(size_t rows, uint32_t nparts) { return geom::reduce_tmp_accumulators(rows, nparts) * (4 * kPartialWords); }
 template <bool AFFINE>
-static void launch_reduce(uint32_t* out, const uint32_t* partial, size_t rows, uint32_t nparts, uint32_t lg_lpr, uint32_t* tmp, hipStream_t s,
-                          bool alone = false) {
-    if (tmp && lg_lpr == 6 && nparts >= 4 * kReduceGroup && nparts % kReduceGroup == 0) {
-        const uint32_t groups = nparts / kReduceGroup;
-        commit_reduce_kernel<false><<<(unsigned)(rows * groups), 64, 0, s>>>(tmp, partial, rows * groups, kReduceGroup, 6);
-        uint32_t lg2 = 0;
-        while ((1u << lg2) < groups && lg2 < 6) lg2++;
-        const size_t per_wave = (size_t)64 >> lg2;
-        commit_reduce_kernel<AFFINE><<<(unsigned)((rows + per_wave - 1) / per_wave), 64, 0, s>>>(out, tmp, rows, groups, lg2);
-        return;
-    }
-    // `alone`: the caller waits for this result with nothing queued behind it - the four-wave kernel's shorter
-    // chain is the gain (0.29 against 0.35 ms for 4096 rows of 64).  Beside other kernels it is the loss: its
-    // waves hold half as many wave slots again while they wait at the barriers, and a commitment queued
-    // behind this one runs slower for it (three streams of 4096 x 4096 commitments: 6220 against 6550 Mpoints/s)
-    if (alone && geom::tree_reduction(rows, lg_lpr, nparts)) {
-        commit_reduce_tree_kernel<AFFINE><<<(unsigned)((rows + kTreeRows - 1) / kTreeRows), geom::kTreeThreads, 0, s>>>(out, partial, rows, nparts);
-        return;
-    }
-    const size_t per_wave = (size_t)64 >> lg_lpr;
-    commit_reduce_kernel<AFFINE><<<(unsigned)((rows + per_wave - 1) / per_wave), 64, 0, s>>>(out, partial, rows, nparts, lg_lpr);
+static void launch_reduce(uint32_t* out, const uint32_t* partial, size_t rows, uint32_t nparts, uint32_t* tmp, hipStream_t s) {
+    const geom::ReducePlan plan = geom::reduce_plan(rows, nparts);
+    auto quads = [&](uint32_t* to, const uint32_t* from, size_t units, uint32_t parts, uint32_t lg_qpr) {
+        commit_reduce_quad_kernel<<<blocks_for(units << (lg_qpr + 2)), kBlock, 0, s>>>(to, from, units, parts, lg_qpr);
+    };
+    if (plan.lanes)
+        commit_reduce_lane_kernel<<<blocks_for(rows * plan.left), kBlock, 0, s>>>(tmp, partial, rows, nparts, plan.left);
+    else if (plan.left < nparts)
+        quads(tmp, partial, rows * plan.left, nparts / plan.left, geom::kQuadsPerWaveLog2);
+    const uint32_t* const last = plan.left < nparts ? tmp : partial;
+    uint32_t* const sums = AFFINE ? tmp + (last == tmp ? geom::partial_word(rows * plan.left) : 0) : out;
+    quads(sums, last, rows, plan.left, plan.lg_qpr);
+    if (AFFINE) quad_affine_kernel<<<blocks_for(rows * 4), kBlock, 0, s>>>(out, sums, rows);
 }
 
 template <bool FR>
@@ -1070,7 +1034,7 @@ static int commit_wide_impl(uint32_t* out, const void* scalars, size_t size, uin
     // rows go through in slabs so that the per-lane partial sums stay within 512 MiB whatever the
     // number of rows (a row segment leaves 64 partial sums of 256 bytes)
     const geom::WidePlan plan = geom::wide_plan(size, rowlen, geom::kSlabSegments);
-    const uint32_t lg_lpr = plan.lg_lpr, nseg = plan.nseg, seg = plan.seg;
+    const uint32_t nseg = plan.nseg, seg = plan.seg;
     const size_t slab = plan.slab, partial_bytes = plan.partial_bytes;
     void* ws;
     const size_t tmp_bytes = reduce_tmp_bytes(slab, nseg * 64);
@@ -1092,7 +1056,7 @@ static int commit_wide_impl(uint32_t* out, const void* scalars, size_t size, uin
         profile_mark(s);
         commit_wide_kernel<FR><<<blocks_for(nr * nseg * 64), kBlock, 0, s>>>((uint32_t*)ws, sc, rowlen, nr, seg, nseg, table, N, c, nw, K, err);
         profile_mark(s);
-        launch_reduce<true>(out + r0 * (size_t)(2 * FW), (const uint32_t*)ws, nr, nseg * 64, lg_lpr, red_tmp, s, caller_flag == nullptr);
+        launch_reduce<true>(out + r0 * (size_t)(2 * FW), (const uint32_t*)ws, nr, nseg * 64, red_tmp, s);
         profile_mark(s);
     }
     GRAPE_LAUNCH_CHECK();
@@ -1141,7 +1105,7 @@ static int commit_ref_impl(uint32_t* out, const void* scalars, size_t size, uint
         const size_t units = nr * nwin * nseg;
         const uint32_t* sc = (const uint32_t*)scalars + r0 * rowlen * elem_words;
         commit_ref28_kernel<FR><<<blocks_for(units * 64), kBlock, 0, s>>>((uint32_t*)ws, sc, rowlen, nr, seg, nseg, table, npoints);
-        launch_reduce<true>(sums, (const uint32_t*)ws, nr * nwin, nseg * 64, lg_lpr, red_tmp, s);
+        launch_reduce<true>(sums, (const uint32_t*)ws, nr * nwin, nseg * 64, red_tmp, s);
         commit_ref_horner_kernel<<<blocks_for(nr, 64), 64, 0, s>>>(out + r0 * (size_t)(2 * FW), sums, nr, nwin);
     }
     GRAPE_LAUNCH_CHECK();
@@ -1267,7 +1231,7 @@ int grape_commit_fr_strided(uint32_t* out, const uint32_t* scalars, size_t size,
     hipStream_t s = as_stream(st);
     // (row, residue) pairs are the rows of the accumulation and reduction launches
     const geom::WidePlan plan = geom::wide_plan(rows * J * (size_t)rowlen, rowlen, geom::kSlabSegments);
-    const uint32_t lg_lpr = plan.lg_lpr, nseg = plan.nseg, seg = plan.seg;
+    const uint32_t nseg = plan.nseg, seg = plan.seg;
     size_t slab = plan.slab / J;                              // whole rows per launch
     if (slab < 1) slab = 1;
     if (slab > rows) slab = rows;
@@ -1285,7 +1249,7 @@ int grape_commit_fr_strided(uint32_t* out, const uint32_t* scalars, size_t size,
         profile_mark(s);
         commit_strided_kernel<<<blocks_for(nr * J * nseg * 64), kBlock, 0, s>>>((uint32_t*)ws, sc, rowlen, nr, seg, nseg, table, N, c, nw, K, J, nsets);
         profile_mark(s);
-        launch_reduce<false>(sums, (const uint32_t*)ws, nr * J, nseg * 64, lg_lpr, red_tmp, s);
+        launch_reduce<false>(sums, (const uint32_t*)ws, nr * J, nseg * 64, red_tmp, s);
         strided_horner_kernel<<<blocks_for(nr, 64), 64, 0, s>>>(out + r0 * (size_t)(2 * FW), sums, nr, J, c);
         profile_mark(s);
     }
@@ -1340,16 +1304,16 @@ int grape_commit_fr_sparse(uint32_t* out, const uint32_t* scalars, const int32_t
     hipStream_t s = as_stream(st);
     const size_t slab = rows < geom::kSlabSegments ? rows : geom::kSlabSegments;
     const size_t partial_bytes = slab * geom::kWaveLanes * (size_t)(4 * geom::kPartialWords);
+    const size_t tmp_bytes = reduce_tmp_bytes(slab, geom::kWaveLanes);
     void* ws;
-    int rc = scratch_get(kSlotMsm, partial_bytes + 64, &ws, s);
+    int rc = scratch_get(kSlotMsm, partial_bytes + tmp_bytes + 64, &ws, s);
     if (rc) return rc;
-    int* err = (int*)((char*)ws + partial_bytes);
+    uint32_t* red_tmp = (uint32_t*)((char*)ws + partial_bytes);
+    int* err = (int*)((char*)ws + partial_bytes + tmp_bytes);
     rc = zero_fill(err, sizeof(int), s);
     if (rc) return rc;
     for (size_t r0 = 0; r0 < rows; r0 += slab) {
         const size_t nr = rows - r0 < slab ? rows - r0 : slab;
-        const uint32_t lg_lpr = reduce_lanes_log2(nr);
-        const size_t rows_per_wave = (size_t)64 >> lg_lpr;
         // many rows: half a wave per row, so that a thinly populated row still fills its batch
         const bool narrow = nr >= 4096;
         if (narrow)
@@ -1358,8 +1322,7 @@ int grape_commit_fr_sparse(uint32_t* out, const uint32_t* scalars, const int32_t
         else
             commit_sparse_fr_kernel<64><<<(unsigned)nr, 64, 0, s>>>((uint32_t*)ws, scalars + r0 * rowlen * 8, skip + r0 * rowlen, rowlen, nr, table, N,
                                                                    c, nw, K, err);
-        commit_reduce_kernel<true><<<(unsigned)((nr + rows_per_wave - 1) / rows_per_wave), 64, 0, s>>>(out + r0 * (size_t)(2 * FW),
-                                                                                                  (const uint32_t*)ws, nr, narrow ? 32 : 64, lg_lpr);
+        launch_reduce<true>(out + r0 * (size_t)(2 * FW), (const uint32_t*)ws, nr, narrow ? 32 : 64, red_tmp, s);
     }
     GRAPE_LAUNCH_CHECK();
     int h_err = 0;
