@@ -106,6 +106,7 @@ SIGNATURES = {
     "grape_commit_fr_strided": [c_void_p, c_void_p, c_size_t, c_u32, c_void_p, c_size_t, c_u32, c_u32, c_u32, c_void_p],
     "grape_commit_i32_ref_table": [c_void_p, c_void_p, c_size_t, c_u32, c_void_p, c_size_t, c_void_p],
     "grape_commit_fr_ref_table": [c_void_p, c_void_p, c_size_t, c_u32, c_void_p, c_size_t, c_void_p],
+    "grape_g1_msm_windows": [c_void_p, c_void_p, c_void_p, c_size_t, c_void_p],
     "grape_g1_affine_to_jacobian": [c_void_p, c_void_p, c_size_t, c_void_p],
     "grape_g1_jacobian_to_affine": [c_void_p, c_void_p, c_size_t, c_void_p],
     "grape_wit_matmul_rescale": [c_void_p, c_void_p, c_void_p, c_void_p, c_u32, c_u32, c_u32, c_u32, ctypes.c_int64, c_int, c_void_p],

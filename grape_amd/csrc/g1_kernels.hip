@@ -884,6 +884,75 @@ __global__ void __launch_bounds__(kBlock) commit_reduce_lane_kernel(uint32_t* ou
 }
 
 // ------------------------------------------------------------------------------------------------
+// sum_i k_i P_i over arbitrary points (the row commitments of a verification: no table of multiples exists).
+// Signed 4-bit windows: the multiples P, 2P .. 8P of every point, then for each of the 64 windows w the sum
+// S_w = sum_i digit_w(k_i) P_i, everything on quads - a few hundred points are a latency problem, and the only long
+// chain, sum_w 16^w S_w with its 252 doublings, is left to the host, whose core runs a doubling in 0.8 us where a lone
+// quad takes 4.  256 points: 0.1 ms against 200 ms for 255 scalar multiples on the host.
+// ------------------------------------------------------------------------------------------------
+constexpr uint32_t kMsmWindows = GRAPE_MSM_WINDOWS, kMsmBits = 4, kMsmMultiples = 1u << (kMsmBits - 1);
+constexpr uint32_t kMsmGroup = 64;             // points that one wave sums
+// table[i * 8 + k - 1] = k P_i, a quad per entry
+__global__ void __launch_bounds__(kBlock) msm_multiples_kernel(uint32_t* table, const uint32_t* points, size_t n) {
+    const size_t q = ((size_t)blockIdx.x * kBlock + threadIdx.x) >> 2;
+    if (q >= n * kMsmMultiples) return;
+    const uint32_t k = (uint32_t)(q % kMsmMultiples) + 1;
+    const int r = threadIdx.x & 3;
+    const Fp w = ld_fp(points + 3 * FW * (q / kMsmMultiples) + FW * (r < 2 ? r : 2));     // x, y, z, z
+    quad::Acc p;
+    p.inf = quad::perm<quad::ctrl(2, 2, 2, 2)>((int32_t)w.is_zero()) != 0;
+    const Fp28 v = fp28::from_canonical_lazy(w);                                           // (0, 3p)
+    const Fp28 zz = fp28::sqr(v);
+    p.v = quad::select(quad::lanes<0>() | quad::lanes<1>(), v, quad::select(quad::lanes<2>(), zz, fp28::mul(zz, v)));
+    quad::Acc acc = p;
+    for (int b = 30 - __clz((int)k); b >= 0; b--) {
+        quad::dbl(acc);
+        if ((k >> b) & 1) quad::add(acc, p);
+    }
+    st_quad_partial(table, q, acc);
+}
+// partial[w * stride + g] = the sum of window w's digits times the points of group g
+__global__ void __launch_bounds__(kBlock) msm_window_kernel(uint32_t* partial, const uint32_t* table, const uint32_t* scalars, size_t n,
+                                                            uint32_t groups, size_t stride) {
+    const int lane = threadIdx.x & 63;
+    const size_t unit = ((size_t)blockIdx.x * kBlock + threadIdx.x) >> 6;
+    const uint32_t w = (uint32_t)(unit / groups), g = (uint32_t)(unit % groups);
+    if (w >= kMsmWindows) return;
+    const Fr H = window_bias(kMsmBits, kMsmWindows);
+    const uint32_t sub = (uint32_t)lane >> 2;
+    quad::Acc acc = quad::identity();
+    constexpr uint32_t kSerial = kMsmGroup / 16;
+    for (uint32_t step = 0; step < kSerial + 4; step++) {
+        quad::Acc q = quad::identity();
+        if (step < kSerial) {
+            const size_t i = (size_t)g * kMsmGroup + step * 16 + sub;
+            if (i < n) {
+                bool flip;
+                const int32_t d = digit_of(biased_half_range(ld_fr8(scalars, i), H, flip), w, kMsmBits);
+                if (d != 0) {
+                    q = ld_quad_partial(table, i * kMsmMultiples + (uint32_t)(d < 0 ? -d : d) - 1);
+                    quad::cneg(q, (d < 0) != flip);
+                }
+            }
+        } else {
+            const uint32_t off = 8u >> (step - kSerial);
+#pragma unroll
+            for (int k = 0; k < L28; k++) q.v.v[k] = __shfl_down(acc.v.v[k], 4 * off, 64);
+            q.inf = __shfl_down((int)acc.inf, 4 * off, 64) != 0 || sub + off >= 16;
+        }
+        quad::add(acc, q);
+    }
+    if (sub == 0) st_quad_partial(partial, (size_t)w * stride + g, acc);
+}
+// accumulators in the 28-bit form -> XYZZ points in the memory form, a lane per coordinate
+__global__ void __launch_bounds__(64) quad_canonical_kernel(uint32_t* out, const uint32_t* sums, size_t n) {
+    const size_t q = ((size_t)blockIdx.x * 64 + threadIdx.x) >> 2;
+    if (q >= n) return;
+    const quad::Acc a = ld_quad_partial(sums, q);
+    st_fp(out + 4 * FW * q + FW * (threadIdx.x & 3), a.inf ? Fp::zero() : fp28::to_canonical(a.v));
+}
+
+// ------------------------------------------------------------------------------------------------
 // commitment through the reference-format table (entry k * npoints + i = k * G_i, k < 256, canonical
 // affine points): the reference's algorithm (byte windows, 8 doublings between windows,
 // src/Hyrax.cu:46-167) re-ordered so that it fills the chip whatever the number of rows - one wave
@@ -1361,6 +1430,35 @@ int grape_commit_i32_ref_table(uint32_t* out, const int32_t* scalars, size_t siz
 int grape_commit_fr_ref_table(uint32_t* out, const uint32_t* scalars, size_t size, uint32_t rowlen, const uint32_t* table,
                               size_t npoints, grape_stream_t st) {
     return commit_ref_impl<true>(out, scalars, size, rowlen, table, npoints, st);
+}
+
+int grape_g1_msm_windows(uint32_t* sums, const uint32_t* points, const uint32_t* scalars, size_t n, grape_stream_t st) {
+    GRAPE_REQUIRE(n >= 1 && n <= ((size_t)1 << 24), "between 1 and 2^24 points");
+    CHECK_PTR16(sums); CHECK_PTR16(points); CHECK_PTR16(scalars);
+    hipStream_t s = as_stream(st);
+    // points go through in slabs, so that their multiples stay within 64 MiB
+    const size_t slab = n < 32768 ? n : 32768;
+    const size_t groups = (n + kMsmGroup - 1) / kMsmGroup;
+    constexpr size_t kAcc = 4 * kPartialWords;
+    const size_t table_bytes = slab * kMsmMultiples * kAcc, partial_bytes = groups * kMsmWindows * kAcc;
+    void* ws;
+    int rc = scratch_get(kSlotMsm, table_bytes + partial_bytes + reduce_tmp_bytes(kMsmWindows, (uint32_t)groups) + kMsmWindows * kAcc, &ws, s);
+    if (rc) return rc;
+    uint32_t* table = (uint32_t*)ws;
+    uint32_t* partial = (uint32_t*)((char*)ws + table_bytes);
+    uint32_t* total = (uint32_t*)((char*)partial + partial_bytes);
+    uint32_t* tmp = (uint32_t*)((char*)total + kMsmWindows * kAcc);
+    for (size_t i0 = 0; i0 < n; i0 += slab) {
+        const size_t ni = n - i0 < slab ? n - i0 : slab;
+        const uint32_t ng = (uint32_t)((ni + kMsmGroup - 1) / kMsmGroup);
+        msm_multiples_kernel<<<blocks_for(ni * kMsmMultiples * 4), kBlock, 0, s>>>(table, points + 3 * FW * i0, ni);
+        msm_window_kernel<<<blocks_for((size_t)kMsmWindows * ng * 64), kBlock, 0, s>>>(partial + (i0 / kMsmGroup) * kPartialWords, table, scalars + 8 * i0, ni, ng,
+                                                                                   groups);
+    }
+    launch_reduce<false>(total, partial, kMsmWindows, (uint32_t)groups, tmp, s);
+    quad_canonical_kernel<<<blocks_for(kMsmWindows * 4, 64), 64, 0, s>>>(sums, total, kMsmWindows);
+    GRAPE_LAUNCH_CHECK();
+    return GRAPE_OK;
 }
 
 int grape_g1_affine_to_jacobian(uint32_t* out, const uint32_t* in, size_t n, grape_stream_t st) {

@@ -214,6 +214,12 @@ __device__ __forceinline__ Fp28 inverse_by(const Fp28& a) {
     return fp28::mul(out, r3);
 }
 
+__device__ __forceinline__ void cneg(Acc& a, bool flag) {
+    const int32_t m = lanes<1>() & (flag ? -1 : 0);
+#pragma unroll
+    for (int i = 0; i < fp28::N; i++) a.v.v[i] = (a.v.v[i] ^ m) - m;
+}
+
 // affine image in canonical 32-bit form: lane 0 returns x, lane 1 returns y (zero for the identity); lanes 2, 3 nothing of use
 __device__ __forceinline__ Fp to_affine(const Acc& a) {
     using namespace fp28;

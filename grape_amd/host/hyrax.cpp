@@ -446,8 +446,7 @@ Hyrax_proof Hyrax::open_impl(FrTensor* tensor_in, const int* ints, const std::ve
     FrTensor d_fold(d);                         // folded in place: a copy, the commitment may still be reading d
     d_fold.partial_eval(d_fold.size, eval_point, new_N, 0, 1);
     Fr sum_ad = grape_host::download(d_fold.gpu_data);
-    if (!G_multiples_) G_multiples_.reset(new G1FixedBase(G));
-    bn128 commit_ad = G_multiples_->mul(sum_ad);
+    bn128 commit_ad = multiple_of_G(sum_ad);
 
     struct { affine_t p; int flag[4]; } com_d_host;
     static_assert(sizeof(com_d_host) == sizeof(affine_t) + 16, "point and flag travel together");
@@ -471,25 +470,47 @@ bool Hyrax::verify(Hyrax_proof& proof, jacob_t* commitment, const std::vector<Fr
     const uint rowlen = N * com_scale;
     const uint rows = size / rowlen;
     const uint new_N = (uint)proof.z_size;
-    std::vector<jacob_t> raw(rows);
-    check(grape_memcpy_d2h(raw.data(), commitment, sizeof(jacob_t) * (size_t)rows, nullptr), "d2h");
-    std::vector<bn128> coms(rows);
-    for (uint i = 0; i < rows; i++) coms[i] = bn128(raw[i]);
     const uint inner = Log2(rowlen);
-    bn128 C = host_partial_me<bn128>(coms.data(), rows, eval_point.begin() + inner, eval_point.end());
+    // c * C, C the row commitments folded at the outer variables: sum_i c eq(outer, i) C_i, its window sums on the device
+    // and their doubling chain here.  (Folding fewer variables than the rows need leaves the first 2^variables rows.)
+    const std::vector<Fr> outer(eval_point.begin() + inner, eval_point.end());
+    const uint used = outer.size() < 32 && ((uint64_t)1 << outer.size()) < rows ? 1u << outer.size() : rows;
+    FrTensor pyramid((uint)grape_eq_pyramid_elems((uint)outer.size()));
+    fr_t* d_outer = grape_host::upload(outer);
+    check(grape_eq_pyramid(W(pyramid.gpu_data), W(d_outer), (uint)outer.size(), nullptr), "grape_eq_pyramid");
+    grape_free(d_outer);
+    fr_t* const weights = pyramid.gpu_data + (((size_t)1 << outer.size()) - 1);
+    check(grape_fr_bcast_mul(W(weights), W(weights), W(grape_host::device_scalar(c)), (size_t)1 << outer.size(), nullptr), "grape_fr_bcast_mul");
+    bucket_t* d_windows = nullptr;
+    check(grape_malloc((void**)&d_windows, sizeof(bucket_t) * GRAPE_MSM_WINDOWS), "grape_malloc");
+    check(grape_g1_msm_windows(W(d_windows), W(commitment), W(weights), used, nullptr), "grape_g1_msm_windows");
     // com(z) on the device
     std::vector<Fr> zv(proof.z, proof.z + new_N);
     FrTensor z = FrTensor::from_host(zv);
     affine_t* com_z_dev = nullptr;
     check(grape_malloc((void**)&com_z_dev, sizeof(affine_t)), "grape_malloc");
     commit_fr_rows(com_z_dev, z.gpu_data, new_N, new_N, false);
+    std::vector<bucket_t> windows(GRAPE_MSM_WINDOWS);
     affine_t com_z;
+    check(grape_memcpy_d2h(windows.data(), d_windows, sizeof(bucket_t) * windows.size(), nullptr), "grape_memcpy_d2h");
     check(grape_memcpy_d2h(&com_z, com_z_dev, sizeof(affine_t), nullptr), "d2h");
     grape_free(com_z_dev);
-    if (!(c * C + proof.commit_d == bn128(com_z))) return false;
+    grape_free(d_windows);
+    bucket_t cC = windows[GRAPE_MSM_WINDOWS - 1];
+    for (int w = GRAPE_MSM_WINDOWS - 2; w >= 0; w--) {
+        for (int d = 0; d < 4; d++) grape::xyzz_dbl(cC);
+        grape::xyzz_add(cC, windows[w]);
+    }
+    if (!(bn128(grape::xyzz_to_jac(cC)) + proof.commit_d == bn128(com_z))) return false;
+    // (c * result) * G + commit_ad == az * G, with one multiple of G
     std::vector<Fr> inner_point(eval_point.begin(), eval_point.begin() + inner);
     Fr az = z(inner_point);
-    return (c * proof.result) * G + proof.commit_ad == az * G;
+    return proof.commit_ad == multiple_of_G(az - c * proof.result);
+}
+
+bn128 Hyrax::multiple_of_G(const Fr& k) {
+    if (!G_multiples_) G_multiples_.reset(new G1FixedBase(G));
+    return G_multiples_->mul(k);
 }
 
 void Hyrax::verify(Hyrax_proof& proof, jacob_t* commitment, Fr c, uint size, uint N) {

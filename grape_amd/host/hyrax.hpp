@@ -117,11 +117,12 @@ private:
     bool commit_fr_rows(affine_t* out, fr_t* scalars, size_t size, uint rowlen, bool may_build, void* stream = nullptr, int* d_flag = nullptr);
     void commit_i32_rows(affine_t* out, int* tensor, size_t size, uint rowlen, int* d_flag, void* stream = nullptr);
     void check_shape(uint size, uint N) const;
+    bn128 multiple_of_G(const Fr& k);
     WideTable int16_table_, int16x2_table_, int32_table_, fr_table_;
     StridedTable fr_strided_;
     bool int16_ok_ = true;
     size_t scaled_bytes_ = 0;
     std::vector<Fr> last_open_point_;
-    std::unique_ptr<G1FixedBase> G_multiples_;      // built by the first opening
+    std::unique_ptr<G1FixedBase> G_multiples_;      // built by the first opening or verification
     size_t table_budget_ = (size_t)128 << 30;
 };

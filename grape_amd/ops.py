@@ -566,6 +566,14 @@ def commit_fr_ref_table(scalars, rowlen, table, npoints):
     return out
 
 
+def g1_msm_windows(points_jac, scalars):
+    """window sums (64 XYZZ points) of sum_i scalars[i] * points[i]; the sum itself is sum_w 16^w * out[w]"""
+    lib = init()
+    out = torch.empty((64, 4 * _capi.FP_WORDS), dtype=torch.int32, device="cuda")
+    _capi.check(lib.grape_g1_msm_windows(_p(out), _p(points_jac), _p(scalars), scalars.shape[0], _s()))
+    return out
+
+
 def g1_affine_to_jacobian(a):
     lib = init()
     out = torch.empty((a.shape[0], 3 * _capi.FP_WORDS), dtype=torch.int32, device="cuda")

@@ -475,6 +475,12 @@ int grape_commit_fr_ref_table(uint32_t *d_out_affine, const uint32_t *d_scalars_
 int grape_commit_fr_sparse(uint32_t *d_out_affine, const uint32_t *d_scalars_mont, const int32_t *d_skip, size_t size,
                            uint32_t rowlen, const uint32_t *d_wide_table, size_t N, uint32_t c, uint32_t nw, uint32_t K,
                            grape_stream_t stream);
+/* Window sums of sum_i k_i P_i over n arbitrary points (Jacobian, as grape_g1_affine_to_jacobian leaves them; Montgomery
+ * scalars): d_sums receives GRAPE_MSM_WINDOWS XYZZ points S_w with sum_i k_i P_i = sum_w 16^w S_w.  The chain of doublings
+ * that combines them is the caller's (the host: one core is faster at it than one lane).  1 <= n <= 2^24.  The fold of
+ * the row commitments in a verification, test/HyraxTest.cu:87-125. */
+#define GRAPE_MSM_WINDOWS 64
+int grape_g1_msm_windows(uint32_t *d_sums, const uint32_t *d_points, const uint32_t *d_scalars, size_t n, grape_stream_t stream);
 /* out[i] = a[i] + b[i] for n affine points (infinity, equal and opposite operands included); the
  * group law of include/curve/xyzz_t.cuh.  Combines two partial row commitments. */
 int grape_g1_affine_add(uint32_t *d_out_affine, const uint32_t *d_a_affine, const uint32_t *d_b_affine, size_t n,
