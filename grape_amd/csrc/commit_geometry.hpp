@@ -111,6 +111,30 @@ constexpr int kTreeThreads = 256;
 GRAPE_HD size_t tree_row(size_t block, int t) { return block * (size_t)kTreeRows + (size_t)(t & (kTreeRows - 1)); }
 GRAPE_HD uint32_t tree_share(int t) { return (uint32_t)t >> 3; }
 GRAPE_HD bool tree_reduction(size_t rows, uint32_t lg_lpr, uint32_t nparts) { return lg_lpr <= 5 && rows <= 4096 && nparts <= 4096; }
+// Workgroups are dealt to the chip's 32 shader engines in turn (workgroup i to XCD i mod 8, and in turn within it), whether
+// or not that engine has room.  Where the work of a unit depends on its position - rows of 11008 padded to 16384 leave
+// every fourth committed row empty - units in launch order leave whole engines idle.  spread_unit is a permutation
+// of 0 .. n - 1 under which every engine's workgroups sweep all positions: engine a = i mod 32 takes the a-th stretch of
+// n / 32 steps of a walk with stride `step`, a number near the golden section of n and prime to it.
+// (2^25 full-width scalars on such rows: 73.4 ms in launch order, 56.6 this way, 79 to 81 with no row empty.)
+GRAPE_HD size_t spread_unit(size_t i, size_t n, size_t step) {
+    const size_t whole = n >> 5;
+    if (i >= whole << 5) return i;
+    return (((i & 31) * whole + (i >> 5)) * step) % (whole << 5);
+}
+inline size_t spread_step(size_t n) {
+    const size_t m = n >> 5 << 5;
+    size_t step = (size_t)(0.6180339887 * (double)m) | 1;
+    for (;; step += 2) {
+        size_t a = m, b = step;
+        while (b) {
+            const size_t r = a % b;
+            a = b;
+            b = r;
+        }
+        if (a == 1 || m == 0) return step;
+    }
+}
 // workgroups of a launch of `threads` threads in groups of `per_block`
 GRAPE_HD size_t blocks_needed(size_t threads, size_t per_block) { return (threads + per_block - 1) / per_block; }
 

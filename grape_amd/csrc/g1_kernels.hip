@@ -699,6 +699,32 @@ __device__ __forceinline__ int32_t digit_of(const Fr& kb, uint32_t w, uint32_t c
     return (w * c + c - 1 < 256) ? bits - (int32_t)(1u << (c - 1)) : bits;
 }
 
+// acc += the windows j, J + j, 2J + j, ... of k * G_col
+__device__ __forceinline__ void madd_scalar_strided(Xyzz28& acc, const Fr& k_mont, const Fr& H, const uint32_t* table, size_t N, uint32_t col, uint32_t c,
+                                                    uint32_t nw, uint32_t K, uint32_t J, uint32_t nsets, uint32_t j) {
+    bool flip;
+    const Fr kb = biased_half_range(k_mont, H, flip);
+    // digit of set 0 now, the next set's one addition ahead (its table line is touched early)
+    int32_t d = j < nw ? digit_of(kb, j, c) : 0;
+    uint32_t touch = 0;
+    for (uint32_t q = 0; q < nsets; q++) {
+        const uint32_t wn = (q + 1) * J + j;
+        const int32_t d_n = (q + 1 < nsets && wn < nw) ? digit_of(kb, wn, c) : 0;
+        if (d != 0) {
+            const bool neg = d < 0;
+            const uint32_t mag = (uint32_t)(neg ? -d : d);
+            const Affine28 e = ld_entry28(table, geom::table_entry(q, K, mag, N, col));
+            const uint32_t mag_n = (uint32_t)(d_n < 0 ? -d_n : d_n);
+            const size_t nxt = mag_n != 0 ? geom::table_entry(q + 1, K, mag_n, N, col) : (size_t)col;
+            touch = table[(size_t)kWideEntryWords * nxt];
+            if (kWideEntryWords % 32 != 0) touch |= table[(size_t)kWideEntryWords * nxt + kWideEntryWords - 1];
+            madd28(acc, e, neg != flip);
+        }
+        d = d_n;
+    }
+    asm volatile("" ::"v"(touch));
+}
+
 __global__ void __launch_bounds__(kBlock) commit_strided_kernel(uint32_t* partial, const uint32_t* scalars, uint32_t rowlen, size_t rows,
                                                                 uint32_t seg, uint32_t nseg, const uint32_t* table, size_t N,
                                                                 uint32_t c, uint32_t nw, uint32_t K, uint32_t J, uint32_t nsets) {
@@ -710,29 +736,8 @@ __global__ void __launch_bounds__(kBlock) commit_strided_kernel(uint32_t* partia
     const uint32_t j = (uint32_t)(span.row - row * J);
     const Fr H = window_bias(c, nw);                      // wave-uniform
     Xyzz28 acc = xyzz28_inf();
-    for (uint32_t col = span.s * seg + lane; col < span.col_end; col += 64) {
-        bool flip;
-        const Fr kb = biased_half_range(ld_fr8(scalars, geom::scalar_index(row, rowlen, col)), H, flip);
-        // digit of set 0 now, the next set's one addition ahead (its table line is touched early)
-        int32_t d = j < nw ? digit_of(kb, j, c) : 0;
-        uint32_t touch = 0;
-        for (uint32_t q = 0; q < nsets; q++) {
-            const uint32_t wn = (q + 1) * J + j;
-            const int32_t d_n = (q + 1 < nsets && wn < nw) ? digit_of(kb, wn, c) : 0;
-            if (d != 0) {
-                const bool neg = d < 0;
-                const uint32_t mag = (uint32_t)(neg ? -d : d);
-                const Affine28 e = ld_entry28(table, geom::table_entry(q, K, mag, N, col));
-                const uint32_t mag_n = (uint32_t)(d_n < 0 ? -d_n : d_n);
-                const size_t nxt = mag_n != 0 ? geom::table_entry(q + 1, K, mag_n, N, col) : (size_t)col;
-                touch = table[(size_t)kWideEntryWords * nxt];
-                if (kWideEntryWords % 32 != 0) touch |= table[(size_t)kWideEntryWords * nxt + kWideEntryWords - 1];
-                madd28(acc, e, neg != flip);
-            }
-            d = d_n;
-        }
-        asm volatile("" ::"v"(touch));
-    }
+    for (uint32_t col = span.s * seg + lane; col < span.col_end; col += 64)
+        madd_scalar_strided(acc, ld_fr8(scalars, geom::scalar_index(row, rowlen, col)), H, table, N, col, c, nw, K, J, nsets, j);
     st_partial28(partial, wave * 64 + lane, acc);
 }
 
@@ -761,13 +766,13 @@ __global__ void __launch_bounds__(64) strided_horner_kernel(uint32_t* out, const
 // 27 live elements fills 27 of 32 lanes of its batch instead of 27 of 64.
 template <int G>
 __global__ void __launch_bounds__(64) commit_sparse_fr_kernel(uint32_t* partial, const uint32_t* scalars, const int32_t* __restrict__ skip,
-                                                              uint32_t rowlen, size_t rows, const uint32_t* table, size_t N,
+                                                              uint32_t rowlen, size_t rows, size_t step, const uint32_t* table, size_t N,
                                                               uint32_t c, uint32_t nw, uint32_t K, int* err_flag) {
     constexpr int R = 64 / G;                            // rows per wave
     __shared__ uint32_t queue[R][2 * G];
     const int lane = threadIdx.x;
     const int grp = lane / G, sub = lane % G;
-    const size_t row = (size_t)blockIdx.x * R + grp;
+    const size_t row = geom::spread_unit(blockIdx.x, gridDim.x, step) * R + grp;
     const bool have_row = row < rows;
     const unsigned long long gmask = (G == 64 ? ~0ull : ((1ull << (G & 63)) - 1ull)) << (grp * G);
     Xyzz28 acc = xyzz28_inf();
@@ -801,6 +806,48 @@ __global__ void __launch_bounds__(64) commit_sparse_fr_kernel(uint32_t* partial,
         if (last) break;
     }
     if (have_row) st_partial28(partial, row * G + sub, acc);
+}
+
+// The same through the strided table: one wave per (row, residue) queues the row's live columns and works on them in
+// batches of 64, so dead elements cost a look at their flag whether they lie scattered or in stretches, and a live one
+// the strided table's 16 to 18 additions instead of the per-window table's 20.  Worth it from some hundred live elements a
+// row (every residue leaves 64 partial sums).  One-wave workgroups, dealt by geom::spread_unit: the rows differ.
+__global__ void __launch_bounds__(64) commit_sparse_strided_kernel(uint32_t* partial, const uint32_t* scalars, const int32_t* __restrict__ skip,
+                                                                   uint32_t rowlen, size_t units, size_t step, const uint32_t* table, size_t N,
+                                                                   uint32_t c, uint32_t nw, uint32_t K, uint32_t J, uint32_t nsets) {
+    __shared__ uint32_t queue[2 * 64];
+    const int lane = threadIdx.x;
+    const size_t unit = geom::spread_unit(blockIdx.x, units, step), row = unit / J;
+    const uint32_t j = (uint32_t)(unit - row * J);
+    const Fr H = window_bias(c, nw);
+    Xyzz28 acc = xyzz28_inf();
+    uint32_t qn = 0;                                     // queued columns (uniform)
+    for (uint32_t base = 0;; base += 64) {
+        const bool last = base >= rowlen;
+        if (!last) {
+            const uint32_t col = base + lane;
+            const bool take = col < rowlen && skip[geom::scalar_index(row, rowlen, col)] == 0;
+            const unsigned long long m = __ballot(take);
+            if (take) queue[qn + __popcll(m & ((1ull << lane) - 1ull))] = col;
+            qn += (uint32_t)__popcll(m);
+            __syncthreads();
+        }
+        if (qn >= 64 || (last && qn > 0)) {
+            const uint32_t n = qn < 64 ? qn : 64;
+            if ((uint32_t)lane < n) {
+                const uint32_t col = queue[lane];
+                madd_scalar_strided(acc, ld_fr8(scalars, geom::scalar_index(row, rowlen, col)), H, table, N, col, c, nw, K, J, nsets, j);
+            }
+            __syncthreads();
+            const uint32_t moved = (uint32_t)lane + 64 < qn ? queue[lane + 64] : 0u;
+            __syncthreads();
+            if ((uint32_t)lane + 64 < qn) queue[lane] = moved;
+            qn -= n;
+            __syncthreads();
+        }
+        if (last) break;
+    }
+    st_partial28(partial, unit * 64 + lane, acc);
 }
 
 // Row epilogue: the partial sums of a row become one point, the point its affine image.  Three kernels:
@@ -1286,8 +1333,8 @@ int grape_g1_strided_table_gen(uint32_t* table, const uint32_t* gens, size_t N, 
 
 // Full-width scalars through a strided table (see commit_strided_kernel): nw = ceil(255 / c) windows,
 // J residues, nsets = ceil(nw / J) table sets of K = 2^(c-1) multiples.
-int grape_commit_fr_strided(uint32_t* out, const uint32_t* scalars, size_t size, uint32_t rowlen, const uint32_t* table, size_t N,
-                            uint32_t c, uint32_t J, uint32_t nsets, grape_stream_t st) {
+static int commit_strided_impl(uint32_t* out, const uint32_t* scalars, const int32_t* skip, size_t size, uint32_t rowlen, const uint32_t* table,
+                               size_t N, uint32_t c, uint32_t J, uint32_t nsets, grape_stream_t st) {
     if (size == 0) return GRAPE_OK;
     GRAPE_REQUIRE(size <= kMaxCommitScalars, "more than 2^28 scalars in one call: commit the rows in several calls");
     CHECK_PTR16(out); CHECK_PTR16(scalars); CHECK_PTR16(table);
@@ -1300,8 +1347,8 @@ int grape_commit_fr_strided(uint32_t* out, const uint32_t* scalars, size_t size,
     hipStream_t s = as_stream(st);
     // (row, residue) pairs are the rows of the accumulation and reduction launches
     const geom::WidePlan plan = geom::wide_plan(rows * J * (size_t)rowlen, rowlen, geom::kSlabSegments);
-    const uint32_t nseg = plan.nseg, seg = plan.seg;
-    size_t slab = plan.slab / J;                              // whole rows per launch
+    const uint32_t nseg = skip ? 1 : plan.nseg, seg = plan.seg;      // with flags a wave takes a whole row
+    size_t slab = (skip ? geom::kSlabSegments : plan.slab) / J;                              // whole rows per launch
     if (slab < 1) slab = 1;
     if (slab > rows) slab = rows;
     const size_t partial_bytes = slab * J * nseg * 64 * (size_t)(4 * kPartialWords);
@@ -1316,7 +1363,11 @@ int grape_commit_fr_strided(uint32_t* out, const uint32_t* scalars, size_t size,
         const size_t nr = rows - r0 < slab ? rows - r0 : slab;
         const uint32_t* sc = scalars + r0 * rowlen * 8;
         profile_mark(s);
-        commit_strided_kernel<<<blocks_for(nr * J * nseg * 64), kBlock, 0, s>>>((uint32_t*)ws, sc, rowlen, nr, seg, nseg, table, N, c, nw, K, J, nsets);
+        if (skip)
+            commit_sparse_strided_kernel<<<(unsigned)(nr * J), 64, 0, s>>>((uint32_t*)ws, sc, skip + r0 * rowlen, rowlen, nr * J, geom::spread_step(nr * J),
+                                                                           table, N, c, nw, K, J, nsets);
+        else
+            commit_strided_kernel<<<blocks_for(nr * J * nseg * 64), kBlock, 0, s>>>((uint32_t*)ws, sc, rowlen, nr, seg, nseg, table, N, c, nw, K, J, nsets);
         profile_mark(s);
         launch_reduce<false>(sums, (const uint32_t*)ws, nr * J, nseg * 64, red_tmp, s);
         strided_horner_kernel<<<blocks_for(nr, 64), 64, 0, s>>>(out + r0 * (size_t)(2 * FW), sums, nr, J, c);
@@ -1324,6 +1375,16 @@ int grape_commit_fr_strided(uint32_t* out, const uint32_t* scalars, size_t size,
     }
     GRAPE_LAUNCH_CHECK();
     return GRAPE_OK;
+}
+
+int grape_commit_fr_strided(uint32_t* out, const uint32_t* scalars, size_t size, uint32_t rowlen, const uint32_t* table, size_t N,
+                            uint32_t c, uint32_t J, uint32_t nsets, grape_stream_t st) {
+    return commit_strided_impl(out, scalars, nullptr, size, rowlen, table, N, c, J, nsets, st);
+}
+int grape_commit_fr_strided_masked(uint32_t* out, const uint32_t* scalars, const int32_t* skip, size_t size, uint32_t rowlen, const uint32_t* table,
+                                   size_t N, uint32_t c, uint32_t J, uint32_t nsets, grape_stream_t st) {
+    GRAPE_REQUIRE(size == 0 || skip != nullptr, "no flag array");
+    return commit_strided_impl(out, scalars, skip, size, rowlen, table, N, c, J, nsets, st);
 }
 
 int grape_g1_scaled_table_gen(uint32_t* out, const uint32_t* scalars, size_t len, size_t ncols, const uint32_t* table, size_t N,
@@ -1387,10 +1448,10 @@ int grape_commit_fr_sparse(uint32_t* out, const uint32_t* scalars, const int32_t
         const bool narrow = nr >= 4096;
         if (narrow)
             commit_sparse_fr_kernel<32><<<(unsigned)((nr + 1) / 2), 64, 0, s>>>((uint32_t*)ws, scalars + r0 * rowlen * 8, skip + r0 * rowlen, rowlen, nr,
-                                                                              table, N, c, nw, K, err);
+                                                                              geom::spread_step((nr + 1) / 2), table, N, c, nw, K, err);
         else
-            commit_sparse_fr_kernel<64><<<(unsigned)nr, 64, 0, s>>>((uint32_t*)ws, scalars + r0 * rowlen * 8, skip + r0 * rowlen, rowlen, nr, table, N,
-                                                                   c, nw, K, err);
+            commit_sparse_fr_kernel<64><<<(unsigned)nr, 64, 0, s>>>((uint32_t*)ws, scalars + r0 * rowlen * 8, skip + r0 * rowlen, rowlen, nr,
+                                                                   geom::spread_step(nr), table, N, c, nw, K, err);
         launch_reduce<true>(out + r0 * (size_t)(2 * FW), (const uint32_t*)ws, nr, narrow ? 32 : 64, red_tmp, s);
     }
     GRAPE_LAUNCH_CHECK();

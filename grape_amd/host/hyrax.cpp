@@ -339,12 +339,26 @@ affine_t* Hyrax::commit_indexed_affine(int* idx_plus1, uint size, uint N, affine
     return out;
 }
 
-affine_t* Hyrax::commit_sparse_affine(FrTensor& tensor, int* skip, uint size, uint N) {
+affine_t* Hyrax::commit_sparse_affine(FrTensor& tensor, int* skip, uint size, uint N, uint64_t live) {
     check_shape(size, N);
     const uint rowlen = N * com_scale;
+    const uint rows = size / rowlen;
+    // From 512 live elements a row the strided table is the better one: 16 to 18 additions per element instead of 20, against
+    // 64 partial sums per residue and row (2^25 elements on rows of 11008 padded to 16384, 67 % live: 56 against 92 ms; 27
+    // live elements a row: the queue of half waves over the per-window table).  It is built for a tensor at least a quarter
+    // of which is live - the build costs what 2^24 live elements save.
+    if (live >= (uint64_t)512 * rows && rows > 1 && ensure_strided_table(rowlen, 4 * live >= size)) {
+        const StridedTable& t = fr_strided_;
+        affine_t* out = nullptr;
+        check(grape_malloc((void**)&out, sizeof(affine_t) * (size_t)rows), "grape_malloc");
+        check(for_row_chunks(size, rowlen, [&](size_t e0, size_t n, size_t r0) {
+                  return grape_commit_fr_strided_masked(W(out + r0), W(tensor.gpu_data + e0), skip + e0, n, rowlen, W(t.d), t.ngen, t.c, t.J, t.nsets, nullptr);
+              }),
+              "grape_commit_fr_strided_masked");
+        return out;
+    }
     if (!ensure_fr_table(rowlen, false)) return nullptr;
     const WideTable& t = fr_table_;
-    const uint rows = size / rowlen;
     affine_t* out = nullptr;
     check(grape_malloc((void**)&out, sizeof(affine_t) * (size_t)rows), "grape_malloc");
     check(for_row_chunks(size, rowlen, [&](size_t e0, size_t n, size_t r0) {

@@ -83,9 +83,10 @@ public:
     // idx_plus1[j] = idx_j + 1 (0 = contributes nothing); rows of N*com_scale, affine output.
     affine_t* commit_indexed_affine(int* idx_plus1, uint size, uint N, affine_t* scaled_table, uint ncols, uint len, int* d_flag = nullptr);
 
-    // Row commitments of the elements whose flag skip[j] is zero, the others left out; through the
-    // per-window table that scaled tables are built with.  nullptr when that table does not exist.
-    affine_t* commit_sparse_affine(FrTensor& tensor, int* skip, uint size, uint N);
+    // Row commitments of the elements whose flag skip[j] is zero (`live` of them), the others left out; through the
+    // strided table where rows hold many of them, through the per-window table that scaled tables are built with
+    // otherwise.  nullptr when there is neither.
+    affine_t* commit_sparse_affine(FrTensor& tensor, int* skip, uint size, uint N, uint64_t live);
 
     // Upper bound for the wide fixed-base tables this object may build (default 128 GiB of the 288 GB; GRAPE_TABLE_BUDGET_GIB overrides).  When a
     // table would not fit, commitments go through the reference-format table instead.

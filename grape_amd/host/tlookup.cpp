@@ -187,7 +187,7 @@ bool tLookup::commit_A_by_occupancy(FrTensor& A, uint D, uint msm_size, Hyrax& h
         com_A = hyrax.commit_indexed_affine(d_hot, D, msm_size, hot_table_, rowlen, hot_rows_);
         if (cold != 0) {
             // the elements without a table row: queued per row and committed as full-width scalars
-            com_cold = hyrax.commit_sparse_affine(A, d_hot, D, msm_size);
+            com_cold = hyrax.commit_sparse_affine(A, d_hot, D, msm_size, cold);
             if (!com_cold) {
                 FrTensor Acold(D);
                 check(grape_fr_mask_cold(W(Acold.gpu_data), W(A.gpu_data), d_hot, D, nullptr), "grape_fr_mask_cold");

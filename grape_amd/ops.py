@@ -550,6 +550,14 @@ def commit_fr_strided(scalars, rowlen, table, N, c, J, nsets, out=None):
     return out
 
 
+def commit_fr_strided_masked(scalars, skip, rowlen, table, N, c, J, nsets):
+    lib = init()
+    size = scalars.shape[0]
+    out = g1_empty(size // rowlen)
+    _capi.check(lib.grape_commit_fr_strided_masked(_p(out), _p(scalars), _p(skip), size, rowlen, _p(table), N, c, J, nsets, _s()))
+    return out
+
+
 def commit_i32_ref_table(scalars, rowlen, table, npoints):
     lib = init()
     size = scalars.numel()

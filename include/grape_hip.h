@@ -458,6 +458,10 @@ int grape_g1_strided_table_gen(uint32_t *d_table, const uint32_t *d_gens_affine,
                                grape_stream_t stream);
 int grape_commit_fr_strided(uint32_t *d_out_affine, const uint32_t *d_scalars_mont, size_t size, uint32_t rowlen,
                             const uint32_t *d_table, size_t N, uint32_t c, uint32_t J, uint32_t nsets, grape_stream_t stream);
+/* The same over the elements whose flag skip[j] is zero, the others left out (grape_commit_fr_sparse for tensors most of
+ * whose elements are left out). */
+int grape_commit_fr_strided_masked(uint32_t *d_out_affine, const uint32_t *d_scalars_mont, const int32_t *d_skip, size_t size, uint32_t rowlen,
+                                   const uint32_t *d_table, size_t N, uint32_t c, uint32_t J, uint32_t nsets, grape_stream_t stream);
 /* Commitments through the reference-format table (k*G_i, k < 256, byte windows of |s| resp. of
  * the canonical scalar) — the reference's own algorithm, kept for tables loaded from its
  * points.bin.  Output affine. */

@@ -47,3 +47,40 @@ def test_equal_and_opposite_partial_sums(setup):
         got = ops.g1_to_host(ops.commit_i32(torch.from_numpy(rows).cuda(), 128, table, 128, 8, 2, 128))
         want = orc.commit_i32(w, ref, 128, 128)
         assert np.array_equal(got[:6], want) and np.array_equal(got[-6:], want)
+
+
+@pytest.mark.parametrize("rowlen,rows,live", [(64, 1, 1.0), (100, 33, 0.5), (128, 35, 1.0), (65, 40, 0.02), (128, 3000, 0.7)])
+@pytest.mark.parametrize("c,J", [(8, 32), (13, 5), (11, 1)])
+def test_masked_strided_commitment(setup, rowlen, rows, live, c, J):
+    """flagged-in elements only, through the strided table: the dense commitment of the tensor with the others zeroed (row
+    counts around a multiple of 32, full batches, a last partial one, rows with none)"""
+    ops, orc, _, _ = setup
+    from gpuutil import rand_fr
+    gens = ops.g1_make_generators(rand_fr(128, 501))
+    nw = (255 + c - 1) // c
+    nsets = (nw + J - 1) // J
+    table = ops.g1_strided_table_gen(gens, c, J, nsets)
+    s = rand_fr(rows * rowlen, 503)
+    rng = np.random.default_rng(rows)
+    skip = (rng.random(rows * rowlen) >= live).astype(np.int32) * 3
+    if rows > 1:
+        skip[rowlen: 2 * rowlen] = 1
+    got = ops.g1_to_host(ops.commit_fr_strided_masked(ops.to_dev(s), torch.from_numpy(skip).cuda(), rowlen, table, 128, c, J, nsets))
+    s[skip != 0] = 0
+    want = ops.g1_to_host(ops.commit_fr_strided(ops.to_dev(s), rowlen, table, 128, c, J, nsets))
+    assert np.array_equal(got, want)
+    assert rows == 1 or not got[1].any()
+    ref = orc.g1_table(orc.g1_make_generators(rand_fr(128, 501)), 256)
+    assert np.array_equal(got[-1:], orc.commit_fr(s[-rowlen:], ref, rowlen, 128))
+
+
+@pytest.mark.parametrize("n", [1, 7, 31, 32, 33, 96, 1000, 4096, 24577])
+def test_spread_units_are_a_permutation(n):
+    """the host twin of geom::spread_unit"""
+    from math import gcd
+    m = n // 32 * 32
+    step = int(0.6180339887 * m) | 1
+    while m and gcd(m, step) != 1:
+        step += 2
+    seen = {i if i >= m else ((i % 32) * (m // 32) + i // 32) * step % m for i in range(n)}
+    assert seen == set(range(n))
