@@ -29,6 +29,8 @@ SIGNATURES = {
     "grape_malloc": [ctypes.POINTER(c_void_p), c_size_t],
     "grape_free": [c_void_p],
     "grape_alloc_cache_release": [c_void_p],
+    "grape_malloc_on_default": [ctypes.POINTER(c_void_p), c_size_t],
+    "grape_free_on_default": [c_void_p],
     "grape_memcpy_h2d": [c_void_p, c_void_p, c_size_t, c_void_p],
     "grape_memcpy_d2h": [c_void_p, c_void_p, c_size_t, c_void_p],
     "grape_memcpy_d2d": [c_void_p, c_void_p, c_size_t, c_void_p],
@@ -126,6 +128,7 @@ SIGNATURES = {
     "grape_profile_enable": [c_int],
     "grape_profile_last": [ctypes.POINTER(ctypes.c_float), c_int, ctypes.POINTER(c_int)],
     "grape_stream_create": [ctypes.POINTER(c_void_p)],
+    "grape_stream_internal": [c_void_p],
     "grape_stream_destroy": [c_void_p],
     "grape_stream_wait_event": [c_void_p, c_void_p],
     "grape_event_create": [ctypes.POINTER(c_void_p)],

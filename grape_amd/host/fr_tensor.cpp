@@ -40,15 +40,16 @@ fr_t* device_scalar(const Fr& x) {
 }
 DeviceFr::DeviceFr(const Fr& x) {
     ensure_init();
-    check(grape_malloc((void**)&p_, sizeof(fr_t)), "grape_malloc");
+    check(grape_malloc_on_default((void**)&p_, sizeof(fr_t)), "grape_malloc");
     check(grape_memcpy_h2d(p_, &x, sizeof(fr_t), nullptr), "grape_memcpy_h2d");
 }
-DeviceFr::~DeviceFr() { grape_free(p_); }
+DeviceFr::~DeviceFr() { grape_free_on_default(p_); }
 
 fr_t* upload(const std::vector<Fr>& v, void* stream) {
     ensure_init();
     fr_t* d = nullptr;
-    check(grape_malloc((void**)&d, sizeof(fr_t) * std::max<size_t>(v.size(), 1)), "grape_malloc");
+    const size_t bytes = sizeof(fr_t) * std::max<size_t>(v.size(), 1);
+    check(stream ? grape_malloc((void**)&d, bytes) : grape_malloc_on_default((void**)&d, bytes), "grape_malloc");
     check(grape_memcpy_h2d(d, v.data(), sizeof(fr_t) * v.size(), stream), "grape_memcpy_h2d");
     return d;
 }
@@ -88,20 +89,25 @@ void pad_int(int** int_data, uint N, uint pad_N, uint pad_size) {
 
 FrTensor::FrTensor(uint size_) : gpu_data(nullptr), size(size_), capacity_(size_) {
     grape_host::ensure_init();
+    check(grape_malloc_on_default((void**)&gpu_data, sizeof(fr_t) * (size_t)size), "grape_malloc");
+}
+FrTensor::FrTensor(uint size_, OnAnyStream) : gpu_data(nullptr), size(size_), capacity_(size_), on_default_(false) {
+    grape_host::ensure_init();
     check(grape_malloc((void**)&gpu_data, sizeof(fr_t) * (size_t)size), "grape_malloc");
 }
 FrTensor::FrTensor(const FrTensor& t) : gpu_data(nullptr), size(t.size), capacity_(t.size) {
-    check(grape_malloc((void**)&gpu_data, sizeof(fr_t) * (size_t)size), "grape_malloc");
+    check(grape_malloc_on_default((void**)&gpu_data, sizeof(fr_t) * (size_t)size), "grape_malloc");
     check(grape_memcpy_d2d(gpu_data, t.gpu_data, sizeof(fr_t) * (size_t)size, nullptr), "grape_memcpy_d2d");
 }
 FrTensor::FrTensor(uint size_, int* int_data) : gpu_data(nullptr), size(size_), capacity_(size_) {
     grape_host::ensure_init();
-    check(grape_malloc((void**)&gpu_data, sizeof(fr_t) * (size_t)size), "grape_malloc");
+    check(grape_malloc_on_default((void**)&gpu_data, sizeof(fr_t) * (size_t)size), "grape_malloc");
     check(grape_fr_from_i32(W(gpu_data), int_data, size, nullptr), "grape_fr_from_i32");
 }
 FrTensor::~FrTensor() {
     if (gpu_data != nullptr) {
-        grape_free(gpu_data);
+        if (on_default_) grape_free_on_default(gpu_data);
+        else grape_free(gpu_data);
         gpu_data = nullptr;
     }
 }
@@ -136,7 +142,7 @@ Fr FrTensor::operator()(const std::vector<Fr>& u) {
         check(grape_fr_fold(W(gpu_data), size, W(d_u), size, 0, 1, nullptr), "grape_fr_fold");
     }
     Fr ret = grape_host::download(gpu_data);
-    grape_free(d_u);
+    grape_free_on_default(d_u);
     return ret;
 }
 void FrTensor::add_with_size(uint sz, const FrTensor& t) {
@@ -219,7 +225,7 @@ Fr FrTensor::eval_ints(const int* device_int_data, uint size, const std::vector<
     fr_t* d_u = grape_host::upload(u);
     FrTensor t = folded_from_ints(device_int_data, size, d_u, size, 0, 1);
     Fr ret = grape_host::download(t.gpu_data);
-    grape_free(d_u);
+    grape_free_on_default(d_u);
     return ret;
 }
 FrTensor FrTensor::from_host(const std::vector<Fr>& v) {

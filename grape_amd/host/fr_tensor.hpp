@@ -43,6 +43,10 @@ public:
     uint size;
 
     FrTensor(uint size);
+    // memory that is first used on a stream of its own, with nothing to order that stream behind what the default stream
+    // has queued (every other tensor lives on the default stream and takes its memory over in that stream's order)
+    struct OnAnyStream {};
+    FrTensor(uint size, OnAnyStream);
     FrTensor(const FrTensor& t);                 // deep copy
     FrTensor(uint size, int* device_int_data);   // embeds device int32 values
     ~FrTensor();
@@ -88,6 +92,7 @@ public:
 
 private:
     uint capacity_;
+    bool on_default_ = true;
 };
 
 // The fold WITHOUT the compaction that FrTensor::partial_eval adds (src/fr-tensor.cu:168-188): the

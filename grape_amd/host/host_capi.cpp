@@ -198,10 +198,10 @@ int grape_host_hyrax_commit_fr(const uint32_t* d_scalars, uint32_t size, uint32_
     jacob_t* cj = hyrax.commit(t, size, N);
     uint32_t rows = size / (N * com_scale);
     affine_t* ca = nullptr;
-    grape_host::check(grape_malloc((void**)&ca, sizeof(affine_t) * (size_t)rows), "grape_malloc");
+    grape_host::check(grape_malloc_on_default((void**)&ca, sizeof(affine_t) * (size_t)rows), "grape_malloc");
     grape_host::check(grape_g1_jacobian_to_affine((uint32_t*)ca, (const uint32_t*)cj, rows, nullptr), "jac->affine");
     grape_host::check(grape_memcpy_d2h(out_affine, ca, sizeof(affine_t) * (size_t)rows, nullptr), "d2h");
-    grape_free(ca);
+    grape_free_on_default(ca);
     grape_free(cj);
     GUARD_END
 }

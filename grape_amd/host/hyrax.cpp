@@ -425,8 +425,14 @@ Hyrax_proof Hyrax::open_impl(FrTensor* tensor_in, const int* ints, const std::ve
     static void* d_uploaded = nullptr;
     if (!open_stream) {
         check(grape_stream_create(&open_stream), "grape_stream_create");
+        check(grape_stream_internal(open_stream), "grape_stream_internal");
         check(grape_event_create(&d_uploaded), "grape_event_create");
     }
+    // left by an exception: nothing the stream still reads is freed under it
+    struct Join {
+        bool open = true;
+        ~Join() { if (open) grape_stream_sync(open_stream); }
+    } join;
     check(grape_event_record(d_uploaded, nullptr), "grape_event_record");        // a short d travels as a queued launch
     check(grape_stream_wait_event(open_stream, d_uploaded), "grape_stream_wait_event");
     // (the point and, behind it, the digit-range flag of a commitment queued without waiting)
@@ -465,16 +471,17 @@ Hyrax_proof Hyrax::open_impl(FrTensor* tensor_in, const int* ints, const std::ve
     struct { affine_t p; int flag[4]; } com_d_host;
     static_assert(sizeof(com_d_host) == sizeof(affine_t) + 16, "point and flag travel together");
     check(grape_memcpy_d2h(&com_d_host, com_d_dev, sizeof(com_d_host), open_stream), "d2h");     // waits for the commitment
+    join.open = false;
     if (flag_used && com_d_host.flag[0]) {
         grape_free(com_d_dev);
-        grape_free(eval_point);
+        grape_free_on_default(eval_point);
         throw std::runtime_error("Hyrax::open: a blinding scalar does not fit the table's digit range");
     }
     const affine_t& host_com_d = com_d_host.p;
     Hyrax_proof proof(result, new_N, bn128(host_com_d), commit_ad);
     check(grape_memcpy_d2h(proof.z, z.gpu_data, sizeof(fr_t) * (size_t)new_N, nullptr), "d2h");
     grape_free(com_d_dev);
-    grape_free(eval_point);
+    grape_free_on_default(eval_point);
     return proof;
 }
 
@@ -492,24 +499,24 @@ bool Hyrax::verify(Hyrax_proof& proof, jacob_t* commitment, const std::vector<Fr
     FrTensor pyramid((uint)grape_eq_pyramid_elems((uint)outer.size()));
     fr_t* d_outer = grape_host::upload(outer);
     check(grape_eq_pyramid(W(pyramid.gpu_data), W(d_outer), (uint)outer.size(), nullptr), "grape_eq_pyramid");
-    grape_free(d_outer);
+    grape_free_on_default(d_outer);
     fr_t* const weights = pyramid.gpu_data + (((size_t)1 << outer.size()) - 1);
     check(grape_fr_bcast_mul(W(weights), W(weights), W(grape_host::device_scalar(c)), (size_t)1 << outer.size(), nullptr), "grape_fr_bcast_mul");
     bucket_t* d_windows = nullptr;
-    check(grape_malloc((void**)&d_windows, sizeof(bucket_t) * GRAPE_MSM_WINDOWS), "grape_malloc");
+    check(grape_malloc_on_default((void**)&d_windows, sizeof(bucket_t) * GRAPE_MSM_WINDOWS), "grape_malloc");
     check(grape_g1_msm_windows(W(d_windows), W(commitment), W(weights), used, nullptr), "grape_g1_msm_windows");
     // com(z) on the device
     std::vector<Fr> zv(proof.z, proof.z + new_N);
     FrTensor z = FrTensor::from_host(zv);
     affine_t* com_z_dev = nullptr;
-    check(grape_malloc((void**)&com_z_dev, sizeof(affine_t)), "grape_malloc");
+    check(grape_malloc_on_default((void**)&com_z_dev, sizeof(affine_t)), "grape_malloc");
     commit_fr_rows(com_z_dev, z.gpu_data, new_N, new_N, false);
     std::vector<bucket_t> windows(GRAPE_MSM_WINDOWS);
     affine_t com_z;
     check(grape_memcpy_d2h(windows.data(), d_windows, sizeof(bucket_t) * windows.size(), nullptr), "grape_memcpy_d2h");
     check(grape_memcpy_d2h(&com_z, com_z_dev, sizeof(affine_t), nullptr), "d2h");
-    grape_free(com_z_dev);
-    grape_free(d_windows);
+    grape_free_on_default(com_z_dev);
+    grape_free_on_default(d_windows);
     bucket_t cC = windows[GRAPE_MSM_WINDOWS - 1];
     for (int w = GRAPE_MSM_WINDOWS - 2; w >= 0; w--) {
         for (int d = 0; d < 4; d++) grape::xyzz_dbl(cC);

@@ -20,8 +20,8 @@ namespace {
 // device buffer released on scope exit
 struct DeviceBuf {
     void* p = nullptr;
-    explicit DeviceBuf(size_t bytes) { check(grape_malloc(&p, bytes ? bytes : 1), "grape_malloc"); }
-    ~DeviceBuf() { grape_free(p); }
+    explicit DeviceBuf(size_t bytes) { check(grape_malloc_on_default(&p, bytes ? bytes : 1), "grape_malloc"); }
+    ~DeviceBuf() { grape_free_on_default(p); }
     DeviceBuf(const DeviceBuf&) = delete;
     DeviceBuf& operator=(const DeviceBuf&) = delete;
     fr_t* fr() const { return static_cast<fr_t*>(p); }
@@ -109,7 +109,7 @@ void matmul_sumcheck_phase2(FrTensor& A, FrTensor& B, FrTensor& a, FrTensor& b, 
     }
     struct Release {
         fr_t*& p;
-        ~Release() { grape_free(p); }
+        ~Release() { grape_free_on_default(p); }
     } release{d_claim};
     for (uint i = 0; i < rounds; i++) {
         if (d_claim && outputsize >= kClaimRoundMinOut) {
@@ -188,12 +188,12 @@ std::pair<Fr, Fr> prove_matmul_impl(FrTensor* A_in, FrTensor* B_in, const int* A
         if (A_claim * B_claim * eq_accumulate != claim) throw std::runtime_error("prove_matmul: A(v) * B(v) * eq != claim");
         ret = {A_claim, B_claim};
     } catch (...) {
-        grape_free(V);
-        grape_free(U);
+        grape_free_on_default(V);
+        grape_free_on_default(U);
         throw;
     }
-    grape_free(V);
-    grape_free(U);
+    grape_free_on_default(V);
+    grape_free_on_default(U);
     return ret;
 }
 
@@ -256,12 +256,12 @@ std::pair<Fr, Fr> prove_eleMul(FrTensor& A, FrTensor& B, int L, int M, int N, co
         if (A_claim * B_claim * eq_accumulate != claim) throw std::runtime_error("prove_eleMul: A(v) * B(v) * eq != claim");
         ret = {A_claim, B_claim};
     } catch (...) {
-        grape_free(V);
-        grape_free(U);
+        grape_free_on_default(V);
+        grape_free_on_default(U);
         throw;
     }
-    grape_free(V);
-    grape_free(U);
+    grape_free_on_default(V);
+    grape_free_on_default(U);
     return ret;
 }
 
@@ -326,13 +326,13 @@ Fr combine_claims(FrTensor& X, const std::vector<Fr>& claims, const std::vector<
             }
         } catch (...) {
             check(grape_stream_sync(nullptr), "sync");
-            for (fr_t* d : d_u) grape_free(d);
-            grape_free(d_v);
+            for (fr_t* d : d_u) grape_free_on_default(d);
+            grape_free_on_default(d_v);
             throw;
         }
         check(grape_stream_sync(nullptr), "sync");
-        for (fr_t* d : d_u) grape_free(d);
-        grape_free(d_v);
+        for (fr_t* d : d_u) grape_free_on_default(d);
+        grape_free_on_default(d_v);
     }
     Fr ret = X(0u);
     Fr sum = Fr::zero();

@@ -22,18 +22,18 @@ tLookup::~tLookup() {
 
 void tLookup::make_index(const FrTensor& vals, int low_) {
     drop_index();
-    check(grape_malloc((void**)&d_idx_, sizeof(int) * (size_t)(vals.size ? vals.size : 1)), "grape_malloc");
+    check(grape_malloc_on_default((void**)&d_idx_, sizeof(int) * (size_t)(vals.size ? vals.size : 1)), "grape_malloc");
     check(grape_tlookup_index(d_idx_, W(vals.gpu_data), vals.size, low_, T.size, nullptr), "grape_tlookup_index");
 }
 void tLookup::make_index_and_A(const FrTensor& key, int low_, FrTensor& A, const FrTensor* cmp, const FrTensor* cmp_table, bool write_A) {
     drop_index();
     a_ready_ = false;
     a_deferred_ = false;
-    check(grape_malloc((void**)&d_idx_, sizeof(int) * (size_t)(key.size ? key.size : 1)), "grape_malloc");
+    check(grape_malloc_on_default((void**)&d_idx_, sizeof(int) * (size_t)(key.size ? key.size : 1)), "grape_malloc");
     // The pass over the witness is queued first and its count of unmatched elements read last: in between the
     // host queues the proof's weights (a dozen small launches on the second stream) while the chip is busy.
     uint32_t* d_count = nullptr;
-    check(grape_malloc((void**)&d_count, sizeof(uint32_t)), "grape_malloc");
+    check(grape_malloc_on_default((void**)&d_count, sizeof(uint32_t)), "grape_malloc");
     uint32_t mismatches = 1;
     try {
         check(grape_tlookup_index_inverse_nowait(d_idx_, write_A ? W(A.gpu_data) : nullptr, W(key.gpu_data), key.size, low_, T.size, W(B.gpu_data),
@@ -44,10 +44,10 @@ void tLookup::make_index_and_A(const FrTensor& key, int low_, FrTensor& A, const
         check(grape_memcpy_d2h(&mismatches, d_count, sizeof(uint32_t), nullptr), "grape_memcpy_d2h");
     } catch (...) {
         grape_stream_sync(nullptr);
-        grape_free(d_count);
+        grape_free_on_default(d_count);
         throw;
     }
-    grape_free(d_count);
+    grape_free_on_default(d_count);
     a_ready_ = write_A && mismatches == 0;
     a_deferred_ = !write_A && mismatches == 0;
 }
@@ -56,9 +56,9 @@ void tLookup::make_index_and_A_from_ints(const int* key, const int* cmp, uint n,
     drop_index();
     a_ready_ = false;
     a_deferred_ = false;
-    check(grape_malloc((void**)&d_idx_, sizeof(int) * (size_t)(n ? n : 1)), "grape_malloc");
+    check(grape_malloc_on_default((void**)&d_idx_, sizeof(int) * (size_t)(n ? n : 1)), "grape_malloc");
     uint32_t* d_count = nullptr;
-    check(grape_malloc((void**)&d_count, sizeof(uint32_t)), "grape_malloc");
+    check(grape_malloc_on_default((void**)&d_count, sizeof(uint32_t)), "grape_malloc");
     uint32_t mismatches = 1;
     try {
         check(grape_tlookup_index_embed_i32_nowait(d_idx_, write_A ? W(A.gpu_data) : nullptr, W(S.gpu_data), key, cmp, n, low_, T.size,
@@ -69,24 +69,24 @@ void tLookup::make_index_and_A_from_ints(const int* key, const int* cmp, uint n,
         check(grape_memcpy_d2h(&mismatches, d_count, sizeof(uint32_t), nullptr), "grape_memcpy_d2h");
     } catch (...) {
         grape_stream_sync(nullptr);
-        grape_free(d_count);
+        grape_free_on_default(d_count);
         throw;
     }
-    grape_free(d_count);
+    grape_free_on_default(d_count);
     a_ready_ = write_A && mismatches == 0;
     a_deferred_ = !write_A && mismatches == 0;
 }
 void tLookup::pad_index(uint N, uint pad_N, uint pad_size, int fill) {
     if (!d_idx_ || N == pad_N) return;
     int* padded = nullptr;
-    check(grape_malloc((void**)&padded, sizeof(int) * (size_t)pad_size), "grape_malloc");
+    check(grape_malloc_on_default((void**)&padded, sizeof(int) * (size_t)pad_size), "grape_malloc");
     check(grape_i32_pad_fill(padded, d_idx_, N, pad_N, pad_size, fill, nullptr), "grape_i32_pad_fill");
-    grape_free(d_idx_);                       // grape_free hands a block out again only after the work queued so far
+    grape_free_on_default(d_idx_);
     d_idx_ = padded;
 }
 void tLookup::drop_index() {
     if (d_idx_ || d_hist_) {
-        grape_free(d_idx_);
+        grape_free_on_default(d_idx_);
         grape_free(d_hist_);
         d_idx_ = nullptr;
         d_hist_ = nullptr;
@@ -154,7 +154,7 @@ bool tLookup::commit_A_by_occupancy(FrTensor& A, uint D, uint msm_size, Hyrax& h
         uint32_t* d_list = nullptr;
         try {
             check(grape_malloc((void**)&hot_slot1_, sizeof(int) * (size_t)N), "grape_malloc");
-            check(grape_malloc((void**)&d_list, sizeof(uint32_t) * (size_t)N), "grape_malloc");
+            check(grape_malloc_on_default((void**)&d_list, sizeof(uint32_t) * (size_t)N), "grape_malloc");
             uint64_t info[2] = {0, 0};
             check(grape_tlookup_hot_select(d_hist_, N, min_count, (uint32_t)max_hot, hot_slot1_, d_list, info, nullptr), "grape_tlookup_hot_select");
             const uint n_hot = (uint)info[0];
@@ -169,11 +169,11 @@ bool tLookup::commit_A_by_occupancy(FrTensor& A, uint D, uint msm_size, Hyrax& h
             hot_for_ = &hyrax;
         } catch (...) {
             grape_stream_sync(nullptr);
-            grape_free(d_list);
+            grape_free_on_default(d_list);
             drop_hot_rows();
             throw;
         }
-        grape_free(d_list);
+        grape_free_on_default(d_list);
         if (!hot_table_) {
             drop_hot_rows();
             return false;
@@ -182,7 +182,7 @@ bool tLookup::commit_A_by_occupancy(FrTensor& A, uint D, uint msm_size, Hyrax& h
     int* d_hot = nullptr;
     affine_t* com_cold = nullptr;
     try {
-        check(grape_malloc((void**)&d_hot, sizeof(int) * (size_t)D), "grape_malloc");
+        check(grape_malloc_on_default((void**)&d_hot, sizeof(int) * (size_t)D), "grape_malloc");
         check(grape_tlookup_hot_index(d_hot, d_idx_, D, hot_slot1_, N, nullptr), "grape_tlookup_hot_index");
         com_A = hyrax.commit_indexed_affine(d_hot, D, msm_size, hot_table_, rowlen, hot_rows_);
         if (cold != 0) {
@@ -201,10 +201,10 @@ bool tLookup::commit_A_by_occupancy(FrTensor& A, uint D, uint msm_size, Hyrax& h
         check(grape_stream_sync(nullptr), "sync");
     } catch (...) {
         grape_stream_sync(nullptr);
-        grape_free(d_hot); grape_free(com_cold);
+        grape_free_on_default(d_hot); grape_free(com_cold);
         throw;
     }
-    grape_free(d_hot); grape_free(com_cold);
+    grape_free_on_default(d_hot); grape_free(com_cold);
     // a caller that pins the count threshold is measuring one selection: nothing is kept for the next proof
     if (hot_min_count_ != 0) drop_hot_rows();
     return true;
@@ -228,6 +228,7 @@ struct SideChain {
     explicit SideChain(int which) {
         if (!g_side_stream[which]) {
             check(grape_stream_create(&g_side_stream[which]), "grape_stream_create");
+            check(grape_stream_internal(g_side_stream[which]), "grape_stream_internal");
             check(grape_event_create(&g_side_event[which][0]), "grape_event_create");
             check(grape_event_create(&g_side_event[which][1]), "grape_event_create");
         }
@@ -274,7 +275,7 @@ void tLookup::start_weights(uint D) {
     forced_u_.clear();
     E_ready_.reset();
     if (u_ready_.size() != nu) return;          // run() reports the mismatch
-    E_ready_.reset(new FrTensor((uint)grape_eq_pyramid_elems(nu ? nu - 1 : 0)));
+    E_ready_.reset(new FrTensor((uint)grape_eq_pyramid_elems(nu ? nu - 1 : 0), FrTensor::OnAnyStream()));
     // the point travels on the second stream too: on the default stream it would queue behind the pass over the
     // witness, and the pyramid with it
     SideChain side(0);
@@ -447,7 +448,7 @@ Fr tLookup::run(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax& hyrax
         E_own.reset(new FrTensor((uint)grape_eq_pyramid_elems(nu ? nu - 1 : 0)));
         fr_t* d_u = grape_host::upload(u);
         check(grape_eq_pyramid(W(E_own->gpu_data), W(d_u), nu ? nu - 1 : 0, nullptr), "grape_eq_pyramid");
-        grape_free(d_u);                    // no wait: the block is handed out again only after what is queued here
+        grape_free_on_default(d_u);
     }
     FrTensor& E = E_early ? *E_early : *E_own;
     // The prover's challenges are all known before the first round, so the rounds are queued
@@ -552,7 +553,7 @@ Fr tLookup::run(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax& hyrax
             size_t need = 0;
             for (uint c = D; c / 2 >= kLongRoundPairs; c /= 2) need += grape_wround2_partial_bytes(c / 2);
             if (need) {
-                check(grape_malloc((void**)&long_work, need + sizeof(int32_t) * GRAPE_FOLD_TABLE_WORDS * (size_t)rounds), "grape_malloc");
+                check(grape_malloc_on_default((void**)&long_work, need + sizeof(int32_t) * GRAPE_FOLD_TABLE_WORDS * (size_t)rounds), "grape_malloc");
                 d_tabs = reinterpret_cast<int32_t*>(long_work + need);
                 for (uint k0 = 0; k0 < rounds; k0 += 64)
                     check(grape_fold_tables(d_tabs + (size_t)GRAPE_FOLD_TABLE_WORDS * k0, W(d_v + k0), std::min(64u, rounds - k0), nullptr), "grape_fold_tables");
@@ -609,9 +610,9 @@ Fr tLookup::run(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax& hyrax
         }
         S_last = h[n_sums + 1];
         Fr C = alpha_sq - h[n_sums];
-        grape_free(d_v);
+        grape_free_on_default(d_v);
         d_v = nullptr;
-        grape_free(long_work);
+        grape_free_on_default(long_work);
         long_work = nullptr;
 
         Fr alpha_run = alpha, alpha_sq_run = alpha_sq;
@@ -655,8 +656,8 @@ Fr tLookup::run(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax& hyrax
             if (vi < (int)logN) alpha_sq_run *= e;
         }
     } catch (...) {
-        grape_free(d_v);
-        grape_free(long_work);
+        grape_free_on_default(d_v);
+        grape_free_on_default(long_work);
         throw;
     }
     return S_last;
@@ -710,7 +711,7 @@ Fr tLookupRange::prove(const int* device_int_S, FrTensor& S, FrTensor& A, const 
         // proves after its own padding, whose multiplicities are those of the unpadded one plus the padding's zeros
         // (:276-281) - and proved as a witness that needs none
         int* padded = nullptr;
-        check(grape_malloc((void**)&padded, sizeof(int) * (size_t)Dp), "grape_malloc");
+        check(grape_malloc_on_default((void**)&padded, sizeof(int) * (size_t)Dp), "grape_malloc");
         Fr ret;
         try {
             check(grape_i32_pad(padded, device_int_S, 11008, 16384, Dp, nullptr), "grape_i32_pad");
@@ -718,10 +719,10 @@ Fr tLookupRange::prove(const int* device_int_S, FrTensor& S, FrTensor& A, const 
             ret = prove(padded, S, A, v, hyrax, msm_size, commit_time);
         } catch (...) {
             grape_stream_sync(nullptr);
-            grape_free(padded);
+            grape_free_on_default(padded);
             throw;
         }
-        grape_free(padded);
+        grape_free_on_default(padded);
         return ret;
     }
     if (!(D == Dp && A.size >= D)) {
@@ -825,19 +826,19 @@ Fr tLookupRangeMapping::prove(const int* device_int_S_in, const int* device_int_
         int *pin = nullptr, *pout = nullptr;
         Fr ret;
         try {
-            check(grape_malloc((void**)&pin, sizeof(int) * (size_t)Dp), "grape_malloc");
-            check(grape_malloc((void**)&pout, sizeof(int) * (size_t)Dp), "grape_malloc");
+            check(grape_malloc_on_default((void**)&pin, sizeof(int) * (size_t)Dp), "grape_malloc");
+            check(grape_malloc_on_default((void**)&pout, sizeof(int) * (size_t)Dp), "grape_malloc");
             check(grape_i32_pad(pin, device_int_S_in, 11008, 16384, Dp, nullptr), "grape_i32_pad");
             check(grape_i32_pad_fill(pout, device_int_S_out, 11008, 16384, Dp, map_zero_, nullptr), "grape_i32_pad_fill");
             ret = prove(pin, pout, Dp, A, v, hyrax, msm_size, commit_time);
         } catch (...) {
             grape_stream_sync(nullptr);
-            grape_free(pin);
-            grape_free(pout);
+            grape_free_on_default(pin);
+            grape_free_on_default(pout);
             throw;
         }
-        grape_free(pin);
-        grape_free(pout);
+        grape_free_on_default(pin);
+        grape_free_on_default(pout);
         return ret;
     }
     if (!(D == Dp && A.size >= D)) {

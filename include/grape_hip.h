@@ -60,6 +60,13 @@ int grape_free(void *d_ptr);
  * cost tens of microseconds for small blocks and milliseconds and more for multi-GiB ones.  This gives every kept block back to the
  * driver (it also happens by itself when an allocation fails).  No counterpart in the reference. */
 int grape_alloc_cache_release(size_t *bytes_released);
+/* The same for blocks that only the default stream works on, between the allocation and the free (work on other streams
+ * that was ordered before the free counts as the default stream's): such a block goes to its next owner in stream order,
+ * without an event or a wait.  The tensors of the host classes.  While a stream is about that the library cannot vouch for
+ * - one that a caller brought, or one of grape_stream_create that is not declared internal - these behave like
+ * grape_malloc and grape_free. */
+int grape_malloc_on_default(void **d_ptr, size_t bytes);
+int grape_free_on_default(void *d_ptr);
 /* Host to device, ordered like any other work on `stream`; the host buffer may be reused as soon as
  * the call returns.  At most 1 KiB (a scalar, a vector of challenges) is carried by a small kernel
  * as its argument and the call does not wait; a longer copy waits for the stream. */
@@ -566,6 +573,9 @@ int grape_profile_last(float *ms, int cap, int *n);
  * grape_stream_wait_event.  Scratch memory is per stream, so calls on different streams never share
  * any; grape_stream_destroy waits for the stream and frees its scratch. */
 int grape_stream_create(grape_stream_t *out);
+/* Declares a stream of grape_stream_create internal to code that joins it to the default stream (or waits for it) before
+ * anything it worked on is freed. */
+int grape_stream_internal(grape_stream_t stream);
 int grape_stream_destroy(grape_stream_t stream);
 int grape_stream_wait_event(grape_stream_t stream, void *ev);
 /* Event helpers on a stream (HIP events): ordering between streams, and timing for benchmarks that

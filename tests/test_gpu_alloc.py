@@ -1,0 +1,62 @@
+"""Short copies to the host around the size that goes through pinned memory, and the handing-on of default-stream blocks:
+in stream order while only known streams are about, with a wait otherwise."""
+import ctypes
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def lib():
+    from grape_amd import _capi, ops
+    ops.init(0)
+    return _capi.load()
+
+
+@pytest.mark.parametrize("nbytes", [1, 4, 6, 32, 1020, 1024, 16384, 16388, 40000])
+@pytest.mark.parametrize("offset", [0, 4, 2])
+def test_short_copies(lib, nbytes, offset):
+    src = torch.randint(0, 256, (nbytes + 8,), dtype=torch.uint8, device="cuda")
+    out = np.zeros(nbytes, dtype=np.uint8)
+    assert lib.grape_memcpy_d2h(out.ctypes.data_as(ctypes.c_void_p), ctypes.c_void_p(src.data_ptr() + offset), nbytes, None) == 0
+    assert np.array_equal(out, src.cpu().numpy()[offset:offset + nbytes])
+
+
+def _cycle(lib, n_words, value):
+    """fill a block, queue its copy into a second one, give the first back and take it again for other contents"""
+    from grape_amd import _capi
+    p, q = ctypes.c_void_p(), ctypes.c_void_p()
+    host = np.full(n_words, value, dtype=np.uint32)
+    _capi.check(lib.grape_malloc_on_default(ctypes.byref(p), 4 * n_words))
+    _capi.check(lib.grape_malloc_on_default(ctypes.byref(q), 4 * n_words))
+    _capi.check(lib.grape_memcpy_h2d(p, host.ctypes.data_as(ctypes.c_void_p), 4 * n_words, None))
+    _capi.check(lib.grape_memcpy_d2d(q, p, 4 * n_words, None))
+    _capi.check(lib.grape_free_on_default(p))
+    r = ctypes.c_void_p()
+    _capi.check(lib.grape_malloc_on_default(ctypes.byref(r), 4 * n_words))
+    _capi.check(lib.grape_memset_zero(r, 4 * n_words, None))
+    got = np.zeros(n_words, dtype=np.uint32)
+    _capi.check(lib.grape_memcpy_d2h(got.ctypes.data_as(ctypes.c_void_p), q, 4 * n_words, None))
+    again = r.value == p.value
+    for b in (q, r):
+        _capi.check(lib.grape_free_on_default(b))
+    assert np.array_equal(got, host)
+    return again
+
+
+@pytest.mark.parametrize("n_words", [1, 1000, 1 << 22])
+def test_default_blocks_are_handed_on(lib, n_words):
+    for k in range(4):
+        assert _cycle(lib, n_words, 7 + k)
+    from grape_amd import ops
+    h = ops.stream_create()                       # a stream the library cannot vouch for: the same contents, with waits
+    try:
+        for k in range(4):
+            _cycle(lib, n_words, 70 + k)
+    finally:
+        ops.stream_destroy(h)
+    p = ctypes.c_void_p()                         # a block of the other kind is taken over as well
+    assert lib.grape_malloc(ctypes.byref(p), 4 * n_words) == 0 and lib.grape_free(p) == 0
+    _cycle(lib, n_words, 700)
