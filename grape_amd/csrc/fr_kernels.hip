@@ -612,9 +612,10 @@ static int plan_fold(size_t outer, uint32_t c, uint32_t gap, uint32_t id, FoldPa
     return GRAPE_OK;
 }
 
-// grape_fr_fold on t, or - with `ints` - the fold of the integer tensor `ints` left in t: the first pass reads the
-// integers (4 bytes per element) and writes field elements, the later passes work on those as before.
-static int fold_impl(uint32_t* t, const int32_t* ints, size_t N, const uint32_t* x, uint32_t c, uint32_t id, uint32_t gap, grape_stream_t st) {
+// grape_fr_fold on t, or the fold of another tensor left in t: of field elements (`from`), which the first pass reads where
+// they are - a caller that keeps them need not copy them first, as much traffic as the fold itself - or of integers
+// (`ints`, 4 bytes per element); the later passes work on what the first one wrote.
+static int fold_impl(uint32_t* t, const uint32_t* from, const int32_t* ints, size_t N, const uint32_t* x, uint32_t c, uint32_t id, uint32_t gap, grape_stream_t st) {
     if (N == 0) return GRAPE_OK;
     CHECK_PTR16(t); CHECK_PTR16(x);
     GRAPE_REQUIRE(c >= 1 && gap >= 1 && N >= (size_t)c * gap && N % ((size_t)c * gap) == 0, "N must be a multiple of c*gap");
@@ -631,11 +632,14 @@ static int fold_impl(uint32_t* t, const int32_t* ints, size_t N, const uint32_t*
         GRAPE_LAUNCH_CHECK();
         ints = nullptr;
     }
-    if (L == 0) return GRAPE_OK;   // c == 1: nothing to bind, data already compact
+    if (L == 0) {                  // c == 1: nothing to bind, data already compact
+        if (from) GRAPE_HIP_CHECK(hipMemcpyAsync(t, from, N * 32, hipMemcpyDeviceToDevice, s));
+        return GRAPE_OK;
+    }
     plan.first_plain = ints ? 1u : 0u;
     const uint32_t* xs = x + 8 * (size_t)id;
     size_t cur_c = c;
-    const uint32_t* src = ints ? reinterpret_cast<const uint32_t*>(ints) : t;
+    const uint32_t* src = ints ? reinterpret_cast<const uint32_t*>(ints) : from ? from : t;
     // With a single outer index a pass can run in place (thread p reads p + k*stride only).
     // Otherwise passes ping-pong through scratch and the result is copied to the front.
     uint32_t* ws[2] = {nullptr, nullptr};
@@ -674,7 +678,9 @@ static int fold_impl(uint32_t* t, const int32_t* ints, size_t N, const uint32_t*
         const size_t c_out = cur_c < c_lo ? cur_c : c_lo;
         uint32_t* dst;
         if (outer == 1) {
-            dst = t;   // in place (src == t always holds here)
+            dst = t;   // in place, or from the source of the first pass
+        } else if (L == b && src != t) {
+            dst = t;   // the last pass
         } else {
             if (!ws[0]) {
                 void* p;
@@ -713,7 +719,13 @@ static int fold_impl(uint32_t* t, const int32_t* ints, size_t N, const uint32_t*
 }
 
 int grape_fr_fold(uint32_t* t, size_t N, const uint32_t* x, uint32_t c, uint32_t id, uint32_t gap, grape_stream_t st) {
-    return fold_impl(t, nullptr, N, x, c, id, gap, st);
+    return fold_impl(t, nullptr, nullptr, N, x, c, id, gap, st);
+}
+int grape_fr_fold_from(uint32_t* out, const uint32_t* in, size_t N, const uint32_t* x, uint32_t c, uint32_t id, uint32_t gap, grape_stream_t st) {
+    if (N == 0) return GRAPE_OK;
+    CHECK_PTR16(in);
+    GRAPE_REQUIRE(in != out, "the source is kept: grape_fr_fold folds in place");
+    return fold_impl(out, in, nullptr, N, x, c, id, gap, st);
 }
 
 size_t grape_fr_fold_i32_elems(size_t N, uint32_t c, uint32_t gap) {
@@ -729,7 +741,7 @@ size_t grape_fr_fold_i32_elems(size_t N, uint32_t c, uint32_t gap) {
 
 int grape_fr_fold_i32(uint32_t* out, const int32_t* in, size_t N, const uint32_t* x, uint32_t c, uint32_t id, uint32_t gap, grape_stream_t st) {
     GRAPE_REQUIRE(in != nullptr || N == 0, "null input");
-    return fold_impl(out, in, N, x, c, id, gap, st);
+    return fold_impl(out, nullptr, in, N, x, c, id, gap, st);
 }
 
 }  // extern "C"

@@ -95,7 +95,8 @@ __device__ __forceinline__ void wround2_result(uint32_t* out, const Fr* acc) {
 // IDX: A is not read but gathered, A[i] = Bt[idx1[i] - 1] (in_size == 2 n_out): the first round of a lookup whose
 // logUp tensor was never written out - the pass over the witness left the table indices only.
 template <bool BETA, bool PLAIN, bool UNIT, bool TAB, bool NOMID = false, bool IDX = false>
-__global__ void __launch_bounds__(kBlock, 2) wround2_kernel(uint32_t* A, uint32_t* S, const uint32_t* beta, const uint32_t* E,
+__global__ void __launch_bounds__(kBlock, 2) wround2_kernel(uint32_t* Aw, uint32_t* Sw, const uint32_t* A, const uint32_t* S,
+                                                         const uint32_t* beta, const uint32_t* E,
                                                          uint32_t in_size, uint32_t n_out, uint32_t rowlen, uint32_t rowpad,
                                                          const uint32_t* v, const int32_t* __restrict__ tab, uint32_t* partial,
                                                          const int32_t* __restrict__ idx1 = nullptr, const uint32_t* Bt = nullptr) {
@@ -141,11 +142,11 @@ __global__ void __launch_bounds__(kBlock, 2) wround2_kernel(uint32_t* A, uint32_
             sa0 = fr26::add(sa0, a0);
             sa1 = fr26::add(sa1, a1);
         }
-        st_fr(A, g, TAB ? foldt1(tab, a0, da) : fold1(w1, a0, da));
+        st_fr(Aw, g, TAB ? foldt1(tab, a0, da) : fold1(w1, a0, da));
         const fr26::Limbs s0r = ld_l26(S, g);
         const fr26::Limbs s1r = ld_hi26(S, g, n_out, in_size);
         const fr26::Limbs ds = fr26::sub(s1r, s0r);
-        st_fr(S, g, TAB ? foldt1(tab, s0r, ds) : fold1(w1, s0r, ds));
+        st_fr(Sw, g, TAB ? foldt1(tab, s0r, ds) : fold1(w1, s0r, ds));
         fr26::mac(W2, ead, ds);
         if (UNIT) {
             // W0 and WQ stay zero: the finishing kernel writes the coefficients they would give
@@ -317,7 +318,8 @@ static unsigned wround2_blocks(uint32_t n_out) {
 
 // The two launches of a weighted round: the pass over the operands (partial sums per workgroup; `tab`: the table of
 // the challenge's multiples, or nullptr for the single-product fold) and the kernel that finishes the sums.
-static int wround2_main(uint32_t* A, uint32_t* S, const uint32_t* beta, const uint32_t* E, uint32_t in_size, uint32_t n_out,
+// The folded operands go to Aw and Sw (A and S themselves for a round in place).
+static int wround2_main(uint32_t* Aw, uint32_t* Sw, const uint32_t* A, const uint32_t* S, const uint32_t* beta, const uint32_t* E, uint32_t in_size, uint32_t n_out,
                         uint32_t rowlen, uint32_t rowpad, const uint32_t* v, int plain_sums, const int32_t* tab, uint32_t* partial,
                         hipStream_t s) {
     const unsigned nb = wround2_blocks(n_out);
@@ -327,13 +329,13 @@ static int wround2_main(uint32_t* A, uint32_t* S, const uint32_t* beta, const ui
 #define GRAPE_WROUND2(B, P, U)                                                                                        \
     do {                                                                                                              \
         if (use_tab && !((P) && !(U)))                                                                                \
-            wround2_kernel<B, P, U, !((P) && !(U))><<<nb, kBlock, 0, s>>>(A, S, beta, E, in_size, n_out, rowlen, rowpad, v, tab, partial); \
-        else wround2_kernel<B, P, U, false><<<nb, kBlock, 0, s>>>(A, S, beta, E, in_size, n_out, rowlen, rowpad, v, nullptr, partial);    \
+            wround2_kernel<B, P, U, !((P) && !(U))><<<nb, kBlock, 0, s>>>(Aw, Sw, A, S, beta, E, in_size, n_out, rowlen, rowpad, v, tab, partial); \
+        else wround2_kernel<B, P, U, false><<<nb, kBlock, 0, s>>>(Aw, Sw, A, S, beta, E, in_size, n_out, rowlen, rowpad, v, nullptr, partial);    \
     } while (0)
     if (plain_sums == 3) {
         // the middle coefficient is left to the caller (sums[1] = 0); long rounds of a logUp proof
         GRAPE_REQUIRE(beta != nullptr && use_tab, "the round without its middle coefficient is built for logUp rounds of 2^16 index pairs and more");
-        wround2_kernel<true, true, false, true, true><<<nb, kBlock, 0, s>>>(A, S, beta, E, in_size, n_out, rowlen, rowpad, v, tab, partial);
+        wround2_kernel<true, true, false, true, true><<<nb, kBlock, 0, s>>>(Aw, Sw, A, S, beta, E, in_size, n_out, rowlen, rowpad, v, tab, partial);
     } else if (plain_sums == 2) {
         GRAPE_REQUIRE(rowlen == rowpad && in_size == 2 * (uint64_t)n_out,
                       "the inverse-pair round needs whole pairs and unpadded rows (weights that sum to one)");
@@ -370,8 +372,8 @@ static void wround2_final(uint32_t* sums, const uint32_t* partial, uint32_t n_ou
     GRAPE_REQUIRE(rowlen >= 1 && rowlen <= rowpad, "need 1 <= rowlen <= rowpad");                                        \
     if (beta) CHECK_PTR16(beta)
 
-int grape_wround2(uint32_t* A, uint32_t* S, const uint32_t* beta, const uint32_t* E, uint32_t in_size, uint32_t n_out,
-                  uint32_t rowlen, uint32_t rowpad, const uint32_t* v, int plain_sums, uint32_t* sums, grape_stream_t st) {
+static int wround2_impl(uint32_t* Aw, uint32_t* Sw, const uint32_t* A, const uint32_t* S, const uint32_t* beta, const uint32_t* E, uint32_t in_size,
+                        uint32_t n_out, uint32_t rowlen, uint32_t rowpad, const uint32_t* v, int plain_sums, uint32_t* sums, grape_stream_t st) {
     GRAPE_WROUND2_CHECKS();
     CHECK_PTR16(sums);
     hipStream_t s = as_stream(st);
@@ -386,11 +388,20 @@ int grape_wround2(uint32_t* A, uint32_t* S, const uint32_t* beta, const uint32_t
         tab = (int32_t*)((char*)ws + partial_bytes);
         fold_tables_kernel<<<1, 64, 0, s>>>(tab, v, 1);
     }
-    rc = wround2_main(A, S, beta, E, in_size, n_out, rowlen, rowpad, v, plain_sums, tab, partial, s);
+    rc = wround2_main(Aw, Sw, A, S, beta, E, in_size, n_out, rowlen, rowpad, v, plain_sums, tab, partial, s);
     if (rc) return rc;
     wround2_final(sums, partial, n_out, plain_sums, s);
     GRAPE_LAUNCH_CHECK();
     return GRAPE_OK;
+}
+int grape_wround2(uint32_t* A, uint32_t* S, const uint32_t* beta, const uint32_t* E, uint32_t in_size, uint32_t n_out,
+                  uint32_t rowlen, uint32_t rowpad, const uint32_t* v, int plain_sums, uint32_t* sums, grape_stream_t st) {
+    return wround2_impl(A, S, A, S, beta, E, in_size, n_out, rowlen, rowpad, v, plain_sums, sums, st);
+}
+int grape_wround2_from(uint32_t* A_out, uint32_t* S_out, const uint32_t* A, const uint32_t* S, const uint32_t* E, uint32_t in_size, uint32_t n_out,
+                       uint32_t rowlen, uint32_t rowpad, const uint32_t* v, uint32_t* sums, grape_stream_t st) {
+    CHECK_PTR16(A_out); CHECK_PTR16(S_out);
+    return wround2_impl(A_out, S_out, A, S, nullptr, E, in_size, n_out, rowlen, rowpad, v, 0, sums, st);
 }
 
 size_t grape_wround2_partial_bytes(uint32_t n_out) { return (size_t)wround2_blocks(n_out ? n_out : 1) * 5 * 32; }
@@ -411,7 +422,7 @@ int grape_wround2_queue(uint32_t* A, uint32_t* S, const uint32_t* beta, const ui
     GRAPE_WROUND2_CHECKS();
     CHECK_PTR16(partial);
     GRAPE_REQUIRE(tab == nullptr || n_out >= kTableFoldMinOut, "the table fold is built for rounds of 2^16 index pairs and more");
-    int rc = wround2_main(A, S, beta, E, in_size, n_out, rowlen, rowpad, v, plain_sums, tab, partial, as_stream(st));
+    int rc = wround2_main(A, S, A, S, beta, E, in_size, n_out, rowlen, rowpad, v, plain_sums, tab, partial, as_stream(st));
     if (rc) return rc;
     GRAPE_LAUNCH_CHECK();
     return GRAPE_OK;
@@ -424,7 +435,7 @@ int grape_wround2_queue_indexed(uint32_t* A, uint32_t* S, const int32_t* idx1, c
     GRAPE_REQUIRE(idx1 != nullptr && len >= 1, "bad arguments");
     GRAPE_REQUIRE(tab != nullptr && n_out >= kTableFoldMinOut && n_out <= (1u << 30), "built for first rounds of 2^16 index pairs and more");
     wround2_kernel<true, true, true, true, false, true><<<wround2_blocks(n_out), kBlock, 0, as_stream(st)>>>(
-        A, S, beta, E, 2 * n_out, n_out, 1, 1, v, tab, partial, idx1, Bt);
+        A, S, A, S, beta, E, 2 * n_out, n_out, 1, 1, v, tab, partial, idx1, Bt);
     GRAPE_LAUNCH_CHECK();
     return GRAPE_OK;
 }

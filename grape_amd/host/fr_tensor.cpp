@@ -208,6 +208,14 @@ FrTensor FrTensor::random(uint size) {
     for (uint i = 0; i < size; i++) tmp[i] = Fr::random_element();
     return from_host(tmp);
 }
+FrTensor FrTensor::folded_from(const fr_t* device_data, uint N, fr_t* x, uint c, uint id, uint gap) {
+    grape_host::ensure_init();
+    const size_t elems = grape_fr_fold_i32_elems(N, c, gap);
+    FrTensor out((uint)(elems ? elems : 1));
+    check(grape_fr_fold_from(W(out.gpu_data), W(device_data), N, W(x), c, id, gap, nullptr), "grape_fr_fold_from");
+    out.set_size(c && gap ? N / (c * gap) * gap : 0);
+    return out;
+}
 FrTensor FrTensor::folded_from_ints(const int* device_int_data, uint N, fr_t* x, uint c, uint id, uint gap) {
     grape_host::ensure_init();
     const size_t elems = grape_fr_fold_i32_elems(N, c, gap);

@@ -5,6 +5,7 @@
 
 using grape_host::check;
 static inline uint32_t* W(fr_t* p) { return reinterpret_cast<uint32_t*>(p); }
+static inline const uint32_t* W(const fr_t* p) { return reinterpret_cast<const uint32_t*>(p); }
 
 static void record(SumcheckTranscript* t, const Polynomial& p, const Fr& claim) {
     if (t) {
@@ -142,9 +143,25 @@ void matmul_sumcheck_phase2(FrTensor& A, FrTensor& B, FrTensor& a, FrTensor& b, 
     }
 }
 
-// src/prove.cu:175-210
-std::pair<Fr, Fr> prove_matmul(FrTensor& A, FrTensor& B, int L, int N, int M, int K, const std::vector<Fr> u,
-                               const std::vector<Fr> v, Fr& claim, SumcheckTranscript* transcript) {
+namespace {
+// An operand of prove_matmul: a tensor that the proof consumes, or a tensor of field elements or of integers (read as
+// FrTensor::get_data would embed them) that is kept - the fold over its row variables, which reads it once, reads it in place.
+struct Operand {
+    FrTensor* consumed = nullptr;
+    const fr_t* kept = nullptr;
+    const int* ints = nullptr;
+    std::unique_ptr<FrTensor> own;
+    FrTensor& fold(uint size, fr_t* x, uint c, uint id, uint gap) {
+        if (consumed) {
+            consumed->partial_eval(size, x, c, id, gap);
+            return *consumed;
+        }
+        own.reset(new FrTensor(kept ? FrTensor::folded_from(kept, size, x, c, id, gap) : FrTensor::folded_from_ints(ints, size, x, c, id, gap)));
+        return *own;
+    }
+};
+std::pair<Fr, Fr> prove_matmul_impl(Operand A_op, Operand B_op, int L, int N, int M, int K, const std::vector<Fr>& u, const std::vector<Fr>& v,
+                                    Fr& claim, SumcheckTranscript* transcript) {
     // The point u is read as log2(M) variables of the column index, log2(N) of the row index and log2(L)
     // of the batch index, while the reference finds the end of the batch variables at Log2(L*N*M)
     // (src/prove.cu:198): the two agree only when the padded extents multiply to the padded product.
@@ -153,33 +170,12 @@ std::pair<Fr, Fr> prove_matmul(FrTensor& A, FrTensor& B, int L, int N, int M, in
     const uint lu = Log2((uint)L) + Log2((uint)N) + Log2((uint)M);
     if (L < 1 || N < 1 || M < 1 || K < 1 || Log2((uint)(L * N * M)) != lu || u.size() < lu || v.size() < Log2((uint)(L * K)))
         throw std::runtime_error("prove_matmul: Incompatible dimensions");
-    return prove_matmul_impl(&A, &B, nullptr, nullptr, L, N, M, K, u, v, claim, transcript);
-}
-std::pair<Fr, Fr> prove_matmul(const int* device_int_A, const int* device_int_B, int L, int N, int M, int K, const std::vector<Fr> u,
-                               const std::vector<Fr> v, Fr& claim, SumcheckTranscript* transcript) {
-    const uint lu = Log2((uint)L) + Log2((uint)N) + Log2((uint)M);
-    if (L < 1 || N < 1 || M < 1 || K < 1 || Log2((uint)(L * N * M)) != lu || u.size() < lu || v.size() < Log2((uint)(L * K)))
-        throw std::runtime_error("prove_matmul: Incompatible dimensions");
-    return prove_matmul_impl(nullptr, nullptr, device_int_A, device_int_B, L, N, M, K, u, v, claim, transcript);
-}
-// A_in / B_in, or the integer tensors read as FrTensor::get_data would embed them: the folds over the row variables, which
-// read each operand once, then read the integers themselves
-std::pair<Fr, Fr> prove_matmul_impl(FrTensor* A_in, FrTensor* B_in, const int* A_ints, const int* B_ints, int L, int N, int M, int K,
-                                    const std::vector<Fr>& u, const std::vector<Fr>& v, Fr& claim, SumcheckTranscript* transcript) {
     fr_t* U = grape_host::upload(u);
     fr_t* V = grape_host::upload(v);
     std::pair<Fr, Fr> ret;
     try {
-        std::unique_ptr<FrTensor> A_own, B_own;
-        if (A_ints) {
-            A_own.reset(new FrTensor(FrTensor::folded_from_ints(A_ints, (uint)(L * N * K), U, N, Log2(M), K)));
-            B_own.reset(new FrTensor(FrTensor::folded_from_ints(B_ints, (uint)(L * M * K), U, M, 0, K)));
-        } else {
-            A_in->partial_eval(A_in->size, U, N, Log2(M), K);
-            B_in->partial_eval(B_in->size, U, M, 0, K);
-        }
-        FrTensor& A = A_ints ? *A_own : *A_in;
-        FrTensor& B = A_ints ? *B_own : *B_in;
+        FrTensor& A = A_op.fold((uint)(L * N * K), U, N, Log2(M), K);
+        FrTensor& B = B_op.fold((uint)(L * M * K), U, M, 0, K);
         FrTensor a(1), b(1), c(1);      // the reference's coefficient arrays (src/prove.cu:190-192): not used by the fused rounds
         Fr eq_accumulate = matmul_sumcheck_phase1(A, B, a, b, c, U + Log2(L * N * M), V + Log2(L * K), K, K * L, claim, transcript);
         matmul_sumcheck_phase2(A, B, a, b, c, V + Log2(K), K, claim, eq_accumulate, transcript);
@@ -196,6 +192,30 @@ std::pair<Fr, Fr> prove_matmul_impl(FrTensor* A_in, FrTensor* B_in, const int* A
     grape_free_on_default(U);
     return ret;
 }
+}  // namespace
+
+// src/prove.cu:175-210
+std::pair<Fr, Fr> prove_matmul(FrTensor& A, FrTensor& B, int L, int N, int M, int K, const std::vector<Fr> u,
+                               const std::vector<Fr> v, Fr& claim, SumcheckTranscript* transcript) {
+    Operand a, b;
+    a.consumed = &A;
+    b.consumed = &B;
+    return prove_matmul_impl(std::move(a), std::move(b), L, N, M, K, u, v, claim, transcript);
+}
+std::pair<Fr, Fr> prove_matmul(const fr_t* device_A, const fr_t* device_B, int L, int N, int M, int K, const std::vector<Fr> u,
+                               const std::vector<Fr> v, Fr& claim, SumcheckTranscript* transcript) {
+    Operand a, b;
+    a.kept = device_A;
+    b.kept = device_B;
+    return prove_matmul_impl(std::move(a), std::move(b), L, N, M, K, u, v, claim, transcript);
+}
+std::pair<Fr, Fr> prove_matmul(const int* device_int_A, const int* device_int_B, int L, int N, int M, int K, const std::vector<Fr> u,
+                               const std::vector<Fr> v, Fr& claim, SumcheckTranscript* transcript) {
+    Operand a, b;
+    a.ints = device_int_A;
+    b.ints = device_int_B;
+    return prove_matmul_impl(std::move(a), std::move(b), L, N, M, K, u, v, claim, transcript);
+}
 
 // The element-product sumcheck (src/prove.cu:119-172) proves sum_x eq(u, x) A(x) B(x) over tensors
 // of first_size rows of second_size = size / first_size elements, the row index bound first
@@ -204,11 +224,10 @@ std::pair<Fr, Fr> prove_matmul_impl(FrTensor* A_in, FrTensor* B_in, const int* A
 // of u; here a round is one launch that folds A and B and takes the three sums weighted by
 // eq(u_low, x) from a pyramid of tables built once - on rows padded to a power of two, which is
 // where the variables of u live.
-Fr eleMul_sumcheck(FrTensor& A, FrTensor& B, FrTensor& a, FrTensor& b, FrTensor& c, fr_t* u, fr_t* v, uint first_size, uint size,
-                   Fr& claim, SumcheckTranscript* transcript) {
-    (void)a;
-    (void)b;
-    (void)c;
+// A and B are read by the first round, every round leaves its folded halves in Aw and Bw (A and B themselves, or
+// buffers of size / 2 elements where the operands are kept).
+static Fr eleMul_rounds(fr_t* Aw, fr_t* Bw, const fr_t* A, const fr_t* B, fr_t* u, fr_t* v, uint first_size, uint size, Fr& claim,
+                        SumcheckTranscript* transcript) {
     if ((1u << Log2(first_size)) != first_size) throw std::runtime_error("eleMul_sumcheck: first_size is illegal");
     const uint second_size = size / first_size;
     const uint rounds = Log2(size);
@@ -222,9 +241,9 @@ Fr eleMul_sumcheck(FrTensor& A, FrTensor& B, FrTensor& a, FrTensor& b, FrTensor&
     for (uint i = 0; i < rounds; i++) {
         // while whole rows are paired the weights are addressed on padded rows
         const bool rows = in > second_size && second_size != row_pad;
-        check(grape_wround2(W(A.gpu_data), W(B.gpu_data), nullptr, W(eq.level(rounds - 1 - i)), in, out, rows ? second_size : 1,
-                            rows ? row_pad : 1, W(v - i - 1), 0, W(sums.gpu_data + 3 * i), nullptr),
-              "grape_wround2");
+        check(grape_wround2_from(W(Aw), W(Bw), i ? W(Aw) : W(A), i ? W(Bw) : W(B), W(eq.level(rounds - 1 - i)), in, out, rows ? second_size : 1,
+                                 rows ? row_pad : 1, W(v - i - 1), W(sums.gpu_data + 3 * i), nullptr),
+              "grape_wround2_from");
         in = out;
         out = out == second_size ? (1u << (Log2(out) - 1)) : out / 2;
         if (out == 0) out = 1;
@@ -242,17 +261,24 @@ Fr eleMul_sumcheck(FrTensor& A, FrTensor& B, FrTensor& a, FrTensor& b, FrTensor&
     return eq_accumulate;
 }
 
-// src/prove.cu:212-243
-std::pair<Fr, Fr> prove_eleMul(FrTensor& A, FrTensor& B, int L, int M, int N, const std::vector<Fr> u, const std::vector<Fr> v,
-                               Fr& claim, SumcheckTranscript* transcript) {
+Fr eleMul_sumcheck(FrTensor& A, FrTensor& B, FrTensor& a, FrTensor& b, FrTensor& c, fr_t* u, fr_t* v, uint first_size, uint size,
+                   Fr& claim, SumcheckTranscript* transcript) {
+    (void)a;
+    (void)b;
+    (void)c;
+    return eleMul_rounds(A.gpu_data, B.gpu_data, A.gpu_data, B.gpu_data, u, v, first_size, size, claim, transcript);
+}
+
+static std::pair<Fr, Fr> prove_eleMul_impl(fr_t* Aw, fr_t* Bw, const fr_t* A, const fr_t* B, int L, int M, int N, const std::vector<Fr>& u,
+                                           const std::vector<Fr>& v, Fr& claim, SumcheckTranscript* transcript) {
     fr_t* U = grape_host::upload(u);
     fr_t* V = grape_host::upload(v);
     std::pair<Fr, Fr> ret;
     try {
-        FrTensor a(1), b(1), c(1);      // the reference's coefficient arrays (src/prove.cu:224-226): not used by the fused rounds
-        Fr eq_accumulate = eleMul_sumcheck(A, B, a, b, c, U + Log2(L * N * M), V + Log2(L * M * N), L * M, L * M * N, claim, transcript);
-        Fr A_claim = grape_host::download(A.gpu_data);
-        Fr B_claim = grape_host::download(B.gpu_data);
+        const uint size = (uint)(L * M * N);
+        Fr eq_accumulate = eleMul_rounds(Aw, Bw, A, B, U + Log2(size), V + Log2(size), (uint)(L * M), size, claim, transcript);
+        Fr A_claim = grape_host::download(size == 1 ? A : Aw);
+        Fr B_claim = grape_host::download(size == 1 ? B : Bw);
         if (A_claim * B_claim * eq_accumulate != claim) throw std::runtime_error("prove_eleMul: A(v) * B(v) * eq != claim");
         ret = {A_claim, B_claim};
     } catch (...) {
@@ -263,6 +289,17 @@ std::pair<Fr, Fr> prove_eleMul(FrTensor& A, FrTensor& B, int L, int M, int N, co
     grape_free_on_default(V);
     grape_free_on_default(U);
     return ret;
+}
+// src/prove.cu:212-243
+std::pair<Fr, Fr> prove_eleMul(FrTensor& A, FrTensor& B, int L, int M, int N, const std::vector<Fr> u, const std::vector<Fr> v,
+                               Fr& claim, SumcheckTranscript* transcript) {
+    return prove_eleMul_impl(A.gpu_data, B.gpu_data, A.gpu_data, B.gpu_data, L, M, N, u, v, claim, transcript);
+}
+std::pair<Fr, Fr> prove_eleMul(const fr_t* device_A, const fr_t* device_B, int L, int M, int N, const std::vector<Fr> u,
+                               const std::vector<Fr> v, Fr& claim, SumcheckTranscript* transcript) {
+    const uint size = (uint)(L * M * N);
+    FrTensor Aw(size / 2 + 1), Bw(size / 2 + 1);
+    return prove_eleMul_impl(Aw.gpu_data, Bw.gpu_data, device_A, device_B, L, M, N, u, v, claim, transcript);
 }
 
 // combine_claims (src/prove.cu:245-300) merges several claims X(u_j) = claim_j about one tensor into

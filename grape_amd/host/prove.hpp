@@ -43,8 +43,11 @@ std::pair<Fr, Fr> prove_matmul(FrTensor& A, FrTensor& B, int L, int N, int M, in
 // the operands and prove, test/llm.cu:85-95): the folds over the row variables read the integers
 std::pair<Fr, Fr> prove_matmul(const int* device_int_A, const int* device_int_B, int L, int N, int M, int K, const std::vector<Fr> u,
                                const std::vector<Fr> v, Fr& claim, SumcheckTranscript* transcript = nullptr);
-std::pair<Fr, Fr> prove_matmul_impl(FrTensor* A, FrTensor* B, const int* A_ints, const int* B_ints, int L, int N, int M, int K,
-                                    const std::vector<Fr>& u, const std::vector<Fr>& v, Fr& claim, SumcheckTranscript* transcript);
+// additions: the same proofs over field tensors in device memory that are kept (the FrTensor forms consume their operands)
+std::pair<Fr, Fr> prove_matmul(const fr_t* device_A, const fr_t* device_B, int L, int N, int M, int K, const std::vector<Fr> u,
+                               const std::vector<Fr> v, Fr& claim, SumcheckTranscript* transcript = nullptr);
+std::pair<Fr, Fr> prove_eleMul(const fr_t* device_A, const fr_t* device_B, int L, int M, int N, const std::vector<Fr> u,
+                               const std::vector<Fr> v, Fr& claim, SumcheckTranscript* transcript = nullptr);
 std::pair<Fr, Fr> prove_eleMul(FrTensor& A, FrTensor& B, int L, int M, int N, const std::vector<Fr> u,
                                const std::vector<Fr> v, Fr& claim, SumcheckTranscript* transcript = nullptr);
 Fr combine_claims(FrTensor& X, const std::vector<Fr>& claims, const std::vector<std::vector<Fr>>& u,

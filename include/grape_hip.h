@@ -130,6 +130,10 @@ int grape_fr_fold(uint32_t *d_t, size_t N, const uint32_t *d_x, uint32_t c, uint
  * get_data + partial_eval / operator() / Hyrax::open on an integer tensor (test/llm.cu:99-125).
  */
 size_t grape_fr_fold_i32_elems(size_t N, uint32_t c, uint32_t gap);
+/* The fold of a field tensor that is kept: d_in is read by the first pass and not modified, the result and what the passes
+ * leave in between go to d_out, which must hold grape_fr_fold_i32_elems(N, c, gap) elements. */
+int grape_fr_fold_from(uint32_t *d_out, const uint32_t *d_in, size_t N, const uint32_t *d_x, uint32_t c, uint32_t id, uint32_t gap,
+                       grape_stream_t stream);
 int grape_fr_fold_i32(uint32_t *d_out, const int32_t *d_in, size_t N, const uint32_t *d_x, uint32_t c, uint32_t id, uint32_t gap,
                       grape_stream_t stream);
 
@@ -233,6 +237,10 @@ int grape_fold_tables(int32_t *d_tabs, const uint32_t *d_v, uint32_t count, grap
 int grape_wround2_queue(uint32_t *d_A, uint32_t *d_S, const uint32_t *d_beta, const uint32_t *d_e, uint32_t in_size, uint32_t n_out,
                         uint32_t rowlen, uint32_t rowpad, const uint32_t *d_v, int plain_sums, const int32_t *d_tab,
                         uint32_t *d_partial, grape_stream_t stream);
+/* The round of grape_wround2 (plain_sums 0) that keeps its operands: A and S are read, the folded halves written to
+ * d_A_out and d_S_out (n_out elements each). */
+int grape_wround2_from(uint32_t *d_A_out, uint32_t *d_S_out, const uint32_t *d_A, const uint32_t *d_S, const uint32_t *d_eq, uint32_t in_size,
+                       uint32_t n_out, uint32_t rowlen, uint32_t rowpad, const uint32_t *d_v, uint32_t *d_sums, grape_stream_t stream);
 int grape_wround2_finish(uint32_t *d_sums, const uint32_t *d_partial, uint32_t n_out, int plain_sums, grape_stream_t stream);
 /*
  * grape_wround2_queue with plain_sums == 2 for a logUp tensor that was never written out: the first round of a

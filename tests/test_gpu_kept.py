@@ -1,0 +1,44 @@
+"""Folds and rounds that keep their operands, against the in-place forms."""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from grape_amd import ops
+    ops.init(0)
+    return ops
+
+
+# (outer, c, gap): nothing to bind, the finish kernel alone, one pass and several, with one outer index and many, ragged extents
+@pytest.mark.parametrize("outer,c,gap", [(1, 1, 5), (3, 1, 7), (1, 2048, 1), (5, 100, 3), (1, 1 << 17, 1), (1, 11008, 16), (3, 5000, 40), (300, 16, 8),
+                                         (300, 33, 100)])
+def test_fold_of_a_kept_tensor(ops, outer, c, gap):
+    from gpuutil import rand_fr
+    from grape_amd import _capi
+    N = outer * c * gap
+    t = ops.to_dev(rand_fr(N, 701))
+    x = ops.to_dev(rand_fr(20, 702))
+    keep = t.clone()
+    lib = _capi.load()
+    out = torch.full((max(1, lib.grape_fr_fold_i32_elems(N, c, gap)), 8), -1, dtype=torch.int32, device="cuda")
+    _capi.check(lib.grape_fr_fold_from(ops._p(out), ops._p(t), N, ops._p(x), c, 1, gap, ops._s()))
+    assert torch.equal(t, keep)
+    ops.fr_fold(t, N, x, c, 1, gap)
+    assert torch.equal(out[: outer * gap], t[: outer * gap])
+
+
+@pytest.mark.parametrize("in_size,n_out", [(2, 1), (600, 300), (1023, 512), (1 << 18, 1 << 17)])
+def test_weighted_round_of_kept_operands(ops, in_size, n_out):
+    from gpuutil import rand_fr
+    from grape_amd import _capi
+    A, S, E, v = (ops.to_dev(rand_fr(n, 710 + k)) for k, n in enumerate((in_size, in_size, n_out, 1)))
+    a, s = A.clone(), S.clone()
+    Aw, Sw, sums = ops.fr_empty(n_out), ops.fr_empty(n_out), ops.fr_empty(3)
+    _capi.check(_capi.load().grape_wround2_from(ops._p(Aw), ops._p(Sw), ops._p(A), ops._p(S), ops._p(E), in_size, n_out, 1, 1, ops._p(v), ops._p(sums), ops._s()))
+    assert torch.equal(A, a) and torch.equal(S, s)
+    want = ops.wround2(a, s, None, E, in_size, n_out, v)
+    assert torch.equal(sums, want) and torch.equal(Aw, a[:n_out]) and torch.equal(Sw, s[:n_out])
