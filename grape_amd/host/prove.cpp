@@ -160,6 +160,52 @@ struct Operand {
         return *own;
     }
 };
+// Both phases where the folded operands are short: all rounds in one call, and one copy brings their sums and the two
+// elements that are left.  u, v (host) and U, V (device) point behind the variables of the batch and inner index.
+std::pair<Fr, Fr> matmul_short_rounds(FrTensor& A, FrTensor& B, int L, int K, const Fr* u, const Fr* v, const fr_t* U, const fr_t* V, Fr& claim,
+                                      Fr& eq_accumulate, SumcheckTranscript* transcript) {
+    const uint phase1 = Log2((uint)L), rounds = phase1 + Log2((uint)K);
+    FrTensor sums(3 * rounds + 2);
+    grape_short_rounds_args a{};
+    a.kind = GRAPE_SHORT_PAIR;
+    a.size = (uint)L * (uint)K;
+    a.row = (uint)K;
+    a.v_end = W(V);
+    a.sums = W(sums.gpu_data);
+    a.stride = 3;
+    FrTensor* const x[2] = {&A, &B};
+    for (uint k = 0; k < 2; k++) {
+        a.x[k] = a.last[k] = W(x[k]->gpu_data);
+        a.last_copy[k] = W(sums.gpu_data + 3 * rounds + k);
+    }
+    std::unique_ptr<EqPyramid> eq;
+    if (phase1) {
+        eq.reset(new EqPyramid(U - phase1, phase1 - 1));
+        a.weights = GRAPE_SHORT_ROWS;
+        a.pyramid = W(eq->level(0));
+        a.top_level = phase1 - 1;
+    }
+    check(grape_short_rounds(&a, nullptr), "grape_short_rounds");
+    const std::vector<Fr> s = download_vec(sums.gpu_data, 3 * (size_t)rounds + 2);
+    eq_accumulate = Fr::one();
+    for (uint i = 0; i < rounds; i++) {
+        const Fr& v_now = *(v - 1 - i);
+        Polynomial p;
+        if (i < phase1) {
+            const Fr& u_now = *(u - 1 - i);
+            p = Polynomial({s[3 * i], s[3 * i + 1], s[3 * i + 2]});
+            p *= (Polynomial::eq(u_now) * eq_accumulate);
+            if (p(0) + p(1) != claim) throw std::runtime_error("matmul_phase1: claim != p(0) + p(1)");
+            eq_accumulate *= Polynomial::eq(u_now, v_now);
+        } else {
+            p = Polynomial({s[3 * i] * eq_accumulate, s[3 * i + 1] * eq_accumulate, s[3 * i + 2] * eq_accumulate});
+            if (p(0) + p(1) != claim) throw std::runtime_error("matmul_phase2: claim != p(0) + p(1)");
+        }
+        claim = p(v_now);
+        record(transcript, p, claim);
+    }
+    return {s[3 * (size_t)rounds], s[3 * (size_t)rounds + 1]};
+}
 std::pair<Fr, Fr> prove_matmul_impl(Operand A_op, Operand B_op, int L, int N, int M, int K, const std::vector<Fr>& u, const std::vector<Fr>& v,
                                     Fr& claim, SumcheckTranscript* transcript) {
     // The point u is read as log2(M) variables of the column index, log2(N) of the row index and log2(L)
@@ -176,13 +222,18 @@ std::pair<Fr, Fr> prove_matmul_impl(Operand A_op, Operand B_op, int L, int N, in
     try {
         FrTensor& A = A_op.fold((uint)(L * N * K), U, N, Log2(M), K);
         FrTensor& B = B_op.fold((uint)(L * M * K), U, M, 0, K);
-        FrTensor a(1), b(1), c(1);      // the reference's coefficient arrays (src/prove.cu:190-192): not used by the fused rounds
-        Fr eq_accumulate = matmul_sumcheck_phase1(A, B, a, b, c, U + Log2(L * N * M), V + Log2(L * K), K, K * L, claim, transcript);
-        matmul_sumcheck_phase2(A, B, a, b, c, V + Log2(K), K, claim, eq_accumulate, transcript);
-        Fr A_claim = grape_host::download(A.gpu_data);
-        Fr B_claim = grape_host::download(B.gpu_data);
-        if (A_claim * B_claim * eq_accumulate != claim) throw std::runtime_error("prove_matmul: A(v) * B(v) * eq != claim");
-        ret = {A_claim, B_claim};
+        Fr eq_accumulate;
+        if ((uint)(L * K) >= 2 && (uint)(L * K) <= GRAPE_SHORT_MAX && (L & (L - 1)) == 0) {
+            ret = matmul_short_rounds(A, B, L, K, u.data() + Log2(L * N * M), v.data() + Log2(L * K), U + Log2(L * N * M), V + Log2(L * K), claim,
+                                      eq_accumulate, transcript);
+        } else {
+            FrTensor a(1), b(1), c(1);      // the reference's coefficient arrays (src/prove.cu:190-192): not used by the fused rounds
+            eq_accumulate = matmul_sumcheck_phase1(A, B, a, b, c, U + Log2(L * N * M), V + Log2(L * K), K, K * L, claim, transcript);
+            matmul_sumcheck_phase2(A, B, a, b, c, V + Log2(K), K, claim, eq_accumulate, transcript);
+            ret.first = grape_host::download(A.gpu_data);
+            ret.second = grape_host::download(B.gpu_data);
+        }
+        if (ret.first * ret.second * eq_accumulate != claim) throw std::runtime_error("prove_matmul: A(v) * B(v) * eq != claim");
     } catch (...) {
         grape_free_on_default(V);
         grape_free_on_default(U);
@@ -225,32 +276,64 @@ std::pair<Fr, Fr> prove_matmul(const int* device_int_A, const int* device_int_B,
 // eq(u_low, x) from a pyramid of tables built once - on rows padded to a power of two, which is
 // where the variables of u live.
 // A and B are read by the first round, every round leaves its folded halves in Aw and Bw (A and B themselves, or
-// buffers of size / 2 elements where the operands are kept).
-static Fr eleMul_rounds(fr_t* Aw, fr_t* Bw, const fr_t* A, const fr_t* B, fr_t* u, fr_t* v, uint first_size, uint size, Fr& claim,
-                        SumcheckTranscript* transcript) {
+// buffers of size / 2 elements where the operands are kept).  u and v (device) point behind the variables, as do hu and hv (host; where
+// the caller has no host copy they are downloaded).  The elements that are left go to claims where that is given.
+static Fr eleMul_rounds(fr_t* Aw, fr_t* Bw, const fr_t* A, const fr_t* B, fr_t* u, fr_t* v, const Fr* hu, const Fr* hv, uint first_size, uint size,
+                        Fr& claim, std::pair<Fr, Fr>* claims, SumcheckTranscript* transcript) {
     if ((1u << Log2(first_size)) != first_size) throw std::runtime_error("eleMul_sumcheck: first_size is illegal");
     const uint second_size = size / first_size;
     const uint rounds = Log2(size);
     Fr eq_accumulate = Fr::one();
-    if (rounds == 0) return eq_accumulate;
+    if (rounds == 0) {
+        if (claims) *claims = {grape_host::download(A), grape_host::download(B)};
+        return eq_accumulate;
+    }
     const uint row_pad = 1u << Log2(second_size);
-    const std::vector<Fr> us = download_vec(u - rounds, rounds), vs = download_vec(v - rounds, rounds);
+    std::vector<Fr> us, vs;
+    if (!hu) {
+        us = download_vec(u - rounds, rounds);
+        vs = download_vec(v - rounds, rounds);
+        hu = us.data() + rounds;
+        hv = vs.data() + rounds;
+    }
     EqPyramid eq(u - rounds, rounds - 1);
-    FrTensor sums(3 * rounds);
+    FrTensor sums(3 * rounds + 2);
     uint in = size, out = size / 2;
     for (uint i = 0; i < rounds; i++) {
+        const fr_t *Ai = i ? Aw : A, *Bi = i ? Bw : B;
+        // short rounds in one call; a single row that is no power of two has no defined first round and is refused below
+        if (in <= GRAPE_SHORT_MAX && out < (1u << 16) && ((in & (in - 1)) == 0 || (first_size > 1 && in % second_size == 0))) {
+            grape_short_rounds_args a{};
+            a.kind = GRAPE_SHORT_PAIR;
+            a.weights = GRAPE_SHORT_FULL;
+            a.size = in;
+            a.row = in < second_size ? in : second_size;
+            a.x[0] = W(Ai);
+            a.x[1] = W(Bi);
+            a.v_end = W(v - i);
+            a.pyramid = W(eq.level(0));
+            a.top_level = rounds - 1 - i;
+            a.sums = W(sums.gpu_data + 3 * i);
+            a.stride = 3;
+            a.last[0] = W(Aw);
+            a.last[1] = W(Bw);
+            a.last_copy[0] = W(sums.gpu_data + 3 * rounds);
+            a.last_copy[1] = W(sums.gpu_data + 3 * rounds + 1);
+            check(grape_short_rounds(&a, nullptr), "grape_short_rounds");
+            break;
+        }
         // while whole rows are paired the weights are addressed on padded rows
         const bool rows = in > second_size && second_size != row_pad;
-        check(grape_wround2_from(W(Aw), W(Bw), i ? W(Aw) : W(A), i ? W(Bw) : W(B), W(eq.level(rounds - 1 - i)), in, out, rows ? second_size : 1,
+        check(grape_wround2_from(W(Aw), W(Bw), W(Ai), W(Bi), W(eq.level(rounds - 1 - i)), in, out, rows ? second_size : 1,
                                  rows ? row_pad : 1, W(v - i - 1), W(sums.gpu_data + 3 * i), nullptr),
               "grape_wround2_from");
         in = out;
         out = out == second_size ? (1u << (Log2(out) - 1)) : out / 2;
         if (out == 0) out = 1;
     }
-    const std::vector<Fr> s = download_vec(sums.gpu_data, 3 * (size_t)rounds);
+    const std::vector<Fr> s = download_vec(sums.gpu_data, 3 * (size_t)rounds + 2);
     for (uint i = 0; i < rounds; i++) {
-        const Fr &u_now = us[rounds - 1 - i], &v_now = vs[rounds - 1 - i];
+        const Fr &u_now = *(hu - 1 - i), &v_now = *(hv - 1 - i);
         Polynomial p({s[3 * i], s[3 * i + 1], s[3 * i + 2]});
         p *= (Polynomial::eq(u_now) * eq_accumulate);
         if (p(0) + p(1) != claim) throw std::runtime_error("ele_Mul: claim != p(0) + p(1)");
@@ -258,6 +341,7 @@ static Fr eleMul_rounds(fr_t* Aw, fr_t* Bw, const fr_t* A, const fr_t* B, fr_t* 
         record(transcript, p, claim);
         eq_accumulate *= Polynomial::eq(u_now, v_now);
     }
+    if (claims) *claims = {s[3 * (size_t)rounds], s[3 * (size_t)rounds + 1]};
     return eq_accumulate;
 }
 
@@ -266,7 +350,7 @@ Fr eleMul_sumcheck(FrTensor& A, FrTensor& B, FrTensor& a, FrTensor& b, FrTensor&
     (void)a;
     (void)b;
     (void)c;
-    return eleMul_rounds(A.gpu_data, B.gpu_data, A.gpu_data, B.gpu_data, u, v, first_size, size, claim, transcript);
+    return eleMul_rounds(A.gpu_data, B.gpu_data, A.gpu_data, B.gpu_data, u, v, nullptr, nullptr, first_size, size, claim, nullptr, transcript);
 }
 
 static std::pair<Fr, Fr> prove_eleMul_impl(fr_t* Aw, fr_t* Bw, const fr_t* A, const fr_t* B, int L, int M, int N, const std::vector<Fr>& u,
@@ -276,11 +360,10 @@ static std::pair<Fr, Fr> prove_eleMul_impl(fr_t* Aw, fr_t* Bw, const fr_t* A, co
     std::pair<Fr, Fr> ret;
     try {
         const uint size = (uint)(L * M * N);
-        Fr eq_accumulate = eleMul_rounds(Aw, Bw, A, B, U + Log2(size), V + Log2(size), (uint)(L * M), size, claim, transcript);
-        Fr A_claim = grape_host::download(size == 1 ? A : Aw);
-        Fr B_claim = grape_host::download(size == 1 ? B : Bw);
-        if (A_claim * B_claim * eq_accumulate != claim) throw std::runtime_error("prove_eleMul: A(v) * B(v) * eq != claim");
-        ret = {A_claim, B_claim};
+        const uint lg = Log2(size);
+        if (u.size() < lg || v.size() < lg) throw std::runtime_error("prove_eleMul: the point has too few variables");
+        Fr eq_accumulate = eleMul_rounds(Aw, Bw, A, B, U + lg, V + lg, u.data() + lg, v.data() + lg, (uint)(L * M), size, claim, &ret, transcript);
+        if (ret.first * ret.second * eq_accumulate != claim) throw std::runtime_error("prove_eleMul: A(v) * B(v) * eq != claim");
     } catch (...) {
         grape_free_on_default(V);
         grape_free_on_default(U);

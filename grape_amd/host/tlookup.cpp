@@ -468,8 +468,15 @@ Fr tLookup::run(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax& hyrax
     fr_t* d_v = grape_host::upload(v);
     Fr S_last;
     char* long_work = nullptr;             // partial sums of the long rounds and the challenges' tables (overlap mode)
-    FrTensor Bw(B), Tw(T), mw(N);          // phase 2 binds copies; T, B, m of this object stay intact
-    if (!m_late) check(grape_memcpy_d2d(mw.gpu_data, m.gpu_data, sizeof(fr_t) * (size_t)N, nullptr), "grape_memcpy_d2d");
+    // phase 2 binds copies where its rounds work in place; T, B, m of this object stay intact
+    const bool table_long = N / 2 >= kLongRoundPairs;
+    FrTensor Bw(table_long ? N : 1), Tw(table_long ? N : 1), mw(table_long ? N : 1);
+    auto copy_table = [&](FrTensor& to, const FrTensor& from, grape_stream_t st) {
+        if (table_long) check(grape_memcpy_d2d(to.gpu_data, from.gpu_data, sizeof(fr_t) * (size_t)N, st), "grape_memcpy_d2d");
+    };
+    copy_table(Bw, B, nullptr);
+    copy_table(Tw, T, nullptr);
+    if (!m_late) copy_table(mw, m, nullptr);
     try {
         // The table side of phase 2 (B, T, m: sums and folds of the last log2(N) rounds) depends on
         // nothing the witness side produces, so it runs as a chain of its own on a second stream,
@@ -524,6 +531,19 @@ Fr tLookup::run(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax& hyrax
             vi--;
             k++;
         };
+        // all rounds from round `first` on, over tensors of `size` elements
+        auto short_args = [&](uint32_t kind, uint first, uint size) {
+            grape_short_rounds_args a{};
+            a.kind = kind;
+            a.weights = GRAPE_SHORT_FULL;
+            a.size = a.row = size;
+            a.beta = W(d_beta);
+            a.v_end = W(d_v + (rounds - first));
+            a.pyramid = W(E.gpu_data);
+            a.top_level = nu - 1 - first;
+            a.stride = 13;
+            return a;
+        };
         // the table side of phase 2: per round one launch for the five sums over (B, T), the three over
         // (m, B) and the fold of all three, and one finishing launch
         auto table_side = [&] {
@@ -531,6 +551,14 @@ Fr tLookup::run(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax& hyrax
             for (int vt = (int)logN - 1; vt >= 0 && vt < (int)rounds; vt--) {
                 const uint kt = rounds - 1 - (uint)vt;
                 const uint half = cur_t / 2;
+                if (half < kLongRoundPairs) {
+                    grape_short_rounds_args a = short_args(GRAPE_SHORT_TABLE, kt, cur_t);
+                    const FrTensor *const own[3] = {&B, &T, &m}, *const work[3] = {&Bw, &Tw, &mw};
+                    for (int i = 0; i < 3; i++) a.x[i] = W((table_long ? work[i] : own[i])->gpu_data);
+                    a.sums = W(sums.gpu_data + 13 * (size_t)kt + 5);
+                    check(grape_short_rounds(&a, side.stream), "grape_short_rounds");
+                    break;
+                }
                 fr_t* slot = sums.gpu_data + 13 * (size_t)kt;
                 const fr_t* e = E.gpu_data + (((size_t)1 << (nu - 1 - kt)) - 1);
                 check(grape_tlookup_table_round(W(Bw.gpu_data), W(Tw.gpu_data), W(mw.gpu_data), W(d_beta), W(e), half, W(d_v + vt),
@@ -568,7 +596,7 @@ Fr tLookup::run(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax& hyrax
                 index_to_m(m_pending_size_, m_pending_low_, side.stream);
                 check(grape_fr_mul(W(Bm.gpu_data), W(Bm.gpu_data), W(m.gpu_data), N, side.stream), "grape_fr_mul");
                 check(grape_fr_sum(W(d_sum_Bm), W(Bm.gpu_data), N, side.stream), "grape_fr_sum");
-                check(grape_memcpy_d2d(mw.gpu_data, m.gpu_data, sizeof(fr_t) * (size_t)N, side.stream), "grape_memcpy_d2d");
+                copy_table(mw, m, side.stream);
             }
             table_side();
             const uint m_N = 1u << (Log2(N) / 2);
@@ -590,8 +618,19 @@ Fr tLookup::run(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax& hyrax
             });
             check(grape_event_record(commit_events().second, nullptr), "grape_event_record");
         }
-        while (vi >= 0) witness_round(ws);
-        check(grape_memcpy_d2d(d_S_last, S.gpu_data, sizeof(fr_t), ws), "grape_memcpy_d2d");   // S(v), behind the last round
+        while (vi >= 0 && cur / 2 >= kLongRoundPairs) witness_round(ws);
+        if (vi >= 0) {
+            grape_short_rounds_args a = short_args(GRAPE_SHORT_LOGUP, k, cur);
+            a.x[0] = a.last[0] = W(A.gpu_data);
+            a.x[1] = a.last[1] = W(S.gpu_data);
+            a.last_copy[1] = W(d_S_last);                      // S(v)
+            a.sums = W(sums.gpu_data + 13 * (size_t)k);
+            check(grape_short_rounds(&a, ws), "grape_short_rounds");
+            A.set_size(1);
+            S.set_size(1);
+        } else {
+            check(grape_memcpy_d2d(d_S_last, S.gpu_data, sizeof(fr_t), ws), "grape_memcpy_d2d");
+        }
         // without the overlap the table side is queued last: its small launches reach the chip while it
         // works on the first, long rounds of the witness side
         if (!overlap) table_side();

@@ -196,6 +196,29 @@ def sumcheck_round2_tail(A, B, in_size, rounds, v, v_end_index):
     return sums
 
 
+class _ShortRounds(ctypes.Structure):
+    _fields_ = [("kind", ctypes.c_uint32), ("weights", ctypes.c_uint32), ("size", ctypes.c_uint32), ("row", ctypes.c_uint32),
+                ("x", ctypes.c_void_p * 3), ("beta", ctypes.c_void_p), ("v_end", ctypes.c_void_p), ("pyramid", ctypes.c_void_p),
+                ("top_level", ctypes.c_uint32), ("stride", ctypes.c_uint32), ("sums", ctypes.c_void_p),
+                ("last", ctypes.c_void_p * 3), ("last_copy", ctypes.c_void_p * 3)]
+
+
+def short_rounds(kind, x, size, row, v, pyramid=None, top_level=0, beta=None, weights=0):
+    """all rounds left of a sumcheck over 2 to 2^17 elements (kind 0: pair, 1: logUp, 2: table side); challenges from the
+    end of v.  Returns the sums, one row of elements per round, and the elements left of the tensors."""
+    lib = init()
+    nv = (3, 5, 8)[kind]
+    rounds = (size // row - 1).bit_length() + (row - 1).bit_length()
+    sums, last = fr_empty(rounds * nv), fr_empty(len(x))
+    a = _ShortRounds(kind=kind, weights=weights, size=size, row=row, beta=beta.data_ptr() if beta is not None else None,
+                     v_end=v.data_ptr() + 32 * v.shape[0], pyramid=pyramid.data_ptr() if pyramid is not None else None,
+                     top_level=top_level, stride=nv, sums=sums.data_ptr())
+    for k, t in enumerate(x):
+        a.x[k], a.last[k] = t.data_ptr(), last.data_ptr() + 32 * k
+    _capi.check(lib.grape_short_rounds(ctypes.byref(a), _s()))
+    return sums.view(rounds, nv, 8), last
+
+
 def sumcheck_round2_coeffs(A, B, a, b, c, in_size, out_size, v, want_sums=True):
     lib = init()
     sums = fr_empty(3) if want_sums else None

@@ -377,6 +377,28 @@ int grape_tlookup_mb_sums(const uint32_t *d_m, const uint32_t *d_B, size_t n_out
  */
 int grape_tlookup_table_round(uint32_t *d_B, uint32_t *d_T, uint32_t *d_m, const uint32_t *d_beta, const uint32_t *d_eq,
                               size_t n_out, const uint32_t *d_v, uint32_t *d_sums, grape_stream_t stream);
+/*
+ * All rounds that are left of a sumcheck over 2 to 2^17 elements: round t binds the top remaining variable to
+ * d_v_end[-(t+1)] and leaves its sums at element t * stride of d_sums.  The tensors are read and not changed; the
+ * element that is left of tensor k goes to last[k] and last_copy[k] where those are given.
+ *   GRAPE_SHORT_PAIR    x = (A, B), 3 sums as grape_wround2(plain_sums = 0) resp. grape_sumcheck_round2[_seg]
+ *   GRAPE_SHORT_LOGUP   x = (A, S), 5 sums as grape_wround2(plain_sums = 1) with the shift beta
+ *   GRAPE_SHORT_TABLE   x = (B, T, m), 8 sums as grape_tlookup_table_round
+ * `size` elements in rows of `row` (a power of two of them): whole rows are paired until one is left, and that one is
+ * taken as padded with zeros to a power of two.  Weights of round t: none; every index (level top_level - t of an eq
+ * pyramid, on rows padded to a power of two); or every row while more than one is left, none after.
+ */
+enum { GRAPE_SHORT_PAIR = 0, GRAPE_SHORT_LOGUP = 1, GRAPE_SHORT_TABLE = 2 };
+enum { GRAPE_SHORT_NONE = 0, GRAPE_SHORT_FULL = 1, GRAPE_SHORT_ROWS = 2 };
+#define GRAPE_SHORT_MAX 131072u
+struct grape_short_rounds_args {
+    uint32_t kind, weights, size, row;
+    const uint32_t *x[3];
+    const uint32_t *beta, *v_end, *pyramid;
+    uint32_t top_level, stride;
+    uint32_t *sums, *last[3], *last_copy[3];
+};
+int grape_short_rounds(const struct grape_short_rounds_args *rounds, grape_stream_t stream);
 /* e[i] = prod_j (u_j if bit_j(i) else 1 - u_j) for i < 2^nu; u is a device array of nu challenges. */
 int grape_eq_table(uint32_t *d_eq, const uint32_t *d_u, uint32_t nu, grape_stream_t stream);
 /* e'[x] = e[x] + e[x + n_out] for x < n_out: the table of the remaining variables after the
