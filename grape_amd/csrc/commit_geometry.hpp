@@ -48,6 +48,22 @@ GRAPE_HD WidePlan wide_plan(size_t size, uint32_t rowlen, size_t slab_segments) 
     return p;
 }
 
+// Windows of full-width scalars over several waves: a call with few rows runs one wave per SIMD or less, each lane a chain of
+// one addition (10 us) per window.  Up to 1024 waves take shares of the windows, the partial sums they leave more
+// cost the row reduction a level of groups (one row of 4096 with 20 windows: 354 -> 232 us; 16 rows
+// 386 -> 377; one row of 256 with 15 windows 289 -> 139, 64 rows 301 -> 163).  With 1024 waves and more the chip is busy and nothing is split.
+struct WindowSplit {
+    uint32_t parts, per;    // shares per (row, segment) and windows in each
+};
+GRAPE_HD WindowSplit window_split(size_t waves, uint32_t nwin) {
+    const size_t room = waves ? 1024 / waves : 1;
+    WindowSplit w;
+    w.parts = room < 1 ? 1 : room < nwin ? (uint32_t)room : nwin;
+    w.per = (nwin + w.parts - 1) / w.parts;
+    w.parts = (nwin + w.per - 1) / w.per;
+    return w;
+}
+
 // what wave `wave` of a launch over `rows` rows works on
 struct WaveSpan {
     size_t row;
@@ -79,28 +95,32 @@ GRAPE_HD uint32_t quad_share(int lane, uint32_t lg_qpr) { return (uint32_t)(lane
 //     at 8192 rows quads alone are as fast (209 against 199) and one launch less;
 //   - up to 512 rows of more than 64 partial sums: quads in groups of 64 first, so that the chain stays at 7 additions
 //     (512 rows of 512: 196 against 243; 64 of 4096: 223 against 1430; 1024 rows of 256: 190 against 162, so not there);
+//     and again in groups of 16 where that leaves more than 64 (rows whose windows were split);
 //   - quads per row: as many as a wave holds while rows * quads stays below 2^15, i.e. two waves per SIMD (2048 rows
 //     of 128: 154 with 16, 151 with 8, 232 with 4; 8192 of 64: 285, 225, 209 with 16, 8, 4).
 constexpr uint32_t kQuadsPerWaveLog2 = 4;
 constexpr uint32_t kReduceGroup = 64;      // partial sums of a group
+constexpr uint32_t kReduceGroup2 = 16;     // and of a group of groups
 constexpr uint32_t kReduceKeep = 8;        // partial sums per row that the lane kernel leaves
 struct ReducePlan {
     bool lanes;             // first stage by commit_reduce_lane_kernel
     uint32_t left;          // partial sums per row after the first stage (nparts when there is none)
+    uint32_t left2;         // and after the second (left when there is none)
     uint32_t lg_qpr;        // log2 of the quads per row in the last stage
 };
 GRAPE_HD ReducePlan reduce_plan(size_t rows, uint32_t nparts) {
     ReducePlan p;
     p.lanes = rows > 8192 && nparts > kReduceKeep;
     p.left = p.lanes ? kReduceKeep : (rows <= 512 && nparts > kReduceGroup && nparts % kReduceGroup == 0) ? nparts / kReduceGroup : nparts;
+    p.left2 = !p.lanes && p.left < nparts && p.left > kReduceGroup && p.left % kReduceGroup2 == 0 ? p.left / kReduceGroup2 : p.left;
     p.lg_qpr = 0;
-    while (p.lg_qpr < kQuadsPerWaveLog2 && (2u << p.lg_qpr) <= p.left && (rows << (p.lg_qpr + 1)) <= 32768) p.lg_qpr++;
+    while (p.lg_qpr < kQuadsPerWaveLog2 && (2u << p.lg_qpr) <= p.left2 && (rows << (p.lg_qpr + 1)) <= 32768) p.lg_qpr++;
     if (p.lanes) p.lg_qpr = 1;
     return p;
 }
-// accumulators of work space for at most `rows` rows: what the first stage leaves, and the row sums
+// accumulators of work space for at most `rows` rows: what the first two stages leave, and the row sums
 GRAPE_HD size_t reduce_tmp_accumulators(size_t rows, uint32_t nparts) {
-    const size_t grouped = (rows < 512 ? rows : 512) * (size_t)(nparts / kReduceGroup), kept = rows > 8192 ? rows * kReduceKeep : 0;
+    const size_t groups = nparts / kReduceGroup, grouped = (rows < 512 ? rows : 512) * (groups + groups / kReduceGroup2), kept = rows > 8192 ? rows * kReduceKeep : 0;
     return rows + (grouped > kept ? grouped : kept);
 }
 

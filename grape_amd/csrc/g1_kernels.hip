@@ -212,9 +212,9 @@ __device__ __forceinline__ uint32_t fr_digit(const Fr& k, uint32_t w, uint32_t c
 
 // acc += k * G_col through the wide table: one gather and one mixed addition per non-zero digit.
 // While the addition of digit w runs, the table line of digit w+1 is already on its way (one
-// word of it is touched right after the entry of digit w has been requested).
+// word of it is touched right after the entry of digit w has been requested).  Only the digits w0 .. w1 - 1 are added.
 __device__ __forceinline__ void madd_scalar_fr(Xyzz28& acc, const Fr& k_in, const uint32_t* table, size_t N, uint32_t col,
-                                               uint32_t c, uint32_t nw, uint32_t K, int* err_flag) {
+                                               uint32_t c, uint32_t nw, uint32_t K, int* err_flag, uint32_t w0 = 0, uint32_t w1 = ~0u) {
     // The scalar is taken as +-|k| with |k| <= (r-1)/2 < 2^254 (r - k and the negated point when k is
     // in the upper half): the top window then never carries out, and nw = ceil(255/c) windows are
     // enough - one addition fewer per scalar at c = 15.
@@ -230,13 +230,16 @@ __device__ __forceinline__ void madd_scalar_fr(Xyzz28& acc, const Fr& k_in, cons
     k = cneg(k, flip);
     uint32_t nwin = nw;
     while (nwin > 0 && (nwin - 1) * c >= 256) nwin--;     // windows that start inside the scalar
+    const uint32_t end = w1 < nwin ? w1 : nwin;
     uint32_t carry = 0;
     bool neg = false;
-    uint32_t mag = nwin ? fr_digit(k, 0, c, carry, neg) : 0;
+    for (uint32_t w = 0; w < w0 && w < end; w++) (void)fr_digit(k, w, c, carry, neg);
+    neg = false;
+    uint32_t mag = w0 < end ? fr_digit(k, w0, c, carry, neg) : 0;
     uint32_t touch = 0;
-    for (uint32_t w = 0; w < nwin; w++) {
+    for (uint32_t w = w0; w < end; w++) {
         bool neg_n = false;
-        const uint32_t mag_n = (w + 1 < nwin) ? fr_digit(k, w + 1, c, carry, neg_n) : 0;
+        const uint32_t mag_n = (w + 1 < end) ? fr_digit(k, w + 1, c, carry, neg_n) : 0;
         if (mag != 0) {
             if (mag > K) {
                 *err_flag = 1;
@@ -253,7 +256,7 @@ __device__ __forceinline__ void madd_scalar_fr(Xyzz28& acc, const Fr& k_in, cons
         neg = neg_n;
     }
     asm volatile("" ::"v"(touch));      // keeps the last touch alive until here
-    if (carry) *err_flag = 1;   // cannot happen for canonical scalars when nw*c >= 255
+    if (carry && end == nwin) *err_flag = 1;   // cannot happen for canonical scalars when nw*c >= 255
 }
 
 __device__ __forceinline__ G1Xyzz shfl_down_xyzz(const G1Xyzz& a, int off) {
@@ -512,15 +515,19 @@ __global__ void __launch_bounds__(kBlock) ref_from_wide_kernel(uint32_t* out, co
 // commitment, wide table
 // ------------------------------------------------------------------------------------------------
 // Each wave owns one row segment of `seg` columns; lane l takes columns l, l+64, ...
-// partial[(row*nseg + s)*64 + lane] receives the lane's XYZZ accumulator.
+// partial[(row*nseg + s)*64 + lane] receives the lane's XYZZ accumulator; full-width scalars of few rows go over split.parts
+// waves per segment (geom::window_split), partial[((row*nseg + s)*parts + part)*64 + lane].
 template <bool FR>
 __global__ void __launch_bounds__(kBlock) commit_wide_kernel(uint32_t* partial, const void* scalars, uint32_t rowlen, size_t rows,
                                                              uint32_t seg, uint32_t nseg, const uint32_t* table, size_t N,
-                                                             uint32_t c, uint32_t nw, uint32_t K, int* err_flag) {
+                                                             uint32_t c, uint32_t nw, uint32_t K, int* err_flag, geom::WindowSplit split) {
     const int lane = threadIdx.x & 63;
     const size_t wave = ((size_t)blockIdx.x * kBlock + threadIdx.x) >> 6;
-    if (wave >= rows * nseg) return;
-    const geom::WaveSpan span = geom::wave_span(wave, nseg, seg, rowlen);
+    const uint32_t parts = FR ? split.parts : 1;
+    if (wave >= rows * nseg * parts) return;
+    const size_t unit = FR ? wave / parts : wave;
+    const uint32_t w0 = (uint32_t)(wave - unit * parts) * split.per;
+    const geom::WaveSpan span = geom::wave_span(unit, nseg, seg, rowlen);
     const size_t row = span.row;
     const uint32_t s = span.s, col_end = span.col_end;
     const uint32_t half = 1u << (c - 1), mask = (c == 32) ? 0xffffffffu : ((1u << c) - 1u);
@@ -541,7 +548,7 @@ __global__ void __launch_bounds__(kBlock) commit_wide_kernel(uint32_t* partial, 
     for (uint32_t col = s * seg + lane; col < col_end; col += 64) {
         if (FR) {
             const Fr k = from_mont(ld_fr8((const uint32_t*)scalars, geom::scalar_index(row, rowlen, col)));
-            madd_scalar_fr(acc, k, table, N, col, c, nw, K, err_flag);
+            madd_scalar_fr(acc, k, table, N, col, c, nw, K, err_flag, w0, w0 + split.per);
         } else {
             int64_t v = sc0;
             const int64_t v_next = sc1;
@@ -699,17 +706,17 @@ __device__ __forceinline__ int32_t digit_of(const Fr& kb, uint32_t w, uint32_t c
     return (w * c + c - 1 < 256) ? bits - (int32_t)(1u << (c - 1)) : bits;
 }
 
-// acc += the windows j, J + j, 2J + j, ... of k * G_col
+// acc += the windows q J + j, q0 <= q < q1, of k * G_col
 __device__ __forceinline__ void madd_scalar_strided(Xyzz28& acc, const Fr& k_mont, const Fr& H, const uint32_t* table, size_t N, uint32_t col, uint32_t c,
-                                                    uint32_t nw, uint32_t K, uint32_t J, uint32_t nsets, uint32_t j) {
+                                                    uint32_t nw, uint32_t K, uint32_t J, uint32_t j, uint32_t q0, uint32_t q1) {
     bool flip;
     const Fr kb = biased_half_range(k_mont, H, flip);
-    // digit of set 0 now, the next set's one addition ahead (its table line is touched early)
-    int32_t d = j < nw ? digit_of(kb, j, c) : 0;
+    // digit of set q0 now, the next set's one addition ahead (its table line is touched early)
+    int32_t d = q0 * J + j < nw ? digit_of(kb, q0 * J + j, c) : 0;
     uint32_t touch = 0;
-    for (uint32_t q = 0; q < nsets; q++) {
+    for (uint32_t q = q0; q < q1; q++) {
         const uint32_t wn = (q + 1) * J + j;
-        const int32_t d_n = (q + 1 < nsets && wn < nw) ? digit_of(kb, wn, c) : 0;
+        const int32_t d_n = (q + 1 < q1 && wn < nw) ? digit_of(kb, wn, c) : 0;
         if (d != 0) {
             const bool neg = d < 0;
             const uint32_t mag = (uint32_t)(neg ? -d : d);
@@ -727,30 +734,21 @@ __device__ __forceinline__ void madd_scalar_strided(Xyzz28& acc, const Fr& k_mon
 
 __global__ void __launch_bounds__(kBlock) commit_strided_kernel(uint32_t* partial, const uint32_t* scalars, uint32_t rowlen, size_t rows,
                                                                 uint32_t seg, uint32_t nseg, const uint32_t* table, size_t N,
-                                                                uint32_t c, uint32_t nw, uint32_t K, uint32_t J, uint32_t nsets) {
+                                                                uint32_t c, uint32_t nw, uint32_t K, uint32_t J, uint32_t nsets,
+                                                                geom::WindowSplit split) {
     const int lane = threadIdx.x & 63;
     const size_t wave = ((size_t)blockIdx.x * kBlock + threadIdx.x) >> 6;
-    if (wave >= rows * J * nseg) return;
-    const geom::WaveSpan span = geom::wave_span(wave, nseg, seg, rowlen);   // "row" here is (row, residue)
+    if (wave >= rows * J * nseg * split.parts) return;
+    const size_t unit = wave / split.parts;
+    const uint32_t q0 = (uint32_t)(wave - unit * split.parts) * split.per, q1 = q0 + split.per < nsets ? q0 + split.per : nsets;
+    const geom::WaveSpan span = geom::wave_span(unit, nseg, seg, rowlen);   // "row" here is (row, residue)
     const size_t row = span.row / J;
     const uint32_t j = (uint32_t)(span.row - row * J);
     const Fr H = window_bias(c, nw);                      // wave-uniform
     Xyzz28 acc = xyzz28_inf();
     for (uint32_t col = span.s * seg + lane; col < span.col_end; col += 64)
-        madd_scalar_strided(acc, ld_fr8(scalars, geom::scalar_index(row, rowlen, col)), H, table, N, col, c, nw, K, J, nsets, j);
+        madd_scalar_strided(acc, ld_fr8(scalars, geom::scalar_index(row, rowlen, col)), H, table, N, col, c, nw, K, J, j, q0, q1);
     st_partial28(partial, wave * 64 + lane, acc);
-}
-
-// total_row = sum_j 2^(c j) A[row * J + j] by Horner from the top residue down, then affine
-__global__ void __launch_bounds__(64) strided_horner_kernel(uint32_t* out, const uint32_t* sums, size_t rows, uint32_t J, uint32_t c) {
-    const size_t row = (size_t)blockIdx.x * 64 + threadIdx.x;
-    if (row >= rows) return;
-    Xyzz28 total = ld_partial28(sums, row * J + (J - 1));
-    for (int j = (int)J - 2; j >= 0; j--) {
-        for (uint32_t d = 0; d < c; d++) xyzz28_dbl(total);
-        padd28(total, ld_partial28(sums, row * J + j));
-    }
-    st_affine(out, row, xyzz28_to_affine(total));
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -836,7 +834,7 @@ __global__ void __launch_bounds__(64) commit_sparse_strided_kernel(uint32_t* par
             const uint32_t n = qn < 64 ? qn : 64;
             if ((uint32_t)lane < n) {
                 const uint32_t col = queue[lane];
-                madd_scalar_strided(acc, ld_fr8(scalars, geom::scalar_index(row, rowlen, col)), H, table, N, col, c, nw, K, J, nsets, j);
+                madd_scalar_strided(acc, ld_fr8(scalars, geom::scalar_index(row, rowlen, col)), H, table, N, col, c, nw, K, J, j, 0, nsets);
             }
             __syncthreads();
             const uint32_t moved = (uint32_t)lane + 64 < qn ? queue[lane + 64] : 0u;
@@ -918,6 +916,21 @@ __global__ void __launch_bounds__(kBlock) quad_affine_kernel(uint32_t* out, cons
     const Fp c = quad::to_affine(ld_quad_partial(sums, row));
     const uint32_t r = threadIdx.x & 3;
     if (r < 2) st_fp(out + 2 * FW * row + FW * r, c);
+}
+// out[row] = sum_j 2^(c j) A[row * J + j] by Horner from the top residue or window down, then affine: a chain of (J - 1) c
+// doublings, so a quad per row (three products' time a doubling, where one lane runs nine products.
+// One row of 32 byte windows, 248 doublings: 6.6 -> 1.1 ms; four residues of 16 bits, 48 doublings: 0.54 -> 0.26 ms).
+__global__ void __launch_bounds__(64) quad_horner_kernel(uint32_t* out, const uint32_t* sums, size_t rows, uint32_t J, uint32_t c) {
+    const size_t row = ((size_t)blockIdx.x * 64 + threadIdx.x) >> 2;
+    if (row >= rows) return;
+    quad::Acc total = ld_quad_partial(sums, row * J + (J - 1));
+    for (int j = (int)J - 2; j >= 0; j--) {
+        for (uint32_t d = 0; d < c; d++) quad::dbl(total);
+        quad::add(total, ld_quad_partial(sums, row * J + j));
+    }
+    const Fp v = quad::to_affine(total);
+    const uint32_t r = threadIdx.x & 3;
+    if (r < 2) st_fp(out + 2 * FW * row + FW * r, v);
 }
 // out[row * keep + k] = the sum of the row's partial sums k, k + keep, ...
 __global__ void __launch_bounds__(kBlock) commit_reduce_lane_kernel(uint32_t* out, const uint32_t* partial, size_t rows, uint32_t nparts, uint32_t keep) {
@@ -1054,18 +1067,6 @@ __global__ void __launch_bounds__(kBlock, 2) commit_ref28_kernel(uint32_t* parti
     st_partial28(partial, unit * 64 + lane, acc);
 }
 
-// total = sum_w 2^(8 w) * sums[row * nwin + w]: one thread per row
-__global__ void __launch_bounds__(64) commit_ref_horner_kernel(uint32_t* out, const uint32_t* sums, size_t rows, uint32_t nwin) {
-    const size_t row = (size_t)blockIdx.x * 64 + threadIdx.x;
-    if (row >= rows) return;
-    G1Xyzz total = G1Xyzz::inf();
-    for (int w = (int)nwin - 1; w >= 0; w--) {
-        for (int d = 0; d < 8; d++) pdbl(total);
-        madd(total, ld_affine(sums, row * nwin + w), false);
-    }
-    st_affine(out, row, to_affine(total));
-}
-
 __global__ void __launch_bounds__(64) affine_to_jac_kernel(uint32_t* out, const uint32_t* in, size_t n) {
     size_t i = (size_t)blockIdx.x * 64 + threadIdx.x;
     if (i >= n) return;
@@ -1125,9 +1126,18 @@ static void launch_reduce(uint32_t* out, const uint32_t* partial, size_t rows, u
         commit_reduce_lane_kernel<<<blocks_for(rows * plan.left), kBlock, 0, s>>>(tmp, partial, rows, nparts, plan.left);
     else if (plan.left < nparts)
         quads(tmp, partial, rows * plan.left, nparts / plan.left, geom::kQuadsPerWaveLog2);
-    const uint32_t* const last = plan.left < nparts ? tmp : partial;
-    uint32_t* const sums = AFFINE ? tmp + (last == tmp ? geom::partial_word(rows * plan.left) : 0) : out;
-    quads(sums, last, rows, plan.left, plan.lg_qpr);
+    const uint32_t* last = partial;
+    if (plan.left < nparts) {
+        last = tmp;
+        tmp += geom::partial_word(rows * plan.left);
+    }
+    if (plan.left2 < plan.left) {
+        quads(tmp, last, rows * plan.left2, geom::kReduceGroup2, geom::kQuadsPerWaveLog2);
+        last = tmp;
+        tmp += geom::partial_word(rows * plan.left2);
+    }
+    uint32_t* const sums = AFFINE ? tmp : out;
+    quads(sums, last, rows, plan.left2, plan.lg_qpr);
     if (AFFINE) quad_affine_kernel<<<blocks_for(rows * 4), kBlock, 0, s>>>(out, sums, rows);
 }
 
@@ -1151,9 +1161,12 @@ static int commit_wide_impl(uint32_t* out, const void* scalars, size_t size, uin
     // number of rows (a row segment leaves 64 partial sums of 256 bytes)
     const geom::WidePlan plan = geom::wide_plan(size, rowlen, geom::kSlabSegments);
     const uint32_t nseg = plan.nseg, seg = plan.seg;
-    const size_t slab = plan.slab, partial_bytes = plan.partial_bytes;
+    geom::WindowSplit split = {1, nw};
+    if (FR) split = geom::window_split(rows * nseg, nw);
+    const uint32_t nparts = nseg * split.parts * 64;
+    const size_t slab = plan.slab, partial_bytes = plan.partial_bytes * split.parts;
     void* ws;
-    const size_t tmp_bytes = reduce_tmp_bytes(slab, nseg * 64);
+    const size_t tmp_bytes = reduce_tmp_bytes(slab, nparts);
     int rc = scratch_get(kSlotMsm, partial_bytes + tmp_bytes + 64, &ws, s);
     if (rc) return rc;
     uint32_t* red_tmp = (uint32_t*)((char*)ws + partial_bytes);
@@ -1170,9 +1183,9 @@ static int commit_wide_impl(uint32_t* out, const void* scalars, size_t size, uin
         const size_t nr = rows - r0 < slab ? rows - r0 : slab;
         const uint32_t* sc = (const uint32_t*)scalars + r0 * rowlen * elem_words;
         profile_mark(s);
-        commit_wide_kernel<FR><<<blocks_for(nr * nseg * 64), kBlock, 0, s>>>((uint32_t*)ws, sc, rowlen, nr, seg, nseg, table, N, c, nw, K, err);
+        commit_wide_kernel<FR><<<blocks_for(nr * nparts), kBlock, 0, s>>>((uint32_t*)ws, sc, rowlen, nr, seg, nseg, table, N, c, nw, K, err, split);
         profile_mark(s);
-        launch_reduce<true>(out + r0 * (size_t)(2 * FW), (const uint32_t*)ws, nr, nseg * 64, red_tmp, s);
+        launch_reduce<true>(out + r0 * (size_t)(2 * FW), (const uint32_t*)ws, nr, nparts, red_tmp, s);
         profile_mark(s);
     }
     GRAPE_LAUNCH_CHECK();
@@ -1210,7 +1223,7 @@ static int commit_ref_impl(uint32_t* out, const void* scalars, size_t size, uint
     if (slab > rows) slab = rows;
     const size_t partial_bytes = slab * nwin * nseg * 64 * (size_t)(4 * kPartialWords);
     void* ws;
-    const size_t sums_bytes = (slab * nwin * (size_t)(8 * FW) + 255) & ~(size_t)255;
+    const size_t sums_bytes = slab * nwin * (size_t)(4 * kPartialWords);
     int rc = scratch_get(kSlotMsm, partial_bytes + sums_bytes + reduce_tmp_bytes(slab * nwin, nseg * 64) + 64, &ws, s);
     if (rc) return rc;
     uint32_t* sums = (uint32_t*)((char*)ws + partial_bytes);
@@ -1221,8 +1234,8 @@ static int commit_ref_impl(uint32_t* out, const void* scalars, size_t size, uint
         const size_t units = nr * nwin * nseg;
         const uint32_t* sc = (const uint32_t*)scalars + r0 * rowlen * elem_words;
         commit_ref28_kernel<FR><<<blocks_for(units * 64), kBlock, 0, s>>>((uint32_t*)ws, sc, rowlen, nr, seg, nseg, table, npoints);
-        launch_reduce<true>(sums, (const uint32_t*)ws, nr * nwin, nseg * 64, red_tmp, s);
-        commit_ref_horner_kernel<<<blocks_for(nr, 64), 64, 0, s>>>(out + r0 * (size_t)(2 * FW), sums, nr, nwin);
+        launch_reduce<false>(sums, (const uint32_t*)ws, nr * nwin, nseg * 64, red_tmp, s);
+        quad_horner_kernel<<<blocks_for(nr * 4, 64), 64, 0, s>>>(out + r0 * (size_t)(2 * FW), sums, nr, nwin, 8);
     }
     GRAPE_LAUNCH_CHECK();
     return GRAPE_OK;
@@ -1351,10 +1364,13 @@ static int commit_strided_impl(uint32_t* out, const uint32_t* scalars, const int
     size_t slab = (skip ? geom::kSlabSegments : plan.slab) / J;                              // whole rows per launch
     if (slab < 1) slab = 1;
     if (slab > rows) slab = rows;
-    const size_t partial_bytes = slab * J * nseg * 64 * (size_t)(4 * kPartialWords);
+    geom::WindowSplit split = {1, nsets};
+    if (!skip) split = geom::window_split(rows * J * nseg, nsets);
+    const uint32_t nparts = nseg * split.parts * 64;
+    const size_t partial_bytes = slab * J * nparts * (size_t)(4 * kPartialWords);
     const size_t sums_bytes = slab * J * (size_t)(4 * kPartialWords);
     void* ws;
-    int rc = scratch_get(kSlotMsm, partial_bytes + sums_bytes + reduce_tmp_bytes(slab * J, nseg * 64), &ws, s);
+    int rc = scratch_get(kSlotMsm, partial_bytes + sums_bytes + reduce_tmp_bytes(slab * J, nparts), &ws, s);
     if (rc) return rc;
     uint32_t* sums = (uint32_t*)((char*)ws + partial_bytes);
     uint32_t* red_tmp = (uint32_t*)((char*)ws + partial_bytes + sums_bytes);
@@ -1367,10 +1383,10 @@ static int commit_strided_impl(uint32_t* out, const uint32_t* scalars, const int
             commit_sparse_strided_kernel<<<(unsigned)(nr * J), 64, 0, s>>>((uint32_t*)ws, sc, skip + r0 * rowlen, rowlen, nr * J, geom::spread_step(nr * J),
                                                                            table, N, c, nw, K, J, nsets);
         else
-            commit_strided_kernel<<<blocks_for(nr * J * nseg * 64), kBlock, 0, s>>>((uint32_t*)ws, sc, rowlen, nr, seg, nseg, table, N, c, nw, K, J, nsets);
+            commit_strided_kernel<<<blocks_for(nr * J * nparts), kBlock, 0, s>>>((uint32_t*)ws, sc, rowlen, nr, seg, nseg, table, N, c, nw, K, J, nsets, split);
         profile_mark(s);
-        launch_reduce<false>(sums, (const uint32_t*)ws, nr * J, nseg * 64, red_tmp, s);
-        strided_horner_kernel<<<blocks_for(nr, 64), 64, 0, s>>>(out + r0 * (size_t)(2 * FW), sums, nr, J, c);
+        launch_reduce<false>(sums, (const uint32_t*)ws, nr * J, nparts, red_tmp, s);
+        quad_horner_kernel<<<blocks_for(nr * 4, 64), 64, 0, s>>>(out + r0 * (size_t)(2 * FW), sums, nr, J, c);
         profile_mark(s);
     }
     GRAPE_LAUNCH_CHECK();

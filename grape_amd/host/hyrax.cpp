@@ -249,7 +249,7 @@ bool Hyrax::ensure_strided_table(uint rowlen, bool build) {
 bool Hyrax::commit_fr_rows(affine_t* out, fr_t* scalars, size_t size, uint rowlen, bool may_build, void* stream, int* d_flag) {
     // one row only (an opening's blinding row): a table that is already there is used, none is built for it,
     // and the per-window table is preferred - its 20 additions per scalar are nothing for one row, while the
-    // strided table's (J-1)*c doublings per row are a chain of half a millisecond on one lane
+    // strided table's (J-1)*c doublings per row are a chain (4096 columns: 0.23 against 0.34 ms, the byte windows 1.26)
     const bool single = size == rowlen;
     if (single && ensure_fr_table(rowlen, false)) {
         const WideTable& t = fr_table_;

@@ -84,3 +84,36 @@ def test_spread_units_are_a_permutation(n):
         step += 2
     seen = {i if i >= m else ((i % 32) * (m // 32) + i // 32) * step % m for i in range(n)}
     assert seen == set(range(n))
+
+
+# few rows of full-width scalars: the windows go over several waves (window_split: 1, 2, 3, 16 shares, shares of unequal
+# length), the partial sums over one, two and three levels of groups
+@pytest.mark.parametrize("rows,cols", [(1, 1), (1, 128), (3, 100), (15, 128), (129, 64), (300, 65)])
+def test_windows_over_several_waves(setup, rows, cols):
+    ops, orc, _, ref = setup
+    from gpuutil import rand_fr
+    gens = ops.g1_make_generators(rand_fr(128, 501))
+    s = rand_fr(rows * cols, 600 + rows)
+    s[:: 7] = 0
+    some = sorted({0, rows // 2, rows - 1})
+    want = orc.commit_fr(np.ascontiguousarray(s.reshape(rows, cols, 4)[some].reshape(-1, 4)), ref, cols, 128)
+    d = ops.to_dev(s)
+    for c, nw in ((8, 32), (13, 20)):
+        got = ops.g1_to_host(ops.commit_fr(d, cols, ops.g1_wide_table_gen(gens, c, nw, 1 << (c - 1)), 128, c, nw, 1 << (c - 1)))
+        assert np.array_equal(got[some], want), (c, nw)
+    for c, J, nsets in ((11, 1, 24), (8, 5, 7), (8, 32, 1)):
+        got = ops.g1_to_host(ops.commit_fr_strided(d, cols, ops.g1_strided_table_gen(gens, c, J, nsets), 128, c, J, nsets))
+        assert np.array_equal(got[some], want), (c, J)
+
+
+def test_one_long_row_in_three_levels(setup):
+    """a row of 4096: 64 segments x 10 shares x 64 lanes = 40960 partial sums -> 640 -> 40 -> 1"""
+    ops, orc, _, _ = setup
+    from gpuutil import rand_fr
+    gens = ops.g1_make_generators(rand_fr(4096, 503))
+    s = ops.to_dev(rand_fr(4096, 504))
+    a = ops.g1_to_host(ops.commit_fr(s, 4096, ops.g1_wide_table_gen(gens, 8, 32, 128), 4096, 8, 32, 128))
+    b = ops.g1_to_host(ops.commit_fr_strided(s, 4096, ops.g1_strided_table_gen(gens, 8, 8, 4), 4096, 8, 8, 4))
+    c = ops.g1_to_host(ops.commit_fr_ref_table(s, 4096, ops.g1_table_gen(gens, 256), 4096))
+    halves = [ops.g1_to_host(ops.commit_fr(s[:2048].contiguous(), 2048, ops.g1_wide_table_gen(gens[:2048].contiguous(), 8, 32, 128), 2048, 8, 32, 128))]
+    assert np.array_equal(a, b) and np.array_equal(a, c) and not np.array_equal(a, halves[0])
