@@ -421,9 +421,35 @@ static void give_peek_buffer(void* p) {
     std::lock_guard<std::mutex> lock(g_peek_mu);
     g_peek_free->push_back(p);
 }
+// The kernel may read the source only where all of it is memory of the current device: a block of grape_malloc, or what
+// the runtime knows of the address.  Host memory, another device's and ranges that end outside their allocation stay with
+// the runtime's copy, which serves or refuses them.
+static bool peek_readable(const void* s, size_t bytes) {
+    {
+        std::lock_guard<std::mutex> lock(g_alloc_mu);
+        alloc_tables();
+        auto it = g_live->upper_bound(const_cast<void*>(s));
+        if (it != g_live->begin()) {
+            --it;
+            const size_t off = (size_t)((const char*)s - (const char*)it->first);
+            if (off < it->second) return bytes <= it->second - off;
+        }
+    }
+    hipPointerAttribute_t at{};
+    int device = -1;
+    hipDeviceptr_t base = nullptr;
+    size_t size = 0;
+    if (hipPointerGetAttributes(&at, s) == hipSuccess && at.type == hipMemoryTypeDevice && hipGetDevice(&device) == hipSuccess && at.device == device &&
+        hipMemGetAddressRange(&base, &size, const_cast<void*>(s)) == hipSuccess) {
+        const size_t off = (size_t)((const char*)s - (const char*)base);
+        return off <= size && bytes <= size - off;
+    }
+    (void)hipGetLastError();
+    return false;
+}
 int grape_memcpy_d2h(void* d, const void* s, size_t bytes, grape_stream_t st) {
     if (!bytes) return GRAPE_OK;
-    if (bytes <= kPeekBytes && (bytes & 3) == 0 && (reinterpret_cast<uintptr_t>(s) & 3) == 0 && s != nullptr && d != nullptr) {
+    if (bytes <= kPeekBytes && (bytes & 3) == 0 && (reinterpret_cast<uintptr_t>(s) & 3) == 0 && s != nullptr && d != nullptr && peek_readable(s, bytes)) {
         if (void* pinned = take_peek_buffer()) {
             peek_kernel<<<1, 256, 0, as_stream(st)>>>((uint32_t*)pinned, (const uint32_t*)s, (uint32_t)(bytes / 4));
             hipError_t e = hipGetLastError();
@@ -434,7 +460,9 @@ int grape_memcpy_d2h(void* d, const void* s, size_t bytes, grape_stream_t st) {
             return GRAPE_OK;
         }
     }
-    GRAPE_HIP_CHECK(hipMemcpyAsync(d, s, bytes, hipMemcpyDeviceToHost, as_stream(st)));
+    const hipError_t e = hipMemcpyAsync(d, s, bytes, hipMemcpyDeviceToHost, as_stream(st));
+    if (e != hipSuccess) (void)hipGetLastError();          // a refused copy is reported here and not by the next launch
+    GRAPE_HIP_CHECK(e);
     GRAPE_HIP_CHECK(hipStreamSynchronize(as_stream(st)));
     return GRAPE_OK;
 }

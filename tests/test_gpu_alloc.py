@@ -24,6 +24,30 @@ def test_short_copies(lib, nbytes, offset):
     assert np.array_equal(out, src.cpu().numpy()[offset:offset + nbytes])
 
 
+@pytest.mark.parametrize("pinned", [False, True])
+def test_short_copies_of_host_memory(lib, pinned):
+    """a source that is host memory stays with the runtime's copy, which serves pinned memory and refuses the rest: no kernel reads it"""
+    src = torch.arange(64, dtype=torch.int32)
+    src = src.pin_memory() if pinned else src
+    out = np.zeros(64, dtype=np.int32)
+    rc = lib.grape_memcpy_d2h(out.ctypes.data_as(ctypes.c_void_p), ctypes.c_void_p(src.data_ptr()), 256, None)
+    assert rc == (0 if pinned else -2)
+    assert np.array_equal(out, src.numpy() if pinned else np.zeros(64, dtype=np.int32))
+    dev = torch.arange(64, dtype=torch.int32, device="cuda")
+    assert lib.grape_memcpy_d2h(out.ctypes.data_as(ctypes.c_void_p), ctypes.c_void_p(dev.data_ptr()), 256, None) == 0
+    assert np.array_equal(out, np.arange(64))
+
+
+def test_short_copy_of_the_last_bytes_of_a_block(lib):
+    from grape_amd import _capi
+    p = ctypes.c_void_p()
+    _capi.check(lib.grape_malloc(ctypes.byref(p), 1 << 21))
+    out = np.zeros(64, dtype=np.int32)
+    dst = out.ctypes.data_as(ctypes.c_void_p)
+    assert lib.grape_memcpy_d2h(dst, ctypes.c_void_p(p.value + (1 << 21) - 256), 256, None) == 0
+    _capi.check(lib.grape_free(p))
+
+
 def _cycle(lib, n_words, value):
     """fill a block, queue its copy into a second one, give the first back and take it again for other contents"""
     from grape_amd import _capi
