@@ -61,6 +61,9 @@ SIGNATURES = {
     "grape_sumcheck_round2_noalloc": [c_void_p, c_void_p, c_u32, c_u32, c_void_p, c_void_p, c_void_p],
     "grape_sumcheck_round2_tail": [c_void_p, c_void_p, c_u32, c_u32, c_void_p, c_void_p, c_void_p],
     "grape_short_rounds": [c_void_p, c_void_p],
+    "grape_wround_partial_bytes": [c_void_p],
+    "grape_wround_queue": [c_void_p, c_void_p],
+    "grape_wround_finish": [c_void_p, c_u32, c_void_p, c_u32, c_void_p],
     "grape_sumcheck_round2_coeffs": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_u32, c_u32, c_void_p, c_void_p, c_void_p],
     "grape_sumcheck_round1": [c_void_p, c_void_p, c_void_p, c_u32, c_u32, c_void_p, c_void_p],
     "grape_eq_pyramid_elems": [c_u32],
@@ -140,7 +143,7 @@ SIGNATURES = {
     "grape_event_elapsed_ms": [ctypes.POINTER(ctypes.c_float), c_void_p, c_void_p],
 }
 _RESTYPES = {"grape_last_error": ctypes.c_char_p, "grape_g1_wide_table_bytes": c_size_t, "grape_eq_pyramid_elems": c_size_t,
-             "grape_wround2_partial_bytes": c_size_t, "grape_fr_fold_i32_elems": c_size_t}
+             "grape_wround2_partial_bytes": c_size_t, "grape_wround_partial_bytes": c_size_t, "grape_fr_fold_i32_elems": c_size_t}
 
 _lib = None
 

@@ -94,12 +94,17 @@ __device__ __forceinline__ void wround2_result(uint32_t* out, const Fr* acc) {
 // is not accumulated - one product and one double-width accumulator less per index.
 // IDX: A is not read but gathered, A[i] = Bt[idx1[i] - 1] (in_size == 2 n_out): the first round of a lookup whose
 // logUp tensor was never written out - the pass over the witness left the table indices only.
-template <bool BETA, bool PLAIN, bool UNIT, bool TAB, bool NOMID = false, bool IDX = false>
+// SPLIT: the weight of index h * period + l is Eh[h] * E[l].  A thread keeps one l, so E[l] is applied once, to its three sums,
+// and what it reads per index is Eh[h] - the same word for a whole wave.  No table of n_out weights is made or read: building
+// one and reading it back is 64 to 96 bytes an index pair beside the 192 of the operands (2^23 pairs and the levels below
+// 2^20: 0.16 ms of launches, element product of 2048 x 11008: 0.30 ms).
+template <bool BETA, bool PLAIN, bool UNIT, bool TAB, bool NOMID = false, bool IDX = false, bool SPLIT = false>
 __global__ void __launch_bounds__(kBlock, 2) wround2_kernel(uint32_t* Aw, uint32_t* Sw, const uint32_t* A, const uint32_t* S,
                                                          const uint32_t* beta, const uint32_t* E,
                                                          uint32_t in_size, uint32_t n_out, uint32_t rowlen, uint32_t rowpad,
                                                          const uint32_t* v, const int32_t* __restrict__ tab, uint32_t* partial,
-                                                         const int32_t* __restrict__ idx1 = nullptr, const uint32_t* Bt = nullptr) {
+                                                         const int32_t* __restrict__ idx1 = nullptr, const uint32_t* Bt = nullptr,
+                                                         const uint32_t* Eh = nullptr, uint32_t period = 1) {
     constexpr int NV = PLAIN ? 5 : 3;
     __shared__ Fr lds[NV * (kBlock / 64)];
     fr26::Limbs w1;
@@ -113,11 +118,19 @@ __global__ void __launch_bounds__(kBlock, 2) wround2_kernel(uint32_t* Aw, uint32
     fr26::Limbs sa0, sa1;                       // plain limb-wise sums of A's halves (24 terms below 2^26)
 #pragma unroll
     for (int k = 0; k < fr26::N; k++) sa0.v[k] = sa1.v[k] = 0;
-    const size_t stride = (size_t)gridDim.x * kBlock;
-    for (size_t g = (size_t)blockIdx.x * kBlock + threadIdx.x; g < n_out; g += stride) {
+    size_t stride = (size_t)gridDim.x * kBlock;
+    const size_t first = (size_t)blockIdx.x * kBlock + threadIdx.x;
+    uint32_t h = 0, low = 0, hstep = 0;
+    if (SPLIT) {
+        hstep = (uint32_t)stride / period;
+        stride = (size_t)hstep * period;             // whole periods: the threads behind them have no index
+        h = (uint32_t)first / period;
+        low = (uint32_t)first - h * period;
+    }
+    for (size_t g = SPLIT && first >= stride ? n_out : first; g < n_out; g += stride, h += hstep) {
         // weights live on rows of `rowpad` entries when the tensors' rows hold `rowlen` < rowpad
         const size_t ei = rowlen == rowpad ? g : g + (size_t)((uint32_t)g / rowlen) * (rowpad - rowlen);
-        const fr26::Limbs e16 = fr26::pack16(ld_fr(E, ei));
+        const fr26::Limbs e16 = fr26::pack16(SPLIT ? ld_fr(Eh, h) : ld_fr(E, ei));
         fr26::Limbs a0, a1;
         if (IDX) {
             const uint32_t j0 = (uint32_t)idx1[g], j1 = (uint32_t)idx1[g + n_out];     // 0 marks an element outside the table
@@ -163,6 +176,12 @@ __global__ void __launch_bounds__(kBlock, 2) wround2_kernel(uint32_t* Aw, uint32
     acc[0] = reduce_to_fr(W0, 3);
     acc[1] = NOMID ? Fr::zero() : reduce_to_fr(WQ, 6);
     acc[2] = reduce_to_fr(W2, 3);
+    if (SPLIT) {
+        const Fr el = ld_fr(E, low);
+        if (!UNIT) acc[0] = fr26::mulc(acc[0], el);
+        if (!UNIT && !NOMID) acc[1] = fr26::mulc(acc[1], el);
+        acc[2] = fr26::mulc(acc[2], el);
+    }
     if (PLAIN) {
         acc[3] = fr26::limb_sum_to_fr(sa0, 0);      // below 24 r
         acc[4] = fr26::limb_sum_to_fr(sa1, 0);
@@ -173,13 +192,20 @@ __global__ void __launch_bounds__(kBlock, 2) wround2_kernel(uint32_t* Aw, uint32
         for (int k = 0; k < NV; k++) st_fr(partial, (size_t)blockIdx.x * NV + k, acc[k]);
     }
 }
+// One workgroup finishes one round; a proof that reads its sums at the end finishes all its long rounds in one launch.
+constexpr uint32_t kMaxFinish = 32;
+struct WFinish {
+    const uint32_t* partial[kMaxFinish];
+    uint32_t nblocks[kMaxFinish];
+    uint32_t* out[kMaxFinish];
+};
 template <bool PLAIN, bool UNIT, bool NOMID, int BLOCK>
-__global__ void __launch_bounds__(BLOCK) wround2_final_kernel(uint32_t* out, const uint32_t* partial, unsigned nblocks) {
+__global__ void __launch_bounds__(BLOCK) wround2_final_kernel(WFinish f) {
     constexpr int NV = PLAIN ? 5 : 3;
     __shared__ uint32_t lds9[NV * (BLOCK / 64) * 9];
     Fr tot[NV];
-    workgroup_totals<NV, BLOCK, NOMID ? 2u : 0u>(tot, partial, nblocks, lds9);
-    if (threadIdx.x == 0) wround2_result<PLAIN, UNIT, NOMID>(out, tot);
+    workgroup_totals<NV, BLOCK, NOMID ? 2u : 0u>(tot, f.partial[blockIdx.x], f.nblocks[blockIdx.x], lds9);
+    if (threadIdx.x == 0) wround2_result<PLAIN, UNIT, NOMID>(f.out[blockIdx.x], tot);
 }
 
 // ---------------------------------------------------------------- matmul phase 1: weights per segment
@@ -353,12 +379,13 @@ static int wround2_main(uint32_t* Aw, uint32_t* Sw, const uint32_t* A, const uin
 #undef GRAPE_WROUND2
     return GRAPE_OK;
 }
-static void wround2_final(uint32_t* sums, const uint32_t* partial, uint32_t n_out, int plain_sums, hipStream_t s) {
-    const unsigned nb = wround2_blocks(n_out);
-#define GRAPE_WFINAL(P, U, M)                                                                                    \
-    do {                                                                                                         \
-        if (nb >= kFinalWideMin) wround2_final_kernel<P, U, M, kFinalBlock><<<1, kFinalBlock, 0, s>>>(sums, partial, nb); \
-        else wround2_final_kernel<P, U, M, kBlock><<<1, kBlock, 0, s>>>(sums, partial, nb);                      \
+static void wround2_final(const WFinish& f, uint32_t count, int plain_sums, hipStream_t s) {
+    unsigned nb = 0;
+    for (uint32_t i = 0; i < count; i++) nb = std::max(nb, f.nblocks[i]);
+#define GRAPE_WFINAL(P, U, M)                                                                            \
+    do {                                                                                                 \
+        if (nb >= kFinalWideMin) wround2_final_kernel<P, U, M, kFinalBlock><<<count, kFinalBlock, 0, s>>>(f); \
+        else wround2_final_kernel<P, U, M, kBlock><<<count, kBlock, 0, s>>>(f);                          \
     } while (0)
     if (plain_sums == 3) GRAPE_WFINAL(true, false, true);
     else if (plain_sums == 2) GRAPE_WFINAL(true, true, false);
@@ -366,6 +393,25 @@ static void wround2_final(uint32_t* sums, const uint32_t* partial, uint32_t n_ou
     else GRAPE_WFINAL(false, false, false);
 #undef GRAPE_WFINAL
 }
+static void wround2_final(uint32_t* sums, const uint32_t* partial, uint32_t n_out, int plain_sums, hipStream_t s) {
+    WFinish f{};
+    f.partial[0] = partial;
+    f.nblocks[0] = wround2_blocks(n_out);
+    f.out[0] = sums;
+    wround2_final(f, 1, plain_sums, s);
+}
+// workgroups of a round with split weights: a power of two, so that 256 CUs with two workgroups each are filled evenly, and
+// enough of them for at most kWIters whole periods per thread
+static unsigned wround_split_blocks(uint32_t n_out, uint32_t period) {
+    const uint64_t periods = ((uint64_t)n_out + period - 1) / period;
+    unsigned nb = kNumCU * 4;
+    while (true) {
+        const uint64_t step = (uint64_t)nb * kBlock / period;
+        if (step && (periods + step - 1) / step <= kWIters) return nb;
+        nb *= 2;
+    }
+}
+static unsigned wround_blocks(const grape_wround_args& a) { return a.eq_high ? wround_split_blocks(a.n_out, a.period) : wround2_blocks(a.n_out); }
 #define GRAPE_WROUND2_CHECKS()                                                                                              \
     CHECK_PTR16(A); CHECK_PTR16(S); CHECK_PTR16(E); CHECK_PTR16(v);                                                        \
     GRAPE_REQUIRE(n_out >= 1 && in_size >= n_out && in_size <= 2 * (uint64_t)n_out, "need n_out <= in_size <= 2*n_out"); \
@@ -436,6 +482,63 @@ int grape_wround2_queue_indexed(uint32_t* A, uint32_t* S, const int32_t* idx1, c
     GRAPE_REQUIRE(tab != nullptr && n_out >= kTableFoldMinOut && n_out <= (1u << 30), "built for first rounds of 2^16 index pairs and more");
     wround2_kernel<true, true, true, true, false, true><<<wround2_blocks(n_out), kBlock, 0, as_stream(st)>>>(
         A, S, A, S, beta, E, 2 * n_out, n_out, 1, 1, v, tab, partial, idx1, Bt);
+    GRAPE_LAUNCH_CHECK();
+    return GRAPE_OK;
+}
+
+size_t grape_wround_partial_bytes(const grape_wround_args* args) {
+    if (!args || args->n_out < 1 || (args->eq_high && (args->period < 1 || args->period > GRAPE_WROUND_MAX_PERIOD))) return 0;
+    return (size_t)wround_blocks(*args) * (args->plain_sums ? 5 : 3) * 32;
+}
+int grape_wround_queue(const grape_wround_args* args, grape_stream_t st) {
+    GRAPE_REQUIRE(args != nullptr, "null arguments");
+    const grape_wround_args& a = *args;
+    const uint32_t *A = a.A, *S = a.S, *E = a.eq, *v = a.v, *beta = a.beta;
+    const uint32_t in_size = a.in_size, n_out = a.n_out, rowlen = a.rowlen, rowpad = a.rowpad;
+    GRAPE_WROUND2_CHECKS();
+    CHECK_PTR16(a.A_out); CHECK_PTR16(a.S_out); CHECK_PTR16(a.partial);
+    hipStream_t s = as_stream(st);
+    const unsigned nb = wround_blocks(a);
+    GRAPE_REQUIRE(a.tab == nullptr || n_out >= kTableFoldMinOut, "the table fold is built for rounds of 2^16 index pairs and more");
+    GRAPE_REQUIRE((a.idx1 == nullptr && a.eq_high == nullptr) || a.tab != nullptr, "indexed rounds and split weights need the challenge's table");
+    if (a.idx1) {
+        CHECK_PTR16(a.B);
+        GRAPE_REQUIRE(a.plain_sums == 2 && beta && in_size == 2 * (uint64_t)n_out && rowlen == rowpad, "an indexed round is a lookup's first round");
+    }
+    if (!a.eq_high) {
+        if (a.idx1)
+            wround2_kernel<true, true, true, true, false, true><<<nb, kBlock, 0, s>>>(a.A_out, a.S_out, A, S, beta, E, in_size, n_out, 1, 1, v, a.tab,
+                                                                                     a.partial, a.idx1, a.B);
+        else if (int rc = wround2_main(a.A_out, a.S_out, A, S, beta, E, in_size, n_out, rowlen, rowpad, v, a.plain_sums, a.tab, a.partial, s)) return rc;
+        GRAPE_LAUNCH_CHECK();
+        return GRAPE_OK;
+    }
+    CHECK_PTR16(a.eq_high);
+    GRAPE_REQUIRE(a.period >= 1 && a.period <= GRAPE_WROUND_MAX_PERIOD, "the period of split weights is 1..2^20");
+#define GRAPE_WSPLIT(BETA, P, U, M, I)                                                                                           \
+    wround2_kernel<BETA, P, U, true, M, I, true><<<nb, kBlock, 0, s>>>(a.A_out, a.S_out, A, S, beta, E, in_size, n_out, 1, 1, v, a.tab, \
+                                                                    a.partial, a.idx1, a.B, a.eq_high, a.period)
+    if (a.plain_sums == 0 && !beta) GRAPE_WSPLIT(false, false, false, false, false);
+    else if (a.plain_sums == 3 && beta) GRAPE_WSPLIT(true, true, false, true, false);
+    else if (a.plain_sums == 2 && beta && a.idx1) GRAPE_WSPLIT(true, true, true, false, true);
+    else if (a.plain_sums == 2 && beta && in_size == 2 * (uint64_t)n_out) GRAPE_WSPLIT(true, true, true, false, false);
+    else GRAPE_REQUIRE(false, "split weights are built for plain_sums 0 without beta and for 2 and 3 with it");
+#undef GRAPE_WSPLIT
+    GRAPE_LAUNCH_CHECK();
+    return GRAPE_OK;
+}
+int grape_wround_finish(uint32_t* sums, uint32_t stride, const grape_wround_args* rounds, uint32_t count, grape_stream_t st) {
+    CHECK_PTR16(sums);
+    GRAPE_REQUIRE(rounds != nullptr && count >= 1 && count <= kMaxFinish, "1..32 rounds");
+    WFinish f{};
+    for (uint32_t i = 0; i < count; i++) {
+        CHECK_PTR16(rounds[i].partial);
+        GRAPE_REQUIRE(rounds[i].plain_sums == rounds[0].plain_sums && grape_wround_partial_bytes(&rounds[i]) != 0, "rounds of one kind");
+        f.partial[i] = rounds[i].partial;
+        f.nblocks[i] = wround_blocks(rounds[i]);
+        f.out[i] = sums + (size_t)i * stride * 8;
+    }
+    wround2_final(f, count, rounds[0].plain_sums, as_stream(st));
     GRAPE_LAUNCH_CHECK();
     return GRAPE_OK;
 }

@@ -18,6 +18,8 @@ static void read3(fr_t* d_sums, Fr out[3]) {
 }
 
 namespace {
+constexpr uint kLongRoundPairs = 1u << 16;       // from here on a round folds through the table of its challenge's multiples
+constexpr uint kSplitLow = GRAPE_EQ_SPLIT_LOW, kLongestPrefix = GRAPE_EQ_LONGEST_PREFIX;
 // device buffer released on scope exit
 struct DeviceBuf {
     void* p = nullptr;
@@ -34,6 +36,21 @@ struct EqPyramid {
         check(grape_eq_pyramid(W(buf.fr()), reinterpret_cast<const uint32_t*>(d_u), nvars, nullptr), "grape_eq_pyramid");
     }
     fr_t* level(uint j) const { return buf.fr() + (((size_t)1 << j) - 1); }
+};
+// Weights of the rounds of a long sumcheck over nvars variables at d_u: tables of every prefix as far as `whole` variables; longer
+// rounds take their weight as a product of a table over the lowest `low` variables and one over the rest.
+struct EqWeights {
+    uint low, whole;
+    EqPyramid prefix;
+    std::unique_ptr<EqPyramid> high;
+    EqWeights(const fr_t* d_u, uint nvars, uint low_, uint whole_) : low(low_), whole(std::min(nvars, whole_)), prefix(d_u, whole) {
+        if (nvars > whole) high.reset(new EqPyramid(d_u + low, nvars - low));
+    }
+    void weigh(grape_wround_args& a, uint vars, uint period) const {
+        a.eq = W(prefix.level(vars > whole ? low : vars));
+        a.eq_high = vars > whole ? W(high->level(vars - low)) : nullptr;
+        a.period = period;
+    }
 };
 std::vector<Fr> download_vec(const fr_t* d, size_t n) {
     std::vector<Fr> out(n);
@@ -296,13 +313,26 @@ static Fr eleMul_rounds(fr_t* Aw, fr_t* Bw, const fr_t* A, const fr_t* B, fr_t* 
         hu = us.data() + rounds;
         hv = vs.data() + rounds;
     }
-    EqPyramid eq(u - rounds, rounds - 1);
+    // Long rounds: the weights of a padded row split into row and column, those of whole powers of two at 2^17.  A row whose
+    // padded length has no prefix table of its own (above 2^20) is weighed by whole tables.
+    const uint lg_row = Log2(second_size);
+    const bool padded = second_size != row_pad;
+    const uint low = padded ? lg_row : kSplitLow;
+    const EqWeights eq(u - rounds, rounds - 1, low, padded && lg_row > kLongestPrefix ? rounds : kLongestPrefix);
     FrTensor sums(3 * rounds + 2);
+    // the tables of all challenges' multiples, and every long round's partial sums until one launch finishes them all
+    std::vector<grape_wround_args> queued;
+    std::vector<std::unique_ptr<DeviceBuf>> partials;
+    std::unique_ptr<DeviceBuf> tabs;
+    if (size / 2 >= kLongRoundPairs) {
+        tabs.reset(new DeviceBuf(sizeof(int32_t) * GRAPE_FOLD_TABLE_WORDS * (size_t)rounds));
+        check(grape_fold_tables(static_cast<int32_t*>(tabs->p), W(v - rounds), rounds, nullptr), "grape_fold_tables");
+    }
     uint in = size, out = size / 2;
     for (uint i = 0; i < rounds; i++) {
         const fr_t *Ai = i ? Aw : A, *Bi = i ? Bw : B;
         // short rounds in one call; a single row that is no power of two has no defined first round and is refused below
-        if (in <= GRAPE_SHORT_MAX && out < (1u << 16) && ((in & (in - 1)) == 0 || (first_size > 1 && in % second_size == 0))) {
+        if (in <= GRAPE_SHORT_MAX && out < kLongRoundPairs && ((in & (in - 1)) == 0 || (first_size > 1 && in % second_size == 0))) {
             grape_short_rounds_args a{};
             a.kind = GRAPE_SHORT_PAIR;
             a.weights = GRAPE_SHORT_FULL;
@@ -311,7 +341,7 @@ static Fr eleMul_rounds(fr_t* Aw, fr_t* Bw, const fr_t* A, const fr_t* B, fr_t* 
             a.x[0] = W(Ai);
             a.x[1] = W(Bi);
             a.v_end = W(v - i);
-            a.pyramid = W(eq.level(0));
+            a.pyramid = W(eq.prefix.level(0));
             a.top_level = rounds - 1 - i;
             a.sums = W(sums.gpu_data + 3 * i);
             a.stride = 3;
@@ -323,14 +353,28 @@ static Fr eleMul_rounds(fr_t* Aw, fr_t* Bw, const fr_t* A, const fr_t* B, fr_t* 
             break;
         }
         // while whole rows are paired the weights are addressed on padded rows
-        const bool rows = in > second_size && second_size != row_pad;
-        check(grape_wround2_from(W(Aw), W(Bw), W(Ai), W(Bi), W(eq.level(rounds - 1 - i)), in, out, rows ? second_size : 1,
-                                 rows ? row_pad : 1, W(v - i - 1), W(sums.gpu_data + 3 * i), nullptr),
-              "grape_wround2_from");
+        const bool rows = in > second_size && padded;
+        grape_wround_args a{};
+        a.A_out = W(Aw);
+        a.S_out = W(Bw);
+        a.A = W(Ai);
+        a.S = W(Bi);
+        eq.weigh(a, rounds - 1 - i, rows ? second_size : 1u << kSplitLow);
+        a.rowlen = rows ? second_size : 1;
+        a.rowpad = rows ? row_pad : 1;
+        a.in_size = in;
+        a.n_out = out;
+        a.v = W(v - i - 1);
+        a.tab = out >= kLongRoundPairs ? static_cast<int32_t*>(tabs->p) + (size_t)GRAPE_FOLD_TABLE_WORDS * (rounds - 1 - i) : nullptr;
+        partials.emplace_back(new DeviceBuf(grape_wround_partial_bytes(&a)));
+        a.partial = W(partials.back()->fr());
+        check(grape_wround_queue(&a, nullptr), "grape_wround_queue");
+        queued.push_back(a);
         in = out;
         out = out == second_size ? (1u << (Log2(out) - 1)) : out / 2;
         if (out == 0) out = 1;
     }
+    if (!queued.empty()) check(grape_wround_finish(W(sums.gpu_data), 3, queued.data(), (uint)queued.size(), nullptr), "grape_wround_finish");
     const std::vector<Fr> s = download_vec(sums.gpu_data, 3 * (size_t)rounds + 2);
     for (uint i = 0; i < rounds; i++) {
         const Fr &u_now = *(hu - 1 - i), &v_now = *(hv - 1 - i);

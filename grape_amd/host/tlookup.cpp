@@ -269,18 +269,45 @@ std::pair<void*, void*> commit_events() {
 }
 }  // namespace
 
+// The weights of a lookup's rounds in one tensor: tables of every prefix of the point as far as the table side and rounds of 2^20
+// weights read them, and behind them, for longer rounds, those over the variables from GRAPE_EQ_SPLIT_LOW on (a long round's weight is
+// a product of two tables' entries).
+namespace {
+struct WeightPlan {
+    uint whole = 0, high = 0;
+    WeightPlan(uint nu, uint N) {
+        const uint all = nu ? nu - 1 : 0;
+        whole = std::min(all, std::max(GRAPE_EQ_LONGEST_PREFIX, Log2(N)));
+        if (all > whole) high = all - GRAPE_EQ_SPLIT_LOW;
+    }
+    size_t elems() const { return grape_eq_pyramid_elems(whole) + (high ? grape_eq_pyramid_elems(high) : 0); }
+    void build(fr_t* E, const fr_t* d_u, grape_stream_t st) const {
+        check(grape_eq_pyramid(W(E), W(const_cast<fr_t*>(d_u)), whole, st), "grape_eq_pyramid");
+        if (high)
+            check(grape_eq_pyramid(W(E + grape_eq_pyramid_elems(whole)), W(const_cast<fr_t*>(d_u) + GRAPE_EQ_SPLIT_LOW), high, st), "grape_eq_pyramid");
+    }
+    void weigh(grape_wround_args& a, fr_t* E, uint vars) const {
+        const bool split = vars > whole;
+        a.eq = W(E + (((size_t)1 << (split ? GRAPE_EQ_SPLIT_LOW : vars)) - 1));
+        a.eq_high = split ? W(E + grape_eq_pyramid_elems(whole) + (((size_t)1 << (vars - GRAPE_EQ_SPLIT_LOW)) - 1)) : nullptr;
+        a.period = 1u << GRAPE_EQ_SPLIT_LOW;
+    }
+};
+}  // namespace
+
 void tLookup::start_weights(uint D) {
     const uint nu = Log2(D);
     u_ready_ = forced_u_.empty() ? random_vec(nu) : forced_u_;
     forced_u_.clear();
     E_ready_.reset();
     if (u_ready_.size() != nu) return;          // run() reports the mismatch
-    E_ready_.reset(new FrTensor((uint)grape_eq_pyramid_elems(nu ? nu - 1 : 0), FrTensor::OnAnyStream()));
+    const WeightPlan plan(nu, T.size);
+    E_ready_.reset(new FrTensor((uint)plan.elems(), FrTensor::OnAnyStream()));
     // the point travels on the second stream too: on the default stream it would queue behind the pass over the
     // witness, and the pyramid with it
     SideChain side(0);
     fr_t* d_u = grape_host::upload(u_ready_, side.stream);
-    check(grape_eq_pyramid(W(E_ready_->gpu_data), W(d_u), nu ? nu - 1 : 0, side.stream), "grape_eq_pyramid");
+    plan.build(E_ready_->gpu_data, d_u, side.stream);
     grape_free(d_u);                            // handed out again only after what is queued here
 }
 
@@ -437,17 +464,18 @@ Fr tLookup::run(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax& hyrax
     const Fr two_inv = Fr(2).invert();
     const uint logN = Log2(N);
 
-    // eq tables of every prefix of u[0 .. nu-2]: round k (which binds variable nu-1-k) weights its
-    // D / 2^(k+1) index pairs with level nu-1-k; nothing is halved between rounds
+    // eq tables of the prefixes of u[0 .. nu-2]: round k (which binds variable nu-1-k) weights its
+    // D / 2^(k+1) index pairs with those of nu-1-k variables; nothing is halved between rounds
     const uint nu = (uint)u.size();
+    const WeightPlan plan(nu, N);
     std::unique_ptr<FrTensor> E_own;
     if (E_early) {
         SideChain early(0);
         SideChain::order(nullptr, early.stream);     // the default stream meets the finished pyramid
     } else {
-        E_own.reset(new FrTensor((uint)grape_eq_pyramid_elems(nu ? nu - 1 : 0)));
+        E_own.reset(new FrTensor((uint)plan.elems()));
         fr_t* d_u = grape_host::upload(u);
-        check(grape_eq_pyramid(W(E_own->gpu_data), W(d_u), nu ? nu - 1 : 0, nullptr), "grape_eq_pyramid");
+        plan.build(E_own->gpu_data, d_u, nullptr);
         grape_free_on_default(d_u);
     }
     FrTensor& E = E_early ? *E_early : *E_own;
@@ -491,11 +519,11 @@ Fr tLookup::run(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax& hyrax
         int vi = (int)rounds - 1;
         size_t long_used = 0;
         int32_t* d_tabs = nullptr;
-        // A and S: five sums and the fold of both tensors in one pass
+        std::vector<grape_wround_args> unfinished;
+        // A and S of 2^16 index pairs and more: five sums and the fold of both tensors in one pass
         auto witness_round = [&](grape_stream_t st) {
             const uint half = cur / 2;
             fr_t* slot = sums.gpu_data + 13 * (size_t)k;
-            const fr_t* e = E.gpu_data + (((size_t)1 << (nu - 1 - k)) - 1);
             // first round of a witness that sits on its table: A = B[index] is the exact inverse of S + beta at
             // every index (B holds the inverses of T + beta, none of which is zero for a range table and, for
             // a mapping table with its random r, except with probability 2^-235), and the weights of a full
@@ -503,27 +531,37 @@ Fr tLookup::run(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax& hyrax
             int mode = (k == 0 && from_table && cur == 2 * half && (cur & (cur - 1)) == 0) ? 2 : 1;
             // a long round after the first: its middle coefficient is left to the host, which holds the
             // round's claim when it assembles the polynomials (one limb product per index pair less)
-            if (mode == 1 && half >= kLongRoundPairs) {
+            if (mode == 1) {
                 mode = 3;
                 mid_from_claim[k] = 1;
             }
-            if (long_work && half >= kLongRoundPairs) {
-                // long round beside the commitments: only the pass over the operands stays on the chain of rounds; its
-                // sums are finished on the stream of the short rounds, from a work buffer of the round's own
-                uint32_t* partial = reinterpret_cast<uint32_t*>(long_work + long_used);
-                long_used += grape_wround2_partial_bytes(half);
-                if (k == 0 && gather_first)
-                    check(grape_wround2_queue_indexed(W(A.gpu_data), W(S.gpu_data), d_idx_, W(B.gpu_data), N, W(d_beta), W(e), half, W(d_v + vi),
-                                                      d_tabs + (size_t)GRAPE_FOLD_TABLE_WORDS * (size_t)vi, partial, st),
-                          "grape_wround2_queue_indexed");
-                else
-                    check(grape_wround2_queue(W(A.gpu_data), W(S.gpu_data), W(d_beta), W(e), cur, half, 1, 1, W(d_v + vi), mode,
-                                              d_tabs + (size_t)GRAPE_FOLD_TABLE_WORDS * (size_t)vi, partial, st),
-                          "grape_wround2_queue");
+            // long round: only the pass over the operands stays on the chain of rounds; its sums wait in a work buffer of the
+            // round's own.  Beside the commitments they are finished on the stream of the short rounds, else all together.
+            grape_wround_args a{};
+            a.A_out = W(A.gpu_data);
+            a.S_out = W(S.gpu_data);
+            a.A = W(A.gpu_data);
+            a.S = W(S.gpu_data);
+            if (k == 0 && gather_first) {
+                a.idx1 = d_idx_;
+                a.B = W(B.gpu_data);
+            }
+            a.beta = W(d_beta);
+            plan.weigh(a, E.gpu_data, nu - 1 - k);
+            a.rowlen = a.rowpad = 1;
+            a.in_size = cur;
+            a.n_out = half;
+            a.v = W(d_v + vi);
+            a.plain_sums = mode;
+            a.tab = d_tabs + (size_t)GRAPE_FOLD_TABLE_WORDS * (size_t)vi;
+            a.partial = reinterpret_cast<uint32_t*>(long_work + long_used);
+            long_used += grape_wround_partial_bytes(&a);
+            check(grape_wround_queue(&a, st), "grape_wround_queue");
+            if (overlap) {
                 SideChain::order(witness.stream, st);
-                check(grape_wround2_finish(W(slot), partial, half, mode, witness.stream), "grape_wround2_finish");
+                check(grape_wround_finish(W(slot), 13, &a, 1, witness.stream), "grape_wround_finish");
             } else {
-                check(grape_wround2(W(A.gpu_data), W(S.gpu_data), W(d_beta), W(e), cur, half, 1, 1, W(d_v + vi), mode, W(slot), st), "grape_wround2");
+                unfinished.push_back(a);
             }
             A.set_size(half);
             S.set_size(half);
@@ -567,6 +605,21 @@ Fr tLookup::run(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax& hyrax
                 cur_t = half;
             }
         };
+        // work memory of the long rounds (every round its own partial sums) and the tables of all challenges' multiples
+        size_t need = 0;
+        for (uint c = D, i = 0; c / 2 >= kLongRoundPairs && i < rounds; c /= 2, i++) {
+            grape_wround_args a{};
+            plan.weigh(a, E.gpu_data, nu - 1 - i);
+            a.n_out = c / 2;
+            a.plain_sums = 1;
+            need += grape_wround_partial_bytes(&a);
+        }
+        if (need) {
+            check(grape_malloc_on_default((void**)&long_work, need + sizeof(int32_t) * GRAPE_FOLD_TABLE_WORDS * (size_t)rounds), "grape_malloc");
+            d_tabs = reinterpret_cast<int32_t*>(long_work + need);
+            for (uint k0 = 0; k0 < rounds; k0 += 64)
+                check(grape_fold_tables(d_tabs + (size_t)GRAPE_FOLD_TABLE_WORDS * k0, W(d_v + k0), std::min(64u, rounds - k0), nullptr), "grape_fold_tables");
+        }
         // overlap: the commitments are queued without waiting (their digit-range flags are read after
         // the rounds have been queued too), so the chip works on them while the host issues the
         // rounds' launches; everything that needs the host to wait on the default stream (the sums
@@ -577,15 +630,6 @@ Fr tLookup::run(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax& hyrax
         // wave waits for memory, which made the pair slower than one after the other.  The short
         // rounds (launch-bound) do run beside the commitments, on a stream of their own.
         if (overlap) {
-            // work memory of the long rounds (every round its own partial sums) and the tables of all challenges' multiples
-            size_t need = 0;
-            for (uint c = D; c / 2 >= kLongRoundPairs; c /= 2) need += grape_wround2_partial_bytes(c / 2);
-            if (need) {
-                check(grape_malloc_on_default((void**)&long_work, need + sizeof(int32_t) * GRAPE_FOLD_TABLE_WORDS * (size_t)rounds), "grape_malloc");
-                d_tabs = reinterpret_cast<int32_t*>(long_work + need);
-                for (uint k0 = 0; k0 < rounds; k0 += 64)
-                    check(grape_fold_tables(d_tabs + (size_t)GRAPE_FOLD_TABLE_WORDS * k0, W(d_v + k0), std::min(64u, rounds - k0), nullptr), "grape_fold_tables");
-            }
             while (vi >= 0 && cur / 2 >= kLongRoundPairs) witness_round(nullptr);
             // The table side and the commitment of m (a few rows: a short accumulation and a latency chain of a
             // row reduction) go to the second stream now, so that they run beside the long rounds and the
@@ -619,6 +663,13 @@ Fr tLookup::run(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax& hyrax
             check(grape_event_record(commit_events().second, nullptr), "grape_event_record");
         }
         while (vi >= 0 && cur / 2 >= kLongRoundPairs) witness_round(ws);
+        // the first round may be of another kind than the rest
+        for (size_t i = 0; i < unfinished.size();) {
+            size_t e = i + 1;
+            while (e < unfinished.size() && unfinished[e].plain_sums == unfinished[i].plain_sums) e++;
+            check(grape_wround_finish(W(sums.gpu_data + 13 * i), 13, &unfinished[i], (uint)(e - i), ws), "grape_wround_finish");
+            i = e;
+        }
         if (vi >= 0) {
             grape_short_rounds_args a = short_args(GRAPE_SHORT_LOGUP, k, cur);
             a.x[0] = a.last[0] = W(A.gpu_data);

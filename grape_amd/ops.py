@@ -424,6 +424,29 @@ def wround2_split(A, S, beta, e, in_size, n_out, v, plain_sums=False, rowlen=1, 
     return sums
 
 
+class _Wround(ctypes.Structure):
+    _fields_ = [("A_out", ctypes.c_void_p), ("S_out", ctypes.c_void_p), ("A", ctypes.c_void_p), ("S", ctypes.c_void_p),
+                ("idx1", ctypes.c_void_p), ("B", ctypes.c_void_p), ("beta", ctypes.c_void_p), ("eq", ctypes.c_void_p), ("eq_high", ctypes.c_void_p),
+                ("period", ctypes.c_uint32), ("rowlen", ctypes.c_uint32), ("rowpad", ctypes.c_uint32), ("in_size", ctypes.c_uint32),
+                ("n_out", ctypes.c_uint32), ("v", ctypes.c_void_p), ("plain_sums", ctypes.c_int), ("tab", ctypes.c_void_p), ("partial", ctypes.c_void_p)]
+
+
+def wround_products(A, S, beta, low, high, period, in_size, n_out, v, plain_sums=0, idx1=None, B=None):
+    """a weighted round of 2^16 index pairs and more whose weight at h * period + l is high[h] * low[l], folded in place"""
+    lib = init()
+    nv = 5 if plain_sums else 3
+    tab = torch.empty(100, dtype=torch.int32, device="cuda")
+    _capi.check(lib.grape_fold_tables(_p(tab), _p(v), 1, _s()))
+    a = _Wround(A_out=_p(A), S_out=_p(S), A=_p(A), S=_p(S), idx1=_p(idx1), B=_p(B), beta=_p(beta), eq=_p(low), eq_high=_p(high), period=period,
+                rowlen=1, rowpad=1, in_size=in_size, n_out=n_out, v=_p(v), plain_sums=plain_sums, tab=_p(tab))
+    partial = torch.empty(lib.grape_wround_partial_bytes(ctypes.byref(a)) // 4, dtype=torch.int32, device="cuda")
+    a.partial = _p(partial)
+    sums = fr_empty(nv)
+    _capi.check(lib.grape_wround_queue(ctypes.byref(a), _s()))
+    _capi.check(lib.grape_wround_finish(_p(sums), nv, ctypes.byref(a), 1, _s()))
+    return sums
+
+
 def wround2_first_indexed(S, idx1, B, beta, e, n_out, v):
     """first round of a lookup whose logUp tensor A = B[idx1 - 1] was never written out; returns (sums, folded A)"""
     lib = init()

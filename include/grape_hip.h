@@ -254,6 +254,35 @@ int grape_wround2_queue_indexed(uint32_t *d_A, uint32_t *d_S, const int32_t *d_i
                                 const uint32_t *d_beta, const uint32_t *d_e, uint32_t n_out, const uint32_t *d_v, const int32_t *d_tab,
                                 uint32_t *d_partial, grape_stream_t stream);
 /*
+ * The pass of a weighted round in its general form (fields as the arguments of grape_wround2, grape_wround2_from,
+ * grape_wround2_queue and grape_wround2_queue_indexed; A and A_out, S and S_out may be the same).  With eq_high the
+ * weight of index h * period + l is eq_high[h] * eq[l] and rowlen, rowpad are not used (1, 1): a tensor whose rows hold
+ * fewer elements than the weights' rows takes its row length as the period.  eq_high needs tab and plain_sums 0
+ * without beta, or 2 or 3 with it.  grape_wround_finish finishes `count` <= 32 such rounds of one plain_sums in one launch; round i's
+ * sums go to element i * stride of d_sums.  Every round has its own partial (grape_wround_partial_bytes) until then.
+ */
+#define GRAPE_WROUND_MAX_PERIOD (1u << 20)
+/* Where provers split: rounds of at most 2^20 weights read them from a prefix table.  A split round multiplies a thread's three sums
+ * once more - 3 products beside the 20 of the four indices it has at that size - and making the table of 2^20 takes 14 us. */
+#define GRAPE_EQ_LONGEST_PREFIX 20u
+#define GRAPE_EQ_SPLIT_LOW 17u
+typedef struct {
+    uint32_t *A_out, *S_out;
+    const uint32_t *A, *S;
+    const int32_t *idx1;       /* with it A is B[idx1 - 1] */
+    const uint32_t *B;
+    const uint32_t *beta;
+    const uint32_t *eq, *eq_high;
+    uint32_t period, rowlen, rowpad, in_size, n_out;
+    const uint32_t *v;
+    int plain_sums;
+    const int32_t *tab;
+    uint32_t *partial;
+} grape_wround_args;
+size_t grape_wround_partial_bytes(const grape_wround_args *args);
+int grape_wround_queue(const grape_wround_args *args, grape_stream_t stream);
+int grape_wround_finish(uint32_t *d_sums, uint32_t stride, const grape_wround_args *rounds, uint32_t count, grape_stream_t stream);
+/*
  * One round of matmul_sumcheck_phase1 (src/prove.cu:49-85): grape_sumcheck_round2 on indices
  * g = seg * seglen + k where every index of a segment carries the weight d_e[seg]
  * (out_size / seglen segments): d_sums[t] = sum_seg d_e[seg] * sum_k coefficient_t(seg, k); A and B
