@@ -184,37 +184,61 @@ typedef int v16i_t __attribute__((ext_vector_type(16)));
 constexpr int kMfTN = 64, kMfTM = 128, kMfK = 64, kMfLd = 64;
 constexpr int kBgT = 128;      // rows of a and rows of b per workgroup of the large-tile kernel
 
-// planes[p][row][k] for k < Kp (zero beyond K) for three planes, and the largest magnitude of x folded
-// into *mx with an atomic maximum (one per workgroup): the caller learns from it how many of the
-// planes are non-zero.  A thread takes 4 consecutive k at a time, the grid strides over the tensor.
-__global__ void __launch_bounds__(kBlock) wit_split_kernel(int8_t* planes, uint32_t* mx, const int32_t* x, uint32_t R, uint32_t K, uint32_t Kp) {
-    const uint32_t per_row = Kp / 4;
-    const size_t total = (size_t)R * per_row, stride = (size_t)gridDim.x * kBlock;
-    const size_t plane = (size_t)R * Kp;
+// planes[p][row][k] for k < Kp (zero beyond K) for three planes, and the largest magnitude that each workgroup met in its word of mx:
+// the caller learns from them how many of the planes are non-zero.  Both operands of a product in one launch.
+// Bound by memory (4 bytes in, 3 out): a thread takes groups of 4 consecutive k, four groups in flight before the first is split, and
+// a workgroup walks whole rows (several rows where a row has fewer groups than it has threads), so that nothing is divided per group.
+// A word per workgroup and not one atomic maximum: 4096 of those on one line were most of the launch.
+// Both operands of 2048 x 4096 by 4096 x 4096: 60 -> 30 us (5.9 TB/s); 2048 x 4096 by 11008 x 4096: 100 -> 75 us.
+struct SplitArgs {
+    int8_t* planes;
+    const int32_t* x;
+    uint32_t* mx;
+    uint32_t R, groups;      // rows, workgroups
+};
+constexpr uint32_t kSplitGroups = 2048;          // workgroups of one operand at most: the words of both are one short copy
+constexpr uint32_t kSplitAhead = 4;
+__global__ void __launch_bounds__(kBlock) wit_split_kernel(SplitArgs a, SplitArgs b, uint32_t K, uint32_t Kp) {
+    const SplitArgs p = blockIdx.x < a.groups ? a : b;
+    const uint32_t wg = blockIdx.x < a.groups ? blockIdx.x : blockIdx.x - a.groups;
+    const uint32_t per_row = Kp / 4, width = per_row < (uint32_t)kBlock ? per_row : (uint32_t)kBlock, rows = (uint32_t)kBlock / width;
+    const uint32_t r0 = threadIdx.x / width, c0 = threadIdx.x - r0 * width;
+    const size_t plane = (size_t)p.R * Kp;
     uint32_t m = 0;
-    for (size_t idx = (size_t)blockIdx.x * kBlock + threadIdx.x; idx < total; idx += stride) {
-        const uint32_t row = (uint32_t)(idx / per_row), k = 4u * (uint32_t)(idx - (size_t)row * per_row);
-        int32_t v[4] = {0, 0, 0, 0};
-        if (k < K) {      // K is a multiple of 4
-            const int4 t = *reinterpret_cast<const int4*>(x + (size_t)row * K + k);
-            v[0] = t.x; v[1] = t.y; v[2] = t.z; v[3] = t.w;
-        }
+    for (size_t row = r0 < rows ? (size_t)wg * rows + r0 : p.R; row < p.R; row += (size_t)p.groups * rows) {
+        const int32_t* x = p.x + row * K;
+        int8_t* out = p.planes + row * Kp;
+        for (uint32_t c = c0; c < per_row; c += kSplitAhead * width) {
+            int4 t[kSplitAhead];
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const uint32_t a = v[j] < 0 ? 0u - (uint32_t)v[j] : (uint32_t)v[j];
-            m = a > m ? a : m;
-        }
-#pragma unroll
-        for (int p = 0; p < 3; p++) {
-            uint32_t w = 0;
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const int32_t d = (int32_t)(int8_t)(v[j] & 0xff);
-                // (v - d) is a multiple of 256; the subtraction cannot wrap (|d| <= 128 towards zero)
-                v[j] = (int32_t)(((int64_t)v[j] - d) >> 8);
-                w |= ((uint32_t)d & 0xffu) << (8 * j);
+            for (uint32_t u = 0; u < kSplitAhead; u++) {
+                const uint32_t k = 4u * (c + u * width);
+                t[u] = make_int4(0, 0, 0, 0);
+                if (c + u * width < per_row && k < K) t[u] = *reinterpret_cast<const int4*>(x + k);      // K is a multiple of 4, at most Kp
             }
-            *reinterpret_cast<uint32_t*>(planes + p * plane + (size_t)row * Kp + k) = w;
+#pragma unroll
+            for (uint32_t u = 0; u < kSplitAhead; u++) {
+                const uint32_t k = 4u * (c + u * width);
+                if (c + u * width >= per_row) break;
+                int32_t v[4] = {t[u].x, t[u].y, t[u].z, t[u].w};
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const uint32_t mag = v[j] < 0 ? 0u - (uint32_t)v[j] : (uint32_t)v[j];
+                    m = mag > m ? mag : m;
+                }
+#pragma unroll
+                for (int q = 0; q < 3; q++) {
+                    uint32_t w = 0;
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        const int32_t d = (int32_t)(int8_t)(v[j] & 0xff);
+                        // (v - d) is a multiple of 256; the subtraction cannot wrap (|d| <= 128 towards zero)
+                        v[j] = (int32_t)(((int64_t)v[j] - d) >> 8);
+                        w |= ((uint32_t)d & 0xffu) << (8 * j);
+                    }
+                    *reinterpret_cast<uint32_t*>(out + q * plane + k) = w;
+                }
+            }
         }
     }
 #pragma unroll
@@ -222,14 +246,13 @@ __global__ void __launch_bounds__(kBlock) wit_split_kernel(int8_t* planes, uint3
         const uint32_t o = __shfl_xor(m, off, 64);
         m = o > m ? o : m;
     }
-    // one atomic per workgroup: atomics on one address are served one after the other
     __shared__ uint32_t sh[kBlock / 64];
     if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = m;
     __syncthreads();
     if (threadIdx.x == 0) {
 #pragma unroll
         for (int w = 1; w < kBlock / 64; w++) m = sh[w] > m ? sh[w] : m;
-        if (m) atomicMax(mx, m);
+        p.mx[wg] = m;
     }
 }
 
@@ -540,14 +563,30 @@ __global__ void __launch_bounds__(kBlock) wit_elemul_rescale_kernel(int32_t* q, 
     if (bad) atomicOr(status, bad);
 }
 
+// Four elements a thread where both arrays are 16-byte aligned (VEC): four gathers in flight, one 16-byte load and store.
+// Bound by the gathers' latency: 22.5 M elements in a table of 2^19 95 -> 67 us.
+template <bool VEC>
 __global__ void __launch_bounds__(kBlock) wit_lookup_kernel(int32_t* out, const int32_t* in, size_t n, int32_t low, uint32_t len,
                                                             const int32_t* table, uint32_t* status) {
     const size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x;
-    if (i >= n) return;
-    const int64_t idx = (int64_t)in[i] - (int64_t)low;
-    const bool ok = idx >= 0 && idx < (int64_t)len;
-    out[i] = table[ok ? idx : 0];
-    if (!ok) atomicOr(status, (uint32_t)kWitIndex);
+    bool all_in = true;
+    auto at = [&](int32_t key) {
+        const int64_t idx = (int64_t)key - (int64_t)low;
+        const bool ok = idx >= 0 && idx < (int64_t)len;
+        all_in = all_in && ok;
+        return table[ok ? idx : 0];
+    };
+    if (VEC) {
+        if (4 * i + 3 < n) {
+            const int4 k = reinterpret_cast<const int4*>(in)[i];
+            reinterpret_cast<int4*>(out)[i] = make_int4(at(k.x), at(k.y), at(k.z), at(k.w));
+        } else {
+            for (size_t e = 4 * i; e < n; e++) out[e] = at(in[e]);
+        }
+    } else if (i < n) {
+        out[i] = at(in[i]);
+    }
+    if (!all_in) atomicOr(status, (uint32_t)kWitIndex);
 }
 
 __global__ void __launch_bounds__(kBlock) wit_add_kernel(int32_t* out, const int32_t* a, const int32_t* b, size_t n) {
@@ -741,7 +780,7 @@ int grape_wit_matmul_rescale(int32_t* d_q, int32_t* d_r, const int32_t* d_a, con
     void *pa = nullptr, *pb = nullptr;
     if (g_matmul_method != 1 && L == 1 && aligned && (g_matmul_method == 2 || (uint64_t)N * M * K >= ((uint64_t)1 << 26))) {
         void* mx;
-        rc = scratch_get(kSlotMisc, 64, &mx, s);
+        rc = scratch_get(kSlotMisc, sizeof(uint32_t) * 2 * kSplitGroups, &mx, s);
         if (rc) return rc;
         rc = scratch_get(kSlotWitA, (size_t)3 * N * Kp, &pa, s);
         if (rc) return rc;
@@ -752,17 +791,17 @@ int grape_wit_matmul_rescale(int32_t* d_q, int32_t* d_r, const int32_t* d_a, con
             profile_begin();
             profile_mark(s);
         }
-        wit_status_clear_kernel<<<1, 1, 0, s>>>(d_mx);
-        wit_status_clear_kernel<<<1, 1, 0, s>>>(d_mx + 1);
-        // at least 8 groups of 4 per thread, at most 2048 workgroups (one atomic each)
-        const size_t ga_ = ((size_t)N * (Kp / 4) + kBlock * 8 - 1) / (kBlock * 8), gb_ = ((size_t)M * (Kp / 4) + kBlock * 8 - 1) / (kBlock * 8);
-        wit_split_kernel<<<(unsigned)(ga_ < 2048 ? ga_ : 2048), kBlock, 0, s>>>((int8_t*)pa, d_mx, d_a, N, K, Kp);
-        wit_split_kernel<<<(unsigned)(gb_ < 2048 ? gb_ : 2048), kBlock, 0, s>>>((int8_t*)pb, d_mx + 1, d_b, M, K, Kp);
+        // whole rows per workgroup
+        const uint32_t at_once = Kp / 4 < (uint32_t)kBlock ? (uint32_t)kBlock / (Kp / 4) : 1;
+        auto groups = [&](uint32_t rows) { return std::min(kSplitGroups, (rows + at_once - 1) / at_once); };
+        const SplitArgs sa{(int8_t*)pa, d_a, d_mx, N, groups(N)}, sb{(int8_t*)pb, d_b, d_mx + sa.groups, M, groups(M)};
+        wit_split_kernel<<<sa.groups + sb.groups, kBlock, 0, s>>>(sa, sb, K, Kp);
         GRAPE_LAUNCH_CHECK();
         if (profiling()) profile_mark(s);
-        uint32_t h_mx[2] = {0, 0};
-        GRAPE_HIP_CHECK(hipMemcpyAsync(h_mx, d_mx, sizeof(h_mx), hipMemcpyDeviceToHost, s));
-        GRAPE_HIP_CHECK(hipStreamSynchronize(s));
+        uint32_t h_mx[2] = {0, 0}, h_words[2 * kSplitGroups];
+        rc = grape_memcpy_d2h(h_words, d_mx, sizeof(uint32_t) * (sa.groups + sb.groups), st);       // through pinned memory; waits for the stream
+        if (rc) return rc;
+        for (uint32_t g = 0; g < sa.groups + sb.groups; g++) h_mx[g >= sa.groups] = std::max(h_mx[g >= sa.groups], h_words[g]);
         if (profiling()) profile_mark(s);      // intervals: the split, the host's read of the magnitudes, the product
         PA = planes_for(h_mx[0]);
         PB = planes_for(h_mx[1]);
@@ -840,7 +879,9 @@ int grape_wit_table_lookup(int32_t* d_out, const int32_t* d_in, size_t n, int32_
     uint32_t* status;
     int rc = status_word(&status, s);
     if (rc) return rc;
-    wit_lookup_kernel<<<blocks_for(n), kBlock, 0, s>>>(d_out, d_in, n, low, len, d_table, status);
+    if (((reinterpret_cast<uintptr_t>(d_out) | reinterpret_cast<uintptr_t>(d_in)) & 15) == 0)
+        wit_lookup_kernel<true><<<blocks_for((n + 3) / 4), kBlock, 0, s>>>(d_out, d_in, n, low, len, d_table, status);
+    else wit_lookup_kernel<false><<<blocks_for(n), kBlock, 0, s>>>(d_out, d_in, n, low, len, d_table, status);
     GRAPE_LAUNCH_CHECK();
     return GRAPE_OK;
 }
