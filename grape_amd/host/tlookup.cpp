@@ -243,6 +243,11 @@ struct SideChain {
         check(grape_event_record(ev, other), "grape_event_record");
         check(grape_stream_wait_event(waiter, ev), "grape_stream_wait_event");
     }
+    // the same for this stream, which from then on holds work of the scope
+    void after(grape_stream_t other) {
+        order(stream, other);
+        open = true;
+    }
     void begin() {
         check(grape_event_record(ev_begin, nullptr), "grape_event_record");
         check(grape_stream_wait_event(stream, ev_begin), "grape_stream_wait_event");
@@ -558,7 +563,7 @@ Fr tLookup::run(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax& hyrax
             long_used += grape_wround_partial_bytes(&a);
             check(grape_wround_queue(&a, st), "grape_wround_queue");
             if (overlap) {
-                SideChain::order(witness.stream, st);
+                witness.after(st);
                 check(grape_wround_finish(W(slot), 13, &a, 1, witness.stream), "grape_wround_finish");
             } else {
                 unfinished.push_back(a);
