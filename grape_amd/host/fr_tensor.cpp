@@ -38,21 +38,31 @@ fr_t* device_scalar(const Fr& x) {
     check(grape_memcpy_h2d(slot, &x, sizeof(fr_t), nullptr), "grape_memcpy_h2d");
     return slot;
 }
-DeviceFr::DeviceFr(const Fr& x) {
+template <class T>
+static void allocate(T** p, size_t bytes, bool on_default) {
     ensure_init();
-    check(grape_malloc_on_default((void**)&p_, sizeof(fr_t)), "grape_malloc");
+    check(on_default ? grape_malloc_on_default((void**)p, bytes) : grape_malloc((void**)p, bytes), "grape_malloc");
+}
+static void release(void* p, bool on_default) { on_default ? grape_free_on_default(p) : grape_free(p); }
+
+DeviceFr::DeviceFr(const Fr& x) {
+    allocate(&p_, sizeof(fr_t), false);
     check(grape_memcpy_h2d(p_, &x, sizeof(fr_t), nullptr), "grape_memcpy_h2d");
 }
-DeviceFr::~DeviceFr() { grape_free_on_default(p_); }
+DeviceFr::DeviceFr(const Fr& x, OnDefaultStream) : on_default_(true) {
+    allocate(&p_, sizeof(fr_t), true);
+    check(grape_memcpy_h2d(p_, &x, sizeof(fr_t), nullptr), "grape_memcpy_h2d");
+}
+DeviceFr::~DeviceFr() { release(p_, on_default_); }
 
-fr_t* upload(const std::vector<Fr>& v, void* stream) {
-    ensure_init();
+static fr_t* upload_to(const std::vector<Fr>& v, void* stream, bool on_default) {
     fr_t* d = nullptr;
-    const size_t bytes = sizeof(fr_t) * std::max<size_t>(v.size(), 1);
-    check(stream ? grape_malloc((void**)&d, bytes) : grape_malloc_on_default((void**)&d, bytes), "grape_malloc");
+    allocate(&d, sizeof(fr_t) * std::max<size_t>(v.size(), 1), on_default);
     check(grape_memcpy_h2d(d, v.data(), sizeof(fr_t) * v.size(), stream), "grape_memcpy_h2d");
     return d;
 }
+fr_t* upload(const std::vector<Fr>& v, void* stream) { return upload_to(v, stream, false); }
+fr_t* upload(const std::vector<Fr>& v, OnDefaultStream) { return upload_to(v, nullptr, true); }
 Fr download(const fr_t* d_ptr) {
     Fr out;
     check(grape_memcpy_d2h(&out, d_ptr, sizeof(fr_t), nullptr), "grape_memcpy_d2h");
@@ -62,6 +72,7 @@ Fr download(const fr_t* d_ptr) {
 }  // namespace grape_host
 
 using grape_host::check;
+using grape_host::OnDefaultStream;
 static inline uint32_t* W(fr_t* p) { return reinterpret_cast<uint32_t*>(p); }
 static inline const uint32_t* W(const fr_t* p) { return reinterpret_cast<const uint32_t*>(p); }
 
@@ -87,27 +98,23 @@ void pad_int(int** int_data, uint N, uint pad_N, uint pad_size) {
     check(grape_free(old), "grape_free");
 }
 
-FrTensor::FrTensor(uint size_) : gpu_data(nullptr), size(size_), capacity_(size_) {
-    grape_host::ensure_init();
-    check(grape_malloc_on_default((void**)&gpu_data, sizeof(fr_t) * (size_t)size), "grape_malloc");
+FrTensor::FrTensor(uint size_, Memory memory) : gpu_data(nullptr), size(size_), capacity_(size_), memory_(memory) {
+    grape_host::allocate(&gpu_data, sizeof(fr_t) * (size_t)size, memory_ == kOnDefaultStream);
 }
-FrTensor::FrTensor(uint size_, OnAnyStream) : gpu_data(nullptr), size(size_), capacity_(size_), on_default_(false) {
-    grape_host::ensure_init();
-    check(grape_malloc((void**)&gpu_data, sizeof(fr_t) * (size_t)size), "grape_malloc");
-}
-FrTensor::FrTensor(const FrTensor& t) : gpu_data(nullptr), size(t.size), capacity_(t.size) {
-    check(grape_malloc_on_default((void**)&gpu_data, sizeof(fr_t) * (size_t)size), "grape_malloc");
+FrTensor::FrTensor(uint size_) : FrTensor(size_, kOrdinary) {}
+FrTensor::FrTensor(uint size_, OnDefaultStream) : FrTensor(size_, kOnDefaultStream) {}
+FrTensor::FrTensor(const FrTensor& t) : FrTensor(t.size, kOrdinary) {
     check(grape_memcpy_d2d(gpu_data, t.gpu_data, sizeof(fr_t) * (size_t)size, nullptr), "grape_memcpy_d2d");
 }
-FrTensor::FrTensor(uint size_, int* int_data) : gpu_data(nullptr), size(size_), capacity_(size_) {
-    grape_host::ensure_init();
-    check(grape_malloc_on_default((void**)&gpu_data, sizeof(fr_t) * (size_t)size), "grape_malloc");
+FrTensor::FrTensor(const FrTensor& t, OnDefaultStream) : FrTensor(t.size, kOnDefaultStream) {
+    check(grape_memcpy_d2d(gpu_data, t.gpu_data, sizeof(fr_t) * (size_t)size, nullptr), "grape_memcpy_d2d");
+}
+FrTensor::FrTensor(uint size_, int* int_data) : FrTensor(size_, kOrdinary) {
     check(grape_fr_from_i32(W(gpu_data), int_data, size, nullptr), "grape_fr_from_i32");
 }
 FrTensor::~FrTensor() {
     if (gpu_data != nullptr) {
-        if (on_default_) grape_free_on_default(gpu_data);
-        else grape_free(gpu_data);
+        grape_host::release(gpu_data, memory_ == kOnDefaultStream);
         gpu_data = nullptr;
     }
 }
@@ -134,7 +141,7 @@ void FrTensor::partial_eval(uint N, fr_t* x, uint c, uint id, uint gap) {
 // src/fr-tensor.cu:346-369, including the rows-of-11008 reading of a short tensor
 Fr FrTensor::operator()(const std::vector<Fr>& u) {
     uint log_dim = (uint)u.size();
-    fr_t* d_u = grape_host::upload(u);
+    fr_t* d_u = grape_host::upload(u, OnDefaultStream());
     if ((uint64_t)size < ((uint64_t)1 << log_dim)) {
         check(grape_fr_fold(W(gpu_data), size, W(d_u), size / 11008, Log2(11008), 11008, nullptr), "grape_fr_fold");
         check(grape_fr_fold(W(gpu_data), 11008, W(d_u), 11008, 0, 1, nullptr), "grape_fr_fold");
@@ -208,21 +215,25 @@ FrTensor FrTensor::random(uint size) {
     for (uint i = 0; i < size; i++) tmp[i] = Fr::random_element();
     return from_host(tmp);
 }
-FrTensor FrTensor::folded_from(const fr_t* device_data, uint N, fr_t* x, uint c, uint id, uint gap) {
-    grape_host::ensure_init();
+FrTensor FrTensor::fold_new(const fr_t* field, const int* ints, uint N, fr_t* x, uint c, uint id, uint gap, Memory memory) {
     const size_t elems = grape_fr_fold_i32_elems(N, c, gap);
-    FrTensor out((uint)(elems ? elems : 1));
-    check(grape_fr_fold_from(W(out.gpu_data), W(device_data), N, W(x), c, id, gap, nullptr), "grape_fr_fold_from");
+    FrTensor out((uint)(elems ? elems : 1), memory);
+    if (ints) check(grape_fr_fold_i32(W(out.gpu_data), ints, N, W(x), c, id, gap, nullptr), "grape_fr_fold_i32");
+    else check(grape_fr_fold_from(W(out.gpu_data), W(field), N, W(x), c, id, gap, nullptr), "grape_fr_fold_from");
     out.set_size(c && gap ? N / (c * gap) * gap : 0);
     return out;
 }
+FrTensor FrTensor::folded_from(const fr_t* device_data, uint N, fr_t* x, uint c, uint id, uint gap) {
+    return fold_new(device_data, nullptr, N, x, c, id, gap, kOrdinary);
+}
+FrTensor FrTensor::folded_from(const fr_t* device_data, uint N, fr_t* x, uint c, uint id, uint gap, OnDefaultStream) {
+    return fold_new(device_data, nullptr, N, x, c, id, gap, kOnDefaultStream);
+}
 FrTensor FrTensor::folded_from_ints(const int* device_int_data, uint N, fr_t* x, uint c, uint id, uint gap) {
-    grape_host::ensure_init();
-    const size_t elems = grape_fr_fold_i32_elems(N, c, gap);
-    FrTensor out((uint)(elems ? elems : 1));
-    check(grape_fr_fold_i32(W(out.gpu_data), device_int_data, N, W(x), c, id, gap, nullptr), "grape_fr_fold_i32");
-    out.set_size(c && gap ? N / (c * gap) * gap : 0);
-    return out;
+    return fold_new(nullptr, device_int_data, N, x, c, id, gap, kOrdinary);
+}
+FrTensor FrTensor::folded_from_ints(const int* device_int_data, uint N, fr_t* x, uint c, uint id, uint gap, OnDefaultStream) {
+    return fold_new(nullptr, device_int_data, N, x, c, id, gap, kOnDefaultStream);
 }
 Fr FrTensor::eval_ints(const int* device_int_data, uint size, const std::vector<Fr>& u) {
     if ((uint64_t)size != ((uint64_t)1 << u.size())) {
@@ -230,14 +241,19 @@ Fr FrTensor::eval_ints(const int* device_int_data, uint size, const std::vector<
         FrTensor t(size, const_cast<int*>(device_int_data));
         return t(u);
     }
-    fr_t* d_u = grape_host::upload(u);
-    FrTensor t = folded_from_ints(device_int_data, size, d_u, size, 0, 1);
+    fr_t* d_u = grape_host::upload(u, OnDefaultStream());
+    FrTensor t = folded_from_ints(device_int_data, size, d_u, size, 0, 1, OnDefaultStream());
     Fr ret = grape_host::download(t.gpu_data);
     grape_free_on_default(d_u);
     return ret;
 }
 FrTensor FrTensor::from_host(const std::vector<Fr>& v) {
     FrTensor out((uint)v.size());
+    check(grape_memcpy_h2d(out.gpu_data, v.data(), sizeof(fr_t) * v.size(), nullptr), "grape_memcpy_h2d");
+    return out;
+}
+FrTensor FrTensor::from_host(const std::vector<Fr>& v, OnDefaultStream on) {
+    FrTensor out((uint)v.size(), on);
     check(grape_memcpy_h2d(out.gpu_data, v.data(), sizeof(fr_t) * v.size(), nullptr), "grape_memcpy_h2d");
     return out;
 }
@@ -252,7 +268,7 @@ void Fr_partial_me(uint N, FrTensor& t, fr_t* x, uint id, uint cur_dim, uint win
     const size_t dim = (size_t)cur_dim * window_size;
     if (N % dim != 0) throw std::runtime_error("Fr_partial_me: N is not a multiple of cur_dim * window_size");
     const uint outer = (uint)(N / dim);
-    FrTensor folded(N);
+    FrTensor folded(N, OnDefaultStream());
     check(grape_memcpy_d2d(folded.gpu_data, t.gpu_data, sizeof(fr_t) * (size_t)N, nullptr), "grape_memcpy_d2d");
     check(grape_fr_fold(W(folded.gpu_data), N, W(x), cur_dim, id, window_size, nullptr), "grape_fr_fold");
     for (uint o = 0; o < outer; o++)

@@ -8,6 +8,10 @@
 #include "fr.hpp"
 
 namespace grape_host {
+// Marks memory that no caller gets to see and only the default stream works on: a block goes from one owner to the next in that
+// stream's order (grape_malloc_on_default), with no wait.  Whatever a caller may hold is allocated without it: a caller may work
+// on it on any stream, also on one this library never hears of.
+struct OnDefaultStream {};
 // Throws std::runtime_error carrying grape_last_error() when a C-ABI call fails.
 void check(int rc, const char* what);
 // Uploads one scalar into a small ring of device slots and returns its device address
@@ -20,6 +24,7 @@ fr_t* device_scalar(const Fr& x);
 class DeviceFr {
 public:
     explicit DeviceFr(const Fr& x);
+    DeviceFr(const Fr& x, OnDefaultStream);
     ~DeviceFr();
     DeviceFr(const DeviceFr&) = delete;
     DeviceFr& operator=(const DeviceFr&) = delete;
@@ -27,9 +32,11 @@ public:
 
 private:
     fr_t* p_ = nullptr;
+    bool on_default_ = false;
 };
 // Uploads a challenge vector; the caller frees with grape_free.
 fr_t* upload(const std::vector<Fr>& v, void* stream = nullptr);   // queued on `stream` (nullptr: the default stream)
+fr_t* upload(const std::vector<Fr>& v, OnDefaultStream);          // freed with grape_free_on_default
 Fr download(const fr_t* d_ptr);
 void ensure_init();
 }  // namespace grape_host
@@ -43,11 +50,9 @@ public:
     uint size;
 
     FrTensor(uint size);
-    // memory that is first used on a stream of its own, with nothing to order that stream behind what the default stream
-    // has queued (every other tensor lives on the default stream and takes its memory over in that stream's order)
-    struct OnAnyStream {};
-    FrTensor(uint size, OnAnyStream);
     FrTensor(const FrTensor& t);                 // deep copy
+    FrTensor(uint size, grape_host::OnDefaultStream);
+    FrTensor(const FrTensor& t, grape_host::OnDefaultStream);
     FrTensor(uint size, int* device_int_data);   // embeds device int32 values
     ~FrTensor();
 
@@ -85,15 +90,21 @@ public:
     // operator()(u) for a power-of-two size
     static FrTensor folded_from(const fr_t* device_data, uint N, fr_t* x, uint c, uint id, uint gap);
     static FrTensor folded_from_ints(const int* device_int_data, uint N, fr_t* x, uint c, uint id, uint gap);
+    static FrTensor folded_from(const fr_t* device_data, uint N, fr_t* x, uint c, uint id, uint gap, grape_host::OnDefaultStream);
+    static FrTensor folded_from_ints(const int* device_int_data, uint N, fr_t* x, uint c, uint id, uint gap, grape_host::OnDefaultStream);
     static Fr eval_ints(const int* device_int_data, uint size, const std::vector<Fr>& u);
     // additions: host <-> device transfer of whole tensors
     static FrTensor from_host(const std::vector<Fr>& v);
+    static FrTensor from_host(const std::vector<Fr>& v, grape_host::OnDefaultStream);
     std::vector<Fr> to_host() const;
     uint capacity() const { return capacity_; }
 
 private:
+    enum Memory { kOrdinary, kOnDefaultStream };
+    FrTensor(uint size, Memory memory);
+    static FrTensor fold_new(const fr_t* field, const int* ints, uint N, fr_t* x, uint c, uint id, uint gap, Memory memory);
     uint capacity_;
-    bool on_default_ = true;
+    Memory memory_;
 };
 
 // The fold WITHOUT the compaction that FrTensor::partial_eval adds (src/fr-tensor.cu:168-188): the

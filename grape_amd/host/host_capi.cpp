@@ -72,8 +72,9 @@ static Fr fr_from(const uint32_t* p) {
 static void fr_to(uint32_t* p, const Fr& x) { std::memcpy(p, &x, 32); }
 static int g_input_format = 0;      // 0: field elements, 1: int32 values (grape_host_set_input_format)
 static bool g_int_folds = true;     // integer inputs of an opening or an evaluation are folded from the integers (grape_host_set_int_folds)
+using grape_host::OnDefaultStream;
 static FrTensor tensor_from_device(const uint32_t* d, uint32_t n, uint32_t capacity = 0) {
-    FrTensor t(capacity > n ? capacity : n);
+    FrTensor t(capacity > n ? capacity : n, OnDefaultStream());
     if (g_input_format == 1) {
         // as the reference's drivers hand integers to a tensor: FrTensor::get_data (test/llm.cu:77)
         t.get_data(n, reinterpret_cast<int*>(const_cast<uint32_t*>(d)));
@@ -298,12 +299,12 @@ int grape_host_tlookup_range_prove(const uint32_t* d_S, uint32_t D, int32_t low,
     lk.alpha = fr_from(alpha);
     lk.set_u(vec_from(u, nuv));
     uint32_t Dp = 1u << Log2(D);
-    FrTensor A(Dp);
+    FrTensor A(Dp, OnDefaultStream());
     double ct = 0;
     Fr sc;
     if (g_input_format == 1 && g_int_folds) {
         // the witness stays a tensor of integers: the prover's pass over it embeds it on the way
-        FrTensor S(Dp);
+        FrTensor S(Dp, OnDefaultStream());
         S.set_size(D);
         ProveTimer timer;
         sc = lk.prove(reinterpret_cast<const int*>(d_S), S, A, vec_from(v, nuv), hyrax, msm_size, ct);
@@ -342,7 +343,7 @@ static void mapping_prove_impl(const uint32_t* d_S_in, const uint32_t* d_S_out, 
     lk.alpha = fr_from(alpha);
     lk.set_u(vec_from(u, nuv));
     uint32_t Dp = 1u << Log2(D);
-    FrTensor A(Dp);
+    FrTensor A(Dp, OnDefaultStream());
     double ct = 0;
     Fr sc;
     if (g_input_format == 1 && g_int_folds) {

@@ -6,6 +6,7 @@
 #include "../../include/grape_hip.h"
 
 using grape_host::check;
+using grape_host::OnDefaultStream;
 static inline uint32_t* W(void* p) { return reinterpret_cast<uint32_t*>(p); }
 static inline const uint32_t* W(const void* p) { return reinterpret_cast<const uint32_t*>(p); }
 
@@ -412,11 +413,11 @@ Hyrax_proof Hyrax::open_impl(FrTensor* tensor_in, const int* ints, const std::ve
     uint new_N = pad_N * com_scale;
     assert(eval_point_.size() == Log2(size));
     last_open_point_ = eval_point_;
-    fr_t* eval_point = grape_host::upload(eval_point_);
+    fr_t* eval_point = grape_host::upload(eval_point_, OnDefaultStream());
 
     std::vector<Fr> host_d(new_N);
     for (uint i = 0; i < new_N; i++) host_d[i] = Fr::random_element();
-    FrTensor d = FrTensor::from_host(host_d);
+    FrTensor d = FrTensor::from_host(host_d, OnDefaultStream());
 
     // commitment of d: one row of new_N full-width scalars (single_commit, src/Hyrax.cu:176-185).  A short
     // accumulation and then a latency chain (the row's reduction), so it runs on a stream of its own beside the folds
@@ -442,11 +443,11 @@ Hyrax_proof Hyrax::open_impl(FrTensor* tensor_in, const int* ints, const std::ve
     check(grape_memset_zero(d_flag, sizeof(int), open_stream), "grape_memset_zero");
     const bool flag_used = commit_fr_rows(com_d_dev, d.gpu_data, new_N, new_N, false, open_stream, d_flag);
 
-    FrTensor x(new_N);
+    FrTensor x(new_N, OnDefaultStream());
     std::unique_ptr<FrTensor> rows_of_ints;
     if (ints) {
         rows_of_ints.reset(new FrTensor(FrTensor::folded_from_ints(ints, size, eval_point, (size / layer_num) / (N * com_scale),
-                                                                    Log2(N * com_scale), N * com_scale)));
+                                                                    Log2(N * com_scale), N * com_scale, OnDefaultStream())));
     } else {
         tensor_in->partial_eval(size, eval_point, (size / layer_num) / (N * com_scale), Log2(N * com_scale), N * com_scale);
     }
@@ -458,12 +459,12 @@ Hyrax_proof Hyrax::open_impl(FrTensor* tensor_in, const int* ints, const std::ve
     tensor.partial_eval(new_N, eval_point, new_N, 0, 1);
     Fr result = grape_host::download(tensor.gpu_data);
 
-    FrTensor z(new_N);
+    FrTensor z(new_N, OnDefaultStream());
     z = x;
     z *= c;
     z += d;
 
-    FrTensor d_fold(d);                         // folded in place: a copy, the commitment may still be reading d
+    FrTensor d_fold(d, OnDefaultStream());                         // folded in place: a copy, the commitment may still be reading d
     d_fold.partial_eval(d_fold.size, eval_point, new_N, 0, 1);
     Fr sum_ad = grape_host::download(d_fold.gpu_data);
     bn128 commit_ad = multiple_of_G(sum_ad);
@@ -496,8 +497,8 @@ bool Hyrax::verify(Hyrax_proof& proof, jacob_t* commitment, const std::vector<Fr
     // and their doubling chain here.  (Folding fewer variables than the rows need leaves the first 2^variables rows.)
     const std::vector<Fr> outer(eval_point.begin() + inner, eval_point.end());
     const uint used = outer.size() < 32 && ((uint64_t)1 << outer.size()) < rows ? 1u << outer.size() : rows;
-    FrTensor pyramid((uint)grape_eq_pyramid_elems((uint)outer.size()));
-    fr_t* d_outer = grape_host::upload(outer);
+    FrTensor pyramid((uint)grape_eq_pyramid_elems((uint)outer.size()), OnDefaultStream());
+    fr_t* d_outer = grape_host::upload(outer, OnDefaultStream());
     check(grape_eq_pyramid(W(pyramid.gpu_data), W(d_outer), (uint)outer.size(), nullptr), "grape_eq_pyramid");
     grape_free_on_default(d_outer);
     fr_t* const weights = pyramid.gpu_data + (((size_t)1 << outer.size()) - 1);
@@ -507,7 +508,7 @@ bool Hyrax::verify(Hyrax_proof& proof, jacob_t* commitment, const std::vector<Fr
     check(grape_g1_msm_windows(W(d_windows), W(commitment), W(weights), used, nullptr), "grape_g1_msm_windows");
     // com(z) on the device
     std::vector<Fr> zv(proof.z, proof.z + new_N);
-    FrTensor z = FrTensor::from_host(zv);
+    FrTensor z = FrTensor::from_host(zv, OnDefaultStream());
     affine_t* com_z_dev = nullptr;
     check(grape_malloc_on_default((void**)&com_z_dev, sizeof(affine_t)), "grape_malloc");
     commit_fr_rows(com_z_dev, z.gpu_data, new_N, new_N, false);

@@ -4,6 +4,7 @@
 #include "../../include/grape_hip.h"
 
 using grape_host::check;
+using grape_host::OnDefaultStream;
 static inline uint32_t* W(fr_t* p) { return reinterpret_cast<uint32_t*>(p); }
 static inline const uint32_t* W(const fr_t* p) { return reinterpret_cast<const uint32_t*>(p); }
 
@@ -76,7 +77,7 @@ Fr matmul_sumcheck_phase1(FrTensor& A, FrTensor& B, FrTensor& a, FrTensor& b, Fr
     if (size != (K << rounds)) throw std::runtime_error("matmul_phase1: the batch extent must be a power of two");
     const std::vector<Fr> us = download_vec(u - rounds, rounds), vs = download_vec(v - rounds, rounds);
     EqPyramid eq(u - rounds, rounds - 1);
-    FrTensor sums(3 * rounds);
+    FrTensor sums(3 * rounds, OnDefaultStream());
     uint in = size;
     for (uint i = 0; i < rounds; i++) {
         const uint out = in / 2;
@@ -117,13 +118,13 @@ void matmul_sumcheck_phase2(FrTensor& A, FrTensor& B, FrTensor& a, FrTensor& b, 
     // The challenges are known before the first round, so all rounds are queued back to back,
     // each leaving its three sums in its own slot, and read with one copy at the end (the
     // reference copies and synchronises after every round).
-    FrTensor sums(3 * rounds);
+    FrTensor sums(3 * rounds, OnDefaultStream());
     // Long rounds (2^16 index pairs and more) are bound by their limb products, and one of the three
     // per pair can go when the round is given the running claim: p(0) + p(1) = claim fixes the middle
     // coefficient.  The claim the kernels chain is the one of the bare sums (without eq_accumulate).
     fr_t* d_claim = nullptr;
     if (outputsize >= kClaimRoundMinOut && !(eq_accumulate == Fr::zero())) {
-        d_claim = grape_host::upload(std::vector<Fr>{claim * eq_accumulate.inverse()});
+        d_claim = grape_host::upload(std::vector<Fr>{claim * eq_accumulate.inverse()}, OnDefaultStream());
     }
     struct Release {
         fr_t*& p;
@@ -173,7 +174,8 @@ struct Operand {
             consumed->partial_eval(size, x, c, id, gap);
             return *consumed;
         }
-        own.reset(new FrTensor(kept ? FrTensor::folded_from(kept, size, x, c, id, gap) : FrTensor::folded_from_ints(ints, size, x, c, id, gap)));
+        own.reset(kept ? new FrTensor(FrTensor::folded_from(kept, size, x, c, id, gap, OnDefaultStream()))
+                       : new FrTensor(FrTensor::folded_from_ints(ints, size, x, c, id, gap, OnDefaultStream())));
         return *own;
     }
 };
@@ -182,7 +184,7 @@ struct Operand {
 std::pair<Fr, Fr> matmul_short_rounds(FrTensor& A, FrTensor& B, int L, int K, const Fr* u, const Fr* v, const fr_t* U, const fr_t* V, Fr& claim,
                                       Fr& eq_accumulate, SumcheckTranscript* transcript) {
     const uint phase1 = Log2((uint)L), rounds = phase1 + Log2((uint)K);
-    FrTensor sums(3 * rounds + 2);
+    FrTensor sums(3 * rounds + 2, OnDefaultStream());
     grape_short_rounds_args a{};
     a.kind = GRAPE_SHORT_PAIR;
     a.size = (uint)L * (uint)K;
@@ -233,8 +235,8 @@ std::pair<Fr, Fr> prove_matmul_impl(Operand A_op, Operand B_op, int L, int N, in
     const uint lu = Log2((uint)L) + Log2((uint)N) + Log2((uint)M);
     if (L < 1 || N < 1 || M < 1 || K < 1 || Log2((uint)(L * N * M)) != lu || u.size() < lu || v.size() < Log2((uint)(L * K)))
         throw std::runtime_error("prove_matmul: Incompatible dimensions");
-    fr_t* U = grape_host::upload(u);
-    fr_t* V = grape_host::upload(v);
+    fr_t* U = grape_host::upload(u, OnDefaultStream());
+    fr_t* V = grape_host::upload(v, OnDefaultStream());
     std::pair<Fr, Fr> ret;
     try {
         FrTensor& A = A_op.fold((uint)(L * N * K), U, N, Log2(M), K);
@@ -244,7 +246,7 @@ std::pair<Fr, Fr> prove_matmul_impl(Operand A_op, Operand B_op, int L, int N, in
             ret = matmul_short_rounds(A, B, L, K, u.data() + Log2(L * N * M), v.data() + Log2(L * K), U + Log2(L * N * M), V + Log2(L * K), claim,
                                       eq_accumulate, transcript);
         } else {
-            FrTensor a(1), b(1), c(1);      // the reference's coefficient arrays (src/prove.cu:190-192): not used by the fused rounds
+            FrTensor a(1, OnDefaultStream()), b(1, OnDefaultStream()), c(1, OnDefaultStream());      // the reference's coefficient arrays (src/prove.cu:190-192): not used by the fused rounds
             eq_accumulate = matmul_sumcheck_phase1(A, B, a, b, c, U + Log2(L * N * M), V + Log2(L * K), K, K * L, claim, transcript);
             matmul_sumcheck_phase2(A, B, a, b, c, V + Log2(K), K, claim, eq_accumulate, transcript);
             ret.first = grape_host::download(A.gpu_data);
@@ -319,7 +321,7 @@ static Fr eleMul_rounds(fr_t* Aw, fr_t* Bw, const fr_t* A, const fr_t* B, fr_t* 
     const bool padded = second_size != row_pad;
     const uint low = padded ? lg_row : kSplitLow;
     const EqWeights eq(u - rounds, rounds - 1, low, padded && lg_row > kLongestPrefix ? rounds : kLongestPrefix);
-    FrTensor sums(3 * rounds + 2);
+    FrTensor sums(3 * rounds + 2, OnDefaultStream());
     // the tables of all challenges' multiples, and every long round's partial sums until one launch finishes them all
     std::vector<grape_wround_args> queued;
     std::vector<std::unique_ptr<DeviceBuf>> partials;
@@ -399,8 +401,8 @@ Fr eleMul_sumcheck(FrTensor& A, FrTensor& B, FrTensor& a, FrTensor& b, FrTensor&
 
 static std::pair<Fr, Fr> prove_eleMul_impl(fr_t* Aw, fr_t* Bw, const fr_t* A, const fr_t* B, int L, int M, int N, const std::vector<Fr>& u,
                                            const std::vector<Fr>& v, Fr& claim, SumcheckTranscript* transcript) {
-    fr_t* U = grape_host::upload(u);
-    fr_t* V = grape_host::upload(v);
+    fr_t* U = grape_host::upload(u, OnDefaultStream());
+    fr_t* V = grape_host::upload(v, OnDefaultStream());
     std::pair<Fr, Fr> ret;
     try {
         const uint size = (uint)(L * M * N);
@@ -425,7 +427,7 @@ std::pair<Fr, Fr> prove_eleMul(FrTensor& A, FrTensor& B, int L, int M, int N, co
 std::pair<Fr, Fr> prove_eleMul(const fr_t* device_A, const fr_t* device_B, int L, int M, int N, const std::vector<Fr> u,
                                const std::vector<Fr> v, Fr& claim, SumcheckTranscript* transcript) {
     const uint size = (uint)(L * M * N);
-    FrTensor Aw(size / 2 + 1), Bw(size / 2 + 1);
+    FrTensor Aw(size / 2 + 1, OnDefaultStream()), Bw(size / 2 + 1, OnDefaultStream());
     return prove_eleMul_impl(Aw.gpu_data, Bw.gpu_data, device_A, device_B, L, M, N, u, v, claim, transcript);
 }
 
@@ -447,13 +449,13 @@ Fr combine_claims(FrTensor& X, const std::vector<Fr>& claims, const std::vector<
     const uint rounds = (uint)v.size();
     std::vector<Fr> eq_accumulate(num, Fr::one());
     if (rounds > 0 && num > 0) {
-        fr_t* d_v = grape_host::upload(v);
+        fr_t* d_v = grape_host::upload(v, OnDefaultStream());
         std::vector<std::unique_ptr<EqPyramid>> eq;
         std::vector<fr_t*> d_u(num, nullptr);
-        FrTensor sums(2 * num * rounds);
+        FrTensor sums(2 * num * rounds, OnDefaultStream());
         try {
             for (uint j = 0; j < num; j++) {
-                d_u[j] = grape_host::upload(u[j]);
+                d_u[j] = grape_host::upload(u[j], OnDefaultStream());
                 eq.emplace_back(new EqPyramid(d_u[j], rounds - 1));
             }
             uint in = size;

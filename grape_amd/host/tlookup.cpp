@@ -6,6 +6,7 @@
 #include "../../include/grape_hip.h"
 
 using grape_host::check;
+using grape_host::OnDefaultStream;
 static inline uint32_t* W(fr_t* p) { return reinterpret_cast<uint32_t*>(p); }
 static inline const uint32_t* W(const fr_t* p) { return reinterpret_cast<const uint32_t*>(p); }
 
@@ -160,7 +161,7 @@ bool tLookup::commit_A_by_occupancy(FrTensor& A, uint D, uint msm_size, Hyrax& h
             const uint n_hot = (uint)info[0];
             cold = info[1];
             if (n_hot != 0) {
-                FrTensor Bhot(n_hot);
+                FrTensor Bhot(n_hot, OnDefaultStream());
                 check(grape_fr_gather(W(Bhot.gpu_data), W(B.gpu_data), d_list, n_hot, nullptr), "grape_fr_gather");
                 hot_table_ = hyrax.build_scaled_table(Bhot, rowlen);
             }
@@ -189,7 +190,7 @@ bool tLookup::commit_A_by_occupancy(FrTensor& A, uint D, uint msm_size, Hyrax& h
             // the elements without a table row: queued per row and committed as full-width scalars
             com_cold = hyrax.commit_sparse_affine(A, d_hot, D, msm_size, cold);
             if (!com_cold) {
-                FrTensor Acold(D);
+                FrTensor Acold(D, OnDefaultStream());
                 check(grape_fr_mask_cold(W(Acold.gpu_data), W(A.gpu_data), d_hot, D, nullptr), "grape_fr_mask_cold");
                 com_cold = hyrax.commit_affine(Acold, D, msm_size);
             }
@@ -307,7 +308,7 @@ void tLookup::start_weights(uint D) {
     E_ready_.reset();
     if (u_ready_.size() != nu) return;          // run() reports the mismatch
     const WeightPlan plan(nu, T.size);
-    E_ready_.reset(new FrTensor((uint)plan.elems(), FrTensor::OnAnyStream()));
+    E_ready_.reset(new FrTensor((uint)plan.elems()));       // not OnDefaultStream: first written on the second stream
     // the point travels on the second stream too: on the default stream it would queue behind the pass over the
     // witness, and the pyramid with it
     SideChain side(0);
@@ -377,7 +378,7 @@ Fr tLookup::run(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax& hyrax
 
     // beta is read by kernels on the side streams until the end of the proof: a buffer of its own, not a
     // slot of the ring of grape_host::device_scalar (which is rewritten after 64 further scalars)
-    grape_host::DeviceFr beta_buf(beta);
+    grape_host::DeviceFr beta_buf(beta, OnDefaultStream());
     fr_t* d_beta = beta_buf.get();
     // Commitments of A and m (kept, not dropped).  With the scaled table of a range lookup the
     // commitment of A reads only the indices, so it does not have to finish before the rounds start
@@ -461,7 +462,7 @@ Fr tLookup::run(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax& hyrax
     const bool m_late = m_pending_;
     if (!overlap) timed(commit_all);
 
-    FrTensor Bm(B);
+    FrTensor Bm(B, OnDefaultStream());
     if (!m_late) Bm *= m;
     Fr alpha_sq = alpha * alpha;
     Fr claim = alpha + alpha_sq;
@@ -478,8 +479,8 @@ Fr tLookup::run(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax& hyrax
         SideChain early(0);
         SideChain::order(nullptr, early.stream);     // the default stream meets the finished pyramid
     } else {
-        E_own.reset(new FrTensor((uint)plan.elems()));
-        fr_t* d_u = grape_host::upload(u);
+        E_own.reset(new FrTensor((uint)plan.elems(), OnDefaultStream()));
+        fr_t* d_u = grape_host::upload(u, OnDefaultStream());
         plan.build(E_own->gpu_data, d_u, nullptr);
         grape_free_on_default(d_u);
     }
@@ -493,17 +494,17 @@ Fr tLookup::run(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax& hyrax
     // (Three more slots travel with them: the sum of B * m, the last element left of S - the value the proof
     // returns - and the two digit-range flags of the commitments queued beside the rounds.)
     const size_t n_sums = 13 * (size_t)(rounds ? rounds : 1);
-    FrTensor sums((uint)n_sums + 3);
+    FrTensor sums((uint)n_sums + 3, OnDefaultStream());
     fr_t* const d_sum_Bm = sums.gpu_data + n_sums;
     fr_t* const d_S_last = sums.gpu_data + n_sums + 1;
     int* const d_flags = reinterpret_cast<int*>(sums.gpu_data + n_sums + 2);
     if (!m_late) check(grape_fr_sum(W(d_sum_Bm), W(Bm.gpu_data), N, nullptr), "grape_fr_sum");
-    fr_t* d_v = grape_host::upload(v);
+    fr_t* d_v = grape_host::upload(v, OnDefaultStream());
     Fr S_last;
     char* long_work = nullptr;             // partial sums of the long rounds and the challenges' tables (overlap mode)
     // phase 2 binds copies where its rounds work in place; T, B, m of this object stay intact
     const bool table_long = N / 2 >= kLongRoundPairs;
-    FrTensor Bw(table_long ? N : 1), Tw(table_long ? N : 1), mw(table_long ? N : 1);
+    FrTensor Bw(table_long ? N : 1, OnDefaultStream()), Tw(table_long ? N : 1, OnDefaultStream()), mw(table_long ? N : 1, OnDefaultStream());
     auto copy_table = [&](FrTensor& to, const FrTensor& from, grape_stream_t st) {
         if (table_long) check(grape_memcpy_d2d(to.gpu_data, from.gpu_data, sizeof(fr_t) * (size_t)N, st), "grape_memcpy_d2d");
     };
@@ -893,7 +894,7 @@ Fr tLookupRangeMapping::prove(FrTensor& S_in, FrTensor& S_out, FrTensor& A, cons
         make_index(S_in, low);
     }
     index_to_m(D, low);                       // what prep(S_in) computes, from the shared indices
-    FrTensor S(1u << Log2(D));
+    FrTensor S(1u << Log2(D), OnDefaultStream());
     S.set_size(D);
     check(grape_fr_axpy(W(S.gpu_data), W(S_in.gpu_data), W(grape_host::device_scalar(r)), W(S_out.gpu_data), D, nullptr), "grape_fr_axpy");
     if (D != (1u << Log2(D))) {
@@ -943,7 +944,7 @@ Fr tLookupRangeMapping::prove(const int* device_int_S_in, const int* device_int_
     a_ready_ = false;
     // index, the check S_out = f(S_in) against the integer table, A = B[index] and the combined witness S_in + r * S_out in one
     // pass over the integers
-    FrTensor S(D);
+    FrTensor S(D, OnDefaultStream());
     make_index_and_A_from_ints(device_int_S_in, device_int_S_out, D, low, S, A, d_map_int_, &r, true);
     index_to_m(D, low);
     Fr ret;
@@ -963,7 +964,7 @@ namespace {
 // (tLookup_poly_kernel, src/tlookup.cu:64-81), each evaluated at the remaining variables
 struct PolyArrays {
     FrTensor c0, c1, c2;
-    explicit PolyArrays(uint n) : c0(n ? n : 1), c1(n ? n : 1), c2(n ? n : 1) {
+    explicit PolyArrays(uint n) : c0(n ? n : 1, OnDefaultStream()), c1(n ? n : 1, OnDefaultStream()), c2(n ? n : 1, OnDefaultStream()) {
         c0.set_size(n);
         c1.set_size(n);
         c2.set_size(n);
@@ -1021,7 +1022,7 @@ Fr tLookup_phase2(const Fr& claim, const FrTensor& A, const FrTensor& S, const F
                   const Fr& alpha_, const Fr& beta, const Fr& inv_size_ratio, const Fr& alpha_sq, const std::vector<Fr>& u,
                   const std::vector<Fr>& v2) {
     // the reference recurses on fresh half-size tensors; here one set of working copies is bound in place
-    FrTensor a(A), s(S), b(B), t(T), mm(m);
+    FrTensor a(A, OnDefaultStream()), s(S, OnDefaultStream()), b(B, OnDefaultStream()), t(T, OnDefaultStream()), mm(m, OnDefaultStream());
     Fr running = claim, weight = alpha_, weight_sq = alpha_sq;
     std::vector<Fr> uu(u), vv(v2);
     while (!vv.empty()) {

@@ -62,9 +62,9 @@ int grape_free(void *d_ptr);
 int grape_alloc_cache_release(size_t *bytes_released);
 /* The same for blocks that only the default stream works on, between the allocation and the free (work on other streams
  * that was ordered before the free counts as the default stream's): such a block goes to its next owner in stream order,
- * without an event or a wait.  The tensors of the host classes.  While a stream is about that the library cannot vouch for
- * - one that a caller brought, or one of grape_stream_create that is not declared internal - these behave like
- * grape_malloc and grape_free. */
+ * without an event or a wait.  For memory that stays inside the code that asks for it (what the host classes keep to themselves,
+ * not the tensors they hand out).  While a stream is about that the library cannot vouch for - one that a caller brought, or
+ * one of grape_stream_create that is not declared internal - these behave like grape_malloc and grape_free. */
 int grape_malloc_on_default(void **d_ptr, size_t bytes);
 int grape_free_on_default(void *d_ptr);
 /* Host to device, ordered like any other work on `stream`; the host buffer may be reused as soon as

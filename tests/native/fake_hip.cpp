@@ -20,7 +20,7 @@ std::recursive_mutex mu;
 std::map<const void*, Seen> streams;                     // of each stream: what its next item is ordered behind, itself included
 Seen host;                                               // what the host has waited for
 std::map<const char*, Alloc> memory;
-unsigned long launches = 0, copies = 0;
+unsigned long launches = 0, copies = 0, waits = 0;
 thread_local int device = 0;
 char symbol[1 << 24];
 
@@ -57,6 +57,8 @@ unsigned long fake_unjoined() {
 }
 unsigned long fake_launches() { return launches; }
 unsigned long fake_copies() { return copies; }
+// waits of the host for a stream, an event or the device
+unsigned long fake_waits() { return waits; }
 void fake_queue(const void* stream) { Lock l(mu); push(stream); }
 
 // ---- the runtime
@@ -81,6 +83,7 @@ hipError_t hipMalloc(void** p, size_t bytes) {
 }
 hipError_t hipDeviceSynchronize() {
     Lock l(mu);
+    waits++;
     for (auto& s : streams) merge(host, s.second);
     return hipSuccess;
 }
@@ -125,13 +128,13 @@ hipError_t hipFuncSetAttribute(const void*, hipFuncAttribute, int) { return hipS
 
 hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { *s = (hipStream_t)malloc(16); return hipSuccess; }
 hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
-hipError_t hipStreamSynchronize(hipStream_t s) { Lock l(mu); merge(host, streams[s]); return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t s) { Lock l(mu); waits++; merge(host, streams[s]); return hipSuccess; }
 hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned) { Lock l(mu); merge(streams[s], *(Seen*)e); return hipSuccess; }
 hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { *e = (hipEvent_t) new Seen(); return hipSuccess; }
 hipError_t hipEventCreate(hipEvent_t* e) { return hipEventCreateWithFlags(e, 0); }
 hipError_t hipEventDestroy(hipEvent_t e) { delete (Seen*)e; return hipSuccess; }
 hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) { Lock l(mu); *(Seen*)e = streams[s]; return hipSuccess; }
-hipError_t hipEventSynchronize(hipEvent_t e) { Lock l(mu); merge(host, *(Seen*)e); return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t e) { Lock l(mu); waits++; merge(host, *(Seen*)e); return hipSuccess; }
 hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) { *ms = 0; return hipSuccess; }
 
 thread_local struct { dim3 grid, block; size_t shared; hipStream_t stream; } config;

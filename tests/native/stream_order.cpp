@@ -4,6 +4,7 @@
 #include <cstring>
 #include <functional>
 #include <map>
+#include <memory>
 #include <string>
 #include "../../include/grape_hip.h"
 #include "../../grape_amd/host/hyrax.hpp"
@@ -16,6 +17,7 @@ unsigned long fake_unjoined();
 unsigned long fake_launches();
 unsigned long fake_copies();
 void fake_queue(const void* stream);
+unsigned long fake_waits();
 }
 
 static int failures = 0;
@@ -52,9 +54,42 @@ static void refused_lookup() {
     expect(fake_unjoined() == 0, "no stream is left with work that nothing waits for");
 }
 
+// Memory that a program gets is idle when it gets it, whatever was queued on it before: on the default stream, and - while the
+// library itself has no further stream - on one it has never seen.  So the program may use it on a stream of its own at once.
+static void tensor_memory_is_idle() {
+    const uint n = 5000;
+    FrTensor x(n);
+    std::vector<Fr> host(n, Fr::one());
+    int* ints = reinterpret_cast<int*>(device_points(n));
+    const int unseen = 0;
+    const std::map<std::string, std::function<std::shared_ptr<void>()>> sources = {
+        {"a tensor", [&] { return std::make_shared<FrTensor>(n); }},
+        {"a copy", [&] { return std::make_shared<FrTensor>(x); }},
+        {"embedded integers", [&] { return std::make_shared<FrTensor>(n, ints); }},
+        {"a tensor from the host", [&] { return std::make_shared<FrTensor>(FrTensor::from_host(host)); }},
+        {"row sums", [&] { return std::make_shared<FrTensor>(x.sum(n, 1)); }},
+        {"a vector of challenges", [&] { return std::shared_ptr<void>(grape_host::upload(host), [](void* p) { grape_free(p); }); }},
+        {"a fold", [&] { return std::make_shared<FrTensor>(FrTensor::folded_from_ints(ints, n, x.gpu_data, 8, 0, n / 8)); }},
+        {"a scalar", [&] { return std::make_shared<grape_host::DeviceFr>(host[0]); }},
+    };
+    for (const auto& s : sources) {
+        s.second();                                          // leaves a block of that size behind
+        grape_host::check(grape_stream_sync(nullptr), "sync");
+        std::shared_ptr<void> first = s.second();
+        grape_host::check(grape_memset_zero(x.gpu_data, 32, nullptr), "grape_memset_zero");     // stands for work on the block
+        fake_queue(&unseen);
+        const unsigned long on_default = fake_pending(nullptr);
+        first.reset();
+        const unsigned long before = fake_waits();
+        const std::shared_ptr<void> second = s.second();
+        expect(on_default > 0 && fake_waits() > before && fake_pending(&unseen) == 0, s.first.c_str());
+    }
+}
+
 int main(int argc, char** argv) {
     const std::map<std::string, std::function<void()>> scenarios = {
         {"refused_lookup", refused_lookup},
+        {"tensor_memory_is_idle", tensor_memory_is_idle},
     };
     auto it = scenarios.find(argc > 1 ? argv[1] : "");
     if (it == scenarios.end()) return 2;
