@@ -1,5 +1,6 @@
 #include "hyrax.hpp"
 #include <cstdlib>
+#include <algorithm>
 #include <cassert>
 #include <map>
 #include <utility>
@@ -70,8 +71,7 @@ bool Hyrax::ensure_table(WideTable& t, uint rowlen, uint c, uint nw, uint K) {
     if (t.d && t.ngen >= rowlen && t.c == c && t.nw == nw) return true;
     size_t bytes = grape_g1_wide_table_bytes(rowlen, nw, K);
     // against what every other table of this object holds (the one being replaced gives its bytes back)
-    const size_t others = table_bytes_in_use() - (t.d ? grape_g1_wide_table_bytes(t.ngen, t.nw, t.K) : 0);
-    if (others + bytes > table_budget_) return false;
+    if (!make_room(bytes, t.d ? grape_g1_wide_table_bytes(t.ngen, t.nw, t.K) : 0)) return false;
     if (rowlen > npoints) throw std::runtime_error("row longer than the generator set");
     grape_free(t.d);
     t = WideTable();
@@ -162,12 +162,27 @@ affine_t* Hyrax::commit_affine_i32(int* tensor, uint size, uint N, int* d_flag, 
     return out;
 }
 
+size_t Hyrax::strided_bytes() const {
+    return fr_strided_.d ? grape_g1_wide_table_bytes(fr_strided_.ngen, fr_strided_.nsets, 1u << (fr_strided_.c - 1)) : 0;
+}
+// without a strided table that gives way (make_room)
 size_t Hyrax::table_bytes_in_use() const {
     size_t used = scaled_bytes_;
     for (const WideTable* t : {&int16_table_, &int16x2_table_, &int32_table_, &fr_table_})
         if (t->d) used += grape_g1_wide_table_bytes(t->ngen, t->nw, t->K);
-    if (fr_strided_.d) used += grape_g1_wide_table_bytes(fr_strided_.ngen, fr_strided_.nsets, 1u << (fr_strided_.c - 1));
-    return used;
+    return fr_strided_.spare ? used : used + strided_bytes();
+}
+// Is there room in the budget for a table of `bytes` that replaces one of `replaced` bytes?  A strided table that only sparse
+// commitments asked for goes if it stands in the way: it saves them a fifth to a half of their additions, while a scaled or int16
+// table that is not there costs 16 additions instead of one, or 2.
+bool Hyrax::make_room(size_t bytes, size_t replaced) {
+    const size_t used = table_bytes_in_use() - replaced;
+    if (used + bytes > table_budget_) return false;
+    if (fr_strided_.spare && used + strided_bytes() + bytes > table_budget_) {
+        grape_free(fr_strided_.d);
+        fr_strided_ = StridedTable();
+    }
+    return true;
 }
 
 // A per-window table for full-width scalars (every window has its own set of multiples, so a
@@ -198,11 +213,16 @@ bool Hyrax::ensure_fr_table(uint rowlen, bool build) {
 // tables.  4096 generators: c = 16, J = 4, 4 sets, 69 GB, 16 additions (a per-window table of the
 // same bytes has c = 14 and 19); 65536 generators: c = 13, J = 10; 262144: c = 11, J = 12, against
 // 32 additions plus a doubling chain per row for the reference's byte windows.
-bool Hyrax::ensure_strided_table(uint rowlen, bool build) {
-    if (fr_strided_.d && fr_strided_.ngen >= rowlen) return true;
+// With worth_ms it is built where that takes no longer than worth_ms, and marked as a table that gives way to others; once
+// a call that builds at any price has found it in place it stays.
+bool Hyrax::ensure_strided_table(uint rowlen, bool build, const double* worth_ms) {
+    if (fr_strided_.d && fr_strided_.ngen >= rowlen) {
+        if (build && !worth_ms) fr_strided_.spare = false;
+        return true;
+    }
     if (!build) return false;
     if (rowlen > npoints) throw std::runtime_error("row longer than the generator set");
-    const size_t used = table_bytes_in_use() - (fr_strided_.d ? grape_g1_wide_table_bytes(fr_strided_.ngen, fr_strided_.nsets, 1u << (fr_strided_.c - 1)) : 0);
+    const size_t used = table_bytes_in_use() - (fr_strided_.spare ? 0 : strided_bytes());
     size_t cap = table_budget_ / 2;
     if (used + cap > table_budget_) cap = table_budget_ > used ? table_budget_ - used : 0;
     // the cheapest table over `ngen` generators within the cap: cost per scalar, c, J, number of sets
@@ -236,6 +256,9 @@ bool Hyrax::ensure_strided_table(uint rowlen, bool build) {
     }
     const uint bc = pick.c, bj = pick.J, bs = pick.nsets;
     if (bc == 0) return false;
+    // 64 GiB in 92 ms, 48 in 72 (4096 generators)
+    const double build_ms = 1.35e-9 * (double)grape_g1_wide_table_bytes(ngen, bs, 1u << (bc - 1));
+    if (worth_ms && (build_ms > *worth_ms || (fr_strided_.d && !fr_strided_.spare))) return false;
     grape_free(fr_strided_.d);
     fr_strided_ = StridedTable();
     check(grape_malloc((void**)&fr_strided_.d, grape_g1_wide_table_bytes(ngen, bs, 1u << (bc - 1))), "grape_malloc");
@@ -244,6 +267,7 @@ bool Hyrax::ensure_strided_table(uint rowlen, bool build) {
     fr_strided_.c = bc;
     fr_strided_.J = bj;
     fr_strided_.nsets = bs;
+    fr_strided_.spare = worth_ms != nullptr;
     return true;
 }
 
@@ -297,7 +321,7 @@ affine_t* Hyrax::build_scaled_table(const FrTensor& scalars, uint ncols) {
     size_t bytes = grape_g1_wide_table_bytes(ncols, 1, scalars.size);   // one entry per (scalar, column)
     if (table_bytes_in_use() + bytes > table_budget_) return nullptr;      // before the per-window table is built for nothing
     if (!ensure_fr_table(ncols)) return nullptr;
-    if (table_bytes_in_use() + bytes > table_budget_) return nullptr;
+    if (!make_room(bytes, 0)) return nullptr;
     affine_t* out = nullptr;
     check(grape_malloc((void**)&out, bytes), "grape_malloc");
     check(grape_g1_scaled_table_gen(W(out), W(scalars.gpu_data), scalars.size, ncols, W(fr_table_.d), fr_table_.ngen, fr_table_.c,
@@ -344,11 +368,23 @@ affine_t* Hyrax::commit_sparse_affine(FrTensor& tensor, int* skip, uint size, ui
     check_shape(size, N);
     const uint rowlen = N * com_scale;
     const uint rows = size / rowlen;
-    // From 512 live elements a row the strided table is the better one: 16 to 18 additions per element instead of 20, against
-    // 64 partial sums per residue and row (2^25 elements on rows of 11008 padded to 16384, 67 % live: 56 against 92 ms; 27
-    // live elements a row: the queue of half waves over the per-window table).  It is built for a tensor at least a quarter
-    // of which is live - the build costs what 2^24 live elements save.
-    if (live >= (uint64_t)512 * rows && rows > 1 && ensure_strided_table(rowlen, 4 * live >= size)) {
+    // From 512 live elements a row the strided table is the better one: 16 to 18 additions per element instead of 20 and four waves
+    // or more on a row instead of one, against 64 partial sums per residue and row (64 GiB table; rows of 11008 padded to
+    // 16384, 67 % live: 2^25 elements 53 against 93 ms, 2^21 elements 5.3 against 13.3; a quarter live, scattered: 20.6 against 26.3
+    // and 1.8 against 3.8; 27 live elements a row: the queue of half waves over the per-window table).  Building it takes as long as
+    // two such proofs of 2^25 elements save, and its memory: it is built once the proofs of this object would have saved as
+    // much, so that a program with a few short proofs never pays for it.  Saved are 1.7 ns a live element where the
+    // rows fill the chip, and 2.5 us for each live element of a row where the longest row is what takes the time.
+    bool strided = false;
+    if (live >= (uint64_t)512 * rows && rows > 1) {
+        strided = ensure_strided_table(rowlen, false);
+        if (!strided) {
+            sparse_saving_ms_ += std::max(1.7e-6 * (double)live, 2.5e-3 * (double)live / rows);
+            strided = ensure_strided_table(rowlen, true, &sparse_saving_ms_);
+            if (strided) sparse_saving_ms_ = 0;
+        }
+    }
+    if (strided) {
         const StridedTable& t = fr_strided_;
         affine_t* out = nullptr;
         check(grape_malloc((void**)&out, sizeof(affine_t) * (size_t)rows), "grape_malloc");

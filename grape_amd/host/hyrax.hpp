@@ -91,7 +91,8 @@ public:
     // Upper bound for the wide fixed-base tables this object may build (default 128 GiB of the 288 GB; GRAPE_TABLE_BUDGET_GIB overrides).  When a
     // table would not fit, commitments go through the reference-format table instead.
     void set_table_budget(size_t bytes) { table_budget_ = bytes; }
-    // bytes of that budget not taken by tables that exist now
+    // bytes of that budget not taken by tables that exist now (a strided table that sparse commitments built for themselves is not
+    // counted: it goes when another table needs its place)
     size_t table_bytes_free() const {
         const size_t used = table_bytes_in_use();
         return used < table_budget_ ? table_budget_ - used : 0;
@@ -106,11 +107,15 @@ private:
     struct StridedTable {
         affine_t* d = nullptr;
         uint ngen = 0, c = 0, J = 0, nsets = 0;
+        bool spare = false;             // gives way to any other table (make_room)
     };
     bool ensure_table(WideTable& t, uint rowlen, uint c, uint nw, uint K);
     bool ensure_fr_table(uint rowlen, bool build = true);       // small per-window table (scaled-table builds)
-    bool ensure_strided_table(uint rowlen, bool build = true);  // the table full-width commitments go through
+    bool ensure_strided_table(uint rowlen, bool build = true, const double* worth_ms = nullptr);  // the table full-width commitments go through
     size_t table_bytes_in_use() const;
+    size_t strided_bytes() const;
+    bool make_room(size_t bytes, size_t replaced);
+    double sparse_saving_ms_ = 0;                               // what a strided table would have saved the sparse commitments so far
     // commits `size` full-width scalars in rows of rowlen into out[0 .. size/rowlen)
     // d_flag (single rows through the per-window table only): queued without waiting, digit-range check left in *d_flag;
     // returns whether it was queued that way (false: the call has waited and checked)

@@ -55,6 +55,13 @@ unsigned long fake_unjoined() {
     }
     return n;
 }
+// device memory allocated now
+unsigned long fake_bytes() {
+    Lock l(mu);
+    unsigned long n = 0;
+    for (auto& a : memory) n += a.second.bytes;
+    return n;
+}
 unsigned long fake_launches() { return launches; }
 unsigned long fake_copies() { return copies; }
 // waits of the host for a stream, an event or the device

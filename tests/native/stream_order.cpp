@@ -18,6 +18,7 @@ unsigned long fake_launches();
 unsigned long fake_copies();
 void fake_queue(const void* stream);
 unsigned long fake_waits();
+unsigned long fake_bytes();
 }
 
 static int failures = 0;
@@ -86,10 +87,44 @@ static void tensor_memory_is_idle() {
     }
 }
 
+// The table that sparse commitments go through where rows hold many elements: not built for a short proof or two, built once
+// such proofs have come up often enough, and never in the way of another table.
+static void sparse_commitment_table() {
+    const uint cols = 4096, D = 1u << 21;
+    bn128 G = bn128::one();
+    Hyrax hyrax(1, cols, device_points(256 * cols), G, 1);
+    hyrax.set_table_budget((size_t)96 << 30);
+    expect(hyrax.prepare_scaled_tables(cols), "the per-window table fits");
+    FrTensor A(D);
+    int* skip = reinterpret_cast<int*>(device_points(D / 16));
+    auto prove = [&] { grape_free(hyrax.commit_sparse_affine(A, skip, D, cols, D / 2)); };
+    const unsigned long start = fake_bytes();
+    prove();
+    prove();
+    expect(fake_bytes() - start < (1ul << 30), "two short proofs build no table");
+    for (int i = 0; i < 40; i++) prove();
+    const unsigned long built = fake_bytes();
+    expect(built - start > (8ul << 30), "forty do");
+    FrTensor B(1u << 16);
+    affine_t* scaled = hyrax.build_scaled_table(B, cols);
+    expect(scaled != nullptr, "a lookup's table still fits");
+    grape_free(hyrax.commit_affine(skip, 2 * cols, cols));
+    expect(fake_bytes() - start > (47ul << 30), "and the one for 16-bit integers");
+    Hyrax::release_scaled_table(scaled);
+    // a table that a commitment of full rows finds in place stays
+    Hyrax other(1, cols, hyrax.g_affine, G, 1);
+    other.set_table_budget((size_t)96 << 30);
+    expect(other.prepare_scaled_tables(cols), "the per-window table fits");
+    for (int i = 0; i < 40; i++) grape_free(other.commit_sparse_affine(A, skip, D, cols, D / 2));
+    grape_free(other.commit_affine(A, D, cols));
+    expect(other.table_bytes_free() < (size_t)16 << 30 && other.build_scaled_table(B, cols) == nullptr, "a table in use by others does not give way");
+}
+
 int main(int argc, char** argv) {
     const std::map<std::string, std::function<void()>> scenarios = {
         {"refused_lookup", refused_lookup},
         {"tensor_memory_is_idle", tensor_memory_is_idle},
+        {"sparse_commitment_table", sparse_commitment_table},
     };
     auto it = scenarios.find(argc > 1 ? argv[1] : "");
     if (it == scenarios.end()) return 2;

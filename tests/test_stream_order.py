@@ -20,7 +20,7 @@ def program():
     return EXE
 
 
-@pytest.mark.parametrize("scenario", ["refused_lookup", "tensor_memory_is_idle"])
+@pytest.mark.parametrize("scenario", ["refused_lookup", "tensor_memory_is_idle", "sparse_commitment_table"])
 def test_scenario(program, scenario):
     r = subprocess.run([program, scenario], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr
