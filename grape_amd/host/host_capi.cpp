@@ -84,6 +84,10 @@ static FrTensor tensor_from_device(const uint32_t* d, uint32_t n, uint32_t capac
     grape_host::check(grape_memcpy_d2d(t.gpu_data, d, 32 * (size_t)n, nullptr), "grape_memcpy_d2d");
     return t;
 }
+// field operands that a prover can read where they lie; at any other address (a view into a flat buffer) they are copied first
+static bool kept_in_place(const uint32_t* d_A, const uint32_t* d_B) {
+    return g_input_format == 0 && ((reinterpret_cast<uintptr_t>(d_A) | reinterpret_cast<uintptr_t>(d_B)) & 15) == 0;
+}
 static void put_transcript(const SumcheckTranscript& tr, uint32_t* out, uint32_t* n_rounds) {
     *n_rounds = (uint32_t)tr.rounds.size();
     for (size_t r = 0; r < tr.rounds.size(); r++) {
@@ -118,7 +122,7 @@ int grape_host_prove_matmul(const uint32_t* d_A, const uint32_t* d_B, int L, int
         ProveTimer timer;
         res = prove_matmul(reinterpret_cast<const int*>(d_A), reinterpret_cast<const int*>(d_B), L, N, M, K, vec_from(u, nu), vec_from(v, nv),
                            claim, &tr);
-    } else if (g_input_format == 0) {
+    } else if (kept_in_place(d_A, d_B)) {
         ProveTimer timer;
         res = prove_matmul(reinterpret_cast<const fr_t*>(d_A), reinterpret_cast<const fr_t*>(d_B), L, N, M, K, vec_from(u, nu), vec_from(v, nv),
                            claim, &tr);
@@ -142,7 +146,7 @@ int grape_host_prove_elemul(const uint32_t* d_A, const uint32_t* d_B, int L, int
     Fr claim = fr_from(claim_inout);
     SumcheckTranscript tr;
     std::pair<Fr, Fr> res;
-    if (g_input_format == 0) {
+    if (kept_in_place(d_A, d_B)) {
         ProveTimer timer;
         res = prove_eleMul(reinterpret_cast<const fr_t*>(d_A), reinterpret_cast<const fr_t*>(d_B), L, M, N, vec_from(u, nu), vec_from(v, nv), claim, &tr);
     } else {

@@ -7,6 +7,7 @@
 #include <memory>
 #include <string>
 #include "../../include/grape_hip.h"
+#include "../../grape_amd/host/host_capi.h"
 #include "../../grape_amd/host/hyrax.hpp"
 #include "../../grape_amd/host/prove.hpp"
 #include "../../grape_amd/host/tlookup.hpp"
@@ -120,11 +121,25 @@ static void sparse_commitment_table() {
     expect(other.table_bytes_free() < (size_t)16 << 30 && other.build_scaled_table(B, cols) == nullptr, "a table in use by others does not give way");
 }
 
+// operands of the C calls at addresses that are multiples of 4 only
+static void operands_at_any_address() {
+    uint32_t* at = reinterpret_cast<uint32_t*>(device_points(4096));
+    uint32_t point[8 * 16] = {0}, claim[8] = {0}, transcript[32 * 16], rounds, a[8], b[8];
+    for (int shift = 0; shift < 4; shift++) {
+        const uint32_t *A = at + shift, *B = at + 8 * 4096;
+        expect(grape_host_prove_matmul(A, B, 1, 8, 8, 8, point, 6, point, 3, claim, transcript, &rounds, a, b) == 0, "matrix product, left");
+        expect(grape_host_prove_matmul(B, A, 1, 8, 8, 8, point, 6, point, 3, claim, transcript, &rounds, a, b) == 0, "matrix product, right");
+        expect(grape_host_prove_elemul(A, B, 1, 8, 8, point, 6, point, 6, claim, transcript, &rounds, a, b) == 0, "element product, left");
+        expect(grape_host_prove_elemul(B, A, 1, 8, 8, point, 6, point, 6, claim, transcript, &rounds, a, b) == 0, "element product, right");
+    }
+}
+
 int main(int argc, char** argv) {
     const std::map<std::string, std::function<void()>> scenarios = {
         {"refused_lookup", refused_lookup},
         {"tensor_memory_is_idle", tensor_memory_is_idle},
         {"sparse_commitment_table", sparse_commitment_table},
+        {"operands_at_any_address", operands_at_any_address},
     };
     auto it = scenarios.find(argc > 1 ? argv[1] : "");
     if (it == scenarios.end()) return 2;

@@ -42,3 +42,36 @@ def test_weighted_round_of_kept_operands(ops, in_size, n_out):
     assert torch.equal(A, a) and torch.equal(S, s)
     want = ops.wround2(a, s, None, E, in_size, n_out, v)
     assert torch.equal(sums, want) and torch.equal(Aw, a[:n_out]) and torch.equal(Sw, s[:n_out])
+
+
+@pytest.mark.parametrize("shift", [1, 2, 3])
+def test_provers_take_operands_at_any_address(ops, shift):
+    """views that start 4, 8 or 12 bytes behind a 16-byte boundary: the proofs of the same operands at a boundary"""
+    from gpuutil import rand_fr
+    from grape_amd import _host as host
+    host.load()
+    host.set_input_format("fr")
+
+    def shifted(t):
+        flat = torch.empty(t.numel() + shift, dtype=torch.int32, device="cuda")
+        view = flat[shift:].view(t.shape)
+        view.copy_(t)
+        assert view.data_ptr() % 16 == 4 * shift
+        return view
+
+    n = 16
+    a, b = ops.to_dev(rand_fr(n * n, 720)), ops.to_dev(rand_fr(n * n, 721))
+    u, v = rand_fr(8, 722), rand_fr(8, 723)
+    prod = ops.fr_mul(a, b)
+    claim = host.mle_eval(prod, n * n, u)
+    want = host.prove_elemul(a, b, 1, n, n, u, v, claim)
+    for x, y in ((shifted(a), b), (a, shifted(b)), (shifted(a), shifted(b))):
+        assert all(np.array_equal(p, q) for p, q in zip(want, host.prove_elemul(x, y, 1, n, n, u, v, claim)))
+    # the matrix product's claim is what its proof over operands at a boundary accepts: sum_k A(u_row, k) B(u_col, k)
+    x, y = a.clone(), b.clone()
+    ops.fr_fold(x, n * n, ops.to_dev(u), n, 4, n)
+    ops.fr_fold(y, n * n, ops.to_dev(u), n, 0, n)
+    claim = ops.fr_to_host(ops.fr_sum(ops.fr_mul(x[:n].contiguous(), y[:n].contiguous())))[0]
+    want = host.prove_matmul(a, b, 1, n, n, n, u, v[:4], claim)
+    for x, y in ((shifted(a), b), (a, shifted(b))):
+        assert all(np.array_equal(p, q) for p, q in zip(want, host.prove_matmul(x, y, 1, n, n, n, u, v[:4], claim)))

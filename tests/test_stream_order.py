@@ -20,7 +20,8 @@ def program():
     return EXE
 
 
-@pytest.mark.parametrize("scenario", ["refused_lookup", "tensor_memory_is_idle", "sparse_commitment_table"])
+@pytest.mark.parametrize("scenario", ["refused_lookup", "tensor_memory_is_idle", "sparse_commitment_table",
+                                      "operands_at_any_address"])
 def test_scenario(program, scenario):
     r = subprocess.run([program, scenario], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr
