@@ -530,15 +530,18 @@ bool Hyrax::verify(Hyrax_proof& proof, jacob_t* commitment, const std::vector<Fr
     const uint new_N = (uint)proof.z_size;
     const uint inner = Log2(rowlen);
     // c * C, C the row commitments folded at the outer variables: sum_i c eq(outer, i) C_i, its window sums on the device
-    // and their doubling chain here.  (Folding fewer variables than the rows need leaves the first 2^variables rows.)
-    const std::vector<Fr> outer(eval_point.begin() + inner, eval_point.end());
-    const uint used = outer.size() < 32 && ((uint64_t)1 << outer.size()) < rows ? 1u << outer.size() : rows;
+    // and their doubling chain here.  (Folding fewer variables than the rows need leaves the first 2^variables rows; each
+    // variable beyond them finds the rows above missing, a factor 1 - u, and needs no table.)
+    std::vector<Fr> outer(eval_point.begin() + inner, eval_point.end());
+    Fr scale = c;
+    for (; outer.size() > Log2(rows); outer.pop_back()) scale *= Fr::one() - outer.back();
+    const uint used = ((uint64_t)1 << outer.size()) < rows ? 1u << outer.size() : rows;
     FrTensor pyramid((uint)grape_eq_pyramid_elems((uint)outer.size()), OnDefaultStream());
     fr_t* d_outer = grape_host::upload(outer, OnDefaultStream());
     check(grape_eq_pyramid(W(pyramid.gpu_data), W(d_outer), (uint)outer.size(), nullptr), "grape_eq_pyramid");
     grape_free_on_default(d_outer);
     fr_t* const weights = pyramid.gpu_data + (((size_t)1 << outer.size()) - 1);
-    check(grape_fr_bcast_mul(W(weights), W(weights), W(grape_host::device_scalar(c)), (size_t)1 << outer.size(), nullptr), "grape_fr_bcast_mul");
+    check(grape_fr_bcast_mul(W(weights), W(weights), W(grape_host::device_scalar(scale)), (size_t)1 << outer.size(), nullptr), "grape_fr_bcast_mul");
     bucket_t* d_windows = nullptr;
     check(grape_malloc_on_default((void**)&d_windows, sizeof(bucket_t) * GRAPE_MSM_WINDOWS), "grape_malloc");
     check(grape_g1_msm_windows(W(d_windows), W(commitment), W(weights), used, nullptr), "grape_g1_msm_windows");

@@ -134,12 +134,39 @@ static void operands_at_any_address() {
     }
 }
 
+// An opening that verifies here: every commitment is the identity (device memory reads as zero), so its two equations are
+// commit_d == 0 and commit_ad == -(c * result) * G.
+static Hyrax_proof trivial_opening(const bn128& G, const Fr& c, uint cols) {
+    const Fr result(5);
+    Hyrax_proof proof(result, cols, bn128::zero(), (Fr::zero() - c * result) * G);
+    for (uint i = 0; i < cols; i++) proof.z[i] = Fr::zero();
+    return proof;
+}
+
+// a point with more variables than the rows need: the rows that are missing count as the identity
+static void verify_with_more_variables() {
+    const uint cols = 64, rows = 4;
+    bn128 G = bn128::one();
+    Hyrax hyrax(1, cols, device_points(256 * cols), G, 1);
+    jacob_t* commitment = reinterpret_cast<jacob_t*>(device_points(2 * rows));
+    const Fr c(3);
+    Hyrax_proof proof = trivial_opening(G, c, cols);
+    for (uint more : {0u, 1u, 20u, 40u}) {
+        const unsigned long before = fake_bytes();
+        expect(hyrax.verify(proof, commitment, random_vec(6 + 2 + more), c, rows * cols, cols), "the opening verifies");
+        expect(fake_bytes() - before < (64ul << 20), "without a table over all variables");
+    }
+    Hyrax_proof wrong = trivial_opening(G + G, c, cols);
+    expect(!hyrax.verify(wrong, commitment, random_vec(6 + 2 + 40), c, rows * cols, cols), "a wrong one does not");
+}
+
 int main(int argc, char** argv) {
     const std::map<std::string, std::function<void()>> scenarios = {
         {"refused_lookup", refused_lookup},
         {"tensor_memory_is_idle", tensor_memory_is_idle},
         {"sparse_commitment_table", sparse_commitment_table},
         {"operands_at_any_address", operands_at_any_address},
+        {"verify_with_more_variables", verify_with_more_variables},
     };
     auto it = scenarios.find(argc > 1 ? argv[1] : "");
     if (it == scenarios.end()) return 2;
