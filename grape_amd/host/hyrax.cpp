@@ -2,6 +2,7 @@
 #include <cstdlib>
 #include <algorithm>
 #include <cassert>
+#include <cstring>
 #include <map>
 #include <utility>
 #include "../../include/grape_hip.h"
@@ -569,8 +570,12 @@ bool Hyrax::verify(Hyrax_proof& proof, jacob_t* commitment, const std::vector<Fr
     return proof.commit_ad == multiple_of_G(az - c * proof.result);
 }
 
+// G is a member that a caller may set: the multiples are made anew for another one
 bn128 Hyrax::multiple_of_G(const Fr& k) {
-    if (!G_multiples_) G_multiples_.reset(new G1FixedBase(G));
+    if (!G_multiples_ || std::memcmp(&G_multiples_of_, &G, sizeof G) != 0) {
+        G_multiples_.reset(new G1FixedBase(G));
+        G_multiples_of_ = G;
+    }
     return G_multiples_->mul(k);
 }
 

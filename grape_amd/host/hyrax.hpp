@@ -130,5 +130,6 @@ private:
     size_t scaled_bytes_ = 0;
     std::vector<Fr> last_open_point_;
     std::unique_ptr<G1FixedBase> G_multiples_;      // built by the first opening or verification
+    bn128 G_multiples_of_;
     size_t table_budget_ = (size_t)128 << 30;
 };

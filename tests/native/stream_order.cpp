@@ -160,6 +160,21 @@ static void verify_with_more_variables() {
     expect(!hyrax.verify(wrong, commitment, random_vec(6 + 2 + 40), c, rows * cols, cols), "a wrong one does not");
 }
 
+// the generator of an object is replaced between two checks
+static void verify_with_another_generator() {
+    const uint cols = 64, rows = 4;
+    bn128 G = bn128::one();
+    Hyrax hyrax(1, cols, device_points(256 * cols), G, 1);
+    jacob_t* commitment = reinterpret_cast<jacob_t*>(device_points(2 * rows));
+    const Fr c(3);
+    const std::vector<Fr> point = random_vec(8);
+    Hyrax_proof first = trivial_opening(G, c, cols), second = trivial_opening(G + G, c, cols);
+    expect(hyrax.verify(first, commitment, point, c, rows * cols, cols), "the opening verifies");
+    hyrax.G = G + G;
+    expect(!hyrax.verify(first, commitment, point, c, rows * cols, cols), "an opening under the old generator does not verify under the new one");
+    expect(hyrax.verify(second, commitment, point, c, rows * cols, cols), "one under the new generator does");
+}
+
 int main(int argc, char** argv) {
     const std::map<std::string, std::function<void()>> scenarios = {
         {"refused_lookup", refused_lookup},
@@ -167,6 +182,7 @@ int main(int argc, char** argv) {
         {"sparse_commitment_table", sparse_commitment_table},
         {"operands_at_any_address", operands_at_any_address},
         {"verify_with_more_variables", verify_with_more_variables},
+        {"verify_with_another_generator", verify_with_another_generator},
     };
     auto it = scenarios.find(argc > 1 ? argv[1] : "");
     if (it == scenarios.end()) return 2;
