@@ -154,12 +154,17 @@ static std::mutex g_alloc_mu;
 constexpr int kMaxLibStreams = 16;
 struct CachedBlock {
     void* p = nullptr;
+    int device = -1;
     hipEvent_t ev[1 + kMaxLibStreams];
     int nev = 0;
     bool whole_device = false;
     bool on_default = false;               // freed by grape_free_on_default: nothing but default-stream work is left on it
 };
-static std::map<void*, size_t>* g_live = nullptr;                    // blocks handed out by grape_malloc
+struct LiveBlock {
+    size_t bytes;
+    int device;                            // the current one of the thread that asked for it
+};
+static std::map<void*, LiveBlock>* g_live = nullptr;                 // blocks handed out by grape_malloc
 static std::multimap<size_t, CachedBlock>* g_cached = nullptr;       // freed blocks kept for reuse
 static size_t g_cached_bytes = 0;
 static std::vector<hipEvent_t>* g_event_pool = nullptr;
@@ -204,10 +209,15 @@ static size_t alloc_cache_cap() {
 }
 static void alloc_tables() {
     if (!g_live) {
-        g_live = new std::map<void*, size_t>();
+        g_live = new std::map<void*, LiveBlock>();
         g_cached = new std::multimap<size_t, CachedBlock>();
         g_event_pool = new std::vector<hipEvent_t>();
     }
+}
+static int current_device() {
+    int device = -1;
+    if (hipGetDevice(&device) != hipSuccess) (void)hipGetLastError();
+    return device;
 }
 static bool take_event(hipEvent_t* out) {
     if (!g_event_pool->empty()) {
@@ -308,18 +318,24 @@ static int malloc_impl(void** p, size_t bytes, bool on_default) {
     if (bytes == 0) bytes = 1;
     std::lock_guard<std::mutex> lock(g_alloc_mu);
     alloc_tables();
-    // of the kept blocks of this size one of the caller's own kind is the cheapest: a default-stream block is handed
+    // of the kept blocks of this size on this device one of the caller's own kind is the cheapest: a default-stream block is handed
     // on without a wait, and a block with events need not wait for what the default stream has queued since
+    const int device = current_device();
     auto range = g_cached->equal_range(bytes);
-    auto it = range.first;
-    while (it != range.second && it->second.on_default != on_default) ++it;
-    if (it == range.second) it = range.first;
+    auto it = range.second;
+    for (auto c = range.first; c != range.second; ++c) {
+        if (c->second.device != device) continue;
+        if (it == range.second) it = c;
+        if (c->second.on_default != on_default) continue;
+        it = c;
+        break;
+    }
     if (it != range.second) {
         CachedBlock b = it->second;
         g_cached->erase(it);
         g_cached_bytes -= bytes;
         int rc = on_default && b.on_default && default_order_holds() ? GRAPE_OK : wait_block(b);   // what hipFree would have waited for
-        (*g_live)[b.p] = bytes;
+        (*g_live)[b.p] = LiveBlock{bytes, device};
         *p = b.p;
         return rc;
     }
@@ -333,7 +349,7 @@ static int malloc_impl(void** p, size_t bytes, bool on_default) {
         set_error("hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
         return GRAPE_ENOMEM;
     }
-    (*g_live)[*p] = bytes;
+    (*g_live)[*p] = LiveBlock{bytes, device};
     return GRAPE_OK;
 }
 static int free_impl(void* p, bool on_default) {
@@ -343,11 +359,12 @@ static int free_impl(void* p, bool on_default) {
     alloc_tables();
     auto it = g_live->find(p);
     if (it != g_live->end()) {
-        const size_t bytes = it->second;
+        const size_t bytes = it->second.bytes;
+        CachedBlock b;
+        b.p = p;
+        b.device = it->second.device;
         g_live->erase(it);
         if (g_cached_bytes + bytes <= alloc_cache_cap()) {
-            CachedBlock b;
-            b.p = p;
             b.on_default = on_default && default_order_holds();
             if (!b.on_default) stamp_block(b);
             g_cached->emplace(bytes, b);
@@ -432,14 +449,13 @@ static bool peek_readable(const void* s, size_t bytes) {
         if (it != g_live->begin()) {
             --it;
             const size_t off = (size_t)((const char*)s - (const char*)it->first);
-            if (off < it->second) return bytes <= it->second - off;
+            if (off < it->second.bytes) return it->second.device == current_device() && bytes <= it->second.bytes - off;
         }
     }
     hipPointerAttribute_t at{};
-    int device = -1;
     hipDeviceptr_t base = nullptr;
     size_t size = 0;
-    if (hipPointerGetAttributes(&at, s) == hipSuccess && at.type == hipMemoryTypeDevice && hipGetDevice(&device) == hipSuccess && at.device == device &&
+    if (hipPointerGetAttributes(&at, s) == hipSuccess && at.type == hipMemoryTypeDevice && at.device == current_device() &&
         hipMemGetAddressRange(&base, &size, const_cast<void*>(s)) == hipSuccess) {
         const size_t off = (size_t)((const char*)s - (const char*)base);
         return off <= size && bytes <= size - off;

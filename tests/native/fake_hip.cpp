@@ -68,6 +68,8 @@ unsigned long fake_copies() { return copies; }
 unsigned long fake_waits() { return waits; }
 void fake_queue(const void* stream) { Lock l(mu); push(stream); }
 
+void fake_set_device(int d) { device = d; }
+
 // ---- the runtime
 hipError_t hipGetDevice(int* d) { *d = device; return hipSuccess; }
 hipError_t hipSetDevice(int d) { device = d; return hipSuccess; }

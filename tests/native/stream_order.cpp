@@ -20,6 +20,7 @@ unsigned long fake_copies();
 void fake_queue(const void* stream);
 unsigned long fake_waits();
 unsigned long fake_bytes();
+void fake_set_device(int device);
 }
 
 static int failures = 0;
@@ -175,6 +176,27 @@ static void verify_with_another_generator() {
     expect(hyrax.verify(second, commitment, point, c, rows * cols, cols), "one under the new generator does");
 }
 
+// A short copy from a block that belongs to another device than the thread's current one goes through the runtime, which reads it
+// there: no kernel of this device does.  And a kept block is not handed out on another device.
+static void blocks_of_two_devices() {
+    void *p = nullptr, *q = nullptr;
+    grape_host::ensure_init();
+    grape_host::check(grape_malloc(&p, 1 << 21), "grape_malloc");
+    char out[256];
+    const unsigned long launches = fake_launches(), copies = fake_copies();
+    grape_host::check(grape_memcpy_d2h(out, p, sizeof out, nullptr), "grape_memcpy_d2h");
+    expect(fake_launches() == launches + 1 && fake_copies() == copies, "a kernel reads a block of the current device");
+    fake_set_device(1);
+    grape_host::check(grape_memcpy_d2h(out, p, sizeof out, nullptr), "grape_memcpy_d2h");
+    expect(fake_launches() == launches + 1 && fake_copies() == copies + 1, "the runtime copies from another device");
+    grape_host::check(grape_free(p), "grape_free");
+    grape_host::check(grape_malloc(&q, 1 << 21), "grape_malloc");
+    expect(q != p, "a block stays with its device");
+    fake_set_device(0);
+    grape_host::check(grape_malloc(&q, 1 << 21), "grape_malloc");
+    expect(q == p, "and is handed out there");
+}
+
 int main(int argc, char** argv) {
     const std::map<std::string, std::function<void()>> scenarios = {
         {"refused_lookup", refused_lookup},
@@ -183,6 +205,7 @@ int main(int argc, char** argv) {
         {"operands_at_any_address", operands_at_any_address},
         {"verify_with_more_variables", verify_with_more_variables},
         {"verify_with_another_generator", verify_with_another_generator},
+        {"blocks_of_two_devices", blocks_of_two_devices},
     };
     auto it = scenarios.find(argc > 1 ? argv[1] : "");
     if (it == scenarios.end()) return 2;
