@@ -153,18 +153,6 @@ __device__ __forceinline__ Xyzz28 ld_partial28(const uint32_t* base, size_t i) {
     a.inf = f[4 * L28] != 0;
     return a;
 }
-__device__ __forceinline__ Xyzz28 shfl_down_xyzz28(const Xyzz28& a, int off) {
-    Xyzz28 r;
-#pragma unroll
-    for (int k = 0; k < L28; k++) {
-        r.x.v[k] = __shfl_down(a.x.v[k], off, 64);
-        r.y.v[k] = __shfl_down(a.y.v[k], off, 64);
-        r.zz.v[k] = __shfl_down(a.zz.v[k], off, 64);
-        r.zzz.v[k] = __shfl_down(a.zzz.v[k], off, 64);
-    }
-    r.inf = __shfl_down((int)a.inf, off, 64) != 0;
-    return r;
-}
 // acc += q for two 28-bit accumulators, exceptional cases through the canonical-form addition
 __device__ __forceinline__ void padd28(Xyzz28& acc, const Xyzz28& q) {
     if (!xyzz28_add(acc, q)) {

@@ -350,7 +350,7 @@ static int wround2_main(uint32_t* Aw, uint32_t* Sw, const uint32_t* A, const uin
                         hipStream_t s) {
     const unsigned nb = wround2_blocks(n_out);
     const bool use_tab = tab != nullptr;
-// five sums and three accumulators leave no registers for the table fold's columns (it spills: 1.16 against
+    // five sums and three accumulators leave no registers for the table fold's columns (it spills: 1.16 against
     // 1.10 ms at 2^24 index pairs), so that form keeps the single-product fold at every size
 #define GRAPE_WROUND2(B, P, U)                                                                                        \
     do {                                                                                                              \
@@ -393,13 +393,6 @@ static void wround2_final(const WFinish& f, uint32_t count, int plain_sums, hipS
     else GRAPE_WFINAL(false, false, false);
 #undef GRAPE_WFINAL
 }
-static void wround2_final(uint32_t* sums, const uint32_t* partial, uint32_t n_out, int plain_sums, hipStream_t s) {
-    WFinish f{};
-    f.partial[0] = partial;
-    f.nblocks[0] = wround2_blocks(n_out);
-    f.out[0] = sums;
-    wround2_final(f, 1, plain_sums, s);
-}
 // workgroups of a round with split weights: a power of two, so that 256 CUs with two workgroups each are filled evenly, and
 // enough of them for at most kWIters whole periods per thread
 static unsigned wround_split_blocks(uint32_t n_out, uint32_t period) {
@@ -418,8 +411,26 @@ static unsigned wround_blocks(const grape_wround_args& a) { return a.eq_high ? w
     GRAPE_REQUIRE(rowlen >= 1 && rowlen <= rowpad, "need 1 <= rowlen <= rowpad");                                        \
     if (beta) CHECK_PTR16(beta)
 
-static int wround2_impl(uint32_t* Aw, uint32_t* Sw, const uint32_t* A, const uint32_t* S, const uint32_t* beta, const uint32_t* E, uint32_t in_size,
-                        uint32_t n_out, uint32_t rowlen, uint32_t rowpad, const uint32_t* v, int plain_sums, uint32_t* sums, grape_stream_t st) {
+// The round as a value: what grape_wround_queue and grape_wround_finish take (folded in place, one table of weights).
+static grape_wround_args wround2_args(uint32_t* A, uint32_t* S, const uint32_t* beta, const uint32_t* E, uint32_t in_size, uint32_t n_out, uint32_t rowlen,
+                                      uint32_t rowpad, const uint32_t* v, int plain_sums, const int32_t* tab, uint32_t* partial) {
+    grape_wround_args a{};
+    a.A = a.A_out = A;
+    a.S = a.S_out = S;
+    a.beta = beta;
+    a.eq = E;
+    a.rowlen = rowlen;
+    a.rowpad = rowpad;
+    a.in_size = in_size;
+    a.n_out = n_out;
+    a.v = v;
+    a.plain_sums = plain_sums;
+    a.tab = tab;
+    a.partial = partial;
+    return a;
+}
+int grape_wround2(uint32_t* A, uint32_t* S, const uint32_t* beta, const uint32_t* E, uint32_t in_size, uint32_t n_out,
+                  uint32_t rowlen, uint32_t rowpad, const uint32_t* v, int plain_sums, uint32_t* sums, grape_stream_t st) {
     GRAPE_WROUND2_CHECKS();
     CHECK_PTR16(sums);
     hipStream_t s = as_stream(st);
@@ -427,27 +438,15 @@ static int wround2_impl(uint32_t* Aw, uint32_t* Sw, const uint32_t* A, const uin
     const size_t partial_bytes = (size_t)wround2_blocks(n_out) * (plain_sums ? 5 : 3) * 32;
     int rc = scratch_get(kSlotReduce, partial_bytes + kFoldTableBytes, &ws, s);
     if (rc) return rc;
-    uint32_t* partial = (uint32_t*)ws;
     // long rounds fold through the table of the challenge's multiples (one more small launch)
     int32_t* tab = nullptr;
     if (n_out >= kTableFoldMinOut) {
         tab = (int32_t*)((char*)ws + partial_bytes);
         fold_tables_kernel<<<1, 64, 0, s>>>(tab, v, 1);
     }
-    rc = wround2_main(Aw, Sw, A, S, beta, E, in_size, n_out, rowlen, rowpad, v, plain_sums, tab, partial, s);
-    if (rc) return rc;
-    wround2_final(sums, partial, n_out, plain_sums, s);
-    GRAPE_LAUNCH_CHECK();
-    return GRAPE_OK;
-}
-int grape_wround2(uint32_t* A, uint32_t* S, const uint32_t* beta, const uint32_t* E, uint32_t in_size, uint32_t n_out,
-                  uint32_t rowlen, uint32_t rowpad, const uint32_t* v, int plain_sums, uint32_t* sums, grape_stream_t st) {
-    return wround2_impl(A, S, A, S, beta, E, in_size, n_out, rowlen, rowpad, v, plain_sums, sums, st);
-}
-int grape_wround2_from(uint32_t* A_out, uint32_t* S_out, const uint32_t* A, const uint32_t* S, const uint32_t* E, uint32_t in_size, uint32_t n_out,
-                       uint32_t rowlen, uint32_t rowpad, const uint32_t* v, uint32_t* sums, grape_stream_t st) {
-    CHECK_PTR16(A_out); CHECK_PTR16(S_out);
-    return wround2_impl(A_out, S_out, A, S, nullptr, E, in_size, n_out, rowlen, rowpad, v, 0, sums, st);
+    const grape_wround_args a = wround2_args(A, S, beta, E, in_size, n_out, rowlen, rowpad, v, plain_sums, tab, (uint32_t*)ws);
+    rc = grape_wround_queue(&a, st);
+    return rc ? rc : grape_wround_finish(sums, 0, &a, 1, st);
 }
 
 size_t grape_wround2_partial_bytes(uint32_t n_out) { return (size_t)wround2_blocks(n_out ? n_out : 1) * 5 * 32; }
@@ -465,25 +464,18 @@ int grape_fold_tables(int32_t* tabs, const uint32_t* v, uint32_t count, grape_st
 int grape_wround2_queue(uint32_t* A, uint32_t* S, const uint32_t* beta, const uint32_t* E, uint32_t in_size, uint32_t n_out,
                         uint32_t rowlen, uint32_t rowpad, const uint32_t* v, int plain_sums, const int32_t* tab, uint32_t* partial,
                         grape_stream_t st) {
-    GRAPE_WROUND2_CHECKS();
-    CHECK_PTR16(partial);
-    GRAPE_REQUIRE(tab == nullptr || n_out >= kTableFoldMinOut, "the table fold is built for rounds of 2^16 index pairs and more");
-    int rc = wround2_main(A, S, A, S, beta, E, in_size, n_out, rowlen, rowpad, v, plain_sums, tab, partial, as_stream(st));
-    if (rc) return rc;
-    GRAPE_LAUNCH_CHECK();
-    return GRAPE_OK;
+    const grape_wround_args a = wround2_args(A, S, beta, E, in_size, n_out, rowlen, rowpad, v, plain_sums, tab, partial);
+    return grape_wround_queue(&a, st);
 }
 
 int grape_wround2_queue_indexed(uint32_t* A, uint32_t* S, const int32_t* idx1, const uint32_t* Bt, uint32_t len, const uint32_t* beta,
                                 const uint32_t* E, uint32_t n_out, const uint32_t* v, const int32_t* tab, uint32_t* partial,
                                 grape_stream_t st) {
-    CHECK_PTR16(A); CHECK_PTR16(S); CHECK_PTR16(E); CHECK_PTR16(v); CHECK_PTR16(Bt); CHECK_PTR16(beta); CHECK_PTR16(partial);
-    GRAPE_REQUIRE(idx1 != nullptr && len >= 1, "bad arguments");
-    GRAPE_REQUIRE(tab != nullptr && n_out >= kTableFoldMinOut && n_out <= (1u << 30), "built for first rounds of 2^16 index pairs and more");
-    wround2_kernel<true, true, true, true, false, true><<<wround2_blocks(n_out), kBlock, 0, as_stream(st)>>>(
-        A, S, A, S, beta, E, 2 * n_out, n_out, 1, 1, v, tab, partial, idx1, Bt);
-    GRAPE_LAUNCH_CHECK();
-    return GRAPE_OK;
+    GRAPE_REQUIRE(idx1 != nullptr && len >= 1 && n_out <= (1u << 30), "bad arguments");
+    grape_wround_args a = wround2_args(A, S, beta, E, 2 * n_out, n_out, 1, 1, v, 2, tab, partial);
+    a.idx1 = idx1;
+    a.B = Bt;
+    return grape_wround_queue(&a, st);
 }
 
 size_t grape_wround_partial_bytes(const grape_wround_args* args) {
@@ -544,11 +536,11 @@ int grape_wround_finish(uint32_t* sums, uint32_t stride, const grape_wround_args
 }
 
 int grape_wround2_finish(uint32_t* sums, const uint32_t* partial, uint32_t n_out, int plain_sums, grape_stream_t st) {
-    CHECK_PTR16(sums); CHECK_PTR16(partial);
-    GRAPE_REQUIRE(n_out >= 1, "need n_out >= 1");
-    wround2_final(sums, partial, n_out, plain_sums, as_stream(st));
-    GRAPE_LAUNCH_CHECK();
-    return GRAPE_OK;
+    grape_wround_args a{};
+    a.n_out = n_out;
+    a.plain_sums = plain_sums;
+    a.partial = const_cast<uint32_t*>(partial);
+    return grape_wround_finish(sums, 0, &a, 1, st);
 }
 #undef GRAPE_WROUND2_CHECKS
 

@@ -447,6 +447,18 @@ def wround_products(A, S, beta, low, high, period, in_size, n_out, v, plain_sums
     return sums
 
 
+def wround_kept(A, S, e, in_size, n_out, v):
+    """a weighted round (one table of weights, no shift) that keeps its operands; returns the sums and the folded tensors"""
+    lib = init()
+    Aw, Sw, sums = fr_empty(n_out), fr_empty(n_out), fr_empty(3)
+    a = _Wround(A_out=_p(Aw), S_out=_p(Sw), A=_p(A), S=_p(S), eq=_p(e), rowlen=1, rowpad=1, in_size=in_size, n_out=n_out, v=_p(v))
+    partial = torch.empty(lib.grape_wround_partial_bytes(ctypes.byref(a)) // 4, dtype=torch.int32, device="cuda")
+    a.partial = _p(partial)
+    _capi.check(lib.grape_wround_queue(ctypes.byref(a), _s()))
+    _capi.check(lib.grape_wround_finish(_p(sums), 3, ctypes.byref(a), 1, _s()))
+    return sums, Aw, Sw
+
+
 def wround2_first_indexed(S, idx1, B, beta, e, n_out, v):
     """first round of a lookup whose logUp tensor A = B[idx1 - 1] was never written out; returns (sums, folded A)"""
     lib = init()

@@ -237,10 +237,6 @@ int grape_fold_tables(int32_t *d_tabs, const uint32_t *d_v, uint32_t count, grap
 int grape_wround2_queue(uint32_t *d_A, uint32_t *d_S, const uint32_t *d_beta, const uint32_t *d_e, uint32_t in_size, uint32_t n_out,
                         uint32_t rowlen, uint32_t rowpad, const uint32_t *d_v, int plain_sums, const int32_t *d_tab,
                         uint32_t *d_partial, grape_stream_t stream);
-/* The round of grape_wround2 (plain_sums 0) that keeps its operands: A and S are read, the folded halves written to
- * d_A_out and d_S_out (n_out elements each). */
-int grape_wround2_from(uint32_t *d_A_out, uint32_t *d_S_out, const uint32_t *d_A, const uint32_t *d_S, const uint32_t *d_eq, uint32_t in_size,
-                       uint32_t n_out, uint32_t rowlen, uint32_t rowpad, const uint32_t *d_v, uint32_t *d_sums, grape_stream_t stream);
 int grape_wround2_finish(uint32_t *d_sums, const uint32_t *d_partial, uint32_t n_out, int plain_sums, grape_stream_t stream);
 /*
  * grape_wround2_queue with plain_sums == 2 for a logUp tensor that was never written out: the first round of a
@@ -254,8 +250,9 @@ int grape_wround2_queue_indexed(uint32_t *d_A, uint32_t *d_S, const int32_t *d_i
                                 const uint32_t *d_beta, const uint32_t *d_e, uint32_t n_out, const uint32_t *d_v, const int32_t *d_tab,
                                 uint32_t *d_partial, grape_stream_t stream);
 /*
- * The pass of a weighted round in its general form (fields as the arguments of grape_wround2, grape_wround2_from,
- * grape_wround2_queue and grape_wround2_queue_indexed; A and A_out, S and S_out may be the same).  With eq_high the
+ * The pass of a weighted round in its general form (fields as the arguments of grape_wround2, grape_wround2_queue
+ * and grape_wround2_queue_indexed, which are short forms of it).  A and S are read, the folded halves (n_out elements each)
+ * written to A_out and S_out, which may be A and S.  With eq_high the
  * weight of index h * period + l is eq_high[h] * eq[l] and rowlen, rowpad are not used (1, 1): a tensor whose rows hold
  * fewer elements than the weights' rows takes its row length as the period.  eq_high needs tab and plain_sums 0
  * without beta, or 2 or 3 with it.  grape_wround_finish finishes `count` <= 32 such rounds of one plain_sums in one launch; round i's

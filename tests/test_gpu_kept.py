@@ -34,11 +34,9 @@ def test_fold_of_a_kept_tensor(ops, outer, c, gap):
 @pytest.mark.parametrize("in_size,n_out", [(2, 1), (600, 300), (1023, 512), (1 << 18, 1 << 17)])
 def test_weighted_round_of_kept_operands(ops, in_size, n_out):
     from gpuutil import rand_fr
-    from grape_amd import _capi
     A, S, E, v = (ops.to_dev(rand_fr(n, 710 + k)) for k, n in enumerate((in_size, in_size, n_out, 1)))
     a, s = A.clone(), S.clone()
-    Aw, Sw, sums = ops.fr_empty(n_out), ops.fr_empty(n_out), ops.fr_empty(3)
-    _capi.check(_capi.load().grape_wround2_from(ops._p(Aw), ops._p(Sw), ops._p(A), ops._p(S), ops._p(E), in_size, n_out, 1, 1, ops._p(v), ops._p(sums), ops._s()))
+    sums, Aw, Sw = ops.wround_kept(A, S, E, in_size, n_out, v)
     assert torch.equal(A, a) and torch.equal(S, s)
     want = ops.wround2(a, s, None, E, in_size, n_out, v)
     assert torch.equal(sums, want) and torch.equal(Aw, a[:n_out]) and torch.equal(Sw, s[:n_out])
