@@ -24,7 +24,7 @@ GRAPE_HD uint32_t reduce_lanes_log2(size_t rows) {
 
 struct WidePlan {
     size_t rows;            // size / rowlen
-    uint32_t lg_lpr;        // log2 of the lanes per row in the reduction
+    uint32_t lg_lpr;        // reduce_lanes_log2 of the rows
     uint32_t nseg, seg;     // column segments per row and their length
     size_t slab;            // rows per launch
     size_t partial_bytes;   // work buffer of one launch (slab * nseg * 64 lanes * 256 bytes)
@@ -124,13 +124,35 @@ GRAPE_HD size_t reduce_tmp_accumulators(size_t rows, uint32_t nparts) {
     return rows + (grouped > kept ? grouped : kept);
 }
 
-// The layout of a four-wave reduction (eight rows a workgroup, 32 lanes a row) that no kernel uses any more; the host
-// walk of the tests still goes through it.
-constexpr int kTreeRows = 8;
-constexpr int kTreeThreads = 256;
-GRAPE_HD size_t tree_row(size_t block, int t) { return block * (size_t)kTreeRows + (size_t)(t & (kTreeRows - 1)); }
-GRAPE_HD uint32_t tree_share(int t) { return (uint32_t)t >> 3; }
-GRAPE_HD bool tree_reduction(size_t rows, uint32_t lg_lpr, uint32_t nparts) { return lg_lpr <= 5 && rows <= 4096 && nparts <= 4096; }
+// The launches of a reduction, in order.  A stage reads `units` times `parts` accumulators (the partial sums for the first stage,
+// work space from accumulator `from` on otherwise) and leaves one per unit (`keep` per unit for the lane kernel) in work
+// space from accumulator `to` on; the last stage's are the row sums.
+struct ReduceStage {
+    bool lanes;             // commit_reduce_lane_kernel, else commit_reduce_quad_kernel
+    size_t units;
+    uint32_t parts, keep, lg_qpr;
+    size_t from, to;
+};
+constexpr int kMaxReduceStages = 3;
+GRAPE_HD int reduce_stages(size_t rows, uint32_t nparts, ReduceStage* st) {
+    const ReducePlan p = reduce_plan(rows, nparts);
+    int n = 0;
+    size_t from = 0, used = 0;
+    if (p.lanes) st[n++] = ReduceStage{true, rows, nparts, p.left, 0, 0, 0};
+    else if (p.left < nparts) st[n++] = ReduceStage{false, rows * p.left, nparts / p.left, 1, kQuadsPerWaveLog2, 0, 0};
+    if (n) used = rows * p.left;
+    if (p.left2 < p.left) {
+        st[n++] = ReduceStage{false, rows * p.left2, p.left / p.left2, 1, kQuadsPerWaveLog2, from, used};
+        from = used;
+        used += rows * p.left2;
+    }
+    st[n++] = ReduceStage{false, rows, p.left2, 1, p.lg_qpr, from, used};
+    return n;
+}
+// row and first partial sum of thread `t` of the lane kernel (it goes on in steps of `keep`)
+GRAPE_HD size_t lane_row(size_t t, uint32_t keep) { return t / keep; }
+GRAPE_HD uint32_t lane_share(size_t t, uint32_t keep) { return (uint32_t)(t % keep); }
+
 // Workgroups are dealt to the chip's 32 shader engines in turn (workgroup i to XCD i mod 8, and in turn within it), whether
 // or not that engine has room.  Where the work of a unit depends on its position - rows of 11008 padded to 16384 leave
 // every fourth committed row empty - units in launch order leave whole engines idle.  spread_unit is a permutation

@@ -924,8 +924,8 @@ __global__ void __launch_bounds__(64) quad_horner_kernel(uint32_t* out, const ui
 __global__ void __launch_bounds__(kBlock) commit_reduce_lane_kernel(uint32_t* out, const uint32_t* partial, size_t rows, uint32_t nparts, uint32_t keep) {
     const size_t t = (size_t)blockIdx.x * kBlock + threadIdx.x;
     if (t >= rows * keep) return;
-    const size_t row = t / keep;
-    const uint32_t sub = (uint32_t)(t - row * keep);
+    const size_t row = geom::lane_row(t, keep);
+    const uint32_t sub = geom::lane_share(t, keep);
     Xyzz28 acc = ld_partial28(partial, row * nparts + sub);
     for (uint32_t j = sub + keep; j < nparts; j += keep) padd28(acc, ld_partial28(partial, row * nparts + j));
     st_partial28(out, t, acc);
@@ -1106,26 +1106,15 @@ constexpr size_t kMaxCommitScalars = (size_t)1 << 28;
 static size_t reduce_tmp_bytes(size_t rows, uint32_t nparts) { return geom::reduce_tmp_accumulators(rows, nparts) * (4 * kPartialWords); }
 template <bool AFFINE>
 static void launch_reduce(uint32_t* out, const uint32_t* partial, size_t rows, uint32_t nparts, uint32_t* tmp, hipStream_t s) {
-    const geom::ReducePlan plan = geom::reduce_plan(rows, nparts);
-    auto quads = [&](uint32_t* to, const uint32_t* from, size_t units, uint32_t parts, uint32_t lg_qpr) {
-        commit_reduce_quad_kernel<<<blocks_for(units << (lg_qpr + 2)), kBlock, 0, s>>>(to, from, units, parts, lg_qpr);
-    };
-    if (plan.lanes)
-        commit_reduce_lane_kernel<<<blocks_for(rows * plan.left), kBlock, 0, s>>>(tmp, partial, rows, nparts, plan.left);
-    else if (plan.left < nparts)
-        quads(tmp, partial, rows * plan.left, nparts / plan.left, geom::kQuadsPerWaveLog2);
-    const uint32_t* last = partial;
-    if (plan.left < nparts) {
-        last = tmp;
-        tmp += geom::partial_word(rows * plan.left);
+    geom::ReduceStage st[geom::kMaxReduceStages];
+    const int n = geom::reduce_stages(rows, nparts, st);
+    uint32_t* sums = nullptr;
+    for (int i = 0; i < n; i++) {
+        const uint32_t* from = i == 0 ? partial : tmp + geom::partial_word(st[i].from);
+        sums = i == n - 1 && !AFFINE ? out : tmp + geom::partial_word(st[i].to);
+        if (st[i].lanes) commit_reduce_lane_kernel<<<blocks_for(st[i].units * st[i].keep), kBlock, 0, s>>>(sums, from, st[i].units, st[i].parts, st[i].keep);
+        else commit_reduce_quad_kernel<<<blocks_for(st[i].units << (st[i].lg_qpr + 2)), kBlock, 0, s>>>(sums, from, st[i].units, st[i].parts, st[i].lg_qpr);
     }
-    if (plan.left2 < plan.left) {
-        quads(tmp, last, rows * plan.left2, geom::kReduceGroup2, geom::kQuadsPerWaveLog2);
-        last = tmp;
-        tmp += geom::partial_word(rows * plan.left2);
-    }
-    uint32_t* const sums = AFFINE ? tmp : out;
-    quads(sums, last, rows, plan.left2, plan.lg_qpr);
     if (AFFINE) quad_affine_kernel<<<blocks_for(rows * 4), kBlock, 0, s>>>(out, sums, rows);
 }
 

@@ -74,18 +74,6 @@ def test_masked_strided_commitment(setup, rowlen, rows, live, c, J):
     assert np.array_equal(got[-1:], orc.commit_fr(s[-rowlen:], ref, rowlen, 128))
 
 
-@pytest.mark.parametrize("n", [1, 7, 31, 32, 33, 96, 1000, 4096, 24577])
-def test_spread_units_are_a_permutation(n):
-    """the host twin of geom::spread_unit"""
-    from math import gcd
-    m = n // 32 * 32
-    step = int(0.6180339887 * m) | 1
-    while m and gcd(m, step) != 1:
-        step += 2
-    seen = {i if i >= m else ((i % 32) * (m // 32) + i // 32) * step % m for i in range(n)}
-    assert seen == set(range(n))
-
-
 # few rows of full-width scalars: the windows go over several waves (window_split: 1, 2, 3, 16 shares, shares of unequal
 # length), the partial sums over one, two and three levels of groups
 @pytest.mark.parametrize("rows,cols", [(1, 1), (1, 128), (3, 100), (15, 128), (129, 64), (300, 65)])
