@@ -197,6 +197,70 @@ static void blocks_of_two_devices() {
     expect(q == p, "and is handed out there");
 }
 
+// Blocks that only the default stream works on: handed on with no wait while every other stream is one the library joins itself;
+// waited for when a caller's stream is about, and when memory for any stream takes them over.
+static void default_order_blocks() {
+    auto get = [](bool on_default) {
+        void* p = nullptr;
+        grape_host::check((on_default ? grape_malloc_on_default : grape_malloc)(&p, 5000), "grape_malloc");
+        return p;
+    };
+    grape_host::ensure_init();
+    grape_stream_t side, user;
+    grape_host::check(grape_stream_create(&side), "grape_stream_create");
+    grape_host::check(grape_stream_internal(side), "grape_stream_internal");
+    auto work = [](void* p, grape_stream_t st) { grape_host::check(grape_memset_zero(p, 64, st), "grape_memset_zero"); };
+    void* p = get(true);
+    work(p, nullptr);
+    grape_host::check(grape_free_on_default(p), "grape_free");
+    unsigned long waits = fake_waits();
+    void* q = get(true);
+    expect(q == p && fake_waits() == waits && fake_pending(nullptr) == 1, "handed on in the default stream's order");
+    grape_host::check(grape_free_on_default(q), "grape_free");
+    q = get(false);
+    expect(q == p && fake_pending(nullptr) == 0, "memory for any stream waits for the default stream");
+    work(q, side);
+    grape_host::check(grape_free(q), "grape_free");
+    q = get(true);
+    expect(q == p && fake_pending(side) == 0, "a block of another kind is waited for");
+    grape_host::check(grape_stream_create(&user), "grape_stream_create");
+    work(q, user);
+    grape_host::check(grape_free_on_default(q), "grape_free");
+    q = get(true);
+    expect(q == p && fake_pending(user) == 0, "a caller's stream is waited for");
+    grape_host::check(grape_free_on_default(q), "grape_free");
+    grape_host::check(grape_stream_destroy(user), "grape_stream_destroy");
+    q = get(true);
+    work(q, nullptr);
+    grape_host::check(grape_free_on_default(q), "grape_free");
+    waits = fake_waits();
+    q = get(true);
+    expect(q == p && fake_waits() == waits, "until it is gone");
+    work(q, reinterpret_cast<grape_stream_t>(&waits));       // a stream that the caller brings
+    grape_host::check(grape_free_on_default(q), "grape_free");
+    q = get(true);
+    expect(q == p && fake_pending(&waits) == 0, "a stream that a caller brings is waited for");
+}
+
+// A short copy goes through the kernel where it lies inside one block, through the runtime where it does not.
+static void short_copies() {
+    const size_t bytes = 1 << 20;
+    char *p = nullptr, out[512];
+    grape_host::ensure_init();
+    grape_host::check(grape_malloc((void**)&p, bytes), "grape_malloc");
+    auto by_kernel = [&](const void* from, size_t n) {
+        const unsigned long launches = fake_launches(), copies = fake_copies();
+        grape_host::check(grape_memcpy_d2h(out, from, n, nullptr), "grape_memcpy_d2h");
+        expect(fake_launches() + fake_copies() == launches + copies + 1, "one launch or one copy");
+        return fake_launches() > launches;
+    };
+    expect(by_kernel(p, 256) && by_kernel(p + bytes - 256, 256), "the first and the last bytes of a block");
+    expect(!by_kernel(p + bytes - 252, 256) && !by_kernel(p + bytes - 4, 8), "a range that ends behind its block");
+    expect(!by_kernel(p + 2, 4) && !by_kernel(p, 3), "addresses and lengths that are no words");
+    expect(!by_kernel(out, 4), "host memory");
+    grape_host::check(grape_free(p), "grape_free");
+}
+
 int main(int argc, char** argv) {
     const std::map<std::string, std::function<void()>> scenarios = {
         {"refused_lookup", refused_lookup},
@@ -206,6 +270,8 @@ int main(int argc, char** argv) {
         {"verify_with_more_variables", verify_with_more_variables},
         {"verify_with_another_generator", verify_with_another_generator},
         {"blocks_of_two_devices", blocks_of_two_devices},
+        {"default_order_blocks", default_order_blocks},
+        {"short_copies", short_copies},
     };
     auto it = scenarios.find(argc > 1 ? argv[1] : "");
     if (it == scenarios.end()) return 2;

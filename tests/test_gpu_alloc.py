@@ -42,9 +42,12 @@ def test_short_copy_of_the_last_bytes_of_a_block(lib):
     from grape_amd import _capi
     p = ctypes.c_void_p()
     _capi.check(lib.grape_malloc(ctypes.byref(p), 1 << 21))
+    block = np.random.default_rng(5).integers(0, 1 << 31, 1 << 19).astype(np.int32)
+    _capi.check(lib.grape_memcpy_h2d(p, block.ctypes.data_as(ctypes.c_void_p), 1 << 21, None))
     out = np.zeros(64, dtype=np.int32)
     dst = out.ctypes.data_as(ctypes.c_void_p)
     assert lib.grape_memcpy_d2h(dst, ctypes.c_void_p(p.value + (1 << 21) - 256), 256, None) == 0
+    assert np.array_equal(out, block[-64:])
     _capi.check(lib.grape_free(p))
 
 
@@ -84,3 +87,47 @@ def test_default_blocks_are_handed_on(lib, n_words):
     p = ctypes.c_void_p()                         # a block of the other kind is taken over as well
     assert lib.grape_malloc(ctypes.byref(p), 4 * n_words) == 0 and lib.grape_free(p) == 0
     _cycle(lib, n_words, 700)
+
+
+def _late_reader(lib, reader, take, writer):
+    """Copies of a 256 MB block are queued on `reader`, the block is given back as a default-stream block, taken again with `take`
+    and overwritten on `writer`: the copies hold the old contents."""
+    from grape_amd import _capi
+    words = 1 << 26
+    p, q = ctypes.c_void_p(), ctypes.c_void_p()
+    _capi.check(lib.grape_malloc_on_default(ctypes.byref(p), 4 * words))
+    _capi.check(lib.grape_malloc(ctypes.byref(q), 4 * words))
+    host = np.arange(words, dtype=np.uint32)
+    _capi.check(lib.grape_memcpy_h2d(p, host.ctypes.data_as(ctypes.c_void_p), 4 * words, None))
+    _capi.check(lib.grape_memset_zero(q, 4 * words, None))
+    _capi.check(lib.grape_stream_sync(None))
+    for _ in range(8):
+        _capi.check(lib.grape_memcpy_d2d(q, p, 4 * words, reader))
+    _capi.check(lib.grape_free_on_default(p))
+    r = ctypes.c_void_p()
+    _capi.check(take(ctypes.byref(r), 4 * words))
+    assert r.value == p.value
+    _capi.check(lib.grape_memset_zero(r, 4 * words, writer))
+    for s in (reader, writer):
+        _capi.check(lib.grape_stream_sync(s))
+    got = np.empty(words, dtype=np.uint32)
+    _capi.check(lib.grape_memcpy_d2h(got.ctypes.data_as(ctypes.c_void_p), q, 4 * words, None))
+    for b in (q, r):
+        _capi.check(lib.grape_free(b))
+    assert np.array_equal(got, host)
+
+
+def test_a_block_is_not_overwritten_under_a_reader(lib):
+    from grape_amd import ops
+    user = ops.stream_create()                    # reads a block that the default stream takes over
+    try:
+        _late_reader(lib, user, lib.grape_malloc_on_default, None)
+    finally:
+        ops.stream_destroy(user)
+    side = ops.stream_create()                    # joined by this test itself: a block the default stream reads goes to another stream
+    try:
+        assert lib.grape_stream_internal(side) == 0
+        _late_reader(lib, None, lib.grape_malloc, side)
+        _late_reader(lib, None, lib.grape_malloc_on_default, None)
+    finally:
+        ops.stream_destroy(side)

@@ -22,7 +22,8 @@ def program():
 
 @pytest.mark.parametrize("scenario", ["refused_lookup", "tensor_memory_is_idle", "sparse_commitment_table",
                                       "operands_at_any_address", "verify_with_more_variables",
-                                      "verify_with_another_generator", "blocks_of_two_devices"])
+                                      "verify_with_another_generator", "blocks_of_two_devices",
+                                      "default_order_blocks", "short_copies"])
 def test_scenario(program, scenario):
     r = subprocess.run([program, scenario], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr
