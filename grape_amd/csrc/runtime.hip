@@ -249,9 +249,9 @@ static void stamp_block(CachedBlock& b) {
         b.ev[b.nev++] = e;
     }
 }
-// Blocks that live on the default stream alone (the tensors of the host classes) go from one owner to the next in the
-// order of that stream, with no event and no wait - unless somebody works on a stream this file knows nothing
-// about (its own, or one of grape_stream_create that was not declared internal) and may use a tensor there.
+// Blocks that live on the default stream alone (what the host classes keep to themselves) go from one owner to the next in
+// the order of that stream, with no event and no wait - unless somebody works on a stream this file knows nothing
+// about (its own, or one of grape_stream_create that was not declared internal) and may use a block there.
 static bool default_order_holds() { return !g_foreign_stream.load() && g_n_user_streams.load() == 0 && !g_exit_started.load(); }
 static int wait_block(CachedBlock& b) {
     if (b.on_default) GRAPE_HIP_CHECK(hipStreamSynchronize(nullptr));

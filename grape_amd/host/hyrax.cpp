@@ -244,7 +244,7 @@ bool Hyrax::ensure_strided_table(uint rowlen, bool build, const double* worth_ms
         return best;
     };
     // one table over every generator serves all row lengths; it is preferred to a table over the
-    // first `rowlen` generators (which a longer row would have to replace, at half a second per
+    // first `rowlen` generators (which a longer row would have to replace, at a tenth of a second per
     // build) unless that costs over a quarter more additions per scalar
     Choice pick = choose(rowlen);
     uint ngen = rowlen;

@@ -501,7 +501,7 @@ Fr tLookup::run(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax& hyrax
     if (!m_late) check(grape_fr_sum(W(d_sum_Bm), W(Bm.gpu_data), N, nullptr), "grape_fr_sum");
     fr_t* d_v = grape_host::upload(v, OnDefaultStream());
     Fr S_last;
-    char* long_work = nullptr;             // partial sums of the long rounds and the challenges' tables (overlap mode)
+    char* long_work = nullptr;             // partial sums of the long rounds and the challenges' tables
     // phase 2 binds copies where its rounds work in place; T, B, m of this object stay intact
     const bool table_long = N / 2 >= kLongRoundPairs;
     FrTensor Bw(table_long ? N : 1, OnDefaultStream()), Tw(table_long ? N : 1, OnDefaultStream()), mw(table_long ? N : 1, OnDefaultStream());
