@@ -37,16 +37,16 @@ K_DIGIT = 32768
 # The curve is BLS12-381 (what the benchmark configurations name) unless GRAPE_CURVE=bn254 selects
 # the BN254 build of the libraries and of the oracle.
 CURVE = os.environ.get("GRAPE_CURVE", "bls12_381")
-FP_WORDS, FP_LIMBS28 = (8, 10) if CURVE == "bn254" else (12, 14)
+FP_WORDS, FP_LIMBS30 = (8, 9) if CURVE == "bn254" else (12, 13)
 # Algorithmic work per committed point, the reference's algorithm (two non-zero byte windows of an
 # int16 scalar, each a mixed XYZZ addition of 8M+2S, 2n^2+n 32x32 multiplies per n-limb Montgomery
 # product: 300 for the 12 limbs of BLS12-381, 136 for the 8 of BN254): 2 * 10 * 300 = 6000.
 ALG_MULS_PER_POINT = 2 * 10 * (2 * FP_WORDS * FP_WORDS + FP_WORDS)
-# What the fast path executes: ONE mixed addition per point on L limbs of 28 bits (L = 14 resp.
-# 10): 6 products of L*L + L*L + L multiply-adds, one fused difference of two products
-# (2*L*L + L*L + L) and 2 squares of L(L+1)/2 + L*L + L: 3668 for L = 14, 1900 for L = 10.
-_L = FP_LIMBS28
-EXEC_MULS_PER_POINT = 6 * (2 * _L * _L + _L) + (3 * _L * _L + _L) + 2 * (_L * (_L + 1) // 2 + _L * _L + _L)
+# What the fast path executes: ONE mixed addition per point on L limbs of 30 bits (L = 13 resp.
+# 9): 6 products of L*L + L*L + 1 multiply-adds, one fused difference of two products
+# (2*L*L + L*L + 1), 2 squares of L(L+1)/2 + L*L + 1 and 4 subtractions inside products of L - 1: 3112 for L = 13, 1526 for L = 9.
+_L = FP_LIMBS30
+EXEC_MULS_PER_POINT = 6 * (2 * _L * _L + 1) + (3 * _L * _L + 1) + 2 * (_L * (_L + 1) // 2 + _L * _L + 1) + 4 * (_L - 1)
 # lane-level 32x32 multiplies per second if every SIMD issued one v_mad_u64_u32 per cycle:
 # 256 CUs x 4 SIMDs x 16 lanes x 2.4 GHz
 PEAK_MULS_NOMINAL = 256 * 64 * 2.4e9

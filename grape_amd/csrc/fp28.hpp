@@ -1,24 +1,35 @@
-// Fp on signed limbs of 28 bits with lazy reduction - the working form of the commitment kernels
-// (14 limbs, radix 2^392, for BLS12-381; 10 limbs, radix 2^280, for BN254).
+// Fp on signed limbs of 30 bits with lazy reduction - the working form of the commitment kernels
+// (13 limbs, radix 2^390, for BLS12-381; 9 limbs, radix 2^270, for BN254).  The names keep the 28
+// of the form's first limb width.
 //
 // Why: on gfx950 a 32x32+64 multiply-add (v_mad_i64_i32 / v_mad_u64_u32) issues at the same rate
 // as an addition, so the cost of a field product is its instruction count, and with saturated
-// 32-bit limbs two thirds of the instructions are carry handling.  With 28-bit limbs every limb
-// product is < 2^58, a whole column of an (a*b + m*p) row set fits a 64-bit accumulator, and a
-// limb product is exactly ONE instruction; signed limbs make subtraction limb-wise, with no
-// borrow chain and no bias.
+// 32-bit limbs two thirds of the instructions are carry handling.  Signed limbs make subtraction
+// limb-wise, and BALANCED ones - digits in [-2^29, 2^29) - have products below 2^58, so that a whole
+// column of an (a*b + m*p) row set fits a signed 64-bit accumulator with limbs of 30 bits: 13 limbs where
+// unsigned digits need 28 bits and 14 limbs (338 instead of 392 multiply-adds a product).
 //
-// Representation: x = sum_i v[i] * 2^(28 i), v[i] signed 32-bit.  "Normalised" means
-// 0 <= v[i] < 2^28 for i < N-1 (the top limb carries the sign and the overflow).  A value stands
-// for its residue mod p; arithmetic is Montgomery with radix R' = 2^(28 N).  The canonical memory
-// form elsewhere in the library is the reference's: 32-bit limbs, radix 2^384 resp. 2^256
-// (include/field/mont_t.cuh, include/field/bls12-381.cuh:7-23, include/field/alt_bn128.cuh);
-// conversion is exact both ways.
+// Representation: x = sum_i v[i] * 2^(30 i), v[i] signed 32-bit.  "Balanced": |v[i]| <= 2^29 + 2 for
+// i < N-1, the top limb carries what is left.  "Normalised": 0 <= v[i] < 2^30 for i < N-1, the top
+// limb carries the sign - the form in which values are compared.  A value stands for its residue mod p;
+// arithmetic is Montgomery with radix R' = 2^(30 N).  The canonical memory form elsewhere in the
+// library is the reference's: 32-bit limbs, radix 2^384 resp. 2^256 (include/field/mont_t.cuh,
+// include/field/bls12-381.cuh:7-23, include/field/alt_bn128.cuh); conversion is exact both ways.
 //
-// Bounds (checked by the callers' comments): mul28(a, b) needs |a| < alpha*p, |b| < beta*p with
-// alpha*beta <= 2^11 and limb magnitudes with 14 * 2^(la+lb) < 2^62, i.e. la + lb <= 58; its
-// result is normalised and lies in (0, 3p).  The figures are those of BLS12-381, the tighter
-// case: BN254 leaves R'/p = 2^26 of head-room instead of 2^11 and sums 10 limb products.
+// Reduction: T = T0 + 2^30 T1 becomes T1 + T0 * (2^-30 mod p), column by column - the quotient digit
+// is the column's low 30 bits as they stand, with no product to find it and no carry to wait
+// for.  The factor 2^-30 mod p is taken nearest to zero (for BLS12-381 2^369: p^-1 mod 2^30
+// has 18 bits).  With balanced operands the columns have room for digits of 32 bits, whose cut is a column's word
+// boundary.  The last column takes the ordinary step (a digit of -T0/p, times p), so that the result does not
+// carry the factor 2^30 that the others would leave in it.
+//
+// Bounds (checked by the callers' comments).  Values: mul28(a, b) with |a| < alpha*p, |b| < beta*p
+// is a balanced number of magnitude below (0.51 + alpha*beta/630) p; for BN254 0.94 p (1.4 p from wide digits)
+// instead of 0.51 p, and 86000 instead of 630 - below p for every product here, wide digits on BN254 apart, so that a
+// product is zero mod p only when all its limbs are zero.  Columns: a sum of 12 limb products of balanced operands is
+// 0.38 * 2^63, the reduction adds 0.24 (0.48 in wide digits); so ONE operand may be a lazy sum or difference of two balanced numbers or
+// normalised (0.985 * 2^63 in the worst column; BN254 0.77), and so may two products of balanced operands share
+// their columns.  Lazy operands on both sides do not fit: balance() one.
 #pragma once
 #include "curve.hpp"
 #include "divstep.hpp"
@@ -27,93 +38,117 @@ namespace grape {
 
 #if defined(GRAPE_CURVE_BN254)
 struct Fp28 {
-    int32_t v[10];
+    int32_t v[9];
 };
 
 namespace fp28 {
 
-constexpr int N = 10;
-constexpr int W = 28;
-constexpr uint32_t MASK = (1u << W) - 1;
-constexpr uint32_t PINV = 0x4866389u;   // -p^-1 mod 2^28
+constexpr int N = 9;
+constexpr int W = 30;
+constexpr bool kSmallDown = false;
+constexpr uint32_t PINV = 0x24866389u;   // -p^-1 mod 2^30
 
-GRAPE_HD int32_t P(int i) {
-    constexpr int32_t t[10] = {0x87cfd47, 0x208c16d, 0x1ca8d3c, 0x6a91687, 0x85d9781,
-                               0xb681815, 0x9b85045, 0xe131a02, 0x0644e72, 0x0000003};
+GRAPE_HD int32_t P(int i) {   // balanced, as all tables of limbs here
+    constexpr int32_t t[9] = {0x187cfd47, -0xf7dcfa5, 0x71ca8d4, -0x1fa55ba6, 0x1585d98, 0x116da06, 0x1a029b85, 0x139cb84c, 0x3064};
     return t[i];
 }
 GRAPE_HD int32_t P2(int i) {   // 2p
-    constexpr int32_t t[10] = {0x0f9fa8e, 0x41182db, 0x3951a78, 0xd522d0e, 0x0bb2f02,
-                               0x6d0302b, 0x370a08b, 0xc263405, 0x0c89ce5, 0x0000006};
+    constexpr int32_t t[9] = {-0xf060572, -0x1efb9f49, 0xe3951a8, 0xb548b4, 0x2b0bb2f, 0x22db40c, -0xbfac8f6, -0x18c68f67, 0x60c9};
     return t[i];
 }
-GRAPE_HD int32_t ONE(int i) {   // 2^280 mod p
-    constexpr int32_t t[10] = {0xa0e0d96, 0x6a56a28, 0x56d8f97, 0x1e6c92b, 0xee608fc,
-                               0x10581c8, 0x89f6e5c, 0x8c59c9e, 0x7359fa8, 0x0000000};
+GRAPE_HD int32_t P3(int i) {   // 3p
+    constexpr int32_t t[9] = {0x976f7d5, 0x11869112, 0x1555fa7b, -0x1ef012f2, 0x40918c7, 0x3448e12, 0xe07d28f, -0x529d71b, 0x912d};
     return t[i];
 }
-GRAPE_HD int32_t CMEM(int i) {   // 2^256 mod p: mul28(x*2^280, CMEM) = x*2^256
-    constexpr int32_t t[10] = {0x58f0d9d, 0x5d438dc, 0x70b3dd3, 0xeb28f5c, 0x62c0a78,
-                               0x6f78794, 0xf666ea3, 0x9a07df2, 0xe0a77c1, 0x0000000};
+GRAPE_HD int32_t DOWN(int i) {   // 2^-30 mod p: -0.43 p
+    constexpr int32_t t[9] = {0x1f7dceac, 0x193ed8c9, 0xa1f275e, 0xfa1c301, -0x1de4d6a1, 0x8aff355, -0x93e8175, -0x1142d07b, -0x14c6};
     return t[i];
 }
-// Montgomery (radix 2^256) form of 2^24, 32-bit limbs: mul(x*2^256, MCONV) = x*2^280 mod p
+GRAPE_HD int32_t ONE(int i) {   // 2^270 mod p
+    constexpr int32_t t[9] = {0x24fcf82, -0xe183b72, 0x1ac0210c, 0x1f4f4b0c, 0x100896b9, -0xae44a8a, -0x6d2519d, -0x1ab5fcf1, -0x8c8};
+    return t[i];
+}
+GRAPE_HD int32_t CMEM(int i) {   // 2^256 mod p: mul28(x*2^270, CMEM) = x*2^256
+    constexpr int32_t t[9] = {0x58f0d9d, 0xd750e37, 0x1c70b3dd, 0x1e3aca3d, -0x6b9d3f6, -0x572421e, -0x20d0999, 0x1df06682, 0xe0a};
+    return t[i];
+}
+// Montgomery (radix 2^256) form of 2^14, 32-bit limbs: mul(x*2^256, MCONV) = x*2^270 mod p
 GRAPE_HD uint32_t MCONV(int i) {
-    constexpr uint32_t t[8] = {0x8a0e0d96u, 0x976a56a2u, 0x92b56d8fu, 0x08fc1e6cu,
-                               0x581c8ee6u, 0x9f6e5c10u, 0x8c59c9e8u, 0x07359fa8u};
+    constexpr uint32_t t[8] = {0x5accccc9u, 0xf89a7d3au, 0x9a1dcc9du, 0x50fea7bdu, 0xdf1160f4u, 0x9e7d8ca3u, 0xed6d3304u, 0x279be39au};
     return t[i];
 }
-GRAPE_HD int32_t CIN(int i) {   // 2^304 mod p: mul28(pack(x*2^256), CIN) = x*2^280
-    constexpr int32_t t[10] = {0x8b6fea0, 0xa73d9f9, 0x09603cf, 0xb860a8d, 0x8b33888,
-                               0x9628387, 0xb8b8d5d, 0x9a84442, 0xe142fd5, 0x0000000};
+GRAPE_HD int32_t CIN(int i) {   // 2^284 mod p: mul28(pack(x*2^256), CIN) = x*2^270
+    constexpr int32_t t[9] = {-0x1019212e, -0x66eb814, -0x18cbc210, -0x103b9669, 0x63da561, 0x14d661fb, 0x15e36864, 0x1768c0ce, 0x1291};
+    return t[i];
+}
+GRAPE_HD int32_t R3(int i) {   // R'^3 mod p: turns the plain inverse of a Montgomery-form value back into Montgomery form
+    constexpr int32_t t[9] = {0x70aee79, 0x85cef6a, -0x17012488, 0x1859261c, 0x1a5cb6c3, -0x495f3be, 0x179e76b2, 0x17c5ea5a, 0x574};
     return t[i];
 }
 
 #else
 struct Fp28 {
-    int32_t v[14];
+    int32_t v[13];
 };
 
 namespace fp28 {
 
-constexpr int N = 14;
-constexpr int W = 28;
-constexpr uint32_t MASK = (1u << W) - 1;
-constexpr uint32_t PINV = 0xffcfffdu;   // -p^-1 mod 2^28
+constexpr int N = 13;
+constexpr int W = 30;
+constexpr bool kSmallDown = true;        // DOWN is far below p
+constexpr uint32_t PINV = 0x3ffcfffdu;   // -p^-1 mod 2^30
 
-GRAPE_HD int32_t P(int i) {
-    constexpr int32_t t[14] = {0xfffaaab, 0xfefffff, 0x3ffffb9, 0xfffeb15, 0x6241eab, 0xa0f6b0f, 0xf6730d2,
-                               0xf38512b, 0x4774b84, 0x4bacd76, 0xba7b643, 0xe69a4b1, 0x1ea397f, 0x001a011};
+GRAPE_HD int32_t P(int i) {   // balanced, as all tables of limbs here
+    constexpr int32_t t[13] = {-0x5555, -0x18040000, 0x153ffffc, -0x15000054, -0xf09dbe1, 0x34a83db, 0x112bf673,
+                               0x12e13ce1, -0x13289b89, 0x1ed90d2f, -0x165b4e46, -0x571a006, 0x1a0112};
     return t[i];
 }
 GRAPE_HD int32_t P2(int i) {   // 2p
-    constexpr int32_t t[14] = {0xfff5556, 0xfdfffff, 0x7ffff73, 0xfffd62a, 0xc483d57, 0x41ed61e, 0xece61a5,
-                               0xe70a257, 0x8ee9709, 0x9759aec, 0x74f6c86, 0xcd34963, 0x3d472ff, 0x0034022};
+    constexpr int32_t t[13] = {-0xaaaa, 0xff80000, -0x15800009, 0x15ffff59, -0x1e13b7c3, 0x69507b6, -0x1da8131a,
+                               -0x1a3d863d, 0x19aec8ef, -0x24de5a3, 0x13496375, -0xae3400d, 0x340224};
     return t[i];
 }
-GRAPE_HD int32_t ONE(int i) {   // 2^392 mod p
-    constexpr int32_t t[14] = {0x347fcb8, 0xd800000, 0x002b119, 0x0cde6d2, 0xc7212e0, 0x83a2090, 0x037669f,
-                               0xda0f73e, 0x9b09b42, 0x1297bb0, 0x515d98f, 0x012ca7c, 0x659fcfa, 0x000577a};
+GRAPE_HD int32_t P3(int i) {   // 3p
+    constexpr int32_t t[13] = {-0xffff, -0x80c0000, -0x40000d, 0xffff05, 0x12e26c5c, 0x9df8b90, -0xc7c1ca7,
+                               -0x75c495c, 0x6862d66, 0x1c8b278c, -0x311ead1, -0x1054e013, 0x4e0336};
     return t[i];
 }
-GRAPE_HD int32_t CMEM(int i) {   // 2^384 mod p: mul28(x*2^392, CMEM) = x*2^384
-    constexpr int32_t t[14] = {0x002fffd, 0x0900000, 0xc000276, 0x000bc40, 0x8baebf4, 0x5753c75, 0x55f4898,
-                               0x7052574, 0x7ce5853, 0x56ec6d7, 0x71a97a2, 0xe4935c0, 0xec3fa80, 0x0015f65};
+GRAPE_HD int32_t DOWN(int i) {   // 2^-30 mod p: -0.0002 p
+    constexpr int32_t t[13] = {0x80c0004, 0x4d203d, -0x4fe05, 0xc18fa4, -0x156fd71a, -0x16dd0ad7, 0x10b87b4d,
+                               0xc13f00b, -0x41741a5, -0x121d875c, -0xf9813a5, -0x383c1e2, -0x138};
     return t[i];
 }
-// Montgomery (radix 2^384) form of 2^8, 32-bit limbs: mul(x*2^384, MCONV) = x*2^392 mod p
+GRAPE_HD int32_t ONE(int i) {   // 2^390 mod p
+    constexpr int32_t t[13] = {0xd1ff2e, 0x19d80000, -0xb7ff53c, -0x11ff3219, 0x2431c85, -0x19607c5e, -0x2307f22,
+                               0x9b42da1, -0x1a113d94, 0x15d98f13, 0x4b29f14, -0x1a603060, 0x15dea};
+    return t[i];
+}
+GRAPE_HD int32_t CMEM(int i) {   // 2^384 mod p: mul28(x*2^390, CMEM) = x*2^384
+    constexpr int32_t t[13] = {0x35552, -0xfd80000, -0x147fffd4, 0x12000345, 0x166296cd, 0x1f16d974, 0x14485f81,
+                               0x3339f33, -0x69eca9, 0xb857c2d, 0x1f910eb7, -0x98fbfc1, -0x40ab3};
+    return t[i];
+}
+// Montgomery (radix 2^384) form of 2^6, 32-bit limbs: mul(x*2^384, MCONV) = x*2^390 mod p
 GRAPE_HD uint32_t MCONV(int i) {
-    constexpr uint32_t t[12] = {0x0347fcb8u, 0x19d80000u, 0x6d2002b1u, 0x12e00cdeu, 0xa2090c72u, 0x37669f83u,
-                                0xda0f73e0u, 0x09b09b42u, 0x8f1297bbu, 0xa7c515d9u, 0xfcfa012cu, 0x0577a659u};
+    constexpr uint32_t t[12] = {0x00d1ff2eu, 0x46760000u, 0x9b4800acu, 0x84b80337u, 0xe882431cu, 0x0dd9a7e0u,
+                                0xb683dcf8u, 0xc26c26d0u, 0x63c4a5eeu, 0x29f14576u, 0x7f3e804bu, 0x015de996u};
     return t[i];
 }
-GRAPE_HD int32_t CIN(int i) {   // 2^400 mod p: mul28(pack(x*2^384), CIN) = x*2^392
-    constexpr int32_t t[14] = {0x80e6299, 0x3500034, 0xeb12856, 0xdeb2699, 0xc988670, 0x4ef6697, 0x70983e8,
-                               0xa4e6fe9, 0x3e8a053, 0xecf271e, 0xc20d323, 0x6eb6385, 0x47f1286, 0x00156da};
+GRAPE_HD int32_t CIN(int i) {   // 2^396 mod p: mul28(pack(x*2^384), CIN) = x*2^390
+    constexpr int32_t t[13] = {-0xb7f3481, -0x1f3ffff, -0x1fbd4ed9, -0xcc8550, -0x21b4b2e, 0x1e015cf2, 0x5c540d,
+                               -0xb984e66, -0xad5925c, 0x19d89d1a, -0x1046501a, -0x7b737e8, 0x97730};
+    return t[i];
+}
+GRAPE_HD int32_t R3(int i) {   // R'^3 mod p: turns the plain inverse of a Montgomery-form value back into Montgomery form
+    constexpr int32_t t[13] = {0x1347c98d, -0x13de6b34, 0x1b027ceb, -0x14734a5b, 0x1214bbdf, 0xb5efd04, -0x6122f41,
+                               0x1b2b39a5, -0xd4ff49a, 0x1d1b6db5, -0x470f471, 0x12c853b8, 0x6d0af};
     return t[i];
 }
 
 #endif
+
+constexpr uint32_t MASK = (1u << W) - 1;
+constexpr int32_t HALF = 1 << (W - 1);
 
 GRAPE_HD Fp28 one() {
     Fp28 r;
@@ -129,153 +164,234 @@ GRAPE_HD Fp28 zero() {
 }
 
 // limb-wise, no carries: the caller tracks magnitudes
-GRAPE_HD Fp28 add(const Fp28& a, const Fp28& b) {
-    Fp28 r;
-#pragma unroll
-    for (int i = 0; i < N; i++) r.v[i] = a.v[i] + b.v[i];
-    return r;
-}
 GRAPE_HD Fp28 sub(const Fp28& a, const Fp28& b) {
     Fp28 r;
 #pragma unroll
     for (int i = 0; i < N; i++) r.v[i] = a.v[i] - b.v[i];
     return r;
 }
-GRAPE_HD Fp28 neg(const Fp28& a) {
-    Fp28 r;
-#pragma unroll
-    for (int i = 0; i < N; i++) r.v[i] = -a.v[i];
-    return r;
-}
 GRAPE_HD Fp28 cneg(const Fp28& a, bool flag) {
     Fp28 r;
+    const int32_t m = flag ? -1 : 0;
 #pragma unroll
-    for (int i = 0; i < N; i++) r.v[i] = flag ? -a.v[i] : a.v[i];
+    for (int i = 0; i < N; i++) r.v[i] = (a.v[i] ^ m) - m;
     return r;
 }
 
-// signed carry propagation: same value, limbs 0..N-2 in [0, 2^28)
+// signed carry propagation: same value, limbs 0..N-2 in [0, 2^30); any 32-bit limbs
 GRAPE_HD Fp28 normalize(const Fp28& a) {
     Fp28 r;
     int32_t c = 0;
 #pragma unroll
     for (int i = 0; i < N - 1; i++) {
-        int32_t t = a.v[i] + c;
-        r.v[i] = t & (int32_t)MASK;
-        c = t >> W;   // arithmetic
+        const int32_t t = (int32_t)((uint32_t)a.v[i] & MASK) + c;
+        r.v[i] = (int32_t)((uint32_t)t & MASK);
+        c = (a.v[i] >> W) + (t >> W);   // arithmetic
+    }
+    r.v[N - 1] = a.v[N - 1] + c;
+    return r;
+}
+GRAPE_HD int32_t low30(uint32_t a) { return (int32_t)(a << (32 - W)) >> (32 - W); }   // the nearest to zero of a's residues mod 2^30
+// same value, balanced (up to 2 over 2^29: the limbs' carries are taken side by side, not along a chain).  Limbs below
+// 3 * 2^29 - a sum or difference of two balanced numbers, a double - or, with ANY, any of 32 bits.
+template <bool ANY = false>
+GRAPE_HD Fp28 balance(const Fp28& a) {
+    Fp28 r;
+    int32_t c = 0;
+#pragma unroll
+    for (int i = 0; i < N - 1; i++) {
+        r.v[i] = low30((uint32_t)a.v[i]) + c;
+        c = ANY ? ((a.v[i] >> (W - 1)) + 1) >> 1 : (a.v[i] + HALF) >> W;
     }
     r.v[N - 1] = a.v[N - 1] + c;
     return r;
 }
 
-// Montgomery product a*b/R' (mod p), result normalised in (0, 3p).
-GRAPE_HD Fp28 mul(const Fp28& a, const Fp28& b) {
-    int64_t C[2 * N];
+// The columns of a double-width value, column k of weight 2^(30 k).  The upper ones hold 2^29 more than their value
+// from the start, so that cutting their low 30 bits off rounds to the nearest multiple of 2^30; with WIDE, the lower
+// ones 2^31 more, so that their upper word is the nearest multiple of 2^32.
+struct Columns {
+    int64_t c[2 * N - 1];
+};
+// c + a b as one multiply-add.  Left to itself the compiler reorders a column's sum - starting values last, as additions of
+// their own - and splits products with known factors: 150 instructions more in a mixed addition.  The annotation is
+// gone after the passes that would do so.
+GRAPE_HD void mad(int64_t& c, int32_t a, int32_t b) {
+    c += (int64_t)a * (int64_t)b;
+#if defined(__HIP_DEVICE_COMPILE__)
+    c = __builtin_annotation(c, "sum");
+#endif
+}
+template <class T>
+GRAPE_HD T unknown(T x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm("" : "+s"(x));
+#endif
+    return x;
+}
+template <bool WIDE>
+GRAPE_HD void start(Columns& t) {
+    const int64_t lower = WIDE ? unknown((int64_t)1 << 31) : 0, upper = unknown((int64_t)HALF);
 #pragma unroll
-    for (int k = 0; k < 2 * N; k++) C[k] = 0;
+    for (int k = 0; k < 2 * N - 1; k++) t.c[k] = k < N - 1 ? lower : k < N ? 0 : upper;
+}
+GRAPE_HD void add_row(Columns& t, int i, const int32_t* a, int32_t b) {
 #pragma unroll
-    for (int i = 0; i < N; i++) {
+    for (int j = 0; j < N; j++) mad(t.c[i + j], a[j], b);
+}
+// takes column i, which nothing is added to any more, out of the value
+template <bool WIDE>
+GRAPE_HD void reduce_column(Columns& t, int i) {
+    if (i < N - 1) {
+        int32_t m;
+        if (WIDE) {                      // a signed digit of 32 bits: one instruction less for the column's upper part
+            m = (int32_t)((uint32_t)t.c[i] ^ 0x80000000u);
+            mad(t.c[i + 1], (int32_t)(t.c[i] >> 32), unknown(4));
+        } else {
+            m = (int32_t)((uint32_t)t.c[i] & MASK);
+            t.c[i + 1] += t.c[i] >> W;
+        }
 #pragma unroll
-        for (int j = 0; j < N; j++) C[i + j] += (int64_t)a.v[j] * (int64_t)b.v[i];
-        const int32_t m = (int32_t)(((uint32_t)C[i] * PINV) & MASK);
+        for (int j = 0; j < N; j++) mad(t.c[i + 1 + j], m, DOWN(j));
+    } else {
+        const int32_t m = low30((uint32_t)t.c[i] * PINV);
 #pragma unroll
-        for (int j = 0; j < N; j++) C[i + j] += (int64_t)m * (int64_t)P(j);
-        C[i + 1] += C[i] >> W;   // C[i] is now a multiple of 2^28
+        for (int j = 0; j < N; j++) mad(t.c[i + j], m, P(j));
+        t.c[i + 1] += t.c[i] >> W;       // the column is a multiple of 2^30 now
     }
-    // the quotient may be slightly negative: add p, then carry-propagate
+}
+// the upper columns, carries propagated: the upper words along the columns, the two bits left over above a limb's 30 to the next limb
+GRAPE_HD Fp28 finish(Columns& t) {
     Fp28 r;
-    int64_t c = 0;
+    int32_t over = 0;
 #pragma unroll
     for (int k = 0; k < N - 1; k++) {
-        int64_t t = C[N + k] + (int64_t)P(k) + c;
-        r.v[k] = (int32_t)((uint32_t)t & MASK);
-        c = t >> W;
+        const uint32_t lo = (uint32_t)t.c[N + k];
+        const int32_t hi = (int32_t)(t.c[N + k] >> 32);
+        if (k < N - 2) mad(t.c[N + k + 1], hi, unknown(4));
+        r.v[k] = (int32_t)(lo & MASK) + over - HALF;
+        over = (int32_t)(lo >> W);
+        if (k == N - 2) r.v[N - 1] = (int32_t)((uint32_t)hi << 2) + over;
     }
-    r.v[N - 1] = (int32_t)(C[2 * N - 1] + (int64_t)P(N - 1) + c);
+    return r;
+}
+// the same less w * s: an addend costs a multiply-add a limb here, and the difference comes out balanced
+GRAPE_HD void less(Columns& t, int32_t& top, const Fp28& s, int32_t w) {
+    const int32_t f = unknown(-w);
+#pragma unroll
+    for (int k = 0; k < N - 1; k++) mad(t.c[N + k], s.v[k], f);
+    top += s.v[N - 1] * f;
+}
+
+// Montgomery product a*b/R' (mod p)
+template <bool WIDE>
+GRAPE_HD Fp28 mul_impl(const Fp28& a, const Fp28& b) {
+    Columns t;
+    start<WIDE>(t);
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        add_row(t, i, a.v, b.v[i]);
+        reduce_column<WIDE>(t, i);
+    }
+    return finish(t);
+}
+GRAPE_HD Fp28 mul(const Fp28& a, const Fp28& b) { return mul_impl<false>(a, b); }
+// both operands balanced: reduced in wide digits, 12 instructions less
+GRAPE_HD Fp28 mulb(const Fp28& a, const Fp28& b) { return mul_impl<true>(a, b); }
+// both operands balanced, the product below p (wide digits take DOWN twice: too much where that is near p / 2)
+GRAPE_HD Fp28 mulb_below_p(const Fp28& a, const Fp28& b) { return mul_impl<kSmallDown>(a, b); }
+// a*b/R' - s, both factors balanced
+GRAPE_HD Fp28 mulb_less(const Fp28& a, const Fp28& b, const Fp28& s) {
+    Columns t;
+    start<true>(t);
+    int32_t top = 0;
+    less(t, top, s, 1);
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        add_row(t, i, a.v, b.v[i]);
+        reduce_column<true>(t, i);
+    }
+    Fp28 r = finish(t);
+    r.v[N - 1] += top;
     return r;
 }
 
-// a*b - c*d with one Montgomery reduction: both products accumulate in the same columns.
-// Needs 14*(2^(la+lb) + 2^(lc+ld)) + 14*2^56 < 2^63 for the limb bounds and |ab| + |cd| <= 2^11 p^2
-// for the values; the result is normalised in (0, 3p) like a product.
+// a*b - c*d with one Montgomery reduction: both products accumulate in the same columns, so all four operands have to be
+// balanced.
 GRAPE_HD Fp28 mul_sub(const Fp28& a, const Fp28& b, const Fp28& c, const Fp28& d) {
-    int64_t C[2 * N];
-#pragma unroll
-    for (int k = 0; k < 2 * N; k++) C[k] = 0;
+    Columns t;
+    start<false>(t);
     int32_t nc[N];                        // limb-wise negation keeps every step a multiply-add
 #pragma unroll
     for (int j = 0; j < N; j++) nc[j] = -c.v[j];
 #pragma unroll
     for (int i = 0; i < N; i++) {
-#pragma unroll
-        for (int j = 0; j < N; j++) C[i + j] += (int64_t)a.v[j] * (int64_t)b.v[i];
-#pragma unroll
-        for (int j = 0; j < N; j++) C[i + j] += (int64_t)nc[j] * (int64_t)d.v[i];
-        const int32_t m = (int32_t)(((uint32_t)C[i] * PINV) & MASK);
-#pragma unroll
-        for (int j = 0; j < N; j++) C[i + j] += (int64_t)m * (int64_t)P(j);
-        C[i + 1] += C[i] >> W;
+        add_row(t, i, a.v, b.v[i]);
+        add_row(t, i, nc, d.v[i]);
+        reduce_column<false>(t, i);
     }
-    Fp28 r;
-    int64_t cy = 0;
-#pragma unroll
-    for (int k = 0; k < N - 1; k++) {
-        int64_t t = C[N + k] + (int64_t)P(k) + cy;
-        r.v[k] = (int32_t)((uint32_t)t & MASK);
-        cy = t >> W;
-    }
-    r.v[N - 1] = (int32_t)(C[2 * N - 1] + (int64_t)P(N - 1) + cy);
-    return r;
+    return finish(t);
 }
 
-// a^2/R': the off-diagonal limb products are taken once with a doubled operand.
-GRAPE_HD Fp28 sqr(const Fp28& a) {
-    int64_t C[2 * N];
-#pragma unroll
-    for (int k = 0; k < 2 * N; k++) C[k] = 0;
+// the columns of a^2 (a balanced): the off-diagonal limb products are taken once with a doubled operand
+template <bool WIDE>
+GRAPE_HD void square(Columns& t, const Fp28& a) {
     int32_t a2[N];
 #pragma unroll
     for (int i = 0; i < N; i++) a2[i] = a.v[i] * 2;
 #pragma unroll
     for (int i = 0; i < N; i++) {
-        C[2 * i] += (int64_t)a.v[i] * (int64_t)a.v[i];
+        mad(t.c[2 * i], a.v[i], a.v[i]);
 #pragma unroll
-        for (int j = i + 1; j < N; j++) C[i + j] += (int64_t)a2[i] * (int64_t)a.v[j];
+        for (int j = i + 1; j < N; j++) mad(t.c[i + j], a2[i], a.v[j]);
     }
 #pragma unroll
-    for (int i = 0; i < N; i++) {
-        const int32_t m = (int32_t)(((uint32_t)C[i] * PINV) & MASK);
-#pragma unroll
-        for (int j = 0; j < N; j++) C[i + j] += (int64_t)m * (int64_t)P(j);
-        C[i + 1] += C[i] >> W;
-    }
-    Fp28 r;
-    int64_t c = 0;
-#pragma unroll
-    for (int k = 0; k < N - 1; k++) {
-        int64_t t = C[N + k] + (int64_t)P(k) + c;
-        r.v[k] = (int32_t)((uint32_t)t & MASK);
-        c = t >> W;
-    }
-    r.v[N - 1] = (int32_t)(C[2 * N - 1] + (int64_t)P(N - 1) + c);
+    for (int i = 0; i < N; i++) reduce_column<WIDE>(t, i);
+}
+template <bool WIDE>
+GRAPE_HD Fp28 sqr_impl(const Fp28& a) {
+    Columns t;
+    start<WIDE>(t);
+    square<WIDE>(t, a);
+    return finish(t);
+}
+GRAPE_HD Fp28 sqr(const Fp28& a) { return sqr_impl<true>(a); }
+GRAPE_HD Fp28 sqr_below_p(const Fp28& a) { return sqr_impl<kSmallDown>(a); }
+// a^2/R' - s - 2u
+GRAPE_HD Fp28 sqr_less(const Fp28& a, const Fp28& s, const Fp28& u) {
+    Columns t;
+    start<true>(t);
+    int32_t top = 0;
+    less(t, top, s, 1);
+    less(t, top, u, 2);
+    square<true>(t, a);
+    Fp28 r = finish(t);
+    r.v[N - 1] += top;
     return r;
 }
 
-// Is a normalised value in [0, 3p) congruent to zero, i.e. one of 0, p, 2p?
-GRAPE_HD bool is_zero_mod_p(const Fp28& a) {
-    uint32_t z0 = 0, z1 = 0, z2 = 0;
+// Is a product below p congruent to zero?
+GRAPE_HD bool is_zero(const Fp28& a) {
+    uint32_t z = 0;
 #pragma unroll
-    for (int i = 0; i < N; i++) {
-        z0 |= (uint32_t)a.v[i];
-        z1 |= (uint32_t)(a.v[i] ^ P(i));
-        z2 |= (uint32_t)(a.v[i] ^ P2(i));
-    }
-    return (z0 == 0) | (z1 == 0) | (z2 == 0);
+    for (int i = 0; i < N; i++) z |= (uint32_t)a.v[i];
+    return z == 0;
+}
+// Is a value of up to a few p, one lazy operand, congruent to zero?
+GRAPE_HD bool is_zero_mod_p(const Fp28& a) { return is_zero(mul(a, one())); }
+
+// the value in [0, p), normalised, of a product below p
+GRAPE_HD Fp28 canonical(const Fp28& product) {
+    Fp28 t = normalize(product);
+    const int32_t neg = t.v[N - 1] >> 31;
+#pragma unroll
+    for (int i = 0; i < N; i++) t.v[i] += P(i) & neg;
+    return normalize(t);
 }
 
 // ---- conversions with the canonical 32-bit-limb Montgomery form (radix 2^384 resp. 2^256) ----
 constexpr int FW = FpParams::N;   // 32-bit words of the canonical form
-// pure re-limbing of a non-negative integer of FW words
+// pure re-limbing of a non-negative integer of FW words (normalised)
 GRAPE_HD Fp28 pack(const Fp& x) {
     Fp28 r;
 #pragma unroll
@@ -291,7 +407,7 @@ GRAPE_HD Fp unpack(const Fp28& a) {
     Fp r;
 #pragma unroll
     for (int q = 0; q < FW; q++) {
-        // word q covers bits [32q, 32q+32): limbs k0 = floor(32q/28) .. up to two more
+        // word q covers bits [32q, 32q+32): limbs k0 = floor(32q/30) .. up to two more
         const int k0 = (32 * q) / W;
         uint64_t acc = 0;
 #pragma unroll
@@ -310,47 +426,34 @@ GRAPE_HD Fp unpack(const Fp28& a) {
     }
     return r;
 }
-// canonical memory form (32-bit limbs) -> working form (28-bit limbs), canonical and normalised
+// canonical memory form (32-bit limbs) -> the value in [0, p) in the working form, balanced
 GRAPE_HD Fp28 from_canonical(const Fp& x) {
     Fp m;
 #pragma unroll
     for (int i = 0; i < FW; i++) m.v[i] = MCONV(i);
-    return pack(fmul(x, m));
+    return balance(pack(fmul(x, m)));
 }
-// the same conversion with the 28-bit multiplier only (a third of the instructions): the result is
-// normalised in (0, 3p) instead of canonical, which every consumer of a product accepts
+// the same conversion with the 30-bit multiplier only (a third of the instructions): a product, so in
+// (-p, p) instead of canonical
 GRAPE_HD Fp28 from_canonical_lazy(const Fp& x) {
     Fp28 c;
 #pragma unroll
     for (int i = 0; i < N; i++) c.v[i] = CIN(i);
     return mul(pack(x), c);
 }
-// value in (-9p, 3p), any limb form -> canonical memory form, 32-bit limbs
+// value of up to a few p, one lazy operand -> canonical memory form, 32-bit limbs
 GRAPE_HD Fp to_canonical(const Fp28& a) {
     Fp28 c;
 #pragma unroll
     for (int i = 0; i < N; i++) c.v[i] = CMEM(i);
-    Fp28 t = mul(normalize(a), c);   // in (0, 3p), now with the radix of the memory form
-    // subtract p while the result stays non-negative (at most twice)
-#pragma unroll
-    for (int rep = 0; rep < 2; rep++) {
-        Fp28 d;
-#pragma unroll
-        for (int i = 0; i < N; i++) d.v[i] = t.v[i] - P(i);
-        d = normalize(d);
-        const bool ok = d.v[N - 1] >= 0;
-#pragma unroll
-        for (int i = 0; i < N; i++) t.v[i] = ok ? d.v[i] : t.v[i];
-    }
-    return unpack(t);
+    return unpack(canonical(mul(a, c)));
 }
 
-// a^(p-2) in the 28-bit form (4-bit fixed windows, rolled loops); a in (-9p, 3p), a != 0 mod p.
-// Result normalised in (0, 3p).
+// a^(p-2) (4-bit fixed windows, rolled loops); a of up to a few p, one lazy operand, a != 0 mod p.
 GRAPE_HD Fp28 inverse(const Fp28& a) {
     Fp28 tbl[16];
     tbl[0] = one();
-    tbl[1] = mul(normalize(a), one());      // bring into (0, 3p)
+    tbl[1] = mul(a, one());
     for (int i = 2; i < 16; i++) tbl[i] = mul(tbl[i - 1], tbl[1]);
     Fp28 acc = one();
     bool started = false;
@@ -375,7 +478,7 @@ GRAPE_HD Fp28 inverse(const Fp28& a) {
 }
 
 // ------------------------------------------------------------------------------------------------
-// Modular inversion by divsteps (divstep.hpp) for the 28-bit form: about 800 divsteps for a 381-bit
+// Modular inversion by divsteps (divstep.hpp), whose limbs are of 30 bits too: about 800 divsteps for a 381-bit
 // modulus, i.e. some 27 batches of a few hundred instructions each - one inversion sits on the
 // critical path of every row epilogue.
 // ------------------------------------------------------------------------------------------------
@@ -385,8 +488,9 @@ using divstep::M30;
 using divstep::Mat;
 using divstep::divsteps30;
 
+constexpr int L = N;
+
 #if defined(GRAPE_CURVE_BN254)
-constexpr int L = 9;                        // 9 x 30 = 270 bits
 constexpr uint32_t PINV30 = 0x1b799c77u;    // p^-1 mod 2^30
 GRAPE_HD int32_t P30(int i) {
     constexpr int32_t t[9] = {0x187cfd47, 0x3082305b, 0x071ca8d3, 0x205aa45a, 0x01585d97,
@@ -394,7 +498,6 @@ GRAPE_HD int32_t P30(int i) {
     return t[i];
 }
 #else
-constexpr int L = 13;                       // 13 x 30 = 390 bits
 constexpr uint32_t PINV30 = 0x00030003u;    // p^-1 mod 2^30
 GRAPE_HD int32_t P30(int i) {
     constexpr int32_t t[13] = {0x3fffaaab, 0x27fbffff, 0x153ffffb, 0x2affffac, 0x30f6241e, 0x034a83da, 0x112bf673,
@@ -414,42 +517,15 @@ GRAPE_HD void update_de(int32_t* d, int32_t* e, const Mat& t) { divstep::update_
 
 }  // namespace by
 
-// R'^3 mod p: turns the plain inverse of a Montgomery-form value back into Montgomery form
-GRAPE_HD int32_t R3(int i) {
-#if defined(GRAPE_CURVE_BN254)
-    constexpr int32_t t[10] = {0xfdd47fe, 0xb246b8d, 0x1ffde25, 0xb55ed86, 0x14bbcde,
-                               0xad156f8, 0x483330b, 0x59ae72c, 0x1df6aee, 0x0000000};
-#else
-    constexpr int32_t t[14] = {0x1f7b890, 0x294cc4d, 0x9f3af22, 0xb5ba56c, 0xcb5c0cc, 0xc0d975c, 0xc89a8c5,
-                               0x6c968b4, 0x22672ea, 0x91de8c9, 0x35652a6, 0x84977c8, 0x424bbb9, 0x00141ab};
-#endif
-    return t[i];
-}
-
-// 1/a in Montgomery form (radix R') for a in (-9p, 3p), a != 0 mod p; result normalised in (0, 3p).
+// 1/a in Montgomery form (radix R') for a of up to a few p, one lazy operand, a != 0 mod p; a product.
 GRAPE_HD Fp28 inverse_by(const Fp28& a) {
     using namespace by;
     // canonical integer of a (still carrying the Montgomery factor) in [0, p)
-    Fp28 t = mul(normalize(a), one());
-#pragma unroll
-    for (int rep = 0; rep < 2; rep++) {
-        Fp28 dd;
-#pragma unroll
-        for (int i = 0; i < N; i++) dd.v[i] = t.v[i] - P(i);
-        dd = normalize(dd);
-        const bool ok = dd.v[N - 1] >= 0;
-#pragma unroll
-        for (int i = 0; i < N; i++) t.v[i] = ok ? dd.v[i] : t.v[i];
-    }
-    // re-limb N x 28 -> L x 30
+    const Fp28 t = canonical(mul(a, one()));
     int32_t f[L], g[L], d[L], e[L];
 #pragma unroll
     for (int k = 0; k < L; k++) {
-        const int bit = 30 * k, i0 = bit / W, sh = bit % W;
-        uint64_t w = (uint64_t)(uint32_t)t.v[i0] >> sh;
-        if (i0 + 1 < N) w |= (uint64_t)(uint32_t)t.v[i0 + 1] << (W - sh);
-        if (i0 + 2 < N && 2 * W - sh < 30) w |= (uint64_t)(uint32_t)t.v[i0 + 2] << (2 * W - sh);
-        g[k] = (int32_t)(w & (uint64_t)M30);
+        g[k] = t.v[k];
         f[k] = P30(k);
         d[k] = 0;
         e[k] = 0;
@@ -466,47 +542,29 @@ GRAPE_HD Fp28 inverse_by(const Fp28& a) {
         update_de(d, e, m);
         update_fg(f, g, m);
     }
-    // now g = 0, f = +-1 and d * a = f (mod p): the inverse is d * f; bring it into [0, p)
+    // now g = 0, f = +-1 and d * a = f (mod p): the inverse is d * f, in (-2p, 2p), |limbs| <= 2^30
     const int32_t fneg = f[L - 1] >> 31;          // all-ones when f = -1
-    int64_t c = 0;
-    int32_t x[L];
+    Fp28 x, r3;
 #pragma unroll
-    for (int k = 0; k < L; k++) x[k] = (d[k] ^ fneg) - fneg;   // limb-wise negation when f = -1
-    // x in (-2p, 2p): add 2p, then normalise (limbs to [0, 2^30), top signed but now positive)
-#pragma unroll
-    for (int k = 0; k < L - 1; k++) {
-        int64_t s = (int64_t)x[k] + 2 * (int64_t)P30(k) + c;
-        x[k] = (int32_t)s & M30;
-        c = s >> 30;
+    for (int k = 0; k < L; k++) {
+        x.v[k] = (d[k] ^ fneg) - fneg;            // limb-wise negation when f = -1
+        r3.v[k] = R3(k);
     }
-    x[L - 1] = (int32_t)((int64_t)x[L - 1] + 2 * (int64_t)P30(L - 1) + c);
-    // re-limb L x 30 -> N x 28 (value in (0, 4p), below 2^(32 FW))
-    Fp28 r;
-#pragma unroll
-    for (int k = 0; k < N; k++) {
-        const int bit = W * k, i0 = bit / 30, sh = bit % 30;
-        uint64_t w = (uint64_t)(uint32_t)x[i0] >> sh;
-        if (i0 + 1 < L) w |= (uint64_t)(uint32_t)x[i0 + 1] << (30 - sh);
-        r.v[k] = (int32_t)(w & (uint64_t)MASK);
-    }
-    Fp28 r3;
-#pragma unroll
-    for (int i = 0; i < N; i++) r3.v[i] = R3(i);
-    return mul(r, r3);   // 4 * 1 <= 2^11
+    return mul(x, r3);
 }
 
 }  // namespace fp28
 
 // ------------------------------------------------------------------------------------------------
-// XYZZ accumulator in the 28-bit form.  Invariants between additions:
-//   x in (-9p, 3p) normalised (signed top limb); y in (-3p, 3p) with |limbs| < 2^28;
-//   zz, zzz in (0, 3p) normalised, never congruent to zero; `inf` marks the identity.
+// XYZZ accumulator in the working form.  Invariants between additions: all coordinates balanced, |x| < 3.5p,
+// |y| < p, zz and zzz below p and never congruent to zero; `inf` marks the identity.  All of the values below stay
+// under 14 p, all products of them far under 630 p^2 (BN254: |y| < 1.5p).
 // ------------------------------------------------------------------------------------------------
 struct Xyzz28 {
     Fp28 x, y, zz, zzz;
     bool inf;
 };
-struct Affine28 {   // canonical coordinates (in [0,p), normalised)
+struct Affine28 {   // coordinates in (-p, p), balanced
     Fp28 x, y;
 };
 
@@ -544,38 +602,33 @@ GRAPE_HD Xyzz28 xyzz28_from_canonical(const G1Xyzz& a) {
 // untouched and the caller must take the exact slow path.
 GRAPE_HD bool xyzz28_madd(Xyzz28& acc, const Affine28& p, bool negate) {
     using namespace fp28;
+    const Fp28 py = cneg(p.y, negate);
     if (acc.inf) {
         acc.x = p.x;
-        acc.y = cneg(p.y, negate);
+        acc.y = py;
         acc.zz = one();
         acc.zzz = one();
         acc.inf = false;
         return true;
     }
-    const Fp28 U2 = mul(p.x, acc.zz);                  // 1 * 3            -> (0,3p)
-    const Fp28 S2 = mul(p.y, acc.zzz);                 // 1 * 3            -> (0,3p)
-    const Fp28 Pd = sub(U2, acc.x);                    // (-3p,12p), |limb| < 2^29
-    const Fp28 R = sub(cneg(S2, negate), acc.y);       // (-6p, 6p), |limb| < 2^29
-    const Fp28 PP = sqr(Pd);                           // 144 <= 2^11, 29+29 <= 58
-    const Fp28 ZZ3 = mul(acc.zz, PP);                  // 9
-    if (is_zero_mod_p(ZZ3)) return false;              // PP = 0  <=>  P = 0: doubling or cancellation
-    const Fp28 PPP = mul(Pd, PP);                      // 12 * 3 = 36
-    const Fp28 Q = mul(acc.x, PP);                     // 9 * 3 = 27
-    const Fp28 RR = sqr(R);                            // 36
-    Fp28 X3;
-#pragma unroll
-    for (int i = 0; i < N; i++) X3.v[i] = RR.v[i] - PPP.v[i] - 2 * Q.v[i];   // (-9p, 3p), |limb| < 2^30
-    X3 = normalize(X3);
-    const Fp28 T = sub(Q, X3);                         // (-3p, 12p), |limb| < 2^29
-    const Fp28 Y3 = mul_sub(R, T, acc.y, PPP);         // 6*12 + 3*3 = 81 <= 2^11; limbs 29+29, 28+28 -> (0, 3p)
-    acc.zzz = mul(acc.zzz, PPP);                       // 9
+    const Fp28 Pd = mulb_less(p.x, acc.zz, acc.x);      // U2 - X1
+    const Fp28 R = mulb_less(py, acc.zzz, acc.y);       // S2 - Y1
+    const Fp28 PP = sqr(Pd);
+    const Fp28 ZZ3 = mulb_below_p(acc.zz, PP);
+    if (is_zero(ZZ3)) return false;                    // PP = 0  <=>  P = 0: doubling or cancellation
+    const Fp28 PPP = mulb(Pd, PP);
+    const Fp28 Q = mulb(acc.x, PP);
+    const Fp28 X3 = sqr_less(R, PPP, Q);
+    const Fp28 T = balance(sub(Q, X3));
+    const Fp28 Y3 = mul_sub(R, T, acc.y, PPP);
+    acc.zzz = mulb(acc.zzz, PPP);
     acc.zz = ZZ3;
     acc.x = X3;
     acc.y = Y3;
     return true;
 }
 
-// acc <- 2 * acc in the 28-bit form (curve with a = 0, 6M + 3S: U = 2Y, V = U^2, W = U V, S = X V,
+// acc <- 2 * acc (curve with a = 0, 6M + 3S: U = 2Y, V = U^2, W = U V, S = X V,
 // M = 3 X^2, X3 = M^2 - 2S, Y3 = M (S - X3) - W Y, ZZ3 = V ZZ, ZZZ3 = W ZZZ).  No exceptional case on
 // a group of odd prime order; the identity stays the identity.
 GRAPE_HD void xyzz28_dbl(Xyzz28& acc) {
@@ -583,29 +636,26 @@ GRAPE_HD void xyzz28_dbl(Xyzz28& acc) {
     if (acc.inf) return;
     Fp28 U;
 #pragma unroll
-    for (int i = 0; i < N; i++) U.v[i] = 2 * acc.y.v[i];            // (-6p, 6p), |limb| < 2^29
-    const Fp28 V = sqr(U);                                          // 36
-    const Fp28 Wd = mul(U, V);                                      // 6 * 3
-    const Fp28 S = mul(acc.x, V);                                   // 9 * 3
-    const Fp28 X2 = sqr(acc.x);                                     // 81
+    for (int i = 0; i < N; i++) U.v[i] = 2 * acc.y.v[i];
+    U = balance(U);
+    const Fp28 V = sqr(U);
+    const Fp28 Wd = mulb(U, V);
+    const Fp28 S = mulb(acc.x, V);
+    const Fp28 X2 = sqr(acc.x);
     Fp28 M;
 #pragma unroll
-    for (int i = 0; i < N; i++) M.v[i] = 3 * X2.v[i];               // (0, 9p)
-    M = normalize(M);
-    const Fp28 MM = sqr(M);                                         // 81
-    Fp28 X3;
-#pragma unroll
-    for (int i = 0; i < N; i++) X3.v[i] = MM.v[i] - 2 * S.v[i];     // (-6p, 3p)
-    X3 = normalize(X3);
-    const Fp28 T = sub(S, X3);                                      // (-3p, 9p), |limb| < 2^29
-    const Fp28 Y3 = mul_sub(M, T, Wd, acc.y);                       // 81 + 9; limbs 28+29, 28+28
-    acc.zz = mul(V, acc.zz);                                        // 9
-    acc.zzz = mul(Wd, acc.zzz);                                     // 9
+    for (int i = 0; i < N; i++) M.v[i] = 3 * X2.v[i];
+    M = balance<true>(M);
+    const Fp28 X3 = sqr_less(M, zero(), S);
+    const Fp28 T = balance(sub(S, X3));
+    const Fp28 Y3 = mul_sub(M, T, Wd, acc.y);
+    acc.zz = mulb(V, acc.zz);
+    acc.zzz = mulb(Wd, acc.zzz);
     acc.x = X3;
     acc.y = Y3;
 }
 
-// acc += q, both accumulators in the 28-bit form (12M + 2S).  Returns false, leaving acc
+// acc += q, both accumulators in the working form (12M + 2S).  Returns false, leaving acc
 // untouched, in the exceptional cases q = +-acc; identities are handled here.
 GRAPE_HD bool xyzz28_add(Xyzz28& acc, const Xyzz28& q) {
     using namespace fp28;
@@ -614,25 +664,19 @@ GRAPE_HD bool xyzz28_add(Xyzz28& acc, const Xyzz28& q) {
         acc = q;
         return true;
     }
-    const Fp28 U1 = mul(acc.x, q.zz);                  // 9 * 3 = 27
-    const Fp28 U2 = mul(q.x, acc.zz);
-    const Fp28 S1 = mul(acc.y, q.zzz);                 // 3 * 3
-    const Fp28 S2 = mul(q.y, acc.zzz);
-    const Fp28 Pd = sub(U2, U1);                       // (-3p, 3p)
-    const Fp28 R = sub(S2, S1);                        // (-3p, 3p)
-    const Fp28 PP = sqr(Pd);                           // 9
-    const Fp28 ZZ3 = mul(mul(acc.zz, q.zz), PP);       // 9, 9
-    if (is_zero_mod_p(ZZ3)) return false;
-    const Fp28 PPP = mul(Pd, PP);                      // 9
-    const Fp28 Q = mul(U1, PP);                        // 9
-    const Fp28 RR = sqr(R);                            // 9
-    Fp28 X3;
-#pragma unroll
-    for (int i = 0; i < N; i++) X3.v[i] = RR.v[i] - PPP.v[i] - 2 * Q.v[i];   // (-9p, 3p)
-    X3 = normalize(X3);
-    const Fp28 T = sub(Q, X3);                         // (-3p, 12p)
-    const Fp28 Y3 = mul_sub(R, T, S1, PPP);            // 36 + 9
-    acc.zzz = mul(mul(acc.zzz, q.zzz), PPP);
+    const Fp28 U1 = mulb(acc.x, q.zz);
+    const Fp28 S1 = mulb(acc.y, q.zzz);
+    const Fp28 Pd = mulb_less(q.x, acc.zz, U1);         // U2 - U1
+    const Fp28 R = mulb_less(q.y, acc.zzz, S1);         // S2 - S1
+    const Fp28 PP = sqr(Pd);
+    const Fp28 ZZ3 = mulb_below_p(mulb(acc.zz, q.zz), PP);
+    if (is_zero(ZZ3)) return false;
+    const Fp28 PPP = mulb(Pd, PP);
+    const Fp28 Q = mulb(U1, PP);
+    const Fp28 X3 = sqr_less(R, PPP, Q);
+    const Fp28 T = balance(sub(Q, X3));
+    const Fp28 Y3 = mul_sub(R, T, S1, PPP);
+    acc.zzz = mulb(mulb(acc.zzz, q.zzz), PPP);
     acc.zz = ZZ3;
     acc.x = X3;
     acc.y = Y3;
@@ -653,16 +697,15 @@ GRAPE_HD G1Affine xyzz28_to_affine(const Xyzz28& a) {
 
 // ------------------------------------------------------------------------------------------------
 // Affine + affine with the inversion supplied by the caller (Montgomery's trick over many
-// independent additions: table generation).  Inputs are finite points with canonical coordinates.
+// independent additions: table generation).  Inputs are finite points with balanced coordinates in (-p, p).
 // ------------------------------------------------------------------------------------------------
-// a normalised value in [0, 2^k p) -> the representative in [0, p)
-template <int K>
+// a normalised value in [0, 4p) -> the representative in [0, p)
 GRAPE_HD Fp28 fp28_below_p(Fp28 t) {
 #pragma unroll
-    for (int s = K - 1; s >= 0; s--) {
+    for (int s = 1; s >= 0; s--) {
         Fp28 d;
 #pragma unroll
-        for (int i = 0; i < fp28::N; i++) d.v[i] = t.v[i] - fp28::P(i) * (1 << s);
+        for (int i = 0; i < fp28::N; i++) d.v[i] = t.v[i] - (s ? fp28::P2(i) : fp28::P(i));
         d = fp28::normalize(d);
         const bool ok = d.v[fp28::N - 1] >= 0;
 #pragma unroll
@@ -670,40 +713,40 @@ GRAPE_HD Fp28 fp28_below_p(Fp28 t) {
     }
     return t;
 }
-// denominator of the slope of e + f (x_e - x_f), or of 2 f (2 y_f) when `dbl`; a value congruent
+// denominator of the slope of e + f (x_e - x_f), or of 2 e (2 y_e) when `dbl`; a value congruent
 // to zero means that the sum is no finite affine addition (e = +-f, or a point of order two)
 GRAPE_HD Fp28 affine28_slope_den(const Affine28& e, const Affine28& f, bool dbl) {
     Fp28 r;
 #pragma unroll
-    for (int i = 0; i < fp28::N; i++) r.v[i] = dbl ? 2 * f.y.v[i] : e.x.v[i] - f.x.v[i];
+    for (int i = 0; i < fp28::N; i++) r.v[i] = dbl ? 2 * e.y.v[i] : e.x.v[i] - f.x.v[i];
     return r;
 }
-// e + f (2 f when `dbl`; then e must equal f) given dinv = 1 / affine28_slope_den(e, f, dbl), a
-// product output in (0, 3p): 3M + 1S (one more S for the doubling), coordinates canonical
+// e + f (2 e when `dbl`; then e must equal f) given dinv = 1 / affine28_slope_den(e, f, dbl), a
+// product: 3M + 1S (one more S for the doubling), coordinates in [0, p), normalised
 GRAPE_HD Affine28 affine28_add_given_inverse(const Affine28& e, const Affine28& f, bool dbl, const Fp28& dinv) {
     using namespace fp28;
     Fp28 num;
     if (dbl) {
-        const Fp28 xx = sqr(f.x);                       // (0, 3p)
+        const Fp28 xx = sqr(e.x);       // (of f, which a run of additions keeps, the limb products are kept in registers too)
 #pragma unroll
         for (int i = 0; i < N; i++) num.v[i] = 3 * xx.v[i];
-        num = normalize(num);                           // (0, 9p)
+        num = balance<true>(num);
     } else {
-        num = sub(e.y, f.y);                            // (-p, p)
+        num = sub(e.y, f.y);
     }
-    const Fp28 lam = mul(num, dinv);                    // 9 * 3 = 27 <= 2^11
-    const Fp28 ll = sqr(lam);                           // (0, 3p)
+    const Fp28 lam = mul(num, dinv);
+    const Fp28 ll = sqr_below_p(lam);
     Fp28 x3;
 #pragma unroll
-    for (int i = 0; i < N; i++) x3.v[i] = ll.v[i] - e.x.v[i] - f.x.v[i] + P2(i);   // (0, 5p)
-    x3 = fp28_below_p<3>(normalize(x3));
-    const Fp28 ly = mul(lam, sub(e.x, x3));             // 3 * 1
+    for (int i = 0; i < N; i++) x3.v[i] = ll.v[i] - e.x.v[i] - f.x.v[i] + P3(i);   // in (0, 4p) for coordinates in [0, p)
+    x3 = fp28_below_p(normalize(x3));
+    const Fp28 ly = mul(lam, balance(sub(e.x, x3)));
     Fp28 y3;
 #pragma unroll
-    for (int i = 0; i < N; i++) y3.v[i] = ly.v[i] - e.y.v[i] + P(i);               // (0, 4p)
+    for (int i = 0; i < N; i++) y3.v[i] = ly.v[i] - e.y.v[i] + P2(i);              // in (0, 3p)
     Affine28 r;
     r.x = x3;
-    r.y = fp28_below_p<2>(normalize(y3));
+    r.y = fp28_below_p(normalize(y3));
     return r;
 }
 

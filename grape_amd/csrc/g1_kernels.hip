@@ -24,7 +24,7 @@ __device__ __noinline__ Fp fp_sqr_outline(Fp a) { return sqr(a); }
 
 // Memory images in 32-bit words: an Fp element is FW words (12 for BLS12-381, 8 for BN254), an
 // affine point 2 FW, a Jacobian point 3 FW, an XYZZ point 4 FW; L28 is the limb count of the
-// 28-bit working form.
+// working form of fp28.hpp.
 constexpr int FW = FpParams::N;
 constexpr int L28 = fp28::N;
 
@@ -76,18 +76,18 @@ __device__ __forceinline__ Fr ld_fr8(const uint32_t* base, size_t i) {
     return r;
 }
 
-// Wide-table entry: an affine point in the 28-bit working form, x[L28] then y[L28] as 32-bit
-// words.  BLS12-381's 112 bytes are padded to 128, so that every gather is exactly one cache line;
-// BN254's 80 bytes are stored dense (a multiple of 16 bytes: the loads stay aligned, half of the
+// Wide-table entry: an affine point in the working form, x[L28] then y[L28] as 32-bit
+// words.  BLS12-381's 104 bytes are padded to 128, so that every gather is exactly one cache line;
+// BN254's 72 bytes are stored in 80 (a multiple of 16 bytes: the loads stay aligned, half of the
 // entries straddle two lines) - the table is 37.5 % smaller, which is what lets 15-bit windows fit
 // the table budget there.
-constexpr int kWideEntryWords = (2 * L28 <= 20) ? 2 * L28 : 32;
+constexpr int kWideEntryWords = (2 * L28 <= 20) ? 20 : 32;
 static_assert(kWideEntryWords % 4 == 0 && kWideEntryWords >= 2 * L28, "entry layout");
 __device__ __forceinline__ Affine28 ld_entry28(const uint32_t* table, size_t e) {
     const uint4* q = reinterpret_cast<const uint4*>(table + (size_t)kWideEntryWords * e);
-    uint4 w[L28 / 2];
+    uint4 w[(2 * L28 + 3) / 4];
 #pragma unroll
-    for (int i = 0; i < L28 / 2; i++) w[i] = q[i];
+    for (int i = 0; i < (2 * L28 + 3) / 4; i++) w[i] = q[i];
     const uint32_t* f = reinterpret_cast<const uint32_t*>(w);
     Affine28 r;
 #pragma unroll
@@ -97,13 +97,13 @@ __device__ __forceinline__ Affine28 ld_entry28(const uint32_t* table, size_t e) 
     }
     return r;
 }
-__device__ __forceinline__ void st_entry28(uint32_t* table, size_t e, const G1Affine& a) {
-    Fp28 x = fp28::from_canonical(a.x), y = fp28::from_canonical(a.y);
+// coordinates in [0, p), balanced
+__device__ __forceinline__ void st_entry28_raw(uint32_t* table, size_t e, const Affine28& a) {
     uint32_t f[kWideEntryWords];
 #pragma unroll
     for (int i = 0; i < L28; i++) {
-        f[i] = (uint32_t)x.v[i];
-        f[L28 + i] = (uint32_t)y.v[i];
+        f[i] = (uint32_t)a.x.v[i];
+        f[L28 + i] = (uint32_t)a.y.v[i];
     }
 #pragma unroll
     for (int i = 2 * L28; i < kWideEntryWords; i++) f[i] = 0;
@@ -111,49 +111,54 @@ __device__ __forceinline__ void st_entry28(uint32_t* table, size_t e, const G1Af
 #pragma unroll
     for (int i = 0; i < kWideEntryWords / 4; i++) q[i] = make_uint4(f[4 * i], f[4 * i + 1], f[4 * i + 2], f[4 * i + 3]);
 }
+__device__ __forceinline__ void st_entry28(uint32_t* table, size_t e, const G1Affine& a) {
+    st_entry28_raw(table, e, Affine28{fp28::from_canonical(a.x), fp28::from_canonical(a.y)});
+}
 __device__ __forceinline__ bool entry_is_inf(const Affine28& a) {
     uint32_t z = 0;
 #pragma unroll
     for (int i = 0; i < L28; i++) z |= (uint32_t)a.x.v[i] | (uint32_t)a.y.v[i];
     return z == 0;
 }
-// Per-lane partial accumulator in memory: x, y, zz, zzz (L28 words each), the identity flag and
-// padding = 64 words (256 bytes).
+// Per-lane partial accumulator in memory: x, y, zz, zzz (kCoordWords words each, a multiple of 8 bytes), the identity
+// flag and padding = 64 words (256 bytes).
 using geom::kPartialWords;
+constexpr int kCoordWords = (L28 + 1) & ~1;
+static_assert(4 * kCoordWords + 1 <= kPartialWords && kCoordWords % 2 == 0, "accumulator layout");
 __device__ __forceinline__ void st_partial28(uint32_t* base, size_t i, const Xyzz28& a) {
-    uint32_t f[64];
+    uint32_t f[kPartialWords];
+#pragma unroll
+    for (int k = 0; k < kPartialWords; k++) f[k] = 0;
 #pragma unroll
     for (int k = 0; k < L28; k++) {
         f[k] = (uint32_t)a.x.v[k];
-        f[L28 + k] = (uint32_t)a.y.v[k];
-        f[2 * L28 + k] = (uint32_t)a.zz.v[k];
-        f[3 * L28 + k] = (uint32_t)a.zzz.v[k];
+        f[kCoordWords + k] = (uint32_t)a.y.v[k];
+        f[2 * kCoordWords + k] = (uint32_t)a.zz.v[k];
+        f[3 * kCoordWords + k] = (uint32_t)a.zzz.v[k];
     }
-    f[4 * L28] = a.inf ? 1u : 0u;
-#pragma unroll
-    for (int k = 4 * L28 + 1; k < 64; k++) f[k] = 0;
+    f[4 * kCoordWords] = a.inf ? 1u : 0u;
     uint4* q = reinterpret_cast<uint4*>(base + geom::partial_word(i));
 #pragma unroll
-    for (int k = 0; k < 16; k++) q[k] = make_uint4(f[4 * k], f[4 * k + 1], f[4 * k + 2], f[4 * k + 3]);
+    for (int k = 0; k < kPartialWords / 4; k++) q[k] = make_uint4(f[4 * k], f[4 * k + 1], f[4 * k + 2], f[4 * k + 3]);
 }
 __device__ __forceinline__ Xyzz28 ld_partial28(const uint32_t* base, size_t i) {
     const uint4* q = reinterpret_cast<const uint4*>(base + geom::partial_word(i));
-    uint4 w[L28 + 1];
+    uint4 w[kCoordWords + 1];
 #pragma unroll
-    for (int k = 0; k < L28 + 1; k++) w[k] = q[k];
+    for (int k = 0; k < kCoordWords + 1; k++) w[k] = q[k];
     const uint32_t* f = reinterpret_cast<const uint32_t*>(w);
     Xyzz28 a;
 #pragma unroll
     for (int k = 0; k < L28; k++) {
         a.x.v[k] = (int32_t)f[k];
-        a.y.v[k] = (int32_t)f[L28 + k];
-        a.zz.v[k] = (int32_t)f[2 * L28 + k];
-        a.zzz.v[k] = (int32_t)f[3 * L28 + k];
+        a.y.v[k] = (int32_t)f[kCoordWords + k];
+        a.zz.v[k] = (int32_t)f[2 * kCoordWords + k];
+        a.zzz.v[k] = (int32_t)f[3 * kCoordWords + k];
     }
-    a.inf = f[4 * L28] != 0;
+    a.inf = f[4 * kCoordWords] != 0;
     return a;
 }
-// acc += q for two 28-bit accumulators, exceptional cases through the canonical-form addition
+// acc += q for two accumulators in the working form, exceptional cases through the canonical-form addition
 __device__ __forceinline__ void padd28(Xyzz28& acc, const Xyzz28& q) {
     if (!xyzz28_add(acc, q)) {
         G1Xyzz c = xyzz28_to_canonical(acc);
@@ -162,7 +167,7 @@ __device__ __forceinline__ void padd28(Xyzz28& acc, const Xyzz28& q) {
     }
 }
 
-// acc += +-entry through the 28-bit mixed addition; the rare exceptional step (entry = +-acc)
+// acc += +-entry through the mixed addition of the working form; the rare exceptional step (entry = +-acc)
 // goes through the exact canonical-form addition.
 __device__ __forceinline__ void madd28(Xyzz28& acc, const Affine28& e, bool negate) {
     if (entry_is_inf(e)) return;
@@ -270,7 +275,7 @@ __device__ __forceinline__ G1Xyzz shfl_down_xyzz(const G1Xyzz& a, int off) {
 __device__ __forceinline__ void madd(G1Xyzz& acc, const G1Affine& p, bool negate) { xyzz_add_affine(acc, p, negate); }
 __device__ __forceinline__ void padd(G1Xyzz& acc, const G1Xyzz& q) { xyzz_add(acc, q); }
 __device__ __forceinline__ void pdbl(G1Xyzz& acc) { xyzz_dbl(acc); }
-// 1/a for a canonical, non-zero a: through the 28-bit form and its divstep inversion (about ten
+// 1/a for a canonical, non-zero a: through the working form and its divstep inversion (about ten
 // thousand instructions) instead of the a^(p-2) ladder on saturated limbs (about six hundred thousand)
 __device__ __forceinline__ Fp fp_inverse_fast(const Fp& a) {
     return fp28::to_canonical(fp28::inverse_by(fp28::from_canonical_lazy(a)));
@@ -413,23 +418,10 @@ __device__ __forceinline__ void st_fp28(uint32_t* p, const Fp28& a) {
     for (int i = 0; i < kFp28Quads; i++) q[i] = make_uint4(f[4 * i], f[4 * i + 1], f[4 * i + 2], f[4 * i + 3]);
 }
 static_assert(4 * kFp28Quads <= kWideEntryWords, "a prefix product must fit the entry it is parked in");
-__device__ __forceinline__ void st_entry28_raw(uint32_t* table, size_t e, const Affine28& a) {
-    uint32_t f[kWideEntryWords];
-#pragma unroll
-    for (int i = 0; i < L28; i++) {
-        f[i] = (uint32_t)a.x.v[i];
-        f[L28 + i] = (uint32_t)a.y.v[i];
-    }
-#pragma unroll
-    for (int i = 2 * L28; i < kWideEntryWords; i++) f[i] = 0;
-    uint4* q = reinterpret_cast<uint4*>(table + (size_t)kWideEntryWords * e);
-#pragma unroll
-    for (int i = 0; i < kWideEntryWords / 4; i++) q[i] = make_uint4(f[4 * i], f[4 * i + 1], f[4 * i + 2], f[4 * i + 3]);
-}
 
 // One thread per (run of `run` consecutive k, window w, generator i); i is the fastest index, so a
 // wave reads and writes adjacent entries.
-__global__ void __launch_bounds__(kBlock) wide_extend_kernel(uint32_t* table, size_t N, uint32_t nw, uint32_t K, uint32_t have,
+__global__ void __launch_bounds__(kBlock, 2) wide_extend_kernel(uint32_t* table, size_t N, uint32_t nw, uint32_t K, uint32_t have,
                                                              uint32_t cnt, uint32_t run, int* degenerate) {
     const size_t t = (size_t)blockIdx.x * kBlock + threadIdx.x;
     const size_t per = (size_t)nw * N;
@@ -461,7 +453,8 @@ __global__ void __launch_bounds__(kBlock) wide_extend_kernel(uint32_t* table, si
         const Affine28 e = ld_entry28(table, e0 + (size_t)(k - 1) * N);
         const Fp28 dinv = fp28::mul(inv, ld_fp28(table + (size_t)kWideEntryWords * dst));
         inv = fp28::mul(inv, affine28_slope_den(e, f, k == have));
-        st_entry28_raw(table, dst, affine28_add_given_inverse(e, f, k == have, dinv));
+        const Affine28 sum = affine28_add_given_inverse(e, f, k == have, dinv);
+        st_entry28_raw(table, dst, Affine28{fp28::balance(sum.x), fp28::balance(sum.y)});
     }
 }
 
@@ -837,10 +830,10 @@ __global__ void __launch_bounds__(64) commit_sparse_strided_kernel(uint32_t* par
 }
 
 // Row epilogue: the partial sums of a row become one point, the point its affine image.  Three kernels:
-//   commit_reduce_lane_kernel  rows by the ten thousand: one lane per kept partial sum adds its share (107 wave
-//                              instructions per addition, the fewest, but chains of 7 additions at 18 us each)
+//   commit_reduce_lane_kernel  rows by the ten thousand: one lane per kept partial sum adds its share (88 wave
+//                              instructions per addition, the fewest, but chains of 7 additions at 15 us each)
 //   commit_reduce_quad_kernel  2^lg_qpr quads (quad28.hpp) per row, each adds its share, then a tree of shuffles
-//                              (154 wave instructions per addition, 5.1 us each)
+//                              (140 wave instructions per addition, 4.8 us each)
 //   quad_affine_kernel         the map to affine coordinates, a quad per row
 // geom::reduce_plan picks.  Bound: instruction latency - a SIMD issues hardly faster with two of these waves than with
 // one, so what counts is one wave per SIMD (workgroups of four waves spread evenly over a compute unit's
@@ -851,25 +844,27 @@ __global__ void __launch_bounds__(64) commit_sparse_strided_kernel(uint32_t* par
 // 32768 of 64: 1.08 -> 0.54.
 __device__ __forceinline__ quad::Acc ld_quad_partial(const uint32_t* base, size_t i) {
     const uint32_t* p = base + geom::partial_word(i);
-    const uint2* q = reinterpret_cast<const uint2*>(p + (threadIdx.x & 3) * L28);
+    const uint2* q = reinterpret_cast<const uint2*>(p + (threadIdx.x & 3) * kCoordWords);
+    uint2 w[kCoordWords / 2];
+#pragma unroll
+    for (int k = 0; k < kCoordWords / 2; k++) w[k] = q[k];
+    const uint32_t* f = reinterpret_cast<const uint32_t*>(w);
     quad::Acc a;
 #pragma unroll
-    for (int k = 0; k < L28 / 2; k++) {
-        const uint2 w = q[k];
-        a.v.v[2 * k] = (int32_t)w.x;
-        a.v.v[2 * k + 1] = (int32_t)w.y;
-    }
-    a.inf = p[4 * L28] != 0;
+    for (int k = 0; k < L28; k++) a.v.v[k] = (int32_t)f[k];
+    a.inf = p[4 * kCoordWords] != 0;
     return a;
 }
 __device__ __forceinline__ void st_quad_partial(uint32_t* base, size_t i, const quad::Acc& a) {
     uint32_t* p = base + geom::partial_word(i);
-    uint2* q = reinterpret_cast<uint2*>(p + (threadIdx.x & 3) * L28);
+    uint2* q = reinterpret_cast<uint2*>(p + (threadIdx.x & 3) * kCoordWords);
+    uint32_t f[kCoordWords];
 #pragma unroll
-    for (int k = 0; k < L28 / 2; k++) q[k] = make_uint2((uint32_t)a.v.v[2 * k], (uint32_t)a.v.v[2 * k + 1]);
-    if ((threadIdx.x & 3) == 0) p[4 * L28] = a.inf ? 1u : 0u;
+    for (int k = 0; k < kCoordWords; k++) f[k] = k < L28 ? (uint32_t)a.v.v[k] : 0u;
+#pragma unroll
+    for (int k = 0; k < kCoordWords / 2; k++) q[k] = make_uint2(f[2 * k], f[2 * k + 1]);
+    if ((threadIdx.x & 3) == 0) p[4 * kCoordWords] = a.inf ? 1u : 0u;
 }
-static_assert(L28 % 2 == 0, "a coordinate is moved as 8-byte words");
 __global__ void __launch_bounds__(kBlock) commit_reduce_quad_kernel(uint32_t* out, const uint32_t* partial, size_t rows, uint32_t nparts,
                                                                     uint32_t lg_qpr) {
     const int lane = threadIdx.x & 63;
@@ -949,7 +944,7 @@ __global__ void __launch_bounds__(kBlock) msm_multiples_kernel(uint32_t* table, 
     const Fp w = ld_fp(points + 3 * FW * (q / kMsmMultiples) + FW * (r < 2 ? r : 2));     // x, y, z, z
     quad::Acc p;
     p.inf = quad::perm<quad::ctrl(2, 2, 2, 2)>((int32_t)w.is_zero()) != 0;
-    const Fp28 v = fp28::from_canonical_lazy(w);                                           // (0, 3p)
+    const Fp28 v = fp28::from_canonical_lazy(w);
     const Fp28 zz = fp28::sqr(v);
     p.v = quad::select(quad::lanes<0>() | quad::lanes<1>(), v, quad::select(quad::lanes<2>(), zz, fp28::mul(zz, v)));
     quad::Acc acc = p;
@@ -992,7 +987,7 @@ __global__ void __launch_bounds__(kBlock) msm_window_kernel(uint32_t* partial, c
     }
     if (sub == 0) st_quad_partial(partial, (size_t)w * stride + g, acc);
 }
-// accumulators in the 28-bit form -> XYZZ points in the memory form, a lane per coordinate
+// accumulators in the working form -> XYZZ points in the memory form, a lane per coordinate
 __global__ void __launch_bounds__(64) quad_canonical_kernel(uint32_t* out, const uint32_t* sums, size_t n) {
     const size_t q = ((size_t)blockIdx.x * 64 + threadIdx.x) >> 2;
     if (q >= n) return;
@@ -1004,9 +999,9 @@ __global__ void __launch_bounds__(64) quad_canonical_kernel(uint32_t* out, const
 // commitment through the reference-format table (entry k * npoints + i = k * G_i, k < 256, canonical
 // affine points): the reference's algorithm (byte windows, 8 doublings between windows,
 // src/Hyrax.cu:46-167) re-ordered so that it fills the chip whatever the number of rows - one wave
-// per (row, window, column segment) sums its table entries in the 28-bit form, the row-reduction
+// per (row, window, column segment) sums its table entries in the working form, the row-reduction
 // kernel folds the lanes and segments of every (row, window), and a last kernel runs the Horner
-// chain over a row's windows.  A table entry is converted on the fly (one 28-bit product per
+// chain over a row's windows.  A table entry is converted on the fly (one product per
 // coordinate); no wide table has to be built, which is what single rows (Hyrax::open's blinding
 // row, single_commit) and rows too long for a wide table need.
 // ------------------------------------------------------------------------------------------------
@@ -1042,7 +1037,7 @@ __global__ void __launch_bounds__(kBlock, 2) commit_ref28_kernel(uint32_t* parti
             const G1Affine a = ld_affine(table, (size_t)idx * npoints + col);
             if (!a.is_inf()) {
                 Affine28 e;
-                e.x = fp28::from_canonical_lazy(a.x);      // in (0, 3p): fine for every product it enters
+                e.x = fp28::from_canonical_lazy(a.x);
                 e.y = fp28::from_canonical_lazy(a.y);
                 if (!xyzz28_madd(acc, e, neg)) {           // entry = +-accumulator: exact canonical-form addition
                     G1Xyzz c = xyzz28_to_canonical(acc);

@@ -3,10 +3,10 @@
 //
 // Why: the last steps of a commitment - the row sums, the map to affine coordinates, the one row of an
 // opening - are latency chains, and a lone wave issues an instruction about every 8 cycles here.  One
-// lane's general addition is 6850 instructions long (14 products); its products fall into four groups
-// of up to four independent ones, so a quad takes four products' time (about 2400 instructions), holds
-// 15 registers of state instead of 57 and runs a fraction of the code (17 KB of straight line instead of 55).
-// The price is throughput: 150 instead of 107 wave instructions per addition, so the accumulation
+// lane's general addition is 5600 instructions long (14 products); its products fall into four groups
+// of up to four independent ones, so a quad takes four products' time (about 2200 instructions), holds
+// 14 registers of state instead of 53 and runs a fraction of the code.
+// The price is throughput: 140 instead of 88 wave instructions per addition, so the accumulation
 // kernels, which fill the chip, keep one lane per accumulator.
 //
 // Every lane of a quad must be active and take the same branch.
@@ -48,7 +48,7 @@ __device__ __forceinline__ Fp28 select(int32_t mask, const Fp28& a, const Fp28& 
 }
 
 struct Acc {          // one lane's coordinate of a quad's accumulator
-    Fp28 v;           // invariants per coordinate as for Xyzz28
+    Fp28 v;           // balanced; values per coordinate as for Xyzz28 (|y| below 2p)
     bool inf;         // the same in all four lanes
 };
 __device__ __forceinline__ Acc identity() {
@@ -66,29 +66,30 @@ __device__ __forceinline__ void dbl(Acc& acc) {
     // lane 0: X^2, lane 1: V = (2Y)^2
     Fp28 w;
 #pragma unroll
-    for (int i = 0; i < N; i++) w.v[i] = acc.v.v[i] + (acc.v.v[i] & m1);         // 2y in (-6p, 6p), |limb| < 2^29
-    const Fp28 s1 = sqr(w);                                   // 81 at most; lanes 2, 3 unused
+    for (int i = 0; i < N; i++) w.v[i] = acc.v.v[i] + (acc.v.v[i] & m1);
+    w = balance(w);
+    const Fp28 s1 = sqr(w);                                   // lanes 2, 3 unused
     const Fp28 V = perm<kFrom1>(s1);
     Fp28 M = perm<kFrom0>(s1);
 #pragma unroll
-    for (int i = 0; i < N; i++) M.v[i] = 3 * M.v[i];          // (0, 9p)
-    M = normalize(M);
+    for (int i = 0; i < N; i++) M.v[i] = 3 * M.v[i];
+    M = balance<true>(M);
     // lane 0: S = X V, lane 1: W = 2Y V, lane 2: ZZ V, lane 3: M^2
-    const Fp28 s2 = mul(select(m3, M, w), select(m3, M, V));  // 27, 18, 9, 81
+    const Fp28 s2 = mulb(select(m3, M, w), select(m3, M, V));
     const Fp28 MM = perm<ctrl(3, 3, 3, 3)>(s2);
     const Fp28 Wd = perm<kFrom1>(s2);
     Fp28 X3;                                                  // only lane 0's is used
 #pragma unroll
     for (int i = 0; i < N; i++) X3.v[i] = MM.v[i] - 2 * s2.v[i];
-    X3 = normalize(X3);                                       // (-6p, 3p)
+    X3 = balance<true>(X3);
     // lane 0: M (S - X3), lane 1: W Y, lane 3: W ZZZ
-    const Fp28 s3 = mul(select(m0, M, Wd), select(m0, sub(s2, X3), acc.v));      // 81, 18, -, 18
+    const Fp28 s3 = mul(select(m0, M, Wd), select(m0, sub(s2, X3), acc.v));      // one lazy operand
     const Fp28 y0 = perm<kFrom0>(s3);
+    Fp28 y3;
 #pragma unroll
-    for (int i = 0; i < N; i++) {
-        const int32_t y3 = y0.v[i] - s3.v[i];
-        acc.v.v[i] = select(m0, X3.v[i], select(m1, y3, select(m2, s2.v[i], s3.v[i])));
-    }
+    for (int i = 0; i < N; i++) y3.v[i] = y0.v[i] - s3.v[i];
+    y3 = balance(y3);
+    acc.v = select(m0, X3, select(m1, y3, select(m2, s2, s3)));
 }
 
 // acc += q (the formulas of xyzz28_add, every exceptional case included): four products' time
@@ -101,11 +102,11 @@ __device__ __forceinline__ void add(Acc& acc, const Acc& q) {
     }
     const int32_t m0 = lanes<0>(), m1 = lanes<1>(), m2 = lanes<2>(), m01 = m0 | m1;
     // U1 = X1 ZZ2, S1 = Y1 ZZZ2, U2 = ZZ1 X2, S2 = ZZZ1 Y2
-    const Fp28 t = mul(acc.v, perm<kCross>(q.v));             // 27, 9, 27, 9
-    const Fp28 D = sub(perm<kCross>(t), t);                   // lanes 0, 1: P = U2 - U1, R = S2 - S1 in (-3p, 3p), |limb| < 2^28
+    const Fp28 t = mulb(acc.v, perm<kCross>(q.v));
+    const Fp28 D = balance(sub(perm<kCross>(t), t));          // lanes 0, 1: P = U2 - U1, R = S2 - S1
     // P^2, R^2, ZZ1 ZZ2, ZZZ1 ZZZ2
-    const Fp28 s2 = mul(select(m01, D, acc.v), select(m01, D, q.v));            // 9
-    const int zero = is_zero_mod_p(s2) ? 1 : 0;
+    const Fp28 s2 = mulb_below_p(select(m01, D, acc.v), select(m01, D, q.v));
+    const int zero = is_zero(s2) ? 1 : 0;
     if (perm<kFrom0>(zero)) {                                 // q = +-acc
         if (perm<kFrom1>(zero)) dbl(acc);
         else acc = identity();
@@ -113,18 +114,25 @@ __device__ __forceinline__ void add(Acc& acc, const Acc& q) {
     }
     const Fp28 PP = perm<kFrom0>(s2);
     // PPP, Q = U1 PP, ZZ3
-    const Fp28 s3 = mul(select(m0, D, select(m1, perm<kFrom0>(t), s2)), PP);    // 9
+    const Fp28 s3 = mulb(select(m0, D, select(m1, perm<kFrom0>(t), s2)), PP);
     const Fp28 PPP = perm<kFrom0>(s3);
     Fp28 X3;                                                  // only lane 1's is used: R^2 - PPP - 2Q
+    int32_t c = 0;
 #pragma unroll
-    for (int i = 0; i < N; i++) X3.v[i] = s2.v[i] - PPP.v[i] - 2 * s3.v[i];     // (-9p, 3p), |limb| < 2^30
-    X3 = normalize(X3);
+    for (int i = 0; i < N; i++) {                             // balanced as in balance(); a limb may pass 2^31, its half does not
+        const int32_t x = s2.v[i] - PPP.v[i];
+        const uint32_t limb = (uint32_t)x - 2 * (uint32_t)s3.v[i];
+        X3.v[i] = (i < N - 1 ? low30(limb) : (int32_t)limb) + c;
+        c = ((x >> 1) - s3.v[i] + HALF / 2) >> (W - 1);
+    }
     // S1 PPP, R (Q - X3), -, ZZZ1 ZZZ2 PPP
-    const Fp28 T = sub(s3, X3);                               // lane 1: (-3p, 12p), |limb| < 2^29
-    const Fp28 s4 = mul(select(m0, perm<kFrom1>(t), select(m1, D, s2)), select(m1, T, PPP));   // 9, 36, -, 9
+    const Fp28 T = sub(s3, X3);                               // lazy
+    const Fp28 s4 = mul(select(m0, perm<kFrom1>(t), select(m1, D, s2)), select(m1, T, PPP));
     const Fp28 sp = perm<kFrom0>(s4), x3 = perm<kFrom1>(X3);
+    Fp28 y3;
 #pragma unroll
-    for (int i = 0; i < N; i++) acc.v.v[i] = select(m0, x3.v[i], select(m2, s3.v[i], s4.v[i] - (sp.v[i] & m1)));
+    for (int i = 0; i < N; i++) y3.v[i] = s4.v[i] - (sp.v[i] & m1);
+    acc.v = select(m0, x3, select(m2, s3, balance(y3)));
 }
 
 // 30 divsteps on the low words f, g (lane 0: x1 = f, x2 = g), the columns of the transition matrix in the same registers
@@ -146,24 +154,17 @@ __device__ __forceinline__ int32_t divsteps30(int32_t delta, int32_t& x1, int32_
     return -nd;
 }
 
-// 1/a for the same a in all four lanes (a in (-9p, 3p), not 0 mod p); result normalised in (0, 3p), the same in all
+// 1/a for the same a in all four lanes (up to a few p, not 0 mod p); a product, the same in all
 // four lanes.  inverse_by of fp28.hpp with one of the vectors f, g, d, e per lane: a batch's update of the
 // four vectors is one row of multiply-adds instead of four.
 __device__ __forceinline__ Fp28 inverse_by(const Fp28& a) {
     using namespace fp28;
     using namespace fp28::by;
     const int32_t m0 = lanes<0>(), m1 = lanes<1>(), m2 = lanes<2>(), m3 = lanes<3>();
-    const Fp28 t = fp28_below_p<2>(fp28::mul(normalize(a), one()));   // canonical integer in [0, p), still with the Montgomery factor
+    const Fp28 t = canonical(fp28::mul(a, one()));            // integer in [0, p), still with the Montgomery factor
     int32_t x[L];                                             // lane 0: f, 1: g, 2: d, 3: e
 #pragma unroll
-    for (int k = 0; k < L; k++) {
-        const int bit = 30 * k, i0 = bit / W, sh = bit % W;
-        uint64_t w = (uint64_t)(uint32_t)t.v[i0] >> sh;
-        if (i0 + 1 < N) w |= (uint64_t)(uint32_t)t.v[i0 + 1] << (W - sh);
-        if (i0 + 2 < N && 2 * W - sh < 30) w |= (uint64_t)(uint32_t)t.v[i0 + 2] << (2 * W - sh);
-        const int32_t g = (int32_t)(w & (uint64_t)M30);
-        x[k] = (P30(k) & m0) | (g & m1) | (k == 0 ? m3 & 1 : 0);
-    }
+    for (int k = 0; k < L; k++) x[k] = (P30(k) & m0) | (t.v[k] & m1) | (k == 0 ? m3 & 1 : 0);
     int32_t delta = 1;
     const int32_t de = m2 | m3, ge = m1 | m3;
     for (int batch = 0; batch < kBatches; batch++) {
@@ -192,23 +193,13 @@ __device__ __forceinline__ Fp28 inverse_by(const Fp28& a) {
         }
         x[L - 1] = (int32_t)c;
     }
-    // g = 0, f = +-1, d * a = f (mod p): d to every lane, negated when f = -1, brought into (0, 4p)
+    // g = 0, f = +-1, d * a = f (mod p): d, in (-2p, p) with limbs below 2^30, to every lane, negated when f = -1
     const int32_t fneg = perm<kFrom0>(x[L - 1]) >> 31;
-    int64_t c = 0;
+    Fp28 out, r3;
 #pragma unroll
     for (int k = 0; k < L; k++) {
         const int32_t d = perm<ctrl(2, 2, 2, 2)>(x[k]);
-        const int64_t s = (int64_t)((d ^ fneg) - fneg) + 2 * (int64_t)P30(k) + c;
-        x[k] = k < L - 1 ? ((int32_t)s & M30) : (int32_t)s;
-        c = s >> 30;
-    }
-    Fp28 out, r3;
-#pragma unroll
-    for (int k = 0; k < N; k++) {
-        const int bit = W * k, i0 = bit / 30, sh = bit % 30;
-        uint64_t w = (uint64_t)(uint32_t)x[i0] >> sh;
-        if (i0 + 1 < L) w |= (uint64_t)(uint32_t)x[i0 + 1] << (30 - sh);
-        out.v[k] = (int32_t)(w & (uint64_t)MASK);
+        out.v[k] = (d ^ fneg) - fneg;
         r3.v[k] = R3(k);
     }
     return fp28::mul(out, r3);

@@ -520,8 +520,8 @@ def g1_table_gen(gens, W):
     return out
 
 
-# 32-bit words of a wide-table entry: 2 x 14 limbs padded to 32 (one cache line) on BLS12-381,
-# 2 x 10 limbs stored dense on BN254
+# 32-bit words of a wide-table entry: 2 x 13 limbs padded to 32 (one cache line) on BLS12-381,
+# 2 x 9 limbs padded to 20 on BN254
 WIDE_ENTRY_WORDS = 20 if _capi.CURVE == "bn254" else 32
 
 
@@ -539,15 +539,15 @@ def wide_table_entries_to_host(table, idx):
     """decode entries of a wide table into affine points (x, y) as Python integers
     (None for the identity); for tests."""
     if _capi.CURVE == "bn254":
-        P, L = 21888242871839275222246405745257275088696311157297823662689037894645226208583, 10
+        P, L = 21888242871839275222246405745257275088696311157297823662689037894645226208583, 9
     else:
-        P, L = 0x1a0111ea397fe69a4b1ba7b6434bacd764774b84f38512bf6730d2a0f6b0f6241eabfffeb153ffffb9feffffffffaaab, 14
-    rinv = pow(1 << (28 * L), -1, P)
+        P, L = 0x1a0111ea397fe69a4b1ba7b6434bacd764774b84f38512bf6730d2a0f6b0f6241eabfffeb153ffffb9feffffffffaaab, 13
+    rinv = pow(1 << (30 * L), -1, P)
     rows = table[idx].cpu().numpy()
     out = []
     for r in rows:
-        x = sum(int(r[i]) << (28 * i) for i in range(L))
-        y = sum(int(r[L + i]) << (28 * i) for i in range(L))
+        x = sum(int(r[i]) << (30 * i) for i in range(L))
+        y = sum(int(r[L + i]) << (30 * i) for i in range(L))
         out.append(None if (x == 0 and y == 0) else (x * rinv % P, y * rinv % P))
     return out
 

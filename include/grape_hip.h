@@ -453,8 +453,8 @@ int grape_g1_table_gen(uint32_t *d_table_affine, const uint32_t *d_gens_affine, 
  * nw = 32, K = 128 a 255-bit scalar is 32 signed-digit additions into a single accumulator.
  * The table is private to this library (only the commitment entry points read it): each entry
  * holds the affine coordinates in the working form of the commitment kernels - on BLS12-381
- * 2 x 14 limbs of 28 bits (Montgomery radix 2^392) padded to 128 bytes, so a gather is exactly one
- * cache line; on BN254 2 x 10 limbs (radix 2^280) stored dense in 80 bytes.
+ * 2 x 13 signed limbs of 30 bits (Montgomery radix 2^390) padded to 128 bytes, so a gather is exactly one
+ * cache line; on BN254 2 x 9 limbs (radix 2^270) in 80 bytes.
  * Size: grape_g1_wide_table_bytes(N, nw, K) = nw*K*N entries of 128 bytes (80 in the BN254 build).
  */
 int grape_g1_wide_table_gen(uint32_t *d_table_affine, const uint32_t *d_gens_affine, size_t N, uint32_t c, uint32_t nw,
