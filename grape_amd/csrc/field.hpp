@@ -186,6 +186,33 @@ struct alignas(16) Mont {
 namespace detail {
 
 // One word of a carry / borrow chain (carry and borrow are 0 or 1).  With clang the builtins become
+// c + a b as one multiply-add: a column of a product.  Left to itself the compiler reorders a column's sum - starting
+// values last, as additions of their own - and splits products with known factors (150 instructions more in a mixed
+// addition of fp28.hpp).  The annotation is gone after the passes that would do so.
+GRAPE_HD void keep_sum(int64_t& c) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    c = __builtin_annotation(c, "sum");
+#else
+    (void)c;
+#endif
+}
+GRAPE_HD void mad(int64_t& c, int32_t a, int32_t b) {
+    c += (int64_t)a * (int64_t)b;
+    keep_sum(c);
+}
+GRAPE_HD void madu(int64_t& c, uint32_t a, uint32_t b) {
+    c = (int64_t)((uint64_t)c + (uint64_t)a * (uint64_t)b);
+    keep_sum(c);
+}
+// a value, the same in all lanes, that the compiler is not to know
+template <class T>
+GRAPE_HD T unknown(T x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm("" : "+s"(x));
+#endif
+    return x;
+}
+
 // one add-with-carry / subtract-with-borrow instruction per word on the device (64-bit emulation of
 // the chain costs three to four times as many instructions there); other compilers spell it out.
 GRAPE_HD uint32_t adc32(uint32_t a, uint32_t b, uint32_t& carry) {

@@ -43,6 +43,9 @@ struct Fp28 {
 
 namespace fp28 {
 
+using detail::mad;
+using detail::unknown;
+
 constexpr int N = 9;
 constexpr int W = 30;
 constexpr bool kSmallDown = false;
@@ -92,6 +95,9 @@ struct Fp28 {
 };
 
 namespace fp28 {
+
+using detail::mad;
+using detail::unknown;
 
 constexpr int N = 13;
 constexpr int W = 30;
@@ -213,22 +219,6 @@ GRAPE_HD Fp28 balance(const Fp28& a) {
 struct Columns {
     int64_t c[2 * N - 1];
 };
-// c + a b as one multiply-add.  Left to itself the compiler reorders a column's sum - starting values last, as additions of
-// their own - and splits products with known factors: 150 instructions more in a mixed addition.  The annotation is
-// gone after the passes that would do so.
-GRAPE_HD void mad(int64_t& c, int32_t a, int32_t b) {
-    c += (int64_t)a * (int64_t)b;
-#if defined(__HIP_DEVICE_COMPILE__)
-    c = __builtin_annotation(c, "sum");
-#endif
-}
-template <class T>
-GRAPE_HD T unknown(T x) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    asm("" : "+s"(x));
-#endif
-    return x;
-}
 template <bool WIDE>
 GRAPE_HD void start(Columns& t) {
     const int64_t lower = WIDE ? unknown((int64_t)1 << 31) : 0, upper = unknown((int64_t)HALF);

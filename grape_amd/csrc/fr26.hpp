@@ -171,6 +171,51 @@ GRAPE_HD Limbs reduce(Acc& C, int add_r) {
     r.v[N - 1] = (int32_t)(C.c[2 * N - 1] + (int64_t)add_r * (int64_t)R(N - 1) + c);
     return r;
 }
+// A single product reduced in wide digits: a * b / 2^260 + add_r * r as reduce gives it, with 0 <= M < (1 + 2^-20) 2^260;
+// |a limb| * |b limb| up to 2^57, 0 <= add_r < 32.  r = 1 mod 2^26, so a column leaves the sum as m times (r - 1) / 2^26 in
+// the next ones, with m the column's distance to the next multiple of 2^26 - or of 2^32: then its upper word goes to
+// the next column in one multiply-add, and m is the complement of its lower one if the column holds 2^32 - 1 more than the sum
+// (11 instructions a column instead of 14).  m below 2^32 makes the columns grow by 2^61.2; in the value only the
+// last column's counts, which is cut at 2^26.  For products on their own: beside accumulators that fill the registers the
+// plain sum above is faster, whose order the compiler is free in (tl_round_kernel 0.76 against 0.84 ms at 2^24 index
+// pairs, the five-sum weighted round 1.18 against 1.22; the rounds without a middle coefficient 0.96 -> 0.91).
+GRAPE_HD Limbs product(const Limbs& a, const Limbs& b, int add_r) {
+    using detail::mad;
+    Acc C;
+    const int64_t start = detail::unknown((int64_t)0xffffffff);
+#pragma unroll
+    for (int k = 0; k < 2 * N; k++) C.c[k] = k < N - 1 ? start : 0;
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+#pragma unroll
+        for (int j = 0; j < N; j++) mad(C.c[i + j], a.v[i], b.v[j]);
+    }
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        if (i < N - 1) {
+            const uint32_t m = ~(uint32_t)C.c[i];
+            mad(C.c[i + 1], (int32_t)(C.c[i] >> 32), detail::unknown(1 << (32 - W)));
+#pragma unroll
+            for (int j = 1; j < N; j++) detail::madu(C.c[i + j], m, (uint32_t)R(j));
+        } else {
+            const int32_t m = (int32_t)((0u - (uint32_t)C.c[i]) & MASK) + add_r * (1 << W);
+            C.c[i] += (int64_t)m;
+#pragma unroll
+            for (int j = 1; j < N; j++) mad(C.c[i + j], m, R(j));
+            C.c[i + 1] += C.c[i] >> W;
+        }
+    }
+    Limbs r;
+    int64_t c = 0;
+#pragma unroll
+    for (int k = 0; k < N - 1; k++) {
+        const int64_t t = C.c[N + k] + c;
+        r.v[k] = (int32_t)((uint32_t)t & MASK);
+        c = t >> W;
+    }
+    r.v[N - 1] = (int32_t)(C.c[2 * N - 1] + c);
+    return r;
+}
 // subtract r up to `times` times while the value stays non-negative: [0, (times+1) r) -> [0, r)
 GRAPE_HD Limbs canon(Limbs t, int times) {
     for (int rep = 0; rep < times; rep++) {
@@ -205,10 +250,7 @@ GRAPE_HD Fr limb_sum_to_fr(const Limbs& s, int add_r) {
 
 // canonical product of two memory-form elements (memory form out): 16ab < 16 r^2 -> (0, 1.46r)
 GRAPE_HD Fr mulc(const Fr& a, const Fr& b) {
-    Acc C;
-    acc_zero(C);
-    mac(C, pack16(a), pack(b));
-    return unpack(canon(reduce(C, 0), 1));
+    return unpack(canon(product(pack16(a), pack(b), 0), 1));
 }
 // a finished column sum of memory-form products (value/2^260 within (-lo_r, hi_r) multiples of
 // r, lo_r + hi_r + 1 <= 34) -> canonical memory form of the sum of products

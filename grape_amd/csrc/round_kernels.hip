@@ -84,6 +84,16 @@ __device__ __forceinline__ void wround2_result(uint32_t* out, const Fr* acc) {
     }
 }
 
+// e * x reduced, add_r times r added.  TIGHT: as a plain sum (the five-sum form is at the limit of the registers).
+template <bool TIGHT>
+__device__ __forceinline__ fr26::Limbs weight_product(const fr26::Limbs& e16, const fr26::Limbs& x, int add_r) {
+    if (!TIGHT) return fr26::product(e16, x, add_r);
+    fr26::Acc T;
+    fr26::acc_zero(T);
+    fr26::mac(T, e16, x);
+    return fr26::reduce(T, add_r);
+}
+
 // UNIT: the caller states that A[i] * (S[i] + beta) = 1 at every index (the first round of a logUp
 // proof, where A was made as the inverse of S + beta).  Then the constant coefficient is the sum of
 // the weights and the value at t = 1 equals it, so only the top coefficient sum_g e * dA * dS is
@@ -106,6 +116,7 @@ __global__ void __launch_bounds__(kBlock, 2) wround2_kernel(uint32_t* Aw, uint32
                                                          const int32_t* __restrict__ idx1 = nullptr, const uint32_t* Bt = nullptr,
                                                          const uint32_t* Eh = nullptr, uint32_t period = 1) {
     constexpr int NV = PLAIN ? 5 : 3;
+    constexpr bool TIGHT = PLAIN && !UNIT && !NOMID;
     __shared__ Fr lds[NV * (kBlock / 64)];
     fr26::Limbs w1;
     if (!TAB) w1 = fr26::weight16(ld_fr(v, 0));
@@ -141,16 +152,9 @@ __global__ void __launch_bounds__(kBlock, 2) wround2_kernel(uint32_t* Aw, uint32
             a1 = ld_hi26(A, g, n_out, in_size);
         }
         const fr26::Limbs da = fr26::sub(a1, a0);
-        fr26::Acc T;
         fr26::Limbs ea0;
-        if (!UNIT) {
-            fr26::acc_zero(T);
-            fr26::mac(T, e16, a0);
-            ea0 = fr26::reduce(T, 0);
-        }
-        fr26::acc_zero(T);
-        fr26::mac(T, e16, da);
-        const fr26::Limbs ead = fr26::reduce(T, 1);
+        if (!UNIT) ea0 = weight_product<TIGHT>(e16, a0, 0);
+        const fr26::Limbs ead = weight_product<TIGHT>(e16, da, 1);
         if (PLAIN) {
             sa0 = fr26::add(sa0, a0);
             sa1 = fr26::add(sa1, a1);
@@ -173,8 +177,8 @@ __global__ void __launch_bounds__(kBlock, 2) wround2_kernel(uint32_t* Aw, uint32
     }
     // offsets: |W0| < 71 r^2 -> within 2 r, |W2| < 60 r^2 -> within 1.7 r, |WQ| < 189 r^2 -> within 5.4 r
     Fr acc[NV];
-    acc[0] = reduce_to_fr(W0, 3);
-    acc[1] = NOMID ? Fr::zero() : reduce_to_fr(WQ, 6);
+    acc[0] = UNIT ? Fr::zero() : reduce_to_fr(W0, 3);
+    acc[1] = UNIT || NOMID ? Fr::zero() : reduce_to_fr(WQ, 6);
     acc[2] = reduce_to_fr(W2, 3);
     if (SPLIT) {
         const Fr el = ld_fr(E, low);

@@ -147,17 +147,10 @@ __global__ void __launch_bounds__(64 * (TABLE ? 6 : 3)) round_sums_kernel(RoundS
     } else if (!mb && a.beta) {
         m = fr26::add(m, fr26::pack(ld_fr(a.beta, 0)));
     }
-    fr26::Acc C;
 #pragma unroll
     for (int i = 0; i < fr26::N; i++) l.v[i] *= 16;
-    fr26::acc_zero(C);
-    fr26::mac(C, l, m);
-    fr26::Limbs p = fr26::reduce(C, 0);
-    if (weighted) {
-        fr26::acc_zero(C);
-        fr26::mac(C, fr26::pack16(e), p);
-        p = fr26::reduce(C, 0);
-    }
+    fr26::Limbs p = fr26::product(l, m, 0);
+    if (weighted) p = fr26::product(fr26::pack16(e), p, 0);
     const Fr sum = wave_limb_sum(p, kind != 2 ? 0 : weighted ? 4 : 8);
     uint32_t* slot = a.partial + 8 * (size_t)NV * blockIdx.x;
     if ((threadIdx.x & 63) == 0) st_fr(slot, mb ? q + 2 : q, sum);

@@ -1,7 +1,8 @@
-// The field products of grape_amd/csrc/fp28.hpp on limbs as they are, so that the CPU test-suite can put operands at the
-// bounds of their columns.
+// The field products of grape_amd/csrc/fp28.hpp and fr26.hpp on limbs as they are, so that the CPU test-suite can put
+// operands at the bounds of their columns.
 #include <cstring>
 #include "../../grape_amd/csrc/fp28.hpp"
+#include "../../grape_amd/csrc/fr26.hpp"
 using namespace grape;
 
 static Fp28 load(const int32_t* p) {
@@ -30,6 +31,13 @@ void fp28_apply(int op, const int32_t* a, const int32_t* b, const int32_t* s, co
     case 10: r = fp28::canonical(fp28::mul(A, B)); break;
     default: r = fp28::zero();
     }
+    memcpy(out, r.v, sizeof r.v);
+}
+void fr26_product(const int32_t* a, const int32_t* b, int add_r, int32_t* out) {
+    fr26::Limbs A, B;
+    memcpy(A.v, a, sizeof A.v);
+    memcpy(B.v, b, sizeof B.v);
+    const fr26::Limbs r = fr26::product(A, B, add_r);
     memcpy(out, r.v, sizeof r.v);
 }
 int fp28_zero(const int32_t* a, const int32_t* b) { return fp28::is_zero(fp28::mulb_below_p(load(a), load(b))) ? 1 : 0; }

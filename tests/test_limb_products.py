@@ -1,6 +1,6 @@
-"""The field products of the commitment kernels (host build of grape_amd/csrc/fp28.hpp) on operands whose limbs are at the
-bounds that the columns are laid out for: balanced limbs of +-(2^29 + 2), one lazy operand of twice that, all signs alike
-and mixed, against Python integers."""
+"""The field products of the commitment kernels (host build of grape_amd/csrc/fp28.hpp) and of the round kernels (fr26.hpp) on
+operands whose limbs are at the bounds that the columns are laid out for, all signs alike and mixed, against Python
+integers: balanced limbs of +-(2^29 + 2) and one lazy operand of twice that; limbs of 2^30 times 2^27."""
 import ctypes
 import os
 import random
@@ -10,9 +10,9 @@ import pytest
 import bigref as br
 
 HERE = os.path.dirname(os.path.abspath(__file__))
-SRC = os.path.join(HERE, "native", "fp28_limbs_host.cpp")
+SRC = os.path.join(HERE, "native", "limb_products_host.cpp")
 BN = br.CURVE == "bn254"
-LIB = os.path.join(HERE, "native", "libfp28_limbs_host_bn254.so" if BN else "libfp28_limbs_host.so")
+LIB = os.path.join(HERE, "native", "liblimb_products_host_bn254.so" if BN else "liblimb_products_host.so")
 P = br.P_MOD
 W = 30
 EDGE = (1 << 29) + 2
@@ -20,7 +20,7 @@ EDGE = (1 << 29) + 2
 
 @pytest.fixture(scope="module")
 def lib():
-    deps = [SRC] + [os.path.join(HERE, "..", "grape_amd", "csrc", f) for f in ("fp28.hpp", "divstep.hpp", "curve.hpp", "field.hpp")]
+    deps = [SRC] + [os.path.join(HERE, "..", "grape_amd", "csrc", f) for f in ("fp28.hpp", "fr26.hpp", "divstep.hpp", "curve.hpp", "field.hpp")]
     if not os.path.exists(LIB) or any(os.path.getmtime(d) > os.path.getmtime(LIB) for d in deps):
         subprocess.check_call(["g++", "-O2", "-std=c++17", "-fwrapv", "-fPIC", "-shared", "-Wno-unknown-pragmas"]
                               + (["-DGRAPE_CURVE_BN254"] if BN else []) + ["-o", LIB, SRC])
@@ -97,3 +97,26 @@ def test_carries_and_zero(lib):
             assert lib.fp28_zero(_ptr(a + unit), _ptr(f)) == int(_value(f) % P == 0)
             c = _apply(lib, 10, a + unit, f, zero, zero)
             assert _value(c) == _value(f) * rinv % P and all(0 <= int(x) < 1 << W for x in c[:-1])
+
+
+def test_scalar_product_in_wide_digits(lib):
+    n, r, w, rng = 10, br.R_MOD, 26, random.Random(7)
+    value = lambda limbs: sum(int(v) << (w * i) for i, v in enumerate(limbs))
+    top = (2 * r) >> (w * (n - 1))
+    # e * x with e below 16 r (limbs below 2^30) and x a difference of two elements or a sum of two (limbs below 2^27)
+    es = [np.zeros(n, dtype=np.int32), np.array([(1 << 30) - 16] * (n - 1) + [8 * top], dtype=np.int32)]
+    es += [np.array([rng.randrange(1 << 30) for _ in range(n - 1)] + [rng.randrange(8 * top)], dtype=np.int32) for _ in range(10)]
+    bound = (1 << 27) - 1
+    xs = [np.array([s * bound] * (n - 1) + [s * top], dtype=np.int32) for s in (1, -1)] + [np.zeros(n, dtype=np.int32)]
+    xs += [np.array([rng.randint(-bound, bound) for _ in range(n - 1)] + [rng.randint(-top, top)], dtype=np.int32) for _ in range(20)]
+    out = np.zeros(n, dtype=np.int32)
+    for e in es:
+        for x in xs:
+            for add_r in (0, 1, 4, 31):
+                lib.fr26_product(_ptr(e), _ptr(x), add_r, _ptr(out))
+                v, exact = value(out), value(e) * value(x)
+                assert (v * (1 << (w * n)) - exact) % r == 0
+                assert all(0 <= int(d) < 1 << w for d in out[:-1])
+                # between exact / 2^260 + add_r r and (1 + 2^-20) r above
+                low = v * (1 << (w * n)) - exact - add_r * r * (1 << (w * n))
+                assert 0 <= low < r * ((1 << (w * n)) + (1 << (w * n - 20)))
