@@ -88,6 +88,10 @@ SIGNATURES = {
     "grape_tlookup_hot_coverage": [c_void_p, c_u32, c_void_p, ctypes.POINTER(ctypes.c_uint64), c_void_p],
     "grape_fr_mask_cold": [c_void_p, c_void_p, c_void_p, c_size_t, c_void_p],
     "grape_fr_gather": [c_void_p, c_void_p, c_void_p, c_size_t, c_void_p],
+    "grape_tlookup_index_i32_nowait": [c_void_p, c_void_p, c_void_p, c_size_t, c_i32, c_u32, c_void_p, c_void_p, c_void_p],
+    "grape_wround_queue_gathered": [c_void_p, c_void_p, c_void_p],
+    "grape_commit_fr_sparse_indexed": [c_void_p, c_void_p, c_void_p, c_void_p, c_size_t, c_u32, c_void_p, c_size_t, c_u32, c_u32, c_u32, c_void_p],
+    "grape_commit_fr_strided_masked_indexed": [c_void_p, c_void_p, c_void_p, c_void_p, c_size_t, c_u32, c_void_p, c_size_t, c_u32, c_u32, c_u32, c_void_p],
     "grape_commit_fr_sparse": [c_void_p, c_void_p, c_void_p, c_size_t, c_u32, c_void_p, c_size_t, c_u32, c_u32, c_u32, c_void_p],
     "grape_g1_affine_add": [c_void_p, c_void_p, c_void_p, c_size_t, c_void_p],
     "grape_tlookup_init": [c_void_p, c_void_p, c_i32, c_u32, c_void_p, c_void_p, c_void_p, c_void_p],

@@ -743,9 +743,15 @@ __global__ void __launch_bounds__(kBlock) commit_strided_kernel(uint32_t* partia
 // recoding per element and an addition slot per WAVE that holds one live element - 80 ms for 2^27
 // elements of which 0.7 % are live, against 3 ms here.  With many rows G = 32: a row of 4096 with
 // 27 live elements fills 27 of 32 lanes of its batch instead of 27 of 64.
+// With idx1 the scalars are table entries: element i is scalars[idx1[i] - 1].
+__device__ __forceinline__ Fr ld_scalar(const uint32_t* scalars, const int32_t* __restrict__ idx1, size_t i) {
+    if (!idx1) return ld_fr8(scalars, i);
+    const uint32_t j = (uint32_t)idx1[i];
+    return ld_fr8(scalars, j ? j - 1 : 0);
+}
 template <int G>
-__global__ void __launch_bounds__(64) commit_sparse_fr_kernel(uint32_t* partial, const uint32_t* scalars, const int32_t* __restrict__ skip,
-                                                              uint32_t rowlen, size_t rows, size_t step, const uint32_t* table, size_t N,
+__global__ void __launch_bounds__(64) commit_sparse_fr_kernel(uint32_t* partial, const uint32_t* scalars, const int32_t* __restrict__ idx1,
+                                                              const int32_t* __restrict__ skip, uint32_t rowlen, size_t rows, size_t step, const uint32_t* table, size_t N,
                                                               uint32_t c, uint32_t nw, uint32_t K, int* err_flag) {
     constexpr int R = 64 / G;                            // rows per wave
     __shared__ uint32_t queue[R][2 * G];
@@ -772,7 +778,7 @@ __global__ void __launch_bounds__(64) commit_sparse_fr_kernel(uint32_t* partial,
             const uint32_t n = qn < (uint32_t)G ? qn : (uint32_t)G;
             if ((uint32_t)sub < n) {
                 const uint32_t col = queue[grp][sub];
-                const Fr k = from_mont(ld_fr8(scalars, geom::scalar_index(row, rowlen, col)));
+                const Fr k = from_mont(ld_scalar(scalars, idx1, geom::scalar_index(row, rowlen, col)));
                 madd_scalar_fr(acc, k, table, N, col, c, nw, K, err_flag);
             }
             __syncthreads();
@@ -791,8 +797,8 @@ __global__ void __launch_bounds__(64) commit_sparse_fr_kernel(uint32_t* partial,
 // batches of 64, so dead elements cost a look at their flag whether they lie scattered or in stretches, and a live one
 // the strided table's 16 to 18 additions instead of the per-window table's 20.  Worth it from some hundred live elements a
 // row (every residue leaves 64 partial sums).  One-wave workgroups, dealt by geom::spread_unit: the rows differ.
-__global__ void __launch_bounds__(64) commit_sparse_strided_kernel(uint32_t* partial, const uint32_t* scalars, const int32_t* __restrict__ skip,
-                                                                   uint32_t rowlen, size_t units, size_t step, const uint32_t* table, size_t N,
+__global__ void __launch_bounds__(64) commit_sparse_strided_kernel(uint32_t* partial, const uint32_t* scalars, const int32_t* __restrict__ idx1,
+                                                                   const int32_t* __restrict__ skip, uint32_t rowlen, size_t units, size_t step, const uint32_t* table, size_t N,
                                                                    uint32_t c, uint32_t nw, uint32_t K, uint32_t J, uint32_t nsets) {
     __shared__ uint32_t queue[2 * 64];
     const int lane = threadIdx.x;
@@ -815,7 +821,7 @@ __global__ void __launch_bounds__(64) commit_sparse_strided_kernel(uint32_t* par
             const uint32_t n = qn < 64 ? qn : 64;
             if ((uint32_t)lane < n) {
                 const uint32_t col = queue[lane];
-                madd_scalar_strided(acc, ld_fr8(scalars, geom::scalar_index(row, rowlen, col)), H, table, N, col, c, nw, K, J, j, 0, nsets);
+                madd_scalar_strided(acc, ld_scalar(scalars, idx1, geom::scalar_index(row, rowlen, col)), H, table, N, col, c, nw, K, J, j, 0, nsets);
             }
             __syncthreads();
             const uint32_t moved = (uint32_t)lane + 64 < qn ? queue[lane + 64] : 0u;
@@ -1318,7 +1324,7 @@ int grape_g1_strided_table_gen(uint32_t* table, const uint32_t* gens, size_t N, 
 
 // Full-width scalars through a strided table (see commit_strided_kernel): nw = ceil(255 / c) windows,
 // J residues, nsets = ceil(nw / J) table sets of K = 2^(c-1) multiples.
-static int commit_strided_impl(uint32_t* out, const uint32_t* scalars, const int32_t* skip, size_t size, uint32_t rowlen, const uint32_t* table,
+static int commit_strided_impl(uint32_t* out, const uint32_t* scalars, const int32_t* idx1, const int32_t* skip, size_t size, uint32_t rowlen, const uint32_t* table,
                                size_t N, uint32_t c, uint32_t J, uint32_t nsets, grape_stream_t st) {
     if (size == 0) return GRAPE_OK;
     GRAPE_REQUIRE(size <= kMaxCommitScalars, "more than 2^28 scalars in one call: commit the rows in several calls");
@@ -1349,10 +1355,10 @@ static int commit_strided_impl(uint32_t* out, const uint32_t* scalars, const int
     profile_begin();
     for (size_t r0 = 0; r0 < rows; r0 += slab) {
         const size_t nr = rows - r0 < slab ? rows - r0 : slab;
-        const uint32_t* sc = scalars + r0 * rowlen * 8;
+        const uint32_t* sc = idx1 ? scalars : scalars + r0 * rowlen * 8;
         profile_mark(s);
         if (skip)
-            commit_sparse_strided_kernel<<<(unsigned)(nr * J), 64, 0, s>>>((uint32_t*)ws, sc, skip + r0 * rowlen, rowlen, nr * J, geom::spread_step(nr * J),
+            commit_sparse_strided_kernel<<<(unsigned)(nr * J), 64, 0, s>>>((uint32_t*)ws, sc, idx1 ? idx1 + r0 * rowlen : nullptr, skip + r0 * rowlen, rowlen, nr * J, geom::spread_step(nr * J),
                                                                            table, N, c, nw, K, J, nsets);
         else
             commit_strided_kernel<<<blocks_for(nr * J * nparts), kBlock, 0, s>>>((uint32_t*)ws, sc, rowlen, nr, seg, nseg, table, N, c, nw, K, J, nsets, split);
@@ -1367,12 +1373,17 @@ static int commit_strided_impl(uint32_t* out, const uint32_t* scalars, const int
 
 int grape_commit_fr_strided(uint32_t* out, const uint32_t* scalars, size_t size, uint32_t rowlen, const uint32_t* table, size_t N,
                             uint32_t c, uint32_t J, uint32_t nsets, grape_stream_t st) {
-    return commit_strided_impl(out, scalars, nullptr, size, rowlen, table, N, c, J, nsets, st);
+    return commit_strided_impl(out, scalars, nullptr, nullptr, size, rowlen, table, N, c, J, nsets, st);
 }
 int grape_commit_fr_strided_masked(uint32_t* out, const uint32_t* scalars, const int32_t* skip, size_t size, uint32_t rowlen, const uint32_t* table,
                                    size_t N, uint32_t c, uint32_t J, uint32_t nsets, grape_stream_t st) {
     GRAPE_REQUIRE(size == 0 || skip != nullptr, "no flag array");
-    return commit_strided_impl(out, scalars, skip, size, rowlen, table, N, c, J, nsets, st);
+    return commit_strided_impl(out, scalars, nullptr, skip, size, rowlen, table, N, c, J, nsets, st);
+}
+int grape_commit_fr_strided_masked_indexed(uint32_t* out, const uint32_t* entries, const int32_t* idx1, const int32_t* skip, size_t size, uint32_t rowlen,
+                                           const uint32_t* table, size_t N, uint32_t c, uint32_t J, uint32_t nsets, grape_stream_t st) {
+    GRAPE_REQUIRE(size == 0 || (skip != nullptr && idx1 != nullptr), "no flag or index array");
+    return commit_strided_impl(out, entries, idx1, skip, size, rowlen, table, N, c, J, nsets, st);
 }
 
 int grape_g1_scaled_table_gen(uint32_t* out, const uint32_t* scalars, size_t len, size_t ncols, const uint32_t* table, size_t N,
@@ -1409,8 +1420,8 @@ int grape_g1_scaled_table_gen(uint32_t* out, const uint32_t* scalars, size_t len
     return GRAPE_OK;
 }
 
-int grape_commit_fr_sparse(uint32_t* out, const uint32_t* scalars, const int32_t* skip, size_t size, uint32_t rowlen,
-                           const uint32_t* table, size_t N, uint32_t c, uint32_t nw, uint32_t K, grape_stream_t st) {
+static int commit_sparse_impl(uint32_t* out, const uint32_t* scalars, const int32_t* idx1, const int32_t* skip, size_t size, uint32_t rowlen,
+                              const uint32_t* table, size_t N, uint32_t c, uint32_t nw, uint32_t K, grape_stream_t st) {
     if (size == 0) return GRAPE_OK;
     GRAPE_REQUIRE(size <= kMaxCommitScalars, "more than 2^28 scalars in one call: commit the rows in several calls");
     CHECK_PTR16(out); CHECK_PTR16(scalars); CHECK_PTR16(table);
@@ -1434,11 +1445,13 @@ int grape_commit_fr_sparse(uint32_t* out, const uint32_t* scalars, const int32_t
         const size_t nr = rows - r0 < slab ? rows - r0 : slab;
         // many rows: half a wave per row, so that a thinly populated row still fills its batch
         const bool narrow = nr >= 4096;
+        const uint32_t* sc = idx1 ? scalars : scalars + r0 * rowlen * 8;
+        const int32_t* ix = idx1 ? idx1 + r0 * rowlen : nullptr;
         if (narrow)
-            commit_sparse_fr_kernel<32><<<(unsigned)((nr + 1) / 2), 64, 0, s>>>((uint32_t*)ws, scalars + r0 * rowlen * 8, skip + r0 * rowlen, rowlen, nr,
+            commit_sparse_fr_kernel<32><<<(unsigned)((nr + 1) / 2), 64, 0, s>>>((uint32_t*)ws, sc, ix, skip + r0 * rowlen, rowlen, nr,
                                                                               geom::spread_step((nr + 1) / 2), table, N, c, nw, K, err);
         else
-            commit_sparse_fr_kernel<64><<<(unsigned)nr, 64, 0, s>>>((uint32_t*)ws, scalars + r0 * rowlen * 8, skip + r0 * rowlen, rowlen, nr,
+            commit_sparse_fr_kernel<64><<<(unsigned)nr, 64, 0, s>>>((uint32_t*)ws, sc, ix, skip + r0 * rowlen, rowlen, nr,
                                                                    geom::spread_step(nr), table, N, c, nw, K, err);
         launch_reduce<true>(out + r0 * (size_t)(2 * FW), (const uint32_t*)ws, nr, narrow ? 32 : 64, red_tmp, s);
     }
@@ -1451,6 +1464,16 @@ int grape_commit_fr_sparse(uint32_t* out, const uint32_t* scalars, const int32_t
         return GRAPE_EINVAL;
     }
     return GRAPE_OK;
+}
+
+int grape_commit_fr_sparse(uint32_t* out, const uint32_t* scalars, const int32_t* skip, size_t size, uint32_t rowlen,
+                           const uint32_t* table, size_t N, uint32_t c, uint32_t nw, uint32_t K, grape_stream_t st) {
+    return commit_sparse_impl(out, scalars, nullptr, skip, size, rowlen, table, N, c, nw, K, st);
+}
+int grape_commit_fr_sparse_indexed(uint32_t* out, const uint32_t* entries, const int32_t* idx1, const int32_t* skip, size_t size, uint32_t rowlen,
+                                   const uint32_t* table, size_t N, uint32_t c, uint32_t nw, uint32_t K, grape_stream_t st) {
+    GRAPE_REQUIRE(size == 0 || idx1 != nullptr, "no index array");
+    return commit_sparse_impl(out, entries, idx1, skip, size, rowlen, table, N, c, nw, K, st);
 }
 
 int grape_commit_i32(uint32_t* out, const int32_t* scalars, size_t size, uint32_t rowlen, const uint32_t* table, size_t N,

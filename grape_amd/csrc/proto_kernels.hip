@@ -555,6 +555,53 @@ __global__ void __launch_bounds__(kBlock) index_embed_i32_kernel(int32_t* idx1, 
     if (nbad != 0 && (threadIdx.x & 63) == 0) atomicAdd(mismatches, nbad);
 }
 
+// Indices and check alone, for a prover whose first round gathers A and S by index: 12 bytes an element (8 without second
+// components).  Bound: HBM.  Four elements a thread, as 16-byte accesses where the tensors allow them (VEC).
+template <bool VEC>
+__global__ void __launch_bounds__(kBlock) index_i32_kernel(int32_t* __restrict__ idx1, const int32_t* __restrict__ key, const int32_t* __restrict__ cmp,
+                                                           size_t n, int32_t low, uint32_t len, const int32_t* __restrict__ cmp_table,
+                                                           unsigned int* mismatches) {
+    const size_t i = 4 * ((size_t)blockIdx.x * kBlock + threadIdx.x);
+    unsigned int nbad = 0;
+    if (i < n) {
+        const int cnt = n - i < 4 ? (int)(n - i) : 4;
+        int32_t k[4], c[4], out[4];
+        if (VEC && cnt == 4) {
+            const int4 kv = *reinterpret_cast<const int4*>(key + i);
+            k[0] = kv.x; k[1] = kv.y; k[2] = kv.z; k[3] = kv.w;
+            if (cmp) {
+                const int4 cv = *reinterpret_cast<const int4*>(cmp + i);
+                c[0] = cv.x; c[1] = cv.y; c[2] = cv.z; c[3] = cv.w;
+            }
+        } else {
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                k[q] = q < cnt ? key[i + q] : low;
+                if (cmp) c[q] = q < cnt ? cmp[i + q] : 0;
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int64_t d = (int64_t)k[q] - (int64_t)low;
+            const bool inside = d >= 0 && d < (int64_t)len;
+            out[q] = inside ? (int32_t)(d + 1) : 0;
+            if (q < cnt && (!inside || (cmp && c[q] != cmp_table[d]))) nbad++;
+        }
+        if (VEC && cnt == 4) {
+            *reinterpret_cast<int4*>(idx1 + i) = make_int4(out[0], out[1], out[2], out[3]);
+        } else {
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                if (q < cnt) idx1[i + q] = out[q];
+        }
+    }
+    if (__any(nbad != 0)) {
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1) nbad += __shfl_down(nbad, off, 64);
+        if ((threadIdx.x & 63) == 0) atomicAdd(mismatches, nbad);
+    }
+}
+
 // out[i] = (v_i - low) + 1 for an in-range value, 0 otherwise
 __global__ void __launch_bounds__(kBlock) index_kernel(int32_t* out, const uint32_t* vals, size_t n, int32_t low, uint32_t len) {
     size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x;
@@ -1051,6 +1098,23 @@ int grape_tlookup_index_embed_i32_nowait(int32_t* idx1, uint32_t* A, uint32_t* S
     if (r) CHECK_PTR16(r);
     index_embed_i32_kernel<<<blocks_for(n, kBlock * kEmbedPerThread), kBlock, 0, s>>>(idx1, A, S, key, cmp, n, low, len, B, cmp_table, r,
                                                                                      (unsigned int*)d_mismatches);
+    GRAPE_LAUNCH_CHECK();
+    return GRAPE_OK;
+}
+
+int grape_tlookup_index_i32_nowait(int32_t* idx1, const int32_t* key, const int32_t* cmp, size_t n, int32_t low, uint32_t len, const int32_t* cmp_table,
+                                   uint32_t* d_mismatches, grape_stream_t st) {
+    GRAPE_REQUIRE(d_mismatches != nullptr && idx1 != nullptr && len > 0, "bad arguments");
+    hipStream_t s = as_stream(st);
+    int rc = zero_fill(d_mismatches, sizeof(uint32_t), s);
+    if (rc) return rc;
+    if (n == 0) return GRAPE_OK;
+    GRAPE_REQUIRE(key != nullptr, "null witness");
+    GRAPE_REQUIRE((cmp == nullptr) == (cmp_table == nullptr), "cmp and cmp_table go together");
+    const bool vec = ((reinterpret_cast<uintptr_t>(idx1) | reinterpret_cast<uintptr_t>(key) | reinterpret_cast<uintptr_t>(cmp)) & 15) == 0;
+    const unsigned nb = blocks_for(n, kBlock * 4);
+    if (vec) index_i32_kernel<true><<<nb, kBlock, 0, s>>>(idx1, key, cmp, n, low, len, cmp_table, (unsigned int*)d_mismatches);
+    else index_i32_kernel<false><<<nb, kBlock, 0, s>>>(idx1, key, cmp, n, low, len, cmp_table, (unsigned int*)d_mismatches);
     GRAPE_LAUNCH_CHECK();
     return GRAPE_OK;
 }

@@ -103,18 +103,21 @@ __device__ __forceinline__ fr26::Limbs weight_product(const fr26::Limbs& e16, co
 // round's polynomial took at its challenge), which fixes the middle coefficient: the value at t = 1
 // is not accumulated - one product and one double-width accumulator less per index.
 // IDX: A is not read but gathered, A[i] = Bt[idx1[i] - 1] (in_size == 2 n_out): the first round of a lookup whose
-// logUp tensor was never written out - the pass over the witness left the table indices only.
+// logUp tensor was never written out - the pass over the witness left the table indices only.  IDX = 2: nor is S, S[i] =
+// Tt[idx1[i] - 1]; a witness element is read as its 4-byte index.  The tables' occupied entries sit in the caches (a
+// softmax's in 64 KB), and what is saved is writing and reading both tensors: 2^27 elements, pass over the witness and first
+// round 3.5 + 2.8 ms before.
 // SPLIT: the weight of index h * period + l is Eh[h] * E[l].  A thread keeps one l, so E[l] is applied once, to its three sums,
 // and what it reads per index is Eh[h] - the same word for a whole wave.  No table of n_out weights is made or read: building
 // one and reading it back is 64 to 96 bytes an index pair beside the 192 of the operands (2^23 pairs and the levels below
 // 2^20: 0.16 ms of launches, element product of 2048 x 11008: 0.30 ms).
-template <bool BETA, bool PLAIN, bool UNIT, bool TAB, bool NOMID = false, bool IDX = false, bool SPLIT = false>
+template <bool BETA, bool PLAIN, bool UNIT, bool TAB, bool NOMID = false, int IDX = 0, bool SPLIT = false>
 __global__ void __launch_bounds__(kBlock, 2) wround2_kernel(uint32_t* Aw, uint32_t* Sw, const uint32_t* A, const uint32_t* S,
                                                          const uint32_t* beta, const uint32_t* E,
                                                          uint32_t in_size, uint32_t n_out, uint32_t rowlen, uint32_t rowpad,
                                                          const uint32_t* v, const int32_t* __restrict__ tab, uint32_t* partial,
                                                          const int32_t* __restrict__ idx1 = nullptr, const uint32_t* Bt = nullptr,
-                                                         const uint32_t* Eh = nullptr, uint32_t period = 1) {
+                                                         const uint32_t* Eh = nullptr, uint32_t period = 1, const uint32_t* Tt = nullptr) {
     constexpr int NV = PLAIN ? 5 : 3;
     constexpr bool TIGHT = PLAIN && !UNIT && !NOMID;
     __shared__ Fr lds[NV * (kBlock / 64)];
@@ -143,10 +146,13 @@ __global__ void __launch_bounds__(kBlock, 2) wround2_kernel(uint32_t* Aw, uint32
         const size_t ei = rowlen == rowpad ? g : g + (size_t)((uint32_t)g / rowlen) * (rowpad - rowlen);
         const fr26::Limbs e16 = fr26::pack16(SPLIT ? ld_fr(Eh, h) : ld_fr(E, ei));
         fr26::Limbs a0, a1;
+        size_t t0 = 0, t1 = 0;
         if (IDX) {
             const uint32_t j0 = (uint32_t)idx1[g], j1 = (uint32_t)idx1[g + n_out];     // 0 marks an element outside the table
-            a0 = ld_l26(Bt, j0 ? j0 - 1 : 0);
-            a1 = ld_l26(Bt, j1 ? j1 - 1 : 0);
+            t0 = j0 ? j0 - 1 : 0;
+            t1 = j1 ? j1 - 1 : 0;
+            a0 = ld_l26(Bt, t0);
+            a1 = ld_l26(Bt, t1);
         } else {
             a0 = ld_l26(A, g);
             a1 = ld_hi26(A, g, n_out, in_size);
@@ -160,8 +166,8 @@ __global__ void __launch_bounds__(kBlock, 2) wround2_kernel(uint32_t* Aw, uint32
             sa1 = fr26::add(sa1, a1);
         }
         st_fr(Aw, g, TAB ? foldt1(tab, a0, da) : fold1(w1, a0, da));
-        const fr26::Limbs s0r = ld_l26(S, g);
-        const fr26::Limbs s1r = ld_hi26(S, g, n_out, in_size);
+        const fr26::Limbs s0r = IDX == 2 ? ld_l26(Tt, t0) : ld_l26(S, g);
+        const fr26::Limbs s1r = IDX == 2 ? ld_l26(Tt, t1) : ld_hi26(S, g, n_out, in_size);
         const fr26::Limbs ds = fr26::sub(s1r, s0r);
         st_fr(Sw, g, TAB ? foldt1(tab, s0r, ds) : fold1(w1, s0r, ds));
         fr26::mac(W2, ead, ds);
@@ -486,10 +492,11 @@ size_t grape_wround_partial_bytes(const grape_wround_args* args) {
     if (!args || args->n_out < 1 || (args->eq_high && (args->period < 1 || args->period > GRAPE_WROUND_MAX_PERIOD))) return 0;
     return (size_t)wround_blocks(*args) * (args->plain_sums ? 5 : 3) * 32;
 }
-int grape_wround_queue(const grape_wround_args* args, grape_stream_t st) {
+// T: with idx1, S is gathered from it too
+static int wround_queue_impl(const grape_wround_args* args, const uint32_t* T, grape_stream_t st) {
     GRAPE_REQUIRE(args != nullptr, "null arguments");
     const grape_wround_args& a = *args;
-    const uint32_t *A = a.A, *S = a.S, *E = a.eq, *v = a.v, *beta = a.beta;
+    const uint32_t *A = T ? T : a.A, *S = T ? T : a.S, *E = a.eq, *v = a.v, *beta = a.beta;     // neither is read with T
     const uint32_t in_size = a.in_size, n_out = a.n_out, rowlen = a.rowlen, rowpad = a.rowpad;
     GRAPE_WROUND2_CHECKS();
     CHECK_PTR16(a.A_out); CHECK_PTR16(a.S_out); CHECK_PTR16(a.partial);
@@ -502,9 +509,12 @@ int grape_wround_queue(const grape_wround_args* args, grape_stream_t st) {
         GRAPE_REQUIRE(a.plain_sums == 2 && beta && in_size == 2 * (uint64_t)n_out && rowlen == rowpad, "an indexed round is a lookup's first round");
     }
     if (!a.eq_high) {
-        if (a.idx1)
-            wround2_kernel<true, true, true, true, false, true><<<nb, kBlock, 0, s>>>(a.A_out, a.S_out, A, S, beta, E, in_size, n_out, 1, 1, v, a.tab,
-                                                                                     a.partial, a.idx1, a.B);
+        if (a.idx1 && T)
+            wround2_kernel<true, true, true, true, false, 2><<<nb, kBlock, 0, s>>>(a.A_out, a.S_out, A, S, beta, E, in_size, n_out, 1, 1, v, a.tab,
+                                                                                  a.partial, a.idx1, a.B, nullptr, 1, T);
+        else if (a.idx1)
+            wround2_kernel<true, true, true, true, false, 1><<<nb, kBlock, 0, s>>>(a.A_out, a.S_out, A, S, beta, E, in_size, n_out, 1, 1, v, a.tab,
+                                                                                  a.partial, a.idx1, a.B);
         else if (int rc = wround2_main(a.A_out, a.S_out, A, S, beta, E, in_size, n_out, rowlen, rowpad, v, a.plain_sums, a.tab, a.partial, s)) return rc;
         GRAPE_LAUNCH_CHECK();
         return GRAPE_OK;
@@ -513,15 +523,22 @@ int grape_wround_queue(const grape_wround_args* args, grape_stream_t st) {
     GRAPE_REQUIRE(a.period >= 1 && a.period <= GRAPE_WROUND_MAX_PERIOD, "the period of split weights is 1..2^20");
 #define GRAPE_WSPLIT(BETA, P, U, M, I)                                                                                           \
     wround2_kernel<BETA, P, U, true, M, I, true><<<nb, kBlock, 0, s>>>(a.A_out, a.S_out, A, S, beta, E, in_size, n_out, 1, 1, v, a.tab, \
-                                                                    a.partial, a.idx1, a.B, a.eq_high, a.period)
-    if (a.plain_sums == 0 && !beta) GRAPE_WSPLIT(false, false, false, false, false);
-    else if (a.plain_sums == 3 && beta) GRAPE_WSPLIT(true, true, false, true, false);
-    else if (a.plain_sums == 2 && beta && a.idx1) GRAPE_WSPLIT(true, true, true, false, true);
-    else if (a.plain_sums == 2 && beta && in_size == 2 * (uint64_t)n_out) GRAPE_WSPLIT(true, true, true, false, false);
+                                                                    a.partial, a.idx1, a.B, a.eq_high, a.period, T)
+    if (a.plain_sums == 0 && !beta) GRAPE_WSPLIT(false, false, false, false, 0);
+    else if (a.plain_sums == 3 && beta) GRAPE_WSPLIT(true, true, false, true, 0);
+    else if (a.plain_sums == 2 && beta && a.idx1 && T) GRAPE_WSPLIT(true, true, true, false, 2);
+    else if (a.plain_sums == 2 && beta && a.idx1) GRAPE_WSPLIT(true, true, true, false, 1);
+    else if (a.plain_sums == 2 && beta && in_size == 2 * (uint64_t)n_out) GRAPE_WSPLIT(true, true, true, false, 0);
     else GRAPE_REQUIRE(false, "split weights are built for plain_sums 0 without beta and for 2 and 3 with it");
 #undef GRAPE_WSPLIT
     GRAPE_LAUNCH_CHECK();
     return GRAPE_OK;
+}
+int grape_wround_queue(const grape_wround_args* args, grape_stream_t st) { return wround_queue_impl(args, nullptr, st); }
+int grape_wround_queue_gathered(const grape_wround_args* args, const uint32_t* T, grape_stream_t st) {
+    CHECK_PTR16(T);
+    GRAPE_REQUIRE(args != nullptr && args->idx1 != nullptr, "a gathered round needs the table indices");
+    return wround_queue_impl(args, T, st);
 }
 int grape_wround_finish(uint32_t* sums, uint32_t stride, const grape_wround_args* rounds, uint32_t count, grape_stream_t st) {
     CHECK_PTR16(sums);

@@ -365,7 +365,7 @@ affine_t* Hyrax::commit_indexed_affine(int* idx_plus1, uint size, uint N, affine
     return out;
 }
 
-affine_t* Hyrax::commit_sparse_affine(FrTensor& tensor, int* skip, uint size, uint N, uint64_t live) {
+affine_t* Hyrax::commit_sparse_affine(FrTensor& tensor, int* skip, uint size, uint N, uint64_t live, const int* idx1) {
     check_shape(size, N);
     const uint rowlen = N * com_scale;
     const uint rows = size / rowlen;
@@ -390,6 +390,9 @@ affine_t* Hyrax::commit_sparse_affine(FrTensor& tensor, int* skip, uint size, ui
         affine_t* out = nullptr;
         check(grape_malloc((void**)&out, sizeof(affine_t) * (size_t)rows), "grape_malloc");
         check(for_row_chunks(size, rowlen, [&](size_t e0, size_t n, size_t r0) {
+                  if (idx1)
+                      return grape_commit_fr_strided_masked_indexed(W(out + r0), W(tensor.gpu_data), idx1 + e0, skip + e0, n, rowlen, W(t.d), t.ngen, t.c, t.J,
+                                                                    t.nsets, nullptr);
                   return grape_commit_fr_strided_masked(W(out + r0), W(tensor.gpu_data + e0), skip + e0, n, rowlen, W(t.d), t.ngen, t.c, t.J, t.nsets, nullptr);
               }),
               "grape_commit_fr_strided_masked");
@@ -400,6 +403,8 @@ affine_t* Hyrax::commit_sparse_affine(FrTensor& tensor, int* skip, uint size, ui
     affine_t* out = nullptr;
     check(grape_malloc((void**)&out, sizeof(affine_t) * (size_t)rows), "grape_malloc");
     check(for_row_chunks(size, rowlen, [&](size_t e0, size_t n, size_t r0) {
+              if (idx1)
+                  return grape_commit_fr_sparse_indexed(W(out + r0), W(tensor.gpu_data), idx1 + e0, skip + e0, n, rowlen, W(t.d), t.ngen, t.c, t.nw, t.K, nullptr);
               return grape_commit_fr_sparse(W(out + r0), W(tensor.gpu_data + e0), skip + e0, n, rowlen, W(t.d), t.ngen, t.c, t.nw, t.K, nullptr);
           }),
           "grape_commit_fr_sparse");

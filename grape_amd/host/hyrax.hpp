@@ -85,8 +85,8 @@ public:
 
     // Row commitments of the elements whose flag skip[j] is zero (`live` of them), the others left out; through the
     // strided table where rows hold many of them, through the per-window table that scaled tables are built with
-    // otherwise.  nullptr when there is neither.
-    affine_t* commit_sparse_affine(FrTensor& tensor, int* skip, uint size, uint N, uint64_t live);
+    // otherwise.  nullptr when there is neither.  With idx1 element j of the committed tensor is tensor[idx1[j] - 1].
+    affine_t* commit_sparse_affine(FrTensor& tensor, int* skip, uint size, uint N, uint64_t live, const int* idx1 = nullptr);
 
     // Upper bound for the wide fixed-base tables this object may build (default 128 GiB of the 288 GB; GRAPE_TABLE_BUDGET_GIB overrides).  When a
     // table would not fit, commitments go through the reference-format table instead.

@@ -50,10 +50,10 @@ void tLookup::make_index_and_A(const FrTensor& key, int low_, FrTensor& A, const
     }
     grape_free_on_default(d_count);
     a_ready_ = write_A && mismatches == 0;
-    a_deferred_ = !write_A && mismatches == 0;
+    a_deferred_ = s_by_index_ = !write_A && mismatches == 0;
 }
-void tLookup::make_index_and_A_from_ints(const int* key, const int* cmp, uint n, int low_, FrTensor& S, FrTensor& A, const int* cmp_table,
-                                         const Fr* r, bool write_A) {
+void tLookup::make_index_from_ints(const int* key, const int* cmp, uint n, int low_, FrTensor& S, FrTensor& A, const int* cmp_table, const Fr* r,
+                                   bool gather) {
     drop_index();
     a_ready_ = false;
     a_deferred_ = false;
@@ -61,21 +61,26 @@ void tLookup::make_index_and_A_from_ints(const int* key, const int* cmp, uint n,
     uint32_t* d_count = nullptr;
     check(grape_malloc_on_default((void**)&d_count, sizeof(uint32_t)), "grape_malloc");
     uint32_t mismatches = 1;
-    try {
+    auto embed = [&](bool write_A) {
         check(grape_tlookup_index_embed_i32_nowait(d_idx_, write_A ? W(A.gpu_data) : nullptr, W(S.gpu_data), key, cmp, n, low_, T.size,
                                                    W(B.gpu_data), cmp_table, r ? W(grape_host::device_scalar(*r)) : nullptr, d_count, nullptr),
               "grape_tlookup_index_embed_i32_nowait");
+    };
+    try {
+        if (gather) check(grape_tlookup_index_i32_nowait(d_idx_, key, cmp, n, low_, T.size, cmp_table, d_count, nullptr), "grape_tlookup_index_i32_nowait");
+        else embed(true);
         S.set_size(n);
         start_weights(1u << Log2(n));
         check(grape_memcpy_d2h(&mismatches, d_count, sizeof(uint32_t), nullptr), "grape_memcpy_d2h");
+        if (gather && mismatches != 0) embed(false);     // an element off the table: the tensors have to be there
     } catch (...) {
         grape_stream_sync(nullptr);
         grape_free_on_default(d_count);
         throw;
     }
     grape_free_on_default(d_count);
-    a_ready_ = write_A && mismatches == 0;
-    a_deferred_ = !write_A && mismatches == 0;
+    a_ready_ = !gather && mismatches == 0;
+    a_deferred_ = s_by_index_ = gather && mismatches == 0;
 }
 void tLookup::pad_index(uint N, uint pad_N, uint pad_size, int fill) {
     if (!d_idx_ || N == pad_N) return;
@@ -112,7 +117,12 @@ void tLookup::index_to_m(uint witness_size, int low_, void* stream) {
     d_hist_ = hist;                           // kept for the proof in flight: the commitment of A picks its table entries by count
 }
 
-// com(A) through the entries that occur often.  A[i] = B[index_i]; an entry t that occurs n_t times
+// out[i] = table[index_i]; every element sits on the table
+void tLookup::gather_by_index(FrTensor& out, const FrTensor& table, uint D) {
+    check(grape_fr_gather(W(out.gpu_data), W(table.gpu_data) - 8, reinterpret_cast<const uint32_t*>(d_idx_), D, nullptr), "grape_fr_gather");   // d_idx_ holds index + 1
+}
+
+// com(A) through the entries that occur often (A: nullptr when it has not been written out).  A[i] = B[index_i]; an entry t that occurs n_t times
 // costs n_t full-width scalars (16 to 20 additions each) on the plain path, or one row B[t]*G_i of
 // the scaled table (rowlen entries at 20 additions and a normalisation each, built for this proof
 // only) plus n_t single additions.  So an entry is worth a row when n_t exceeds rowlen by a factor
@@ -129,7 +139,7 @@ void tLookup::drop_hot_rows() {
     hot_for_ = nullptr;
 }
 
-bool tLookup::commit_A_by_occupancy(FrTensor& A, uint D, uint msm_size, Hyrax& hyrax) {
+bool tLookup::commit_A_by_occupancy(FrTensor* A, uint D, uint msm_size, Hyrax& hyrax) {
     const uint N = T.size;
     const uint rowlen = msm_size * hyrax.com_scale;
     const uint rows = D / rowlen;
@@ -188,10 +198,11 @@ bool tLookup::commit_A_by_occupancy(FrTensor& A, uint D, uint msm_size, Hyrax& h
         com_A = hyrax.commit_indexed_affine(d_hot, D, msm_size, hot_table_, rowlen, hot_rows_);
         if (cold != 0) {
             // the elements without a table row: queued per row and committed as full-width scalars
-            com_cold = hyrax.commit_sparse_affine(A, d_hot, D, msm_size, cold);
+            com_cold = A ? hyrax.commit_sparse_affine(*A, d_hot, D, msm_size, cold) : hyrax.commit_sparse_affine(B, d_hot, D, msm_size, cold, d_idx_);
             if (!com_cold) {
                 FrTensor Acold(D, OnDefaultStream());
-                check(grape_fr_mask_cold(W(Acold.gpu_data), W(A.gpu_data), d_hot, D, nullptr), "grape_fr_mask_cold");
+                if (!A) gather_by_index(Acold, B, D);
+                check(grape_fr_mask_cold(W(Acold.gpu_data), W(A ? A->gpu_data : Acold.gpu_data), d_hot, D, nullptr), "grape_fr_mask_cold");
                 com_cold = hyrax.commit_affine(Acold, D, msm_size);
             }
             check(grape_g1_affine_add((uint32_t*)com_A, (const uint32_t*)com_A, (const uint32_t*)com_cold, rows, nullptr),
@@ -408,9 +419,12 @@ Fr tLookup::run(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax& hyrax
     // left A unwritten, the first round gathers it from B - if that round is one of the long ones queued
     // beside the commitments; otherwise A is written out now.
     bool from_table = a_ready_;
-    const bool gather_first = a_deferred_ && overlap && D == (1u << Log2(D)) && D / 2 >= kLongRoundPairs && A.size >= D;
+    const bool gather_first = a_deferred_ && D == (1u << Log2(D)) && D / 2 >= kLongRoundPairs && A.size >= D;
+    // the witness itself too: what prove() did not write out is written now where the first round cannot gather
+    const bool gather_S = gather_first && s_by_index_;
     a_ready_ = false;
     a_deferred_ = false;
+    s_by_index_ = false;
     if (gather_first) from_table = true;
     if (!from_table && d_idx_) {
         size_t mismatches = 0;
@@ -441,9 +455,11 @@ Fr tLookup::run(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax& hyrax
             com_A = hyrax.commit_indexed_affine(d_idx, D, msm_size, scaled_table_, scaled_cols_, N);
             check(grape_stream_sync(nullptr), "sync");
             if (d_idx != d_idx_) grape_free(d_idx);
-        } else if (indexed_commit_ && from_table && d_idx_ && d_hist_ && D / rowlen > 1 && commit_A_by_occupancy(A, D, msm_size, hyrax)) {
+        } else if (indexed_commit_ && from_table && d_idx_ && d_hist_ && D / rowlen > 1 &&
+                   commit_A_by_occupancy(gather_first ? nullptr : &A, D, msm_size, hyrax)) {
             // committed through a table of the entries that occur often
         } else {
+            if (gather_first) gather_by_index(A, B, D);
             com_A = hyrax.commit_affine(A, D, msm_size);
         }
         com_A_rows = D / (msm_size * hyrax.com_scale);
@@ -562,7 +578,8 @@ Fr tLookup::run(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax& hyrax
             a.tab = d_tabs + (size_t)GRAPE_FOLD_TABLE_WORDS * (size_t)vi;
             a.partial = reinterpret_cast<uint32_t*>(long_work + long_used);
             long_used += grape_wround_partial_bytes(&a);
-            check(grape_wround_queue(&a, st), "grape_wround_queue");
+            if (k == 0 && gather_S) check(grape_wround_queue_gathered(&a, W(T.gpu_data), st), "grape_wround_queue_gathered");
+            else check(grape_wround_queue(&a, st), "grape_wround_queue");
             if (overlap) {
                 witness.after(st);
                 check(grape_wround_finish(W(slot), 13, &a, 1, witness.stream), "grape_wround_finish");
@@ -828,7 +845,7 @@ Fr tLookupRange::prove(const int* device_int_S, FrTensor& S, FrTensor& A, const 
     }
     a_ready_ = false;
     const bool gather = indexed_commit_ && index_known_ && D / 2 >= (1u << 16);
-    make_index_and_A_from_ints(device_int_S, nullptr, D, low, S, A, nullptr, nullptr, !gather);
+    make_index_from_ints(device_int_S, nullptr, D, low, S, A, nullptr, nullptr, gather);
     m_pending_ = true;
     m_pending_size_ = D;
     m_pending_low_ = low;
@@ -942,10 +959,10 @@ Fr tLookupRangeMapping::prove(const int* device_int_S_in, const int* device_int_
         return prove(S_in, S_out, A, v, hyrax, msm_size, commit_time);
     }
     a_ready_ = false;
-    // index, the check S_out = f(S_in) against the integer table, A = B[index] and the combined witness S_in + r * S_out in one
-    // pass over the integers
+    // index and the check S_out = f(S_in) against the integer table in one pass over the integers; A = B[index] and the combined witness
+    // S_in + r * S_out = T[index] are gathered by a long first round, written by the same pass for a short one
     FrTensor S(D, OnDefaultStream());
-    make_index_and_A_from_ints(device_int_S_in, device_int_S_out, D, low, S, A, d_map_int_, &r, true);
+    make_index_from_ints(device_int_S_in, device_int_S_out, D, low, S, A, d_map_int_, &r, D / 2 >= (1u << 16));
     index_to_m(D, low);
     Fr ret;
     try {

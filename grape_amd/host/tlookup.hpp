@@ -67,12 +67,14 @@ protected:
     // write_A = false: the indices and the check only (a_deferred_ when every element matched); the first round then
     // gathers A from B, or run() writes it out where that round cannot.
     void make_index_and_A(const FrTensor& key, int low_, FrTensor& A, const FrTensor* cmp, const FrTensor* cmp_table, bool write_A = true);
-    // the same pass over a witness that is still a tensor of integers: also leaves the witness as field elements in S
-    // (key, or key + r * cmp with the integer table cmp_table of a mapping lookup)
-    void make_index_and_A_from_ints(const int* key, const int* cmp, uint n, int low_, FrTensor& S, FrTensor& A, const int* cmp_table,
-                                    const Fr* r, bool write_A);
+    // the same for a witness that is still a tensor of integers, which also leaves the witness as field elements in S
+    // (key, or key + r * cmp with the integer table cmp_table of a mapping lookup); gather = true: the indices and the check only,
+    // S and A are written where an element misses the table
+    void make_index_from_ints(const int* key, const int* cmp, uint n, int low_, FrTensor& S, FrTensor& A, const int* cmp_table, const Fr* r, bool gather);
     bool a_ready_ = false;              // A of the proof in flight already holds B[index]
     bool a_deferred_ = false;           // every element sits in the table, A not written yet
+    bool s_by_index_ = false;           // and the witness is T[index], whether S is written or not
+    void gather_by_index(FrTensor& out, const FrTensor& table, uint D);
     void drop_index();
     void pad_index(uint N, uint pad_N, uint pad_size, int fill);   // rows of N indices -> rows of pad_N
     void index_to_m(uint witness_size, int low_, void* stream = nullptr);
@@ -87,7 +89,7 @@ protected:
     uint hot_entries_ = 0;
     uint64_t cold_elements_ = 0;
     bool hot_reused_ = false;
-    bool commit_A_by_occupancy(FrTensor& A, uint D, uint msm_size, Hyrax& hyrax);
+    bool commit_A_by_occupancy(FrTensor* A, uint D, uint msm_size, Hyrax& hyrax);
     // Rows B[t]*G_i of the entries that were occupied in an earlier witness, with their slot
     // assignment: B is fixed for the object's life (the reference keeps one lookup object for all
     // layers of a model, test/llm.cu:57-64), so the rows serve later proofs as long as they cover

@@ -278,6 +278,10 @@ typedef struct {
 } grape_wround_args;
 size_t grape_wround_partial_bytes(const grape_wround_args *args);
 int grape_wround_queue(const grape_wround_args *args, grape_stream_t stream);
+/* The first round of a lookup from its indices alone: as grape_wround_queue with idx1 and plain_sums == 2, and S is gathered
+ * too, S[i] = d_T[idx1[i] - 1] (A and S of args are not read).  For a witness of which every element sits on its table entry
+ * (grape_tlookup_index_i32_nowait counted no other): neither tensor is ever written out (src/tlookup.cu:52-62, :117-151). */
+int grape_wround_queue_gathered(const grape_wround_args *args, const uint32_t *d_T, grape_stream_t stream);
 int grape_wround_finish(uint32_t *d_sums, uint32_t stride, const grape_wround_args *rounds, uint32_t count, grape_stream_t stream);
 /*
  * One round of matmul_sumcheck_phase1 (src/prove.cu:49-85): grape_sumcheck_round2 on indices
@@ -333,6 +337,10 @@ int grape_tlookup_index_inverse_nowait(int32_t *d_idx1, uint32_t *d_A, const uin
 int grape_tlookup_index_embed_i32_nowait(int32_t *d_idx1, uint32_t *d_A, uint32_t *d_S, const int32_t *d_key, const int32_t *d_cmp,
                                          size_t n, int32_t low, uint32_t len, const uint32_t *d_B, const int32_t *d_cmp_table,
                                          const uint32_t *d_r, uint32_t *d_mismatches, grape_stream_t stream);
+/* Indices, check and count of that pass without the witness as field elements, for a caller whose first round gathers both
+ * tensors by index (grape_wround_queue_gathered). */
+int grape_tlookup_index_i32_nowait(int32_t *d_idx1, const int32_t *d_key, const int32_t *d_cmp, size_t n, int32_t low, uint32_t len,
+                                   const int32_t *d_cmp_table, uint32_t *d_mismatches, grape_stream_t stream);
 /* The same histogram from indices already made by grape_tlookup_index (d_idx1[i] = index + 1,
  * 0 = outside the table): hist[d_idx1[i] - 1] += 1. */
 int grape_tlookup_hist_index(uint32_t *d_hist, const int32_t *d_idx1, size_t n, uint32_t len, grape_stream_t stream);
@@ -525,6 +533,11 @@ int grape_commit_fr_strided(uint32_t *d_out_affine, const uint32_t *d_scalars_mo
  * whose elements are left out). */
 int grape_commit_fr_strided_masked(uint32_t *d_out_affine, const uint32_t *d_scalars_mont, const int32_t *d_skip, size_t size, uint32_t rowlen,
                                    const uint32_t *d_table, size_t N, uint32_t c, uint32_t J, uint32_t nsets, grape_stream_t stream);
+/* The same for scalars that are entries of a table: element i is d_entries[d_idx1[i] - 1] (an index 0 reads entry 0); a logUp
+ * tensor A[i] = B[index_i] is committed without being written out. */
+int grape_commit_fr_strided_masked_indexed(uint32_t *d_out_affine, const uint32_t *d_entries, const int32_t *d_idx1, const int32_t *d_skip, size_t size,
+                                           uint32_t rowlen, const uint32_t *d_table, size_t N, uint32_t c, uint32_t J, uint32_t nsets,
+                                           grape_stream_t stream);
 /* Commitments through the reference-format table (k*G_i, k < 256, byte windows of |s| resp. of
  * the canonical scalar) — the reference's own algorithm, kept for tables loaded from its
  * points.bin.  Output affine. */
@@ -542,6 +555,10 @@ int grape_commit_fr_ref_table(uint32_t *d_out_affine, const uint32_t *d_scalars_
 int grape_commit_fr_sparse(uint32_t *d_out_affine, const uint32_t *d_scalars_mont, const int32_t *d_skip, size_t size,
                            uint32_t rowlen, const uint32_t *d_wide_table, size_t N, uint32_t c, uint32_t nw, uint32_t K,
                            grape_stream_t stream);
+/* The same for scalars that are entries of a table, as grape_commit_fr_strided_masked_indexed. */
+int grape_commit_fr_sparse_indexed(uint32_t *d_out_affine, const uint32_t *d_entries, const int32_t *d_idx1, const int32_t *d_skip, size_t size,
+                                   uint32_t rowlen, const uint32_t *d_wide_table, size_t N, uint32_t c, uint32_t nw, uint32_t K,
+                                   grape_stream_t stream);
 /* Window sums of sum_i k_i P_i over n arbitrary points (Jacobian, as grape_g1_affine_to_jacobian leaves them; Montgomery
  * scalars): d_sums receives GRAPE_MSM_WINDOWS XYZZ points S_w with sum_i k_i P_i = sum_w 16^w S_w.  The chain of doublings
  * that combines them is the caller's (the host: one core is faster at it than one lane).  1 <= n <= 2^24.  The fold of
