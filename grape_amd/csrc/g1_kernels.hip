@@ -749,6 +749,10 @@ __device__ __forceinline__ Fr ld_scalar(const uint32_t* scalars, const int32_t* 
     const uint32_t j = (uint32_t)idx1[i];
     return ld_fr8(scalars, j ? j - 1 : 0);
 }
+// The batch that ends a row deals shares of its columns' windows over the lanes: 27 live elements of a row and the larger of a
+// wave's two rows decides (33 columns are two batches, half of the waves' lanes idle in the second).  2^27 elements of which
+// 0.7 % are live, in rows of 4096: 3.77 -> 3.33 ms.
+constexpr uint32_t kSparseShares = 5;
 template <int G>
 __global__ void __launch_bounds__(64) commit_sparse_fr_kernel(uint32_t* partial, const uint32_t* scalars, const int32_t* __restrict__ idx1,
                                                               const int32_t* __restrict__ skip, uint32_t rowlen, size_t rows, size_t step, const uint32_t* table, size_t N,
@@ -776,10 +780,13 @@ __global__ void __launch_bounds__(64) commit_sparse_fr_kernel(uint32_t* partial,
         const bool go = last ? __any(qn > 0) : __any(qn >= (uint32_t)G);
         if (go) {
             const uint32_t n = qn < (uint32_t)G ? qn : (uint32_t)G;
-            if ((uint32_t)sub < n) {
-                const uint32_t col = queue[grp][sub];
+            // A full batch keeps every lane busy with a column of its own, the batch that ends a row does not: there a
+            // lane takes a share of a column's windows, n * shares of them dealt over G lanes.
+            const uint32_t units = last ? n * kSparseShares : n, per = last ? (nw + kSparseShares - 1) / kSparseShares : nw;
+            for (uint32_t u = sub; u < units; u += G) {
+                const uint32_t col = queue[grp][last ? u / kSparseShares : u], w0 = last ? (u % kSparseShares) * per : 0;
                 const Fr k = from_mont(ld_scalar(scalars, idx1, geom::scalar_index(row, rowlen, col)));
-                madd_scalar_fr(acc, k, table, N, col, c, nw, K, err_flag);
+                madd_scalar_fr(acc, k, table, N, col, c, nw, K, err_flag, w0, w0 + per);
             }
             __syncthreads();
             const uint32_t moved = (uint32_t)sub + G < qn ? queue[grp][sub + G] : 0u;
