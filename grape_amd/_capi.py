@@ -89,6 +89,11 @@ SIGNATURES = {
     "grape_fr_mask_cold": [c_void_p, c_void_p, c_void_p, c_size_t, c_void_p],
     "grape_fr_gather": [c_void_p, c_void_p, c_void_p, c_size_t, c_void_p],
     "grape_tlookup_index_i32_nowait": [c_void_p, c_void_p, c_void_p, c_size_t, c_i32, c_u32, c_void_p, c_void_p, c_void_p],
+    "grape_carried_halves": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_u32, c_void_p],
+    "grape_carried_partial_bytes": [c_void_p],
+    "grape_carried_queue": [c_void_p, c_void_p],
+    "grape_carried_finish": [c_void_p, c_u32, c_void_p, c_u32, c_void_p],
+    "grape_carried_end": [c_void_p, c_void_p, c_u32, c_void_p, c_u32, c_void_p, c_void_p],
     "grape_wround_queue_gathered": [c_void_p, c_void_p, c_void_p],
     "grape_commit_fr_sparse_indexed": [c_void_p, c_void_p, c_void_p, c_void_p, c_size_t, c_u32, c_void_p, c_size_t, c_u32, c_u32, c_u32, c_void_p],
     "grape_commit_fr_strided_masked_indexed": [c_void_p, c_void_p, c_void_p, c_void_p, c_size_t, c_u32, c_void_p, c_size_t, c_u32, c_u32, c_u32, c_void_p],
@@ -146,7 +151,7 @@ SIGNATURES = {
     "grape_event_elapsed_ms": [ctypes.POINTER(ctypes.c_float), c_void_p, c_void_p],
 }
 _RESTYPES = {"grape_last_error": ctypes.c_char_p, "grape_g1_wide_table_bytes": c_size_t, "grape_eq_pyramid_elems": c_size_t,
-             "grape_wround2_partial_bytes": c_size_t, "grape_wround_partial_bytes": c_size_t, "grape_fr_fold_i32_elems": c_size_t}
+             "grape_wround2_partial_bytes": c_size_t, "grape_wround_partial_bytes": c_size_t, "grape_carried_partial_bytes": c_size_t, "grape_fr_fold_i32_elems": c_size_t}
 
 _lib = None
 

@@ -1,4 +1,6 @@
 #include "tlookup.hpp"
+#include "carried.hpp"
+#include <algorithm>
 #include <cassert>
 #include <chrono>
 #include <cstdio>
@@ -287,26 +289,29 @@ std::pair<void*, void*> commit_events() {
 }  // namespace
 
 // The weights of a lookup's rounds in one tensor: tables of every prefix of the point as far as the table side and rounds of 2^20
-// weights read them, and behind them, for longer rounds, those over the variables from GRAPE_EQ_SPLIT_LOW on (a long round's weight is
-// a product of two tables' entries).
+// weights read them, and behind them those over the variables from GRAPE_EQ_SPLIT_LOW on (a long round's weight is a product of
+// two tables' entries, and the carried weights are the second one's).
 namespace {
 struct WeightPlan {
     uint whole = 0, high = 0;
+    bool split = false;
     WeightPlan(uint nu, uint N) {
         const uint all = nu ? nu - 1 : 0;
         whole = std::min(all, std::max(GRAPE_EQ_LONGEST_PREFIX, Log2(N)));
-        if (all > whole) high = all - GRAPE_EQ_SPLIT_LOW;
+        split = all >= GRAPE_EQ_SPLIT_LOW;
+        if (split) high = all - GRAPE_EQ_SPLIT_LOW;
     }
-    size_t elems() const { return grape_eq_pyramid_elems(whole) + (high ? grape_eq_pyramid_elems(high) : 0); }
+    size_t elems() const { return grape_eq_pyramid_elems(whole) + (split ? grape_eq_pyramid_elems(high) : 0); }
+    uint32_t* high_level(fr_t* E, uint level) const { return W(E + grape_eq_pyramid_elems(whole) + (((size_t)1 << level) - 1)); }
     void build(fr_t* E, const fr_t* d_u, grape_stream_t st) const {
         check(grape_eq_pyramid(W(E), W(const_cast<fr_t*>(d_u)), whole, st), "grape_eq_pyramid");
-        if (high)
+        if (split)
             check(grape_eq_pyramid(W(E + grape_eq_pyramid_elems(whole)), W(const_cast<fr_t*>(d_u) + GRAPE_EQ_SPLIT_LOW), high, st), "grape_eq_pyramid");
     }
     void weigh(grape_wround_args& a, fr_t* E, uint vars) const {
-        const bool split = vars > whole;
-        a.eq = W(E + (((size_t)1 << (split ? GRAPE_EQ_SPLIT_LOW : vars)) - 1));
-        a.eq_high = split ? W(E + grape_eq_pyramid_elems(whole) + (((size_t)1 << (vars - GRAPE_EQ_SPLIT_LOW)) - 1)) : nullptr;
+        const bool product = vars > whole;
+        a.eq = W(E + (((size_t)1 << (product ? GRAPE_EQ_SPLIT_LOW : vars)) - 1));
+        a.eq_high = product ? high_level(E, vars - GRAPE_EQ_SPLIT_LOW) : nullptr;
         a.period = 1u << GRAPE_EQ_SPLIT_LOW;
     }
 };
@@ -518,6 +523,8 @@ Fr tLookup::run(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax& hyrax
     fr_t* d_v = grape_host::upload(v, OnDefaultStream());
     Fr S_last;
     char* long_work = nullptr;             // partial sums of the long rounds and the challenges' tables
+    std::unique_ptr<CarriedFactors> factors;                      // of long rounds that carry their weights
+    std::unique_ptr<FrTensor> ratio_tabs, consts, halves;
     // phase 2 binds copies where its rounds work in place; T, B, m of this object stay intact
     const bool table_long = N / 2 >= kLongRoundPairs;
     FrTensor Bw(table_long ? N : 1, OnDefaultStream()), Tw(table_long ? N : 1, OnDefaultStream()), mw(table_long ? N : 1, OnDefaultStream());
@@ -630,13 +637,72 @@ Fr tLookup::run(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax& hyrax
         };
         // work memory of the long rounds (every round its own partial sums) and the tables of all challenges' multiples
         size_t need = 0;
+        std::vector<grape_carried_args> carried;
         for (uint c = D, i = 0; c / 2 >= kLongRoundPairs && i < rounds; c /= 2, i++) {
             grape_wround_args a{};
             plan.weigh(a, E.gpu_data, nu - 1 - i);
             a.n_out = c / 2;
             a.plain_sums = 1;
             need += grape_wround_partial_bytes(&a);
+            grape_carried_args b{};
+            b.A_out = W(A.gpu_data);
+            b.Z_out = W(S.gpu_data);
+            b.A = W(A.gpu_data);
+            b.Z = W(S.gpu_data);
+            b.eq = W(E.gpu_data + (((size_t)1 << GRAPE_EQ_SPLIT_LOW) - 1));
+            b.period = 1u << GRAPE_EQ_SPLIT_LOW;
+            b.n_out = c / 2;
+            b.plain_sums = 1;
+            carried.push_back(b);
         }
+        // A witness on its table that is gathered in the first round: the long rounds carry their weights in S, from the third long
+        // round on (2^19 elements: 0.68 ms either way; 2^17, one round: 0.49 against 0.47 ms, the factors' upload and tables are not
+        // paid for; 2^22: 1.50 against 1.62 ms).
+        if (gather_S && carried.size() >= 3) factors.reset(new CarriedFactors(u.data(), v.data(), nu, (uint)carried.size(), GRAPE_EQ_SPLIT_LOW));
+        const bool carry = factors && factors->ok;
+        static_assert(kLongRoundPairs == 1u << GRAPE_EQ_SPLIT_LOW, "the last long round's pairs are one period");
+        if (carry) {
+            carried[0].idx1 = d_idx_;
+            carried[0].len = N;
+            carried[0].eq_high = plan.high_level(E.gpu_data, nu - 1 - GRAPE_EQ_SPLIT_LOW);
+            need = 0;
+            for (const grape_carried_args& b : carried) need += grape_carried_partial_bytes(&b);
+            // the ratios' tables and the two multiples of every table entry
+            ratio_tabs.reset(new FrTensor((uint)((sizeof(int32_t) * GRAPE_FOLD_TABLE_WORDS * carried.size() + sizeof(fr_t) - 1) / sizeof(fr_t)), OnDefaultStream()));
+            consts.reset(new FrTensor((uint)carried.size() + 1, OnDefaultStream()));
+            halves.reset(new FrTensor(4 * N, OnDefaultStream()));
+            carried[0].halves = W(halves->gpu_data);
+        }
+        // the long rounds that carry, their sums finished on the witness stream beside the commitments
+        auto carried_rounds = [&] {
+            std::vector<Fr> c(factors->ratio);
+            c.push_back(factors->end[0]);
+            check(grape_memcpy_h2d(consts->gpu_data, c.data(), sizeof(fr_t) * c.size(), nullptr), "h2d");
+            int32_t* tabs = reinterpret_cast<int32_t*>(ratio_tabs->gpu_data);
+            check(grape_fold_tables(tabs, W(consts->gpu_data), (uint)carried.size(), nullptr), "grape_fold_tables");
+            check(grape_carried_halves(W(halves->gpu_data), W(B.gpu_data), W(T.gpu_data), W(d_beta), W(d_v + vi), N, nullptr), "grape_carried_halves");
+            for (size_t i = 0; i < carried.size(); i++, vi--, k++) {
+                grape_carried_args& b = carried[i];
+                b.tab_a = d_tabs + (size_t)GRAPE_FOLD_TABLE_WORDS * (size_t)vi;
+                b.tab_z = tabs + GRAPE_FOLD_TABLE_WORDS * i;
+                b.partial = reinterpret_cast<uint32_t*>(long_work + long_used);
+                long_used += grape_carried_partial_bytes(&b);
+                check(grape_carried_queue(&b, nullptr), "grape_carried_queue");
+                cur /= 2;
+            }
+            grape_stream_t fs = nullptr;
+            if (overlap) {
+                witness.after(nullptr);
+                fs = witness.stream;
+            }
+            check(grape_carried_finish(W(sums.gpu_data), 13, carried.data(), 1, fs), "grape_carried_finish");
+            if (carried.size() > 1)
+                check(grape_carried_finish(W(sums.gpu_data + 13), 13, carried.data() + 1, (uint)carried.size() - 1, fs), "grape_carried_finish");
+            check(grape_carried_end(W(S.gpu_data), W(S.gpu_data), cur, W(consts->gpu_data + carried.size()), 1u << GRAPE_EQ_SPLIT_LOW, W(d_beta), nullptr),
+                  "grape_carried_end");
+            A.set_size(cur);
+            S.set_size(cur);
+        };
         if (need) {
             check(grape_malloc_on_default((void**)&long_work, need + sizeof(int32_t) * GRAPE_FOLD_TABLE_WORDS * (size_t)rounds), "grape_malloc");
             d_tabs = reinterpret_cast<int32_t*>(long_work + need);
@@ -653,6 +719,7 @@ Fr tLookup::run(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax& hyrax
         // wave waits for memory, which made the pair slower than one after the other.  The short
         // rounds (launch-bound) do run beside the commitments, on a stream of their own.
         if (overlap) {
+            if (carry) carried_rounds();
             while (vi >= 0 && cur / 2 >= kLongRoundPairs) witness_round(nullptr);
             // The table side and the commitment of m (a few rows: a short accumulation and a latency chain of a
             // row reduction) go to the second stream now, so that they run beside the long rounds and the
@@ -685,6 +752,7 @@ Fr tLookup::run(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax& hyrax
             });
             check(grape_event_record(commit_events().second, nullptr), "grape_event_record");
         }
+        if (carry && !overlap) carried_rounds();
         while (vi >= 0 && cur / 2 >= kLongRoundPairs) witness_round(ws);
         // the first round may be of another kind than the rest
         for (size_t i = 0; i < unfinished.size();) {
@@ -727,6 +795,20 @@ Fr tLookup::run(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax& hyrax
         d_v = nullptr;
         grape_free_on_default(long_work);
         long_work = nullptr;
+
+        // the polynomials of rounds that carried their weights, from the last one up
+        for (uint i = carry ? (uint)carried.size() : 0; i-- > 0;) {
+            Fr *a = &h[13 * (size_t)i], *next = a + 13;
+            const Fr next0 = next[0], next1 = next[0] + next[1] + next[2];      // its coefficients, whichever kind it is
+            const Fr q0 = i ? a[0] * factors->at0[i] : Fr::one(), q1 = i ? a[1] * factors->at1[i] : Fr::one();
+            const std::array<Fr, 3> q = factors->polynomial(i, q0, q1, next0, next1);
+            std::copy(q.begin(), q.end(), a);
+            if (i == 0) {
+                a[3] = a[3] * factors->inv_1v[0];
+                a[4] = a[4] * factors->inv_v[0];
+            }
+            a[4] = a[4] - a[3];
+        }
 
         Fr alpha_run = alpha, alpha_sq_run = alpha_sq;
         int ui = (int)nu - 1;      // index of the variable bound in this round (u.back())

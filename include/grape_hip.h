@@ -262,7 +262,7 @@ int grape_wround2_queue_indexed(uint32_t *d_A, uint32_t *d_S, const int32_t *d_i
 /* Where provers split: rounds of at most 2^20 weights read them from a prefix table.  A split round multiplies a thread's three sums
  * once more - 3 products beside the 20 of the four indices it has at that size - and making the table of 2^20 takes 14 us. */
 #define GRAPE_EQ_LONGEST_PREFIX 20u
-#define GRAPE_EQ_SPLIT_LOW 17u
+#define GRAPE_EQ_SPLIT_LOW 16u
 typedef struct {
     uint32_t *A_out, *S_out;
     const uint32_t *A, *S;
@@ -283,6 +283,41 @@ int grape_wround_queue(const grape_wround_args *args, grape_stream_t stream);
  * (grape_tlookup_index_i32_nowait counted no other): neither tensor is ever written out (src/tlookup.cu:52-62, :117-151). */
 int grape_wround_queue_gathered(const grape_wround_args *args, const uint32_t *d_T, grape_stream_t stream);
 int grape_wround_finish(uint32_t *d_sums, uint32_t stride, const grape_wround_args *rounds, uint32_t count, grape_stream_t stream);
+/*
+ * Long weighted rounds that carry the high variables' weights in the second tensor: Z = e S instead of S, so that no
+ * later round weighs anything (the rounds of eleMul_sumcheck and tLookup, src/prove.cu:119-172, src/tlookup.cu:117-151).
+ * Index h * period + l has the weight eq_high[h] eq[l]; n_out is a whole number of periods.  Three kinds of round:
+ *   idx1      a lookup's first round, A (S + beta) = 1 everywhere: A_out = the folded A = B[index], Z_out = eq_high[h] times the
+ *             folded S + beta = (T + beta)[index], from `halves` (4 len elements, grape_carried_halves).  Sums: slots 3 and 4
+ *             receive (1 - v) sum A0 and v sum A1.
+ *   eq_high   an element product's first round, Z is S: slots 0 and 1 receive q(0) = sum e a0 s0 and q(1) = sum e a1 s1;
+ *             A_out and Z_out the folds by tab_a's challenge, Z_out weighted.
+ *   neither   a later round over A and Z: slots 0 and 1 receive sum eq[l] a0 Z0 and sum eq[l] a1 Z1, with plain_sums slots 3
+ *             and 4 sum A0 and sum A1; A_out is folded by tab_a, Z_out = Z0 + k Z1 by tab_z = the table of k.
+ * The factors between these sums and the round polynomial, and k, are the caller's (1 / f_0, 1 / f_1 and k = v f_0 / (f_1 (1 - v))
+ * up to the carried factor; see the prover).  A_out may be A, Z_out may be Z.  Tables as grape_fold_tables makes them.
+ */
+typedef struct {
+    uint32_t *A_out, *Z_out;
+    const uint32_t *A, *Z;
+    const int32_t *idx1;
+    const uint32_t *halves;
+    uint32_t len;
+    const uint32_t *eq, *eq_high;
+    uint32_t period, n_out;
+    const int32_t *tab_a, *tab_z;
+    int plain_sums;
+    uint32_t *partial;
+} grape_carried_args;
+int grape_carried_halves(uint32_t *d_halves, const uint32_t *d_B, const uint32_t *d_T, const uint32_t *d_beta, const uint32_t *d_v, uint32_t len,
+                         grape_stream_t stream);
+size_t grape_carried_partial_bytes(const grape_carried_args *args);
+int grape_carried_queue(const grape_carried_args *args, grape_stream_t stream);
+/* finishes `count` <= 32 rounds of one kind; round i's sums go to element i * stride of d_sums */
+int grape_carried_finish(uint32_t *d_sums, uint32_t stride, const grape_carried_args *rounds, uint32_t count, grape_stream_t stream);
+/* S back from what is left of Z: out[i] = Z[i] factor[i / period] - beta (beta may be NULL; out may be Z) */
+int grape_carried_end(uint32_t *d_out, const uint32_t *d_Z, uint32_t n, const uint32_t *d_factor, uint32_t period, const uint32_t *d_beta,
+                      grape_stream_t stream);
 /*
  * One round of matmul_sumcheck_phase1 (src/prove.cu:49-85): grape_sumcheck_round2 on indices
  * g = seg * seglen + k where every index of a segment carries the weight d_e[seg]
