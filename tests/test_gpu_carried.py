@@ -20,6 +20,17 @@ def ops():
     return ops
 
 
+# the host objects are found by their table's address: it stays taken until the process ends
+_TABLES = []
+
+
+@pytest.fixture(scope="module")
+def table(ops):
+    if not _TABLES:
+        _TABLES.append(ops.g1_table_gen(ops.g1_make_generators(rand_fr(256, 915)), 256))
+    return _TABLES[0]
+
+
 @pytest.fixture(scope="module")
 def host():
     from grape_amd import _host
@@ -56,7 +67,7 @@ def test_element_product(ops, host, rows, cols, special):
 
 
 @pytest.mark.parametrize("logD,special", [(17, None), (18, None), (20, None)] + [(19, s) for s in POINTS])
-def test_lookup(ops, host, logD, special):
+def test_lookup(ops, host, table, logD, special):
     import torch
     D, N, low = 1 << logD, 1 << 6, -17
     rng = np.random.default_rng(logD)
@@ -66,7 +77,6 @@ def test_lookup(ops, host, logD, special):
     alpha, r = rand_fr(1, 911), rand_fr(1, 912)
     u, v = _point(logD, 913, special)
     beta = br.fr_pack([N])[0]
-    table = ops.g1_table_gen(ops.g1_make_generators(rand_fr(256, 915)), 256)
     host.set_input_format("i32")
     dx, dy = torch.from_numpy(x).cuda(), torch.from_numpy(y).cuda()
     m = orc.tlookup_prep(orc.from_i32(x), low, N)
