@@ -853,7 +853,7 @@ __global__ void __launch_bounds__(64) commit_sparse_strided_kernel(uint32_t* par
 // SIMDs, one-wave workgroups do not: 139 against 175 us for 4096 rows of 64) and few additions in a chain.
 // The map is a kernel of its own so that every quad of a wave inverts: left to the sum kernel's first quads
 // it took 0.1 ms longer.  Measured, one box, before (one lane per accumulator, shuffle or LDS trees) and now:
-// 4096 rows of 64: 0.291 -> 0.148 ms; 512 of 64: 0.196 -> 0.079; one of 4096: 0.277 -> 0.124; 64 of 256: 0.237 -> 0.093;
+// 4096 rows of 64: 0.291 -> 0.148 ms (0.136 on 13 limbs); 512 of 64: 0.196 -> 0.079; one of 4096: 0.277 -> 0.124; 64 of 256: 0.237 -> 0.093;
 // 32768 of 64: 1.08 -> 0.54.
 __device__ __forceinline__ quad::Acc ld_quad_partial(const uint32_t* base, size_t i) {
     const uint32_t* p = base + geom::partial_word(i);
