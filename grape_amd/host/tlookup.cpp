@@ -30,8 +30,6 @@ void tLookup::make_index(const FrTensor& vals, int low_) {
 }
 void tLookup::make_index_and_A(const FrTensor& key, int low_, FrTensor& A, const FrTensor* cmp, const FrTensor* cmp_table, bool write_A) {
     drop_index();
-    a_ready_ = false;
-    a_deferred_ = false;
     check(grape_malloc_on_default((void**)&d_idx_, sizeof(int) * (size_t)(key.size ? key.size : 1)), "grape_malloc");
     // The pass over the witness is queued first and its count of unmatched elements read last: in between the
     // host queues the proof's weights (a dozen small launches on the second stream) while the chip is busy.
@@ -57,8 +55,6 @@ void tLookup::make_index_and_A(const FrTensor& key, int low_, FrTensor& A, const
 void tLookup::make_index_from_ints(const int* key, const int* cmp, uint n, int low_, FrTensor& S, FrTensor& A, const int* cmp_table, const Fr* r,
                                    bool gather) {
     drop_index();
-    a_ready_ = false;
-    a_deferred_ = false;
     check(grape_malloc_on_default((void**)&d_idx_, sizeof(int) * (size_t)(n ? n : 1)), "grape_malloc");
     uint32_t* d_count = nullptr;
     check(grape_malloc_on_default((void**)&d_count, sizeof(uint32_t)), "grape_malloc");
@@ -92,7 +88,9 @@ void tLookup::pad_index(uint N, uint pad_N, uint pad_size, int fill) {
     grape_free_on_default(d_idx_);
     d_idx_ = padded;
 }
+// what the object knows about the witness of the proof in flight: every proof starts from here, whatever became of the last one
 void tLookup::drop_index() {
+    a_ready_ = a_deferred_ = s_by_index_ = false;
     if (d_idx_ || d_hist_) {
         grape_free_on_default(d_idx_);
         grape_free(d_hist_);
@@ -427,9 +425,7 @@ Fr tLookup::run(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax& hyrax
     const bool gather_first = a_deferred_ && D == (1u << Log2(D)) && D / 2 >= kLongRoundPairs && A.size >= D;
     // the witness itself too: what prove() did not write out is written now where the first round cannot gather
     const bool gather_S = gather_first && s_by_index_;
-    a_ready_ = false;
-    a_deferred_ = false;
-    s_by_index_ = false;
+    a_ready_ = a_deferred_ = s_by_index_ = false;
     if (gather_first) from_table = true;
     if (!from_table && d_idx_) {
         size_t mismatches = 0;
@@ -860,7 +856,6 @@ Fr tLookup::run(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax& hyrax
 
 Fr tLookupRange::prove(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax& hyrax, uint msm_size, double& commit_time) {
     uint D = S.size;
-    a_ready_ = false;
     if (D == (1u << Log2(D)) && A.size >= D) {
         // no padding: index and A = B[index] in one pass (starts the weights too); A stays unwritten where the
         // first round can gather it from B (a witness of 2^17 elements and more, committed through its indices)
@@ -925,7 +920,6 @@ Fr tLookupRange::prove(const int* device_int_S, FrTensor& S, FrTensor& A, const 
         S.get_data(D, const_cast<int*>(device_int_S));
         return prove(S, A, v, hyrax, msm_size, commit_time);
     }
-    a_ready_ = false;
     const bool gather = indexed_commit_ && index_known_ && D / 2 >= (1u << 16);
     make_index_from_ints(device_int_S, nullptr, D, low, S, A, nullptr, nullptr, gather);
     m_pending_ = true;
@@ -983,7 +977,6 @@ void tLookupRangeMapping::prep(const FrTensor& vals) { histogram_to_m(m, vals, l
 Fr tLookupRangeMapping::prove(FrTensor& S_in, FrTensor& S_out, FrTensor& A, const std::vector<Fr>& v, Hyrax& hyrax,
                               uint msm_size, double& commit_time) {
     uint D = S_in.size;
-    a_ready_ = false;
     if (S_out.size != D) throw std::runtime_error("tLookupRangeMapping: S_in.size != S_out.size");
     // no padding: index, the check S_out = f(S_in) and A = B[index] in one pass (starts the weights too)
     if (D == (1u << Log2(D)) && A.size >= D) {
@@ -1040,7 +1033,6 @@ Fr tLookupRangeMapping::prove(const int* device_int_S_in, const int* device_int_
         FrTensor S_in(D, const_cast<int*>(device_int_S_in)), S_out(D, const_cast<int*>(device_int_S_out));
         return prove(S_in, S_out, A, v, hyrax, msm_size, commit_time);
     }
-    a_ready_ = false;
     // index and the check S_out = f(S_in) against the integer table in one pass over the integers; A = B[index] and the combined witness
     // S_in + r * S_out = T[index] are gathered by a long first round, written by the same pass for a short one
     FrTensor S(D, OnDefaultStream());

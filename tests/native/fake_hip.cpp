@@ -8,6 +8,7 @@
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <string>
 #include <vector>
 
 namespace {
@@ -20,6 +21,15 @@ std::recursive_mutex mu;
 std::map<const void*, Seen> streams;                     // of each stream: what its next item is ordered behind, itself included
 Seen host;                                               // what the host has waited for
 std::map<const char*, Alloc> memory;
+struct Kernel {
+    std::string name;                                     // mangled
+    unsigned long launched = 0;
+};
+// by the host's stub; made by the first registration, which comes before this library's own variables are
+std::map<const void*, Kernel>& kernels() {
+    static std::map<const void*, Kernel> k;
+    return k;
+}
 unsigned long launches = 0, copies = 0, waits = 0;
 thread_local int device = 0;
 char symbol[1 << 24];
@@ -63,6 +73,14 @@ unsigned long fake_bytes() {
     return n;
 }
 unsigned long fake_launches() { return launches; }
+// launches of the kernels whose name holds `part`
+unsigned long fake_launched(const char* part) {
+    Lock l(mu);
+    unsigned long n = 0;
+    for (auto& k : kernels())
+        if (k.second.name.find(part) != std::string::npos) n += k.second.launched;
+    return n;
+}
 unsigned long fake_copies() { return copies; }
 // waits of the host for a stream, an event or the device
 unsigned long fake_waits() { return waits; }
@@ -155,14 +173,15 @@ hipError_t __hipPopCallConfiguration(dim3* g, dim3* b, size_t* sh, hipStream_t* 
     *s = config.stream;
     return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void*, dim3, dim3, void**, size_t, hipStream_t s) {
+hipError_t hipLaunchKernel(const void* stub, dim3, dim3, void**, size_t, hipStream_t s) {
     Lock l(mu);
     push(s);
     launches++;
+    kernels()[stub].launched++;
     return hipSuccess;
 }
 void** __hipRegisterFatBinary(const void*) { static void* handle; return &handle; }
-void __hipRegisterFunction(void**, const void*, char*, const char*, unsigned, void*, void*, void*, void*, int*) {}
+void __hipRegisterFunction(void**, const void* stub, char*, const char* name, unsigned, void*, void*, void*, void*, int*) { kernels()[stub].name = name; }
 void __hipRegisterVar(void**, void*, char*, char*, int, size_t, int, int) {}
 void __hipUnregisterFatBinary(void**) {}
 }

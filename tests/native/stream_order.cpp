@@ -16,6 +16,7 @@ extern "C" {
 unsigned long fake_pending(const void* stream);
 unsigned long fake_unjoined();
 unsigned long fake_launches();
+unsigned long fake_launched(const char* part);
 unsigned long fake_copies();
 void fake_queue(const void* stream);
 unsigned long fake_waits();
@@ -55,6 +56,46 @@ static void refused_lookup() {
     }
     expect(error.find("Size too small") == 0, "the commitment of the multiplicities is refused");
     expect(fake_unjoined() == 0, "no stream is left with work that nothing waits for");
+}
+
+// A proof that is refused for its arguments leaves nothing behind: the next one on the object, of field tensors in rows of 11008, has
+// its witness compared with the table as on an object that has refused none.
+static void proof_after_a_refused_one() {
+    const uint rows = 16, D = rows * 11008, Dp = rows * 16384, cols = 64, len = 1024;
+    bn128 G = bn128::one();
+    Hyrax hyrax(1, cols, device_points(256 * cols), G, 1);
+    const std::vector<int> map(len, 7);
+    int* ints = reinterpret_cast<int*>(device_points(Dp / 8));
+    double seconds = 0;
+    auto proved = [&](const std::function<void()>& prove) {
+        try {
+            prove();
+        } catch (const std::exception& e) {
+            return std::string(e.what());
+        }
+        return std::string();
+    };
+    FrTensor A(Dp), S(Dp), S_out(D);
+    S_out.set_size(D);
+    tLookupRangeMapping mapping(-512, len, map.data());
+    tLookupRange range(-512, len);
+    auto compared = [&](bool is_mapping) {
+        const unsigned long before = fake_launched("inverse_by_table");
+        A.set_size(Dp);
+        S.set_size(D);
+        proved([&] {
+            if (is_mapping) mapping.prove(S, S_out, A, random_vec(18), hyrax, cols, seconds);
+            else range.prove(S, A, random_vec(18), hyrax, cols, seconds);
+        });
+        return fake_launched("inverse_by_table") - before;
+    };
+    expect(compared(true) == 1 && compared(false) == 1, "a padded witness of field elements is compared with the table");
+    A.set_size(Dp);
+    expect(proved([&] { mapping.prove(ints, ints, Dp, A, random_vec(17), hyrax, cols, seconds); }) == "u.size() != v.size()", "a mapping of integers is refused");
+    S.set_size(Dp);
+    expect(proved([&] { range.prove(ints, S, A, random_vec(17), hyrax, cols, seconds); }) == "u.size() != v.size()", "a range of integers is refused");
+    expect(compared(true) == 1, "so it is after a mapping that was refused");
+    expect(compared(false) == 1, "so it is after a range that was refused");
 }
 
 // Memory that a program gets is idle when it gets it, whatever was queued on it before: on the default stream, and - while the
@@ -264,6 +305,7 @@ static void short_copies() {
 int main(int argc, char** argv) {
     const std::map<std::string, std::function<void()>> scenarios = {
         {"refused_lookup", refused_lookup},
+        {"proof_after_a_refused_one", proof_after_a_refused_one},
         {"tensor_memory_is_idle", tensor_memory_is_idle},
         {"sparse_commitment_table", sparse_commitment_table},
         {"operands_at_any_address", operands_at_any_address},
