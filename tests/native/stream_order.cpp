@@ -98,6 +98,35 @@ static void proof_after_a_refused_one() {
     expect(compared(false) == 1, "so it is after a range that was refused");
 }
 
+// Mapping objects of the C calls are found by the mapped values: one other value is another object, also where the words it sits
+// in agree under xor with a rotated product; the same values are the same object.
+static void mapping_objects() {
+    const uint32_t len = 1024, D = 2048, cols = 64;
+    const uint32_t* ints = reinterpret_cast<uint32_t*>(device_points(64));
+    const uint32_t* table = reinterpret_cast<uint32_t*>(device_points(256 * cols));
+    uint32_t point[8 * 11] = {0}, alpha[8] = {1}, r[8] = {2}, transcript[32 * 16], rounds, claim[8];
+    auto made = [&](const std::vector<int32_t>& map) {
+        const unsigned long before = fake_launched("tl_table_kernel");          // the object's T
+        grape_host_tlookup_mapping_prove(ints, ints, D, -512, len, map.data(), alpha, r, point, point, 11, table, cols, 1, cols, transcript, &rounds, claim);
+        return fake_launched("tl_table_kernel") - before;
+    };
+    grape_host_set_input_format(1);
+    std::vector<int32_t> map(len);
+    for (uint32_t i = 0; i < len; i++) map[i] = (int32_t)(i * 2654435761u);
+    const unsigned long first = made(map);
+    expect(first > 0 && made(map) == 0, "the same values find their object");
+    std::vector<int32_t> other(map);
+    other[1] ^= INT32_MIN;
+    other[16] ^= 1 << 26;
+    expect(made(other) == first, "two changed words make another object");
+    expect(made(map) == 0 && made(other) == 0, "both are kept");
+    for (uint32_t i : {0u, 777u, len - 1}) {
+        std::vector<int32_t> one(map);
+        one[i] ^= 1;
+        expect(made(one) == first, "one changed value makes another object");
+    }
+}
+
 // Memory that a program gets is idle when it gets it, whatever was queued on it before: on the default stream, and - while the
 // library itself has no further stream - on one it has never seen.  So the program may use it on a stream of its own at once.
 static void tensor_memory_is_idle() {
@@ -306,6 +335,7 @@ int main(int argc, char** argv) {
     const std::map<std::string, std::function<void()>> scenarios = {
         {"refused_lookup", refused_lookup},
         {"proof_after_a_refused_one", proof_after_a_refused_one},
+        {"mapping_objects", mapping_objects},
         {"tensor_memory_is_idle", tensor_memory_is_idle},
         {"sparse_commitment_table", sparse_commitment_table},
         {"operands_at_any_address", operands_at_any_address},
