@@ -61,9 +61,15 @@ struct CarriedFactors {
             at1.push_back(c * inv_u(j));
             c = c * (one - v[j]) * inv_1u(j);
         }
-        end.assign((size_t)1 << (left - low), c);
-        for (size_t h = 0; h < end.size(); h++)
-            for (unsigned j = low; j < left; j++) end[h] = end[h] * ((h >> (j - low)) & 1 ? inv_u(j) : inv_1u(j));
+        end.assign(1, c);
+        for (unsigned j = low; j < left; j++) {
+            const size_t n = end.size();
+            end.resize(2 * n);
+            for (size_t h = 0; h < n; h++) {
+                end[n + h] = end[h] * inv_u(j);
+                end[h] = end[h] * inv_1u(j);
+            }
+        }
         ok = true;
     }
     // q of round k from its values at 0 and 1 and those of the next round's

@@ -22,6 +22,7 @@ static void read3(fr_t* d_sums, Fr out[3]) {
 
 namespace {
 constexpr uint kLongRoundPairs = 1u << 16;       // from here on a round folds through the table of its challenge's multiples
+constexpr uint kCarriedRow = 256;                // shortest row of an element product that carries its weights
 constexpr uint kSplitLow = GRAPE_EQ_SPLIT_LOW, kLongestPrefix = GRAPE_EQ_LONGEST_PREFIX;
 // device buffer released on scope exit
 struct DeviceBuf {
@@ -336,9 +337,11 @@ static Fr eleMul_rounds(fr_t* Aw, fr_t* Bw, const fr_t* A, const fr_t* B, fr_t* 
     // The leading long rounds that pair whole rows (whole powers of two) carry their weights in B from the first one on, from 2^20
     // pairs: 0.39 ms either way there, while 2^18 elements take 0.225 against 0.210 ms (an upload, two launches for tables, one
     // to end) and 1024 x 11008 take 0.82 against 0.96.
+    // What is left in B takes a factor per row, made here and uploaded: rows of kCarriedRow elements leave fewer than 512 (2^13 x 257:
+    // 0.41-0.43 against 0.45 ms, 2^16 x 257: 1.10 against 1.30), rows of 5 would leave 2^14.
     const uint period = padded ? second_size : 1u << kSplitLow;
     uint carrying = 0;
-    if (period <= GRAPE_WROUND_MAX_PERIOD && size / 2 >= 1u << 20)
+    if (period >= kCarriedRow && period <= GRAPE_WROUND_MAX_PERIOD && size / 2 >= 1u << 20)
         for (uint n = size; n % 2 == 0 && n / 2 >= kLongRoundPairs && (n / 2) % period == 0; n /= 2) carrying++;
     const CarriedFactors factors(hu - rounds, hv - rounds, rounds, carrying, low);
     std::vector<grape_carried_args> carried;

@@ -205,6 +205,21 @@ static void operands_at_any_address() {
     }
 }
 
+// An element product carries its weights where few rows are left in the end: each of them costs the host a factor.
+static void element_products_that_carry() {
+    uint32_t *a = reinterpret_cast<uint32_t*>(device_points(1u << 20)), claim[8] = {0}, transcript[32 * 32], rounds, at_a[8], at_b[8];
+    std::vector<uint32_t> point(8 * 32, 3);
+    auto carried = [&](uint rows, uint cols) {
+        const unsigned long before = fake_launched("carried_round_kernel");
+        const int vars = (int)Log2(rows) + (int)Log2(cols);
+        grape_host_prove_elemul(a, a, 1, rows, cols, point.data(), vars, point.data(), vars, claim, transcript, &rounds, at_a, at_b);
+        return fake_launched("carried_round_kernel") - before;
+    };
+    grape_host_set_input_format(0);
+    expect(carried(1u << 10, 3000) == 5 && carried(1u << 11, 1u << 10) == 5 && carried(1u << 13, 257) == 5, "from rows of 256 on");
+    expect(carried(1u << 19, 5) == 0 && carried(1u << 15, 65) == 0 && carried(1u << 14, 255) == 0, "not with shorter rows");
+}
+
 // An opening that verifies here: every commitment is the identity (device memory reads as zero), so its two equations are
 // commit_d == 0 and commit_ad == -(c * result) * G.
 static Hyrax_proof trivial_opening(const bn128& G, const Fr& c, uint cols) {
@@ -339,6 +354,7 @@ int main(int argc, char** argv) {
         {"tensor_memory_is_idle", tensor_memory_is_idle},
         {"sparse_commitment_table", sparse_commitment_table},
         {"operands_at_any_address", operands_at_any_address},
+        {"element_products_that_carry", element_products_that_carry},
         {"verify_with_more_variables", verify_with_more_variables},
         {"verify_with_another_generator", verify_with_another_generator},
         {"blocks_of_two_devices", blocks_of_two_devices},
