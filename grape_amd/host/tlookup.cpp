@@ -226,6 +226,7 @@ namespace {
 // A witness round over at least this many index pairs runs before the commitments of its proof, a
 // shorter one (launch-bound) beside them.
 constexpr uint kLongRoundPairs = 1u << 16;
+constexpr uint kCarriedTable = 1u << 24;           // longest table whose multiples carried rounds gather: 2 GiB
 // A stream beside the default one (two per process, created on first use) and the two events that order it against
 // the default stream: begin() makes it wait for what the default stream has queued, end() makes the
 // default stream wait for it.  If the scope is left by an exception the destructor waits for the
@@ -653,8 +654,10 @@ Fr tLookup::run(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax& hyrax
         }
         // A witness on its table that is gathered in the first round: the long rounds carry their weights in S, from the third long
         // round on (2^19 elements: 0.68 ms either way; 2^17, one round: 0.49 against 0.47 ms, the factors' upload and tables are not
-        // paid for; 2^22: 1.50 against 1.62 ms).
-        if (gather_S && carried.size() >= 3) factors.reset(new CarriedFactors(u.data(), v.data(), nu, (uint)carried.size(), GRAPE_EQ_SPLIT_LOW));
+        // paid for; 2^22: 1.50 against 1.62 ms).  A table as long as the witness is no worse for it, though two multiples of every entry are
+        // made and gathered past the caches (2^24 entries, 2^24 elements: 20.1 against 31.3 ms with what went before; 2^22 and 2^19:
+        // 5.2 against 8.0, 2.6 against 3.1); beyond kCarriedTable their 128 bytes an entry are memory that such a proof has not asked for.
+        if (gather_S && carried.size() >= 3 && N <= kCarriedTable) factors.reset(new CarriedFactors(u.data(), v.data(), nu, (uint)carried.size(), GRAPE_EQ_SPLIT_LOW));
         const bool carry = factors && factors->ok;
         static_assert(kLongRoundPairs == 1u << GRAPE_EQ_SPLIT_LOW, "the last long round's pairs are one period");
         if (carry) {

@@ -98,6 +98,29 @@ static void proof_after_a_refused_one() {
     expect(compared(false) == 1, "so it is after a range that was refused");
 }
 
+// Carried rounds gather two multiples of every table entry: made for tables of up to 2^24 entries, and no room is asked for beyond.
+static void carried_lookups() {
+    const uint cols = 64, gens = 1u << 15;                // the multiplicities are committed in rows of 2^(log_len / 2)
+    bn128 G = bn128::one();
+    Hyrax hyrax(1, gens, device_points(256 * (size_t)gens), G, 1);
+    double seconds = 0;
+    auto carried = [&](uint log_len, uint log_D) {
+        const uint D = 1u << log_D;
+        tLookupRange lookup(-(int)(1u << (log_len - 1)), 1u << log_len);
+        FrTensor S(D), A(D);
+        const std::unique_ptr<FrTensor> ints(new FrTensor(D / 8));
+        const unsigned long before = fake_launched("carried_gather_kernel");
+        try {
+            lookup.prove(reinterpret_cast<const int*>(ints->gpu_data), S, A, random_vec(log_D), hyrax, cols, seconds);
+        } catch (const std::exception&) {                    // nothing is computed here, so its claims do not hold
+        }
+        return fake_launched("carried_gather_kernel") - before;
+    };
+    expect(carried(8, 19) == 1 && carried(19, 19) == 1 && carried(24, 24) == 1, "tables of up to 2^24 entries");
+    expect(carried(25, 25) == 0 && carried(30, 30) == 0, "longer ones are left to the weighted rounds");
+    expect(carried(8, 18) == 0, "as are short proofs");
+}
+
 // Mapping objects of the C calls are found by the mapped values: one other value is another object, also where the words it sits
 // in agree under xor with a rotated product; the same values are the same object.
 static void mapping_objects() {
@@ -351,6 +374,7 @@ int main(int argc, char** argv) {
         {"refused_lookup", refused_lookup},
         {"proof_after_a_refused_one", proof_after_a_refused_one},
         {"mapping_objects", mapping_objects},
+        {"carried_lookups", carried_lookups},
         {"tensor_memory_is_idle", tensor_memory_is_idle},
         {"sparse_commitment_table", sparse_commitment_table},
         {"operands_at_any_address", operands_at_any_address},
