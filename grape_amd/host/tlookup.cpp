@@ -41,7 +41,7 @@ void tLookup::make_index_and_A(const FrTensor& key, int low_, FrTensor& A, const
                                                  cmp ? W(cmp->gpu_data) : nullptr, cmp_table ? W(cmp_table->gpu_data) : nullptr, d_count,
                                                  nullptr),
               "grape_tlookup_index_inverse_nowait");
-        start_weights(1u << Log2(key.size));
+        start_weights(1u << Log2(key.size), !write_A);
         check(grape_memcpy_d2h(&mismatches, d_count, sizeof(uint32_t), nullptr), "grape_memcpy_d2h");
     } catch (...) {
         grape_stream_sync(nullptr);
@@ -68,7 +68,7 @@ void tLookup::make_index_from_ints(const int* key, const int* cmp, uint n, int l
         if (gather) check(grape_tlookup_index_i32_nowait(d_idx_, key, cmp, n, low_, T.size, cmp_table, d_count, nullptr), "grape_tlookup_index_i32_nowait");
         else embed(true);
         S.set_size(n);
-        start_weights(1u << Log2(n));
+        start_weights(1u << Log2(n), gather);
         check(grape_memcpy_d2h(&mismatches, d_count, sizeof(uint32_t), nullptr), "grape_memcpy_d2h");
         if (gather && mismatches != 0) embed(false);     // an element off the table: the tensors have to be there
     } catch (...) {
@@ -288,16 +288,16 @@ std::pair<void*, void*> commit_events() {
 }  // namespace
 
 // The weights of a lookup's rounds in one tensor: tables of every prefix of the point as far as the table side and rounds of 2^20
-// weights read them, and behind them those over the variables from GRAPE_EQ_SPLIT_LOW on (a long round's weight is a product of
-// two tables' entries, and the carried weights are the second one's).
+// weights read them, and behind them those over the variables from GRAPE_EQ_SPLIT_LOW on where something reads them (a longer round's
+// weight is a product of two tables' entries, and the carried weights are the second one's).
 namespace {
 struct WeightPlan {
     uint whole = 0, high = 0;
     bool split = false;
-    WeightPlan(uint nu, uint N) {
+    WeightPlan(uint nu, uint N, bool carry) {
         const uint all = nu ? nu - 1 : 0;
         whole = std::min(all, std::max(GRAPE_EQ_LONGEST_PREFIX, Log2(N)));
-        split = all >= GRAPE_EQ_SPLIT_LOW;
+        split = all > whole || carry;
         if (split) high = all - GRAPE_EQ_SPLIT_LOW;
     }
     size_t elems() const { return grape_eq_pyramid_elems(whole) + (split ? grape_eq_pyramid_elems(high) : 0); }
@@ -314,15 +314,21 @@ struct WeightPlan {
         a.period = 1u << GRAPE_EQ_SPLIT_LOW;
     }
 };
+// A witness on its table that is gathered in the first round: the long rounds carry their weights in S, from the third long
+// round on (2^19 elements: 0.68 ms either way; 2^17, one round: 0.49 against 0.47 ms, the factors' upload and tables are not
+// paid for; 2^22: 1.50 against 1.62 ms).  A table as long as the witness is no worse for it, though two multiples of every entry are
+// made and gathered past the caches (2^24 entries, 2^24 elements: 20.1 against 31.3 ms with what went before; 2^22 and 2^19:
+// 5.2 against 8.0, 2.6 against 3.1); beyond kCarriedTable their 128 bytes an entry are memory that such a proof has not asked for.
+bool may_carry(uint D, uint N) { return D / 8 >= kLongRoundPairs && N <= kCarriedTable; }
 }  // namespace
 
-void tLookup::start_weights(uint D) {
+void tLookup::start_weights(uint D, bool gather) {
     const uint nu = Log2(D);
     u_ready_ = forced_u_.empty() ? random_vec(nu) : forced_u_;
     forced_u_.clear();
     E_ready_.reset();
     if (u_ready_.size() != nu) return;          // run() reports the mismatch
-    const WeightPlan plan(nu, T.size);
+    const WeightPlan plan(nu, T.size, gather && may_carry(D, T.size));
     E_ready_.reset(new FrTensor((uint)plan.elems()));       // not OnDefaultStream: first written on the second stream
     // the point travels on the second stream too: on the default stream it would queue behind the pass over the
     // witness, and the pyramid with it
@@ -491,7 +497,8 @@ Fr tLookup::run(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax& hyrax
     // eq tables of the prefixes of u[0 .. nu-2]: round k (which binds variable nu-1-k) weights its
     // D / 2^(k+1) index pairs with those of nu-1-k variables; nothing is halved between rounds
     const uint nu = (uint)u.size();
-    const WeightPlan plan(nu, N);
+    const bool may = gather_S && may_carry(D, N);            // then start_weights was told to gather
+    const WeightPlan plan(nu, N, may);
     std::unique_ptr<FrTensor> E_own;
     if (E_early) {
         SideChain early(0);
@@ -652,12 +659,7 @@ Fr tLookup::run(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax& hyrax
             b.plain_sums = 1;
             carried.push_back(b);
         }
-        // A witness on its table that is gathered in the first round: the long rounds carry their weights in S, from the third long
-        // round on (2^19 elements: 0.68 ms either way; 2^17, one round: 0.49 against 0.47 ms, the factors' upload and tables are not
-        // paid for; 2^22: 1.50 against 1.62 ms).  A table as long as the witness is no worse for it, though two multiples of every entry are
-        // made and gathered past the caches (2^24 entries, 2^24 elements: 20.1 against 31.3 ms with what went before; 2^22 and 2^19:
-        // 5.2 against 8.0, 2.6 against 3.1); beyond kCarriedTable their 128 bytes an entry are memory that such a proof has not asked for.
-        if (gather_S && carried.size() >= 3 && N <= kCarriedTable) factors.reset(new CarriedFactors(u.data(), v.data(), nu, (uint)carried.size(), GRAPE_EQ_SPLIT_LOW));
+        if (may) factors.reset(new CarriedFactors(u.data(), v.data(), nu, (uint)carried.size(), GRAPE_EQ_SPLIT_LOW));
         const bool carry = factors && factors->ok;
         static_assert(kLongRoundPairs == 1u << GRAPE_EQ_SPLIT_LOW, "the last long round's pairs are one period");
         if (carry) {

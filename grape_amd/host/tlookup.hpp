@@ -50,8 +50,8 @@ protected:
     std::vector<Fr> forced_u_;
     // The weights of a proof over a witness of D (padded) elements - the object's random point u and the pyramid of
     // its eq tables - started on the second stream before the witness is indexed and counted, so that they are
-    // built beside those passes; run() takes them over.
-    void start_weights(uint D);
+    // built beside those passes; run() takes them over.  gather: the first round may work from the indices.
+    void start_weights(uint D, bool gather = false);
     std::vector<Fr> u_ready_;
     std::unique_ptr<FrTensor> E_ready_;
     bool indexed_commit_ = true;

@@ -121,6 +121,32 @@ static void carried_lookups() {
     expect(carried(8, 18) == 0, "as are short proofs");
 }
 
+// The weights over the high variables are made for the proofs that read them: rounds of more than 2^20 weights and carried ones.
+static void weights_that_are_read() {
+    const uint cols = 64, len = 256;
+    bn128 G = bn128::one();
+    Hyrax hyrax(1, cols, device_points(256 * cols), G, 1);
+    tLookupRange lookup(-128, len);
+    double seconds = 0;
+    auto pyramids = [&](uint log_D, bool ints) {
+        const uint D = 1u << log_D;
+        FrTensor S(D), A(D), S_out(D);
+        int* x = reinterpret_cast<int*>(device_points(D / 16));
+        const std::vector<int> map(len, 7);
+        tLookupRangeMapping mapping(-128, len, map.data());
+        const unsigned long before = fake_launched("eq_pyramid_head_kernel");
+        try {
+            if (ints) lookup.prove(x, S, A, random_vec(log_D), hyrax, cols, seconds);
+            else mapping.prove(S, S_out, A, random_vec(log_D), hyrax, cols, seconds);
+        } catch (const std::exception&) {
+        }
+        return fake_launched("eq_pyramid_head_kernel") - before;
+    };
+    expect(pyramids(16, true) == 1 && pyramids(17, true) == 1 && pyramids(18, true) == 1, "not for short proofs");
+    expect(pyramids(19, true) == 2 && pyramids(22, true) == 2, "for carried weights");
+    expect(pyramids(19, false) == 1 && pyramids(21, false) == 1 && pyramids(22, false) == 2, "without them, from 2^22 elements on");
+}
+
 // Mapping objects of the C calls are found by the mapped values: one other value is another object, also where the words it sits
 // in agree under xor with a rotated product; the same values are the same object.
 static void mapping_objects() {
@@ -375,6 +401,7 @@ int main(int argc, char** argv) {
         {"proof_after_a_refused_one", proof_after_a_refused_one},
         {"mapping_objects", mapping_objects},
         {"carried_lookups", carried_lookups},
+        {"weights_that_are_read", weights_that_are_read},
         {"tensor_memory_is_idle", tensor_memory_is_idle},
         {"sparse_commitment_table", sparse_commitment_table},
         {"operands_at_any_address", operands_at_any_address},
