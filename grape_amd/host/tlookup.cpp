@@ -12,6 +12,14 @@ using grape_host::OnDefaultStream;
 static inline uint32_t* W(fr_t* p) { return reinterpret_cast<uint32_t*>(p); }
 static inline const uint32_t* W(const fr_t* p) { return reinterpret_cast<const uint32_t*>(p); }
 
+namespace {
+// A witness round over at least this many index pairs runs before the commitments of its proof, a
+// shorter one (launch-bound) beside them.
+constexpr uint kLongRoundPairs = 1u << 16;
+// The first round of a witness of D elements may take A and S from the tables by index: it is a long one and pairs whole halves.
+bool first_round_gathers(uint D) { return D == (1u << Log2(D)) && D / 2 >= kLongRoundPairs; }
+}  // namespace
+
 // src/tlookup.cu:247: beta is the table size, alpha is random
 tLookup::tLookup(const uint size) : alpha(Fr::random_element()), beta(Fr((long)size)), T(size), B(size), m(size) {}
 tLookup::~tLookup() {
@@ -223,9 +231,6 @@ bool tLookup::commit_A_by_occupancy(FrTensor* A, uint D, uint msm_size, Hyrax& h
 }
 
 namespace {
-// A witness round over at least this many index pairs runs before the commitments of its proof, a
-// shorter one (launch-bound) beside them.
-constexpr uint kLongRoundPairs = 1u << 16;
 constexpr uint kCarriedTable = 1u << 24;           // longest table whose multiples carried rounds gather: 2 GiB
 // A stream beside the default one (two per process, created on first use) and the two events that order it against
 // the default stream: begin() makes it wait for what the default stream has queued, end() makes the
@@ -429,9 +434,10 @@ Fr tLookup::run(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax& hyrax
     // left A unwritten, the first round gathers it from B - if that round is one of the long ones queued
     // beside the commitments; otherwise A is written out now.
     bool from_table = a_ready_;
-    const bool gather_first = a_deferred_ && D == (1u << Log2(D)) && D / 2 >= kLongRoundPairs && A.size >= D;
-    // the witness itself too: what prove() did not write out is written now where the first round cannot gather
+    const bool gather_first = a_deferred_ && first_round_gathers(D) && A.size >= D;
+    // the witness itself too; prove() may have left it unwritten, and where the first round cannot gather it is written now
     const bool gather_S = gather_first && s_by_index_;
+    if (s_by_index_ && !gather_S) gather_by_index(S, T, D);
     a_ready_ = a_deferred_ = s_by_index_ = false;
     if (gather_first) from_table = true;
     if (!from_table && d_idx_) {
@@ -864,7 +870,7 @@ Fr tLookupRange::prove(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax
     if (D == (1u << Log2(D)) && A.size >= D) {
         // no padding: index and A = B[index] in one pass (starts the weights too); A stays unwritten where the
         // first round can gather it from B (a witness of 2^17 elements and more, committed through its indices)
-        const bool gather = indexed_commit_ && index_known_ && D / 2 >= (1u << 16);
+        const bool gather = indexed_commit_ && index_known_ && first_round_gathers(D);
         make_index_and_A(S, low, A, nullptr, nullptr, !gather);
     } else {
         start_weights(1u << Log2(D));
@@ -925,7 +931,7 @@ Fr tLookupRange::prove(const int* device_int_S, FrTensor& S, FrTensor& A, const 
         S.get_data(D, const_cast<int*>(device_int_S));
         return prove(S, A, v, hyrax, msm_size, commit_time);
     }
-    const bool gather = indexed_commit_ && index_known_ && D / 2 >= (1u << 16);
+    const bool gather = indexed_commit_ && index_known_ && first_round_gathers(D);
     make_index_from_ints(device_int_S, nullptr, D, low, S, A, nullptr, nullptr, gather);
     m_pending_ = true;
     m_pending_size_ = D;
@@ -1041,7 +1047,7 @@ Fr tLookupRangeMapping::prove(const int* device_int_S_in, const int* device_int_
     // index and the check S_out = f(S_in) against the integer table in one pass over the integers; A = B[index] and the combined witness
     // S_in + r * S_out = T[index] are gathered by a long first round, written by the same pass for a short one
     FrTensor S(D, OnDefaultStream());
-    make_index_from_ints(device_int_S_in, device_int_S_out, D, low, S, A, d_map_int_, &r, D / 2 >= (1u << 16));
+    make_index_from_ints(device_int_S_in, device_int_S_out, D, low, S, A, d_map_int_, &r, first_round_gathers(D));
     index_to_m(D, low);
     Fr ret;
     try {
