@@ -5,7 +5,9 @@ import ctypes
 import numpy as np
 import pytest
 import torch
-from gpuutil import rand_fr
+import bigref as br
+import orc
+from gpuutil import assert_same, rand_fr
 
 pytestmark = pytest.mark.gpu
 
@@ -116,3 +118,64 @@ def test_sparse_commitment_of_table_entries(ops, rows, live):
     out2 = ops.g1_empty(rows)
     _capi.check(lib.grape_commit_fr_strided_masked_indexed(p(out2), p(entries), p(idx), p(dskip), rows * cols, cols, p(strided), cols, c, J, nsets, None))
     assert torch.equal(out2, plain)
+
+
+_TABLES = []        # the host objects are found by their table's address: it stays taken until the process ends
+
+
+# one long round, and long rounds that carry their weights
+@pytest.mark.parametrize("logD", [17, 19])
+@pytest.mark.parametrize("kind", ["range, key below", "range, key above", "mapping, key above", "mapping, wrong output"])
+def test_proof_of_a_witness_off_its_table(ops, logD, kind):
+    """one element off the table is refused; the object then proves a witness on it, refuses a point that is too short, and still
+    refuses a padded witness of field elements that is off the table"""
+    from grape_amd import _host as host
+    host.load()
+    if not _TABLES:
+        _TABLES.append(ops.g1_table_gen(ops.g1_make_generators(rand_fr(256, 31)), 256))
+    table = _TABLES[0]
+    D, N, low, mapping = 1 << logD, 1 << 7, -40, kind.startswith("mapping")
+    rng = np.random.default_rng(logD)
+    fmap = rng.integers(-1000, 1000, N).astype(np.int32)
+    alpha, r, u, v = rand_fr(1, 32), rand_fr(1, 33), rand_fr(logD, 34), rand_fr(logD, 35)
+    beta = br.fr_pack([N])[0]
+    T, B = orc.tlookup_init(low, N, beta, *((orc.from_i32(fmap), r[0]) if mapping else ()))
+
+    def prove(x, y, fmt="i32", vars=logD):
+        host.set_input_format(fmt)
+        if fmt == "fr":
+            dx, dy = (ops.to_dev(orc.from_i32(a)) for a in (x, y))
+        else:
+            dx, dy = (torch.from_numpy(a).cuda() for a in (x, y))
+        try:
+            if mapping:
+                return host.tlookup_mapping_prove(dx, dy, x.size, low, N, fmap, alpha, r, u[:vars], v[:vars], table, 256, 1, 256)
+            res = host.tlookup_range_prove(dx, x.size, low, N, alpha, u[:vars], v[:vars], table, 256, 1, 256)
+            return res["transcript"], res["S_claim"]
+        finally:
+            host.set_input_format("fr")
+
+    x = rng.integers(low, low + N, D).astype(np.int32)
+    y = fmap[x - low]
+    bad_x, bad_y = x.copy(), y.copy()
+    if "output" in kind:
+        bad_y[D // 3] += 1
+    else:
+        bad_x[D // 3] = low - 1 if "below" in kind else low + N
+    with pytest.raises(host.HostError, match="claim != p\\(0\\) \\+ p\\(1\\)"):
+        prove(bad_x, bad_y)
+    S = orc.from_i32(x)
+    if mapping:
+        S = orc.vec2("orc_fr_vec_add", orc.vec_bcast("orc_fr_vec_bcast_mul", orc.from_i32(y), r[0]), S)
+    st, transcript, at_v = orc.tlookup_prove(S, T, B, orc.tlookup_prep(orc.from_i32(x), low, N), alpha[0], beta, u, v)
+    assert st == 0
+    got, claim = prove(x, y)
+    assert_same(got, transcript, "transcript")
+    assert_same(claim, at_v, "S(v)")
+    with pytest.raises(host.HostError, match="size"):
+        prove(x, y, vars=logD - 1)
+    n = D // 16384 * 11008                               # rows that the prover pads to 16384
+    assert D // 3 < n
+    x, y = bad_x[:n].copy(), bad_y[:n].copy()
+    with pytest.raises(host.HostError, match="claim != p\\(0\\) \\+ p\\(1\\)"):
+        prove(x, y, "fr")
