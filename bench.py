@@ -44,7 +44,7 @@ FP_WORDS, FP_LIMBS30 = (8, 9) if CURVE == "bn254" else (12, 13)
 ALG_MULS_PER_POINT = 2 * 10 * (2 * FP_WORDS * FP_WORDS + FP_WORDS)
 # What the fast path executes: ONE mixed addition per point on L limbs of 30 bits (L = 13 resp.
 # 9): 6 products of L*L + L*L + 1 multiply-adds, one fused difference of two products
-# (2*L*L + L*L + 1), 2 squares of L(L+1)/2 + L*L + 1 and 4 subtractions inside products of L - 1: 3112 for L = 13, 1526 for L = 9.
+# (2*L*L + L*L + 1), 2 squares of L(L+1)/2 + L*L + 1 and 4 subtractions inside products of L - 1: 3112 for L = 13, 1508 for L = 9.
 _L = FP_LIMBS30
 EXEC_MULS_PER_POINT = 6 * (2 * _L * _L + 1) + (3 * _L * _L + 1) + 2 * (_L * (_L + 1) // 2 + _L * _L + 1) + 4 * (_L - 1)
 # lane-level 32x32 multiplies per second if every SIMD issued one v_mad_u64_u32 per cycle:

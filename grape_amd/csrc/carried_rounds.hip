@@ -12,7 +12,8 @@
 // long round is a factor per period.  Challenges and coordinates of the point that are 0 or 1 have no inverse: such proofs
 // take wround2_kernel (the host asks).
 //
-// A lookup's first round has A (S + beta) = 1 at every index, so q(0) = q(1) = 1 and it sums nothing weighted.  Gathered by
+// A lookup's first round has A (S + beta) = 1 at every index, so q(0) = q(1) = 1 and it sums nothing weighted (a table with an
+// entry that has no inverse is refused by the table side's rounds, which sum B (T + beta)).  Gathered by
 // index, its folds are sums of two table entries: v x1 + (1 - v) x0 with both multiples of every entry made before.
 // Bound: instruction issue and HBM about evenly (a pair of later rounds is six elements, 192 bytes, at 4.7 TB/s).  Against
 // wround2_kernel: the gathered first round of 2^26 pairs 2.8 -> 2.1 ms, a round of 2^25 pairs 1.77 -> 1.34 ms, the first

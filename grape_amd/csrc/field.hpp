@@ -185,7 +185,6 @@ struct alignas(16) Mont {
 
 namespace detail {
 
-// One word of a carry / borrow chain (carry and borrow are 0 or 1).  With clang the builtins become
 // c + a b as one multiply-add: a column of a product.  Left to itself the compiler reorders a column's sum - starting
 // values last, as additions of their own - and splits products with known factors (150 instructions more in a mixed
 // addition of fp28.hpp).  The annotation is gone after the passes that would do so.
@@ -213,6 +212,7 @@ GRAPE_HD T unknown(T x) {
     return x;
 }
 
+// One word of a carry / borrow chain (carry and borrow are 0 or 1).  With clang the builtins become
 // one add-with-carry / subtract-with-borrow instruction per word on the device (64-bit emulation of
 // the chain costs three to four times as many instructions there); other compilers spell it out.
 GRAPE_HD uint32_t adc32(uint32_t a, uint32_t b, uint32_t& carry) {

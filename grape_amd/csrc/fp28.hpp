@@ -546,9 +546,10 @@ GRAPE_HD Fp28 inverse_by(const Fp28& a) {
 }  // namespace fp28
 
 // ------------------------------------------------------------------------------------------------
-// XYZZ accumulator in the working form.  Invariants between additions: all coordinates balanced, |x| < 3.5p,
-// |y| < p, zz and zzz below p and never congruent to zero; `inf` marks the identity.  All of the values below stay
-// under 14 p, all products of them far under 630 p^2 (BN254: |y| < 1.5p).
+// XYZZ accumulator in the working form.  Invariants between additions: all coordinates balanced, zz below p, zz and zzz
+// never congruent to zero, |x| < 3.5p, |y| and zzz below p; on BN254, where a product in wide digits reaches 1.4p,
+// |x| < 5.7p (R^2 less PPP and 2Q) and zzz < 1.4p.  `inf` marks the identity.  All of the values below stay under 14 p (BN254: 23 p),
+// all products of them far under 630 p^2 (86000 p^2).
 // ------------------------------------------------------------------------------------------------
 struct Xyzz28 {
     Fp28 x, y, zz, zzz;

@@ -239,8 +239,8 @@ GRAPE_HD Limbs canon_wide(const Limbs& t) {
     return canon(normalize(d), 1);
 }
 
-// limb-wise sum of at most 16 packed elements or differences of packed elements (|limb| < 2^30,
-// value within (-add_r * r, (32 - add_r) * r)) -> canonical element of memory form
+// limb-wise sum of packed elements or differences of packed elements (|limb + add_r * R| < 2^31: up to 31 elements or 16 differences
+// with add_r = 16; value within (-add_r * r, (32 - add_r) * r)) -> canonical element of memory form
 GRAPE_HD Fr limb_sum_to_fr(const Limbs& s, int add_r) {
     Limbs d;
 #pragma unroll

@@ -318,7 +318,7 @@ static Fr eleMul_rounds(fr_t* Aw, fr_t* Bw, const fr_t* A, const fr_t* B, fr_t* 
         hu = us.data() + rounds;
         hv = vs.data() + rounds;
     }
-    // Long rounds: the weights of a padded row split into row and column, those of whole powers of two at 2^17.  A row whose
+    // Long rounds: the weights of a padded row split into row and column, those of whole powers of two at 2^kSplitLow.  A row whose
     // padded length has no prefix table of its own (above 2^20) is weighed by whole tables.
     const uint lg_row = Log2(second_size);
     const bool padded = second_size != row_pad;

@@ -1,4 +1,4 @@
-// Host build of the 28-bit-limb Fp arithmetic (grape_amd/csrc/fp28.hpp) behind a few C entry
+// Host build of the Fp arithmetic on 30-bit limbs (grape_amd/csrc/fp28.hpp) behind a few C entry
 // points, so that the CPU test-suite can check it against Python integers and the oracle.
 #include <cstring>
 #include <vector>
@@ -8,7 +8,7 @@ static constexpr int FW = FpParams::N;     // 32-bit words of an Fp element in m
 static constexpr size_t FB = 4 * FW;       // bytes
 
 extern "C" {
-// canonical memory form (FW x u32) in, canonical out, through the 28-bit domain
+// canonical memory form (FW x u32) in, canonical out, through the working form
 void t28_mul(const uint32_t* a, const uint32_t* b, uint32_t* out) {
     Fp x, y;
     memcpy(&x, a, FB);
@@ -52,7 +52,7 @@ int t28_is_zero(const uint32_t* a, int times_p) {
     for (int i = 0; i < fp28::N; i++) v.v[i] += times_p * fp28::P(i);
     return fp28::is_zero_mod_p(fp28::normalize(v)) ? 1 : 0;
 }
-// sum_i (+-) points[i] through the 28-bit mixed addition; affine points canonical 2 FW x u32;
+// sum_i (+-) points[i] through the working form's mixed addition; affine points canonical 2 FW x u32;
 // returns the number of exceptional steps that had to take the exact path
 int t28_sum(const uint32_t* points, const int* negate, int n, uint32_t* out_xyzz) {
     Xyzz28 acc = xyzz28_inf();
@@ -76,7 +76,7 @@ int t28_sum(const uint32_t* points, const int* negate, int n, uint32_t* out_xyzz
     return slow;
 }
 // tree-style sum: partial sums of two halves combined with the accumulator+accumulator addition,
-// affine result through the 28-bit inversion
+// affine result through the working form's inversion
 int t28_sum_tree(const uint32_t* points, const int* negate, int n, uint32_t* out_affine) {
     Xyzz28 part[2] = {xyzz28_inf(), xyzz28_inf()};
     int slow = 0;

@@ -40,5 +40,11 @@ void fr26_product(const int32_t* a, const int32_t* b, int add_r, int32_t* out) {
     const fr26::Limbs r = fr26::product(A, B, add_r);
     memcpy(out, r.v, sizeof r.v);
 }
+void fr26_limb_sum(const int32_t* sum, int add_r, uint32_t* out) {
+    fr26::Limbs s;
+    memcpy(s.v, sum, sizeof s.v);
+    const Fr r = fr26::limb_sum_to_fr(s, add_r);
+    memcpy(out, r.v, sizeof r.v);
+}
 int fp28_zero(const int32_t* a, const int32_t* b) { return fp28::is_zero(fp28::mulb_below_p(load(a), load(b))) ? 1 : 0; }
 }

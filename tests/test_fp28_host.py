@@ -1,6 +1,6 @@
-"""CPU checks of the 28-bit-limb lazy Fp arithmetic used by the commitment kernels (host build of
+"""CPU checks of the lazy Fp arithmetic on 30-bit limbs used by the commitment kernels (host build of
 grape_amd/csrc/fp28.hpp): products, squares, conversions and lazily reduced expressions against
-Python integers; sums of points through the 28-bit mixed addition against textbook affine
+Python integers; sums of points through its mixed addition against textbook affine
 arithmetic, including the exceptional cases (doubling, cancellation, identity)."""
 import ctypes
 import os
@@ -168,7 +168,7 @@ def test_accumulator_plus_accumulator(lib):
 
 
 def test_doubling_chain_horner(lib):
-    """sum_j 2^(d j) P_j by Horner with the 28-bit doubling (from the top point down): against the
+    """sum_j 2^(d j) P_j by Horner with the working form's doubling (from the top point down): against the
     textbook group law for several chain lengths, with identities among the points and after them"""
     rng = random.Random(6)
     for n, d in ((1, 3), (2, 1), (3, 16), (5, 7), (4, 17)):

@@ -120,3 +120,27 @@ def test_scalar_product_in_wide_digits(lib):
                 # between exact / 2^260 + add_r r and (1 + 2^-20) r above
                 low = v * (1 << (w * n)) - exact - add_r * r * (1 << (w * n))
                 assert 0 <= low < r * ((1 << (w * n)) + (1 << (w * n - 20)))
+
+
+def test_limb_sums_at_their_bounds(lib):
+    """sums of up to 31 elements and of 16 differences, with the largest limbs that elements have: 24 are what a thread of the carried
+    rounds adds up"""
+    n, r, w, rng = 10, br.R_MOD, 26, random.Random(8)
+    limbs = lambda v: np.array([(v >> (w * i)) & ((1 << w) - 1) for i in range(n)], dtype=np.int32)
+    ones = (1 << (w * (n - 1))) - 1                      # the low limbs all ones
+    elements = [0, 1, r - 1, ones, (((r >> (w * (n - 1))) - 1) << (w * (n - 1))) + ones, rng.randrange(r)]
+    out = np.zeros(8, dtype=np.uint32)
+
+    def check(total, add_r, want):
+        assert np.abs(total + add_r * limbs(r).astype(np.int64)).max() < 1 << 31
+        lib.fr26_limb_sum(_ptr(total.astype(np.int32)), add_r, out.ctypes.data_as(ctypes.POINTER(ctypes.c_uint32)))
+        assert sum(int(x) << (32 * i) for i, x in enumerate(out)) == want % r
+
+    for count in (1, 16, 24, 31):
+        for v in elements:
+            check(count * limbs(v).astype(np.int64), 0, count * v)
+        mixed = [rng.choice(elements + [rng.randrange(r)]) for _ in range(count)]
+        check(sum(limbs(v).astype(np.int64) for v in mixed), 0, sum(mixed))
+    for a in elements:
+        for b in elements:
+            check(16 * (limbs(a).astype(np.int64) - limbs(b)), 16, 16 * (a - b))
