@@ -1,5 +1,5 @@
 // Modular inversion by divsteps (Bernstein-Yang "safegcd"), batched 30 steps at a time on signed
-// 30-bit limbs: the pieces shared by the base field's working form (fp28.hpp) and the memory form
+// 30-bit limbs: the pieces shared by the base field's working form (fp30.hpp) and the memory form
 // of either field (inverse_by below).  A 255-bit modulus takes at most 741 divsteps (25 batches of
 // a few hundred instructions), a 381-bit one 1110 - an order of magnitude fewer sequential
 // instructions than the a^(m-2) ladder, which matters wherever one inversion is a latency chain

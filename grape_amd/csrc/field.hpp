@@ -187,7 +187,7 @@ namespace detail {
 
 // c + a b as one multiply-add: a column of a product.  Left to itself the compiler reorders a column's sum - starting
 // values last, as additions of their own - and splits products with known factors (150 instructions more in a mixed
-// addition of fp28.hpp).  The annotation is gone after the passes that would do so.
+// addition of fp30.hpp).  The annotation is gone after the passes that would do so.
 GRAPE_HD void keep_sum(int64_t& c) {
 #if defined(__HIP_DEVICE_COMPILE__)
     c = __builtin_annotation(c, "sum");

@@ -1,6 +1,5 @@
 // Fp on signed limbs of 30 bits with lazy reduction - the working form of the commitment kernels
-// (13 limbs, radix 2^390, for BLS12-381; 9 limbs, radix 2^270, for BN254).  The names keep the 28
-// of the form's first limb width.
+// (13 limbs, radix 2^390, for BLS12-381; 9 limbs, radix 2^270, for BN254).
 //
 // Why: on gfx950 a 32x32+64 multiply-add (v_mad_i64_i32 / v_mad_u64_u32) issues at the same rate
 // as an addition, so the cost of a field product is its instruction count, and with saturated
@@ -23,7 +22,7 @@
 // boundary.  The last column takes the ordinary step (a digit of -T0/p, times p), so that the result does not
 // carry the factor 2^30 that the others would leave in it.
 //
-// Bounds (checked by the callers' comments).  Values: mul28(a, b) with |a| < alpha*p, |b| < beta*p
+// Bounds (checked by the callers' comments).  Values: mul30(a, b) with |a| < alpha*p, |b| < beta*p
 // is a balanced number of magnitude below (0.51 + alpha*beta/630) p; for BN254 0.94 p (1.4 p from wide digits)
 // instead of 0.51 p, and 86000 instead of 630 - below p for every product here, wide digits on BN254 apart, so that a
 // product is zero mod p only when all its limbs are zero.  Columns: a sum of 12 limb products of balanced operands is
@@ -37,11 +36,11 @@
 namespace grape {
 
 #if defined(GRAPE_CURVE_BN254)
-struct Fp28 {
+struct Fp30 {
     int32_t v[9];
 };
 
-namespace fp28 {
+namespace fp30 {
 
 using detail::mad;
 using detail::unknown;
@@ -71,7 +70,7 @@ GRAPE_HD int32_t ONE(int i) {   // 2^270 mod p
     constexpr int32_t t[9] = {0x24fcf82, -0xe183b72, 0x1ac0210c, 0x1f4f4b0c, 0x100896b9, -0xae44a8a, -0x6d2519d, -0x1ab5fcf1, -0x8c8};
     return t[i];
 }
-GRAPE_HD int32_t CMEM(int i) {   // 2^256 mod p: mul28(x*2^270, CMEM) = x*2^256
+GRAPE_HD int32_t CMEM(int i) {   // 2^256 mod p: mul30(x*2^270, CMEM) = x*2^256
     constexpr int32_t t[9] = {0x58f0d9d, 0xd750e37, 0x1c70b3dd, 0x1e3aca3d, -0x6b9d3f6, -0x572421e, -0x20d0999, 0x1df06682, 0xe0a};
     return t[i];
 }
@@ -80,7 +79,7 @@ GRAPE_HD uint32_t MCONV(int i) {
     constexpr uint32_t t[8] = {0x5accccc9u, 0xf89a7d3au, 0x9a1dcc9du, 0x50fea7bdu, 0xdf1160f4u, 0x9e7d8ca3u, 0xed6d3304u, 0x279be39au};
     return t[i];
 }
-GRAPE_HD int32_t CIN(int i) {   // 2^284 mod p: mul28(pack(x*2^256), CIN) = x*2^270
+GRAPE_HD int32_t CIN(int i) {   // 2^284 mod p: mul30(pack(x*2^256), CIN) = x*2^270
     constexpr int32_t t[9] = {-0x1019212e, -0x66eb814, -0x18cbc210, -0x103b9669, 0x63da561, 0x14d661fb, 0x15e36864, 0x1768c0ce, 0x1291};
     return t[i];
 }
@@ -90,11 +89,11 @@ GRAPE_HD int32_t R3(int i) {   // R'^3 mod p: turns the plain inverse of a Montg
 }
 
 #else
-struct Fp28 {
+struct Fp30 {
     int32_t v[13];
 };
 
-namespace fp28 {
+namespace fp30 {
 
 using detail::mad;
 using detail::unknown;
@@ -129,7 +128,7 @@ GRAPE_HD int32_t ONE(int i) {   // 2^390 mod p
                                0x9b42da1, -0x1a113d94, 0x15d98f13, 0x4b29f14, -0x1a603060, 0x15dea};
     return t[i];
 }
-GRAPE_HD int32_t CMEM(int i) {   // 2^384 mod p: mul28(x*2^390, CMEM) = x*2^384
+GRAPE_HD int32_t CMEM(int i) {   // 2^384 mod p: mul30(x*2^390, CMEM) = x*2^384
     constexpr int32_t t[13] = {0x35552, -0xfd80000, -0x147fffd4, 0x12000345, 0x166296cd, 0x1f16d974, 0x14485f81,
                                0x3339f33, -0x69eca9, 0xb857c2d, 0x1f910eb7, -0x98fbfc1, -0x40ab3};
     return t[i];
@@ -140,7 +139,7 @@ GRAPE_HD uint32_t MCONV(int i) {
                                 0xb683dcf8u, 0xc26c26d0u, 0x63c4a5eeu, 0x29f14576u, 0x7f3e804bu, 0x015de996u};
     return t[i];
 }
-GRAPE_HD int32_t CIN(int i) {   // 2^396 mod p: mul28(pack(x*2^384), CIN) = x*2^390
+GRAPE_HD int32_t CIN(int i) {   // 2^396 mod p: mul30(pack(x*2^384), CIN) = x*2^390
     constexpr int32_t t[13] = {-0xb7f3481, -0x1f3ffff, -0x1fbd4ed9, -0xcc8550, -0x21b4b2e, 0x1e015cf2, 0x5c540d,
                                -0xb984e66, -0xad5925c, 0x19d89d1a, -0x1046501a, -0x7b737e8, 0x97730};
     return t[i];
@@ -156,28 +155,28 @@ GRAPE_HD int32_t R3(int i) {   // R'^3 mod p: turns the plain inverse of a Montg
 constexpr uint32_t MASK = (1u << W) - 1;
 constexpr int32_t HALF = 1 << (W - 1);
 
-GRAPE_HD Fp28 one() {
-    Fp28 r;
+GRAPE_HD Fp30 one() {
+    Fp30 r;
 #pragma unroll
     for (int i = 0; i < N; i++) r.v[i] = ONE(i);
     return r;
 }
-GRAPE_HD Fp28 zero() {
-    Fp28 r;
+GRAPE_HD Fp30 zero() {
+    Fp30 r;
 #pragma unroll
     for (int i = 0; i < N; i++) r.v[i] = 0;
     return r;
 }
 
 // limb-wise, no carries: the caller tracks magnitudes
-GRAPE_HD Fp28 sub(const Fp28& a, const Fp28& b) {
-    Fp28 r;
+GRAPE_HD Fp30 sub(const Fp30& a, const Fp30& b) {
+    Fp30 r;
 #pragma unroll
     for (int i = 0; i < N; i++) r.v[i] = a.v[i] - b.v[i];
     return r;
 }
-GRAPE_HD Fp28 cneg(const Fp28& a, bool flag) {
-    Fp28 r;
+GRAPE_HD Fp30 cneg(const Fp30& a, bool flag) {
+    Fp30 r;
     const int32_t m = flag ? -1 : 0;
 #pragma unroll
     for (int i = 0; i < N; i++) r.v[i] = (a.v[i] ^ m) - m;
@@ -185,8 +184,8 @@ GRAPE_HD Fp28 cneg(const Fp28& a, bool flag) {
 }
 
 // signed carry propagation: same value, limbs 0..N-2 in [0, 2^30); any 32-bit limbs
-GRAPE_HD Fp28 normalize(const Fp28& a) {
-    Fp28 r;
+GRAPE_HD Fp30 normalize(const Fp30& a) {
+    Fp30 r;
     int32_t c = 0;
 #pragma unroll
     for (int i = 0; i < N - 1; i++) {
@@ -201,8 +200,8 @@ GRAPE_HD int32_t low30(uint32_t a) { return (int32_t)(a << (32 - W)) >> (32 - W)
 // same value, balanced (up to 2 over 2^29: the limbs' carries are taken side by side, not along a chain).  Limbs below
 // 3 * 2^29 - a sum or difference of two balanced numbers, a double - or, with ANY, any of 32 bits.
 template <bool ANY = false>
-GRAPE_HD Fp28 balance(const Fp28& a) {
-    Fp28 r;
+GRAPE_HD Fp30 balance(const Fp30& a) {
+    Fp30 r;
     int32_t c = 0;
 #pragma unroll
     for (int i = 0; i < N - 1; i++) {
@@ -251,8 +250,8 @@ GRAPE_HD void reduce_column(Columns& t, int i) {
     }
 }
 // the upper columns, carries propagated: the upper words along the columns, the two bits left over above a limb's 30 to the next limb
-GRAPE_HD Fp28 finish(Columns& t) {
-    Fp28 r;
+GRAPE_HD Fp30 finish(Columns& t) {
+    Fp30 r;
     int32_t over = 0;
 #pragma unroll
     for (int k = 0; k < N - 1; k++) {
@@ -266,7 +265,7 @@ GRAPE_HD Fp28 finish(Columns& t) {
     return r;
 }
 // the same less w * s: an addend costs a multiply-add a limb here, and the difference comes out balanced
-GRAPE_HD void less(Columns& t, int32_t& top, const Fp28& s, int32_t w) {
+GRAPE_HD void less(Columns& t, int32_t& top, const Fp30& s, int32_t w) {
     const int32_t f = unknown(-w);
 #pragma unroll
     for (int k = 0; k < N - 1; k++) mad(t.c[N + k], s.v[k], f);
@@ -275,7 +274,7 @@ GRAPE_HD void less(Columns& t, int32_t& top, const Fp28& s, int32_t w) {
 
 // Montgomery product a*b/R' (mod p)
 template <bool WIDE>
-GRAPE_HD Fp28 mul_impl(const Fp28& a, const Fp28& b) {
+GRAPE_HD Fp30 mul_impl(const Fp30& a, const Fp30& b) {
     Columns t;
     start<WIDE>(t);
 #pragma unroll
@@ -285,13 +284,13 @@ GRAPE_HD Fp28 mul_impl(const Fp28& a, const Fp28& b) {
     }
     return finish(t);
 }
-GRAPE_HD Fp28 mul(const Fp28& a, const Fp28& b) { return mul_impl<false>(a, b); }
+GRAPE_HD Fp30 mul(const Fp30& a, const Fp30& b) { return mul_impl<false>(a, b); }
 // both operands balanced: reduced in wide digits, 12 instructions less
-GRAPE_HD Fp28 mulb(const Fp28& a, const Fp28& b) { return mul_impl<true>(a, b); }
+GRAPE_HD Fp30 mulb(const Fp30& a, const Fp30& b) { return mul_impl<true>(a, b); }
 // both operands balanced, the product below p (wide digits take DOWN twice: too much where that is near p / 2)
-GRAPE_HD Fp28 mulb_below_p(const Fp28& a, const Fp28& b) { return mul_impl<kSmallDown>(a, b); }
+GRAPE_HD Fp30 mulb_below_p(const Fp30& a, const Fp30& b) { return mul_impl<kSmallDown>(a, b); }
 // a*b/R' - s, both factors balanced
-GRAPE_HD Fp28 mulb_less(const Fp28& a, const Fp28& b, const Fp28& s) {
+GRAPE_HD Fp30 mulb_less(const Fp30& a, const Fp30& b, const Fp30& s) {
     Columns t;
     start<true>(t);
     int32_t top = 0;
@@ -301,14 +300,14 @@ GRAPE_HD Fp28 mulb_less(const Fp28& a, const Fp28& b, const Fp28& s) {
         add_row(t, i, a.v, b.v[i]);
         reduce_column<true>(t, i);
     }
-    Fp28 r = finish(t);
+    Fp30 r = finish(t);
     r.v[N - 1] += top;
     return r;
 }
 
 // a*b - c*d with one Montgomery reduction: both products accumulate in the same columns, so all four operands have to be
 // balanced.
-GRAPE_HD Fp28 mul_sub(const Fp28& a, const Fp28& b, const Fp28& c, const Fp28& d) {
+GRAPE_HD Fp30 mul_sub(const Fp30& a, const Fp30& b, const Fp30& c, const Fp30& d) {
     Columns t;
     start<false>(t);
     int32_t nc[N];                        // limb-wise negation keeps every step a multiply-add
@@ -325,7 +324,7 @@ GRAPE_HD Fp28 mul_sub(const Fp28& a, const Fp28& b, const Fp28& c, const Fp28& d
 
 // the columns of a^2 (a balanced): the off-diagonal limb products are taken once with a doubled operand
 template <bool WIDE>
-GRAPE_HD void square(Columns& t, const Fp28& a) {
+GRAPE_HD void square(Columns& t, const Fp30& a) {
     int32_t a2[N];
 #pragma unroll
     for (int i = 0; i < N; i++) a2[i] = a.v[i] * 2;
@@ -339,40 +338,40 @@ GRAPE_HD void square(Columns& t, const Fp28& a) {
     for (int i = 0; i < N; i++) reduce_column<WIDE>(t, i);
 }
 template <bool WIDE>
-GRAPE_HD Fp28 sqr_impl(const Fp28& a) {
+GRAPE_HD Fp30 sqr_impl(const Fp30& a) {
     Columns t;
     start<WIDE>(t);
     square<WIDE>(t, a);
     return finish(t);
 }
-GRAPE_HD Fp28 sqr(const Fp28& a) { return sqr_impl<true>(a); }
-GRAPE_HD Fp28 sqr_below_p(const Fp28& a) { return sqr_impl<kSmallDown>(a); }
+GRAPE_HD Fp30 sqr(const Fp30& a) { return sqr_impl<true>(a); }
+GRAPE_HD Fp30 sqr_below_p(const Fp30& a) { return sqr_impl<kSmallDown>(a); }
 // a^2/R' - s - 2u
-GRAPE_HD Fp28 sqr_less(const Fp28& a, const Fp28& s, const Fp28& u) {
+GRAPE_HD Fp30 sqr_less(const Fp30& a, const Fp30& s, const Fp30& u) {
     Columns t;
     start<true>(t);
     int32_t top = 0;
     less(t, top, s, 1);
     less(t, top, u, 2);
     square<true>(t, a);
-    Fp28 r = finish(t);
+    Fp30 r = finish(t);
     r.v[N - 1] += top;
     return r;
 }
 
 // Is a product below p congruent to zero?
-GRAPE_HD bool is_zero(const Fp28& a) {
+GRAPE_HD bool is_zero(const Fp30& a) {
     uint32_t z = 0;
 #pragma unroll
     for (int i = 0; i < N; i++) z |= (uint32_t)a.v[i];
     return z == 0;
 }
 // Is a value of up to a few p, one lazy operand, congruent to zero?
-GRAPE_HD bool is_zero_mod_p(const Fp28& a) { return is_zero(mul(a, one())); }
+GRAPE_HD bool is_zero_mod_p(const Fp30& a) { return is_zero(mul(a, one())); }
 
 // the value in [0, p), normalised, of a product below p
-GRAPE_HD Fp28 canonical(const Fp28& product) {
-    Fp28 t = normalize(product);
+GRAPE_HD Fp30 canonical(const Fp30& product) {
+    Fp30 t = normalize(product);
     const int32_t neg = t.v[N - 1] >> 31;
 #pragma unroll
     for (int i = 0; i < N; i++) t.v[i] += P(i) & neg;
@@ -382,8 +381,8 @@ GRAPE_HD Fp28 canonical(const Fp28& product) {
 // ---- conversions with the canonical 32-bit-limb Montgomery form (radix 2^384 resp. 2^256) ----
 constexpr int FW = FpParams::N;   // 32-bit words of the canonical form
 // pure re-limbing of a non-negative integer of FW words (normalised)
-GRAPE_HD Fp28 pack(const Fp& x) {
-    Fp28 r;
+GRAPE_HD Fp30 pack(const Fp& x) {
+    Fp30 r;
 #pragma unroll
     for (int k = 0; k < N; k++) {
         const int bit = W * k, q = bit >> 5, s = bit & 31;
@@ -393,7 +392,7 @@ GRAPE_HD Fp28 pack(const Fp& x) {
     return r;
 }
 // inverse of pack for a normalised, non-negative value below 2^(32 FW)
-GRAPE_HD Fp unpack(const Fp28& a) {
+GRAPE_HD Fp unpack(const Fp30& a) {
     Fp r;
 #pragma unroll
     for (int q = 0; q < FW; q++) {
@@ -417,7 +416,7 @@ GRAPE_HD Fp unpack(const Fp28& a) {
     return r;
 }
 // canonical memory form (32-bit limbs) -> the value in [0, p) in the working form, balanced
-GRAPE_HD Fp28 from_canonical(const Fp& x) {
+GRAPE_HD Fp30 from_canonical(const Fp& x) {
     Fp m;
 #pragma unroll
     for (int i = 0; i < FW; i++) m.v[i] = MCONV(i);
@@ -425,27 +424,27 @@ GRAPE_HD Fp28 from_canonical(const Fp& x) {
 }
 // the same conversion with the 30-bit multiplier only (a third of the instructions): a product, so in
 // (-p, p) instead of canonical
-GRAPE_HD Fp28 from_canonical_lazy(const Fp& x) {
-    Fp28 c;
+GRAPE_HD Fp30 from_canonical_lazy(const Fp& x) {
+    Fp30 c;
 #pragma unroll
     for (int i = 0; i < N; i++) c.v[i] = CIN(i);
     return mul(pack(x), c);
 }
 // value of up to a few p, one lazy operand -> canonical memory form, 32-bit limbs
-GRAPE_HD Fp to_canonical(const Fp28& a) {
-    Fp28 c;
+GRAPE_HD Fp to_canonical(const Fp30& a) {
+    Fp30 c;
 #pragma unroll
     for (int i = 0; i < N; i++) c.v[i] = CMEM(i);
     return unpack(canonical(mul(a, c)));
 }
 
 // a^(p-2) (4-bit fixed windows, rolled loops); a of up to a few p, one lazy operand, a != 0 mod p.
-GRAPE_HD Fp28 inverse(const Fp28& a) {
-    Fp28 tbl[16];
+GRAPE_HD Fp30 inverse(const Fp30& a) {
+    Fp30 tbl[16];
     tbl[0] = one();
     tbl[1] = mul(a, one());
     for (int i = 2; i < 16; i++) tbl[i] = mul(tbl[i - 1], tbl[1]);
-    Fp28 acc = one();
+    Fp30 acc = one();
     bool started = false;
     for (int limb = FW - 1; limb >= 0; limb--) {
         uint32_t e = 0;
@@ -508,10 +507,10 @@ GRAPE_HD void update_de(int32_t* d, int32_t* e, const Mat& t) { divstep::update_
 }  // namespace by
 
 // 1/a in Montgomery form (radix R') for a of up to a few p, one lazy operand, a != 0 mod p; a product.
-GRAPE_HD Fp28 inverse_by(const Fp28& a) {
+GRAPE_HD Fp30 inverse_by(const Fp30& a) {
     using namespace by;
     // canonical integer of a (still carrying the Montgomery factor) in [0, p)
-    const Fp28 t = canonical(mul(a, one()));
+    const Fp30 t = canonical(mul(a, one()));
     int32_t f[L], g[L], d[L], e[L];
 #pragma unroll
     for (int k = 0; k < L; k++) {
@@ -534,7 +533,7 @@ GRAPE_HD Fp28 inverse_by(const Fp28& a) {
     }
     // now g = 0, f = +-1 and d * a = f (mod p): the inverse is d * f, in (-2p, 2p), |limbs| <= 2^30
     const int32_t fneg = f[L - 1] >> 31;          // all-ones when f = -1
-    Fp28 x, r3;
+    Fp30 x, r3;
 #pragma unroll
     for (int k = 0; k < L; k++) {
         x.v[k] = (d[k] ^ fneg) - fneg;            // limb-wise negation when f = -1
@@ -543,7 +542,7 @@ GRAPE_HD Fp28 inverse_by(const Fp28& a) {
     return mul(x, r3);
 }
 
-}  // namespace fp28
+}  // namespace fp30
 
 // ------------------------------------------------------------------------------------------------
 // XYZZ accumulator in the working form.  Invariants between additions: all coordinates balanced, zz below p, zz and zzz
@@ -551,49 +550,49 @@ GRAPE_HD Fp28 inverse_by(const Fp28& a) {
 // |x| < 5.7p (R^2 less PPP and 2Q) and zzz < 1.4p.  `inf` marks the identity.  All of the values below stay under 14 p (BN254: 23 p),
 // all products of them far under 630 p^2 (86000 p^2).
 // ------------------------------------------------------------------------------------------------
-struct Xyzz28 {
-    Fp28 x, y, zz, zzz;
+struct Xyzz30 {
+    Fp30 x, y, zz, zzz;
     bool inf;
 };
-struct Affine28 {   // coordinates in (-p, p), balanced
-    Fp28 x, y;
+struct Affine30 {   // coordinates in (-p, p), balanced
+    Fp30 x, y;
 };
 
-GRAPE_HD Xyzz28 xyzz28_inf() {
-    Xyzz28 r;
-    r.x = fp28::zero();
-    r.y = fp28::zero();
-    r.zz = fp28::zero();
-    r.zzz = fp28::zero();
+GRAPE_HD Xyzz30 xyzz30_inf() {
+    Xyzz30 r;
+    r.x = fp30::zero();
+    r.y = fp30::zero();
+    r.zz = fp30::zero();
+    r.zzz = fp30::zero();
     r.inf = true;
     return r;
 }
 
-GRAPE_HD G1Xyzz xyzz28_to_canonical(const Xyzz28& a) {
+GRAPE_HD G1Xyzz xyzz30_to_canonical(const Xyzz30& a) {
     if (a.inf) return G1Xyzz::inf();
     G1Xyzz r;
-    r.x = fp28::to_canonical(a.x);
-    r.y = fp28::to_canonical(a.y);
-    r.zz = fp28::to_canonical(a.zz);
-    r.zzz = fp28::to_canonical(a.zzz);
+    r.x = fp30::to_canonical(a.x);
+    r.y = fp30::to_canonical(a.y);
+    r.zz = fp30::to_canonical(a.zz);
+    r.zzz = fp30::to_canonical(a.zzz);
     return r;
 }
-GRAPE_HD Xyzz28 xyzz28_from_canonical(const G1Xyzz& a) {
-    Xyzz28 r;
+GRAPE_HD Xyzz30 xyzz30_from_canonical(const G1Xyzz& a) {
+    Xyzz30 r;
     r.inf = a.is_inf();
-    r.x = fp28::from_canonical(a.x);
-    r.y = fp28::from_canonical(a.y);
-    r.zz = fp28::from_canonical(a.zz);
-    r.zzz = fp28::from_canonical(a.zzz);
+    r.x = fp30::from_canonical(a.x);
+    r.y = fp30::from_canonical(a.y);
+    r.zz = fp30::from_canonical(a.zz);
+    r.zzz = fp30::from_canonical(a.zzz);
     return r;
 }
 
 // acc += (negate ? -p : p) for a finite affine point p (the caller skips the identity).
 // Returns false when the addition is one of the exceptional cases (p = +-acc): then acc is left
 // untouched and the caller must take the exact slow path.
-GRAPE_HD bool xyzz28_madd(Xyzz28& acc, const Affine28& p, bool negate) {
-    using namespace fp28;
-    const Fp28 py = cneg(p.y, negate);
+GRAPE_HD bool xyzz30_madd(Xyzz30& acc, const Affine30& p, bool negate) {
+    using namespace fp30;
+    const Fp30 py = cneg(p.y, negate);
     if (acc.inf) {
         acc.x = p.x;
         acc.y = py;
@@ -602,16 +601,16 @@ GRAPE_HD bool xyzz28_madd(Xyzz28& acc, const Affine28& p, bool negate) {
         acc.inf = false;
         return true;
     }
-    const Fp28 Pd = mulb_less(p.x, acc.zz, acc.x);      // U2 - X1
-    const Fp28 R = mulb_less(py, acc.zzz, acc.y);       // S2 - Y1
-    const Fp28 PP = sqr(Pd);
-    const Fp28 ZZ3 = mulb_below_p(acc.zz, PP);
+    const Fp30 Pd = mulb_less(p.x, acc.zz, acc.x);      // U2 - X1
+    const Fp30 R = mulb_less(py, acc.zzz, acc.y);       // S2 - Y1
+    const Fp30 PP = sqr(Pd);
+    const Fp30 ZZ3 = mulb_below_p(acc.zz, PP);
     if (is_zero(ZZ3)) return false;                    // PP = 0  <=>  P = 0: doubling or cancellation
-    const Fp28 PPP = mulb(Pd, PP);
-    const Fp28 Q = mulb(acc.x, PP);
-    const Fp28 X3 = sqr_less(R, PPP, Q);
-    const Fp28 T = balance(sub(Q, X3));
-    const Fp28 Y3 = mul_sub(R, T, acc.y, PPP);
+    const Fp30 PPP = mulb(Pd, PP);
+    const Fp30 Q = mulb(acc.x, PP);
+    const Fp30 X3 = sqr_less(R, PPP, Q);
+    const Fp30 T = balance(sub(Q, X3));
+    const Fp30 Y3 = mul_sub(R, T, acc.y, PPP);
     acc.zzz = mulb(acc.zzz, PPP);
     acc.zz = ZZ3;
     acc.x = X3;
@@ -622,24 +621,24 @@ GRAPE_HD bool xyzz28_madd(Xyzz28& acc, const Affine28& p, bool negate) {
 // acc <- 2 * acc (curve with a = 0, 6M + 3S: U = 2Y, V = U^2, W = U V, S = X V,
 // M = 3 X^2, X3 = M^2 - 2S, Y3 = M (S - X3) - W Y, ZZ3 = V ZZ, ZZZ3 = W ZZZ).  No exceptional case on
 // a group of odd prime order; the identity stays the identity.
-GRAPE_HD void xyzz28_dbl(Xyzz28& acc) {
-    using namespace fp28;
+GRAPE_HD void xyzz30_dbl(Xyzz30& acc) {
+    using namespace fp30;
     if (acc.inf) return;
-    Fp28 U;
+    Fp30 U;
 #pragma unroll
     for (int i = 0; i < N; i++) U.v[i] = 2 * acc.y.v[i];
     U = balance(U);
-    const Fp28 V = sqr(U);
-    const Fp28 Wd = mulb(U, V);
-    const Fp28 S = mulb(acc.x, V);
-    const Fp28 X2 = sqr(acc.x);
-    Fp28 M;
+    const Fp30 V = sqr(U);
+    const Fp30 Wd = mulb(U, V);
+    const Fp30 S = mulb(acc.x, V);
+    const Fp30 X2 = sqr(acc.x);
+    Fp30 M;
 #pragma unroll
     for (int i = 0; i < N; i++) M.v[i] = 3 * X2.v[i];
     M = balance<true>(M);
-    const Fp28 X3 = sqr_less(M, zero(), S);
-    const Fp28 T = balance(sub(S, X3));
-    const Fp28 Y3 = mul_sub(M, T, Wd, acc.y);
+    const Fp30 X3 = sqr_less(M, zero(), S);
+    const Fp30 T = balance(sub(S, X3));
+    const Fp30 Y3 = mul_sub(M, T, Wd, acc.y);
     acc.zz = mulb(V, acc.zz);
     acc.zzz = mulb(Wd, acc.zzz);
     acc.x = X3;
@@ -648,25 +647,25 @@ GRAPE_HD void xyzz28_dbl(Xyzz28& acc) {
 
 // acc += q, both accumulators in the working form (12M + 2S).  Returns false, leaving acc
 // untouched, in the exceptional cases q = +-acc; identities are handled here.
-GRAPE_HD bool xyzz28_add(Xyzz28& acc, const Xyzz28& q) {
-    using namespace fp28;
+GRAPE_HD bool xyzz30_add(Xyzz30& acc, const Xyzz30& q) {
+    using namespace fp30;
     if (q.inf) return true;
     if (acc.inf) {
         acc = q;
         return true;
     }
-    const Fp28 U1 = mulb(acc.x, q.zz);
-    const Fp28 S1 = mulb(acc.y, q.zzz);
-    const Fp28 Pd = mulb_less(q.x, acc.zz, U1);         // U2 - U1
-    const Fp28 R = mulb_less(q.y, acc.zzz, S1);         // S2 - S1
-    const Fp28 PP = sqr(Pd);
-    const Fp28 ZZ3 = mulb_below_p(mulb(acc.zz, q.zz), PP);
+    const Fp30 U1 = mulb(acc.x, q.zz);
+    const Fp30 S1 = mulb(acc.y, q.zzz);
+    const Fp30 Pd = mulb_less(q.x, acc.zz, U1);         // U2 - U1
+    const Fp30 R = mulb_less(q.y, acc.zzz, S1);         // S2 - S1
+    const Fp30 PP = sqr(Pd);
+    const Fp30 ZZ3 = mulb_below_p(mulb(acc.zz, q.zz), PP);
     if (is_zero(ZZ3)) return false;
-    const Fp28 PPP = mulb(Pd, PP);
-    const Fp28 Q = mulb(U1, PP);
-    const Fp28 X3 = sqr_less(R, PPP, Q);
-    const Fp28 T = balance(sub(Q, X3));
-    const Fp28 Y3 = mul_sub(R, T, S1, PPP);
+    const Fp30 PPP = mulb(Pd, PP);
+    const Fp30 Q = mulb(U1, PP);
+    const Fp30 X3 = sqr_less(R, PPP, Q);
+    const Fp30 T = balance(sub(Q, X3));
+    const Fp30 Y3 = mul_sub(R, T, S1, PPP);
     acc.zzz = mulb(mulb(acc.zzz, q.zzz), PPP);
     acc.zz = ZZ3;
     acc.x = X3;
@@ -675,11 +674,11 @@ GRAPE_HD bool xyzz28_add(Xyzz28& acc, const Xyzz28& q) {
 }
 
 // affine image in canonical 32-bit form; the identity maps to (0,0)
-GRAPE_HD G1Affine xyzz28_to_affine(const Xyzz28& a) {
-    using namespace fp28;
+GRAPE_HD G1Affine xyzz30_to_affine(const Xyzz30& a) {
+    using namespace fp30;
     if (a.inf) return G1Affine::inf();
-    const Fp28 zzz_inv = inverse_by(a.zzz);
-    const Fp28 zinv = mul(zzz_inv, a.zz);             // 1/Z
+    const Fp30 zzz_inv = inverse_by(a.zzz);
+    const Fp30 zinv = mul(zzz_inv, a.zz);             // 1/Z
     G1Affine r;
     r.x = to_canonical(mul(a.x, sqr(zinv)));
     r.y = to_canonical(mul(a.y, zzz_inv));
@@ -691,53 +690,53 @@ GRAPE_HD G1Affine xyzz28_to_affine(const Xyzz28& a) {
 // independent additions: table generation).  Inputs are finite points with balanced coordinates in (-p, p).
 // ------------------------------------------------------------------------------------------------
 // a normalised value in [0, 4p) -> the representative in [0, p)
-GRAPE_HD Fp28 fp28_below_p(Fp28 t) {
+GRAPE_HD Fp30 fp30_below_p(Fp30 t) {
 #pragma unroll
     for (int s = 1; s >= 0; s--) {
-        Fp28 d;
+        Fp30 d;
 #pragma unroll
-        for (int i = 0; i < fp28::N; i++) d.v[i] = t.v[i] - (s ? fp28::P2(i) : fp28::P(i));
-        d = fp28::normalize(d);
-        const bool ok = d.v[fp28::N - 1] >= 0;
+        for (int i = 0; i < fp30::N; i++) d.v[i] = t.v[i] - (s ? fp30::P2(i) : fp30::P(i));
+        d = fp30::normalize(d);
+        const bool ok = d.v[fp30::N - 1] >= 0;
 #pragma unroll
-        for (int i = 0; i < fp28::N; i++) t.v[i] = ok ? d.v[i] : t.v[i];
+        for (int i = 0; i < fp30::N; i++) t.v[i] = ok ? d.v[i] : t.v[i];
     }
     return t;
 }
 // denominator of the slope of e + f (x_e - x_f), or of 2 e (2 y_e) when `dbl`; a value congruent
 // to zero means that the sum is no finite affine addition (e = +-f, or a point of order two)
-GRAPE_HD Fp28 affine28_slope_den(const Affine28& e, const Affine28& f, bool dbl) {
-    Fp28 r;
+GRAPE_HD Fp30 affine30_slope_den(const Affine30& e, const Affine30& f, bool dbl) {
+    Fp30 r;
 #pragma unroll
-    for (int i = 0; i < fp28::N; i++) r.v[i] = dbl ? 2 * e.y.v[i] : e.x.v[i] - f.x.v[i];
+    for (int i = 0; i < fp30::N; i++) r.v[i] = dbl ? 2 * e.y.v[i] : e.x.v[i] - f.x.v[i];
     return r;
 }
-// e + f (2 e when `dbl`; then e must equal f) given dinv = 1 / affine28_slope_den(e, f, dbl), a
+// e + f (2 e when `dbl`; then e must equal f) given dinv = 1 / affine30_slope_den(e, f, dbl), a
 // product: 3M + 1S (one more S for the doubling), coordinates in [0, p), normalised
-GRAPE_HD Affine28 affine28_add_given_inverse(const Affine28& e, const Affine28& f, bool dbl, const Fp28& dinv) {
-    using namespace fp28;
-    Fp28 num;
+GRAPE_HD Affine30 affine30_add_given_inverse(const Affine30& e, const Affine30& f, bool dbl, const Fp30& dinv) {
+    using namespace fp30;
+    Fp30 num;
     if (dbl) {
-        const Fp28 xx = sqr(e.x);       // (of f, which a run of additions keeps, the limb products are kept in registers too)
+        const Fp30 xx = sqr(e.x);       // (of f, which a run of additions keeps, the limb products are kept in registers too)
 #pragma unroll
         for (int i = 0; i < N; i++) num.v[i] = 3 * xx.v[i];
         num = balance<true>(num);
     } else {
         num = sub(e.y, f.y);
     }
-    const Fp28 lam = mul(num, dinv);
-    const Fp28 ll = sqr_below_p(lam);
-    Fp28 x3;
+    const Fp30 lam = mul(num, dinv);
+    const Fp30 ll = sqr_below_p(lam);
+    Fp30 x3;
 #pragma unroll
     for (int i = 0; i < N; i++) x3.v[i] = ll.v[i] - e.x.v[i] - f.x.v[i] + P3(i);   // in (0, 4p) for coordinates in [0, p)
-    x3 = fp28_below_p(normalize(x3));
-    const Fp28 ly = mul(lam, balance(sub(e.x, x3)));
-    Fp28 y3;
+    x3 = fp30_below_p(normalize(x3));
+    const Fp30 ly = mul(lam, balance(sub(e.x, x3)));
+    Fp30 y3;
 #pragma unroll
     for (int i = 0; i < N; i++) y3.v[i] = ly.v[i] - e.y.v[i] + P2(i);              // in (0, 3p)
-    Affine28 r;
+    Affine30 r;
     r.x = x3;
-    r.y = fp28_below_p(normalize(y3));
+    r.y = fp30_below_p(normalize(y3));
     return r;
 }
 

@@ -11,9 +11,9 @@
 #define GRAPE_FP_MUL_OUTLINE 1
 #include "common.hpp"
 #include "commit_geometry.hpp"
-#include "fp28.hpp"
+#include "fp30.hpp"
 #include "fr26.hpp"
-#include "quad28.hpp"
+#include "quad30.hpp"
 
 namespace grape {
 
@@ -23,10 +23,10 @@ __device__ __noinline__ Fp fp_mul_outline(Fp a, Fp b) { return mul(a, b); }
 __device__ __noinline__ Fp fp_sqr_outline(Fp a) { return sqr(a); }
 
 // Memory images in 32-bit words: an Fp element is FW words (12 for BLS12-381, 8 for BN254), an
-// affine point 2 FW, a Jacobian point 3 FW, an XYZZ point 4 FW; L28 is the limb count of the
-// working form of fp28.hpp.
+// affine point 2 FW, a Jacobian point 3 FW, an XYZZ point 4 FW; L30 is the limb count of the
+// working form of fp30.hpp.
 constexpr int FW = FpParams::N;
-constexpr int L28 = fp28::N;
+constexpr int L30 = fp30::N;
 
 __device__ __forceinline__ Fp ld_fp(const uint32_t* p) {
     const uint4* q = reinterpret_cast<const uint4*>(p);
@@ -76,61 +76,61 @@ __device__ __forceinline__ Fr ld_fr8(const uint32_t* base, size_t i) {
     return r;
 }
 
-// Wide-table entry: an affine point in the working form, x[L28] then y[L28] as 32-bit
+// Wide-table entry: an affine point in the working form, x[L30] then y[L30] as 32-bit
 // words.  BLS12-381's 104 bytes are padded to 128, so that every gather is exactly one cache line;
 // BN254's 72 bytes are stored in 80 (a multiple of 16 bytes: the loads stay aligned, half of the
 // entries straddle two lines) - the table is 37.5 % smaller, which is what lets 15-bit windows fit
 // the table budget there.
-constexpr int kWideEntryWords = (2 * L28 <= 20) ? 20 : 32;
-static_assert(kWideEntryWords % 4 == 0 && kWideEntryWords >= 2 * L28, "entry layout");
-__device__ __forceinline__ Affine28 ld_entry28(const uint32_t* table, size_t e) {
+constexpr int kWideEntryWords = (2 * L30 <= 20) ? 20 : 32;
+static_assert(kWideEntryWords % 4 == 0 && kWideEntryWords >= 2 * L30, "entry layout");
+__device__ __forceinline__ Affine30 ld_entry30(const uint32_t* table, size_t e) {
     const uint4* q = reinterpret_cast<const uint4*>(table + (size_t)kWideEntryWords * e);
-    uint4 w[(2 * L28 + 3) / 4];
+    uint4 w[(2 * L30 + 3) / 4];
 #pragma unroll
-    for (int i = 0; i < (2 * L28 + 3) / 4; i++) w[i] = q[i];
+    for (int i = 0; i < (2 * L30 + 3) / 4; i++) w[i] = q[i];
     const uint32_t* f = reinterpret_cast<const uint32_t*>(w);
-    Affine28 r;
+    Affine30 r;
 #pragma unroll
-    for (int i = 0; i < L28; i++) {
+    for (int i = 0; i < L30; i++) {
         r.x.v[i] = (int32_t)f[i];
-        r.y.v[i] = (int32_t)f[L28 + i];
+        r.y.v[i] = (int32_t)f[L30 + i];
     }
     return r;
 }
 // coordinates in [0, p), balanced
-__device__ __forceinline__ void st_entry28_raw(uint32_t* table, size_t e, const Affine28& a) {
+__device__ __forceinline__ void st_entry30_raw(uint32_t* table, size_t e, const Affine30& a) {
     uint32_t f[kWideEntryWords];
 #pragma unroll
-    for (int i = 0; i < L28; i++) {
+    for (int i = 0; i < L30; i++) {
         f[i] = (uint32_t)a.x.v[i];
-        f[L28 + i] = (uint32_t)a.y.v[i];
+        f[L30 + i] = (uint32_t)a.y.v[i];
     }
 #pragma unroll
-    for (int i = 2 * L28; i < kWideEntryWords; i++) f[i] = 0;
+    for (int i = 2 * L30; i < kWideEntryWords; i++) f[i] = 0;
     uint4* q = reinterpret_cast<uint4*>(table + (size_t)kWideEntryWords * e);
 #pragma unroll
     for (int i = 0; i < kWideEntryWords / 4; i++) q[i] = make_uint4(f[4 * i], f[4 * i + 1], f[4 * i + 2], f[4 * i + 3]);
 }
-__device__ __forceinline__ void st_entry28(uint32_t* table, size_t e, const G1Affine& a) {
-    st_entry28_raw(table, e, Affine28{fp28::from_canonical(a.x), fp28::from_canonical(a.y)});
+__device__ __forceinline__ void st_entry30(uint32_t* table, size_t e, const G1Affine& a) {
+    st_entry30_raw(table, e, Affine30{fp30::from_canonical(a.x), fp30::from_canonical(a.y)});
 }
-__device__ __forceinline__ bool entry_is_inf(const Affine28& a) {
+__device__ __forceinline__ bool entry_is_inf(const Affine30& a) {
     uint32_t z = 0;
 #pragma unroll
-    for (int i = 0; i < L28; i++) z |= (uint32_t)a.x.v[i] | (uint32_t)a.y.v[i];
+    for (int i = 0; i < L30; i++) z |= (uint32_t)a.x.v[i] | (uint32_t)a.y.v[i];
     return z == 0;
 }
 // Per-lane partial accumulator in memory: x, y, zz, zzz (kCoordWords words each, a multiple of 8 bytes), the identity
 // flag and padding = 64 words (256 bytes).
 using geom::kPartialWords;
-constexpr int kCoordWords = (L28 + 1) & ~1;
+constexpr int kCoordWords = (L30 + 1) & ~1;
 static_assert(4 * kCoordWords + 1 <= kPartialWords && kCoordWords % 2 == 0, "accumulator layout");
-__device__ __forceinline__ void st_partial28(uint32_t* base, size_t i, const Xyzz28& a) {
+__device__ __forceinline__ void st_partial30(uint32_t* base, size_t i, const Xyzz30& a) {
     uint32_t f[kPartialWords];
 #pragma unroll
     for (int k = 0; k < kPartialWords; k++) f[k] = 0;
 #pragma unroll
-    for (int k = 0; k < L28; k++) {
+    for (int k = 0; k < L30; k++) {
         f[k] = (uint32_t)a.x.v[k];
         f[kCoordWords + k] = (uint32_t)a.y.v[k];
         f[2 * kCoordWords + k] = (uint32_t)a.zz.v[k];
@@ -141,15 +141,15 @@ __device__ __forceinline__ void st_partial28(uint32_t* base, size_t i, const Xyz
 #pragma unroll
     for (int k = 0; k < kPartialWords / 4; k++) q[k] = make_uint4(f[4 * k], f[4 * k + 1], f[4 * k + 2], f[4 * k + 3]);
 }
-__device__ __forceinline__ Xyzz28 ld_partial28(const uint32_t* base, size_t i) {
+__device__ __forceinline__ Xyzz30 ld_partial30(const uint32_t* base, size_t i) {
     const uint4* q = reinterpret_cast<const uint4*>(base + geom::partial_word(i));
     uint4 w[kCoordWords + 1];
 #pragma unroll
     for (int k = 0; k < kCoordWords + 1; k++) w[k] = q[k];
     const uint32_t* f = reinterpret_cast<const uint32_t*>(w);
-    Xyzz28 a;
+    Xyzz30 a;
 #pragma unroll
-    for (int k = 0; k < L28; k++) {
+    for (int k = 0; k < L30; k++) {
         a.x.v[k] = (int32_t)f[k];
         a.y.v[k] = (int32_t)f[kCoordWords + k];
         a.zz.v[k] = (int32_t)f[2 * kCoordWords + k];
@@ -159,25 +159,25 @@ __device__ __forceinline__ Xyzz28 ld_partial28(const uint32_t* base, size_t i) {
     return a;
 }
 // acc += q for two accumulators in the working form, exceptional cases through the canonical-form addition
-__device__ __forceinline__ void padd28(Xyzz28& acc, const Xyzz28& q) {
-    if (!xyzz28_add(acc, q)) {
-        G1Xyzz c = xyzz28_to_canonical(acc);
-        xyzz_add(c, xyzz28_to_canonical(q));
-        acc = xyzz28_from_canonical(c);
+__device__ __forceinline__ void padd30(Xyzz30& acc, const Xyzz30& q) {
+    if (!xyzz30_add(acc, q)) {
+        G1Xyzz c = xyzz30_to_canonical(acc);
+        xyzz_add(c, xyzz30_to_canonical(q));
+        acc = xyzz30_from_canonical(c);
     }
 }
 
 // acc += +-entry through the mixed addition of the working form; the rare exceptional step (entry = +-acc)
 // goes through the exact canonical-form addition.
-__device__ __forceinline__ void madd28(Xyzz28& acc, const Affine28& e, bool negate) {
+__device__ __forceinline__ void madd30(Xyzz30& acc, const Affine30& e, bool negate) {
     if (entry_is_inf(e)) return;
-    if (!xyzz28_madd(acc, e, negate)) {
-        G1Xyzz c = xyzz28_to_canonical(acc);
+    if (!xyzz30_madd(acc, e, negate)) {
+        G1Xyzz c = xyzz30_to_canonical(acc);
         G1Affine a;
-        a.x = fp28::to_canonical(e.x);
-        a.y = fp28::to_canonical(e.y);
+        a.x = fp30::to_canonical(e.x);
+        a.y = fp30::to_canonical(e.y);
         xyzz_add_affine(c, a, negate);
-        acc = xyzz28_from_canonical(c);
+        acc = xyzz30_from_canonical(c);
     }
 }
 
@@ -206,7 +206,7 @@ __device__ __forceinline__ uint32_t fr_digit(const Fr& k, uint32_t w, uint32_t c
 // acc += k * G_col through the wide table: one gather and one mixed addition per non-zero digit.
 // While the addition of digit w runs, the table line of digit w+1 is already on its way (one
 // word of it is touched right after the entry of digit w has been requested).  Only the digits w0 .. w1 - 1 are added.
-__device__ __forceinline__ void madd_scalar_fr(Xyzz28& acc, const Fr& k_in, const uint32_t* table, size_t N, uint32_t col,
+__device__ __forceinline__ void madd_scalar_fr(Xyzz30& acc, const Fr& k_in, const uint32_t* table, size_t N, uint32_t col,
                                                uint32_t c, uint32_t nw, uint32_t K, int* err_flag, uint32_t w0 = 0, uint32_t w1 = ~0u) {
     // The scalar is taken as +-|k| with |k| <= (r-1)/2 < 2^254 (r - k and the negated point when k is
     // in the upper half): the top window then never carries out, and nw = ceil(255/c) windows are
@@ -237,12 +237,12 @@ __device__ __forceinline__ void madd_scalar_fr(Xyzz28& acc, const Fr& k_in, cons
             if (mag > K) {
                 *err_flag = 1;
             } else {
-                const Affine28 e = ld_entry28(table, geom::table_entry(w, K, mag, N, col));
+                const Affine30 e = ld_entry30(table, geom::table_entry(w, K, mag, N, col));
                 // unconditional, so that the compiler counts the outstanding loads exactly
                 const size_t nxt = (mag_n != 0 && mag_n <= K) ? geom::table_entry(w + 1, K, mag_n, N, col) : (size_t)col;
                 touch = table[(size_t)kWideEntryWords * nxt];
                 if (kWideEntryWords % 32 != 0) touch |= table[(size_t)kWideEntryWords * nxt + kWideEntryWords - 1];   // dense entries: both lines
-                madd28(acc, e, neg != flip);
+                madd30(acc, e, neg != flip);
             }
         }
         mag = mag_n;
@@ -278,7 +278,7 @@ __device__ __forceinline__ void pdbl(G1Xyzz& acc) { xyzz_dbl(acc); }
 // 1/a for a canonical, non-zero a: through the working form and its divstep inversion (about ten
 // thousand instructions) instead of the a^(p-2) ladder on saturated limbs (about six hundred thousand)
 __device__ __forceinline__ Fp fp_inverse_fast(const Fp& a) {
-    return fp28::to_canonical(fp28::inverse_by(fp28::from_canonical_lazy(a)));
+    return fp30::to_canonical(fp30::inverse_by(fp30::from_canonical_lazy(a)));
 }
 __device__ __forceinline__ G1Affine to_affine(const G1Xyzz& p) {
     if (p.is_inf()) return G1Affine::inf();
@@ -377,7 +377,7 @@ __global__ void __launch_bounds__(64) wide_normalize_kernel(uint32_t* table, con
             inv = fmul(inv, p.zzz);
             a = xyzz_to_affine_with_inv(p, zi);
         }
-        st_entry28(table, (w * K + kidx) * N + i, a);
+        st_entry30(table, (w * K + kidx) * N + i, a);
     }
 }
 
@@ -397,27 +397,27 @@ __global__ void __launch_bounds__(64) wide_normalize_kernel(uint32_t* table, con
 // ------------------------------------------------------------------------------------------------
 constexpr uint32_t kExtendRun = 64;   // additions that share one inversion
 constexpr uint32_t kFirstChain = 16;  // multiples of a base made by the chain of mixed additions before the levels start
-constexpr int kFp28Quads = (L28 + 3) / 4;
-__device__ __forceinline__ Fp28 ld_fp28(const uint32_t* p) {
+constexpr int kFp30Quads = (L30 + 3) / 4;
+__device__ __forceinline__ Fp30 ld_fp30(const uint32_t* p) {
     const uint4* q = reinterpret_cast<const uint4*>(p);
-    uint4 w[kFp28Quads];
+    uint4 w[kFp30Quads];
 #pragma unroll
-    for (int i = 0; i < kFp28Quads; i++) w[i] = q[i];
+    for (int i = 0; i < kFp30Quads; i++) w[i] = q[i];
     const uint32_t* f = reinterpret_cast<const uint32_t*>(w);
-    Fp28 r;
+    Fp30 r;
 #pragma unroll
-    for (int i = 0; i < L28; i++) r.v[i] = (int32_t)f[i];
+    for (int i = 0; i < L30; i++) r.v[i] = (int32_t)f[i];
     return r;
 }
-__device__ __forceinline__ void st_fp28(uint32_t* p, const Fp28& a) {
-    uint32_t f[4 * kFp28Quads];
+__device__ __forceinline__ void st_fp30(uint32_t* p, const Fp30& a) {
+    uint32_t f[4 * kFp30Quads];
 #pragma unroll
-    for (int i = 0; i < 4 * kFp28Quads; i++) f[i] = i < L28 ? (uint32_t)a.v[i] : 0u;
+    for (int i = 0; i < 4 * kFp30Quads; i++) f[i] = i < L30 ? (uint32_t)a.v[i] : 0u;
     uint4* q = reinterpret_cast<uint4*>(p);
 #pragma unroll
-    for (int i = 0; i < kFp28Quads; i++) q[i] = make_uint4(f[4 * i], f[4 * i + 1], f[4 * i + 2], f[4 * i + 3]);
+    for (int i = 0; i < kFp30Quads; i++) q[i] = make_uint4(f[4 * i], f[4 * i + 1], f[4 * i + 2], f[4 * i + 3]);
 }
-static_assert(4 * kFp28Quads <= kWideEntryWords, "a prefix product must fit the entry it is parked in");
+static_assert(4 * kFp30Quads <= kWideEntryWords, "a prefix product must fit the entry it is parked in");
 
 // One thread per (run of `run` consecutive k, window w, generator i); i is the fastest index, so a
 // wave reads and writes adjacent entries.
@@ -433,28 +433,28 @@ __global__ void __launch_bounds__(kBlock, 2) wide_extend_kernel(uint32_t* table,
     const uint32_t k0 = r * run + 1;                              // first k of the run
     const uint32_t k1 = k0 + run < cnt + 1 ? k0 + run : cnt + 1;  // one past its last
     const size_t e0 = w * K * N + i;                              // entry of the multiple k: e0 + (k-1) N
-    const Affine28 f = ld_entry28(table, e0 + (size_t)(have - 1) * N);
+    const Affine30 f = ld_entry30(table, e0 + (size_t)(have - 1) * N);
     bool bad = entry_is_inf(f);
-    Fp28 acc = fp28::one();
+    Fp30 acc = fp30::one();
     for (uint32_t k = k0; k < k1; k++) {
-        const Affine28 e = ld_entry28(table, e0 + (size_t)(k - 1) * N);
+        const Affine30 e = ld_entry30(table, e0 + (size_t)(k - 1) * N);
         bad |= entry_is_inf(e);
-        st_fp28(table + (size_t)kWideEntryWords * (e0 + (size_t)(have + k - 1) * N), acc);
-        acc = fp28::mul(acc, affine28_slope_den(e, f, k == have));
+        st_fp30(table + (size_t)kWideEntryWords * (e0 + (size_t)(have + k - 1) * N), acc);
+        acc = fp30::mul(acc, affine30_slope_den(e, f, k == have));
     }
-    bad |= fp28::is_zero_mod_p(acc);
+    bad |= fp30::is_zero_mod_p(acc);
     if (bad) {
         *degenerate = 1;
         return;
     }
-    Fp28 inv = fp28::inverse_by(acc);
+    Fp30 inv = fp30::inverse_by(acc);
     for (uint32_t k = k1 - 1; k >= k0; k--) {
         const size_t dst = e0 + (size_t)(have + k - 1) * N;
-        const Affine28 e = ld_entry28(table, e0 + (size_t)(k - 1) * N);
-        const Fp28 dinv = fp28::mul(inv, ld_fp28(table + (size_t)kWideEntryWords * dst));
-        inv = fp28::mul(inv, affine28_slope_den(e, f, k == have));
-        const Affine28 sum = affine28_add_given_inverse(e, f, k == have, dinv);
-        st_entry28_raw(table, dst, Affine28{fp28::balance(sum.x), fp28::balance(sum.y)});
+        const Affine30 e = ld_entry30(table, e0 + (size_t)(k - 1) * N);
+        const Fp30 dinv = fp30::mul(inv, ld_fp30(table + (size_t)kWideEntryWords * dst));
+        inv = fp30::mul(inv, affine30_slope_den(e, f, k == have));
+        const Affine30 sum = affine30_add_given_inverse(e, f, k == have, dinv);
+        st_entry30_raw(table, dst, Affine30{fp30::balance(sum.x), fp30::balance(sum.y)});
     }
 }
 
@@ -469,10 +469,10 @@ __global__ void __launch_bounds__(64) wide_extend_exact_kernel(uint32_t* table, 
         const size_t wi = t - (size_t)(k - 1) * per;
         const size_t w = wi / N, i = wi - w * N;
         const size_t e0 = w * K * N + i;
-        Xyzz28 acc = xyzz28_inf();
-        madd28(acc, ld_entry28(table, e0 + (size_t)(k - 1) * N), false);
-        madd28(acc, ld_entry28(table, e0 + (size_t)(have - 1) * N), false);
-        st_entry28(table, e0 + (size_t)(have + k - 1) * N, xyzz28_to_affine(acc));
+        Xyzz30 acc = xyzz30_inf();
+        madd30(acc, ld_entry30(table, e0 + (size_t)(k - 1) * N), false);
+        madd30(acc, ld_entry30(table, e0 + (size_t)(have - 1) * N), false);
+        st_entry30(table, e0 + (size_t)(have + k - 1) * N, xyzz30_to_affine(acc));
     }
 }
 
@@ -485,9 +485,9 @@ __global__ void __launch_bounds__(kBlock) ref_from_wide_kernel(uint32_t* out, co
     const size_t w = t / ns, i = t - w * ns;
     G1Affine a = G1Affine::inf();
     if (w > 0) {
-        const Affine28 e = ld_entry28(wide, (w - 1) * ns + i);
-        a.x = fp28::to_canonical(e.x);
-        a.y = fp28::to_canonical(e.y);
+        const Affine30 e = ld_entry30(wide, (w - 1) * ns + i);
+        a.x = fp30::to_canonical(e.x);
+        a.y = fp30::to_canonical(e.y);
     }
     st_affine(out, w * N + i0 + i, a);
 }
@@ -512,7 +512,7 @@ __global__ void __launch_bounds__(kBlock) commit_wide_kernel(uint32_t* partial, 
     const size_t row = span.row;
     const uint32_t s = span.s, col_end = span.col_end;
     const uint32_t half = 1u << (c - 1), mask = (c == 32) ? 0xffffffffu : ((1u << c) - 1u);
-    Xyzz28 acc = xyzz28_inf();
+    Xyzz30 acc = xyzz30_inf();
     // int path: the scalars of the next two columns are kept in flight (the next one addresses
     // the table line to touch, the one after is being loaded)
     int32_t sc1 = 0, sc2 = 0;
@@ -567,17 +567,17 @@ __global__ void __launch_bounds__(kBlock) commit_wide_kernel(uint32_t* partial, 
                 const uint32_t mag = (uint32_t)(neg ? -d : d);
                 if (mag != 0) {
                     if (mag > K) { *err_flag = 1; continue; }
-                    const Affine28 e = ld_entry28(table, geom::table_entry(w, K, mag, N, col));
+                    const Affine30 e = ld_entry30(table, geom::table_entry(w, K, mag, N, col));
                     touch = *touch_ptr;
                     if (kWideEntryWords % 32 != 0) touch |= touch_ptr[kWideEntryWords - 1];   // dense entries: both lines
-                    madd28(acc, e, neg);
+                    madd30(acc, e, neg);
                 }
             }
             if (v != 0) *err_flag = 1;              // scalar does not fit nw windows
         }
     }
     asm volatile("" ::"v"(touch));                  // keeps the touches alive until here
-    st_partial28(partial, wave * 64 + lane, acc);
+    st_partial30(partial, wave * 64 + lane, acc);
 }
 
 // Scaled table: out[t*ncols + i] = s_t * G_i for a short list of scalars s_t (Montgomery Fr).
@@ -591,9 +591,9 @@ __global__ void __launch_bounds__(kBlock) scaled_chain_kernel(uint32_t* tmp, con
     const size_t tt = tid / ncols;
     const uint32_t col = (uint32_t)(tid - tt * ncols);
     const Fr k = from_mont(ld_fr8(scalars, t0 + tt));
-    Xyzz28 acc = xyzz28_inf();
+    Xyzz30 acc = xyzz30_inf();
     madd_scalar_fr(acc, k, table, N, col, c, nw, K, err_flag);
-    st_xyzz(tmp, tid, xyzz28_to_canonical(acc));
+    st_xyzz(tmp, tid, xyzz30_to_canonical(acc));
 }
 __global__ void __launch_bounds__(64) scaled_normalize_kernel(uint32_t* out, const uint32_t* tmp, size_t e0, size_t n_entries) {
     size_t t0 = (size_t)blockIdx.x * 64 + threadIdx.x;
@@ -622,7 +622,7 @@ __global__ void __launch_bounds__(64) scaled_normalize_kernel(uint32_t* out, con
             inv = fmul(inv, p.zzz);
             a = xyzz_to_affine_with_inv(p, zi);
         }
-        st_entry28(out, e0 + e, a);
+        st_entry30(out, e0 + e, a);
     }
 }
 
@@ -688,7 +688,7 @@ __device__ __forceinline__ int32_t digit_of(const Fr& kb, uint32_t w, uint32_t c
 }
 
 // acc += the windows q J + j, q0 <= q < q1, of k * G_col
-__device__ __forceinline__ void madd_scalar_strided(Xyzz28& acc, const Fr& k_mont, const Fr& H, const uint32_t* table, size_t N, uint32_t col, uint32_t c,
+__device__ __forceinline__ void madd_scalar_strided(Xyzz30& acc, const Fr& k_mont, const Fr& H, const uint32_t* table, size_t N, uint32_t col, uint32_t c,
                                                     uint32_t nw, uint32_t K, uint32_t J, uint32_t j, uint32_t q0, uint32_t q1) {
     bool flip;
     const Fr kb = biased_half_range(k_mont, H, flip);
@@ -701,12 +701,12 @@ __device__ __forceinline__ void madd_scalar_strided(Xyzz28& acc, const Fr& k_mon
         if (d != 0) {
             const bool neg = d < 0;
             const uint32_t mag = (uint32_t)(neg ? -d : d);
-            const Affine28 e = ld_entry28(table, geom::table_entry(q, K, mag, N, col));
+            const Affine30 e = ld_entry30(table, geom::table_entry(q, K, mag, N, col));
             const uint32_t mag_n = (uint32_t)(d_n < 0 ? -d_n : d_n);
             const size_t nxt = mag_n != 0 ? geom::table_entry(q + 1, K, mag_n, N, col) : (size_t)col;
             touch = table[(size_t)kWideEntryWords * nxt];
             if (kWideEntryWords % 32 != 0) touch |= table[(size_t)kWideEntryWords * nxt + kWideEntryWords - 1];
-            madd28(acc, e, neg != flip);
+            madd30(acc, e, neg != flip);
         }
         d = d_n;
     }
@@ -726,10 +726,10 @@ __global__ void __launch_bounds__(kBlock) commit_strided_kernel(uint32_t* partia
     const size_t row = span.row / J;
     const uint32_t j = (uint32_t)(span.row - row * J);
     const Fr H = window_bias(c, nw);                      // wave-uniform
-    Xyzz28 acc = xyzz28_inf();
+    Xyzz30 acc = xyzz30_inf();
     for (uint32_t col = span.s * seg + lane; col < span.col_end; col += 64)
         madd_scalar_strided(acc, ld_fr8(scalars, geom::scalar_index(row, rowlen, col)), H, table, N, col, c, nw, K, J, j, q0, q1);
-    st_partial28(partial, wave * 64 + lane, acc);
+    st_partial30(partial, wave * 64 + lane, acc);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -764,7 +764,7 @@ __global__ void __launch_bounds__(64) commit_sparse_fr_kernel(uint32_t* partial,
     const size_t row = geom::spread_unit(blockIdx.x, gridDim.x, step) * R + grp;
     const bool have_row = row < rows;
     const unsigned long long gmask = (G == 64 ? ~0ull : ((1ull << (G & 63)) - 1ull)) << (grp * G);
-    Xyzz28 acc = xyzz28_inf();
+    Xyzz30 acc = xyzz30_inf();
     uint32_t qn = 0;                                     // queued columns of this lane's row (uniform within the group)
     for (uint32_t base = 0;; base += G) {
         const bool last = base >= rowlen;
@@ -797,7 +797,7 @@ __global__ void __launch_bounds__(64) commit_sparse_fr_kernel(uint32_t* partial,
         }
         if (last) break;
     }
-    if (have_row) st_partial28(partial, row * G + sub, acc);
+    if (have_row) st_partial30(partial, row * G + sub, acc);
 }
 
 // The same through the strided table: one wave per (row, residue) queues the row's live columns and works on them in
@@ -812,7 +812,7 @@ __global__ void __launch_bounds__(64) commit_sparse_strided_kernel(uint32_t* par
     const size_t unit = geom::spread_unit(blockIdx.x, units, step), row = unit / J;
     const uint32_t j = (uint32_t)(unit - row * J);
     const Fr H = window_bias(c, nw);
-    Xyzz28 acc = xyzz28_inf();
+    Xyzz30 acc = xyzz30_inf();
     uint32_t qn = 0;                                     // queued columns (uniform)
     for (uint32_t base = 0;; base += 64) {
         const bool last = base >= rowlen;
@@ -839,13 +839,13 @@ __global__ void __launch_bounds__(64) commit_sparse_strided_kernel(uint32_t* par
         }
         if (last) break;
     }
-    st_partial28(partial, unit * 64 + lane, acc);
+    st_partial30(partial, unit * 64 + lane, acc);
 }
 
 // Row epilogue: the partial sums of a row become one point, the point its affine image.  Three kernels:
 //   commit_reduce_lane_kernel  rows by the ten thousand: one lane per kept partial sum adds its share (88 wave
 //                              instructions per addition, the fewest, but chains of 7 additions at 15 us each)
-//   commit_reduce_quad_kernel  2^lg_qpr quads (quad28.hpp) per row, each adds its share, then a tree of shuffles
+//   commit_reduce_quad_kernel  2^lg_qpr quads (quad30.hpp) per row, each adds its share, then a tree of shuffles
 //                              (140 wave instructions per addition, 4.8 us each)
 //   quad_affine_kernel         the map to affine coordinates, a quad per row
 // geom::reduce_plan picks.  Bound: instruction latency - a SIMD issues hardly faster with two of these waves than with
@@ -864,7 +864,7 @@ __device__ __forceinline__ quad::Acc ld_quad_partial(const uint32_t* base, size_
     const uint32_t* f = reinterpret_cast<const uint32_t*>(w);
     quad::Acc a;
 #pragma unroll
-    for (int k = 0; k < L28; k++) a.v.v[k] = (int32_t)f[k];
+    for (int k = 0; k < L30; k++) a.v.v[k] = (int32_t)f[k];
     a.inf = p[4 * kCoordWords] != 0;
     return a;
 }
@@ -873,7 +873,7 @@ __device__ __forceinline__ void st_quad_partial(uint32_t* base, size_t i, const 
     uint2* q = reinterpret_cast<uint2*>(p + (threadIdx.x & 3) * kCoordWords);
     uint32_t f[kCoordWords];
 #pragma unroll
-    for (int k = 0; k < kCoordWords; k++) f[k] = k < L28 ? (uint32_t)a.v.v[k] : 0u;
+    for (int k = 0; k < kCoordWords; k++) f[k] = k < L30 ? (uint32_t)a.v.v[k] : 0u;
 #pragma unroll
     for (int k = 0; k < kCoordWords / 2; k++) q[k] = make_uint2(f[2 * k], f[2 * k + 1]);
     if ((threadIdx.x & 3) == 0) p[4 * kCoordWords] = a.inf ? 1u : 0u;
@@ -899,7 +899,7 @@ __global__ void __launch_bounds__(kBlock) commit_reduce_quad_kernel(uint32_t* ou
         } else {
             const uint32_t off = (qpr >> 1) >> (step - nserial);
 #pragma unroll
-            for (int k = 0; k < L28; k++) q.v.v[k] = __shfl_down(acc.v.v[k], 4 * off, 64);
+            for (int k = 0; k < L30; k++) q.v.v[k] = __shfl_down(acc.v.v[k], 4 * off, 64);
             q.inf = __shfl_down((int)acc.inf, 4 * off, 64) != 0 || sub + off >= qpr;
         }
         quad::add(acc, q);
@@ -934,9 +934,9 @@ __global__ void __launch_bounds__(kBlock) commit_reduce_lane_kernel(uint32_t* ou
     if (t >= rows * keep) return;
     const size_t row = geom::lane_row(t, keep);
     const uint32_t sub = geom::lane_share(t, keep);
-    Xyzz28 acc = ld_partial28(partial, row * nparts + sub);
-    for (uint32_t j = sub + keep; j < nparts; j += keep) padd28(acc, ld_partial28(partial, row * nparts + j));
-    st_partial28(out, t, acc);
+    Xyzz30 acc = ld_partial30(partial, row * nparts + sub);
+    for (uint32_t j = sub + keep; j < nparts; j += keep) padd30(acc, ld_partial30(partial, row * nparts + j));
+    st_partial30(out, t, acc);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -957,9 +957,9 @@ __global__ void __launch_bounds__(kBlock) msm_multiples_kernel(uint32_t* table, 
     const Fp w = ld_fp(points + 3 * FW * (q / kMsmMultiples) + FW * (r < 2 ? r : 2));     // x, y, z, z
     quad::Acc p;
     p.inf = quad::perm<quad::ctrl(2, 2, 2, 2)>((int32_t)w.is_zero()) != 0;
-    const Fp28 v = fp28::from_canonical_lazy(w);
-    const Fp28 zz = fp28::sqr(v);
-    p.v = quad::select(quad::lanes<0>() | quad::lanes<1>(), v, quad::select(quad::lanes<2>(), zz, fp28::mul(zz, v)));
+    const Fp30 v = fp30::from_canonical_lazy(w);
+    const Fp30 zz = fp30::sqr(v);
+    p.v = quad::select(quad::lanes<0>() | quad::lanes<1>(), v, quad::select(quad::lanes<2>(), zz, fp30::mul(zz, v)));
     quad::Acc acc = p;
     for (int b = 30 - __clz((int)k); b >= 0; b--) {
         quad::dbl(acc);
@@ -993,7 +993,7 @@ __global__ void __launch_bounds__(kBlock) msm_window_kernel(uint32_t* partial, c
         } else {
             const uint32_t off = 8u >> (step - kSerial);
 #pragma unroll
-            for (int k = 0; k < L28; k++) q.v.v[k] = __shfl_down(acc.v.v[k], 4 * off, 64);
+            for (int k = 0; k < L30; k++) q.v.v[k] = __shfl_down(acc.v.v[k], 4 * off, 64);
             q.inf = __shfl_down((int)acc.inf, 4 * off, 64) != 0 || sub + off >= 16;
         }
         quad::add(acc, q);
@@ -1005,7 +1005,7 @@ __global__ void __launch_bounds__(64) quad_canonical_kernel(uint32_t* out, const
     const size_t q = ((size_t)blockIdx.x * 64 + threadIdx.x) >> 2;
     if (q >= n) return;
     const quad::Acc a = ld_quad_partial(sums, q);
-    st_fp(out + 4 * FW * q + FW * (threadIdx.x & 3), a.inf ? Fp::zero() : fp28::to_canonical(a.v));
+    st_fp(out + 4 * FW * q + FW * (threadIdx.x & 3), a.inf ? Fp::zero() : fp30::to_canonical(a.v));
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -1019,7 +1019,7 @@ __global__ void __launch_bounds__(64) quad_canonical_kernel(uint32_t* out, const
 // row, single_commit) and rows too long for a wide table need.
 // ------------------------------------------------------------------------------------------------
 template <bool FR>
-__global__ void __launch_bounds__(kBlock, 2) commit_ref28_kernel(uint32_t* partial, const void* scalars, uint32_t rowlen, size_t rows,
+__global__ void __launch_bounds__(kBlock, 2) commit_ref30_kernel(uint32_t* partial, const void* scalars, uint32_t rowlen, size_t rows,
                                                                  uint32_t seg, uint32_t nseg, const uint32_t* table, size_t npoints) {
     constexpr uint32_t nwin = FR ? 32 : 4;
     const size_t unit = ((size_t)blockIdx.x * kBlock + threadIdx.x) >> 6;      // one wave per unit
@@ -1030,7 +1030,7 @@ __global__ void __launch_bounds__(kBlock, 2) commit_ref28_kernel(uint32_t* parti
     const uint32_t w = (uint32_t)(rw % nwin);
     const size_t row = rw / nwin;
     const uint32_t col_end = (sg + 1) * seg < rowlen ? (sg + 1) * seg : rowlen;
-    Xyzz28 acc = xyzz28_inf();
+    Xyzz30 acc = xyzz30_inf();
     for (uint32_t col = sg * seg + lane; col < col_end; col += 64) {
         uint32_t idx;
         bool neg = false;
@@ -1049,18 +1049,18 @@ __global__ void __launch_bounds__(kBlock, 2) commit_ref28_kernel(uint32_t* parti
         if (idx) {
             const G1Affine a = ld_affine(table, (size_t)idx * npoints + col);
             if (!a.is_inf()) {
-                Affine28 e;
-                e.x = fp28::from_canonical_lazy(a.x);
-                e.y = fp28::from_canonical_lazy(a.y);
-                if (!xyzz28_madd(acc, e, neg)) {           // entry = +-accumulator: exact canonical-form addition
-                    G1Xyzz c = xyzz28_to_canonical(acc);
+                Affine30 e;
+                e.x = fp30::from_canonical_lazy(a.x);
+                e.y = fp30::from_canonical_lazy(a.y);
+                if (!xyzz30_madd(acc, e, neg)) {           // entry = +-accumulator: exact canonical-form addition
+                    G1Xyzz c = xyzz30_to_canonical(acc);
                     xyzz_add_affine(c, a, neg);
-                    acc = xyzz28_from_canonical(c);
+                    acc = xyzz30_from_canonical(c);
                 }
             }
         }
     }
-    st_partial28(partial, unit * 64 + lane, acc);
+    st_partial30(partial, unit * 64 + lane, acc);
 }
 
 __global__ void __launch_bounds__(64) affine_to_jac_kernel(uint32_t* out, const uint32_t* in, size_t n) {
@@ -1218,7 +1218,7 @@ static int commit_ref_impl(uint32_t* out, const void* scalars, size_t size, uint
         const size_t nr = rows - r0 < slab ? rows - r0 : slab;
         const size_t units = nr * nwin * nseg;
         const uint32_t* sc = (const uint32_t*)scalars + r0 * rowlen * elem_words;
-        commit_ref28_kernel<FR><<<blocks_for(units * 64), kBlock, 0, s>>>((uint32_t*)ws, sc, rowlen, nr, seg, nseg, table, npoints);
+        commit_ref30_kernel<FR><<<blocks_for(units * 64), kBlock, 0, s>>>((uint32_t*)ws, sc, rowlen, nr, seg, nseg, table, npoints);
         launch_reduce<false>(sums, (const uint32_t*)ws, nr * nwin, nseg * 64, red_tmp, s);
         quad_horner_kernel<<<blocks_for(nr * 4, 64), 64, 0, s>>>(out + r0 * (size_t)(2 * FW), sums, nr, nwin, 8);
     }

@@ -1,5 +1,5 @@
 // Group operations on four lanes: lane 4q + r of a wave holds coordinate r of an XYZZ accumulator of
-// fp28.hpp (x, y, zz, zzz).
+// fp30.hpp (x, y, zz, zzz).
 //
 // Why: the last steps of a commitment - the row sums, the map to affine coordinates, the one row of an
 // opening - are latency chains, and a lone wave issues an instruction about every 8 cycles here.  One
@@ -11,7 +11,7 @@
 //
 // Every lane of a quad must be active and take the same branch.
 #pragma once
-#include "fp28.hpp"
+#include "fp30.hpp"
 
 namespace grape {
 namespace quad {
@@ -22,10 +22,10 @@ __device__ __forceinline__ int32_t perm(int32_t x) {
     return __builtin_amdgcn_update_dpp(0, x, CTRL, 0xf, 0xf, true);
 }
 template <int CTRL>
-__device__ __forceinline__ Fp28 perm(const Fp28& a) {
-    Fp28 r;
+__device__ __forceinline__ Fp30 perm(const Fp30& a) {
+    Fp30 r;
 #pragma unroll
-    for (int i = 0; i < fp28::N; i++) r.v[i] = perm<CTRL>(a.v[i]);
+    for (int i = 0; i < fp30::N; i++) r.v[i] = perm<CTRL>(a.v[i]);
     return r;
 }
 constexpr int ctrl(int a, int b, int c, int d) { return a | (b << 2) | (c << 4) | (d << 6); }
@@ -40,61 +40,61 @@ __device__ __forceinline__ int32_t lanes() {
     return m;
 }
 __device__ __forceinline__ int32_t select(int32_t mask, int32_t a, int32_t b) { return (a & mask) | (b & ~mask); }
-__device__ __forceinline__ Fp28 select(int32_t mask, const Fp28& a, const Fp28& b) {
-    Fp28 r;
+__device__ __forceinline__ Fp30 select(int32_t mask, const Fp30& a, const Fp30& b) {
+    Fp30 r;
 #pragma unroll
-    for (int i = 0; i < fp28::N; i++) r.v[i] = select(mask, a.v[i], b.v[i]);
+    for (int i = 0; i < fp30::N; i++) r.v[i] = select(mask, a.v[i], b.v[i]);
     return r;
 }
 
 struct Acc {          // one lane's coordinate of a quad's accumulator
-    Fp28 v;           // balanced; values per coordinate as for Xyzz28 (|y| below 2p)
+    Fp30 v;           // balanced; values per coordinate as for Xyzz30 (|y| below 2p)
     bool inf;         // the same in all four lanes
 };
 __device__ __forceinline__ Acc identity() {
     Acc a;
-    a.v = fp28::zero();
+    a.v = fp30::zero();
     a.inf = true;
     return a;
 }
 
-// acc <- 2 acc (the formulas of xyzz28_dbl): three products' time
+// acc <- 2 acc (the formulas of xyzz30_dbl): three products' time
 __device__ __forceinline__ void dbl(Acc& acc) {
-    using namespace fp28;
+    using namespace fp30;
     if (acc.inf) return;
     const int32_t m0 = lanes<0>(), m1 = lanes<1>(), m2 = lanes<2>(), m3 = lanes<3>();
     // lane 0: X^2, lane 1: V = (2Y)^2
-    Fp28 w;
+    Fp30 w;
 #pragma unroll
     for (int i = 0; i < N; i++) w.v[i] = acc.v.v[i] + (acc.v.v[i] & m1);
     w = balance(w);
-    const Fp28 s1 = sqr(w);                                   // lanes 2, 3 unused
-    const Fp28 V = perm<kFrom1>(s1);
-    Fp28 M = perm<kFrom0>(s1);
+    const Fp30 s1 = sqr(w);                                   // lanes 2, 3 unused
+    const Fp30 V = perm<kFrom1>(s1);
+    Fp30 M = perm<kFrom0>(s1);
 #pragma unroll
     for (int i = 0; i < N; i++) M.v[i] = 3 * M.v[i];
     M = balance<true>(M);
     // lane 0: S = X V, lane 1: W = 2Y V, lane 2: ZZ V, lane 3: M^2
-    const Fp28 s2 = mulb(select(m3, M, w), select(m3, M, V));
-    const Fp28 MM = perm<ctrl(3, 3, 3, 3)>(s2);
-    const Fp28 Wd = perm<kFrom1>(s2);
-    Fp28 X3;                                                  // only lane 0's is used
+    const Fp30 s2 = mulb(select(m3, M, w), select(m3, M, V));
+    const Fp30 MM = perm<ctrl(3, 3, 3, 3)>(s2);
+    const Fp30 Wd = perm<kFrom1>(s2);
+    Fp30 X3;                                                  // only lane 0's is used
 #pragma unroll
     for (int i = 0; i < N; i++) X3.v[i] = MM.v[i] - 2 * s2.v[i];
     X3 = balance<true>(X3);
     // lane 0: M (S - X3), lane 1: W Y, lane 3: W ZZZ
-    const Fp28 s3 = mul(select(m0, M, Wd), select(m0, sub(s2, X3), acc.v));      // one lazy operand
-    const Fp28 y0 = perm<kFrom0>(s3);
-    Fp28 y3;
+    const Fp30 s3 = mul(select(m0, M, Wd), select(m0, sub(s2, X3), acc.v));      // one lazy operand
+    const Fp30 y0 = perm<kFrom0>(s3);
+    Fp30 y3;
 #pragma unroll
     for (int i = 0; i < N; i++) y3.v[i] = y0.v[i] - s3.v[i];
     y3 = balance(y3);
     acc.v = select(m0, X3, select(m1, y3, select(m2, s2, s3)));
 }
 
-// acc += q (the formulas of xyzz28_add, every exceptional case included): four products' time
+// acc += q (the formulas of xyzz30_add, every exceptional case included): four products' time
 __device__ __forceinline__ void add(Acc& acc, const Acc& q) {
-    using namespace fp28;
+    using namespace fp30;
     if (q.inf) return;
     if (acc.inf) {
         acc = q;
@@ -102,21 +102,21 @@ __device__ __forceinline__ void add(Acc& acc, const Acc& q) {
     }
     const int32_t m0 = lanes<0>(), m1 = lanes<1>(), m2 = lanes<2>(), m01 = m0 | m1;
     // U1 = X1 ZZ2, S1 = Y1 ZZZ2, U2 = ZZ1 X2, S2 = ZZZ1 Y2
-    const Fp28 t = mulb(acc.v, perm<kCross>(q.v));
-    const Fp28 D = balance(sub(perm<kCross>(t), t));          // lanes 0, 1: P = U2 - U1, R = S2 - S1
+    const Fp30 t = mulb(acc.v, perm<kCross>(q.v));
+    const Fp30 D = balance(sub(perm<kCross>(t), t));          // lanes 0, 1: P = U2 - U1, R = S2 - S1
     // P^2, R^2, ZZ1 ZZ2, ZZZ1 ZZZ2
-    const Fp28 s2 = mulb_below_p(select(m01, D, acc.v), select(m01, D, q.v));
+    const Fp30 s2 = mulb_below_p(select(m01, D, acc.v), select(m01, D, q.v));
     const int zero = is_zero(s2) ? 1 : 0;
     if (perm<kFrom0>(zero)) {                                 // q = +-acc
         if (perm<kFrom1>(zero)) dbl(acc);
         else acc = identity();
         return;
     }
-    const Fp28 PP = perm<kFrom0>(s2);
+    const Fp30 PP = perm<kFrom0>(s2);
     // PPP, Q = U1 PP, ZZ3
-    const Fp28 s3 = mulb(select(m0, D, select(m1, perm<kFrom0>(t), s2)), PP);
-    const Fp28 PPP = perm<kFrom0>(s3);
-    Fp28 X3;                                                  // only lane 1's is used: R^2 - PPP - 2Q
+    const Fp30 s3 = mulb(select(m0, D, select(m1, perm<kFrom0>(t), s2)), PP);
+    const Fp30 PPP = perm<kFrom0>(s3);
+    Fp30 X3;                                                  // only lane 1's is used: R^2 - PPP - 2Q
     int32_t c = 0;
 #pragma unroll
     for (int i = 0; i < N; i++) {                             // balanced as in balance(); a limb may pass 2^31, its half does not
@@ -126,10 +126,10 @@ __device__ __forceinline__ void add(Acc& acc, const Acc& q) {
         c = ((x >> 1) - s3.v[i] + HALF / 2) >> (W - 1);
     }
     // S1 PPP, R (Q - X3), -, ZZZ1 ZZZ2 PPP
-    const Fp28 T = sub(s3, X3);                               // lazy
-    const Fp28 s4 = mul(select(m0, perm<kFrom1>(t), select(m1, D, s2)), select(m1, T, PPP));
-    const Fp28 sp = perm<kFrom0>(s4), x3 = perm<kFrom1>(X3);
-    Fp28 y3;
+    const Fp30 T = sub(s3, X3);                               // lazy
+    const Fp30 s4 = mul(select(m0, perm<kFrom1>(t), select(m1, D, s2)), select(m1, T, PPP));
+    const Fp30 sp = perm<kFrom0>(s4), x3 = perm<kFrom1>(X3);
+    Fp30 y3;
 #pragma unroll
     for (int i = 0; i < N; i++) y3.v[i] = s4.v[i] - (sp.v[i] & m1);
     acc.v = select(m0, x3, select(m2, s3, balance(y3)));
@@ -155,13 +155,13 @@ __device__ __forceinline__ int32_t divsteps30(int32_t delta, int32_t& x1, int32_
 }
 
 // 1/a for the same a in all four lanes (up to a few p, not 0 mod p); a product, the same in all
-// four lanes.  inverse_by of fp28.hpp with one of the vectors f, g, d, e per lane: a batch's update of the
+// four lanes.  inverse_by of fp30.hpp with one of the vectors f, g, d, e per lane: a batch's update of the
 // four vectors is one row of multiply-adds instead of four.
-__device__ __forceinline__ Fp28 inverse_by(const Fp28& a) {
-    using namespace fp28;
-    using namespace fp28::by;
+__device__ __forceinline__ Fp30 inverse_by(const Fp30& a) {
+    using namespace fp30;
+    using namespace fp30::by;
     const int32_t m0 = lanes<0>(), m1 = lanes<1>(), m2 = lanes<2>(), m3 = lanes<3>();
-    const Fp28 t = canonical(fp28::mul(a, one()));            // integer in [0, p), still with the Montgomery factor
+    const Fp30 t = canonical(fp30::mul(a, one()));            // integer in [0, p), still with the Montgomery factor
     int32_t x[L];                                             // lane 0: f, 1: g, 2: d, 3: e
 #pragma unroll
     for (int k = 0; k < L; k++) x[k] = (P30(k) & m0) | (t.v[k] & m1) | (k == 0 ? m3 & 1 : 0);
@@ -195,28 +195,28 @@ __device__ __forceinline__ Fp28 inverse_by(const Fp28& a) {
     }
     // g = 0, f = +-1, d * a = f (mod p): d, in (-2p, p) with limbs below 2^30, to every lane, negated when f = -1
     const int32_t fneg = perm<kFrom0>(x[L - 1]) >> 31;
-    Fp28 out, r3;
+    Fp30 out, r3;
 #pragma unroll
     for (int k = 0; k < L; k++) {
         const int32_t d = perm<ctrl(2, 2, 2, 2)>(x[k]);
         out.v[k] = (d ^ fneg) - fneg;
         r3.v[k] = R3(k);
     }
-    return fp28::mul(out, r3);
+    return fp30::mul(out, r3);
 }
 
 __device__ __forceinline__ void cneg(Acc& a, bool flag) {
     const int32_t m = lanes<1>() & (flag ? -1 : 0);
 #pragma unroll
-    for (int i = 0; i < fp28::N; i++) a.v.v[i] = (a.v.v[i] ^ m) - m;
+    for (int i = 0; i < fp30::N; i++) a.v.v[i] = (a.v.v[i] ^ m) - m;
 }
 
 // affine image in canonical 32-bit form: lane 0 returns x, lane 1 returns y (zero for the identity); lanes 2, 3 nothing of use
 __device__ __forceinline__ Fp to_affine(const Acc& a) {
-    using namespace fp28;
+    using namespace fp30;
     if (a.inf) return Fp::zero();
-    const Fp28 zzz_inv = quad::inverse_by(perm<ctrl(3, 3, 3, 3)>(a.v));
-    const Fp28 zinv = mul(zzz_inv, perm<ctrl(2, 2, 2, 2)>(a.v));      // 1/Z
+    const Fp30 zzz_inv = quad::inverse_by(perm<ctrl(3, 3, 3, 3)>(a.v));
+    const Fp30 zinv = mul(zzz_inv, perm<ctrl(2, 2, 2, 2)>(a.v));      // 1/Z
     return to_canonical(mul(a.v, select(lanes<0>(), sqr(zinv), zzz_inv)));
 }
 

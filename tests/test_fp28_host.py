@@ -1,5 +1,5 @@
 """CPU checks of the lazy Fp arithmetic on 30-bit limbs used by the commitment kernels (host build of
-grape_amd/csrc/fp28.hpp): products, squares, conversions and lazily reduced expressions against
+grape_amd/csrc/fp30.hpp): products, squares, conversions and lazily reduced expressions against
 Python integers; sums of points through its mixed addition against textbook affine
 arithmetic, including the exceptional cases (doubling, cancellation, identity)."""
 import ctypes
@@ -21,7 +21,7 @@ PB = P.bit_length()
 
 @pytest.fixture(scope="module")
 def lib():
-    deps = [SRC] + [os.path.join(HERE, "..", "grape_amd", "csrc", f) for f in ("fp28.hpp", "curve.hpp", "field.hpp")]
+    deps = [SRC] + [os.path.join(HERE, "..", "grape_amd", "csrc", f) for f in ("fp30.hpp", "curve.hpp", "field.hpp")]
     if not os.path.exists(LIB) or any(os.path.getmtime(d) > os.path.getmtime(LIB) for d in deps):
         subprocess.check_call(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wno-unknown-pragmas"]
                               + (["-DGRAPE_CURVE_BN254"] if BN else []) + ["-o", LIB, SRC])

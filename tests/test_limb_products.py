@@ -1,4 +1,4 @@
-"""The field products of the commitment kernels (host build of grape_amd/csrc/fp28.hpp) and of the round kernels (fr26.hpp) on
+"""The field products of the commitment kernels (host build of grape_amd/csrc/fp30.hpp) and of the round kernels (fr26.hpp) on
 operands whose limbs are at the bounds that the columns are laid out for, all signs alike and mixed, against Python
 integers: balanced limbs of +-(2^29 + 2) and one lazy operand of twice that; limbs of 2^30 times 2^27."""
 import ctypes
@@ -20,7 +20,7 @@ EDGE = (1 << 29) + 2
 
 @pytest.fixture(scope="module")
 def lib():
-    deps = [SRC] + [os.path.join(HERE, "..", "grape_amd", "csrc", f) for f in ("fp28.hpp", "fr26.hpp", "divstep.hpp", "curve.hpp", "field.hpp")]
+    deps = [SRC] + [os.path.join(HERE, "..", "grape_amd", "csrc", f) for f in ("fp30.hpp", "fr26.hpp", "divstep.hpp", "curve.hpp", "field.hpp")]
     if not os.path.exists(LIB) or any(os.path.getmtime(d) > os.path.getmtime(LIB) for d in deps):
         subprocess.check_call(["g++", "-O2", "-std=c++17", "-fwrapv", "-fPIC", "-shared", "-Wno-unknown-pragmas"]
                               + (["-DGRAPE_CURVE_BN254"] if BN else []) + ["-o", LIB, SRC])
@@ -48,13 +48,13 @@ def _ptr(a):
 
 
 def _apply(lib, op, a, b, s, u):
-    out = np.zeros(lib.fp28_limbs(), dtype=np.int32)
-    lib.fp28_apply(op, _ptr(a), _ptr(b), _ptr(s), _ptr(u), _ptr(out))
+    out = np.zeros(lib.fp30_limbs(), dtype=np.int32)
+    lib.fp30_apply(op, _ptr(a), _ptr(b), _ptr(s), _ptr(u), _ptr(out))
     return out
 
 
 def test_products_at_the_bounds_of_their_columns(lib):
-    n, rng = lib.fp28_limbs(), random.Random(5)
+    n, rng = lib.fp30_limbs(), random.Random(5)
     rinv = pow(1 << (W * n), -1, P)
     balanced, lazy = _operands(n, EDGE, rng, 12), _operands(n, 2 * EDGE, rng, 6)
     formulas = {0: lambda a, b, s, u: a * b * rinv, 1: lambda a, b, s, u: a * b * rinv, 2: lambda a, b, s, u: a * b * rinv,
@@ -73,7 +73,7 @@ def test_products_at_the_bounds_of_their_columns(lib):
 
 
 def test_carries_and_zero(lib):
-    n, rng = lib.fp28_limbs(), random.Random(6)
+    n, rng = lib.fp30_limbs(), random.Random(6)
     zero = np.zeros(n, dtype=np.int32)
     for op, bound in ((8, (3 << 29) - 1), (11, (1 << 31) - 1)):
         for a in _operands(n, bound, rng, 40):
@@ -93,8 +93,8 @@ def test_carries_and_zero(lib):
             v = (v - d) >> W
         a = np.array(limbs + [v], dtype=np.int32)
         for f in _operands(n, EDGE, rng, 4):
-            assert lib.fp28_zero(_ptr(a), _ptr(f)) == 1
-            assert lib.fp28_zero(_ptr(a + unit), _ptr(f)) == int(_value(f) % P == 0)
+            assert lib.fp30_zero(_ptr(a), _ptr(f)) == 1
+            assert lib.fp30_zero(_ptr(a + unit), _ptr(f)) == int(_value(f) % P == 0)
             c = _apply(lib, 10, a + unit, f, zero, zero)
             assert _value(c) == _value(f) * rinv % P and all(0 <= int(x) < 1 << W for x in c[:-1])
 
