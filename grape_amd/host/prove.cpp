@@ -339,9 +339,10 @@ static Fr eleMul_rounds(fr_t* Aw, fr_t* Bw, const fr_t* A, const fr_t* B, fr_t* 
     // to end) and 1024 x 11008 take 0.82 against 0.96.
     // What is left in B takes a factor per row, made here and uploaded: rows of kCarriedRow elements leave fewer than 512 (2^13 x 257:
     // 0.41-0.43 against 0.45 ms, 2^16 x 257: 1.10 against 1.30), rows of 5 would leave 2^14.
+    // A tensor times itself, bound in place, has one buffer for both folds: its long rounds fail their check, and carried ones would not.
     const uint period = padded ? second_size : 1u << kSplitLow;
     uint carrying = 0;
-    if (period >= kCarriedRow && period <= GRAPE_WROUND_MAX_PERIOD && size / 2 >= 1u << 20)
+    if (Aw != Bw && period >= kCarriedRow && period <= GRAPE_WROUND_MAX_PERIOD && size / 2 >= 1u << 20)
         for (uint n = size; n % 2 == 0 && n / 2 >= kLongRoundPairs && (n / 2) % period == 0; n /= 2) carrying++;
     const CarriedFactors factors(hu - rounds, hv - rounds, rounds, carrying, low);
     std::vector<grape_carried_args> carried;

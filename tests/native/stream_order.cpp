@@ -269,6 +269,22 @@ static void element_products_that_carry() {
     expect(carried(1u << 19, 5) == 0 && carried(1u << 15, 65) == 0 && carried(1u << 14, 255) == 0, "not with shorter rows");
 }
 
+// A tensor times itself, both operands bound in the one buffer: the weighted half would overwrite the plain one, and from the second
+// carried round on nothing compares them.  Two tensors of the same size carry.
+static void a_tensor_times_itself() {
+    const uint rows = 1u << 10, cols = 1u << 11;
+    const std::vector<Fr> point(Log2(rows) + Log2(cols), Fr(3));
+    auto carried = [&](FrTensor& x, FrTensor& y) {
+        const unsigned long before = fake_launched("carried_round_kernel");
+        Fr claim = Fr::zero();
+        prove_eleMul(x, y, 1, rows, cols, point, point, claim);
+        return fake_launched("carried_round_kernel") - before;
+    };
+    FrTensor x(rows * cols), y(rows * cols);
+    expect(carried(x, y) == 5, "two tensors carry");
+    expect(carried(x, x) == 0, "one tensor does not");
+}
+
 // An opening that verifies here: every commitment is the identity (device memory reads as zero), so its two equations are
 // commit_d == 0 and commit_ad == -(c * result) * G.
 static Hyrax_proof trivial_opening(const bn128& G, const Fr& c, uint cols) {
@@ -406,6 +422,7 @@ int main(int argc, char** argv) {
         {"sparse_commitment_table", sparse_commitment_table},
         {"operands_at_any_address", operands_at_any_address},
         {"element_products_that_carry", element_products_that_carry},
+        {"a_tensor_times_itself", a_tensor_times_itself},
         {"verify_with_more_variables", verify_with_more_variables},
         {"verify_with_another_generator", verify_with_another_generator},
         {"blocks_of_two_devices", blocks_of_two_devices},
