@@ -839,11 +839,13 @@ Fr tLookup::run(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax& hyrax
                 Polynomial p2({c3[0], c3[1], c3[2]});
                 return Polynomial::eq(u[ui]) * p0 + p1 - p2 * N_div_D;
             };
+            // a long round after the first is not proved with a weighted term that counts for nothing, whichever kernel summed it
+            const Fr slope = u[ui] * alpha_run;
+            if ((mid_from_claim[k] || (carry && k > 0 && k < carried.size())) && slope.is_zero())
+                throw std::runtime_error("tLookup: a challenge is zero, the round's middle coefficient is not determined by its claim");
             if (mid_from_claim[k]) {
                 // the kernel left a3[1] = 0.  p(0) + p(1) is linear in it with slope eq(u, 1) * alpha_run = u * alpha_run
                 // (only the value at t = 1 of the weighted term contains it), and must equal the claim
-                const Fr slope = u[ui] * alpha_run;
-                if (slope.is_zero()) throw std::runtime_error("tLookup: a challenge is zero, the round's middle coefficient is not determined by its claim");
                 const Polynomial p_without = round_poly();
                 a3[1] = (claim - (p_without(0) + p_without(1))) * slope.inverse();
             }

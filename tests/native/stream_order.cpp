@@ -121,6 +121,32 @@ static void carried_lookups() {
     expect(carried(8, 18) == 0, "as are short proofs");
 }
 
+// A lookup whose alpha is zero proves nothing about A (S + beta) = 1: its long rounds are refused, carried or not.  Nothing is computed
+// here - every sum is zero - so the claim of such a proof holds and the refusal is the rule's.
+static void lookups_without_a_weighted_term() {
+    const uint cols = 64;
+    bn128 G = bn128::one();
+    Hyrax hyrax(1, cols, device_points(256 * cols), G, 1);
+    double seconds = 0;
+    auto refused = [&](uint log_D, Fr alpha) {
+        const uint D = 1u << log_D;
+        struct Lookup : tLookupRange {
+            Lookup(const Fr& a) : tLookupRange(-128, 256) { alpha = a; }
+        } lookup(alpha);
+        FrTensor S(D), A(D);
+        const std::unique_ptr<FrTensor> ints(new FrTensor(D / 8));
+        try {
+            lookup.prove(reinterpret_cast<const int*>(ints->gpu_data), S, A, random_vec(log_D), hyrax, cols, seconds);
+        } catch (const std::exception& e) {
+            return std::string(e.what()).find("a challenge is zero") != std::string::npos;
+        }
+        return false;
+    };
+    expect(refused(18, Fr::zero()), "two weighted long rounds");
+    expect(refused(19, Fr::zero()) && refused(21, Fr::zero()), "carried ones");
+    expect(!refused(10, Fr::zero()), "short rounds are all sums");
+}
+
 // The weights over the high variables are made for the proofs that read them: rounds of more than 2^20 weights and carried ones.
 static void weights_that_are_read() {
     const uint cols = 64, len = 256;
@@ -417,6 +443,7 @@ int main(int argc, char** argv) {
         {"proof_after_a_refused_one", proof_after_a_refused_one},
         {"mapping_objects", mapping_objects},
         {"carried_lookups", carried_lookups},
+        {"lookups_without_a_weighted_term", lookups_without_a_weighted_term},
         {"weights_that_are_read", weights_that_are_read},
         {"tensor_memory_is_idle", tensor_memory_is_idle},
         {"sparse_commitment_table", sparse_commitment_table},
