@@ -262,7 +262,7 @@ static std::map<LKey, std::unique_ptr<tLookupRange>> g_range_lookups;
 // a mapping lookup with its r pinned (the constructor draws r; the table is rebuilt with the given one)
 struct PinnedMapping : tLookupRangeMapping {
     PinnedMapping(int low, uint len, const int* map, const Fr& r_) : tLookupRangeMapping(low, len, map) {
-        r = r_;
+        r = r_in_T_ = r_;
         grape_host::check(grape_tlookup_init((uint32_t*)T.gpu_data, (uint32_t*)B.gpu_data, low, len,
                                              (uint32_t*)grape_host::device_scalar(beta), (uint32_t*)mapped_vals.gpu_data,
                                              (uint32_t*)grape_host::device_scalar(r), nullptr),

@@ -961,6 +961,7 @@ void tLookupRangeMapping::init_from_host(const int* host_table, uint len) {
                              W(grape_host::device_scalar(r)), nullptr),
           "grape_tlookup_init");
     check(grape_stream_sync(nullptr), "sync");
+    r_in_T_ = r;
     grape_free(d_map_int_);
     d_map_int_ = d_int;                   // kept: a witness handed over as integers is checked against it
     have_map_zero_ = low <= 0 && (int64_t)low + (int64_t)len > 0;
@@ -1047,9 +1048,9 @@ Fr tLookupRangeMapping::prove(const int* device_int_S_in, const int* device_int_
         return prove(S_in, S_out, A, v, hyrax, msm_size, commit_time);
     }
     // index and the check S_out = f(S_in) against the integer table in one pass over the integers; A = B[index] and the combined witness
-    // S_in + r * S_out = T[index] are gathered by a long first round, written by the same pass for a short one
+    // S_in + r * S_out = T[index] are gathered by a long first round, written by the same pass for a short one or an r that is not T's
     FrTensor S(D, OnDefaultStream());
-    make_index_from_ints(device_int_S_in, device_int_S_out, D, low, S, A, d_map_int_, &r, first_round_gathers(D));
+    make_index_from_ints(device_int_S_in, device_int_S_out, D, low, S, A, d_map_int_, &r, first_round_gathers(D) && r == r_in_T_);
     index_to_m(D, low);
     Fr ret;
     try {

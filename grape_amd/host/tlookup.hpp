@@ -139,6 +139,9 @@ public:
              uint msm_size, double& commit_time);
     ~tLookupRangeMapping();
 
+protected:
+    Fr r_in_T_;                         // the r that T was made with: a witness is read as T[index] only while r is still that
+
 private:
     void init_from_host(const int* host_table, uint len);
     int* d_map_int_ = nullptr;          // the table's second components as integers (for witnesses handed over as integers)

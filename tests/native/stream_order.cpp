@@ -121,6 +121,34 @@ static void carried_lookups() {
     expect(carried(8, 18) == 0, "as are short proofs");
 }
 
+// A mapping's witness is S_in + r S_out with the r its caller sees: read as T[index] while T was made with it, written out otherwise (the
+// rounds then find that it is not T's).
+static void a_mapping_with_another_r() {
+    const uint cols = 64, log_D = 19, D = 1u << log_D;
+    bn128 G = bn128::one();
+    Hyrax hyrax(1, cols, device_points(256 * cols), G, 1);
+    const std::vector<int> table(256, 7);
+    tLookupRangeMapping lookup(-128, 256, table.data());
+    double seconds = 0;
+    auto written = [&] {
+        FrTensor A(D);
+        const std::unique_ptr<FrTensor> ints(new FrTensor(D / 8));
+        const unsigned long before = fake_launched("index_embed_i32_kernel");
+        const int* x = reinterpret_cast<const int*>(ints->gpu_data);
+        try {
+            lookup.prove(x, x, D, A, random_vec(log_D), hyrax, cols, seconds);
+        } catch (const std::exception&) {                    // nothing is computed here, so its claims do not hold
+        }
+        return fake_launched("index_embed_i32_kernel") - before;
+    };
+    expect(written() == 0, "T's own r");
+    const Fr own = lookup.r;
+    lookup.r = own + Fr::one();
+    expect(written() == 1, "another");
+    lookup.r = own;
+    expect(written() == 0, "T's own again");
+}
+
 // A lookup whose alpha is zero proves nothing about A (S + beta) = 1: its long rounds are refused, carried or not.  Nothing is computed
 // here - every sum is zero - so the claim of such a proof holds and the refusal is the rule's.
 static void lookups_without_a_weighted_term() {
@@ -443,6 +471,7 @@ int main(int argc, char** argv) {
         {"proof_after_a_refused_one", proof_after_a_refused_one},
         {"mapping_objects", mapping_objects},
         {"carried_lookups", carried_lookups},
+        {"a_mapping_with_another_r", a_mapping_with_another_r},
         {"lookups_without_a_weighted_term", lookups_without_a_weighted_term},
         {"weights_that_are_read", weights_that_are_read},
         {"tensor_memory_is_idle", tensor_memory_is_idle},
