@@ -86,6 +86,8 @@ SIGNATURES = {
     "grape_tlookup_hot_select": [c_void_p, c_u32, c_u32, c_u32, c_void_p, c_void_p, ctypes.POINTER(ctypes.c_uint64), c_void_p],
     "grape_tlookup_hot_index": [c_void_p, c_void_p, c_size_t, c_void_p, c_u32, c_void_p],
     "grape_tlookup_hot_coverage": [c_void_p, c_u32, c_void_p, ctypes.POINTER(ctypes.c_uint64), c_void_p],
+    "grape_tlookup_hot_credit": [c_void_p, c_u32, c_void_p, c_void_p, c_u32, ctypes.POINTER(ctypes.c_uint64), c_void_p],
+    "grape_tlookup_hot_extend": [c_void_p, c_void_p, c_u32, c_u32, c_u32, c_u32, c_void_p, c_void_p, ctypes.POINTER(ctypes.c_uint64), c_void_p],
     "grape_fr_mask_cold": [c_void_p, c_void_p, c_void_p, c_size_t, c_void_p],
     "grape_fr_gather": [c_void_p, c_void_p, c_void_p, c_size_t, c_void_p],
     "grape_tlookup_index_i32_nowait": [c_void_p, c_void_p, c_void_p, c_size_t, c_i32, c_u32, c_void_p, c_void_p, c_void_p],

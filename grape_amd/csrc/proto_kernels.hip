@@ -366,14 +366,17 @@ __global__ void __launch_bounds__(kBlock) inverse_by_table_kernel(uint32_t* A, c
 // of the elements ("cold") keep their full-width scalars.  Three small launches: hot entries per tile
 // of 1024, an exclusive scan of the tile counts, slots within every tile.
 constexpr int kHotTile = 1024;          // entries per workgroup: 4 per thread
+// EXTEND: more entries for an assignment that exists.  `weight` is what an entry is chosen by (the counts themselves, or what has
+// been counted over several proofs); entries that hold a slot keep it, the new ones follow from first_slot on.
 // pass 1: hot entries per tile
-__global__ void __launch_bounds__(kBlock) hot_count_kernel(const uint32_t* __restrict__ hist, uint32_t len, uint32_t min_count,
-                                                           uint32_t* __restrict__ tile_count) {
+template <bool EXTEND>
+__global__ void __launch_bounds__(kBlock) hot_count_kernel(const uint32_t* __restrict__ weight, uint32_t len, uint32_t min_count,
+                                                           const int32_t* __restrict__ slot1, uint32_t* __restrict__ tile_count) {
     __shared__ uint32_t wsum[kBlock / 64];
     const uint32_t base = blockIdx.x * kHotTile + threadIdx.x * 4;
     uint32_t mine = 0;
 #pragma unroll
-    for (int k = 0; k < 4; k++) mine += (base + k < len && hist[base + k] >= min_count) ? 1u : 0u;
+    for (int k = 0; k < 4; k++) mine += (base + k < len && weight[base + k] >= min_count && !(EXTEND && slot1[base + k] != 0)) ? 1u : 0u;
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) mine += __shfl_down(mine, off, 64);
     if ((threadIdx.x & 63) == 0) wsum[threadIdx.x >> 6] = mine;
@@ -407,20 +410,23 @@ __global__ void __launch_bounds__(kBlock) hot_scan_kernel(uint32_t* tile_count, 
         info[1] = 0;
     }
 }
-// pass 3: slots in table order; info[1] += witness elements whose entry got none
-__global__ void __launch_bounds__(kBlock) hot_assign_kernel(const uint32_t* __restrict__ hist, uint32_t len, uint32_t min_count,
-                                                            uint32_t max_hot, const uint32_t* __restrict__ tile_base,
-                                                            int32_t* __restrict__ slot1, uint32_t* __restrict__ hot_list,
-                                                            unsigned long long* info) {
+// pass 3: slots in table order; info[1] += witness elements whose entry has none now
+template <bool EXTEND>
+__global__ void __launch_bounds__(kBlock) hot_assign_kernel(const uint32_t* __restrict__ hist, const uint32_t* __restrict__ weight, uint32_t len,
+                                                            uint32_t min_count, uint32_t first_slot, uint32_t max_hot,
+                                                            const uint32_t* __restrict__ tile_base, int32_t* __restrict__ slot1,
+                                                            uint32_t* __restrict__ hot_list, unsigned long long* info) {
     __shared__ uint32_t wsum[kBlock / 64];
     __shared__ unsigned long long wcold[kBlock / 64];
     const uint32_t base = blockIdx.x * kHotTile + threadIdx.x * 4;
-    uint32_t h[4];
+    bool cand[4], held[4];
     uint32_t mine = 0;
 #pragma unroll
     for (int k = 0; k < 4; k++) {
-        h[k] = base + k < len ? hist[base + k] : 0u;
-        mine += (base + k < len && h[k] >= min_count) ? 1u : 0u;
+        const bool in = base + k < len;
+        held[k] = EXTEND && in && slot1[base + k] != 0;
+        cand[k] = in && !held[k] && weight[base + k] >= min_count;
+        mine += cand[k] ? 1u : 0u;
     }
     // exclusive prefix of `mine` over the workgroup: inclusive scan within the wave, then the waves before
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -438,12 +444,11 @@ __global__ void __launch_bounds__(kBlock) hot_assign_kernel(const uint32_t* __re
 #pragma unroll
     for (int k = 0; k < 4; k++) {
         if (base + k >= len) break;
-        const bool cand = h[k] >= min_count;
-        const bool hot = cand && slot < max_hot;
-        slot1[base + k] = hot ? (int32_t)(slot + 1) : 0;
+        const bool hot = cand[k] && slot < max_hot;
+        if (!held[k]) slot1[base + k] = hot ? (int32_t)(first_slot + slot + 1) : 0;
         if (hot) hot_list[slot] = base + k;
-        if (cand) slot++;
-        if (!hot) cold += h[k];
+        if (cand[k]) slot++;
+        if (!hot && !held[k]) cold += hist[base + k];
     }
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) cold += __shfl_down(cold, off, 64);
@@ -452,6 +457,40 @@ __global__ void __launch_bounds__(kBlock) hot_assign_kernel(const uint32_t* __re
     if (threadIdx.x == 0) {
         const unsigned long long c = wcold[0] + wcold[1] + wcold[2] + wcold[3];
         if (c) atomicAdd(&info[1], c);
+    }
+}
+// What a slot assignment made for an earlier witness leaves uncovered in this one: info[0] elements.  CREDIT: the counts of the
+// entries left out are added to what they have been counted before (saturating); those that have reached min_credit hold
+// info[1] of the elements, those that reach it in this witness alone info[2].  One pass over the counts (2^20 entries: 8 and 16 MB).
+template <bool CREDIT>
+__global__ void __launch_bounds__(kBlock) hot_coverage_kernel(const uint32_t* __restrict__ hist, uint32_t len, const int32_t* __restrict__ slot1,
+                                                              uint32_t* __restrict__ credit, uint32_t min_credit, unsigned long long* info) {
+    constexpr int kSums = CREDIT ? 3 : 1;
+    __shared__ unsigned long long part[kSums][kBlock / 64];
+    unsigned long long sums[kSums] = {};
+    for (uint32_t t = blockIdx.x * kBlock + threadIdx.x; t < len; t += gridDim.x * kBlock) {
+        if (slot1[t] != 0) continue;
+        const uint32_t h = hist[t];
+        sums[0] += h;
+        if constexpr (CREDIT) {
+            if (h == 0) continue;
+            const uint32_t before = credit[t], c = before + h < before ? 0xffffffffu : before + h;
+            credit[t] = c;
+            if (c >= min_credit) sums[1] += h;
+            if (h >= min_credit) sums[2] += h;
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < kSums; k++) {
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1) sums[k] += __shfl_xor(sums[k], off, 64);
+        if ((threadIdx.x & 63) == 0) part[k][threadIdx.x >> 6] = sums[k];
+    }
+    __syncthreads();
+    if (threadIdx.x < kSums) {
+        unsigned long long sum = 0;
+        for (int w = 0; w < kBlock / 64; w++) sum += part[threadIdx.x][w];
+        if (sum) atomicAdd(info + threadIdx.x, sum);               // one atomic per workgroup and sum
     }
 }
 // out[i] = slot + 1 of the element's entry (0: cold entry or outside the table)
@@ -1158,47 +1197,60 @@ int grape_tlookup_hot_select(const uint32_t* hist, uint32_t len, uint32_t min_co
     if (rc) return rc;
     unsigned long long* d_info = (unsigned long long*)ws;
     uint32_t* tiles = (uint32_t*)((char*)ws + 64);
-    hot_count_kernel<<<ntiles, kBlock, 0, s>>>(hist, len, min_count, tiles);
+    hot_count_kernel<false><<<ntiles, kBlock, 0, s>>>(hist, len, min_count, nullptr, tiles);
     hot_scan_kernel<<<1, kBlock, 0, s>>>(tiles, ntiles, max_hot, d_info);
-    hot_assign_kernel<<<ntiles, kBlock, 0, s>>>(hist, len, min_count, max_hot, tiles, slot1, hot_list, d_info);
+    hot_assign_kernel<false><<<ntiles, kBlock, 0, s>>>(hist, hist, len, min_count, 0, max_hot, tiles, slot1, hot_list, d_info);
+    GRAPE_LAUNCH_CHECK();
+    GRAPE_HIP_CHECK(hipMemcpyAsync(info, d_info, 2 * sizeof(uint64_t), hipMemcpyDeviceToHost, s));
+    GRAPE_HIP_CHECK(hipStreamSynchronize(s));
+    return GRAPE_OK;
+}
+int grape_tlookup_hot_extend(const uint32_t* hist, const uint32_t* credit, uint32_t len, uint32_t min_credit, uint32_t first_slot, uint32_t max_new,
+                             int32_t* slot1, uint32_t* hot_list, uint64_t* info, grape_stream_t st) {
+    GRAPE_REQUIRE(hist != nullptr && credit != nullptr && slot1 != nullptr && hot_list != nullptr && info != nullptr && len > 0, "bad arguments");
+    GRAPE_REQUIRE(min_credit >= 1, "min_credit must be at least 1");
+    GRAPE_REQUIRE((uint64_t)first_slot + max_new < (1u << 31), "too many slots");
+    hipStream_t s = as_stream(st);
+    const uint32_t ntiles = (len + kHotTile - 1) / kHotTile;
+    void* ws;
+    int rc = scratch_get(kSlotMisc, 64 + sizeof(uint32_t) * (size_t)ntiles, &ws, s);
+    if (rc) return rc;
+    unsigned long long* d_info = (unsigned long long*)ws;
+    uint32_t* tiles = (uint32_t*)((char*)ws + 64);
+    hot_count_kernel<true><<<ntiles, kBlock, 0, s>>>(credit, len, min_credit, slot1, tiles);
+    hot_scan_kernel<<<1, kBlock, 0, s>>>(tiles, ntiles, max_new, d_info);
+    hot_assign_kernel<true><<<ntiles, kBlock, 0, s>>>(hist, credit, len, min_credit, first_slot, max_new, tiles, slot1, hot_list, d_info);
     GRAPE_LAUNCH_CHECK();
     GRAPE_HIP_CHECK(hipMemcpyAsync(info, d_info, 2 * sizeof(uint64_t), hipMemcpyDeviceToHost, s));
     GRAPE_HIP_CHECK(hipStreamSynchronize(s));
     return GRAPE_OK;
 }
 
-// what a slot assignment made for an earlier witness leaves uncovered in this one
-__global__ void __launch_bounds__(kBlock) hot_coverage_kernel(const uint32_t* __restrict__ hist, uint32_t len, const int32_t* __restrict__ slot1,
-                                                              unsigned long long* info) {
-    __shared__ unsigned long long part[kBlock / 64];
-    unsigned long long cold = 0;
-    for (uint32_t t = blockIdx.x * kBlock + threadIdx.x; t < len; t += gridDim.x * kBlock)
-        if (slot1[t] == 0) cold += hist[t];
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) cold += __shfl_xor(cold, off, 64);
-    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = cold;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        unsigned long long sum = 0;
-        for (int w = 0; w < kBlock / 64; w++) sum += part[w];
-        if (sum) atomicAdd(info, sum);               // one atomic per workgroup
-    }
-}
-int grape_tlookup_hot_coverage(const uint32_t* hist, uint32_t len, const int32_t* slot1, uint64_t* cold_elements, grape_stream_t st) {
-    GRAPE_REQUIRE(hist != nullptr && slot1 != nullptr && cold_elements != nullptr && len > 0, "bad arguments");
+static int hot_coverage(const uint32_t* hist, uint32_t len, const int32_t* slot1, uint32_t* credit, uint32_t min_credit, uint64_t* info,
+                        grape_stream_t st) {
     hipStream_t s = as_stream(st);
     void* ws;
     int rc = scratch_get(kSlotMisc, 64, &ws, s);
     if (rc) return rc;
-    rc = zero_fill(ws, 8, s);
+    rc = zero_fill(ws, 32, s);
     if (rc) return rc;
     unsigned nb = blocks_for(len);
     if (nb > 256) nb = 256;
-    hot_coverage_kernel<<<nb, kBlock, 0, s>>>(hist, len, slot1, (unsigned long long*)ws);
+    if (credit) hot_coverage_kernel<true><<<nb, kBlock, 0, s>>>(hist, len, slot1, credit, min_credit, (unsigned long long*)ws);
+    else hot_coverage_kernel<false><<<nb, kBlock, 0, s>>>(hist, len, slot1, nullptr, 0, (unsigned long long*)ws);
     GRAPE_LAUNCH_CHECK();
-    GRAPE_HIP_CHECK(hipMemcpyAsync(cold_elements, ws, sizeof(uint64_t), hipMemcpyDeviceToHost, s));
+    GRAPE_HIP_CHECK(hipMemcpyAsync(info, ws, sizeof(uint64_t) * (credit ? 3 : 1), hipMemcpyDeviceToHost, s));
     GRAPE_HIP_CHECK(hipStreamSynchronize(s));
     return GRAPE_OK;
+}
+int grape_tlookup_hot_coverage(const uint32_t* hist, uint32_t len, const int32_t* slot1, uint64_t* cold_elements, grape_stream_t st) {
+    GRAPE_REQUIRE(hist != nullptr && slot1 != nullptr && cold_elements != nullptr && len > 0, "bad arguments");
+    return hot_coverage(hist, len, slot1, nullptr, 0, cold_elements, st);
+}
+int grape_tlookup_hot_credit(const uint32_t* hist, uint32_t len, const int32_t* slot1, uint32_t* credit, uint32_t min_credit, uint64_t* info,
+                             grape_stream_t st) {
+    GRAPE_REQUIRE(hist != nullptr && slot1 != nullptr && credit != nullptr && info != nullptr && len > 0, "bad arguments");
+    return hot_coverage(hist, len, slot1, credit, min_credit, info, st);
 }
 
 int grape_tlookup_hot_index(int32_t* out, const int32_t* idx1, size_t n, const int32_t* slot1, uint32_t len, grape_stream_t st) {

@@ -44,16 +44,23 @@ Hyrax::Hyrax(uint layer_num_, uint npoints_, affine_t* g, bn128& G_, uint com_sc
         if (end != e) table_budget_ = (size_t)gib << 30;
     }
 }
-// scaled tables handed out: table -> (the Hyrax object whose budget holds it, bytes).  Never
+// scaled tables handed out: table -> the Hyrax object whose budget holds it, its bytes, whether it has been extended.  Never
 // destroyed: lookup objects with static lifetime release their tables while the process exits.
-static std::map<const void*, std::pair<Hyrax*, size_t>>& scaled_registry() {
-    static auto* r = new std::map<const void*, std::pair<Hyrax*, size_t>>();
+namespace {
+struct ScaledTable {
+    Hyrax* owner = nullptr;
+    size_t bytes = 0;
+    bool extended = false;
+};
+}  // namespace
+static std::map<const void*, ScaledTable>& scaled_registry() {
+    static auto* r = new std::map<const void*, ScaledTable>();
     return *r;
 }
 
 Hyrax::~Hyrax() {
     for (auto& e : scaled_registry())
-        if (e.second.first == this) e.second.first = nullptr;
+        if (e.second.owner == this) e.second.owner = nullptr;
     grape_free(int16_table_.d);
     grape_free(int16x2_table_.d);
     grape_free(int32_table_.d);
@@ -325,19 +332,55 @@ affine_t* Hyrax::build_scaled_table(const FrTensor& scalars, uint ncols) {
     if (!make_room(bytes, 0)) return nullptr;
     affine_t* out = nullptr;
     check(grape_malloc((void**)&out, bytes), "grape_malloc");
+    gen_scaled(out, scalars, ncols);
+    scaled_bytes_ += bytes;
+    scaled_registry()[out] = ScaledTable{this, bytes, false};
+    return out;
+}
+
+void Hyrax::gen_scaled(affine_t* out, const FrTensor& scalars, uint ncols) {
     check(grape_g1_scaled_table_gen(W(out), W(scalars.gpu_data), scalars.size, ncols, W(fr_table_.d), fr_table_.ngen, fr_table_.c,
                                     fr_table_.nw, fr_table_.K, nullptr),
           "grape_g1_scaled_table_gen");
-    scaled_bytes_ += bytes;
-    scaled_registry()[out] = std::make_pair(this, bytes);
-    return out;
+}
+
+size_t Hyrax::most_scaled_rows(const affine_t* table, uint ncols) const {
+    size_t share = table_budget_ / 8;
+    for (const auto& e : scaled_registry())
+        if (e.second.owner == this && e.second.extended && e.first != table) share -= std::min(share, e.second.bytes);
+    return share / grape_g1_wide_table_bytes(ncols, 1, 1);
+}
+
+bool Hyrax::extend_scaled_table(affine_t*& table, uint rows, uint& capacity, const FrTensor& more, uint ncols) {
+    auto it = scaled_registry().find(table);
+    if (it == scaled_registry().end() || it->second.owner != this) return false;
+    const size_t row_bytes = grape_g1_wide_table_bytes(ncols, 1, 1), need = (size_t)rows + more.size, most = most_scaled_rows(table, ncols);
+    if (need > most || !ensure_fr_table(ncols)) return false;
+    if (need > capacity) {
+        // with room for twice as many where the share allows it: the rows are copied (4.7 TB/s) a bounded number of times
+        const size_t room = std::max(need, std::min(most, 2 * (size_t)capacity)), bytes = room * row_bytes;
+        if (!make_room(bytes, it->second.bytes)) return false;
+        affine_t* out = nullptr;
+        const int rc = grape_malloc((void**)&out, bytes);
+        if (rc == GRAPE_ENOMEM) return false;
+        check(rc, "grape_malloc");
+        check(grape_memcpy_d2d(out, table, (size_t)rows * row_bytes, nullptr), "grape_memcpy_d2d");
+        release_scaled_table(table);
+        scaled_bytes_ += bytes;
+        it = scaled_registry().emplace(out, ScaledTable{this, bytes, false}).first;
+        table = out;
+        capacity = (uint)room;
+    }
+    it->second.extended = true;
+    gen_scaled(reinterpret_cast<affine_t*>(reinterpret_cast<char*>(table) + (size_t)rows * row_bytes), more, ncols);
+    return true;
 }
 
 void Hyrax::release_scaled_table(affine_t* table) {
     if (!table) return;
     auto it = scaled_registry().find(table);
     if (it != scaled_registry().end()) {
-        if (it->second.first) it->second.first->scaled_bytes_ -= it->second.second;
+        if (it->second.owner) it->second.owner->scaled_bytes_ -= it->second.bytes;
         scaled_registry().erase(it);
     }
     grape_free(table);
@@ -345,7 +388,7 @@ void Hyrax::release_scaled_table(affine_t* table) {
 
 bool Hyrax::owns_scaled_table(const affine_t* table) const {
     auto it = scaled_registry().find(table);
-    return it != scaled_registry().end() && it->second.first == this;
+    return it != scaled_registry().end() && it->second.owner == this;
 }
 
 affine_t* Hyrax::commit_indexed_affine(int* idx_plus1, uint size, uint N, affine_t* scaled_table, uint ncols, uint len, int* d_flag) {

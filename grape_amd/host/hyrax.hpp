@@ -74,6 +74,13 @@ public:
     // not there yet, so that table_bytes_free() afterwards is what a scaled table may really take; false when
     // it does not fit the budget (build_scaled_table would return nullptr).
     bool prepare_scaled_tables(uint ncols);
+    // Puts the rows of `more` behind the `rows` rows of a scaled table over ncols generators that has room for `capacity`: in
+    // place while they fit, else a copy with room for up to twice as many takes its place first (the old one is freed).
+    // False, and the table as it was, where that does not fit the budget, the share of it that tables may grow into
+    // (an eighth, 16 GiB by default, so that growing rows do not keep out the tables of later proofs) or the device's memory.
+    bool extend_scaled_table(affine_t*& table, uint rows, uint& capacity, const FrTensor& more, uint ncols);
+    // scalars that such a table may hold in the end
+    size_t most_scaled_rows(const affine_t* table, uint ncols) const;
     // frees a table that build_scaled_table returned and gives its bytes back to the budget of the
     // Hyrax object that built it, if that object still exists
     static void release_scaled_table(affine_t* table);
@@ -128,6 +135,7 @@ private:
     StridedTable fr_strided_;
     bool int16_ok_ = true;
     size_t scaled_bytes_ = 0;
+    void gen_scaled(affine_t* out, const FrTensor& scalars, uint ncols);
     std::vector<Fr> last_open_point_;
     std::unique_ptr<G1FixedBase> G_multiples_;      // built by the first opening or verification
     bn128 G_multiples_of_;

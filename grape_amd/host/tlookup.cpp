@@ -28,6 +28,7 @@ tLookup::~tLookup() {
     Hyrax::release_scaled_table(scaled_table_);
     Hyrax::release_scaled_table(hot_table_);
     grape_free(hot_slot1_);
+    grape_free(hot_credit_);
     grape_free(d_idx_);
 }
 
@@ -132,38 +133,120 @@ void tLookup::gather_by_index(FrTensor& out, const FrTensor& table, uint D) {
 
 // com(A) through the entries that occur often (A: nullptr when it has not been written out).  A[i] = B[index_i]; an entry t that occurs n_t times
 // costs n_t full-width scalars (16 to 20 additions each) on the plain path, or one row B[t]*G_i of
-// the scaled table (rowlen entries at 20 additions and a normalisation each, built for this proof
-// only) plus n_t single additions.  So an entry is worth a row when n_t exceeds rowlen by a factor
-// somewhat above one; 1.8 is taken (the proof's time is flat from 1.2 to 2.2), and with the
-// activations of a transformer layer nearly all elements sit on such entries.  Elements of the
+// the scaled table (rowlen entries at 20 additions and a normalisation each) plus n_t single additions.  So an entry is worth a row
+// when n_t exceeds rowlen by a factor somewhat above one; 1.8 is taken (the first proof's time is flat from 1.2 to 2.2).  Elements of the
 // other entries keep their scalars and are committed on the plain path; the two sums are added.
 // Returns false (nothing committed) when no entry qualifies or the table does not fit.
 void tLookup::drop_hot_rows() {
     Hyrax::release_scaled_table(hot_table_);
     grape_free(hot_slot1_);
+    grape_free(hot_credit_);
     hot_table_ = nullptr;
     hot_slot1_ = nullptr;
-    hot_rows_ = hot_cols_ = 0;
+    hot_credit_ = nullptr;
+    hot_rows_ = hot_cols_ = hot_capacity_ = 0;
+    hot_missed_ = 0;
     hot_for_ = nullptr;
+}
+
+namespace {
+// a full-width scalar's additions beyond the one through a row, and the additions a row's entry takes to build
+constexpr double kColdAdditions = 19.0, kRowAdditions = 23.0;
+// A growing step costs some 0.3 ms of its own - synchronisations, allocations, at times a copy of the rows.  The entries that
+// are due hold this many elements of a witness when their rows save that in each proof (2.4 to 4.1 ns an element).
+constexpr uint64_t kDueElements = 1u << 17;
+uint hot_threshold(uint rowlen) { return (uint)(1.8 * rowlen) + 1; }
+}  // namespace
+
+// Rows for entries that keep coming back.  Whether a witness repeats is not known in advance, so an entry without a row pays for
+// its elements proof by proof until what it has paid is what its row costs - its occurrences since the object's first proof reach the
+// count that earns a row within one proof - and gets the row then: at most twice what the better choice would have cost, however
+// long the object lives.  A proof builds no more rows than cost what its cold elements cost, so none takes longer than twice its time.
+// SiLU of 2048 x 11008 activations, sigma 4096 (20 000 entries of 200 to 2200 occurrences, 7 of which earn a row in one proof): 56.5 ms a
+// proof; with growing rows the object's proofs take 56 (4th), 94, 62, 43, 37, 29, 31, 28, 26 ... 12 ms (40th).  The exponential of
+// 2^27 scores, sigma 181: 29.5 to 27.5 ms.
+// info: what grape_tlookup_hot_credit has said of this witness.  Returns the elements that the rows leave out.
+uint64_t tLookup::grow_hot_rows(Hyrax& hyrax, const uint64_t info[3]) {
+    const uint N = T.size, due_at = hot_threshold(hot_cols_);
+    const uint64_t cold = info[0];
+    const size_t most = hyrax.most_scaled_rows(hot_table_, hot_cols_);
+    const size_t room = most > hot_rows_ ? most - hot_rows_ : 0;
+    const size_t max_new = std::min({room, (size_t)N, (size_t)(cold * kColdAdditions / (kRowAdditions * hot_cols_))});
+    if (room == 0) hot_missed_ += (double)info[1];
+    if (max_new == 0) return cold;
+    // the new slots are given on a copy: they count once their rows are there
+    uint32_t* d_list = nullptr;
+    int* slots = nullptr;
+    uint64_t left = cold;
+    try {
+        check(grape_malloc_on_default((void**)&d_list, sizeof(uint32_t) * (size_t)N), "grape_malloc");
+        check(grape_malloc((void**)&slots, sizeof(int) * (size_t)N), "grape_malloc");
+        check(grape_memcpy_d2d(slots, hot_slot1_, sizeof(int) * (size_t)N, nullptr), "grape_memcpy_d2d");
+        uint64_t given[2] = {0, 0};
+        check(grape_tlookup_hot_extend(d_hist_, hot_credit_, N, due_at, hot_rows_, (uint32_t)max_new, slots, d_list, given, nullptr),
+              "grape_tlookup_hot_extend");
+        const uint n_new = (uint)given[0];
+        if (n_new != 0) {
+            FrTensor more(n_new, OnDefaultStream());
+            check(grape_fr_gather(W(more.gpu_data), W(B.gpu_data), d_list, n_new, nullptr), "grape_fr_gather");
+            bool built;
+            if (hot_table_) {
+                built = hyrax.extend_scaled_table(hot_table_, hot_rows_, hot_capacity_, more, hot_cols_);
+            } else {
+                hot_table_ = hyrax.build_scaled_table(more, hot_cols_);
+                built = hot_table_ != nullptr;
+                hot_capacity_ = built ? n_new : 0;
+            }
+            if (built) {
+                hot_rows_ += n_new;
+                std::swap(slots, hot_slot1_);
+                left = given[1];
+            } else {
+                hot_missed_ += (double)(cold - given[1]);
+            }
+        }
+    } catch (...) {
+        grape_stream_sync(nullptr);
+        grape_free_on_default(d_list);
+        grape_free(slots);
+        drop_hot_rows();
+        throw;
+    }
+    grape_free_on_default(d_list);
+    grape_free(slots);
+    return left;
 }
 
 bool tLookup::commit_A_by_occupancy(FrTensor* A, uint D, uint msm_size, Hyrax& hyrax) {
     const uint N = T.size;
     const uint rowlen = msm_size * hyrax.com_scale;
     const uint rows = D / rowlen;
-    const uint min_count = hot_min_count_ ? hot_min_count_ : (uint)(1.8 * rowlen) + 1;
+    const uint min_count = hot_min_count_ ? hot_min_count_ : hot_threshold(rowlen);
     hot_reused_ = false;
     uint64_t cold = 0;
-    // rows kept from an earlier proof: used again when the elements they leave out (20 additions
-    // each instead of one) cost less than building rows anew (rowlen entries of 20 additions and a
-    // normalisation per row)
-    if (hot_table_ && (hot_for_ != &hyrax || hot_cols_ != rowlen || !hyrax.owns_scaled_table(hot_table_))) drop_hot_rows();
-    if (hot_table_ && hot_min_count_ == 0) {
-        check(grape_tlookup_hot_coverage(d_hist_, N, hot_slot1_, &cold, nullptr), "grape_tlookup_hot_coverage");
-        if ((double)cold * 19.0 <= (double)hot_rows_ * rowlen * 23.0) hot_reused_ = true;
-    }
-    if (!hot_reused_) {
+    if (hot_slot1_ && (hot_min_count_ != 0 || hot_for_ != &hyrax || hot_cols_ != rowlen || (hot_table_ && !hyrax.owns_scaled_table(hot_table_))))
         drop_hot_rows();
+    if (hot_slot1_) {
+        if (!hot_credit_) {
+            check(grape_malloc((void**)&hot_credit_, sizeof(uint32_t) * (size_t)N), "grape_malloc");
+            check(grape_memset_zero(hot_credit_, sizeof(uint32_t) * (size_t)N, nullptr), "grape_memset_zero");
+        }
+        uint64_t info[3] = {0, 0, 0};
+        check(grape_tlookup_hot_credit(d_hist_, N, hot_slot1_, hot_credit_, min_count, info, nullptr), "grape_tlookup_hot_credit");
+        cold = info[0];
+        // rows kept from earlier proofs: used again, with more of them where entries are due, unless the elements that new rows would
+        // take in (20 additions each instead of one) cost more than building all rows anew (rowlen entries of 20 additions and
+        // a normalisation per row).  Where there is no room for more rows, what the entries that were due have missed counts as well.
+        const double anew = (double)hot_rows_ * rowlen * kRowAdditions;
+        if (info[1] >= kDueElements && hot_missed_ * kColdAdditions <= anew) {
+            hot_reused_ = hot_table_ != nullptr;
+            cold = grow_hot_rows(hyrax, info);
+        } else if (hot_table_) {
+            hot_reused_ = std::max((double)info[2], hot_missed_) * kColdAdditions <= anew;
+            if (!hot_reused_) drop_hot_rows();
+        }
+    }
+    if (!hot_table_) {
         const size_t row_bytes = grape_g1_wide_table_bytes(rowlen, 1, 1);
         // the per-window table the rows are built through comes first: it takes its share of the budget
         if (!hyrax.prepare_scaled_tables(rowlen)) return false;
@@ -172,7 +255,7 @@ bool tLookup::commit_A_by_occupancy(FrTensor* A, uint D, uint msm_size, Hyrax& h
         if (max_hot == 0) return false;
         uint32_t* d_list = nullptr;
         try {
-            check(grape_malloc((void**)&hot_slot1_, sizeof(int) * (size_t)N), "grape_malloc");
+            if (!hot_slot1_) check(grape_malloc((void**)&hot_slot1_, sizeof(int) * (size_t)N), "grape_malloc");
             check(grape_malloc_on_default((void**)&d_list, sizeof(uint32_t) * (size_t)N), "grape_malloc");
             uint64_t info[2] = {0, 0};
             check(grape_tlookup_hot_select(d_hist_, N, min_count, (uint32_t)max_hot, hot_slot1_, d_list, info, nullptr), "grape_tlookup_hot_select");
@@ -182,8 +265,9 @@ bool tLookup::commit_A_by_occupancy(FrTensor* A, uint D, uint msm_size, Hyrax& h
                 FrTensor Bhot(n_hot, OnDefaultStream());
                 check(grape_fr_gather(W(Bhot.gpu_data), W(B.gpu_data), d_list, n_hot, nullptr), "grape_fr_gather");
                 hot_table_ = hyrax.build_scaled_table(Bhot, rowlen);
+                if (!hot_table_) check(grape_memset_zero(hot_slot1_, sizeof(int) * (size_t)N, nullptr), "grape_memset_zero");
             }
-            hot_rows_ = n_hot;
+            hot_rows_ = hot_capacity_ = hot_table_ ? n_hot : 0;
             hot_cols_ = rowlen;
             hot_for_ = &hyrax;
         } catch (...) {
@@ -194,7 +278,8 @@ bool tLookup::commit_A_by_occupancy(FrTensor* A, uint D, uint msm_size, Hyrax& h
         }
         grape_free_on_default(d_list);
         if (!hot_table_) {
-            drop_hot_rows();
+            // nothing has earned a row yet: the slots (none given) and what the entries have paid so far are kept
+            if (hot_min_count_ != 0) drop_hot_rows();
             return false;
         }
     }

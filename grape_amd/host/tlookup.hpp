@@ -38,7 +38,8 @@ public:
     // Where no table over every entry fits (mapping lookups), A is committed through a table of
     // the entries that occur at least `n` times in the witness (0 = the break-even count, 1.8 times
     // the row length), built by the first proof that needs it and kept: a later proof uses the rows
-    // again unless its elements outside them would cost more than new rows.  What the last prove()
+    // again unless its elements outside them would cost more than new rows, and entries whose elements have
+    // cost as much as a row over the proofs get theirs.  What the last prove()
     // did is reported below (hot_rows_reused: it found its rows in place).
     void set_hot_min_count(uint n) { hot_min_count_ = n; }
     uint hot_entries() const { return hot_entries_; }
@@ -96,9 +97,12 @@ protected:
     // the witness well enough.
     affine_t* hot_table_ = nullptr;
     int* hot_slot1_ = nullptr;          // entry -> slot + 1 (0 = no row), T.size entries
-    uint hot_rows_ = 0, hot_cols_ = 0;
+    uint hot_rows_ = 0, hot_cols_ = 0, hot_capacity_ = 0;
     Hyrax* hot_for_ = nullptr;
     void drop_hot_rows();
+    uint32_t* hot_credit_ = nullptr;    // occurrences of entries without a row in the proofs since the rows were made
+    double hot_missed_ = 0;             // elements of entries that had earned a row when there was no more room for it
+    uint64_t grow_hot_rows(Hyrax& hyrax, const uint64_t info[3]);
     affine_t* scaled_table_ = nullptr;  // B[t]*G_i, built on first use
     uint scaled_cols_ = 0;
     Hyrax* scaled_for_ = nullptr;

@@ -409,6 +409,18 @@ int grape_tlookup_hot_select(const uint32_t *d_hist, uint32_t len, uint32_t min_
  * committed as full-width scalars if the rows were used again.  No counterpart in the reference. */
 int grape_tlookup_hot_coverage(const uint32_t *d_hist, uint32_t len, const int32_t *d_slot1, uint64_t *cold_elements,
                                grape_stream_t stream);
+/* The same, and what entries without a slot have been counted over several witnesses: d_credit[t] += d_hist[t] for them
+ * (saturating; len words the caller has cleared at first).  info (HOST, three words; the call synchronises): info[0] =
+ * *cold_elements above, info[1] = those of them whose entry's credit has reached min_credit, info[2] = those whose entry reaches it in
+ * this witness alone.  No counterpart in the reference. */
+int grape_tlookup_hot_credit(const uint32_t *d_hist, uint32_t len, const int32_t *d_slot1, uint32_t *d_credit, uint32_t min_credit,
+                             uint64_t *info, grape_stream_t stream);
+/* More entries for a slot assignment: those without a slot and with d_credit[t] >= min_credit get the slots from first_slot on,
+ * in table order, at most max_new of them (d_hot_list[0 ..] = their entries); slots that are given stay.  info (HOST, two words; the
+ * call synchronises): info[0] = number of slots given now, info[1] = elements of the witness counted in d_hist whose entry
+ * has none even so.  No counterpart in the reference. */
+int grape_tlookup_hot_extend(const uint32_t *d_hist, const uint32_t *d_credit, uint32_t len, uint32_t min_credit, uint32_t first_slot,
+                             uint32_t max_new, int32_t *d_slot1, uint32_t *d_hot_list, uint64_t *info, grape_stream_t stream);
 /* out[i] = d_slot1[d_idx1[i] - 1] (0 when d_idx1[i] is 0 or above len). */
 int grape_tlookup_hot_index(int32_t *d_out, const int32_t *d_idx1, size_t n, const int32_t *d_slot1, uint32_t len,
                             grape_stream_t stream);
