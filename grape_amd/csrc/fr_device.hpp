@@ -30,6 +30,20 @@ __device__ __forceinline__ fr26::Limbs ld_l26(const uint32_t* base, size_t i) { 
 
 using fr26::fold1;
 
+// limb-wise sum over the 16 lanes of a row, valid in its last lane
+__device__ __forceinline__ fr26::Limbs row_sum(fr26::Limbs a) {
+#pragma unroll
+    for (int i = 0; i < fr26::N; i++) {
+        int32_t x = a.v[i];
+        x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);     // row_shr 1, 2, 4, 8
+        x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);
+        x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true);
+        x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true);
+        a.v[i] = x;
+    }
+    return a;
+}
+
 // Table folds of TWO elements by the same challenge, row by row of the table: the ten words of a row
 // arrive through one scalar load and serve both elements, and the row pointer is re-derived from a
 // value the previous row produced, so that the compiler keeps one or two rows in scalar registers

@@ -5,6 +5,7 @@
 // one element with two 16-byte vector accesses, so a wave64 covers 2 KiB of contiguous memory per
 // element index and both halves of every 128-byte line are consumed back to back.
 #include "fr_device.hpp"
+#include <type_traits>
 #include "divstep.hpp"
 
 namespace grape {
@@ -193,40 +194,69 @@ __global__ void __launch_bounds__(kBlock) inv_direct_kernel(uint32_t* out, const
 // ------------------------------------------------------------------------------------------------
 constexpr int kFoldMaxBits = 8;      // bits bound by one pass (at most 64 products per thread)
 constexpr int kFoldMaxPasses = 16;
+constexpr int kFoldJobs = 2;         // tensors folded side by side (grape_fr_fold_pair): one launch serves a pass of both
 
-struct FoldPlan {
-    uint32_t npass;
-    uint32_t lo[kFoldMaxPasses];      // the pass binds challenges lo .. lo+b-1
-    uint32_t b[kFoldMaxPasses];
-    uint32_t off[kFoldMaxPasses];     // first weight of the pass in the weight buffer
-    uint32_t first_plain;             // pass 0 reads plain integers: its weights carry the factor 2^256 that brings
-                                      // a product with a plain value into memory form
+struct FoldWeights {
+    const uint32_t* x[kFoldJobs];
+    uint32_t npass, npass0;                                     // passes of both, of the first
+    uint32_t lo[kFoldJobs * kFoldMaxPasses];                    // the pass binds challenges lo .. lo+b-1
+    uint32_t b[kFoldJobs * kFoldMaxPasses];
+    uint32_t plain;                                             // bit p: pass p reads plain integers, its weights carry the factor 2^256 that
+                                                                // brings a product with a plain value into memory form
 };
 
 // Weights of every pass of a fold, in the 26-bit working form with the radix factor 16 folded
 // in (reduced mod r): workgroup p writes w[i] = prod_k eq(x[lo+k], bit_k(i)) for i < 2^b.
-__global__ void __launch_bounds__(kBlock) fold_weights_kernel(int32_t* wts, const uint32_t* x, FoldPlan plan) {
-    const uint32_t p = blockIdx.x, b = plan.b[p];
-    if (threadIdx.x >= (1u << b)) return;
-    // all challenges first (one memory round trip), then a product tree of depth 3: the
-    // factors of one level are independent, which a single wave needs to issue at full rate
-    Fr f[kFoldMaxBits];
+// Bound by the latency of dependent products: pairs of factors, then fours, then the weight - three products in a row, each on
+// as many lanes as it has values (a tree of seven on every lane took 12 us for a fold, this 5).
+__global__ void __launch_bounds__(kBlock) fold_weights_kernel(int32_t* wts, FoldWeights plan) {
+    __shared__ Fr two[kFoldMaxBits / 2][4], four[2][16];
+    const uint32_t p = blockIdx.x, b = plan.b[p], t = threadIdx.x;
+    const uint32_t* x = plan.x[p >= plan.npass0];
+    const bool plain = (plan.plain >> p) & 1;
+    if (t < 2 * kFoldMaxBits) {
+        const uint32_t k = 2 * (t >> 2);
+        Fr f[2];
 #pragma unroll
-    for (uint32_t k = 0; k < (uint32_t)kFoldMaxBits; k++) f[k] = ld_fr(x, plan.lo[p] + (k < b ? k : 0));
-#pragma unroll
-    for (uint32_t k = 0; k < (uint32_t)kFoldMaxBits; k++)
-        f[k] = k < b ? (((threadIdx.x >> k) & 1) ? f[k] : sub(Fr::one(), f[k])) : Fr::one();
-#pragma unroll
-    for (int width = kFoldMaxBits / 2; width >= 1; width /= 2) {
-#pragma unroll
-        for (int k = 0; k < width; k++) f[k] = fr26::mulc(f[2 * k], f[2 * k + 1]);
+        for (uint32_t i = 0; i < 2; i++) {
+            const Fr v = ld_fr(x, plan.lo[p] + (k + i < b ? k + i : 0));
+            f[i] = k + i < b ? (((t >> i) & 1) ? v : sub(Fr::one(), v)) : Fr::one();
+        }
+        two[t >> 2][t & 3] = fr26::mulc(f[0], f[1]);
     }
-    Fr acc = f[0];
-    if (p == 0 && plan.first_plain) acc = fr26::mulc(acc, Fr::rr());
+    __syncthreads();
+    if (t < 32) four[t >> 4][t & 15] = fr26::mulc(two[2 * (t >> 4)][t & 3], two[2 * (t >> 4) + 1][(t >> 2) & 3]);
+    __syncthreads();
+    if (t >= (1u << b)) return;
+    Fr acc = four[0][t & 15];
+    if (b > 4) acc = fr26::mulc(acc, four[1][t >> 4]);
+    if (plain) acc = fr26::mulc(acc, Fr::rr());
     const fr26::Limbs w = fr26::weight16(acc);
-    int32_t* dst = wts + (size_t)fr26::N * (plan.off[p] + threadIdx.x);
+    int32_t* dst = wts + (size_t)fr26::N * ((p << kFoldMaxBits) + t);
 #pragma unroll
     for (int k = 0; k < fr26::N; k++) dst[k] = w.v[k];
+}
+
+// one tensor's part of a pass
+struct FoldJob {
+    uint32_t* out;
+    const uint32_t* in;
+    const int32_t* wts;
+    uint32_t n_hi_max, outer, c, lg_c_lo, gap;
+};
+struct FoldPassArgs {
+    FoldJob job[kFoldJobs];
+    uint32_t blocks0;                  // the first tensor's workgroups; the others are the second's
+};
+
+// an integer x = l0 + 2^26 l1 with 0 <= l0 < 2^26, -32 <= l1 < 32: a column grows by < 2^53 per term
+__device__ __forceinline__ void fold_mac_int(fr26::Acc& C, const fr26::Limbs& w, int32_t xv) {
+    const int64_t l0 = (int64_t)(xv & (int32_t)fr26::MASK), l1 = (int64_t)(xv >> fr26::W);
+#pragma unroll
+    for (int j = 0; j < fr26::N; j++) {
+        C.c[j] += (int64_t)w.v[j] * l0;
+        C.c[j + 1] += (int64_t)w.v[j] * l1;
+    }
 }
 
 // One pass.  A workgroup is 4 waves: 4/S groups of 64 outputs, each output summed by S waves
@@ -236,19 +266,23 @@ __global__ void __launch_bounds__(kBlock) fold_weights_kernel(int32_t* wts, cons
 // r - |x|): an element is two signed limbs, a product 20 multiply-adds, and 4 bytes are read where the embedded
 // tensor has 32 - the pass that folds an integer tensor without first writing it out as field elements.
 template <int S, bool I32 = false>
-__global__ void __launch_bounds__(kBlock) fold_pass_kernel(uint32_t* __restrict__ out, const uint32_t* __restrict__ in,
-                                                           const int32_t* __restrict__ wts, uint32_t n_hi_max,
-                                                           uint32_t outer, uint32_t c, uint32_t lg_c_lo, uint32_t gap) {
+__global__ void __launch_bounds__(kBlock) fold_pass_kernel(FoldPassArgs args) {
     constexpr int IW = 4 / S;                       // output groups per workgroup
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int iw = wave % IW, part = wave / IW;
+    const bool second = blockIdx.x >= args.blocks0;
+    const FoldJob& job = args.job[second];
+    uint32_t* __restrict__ out = job.out;
+    const uint32_t* __restrict__ in = job.in;
+    const int32_t* __restrict__ wts = job.wts;
+    const uint32_t c = job.c, lg_c_lo = job.lg_c_lo, gap = job.gap, n_hi_max = job.n_hi_max;
     // index arithmetic in 32 bits (the host checks that the output count fits)
     const uint32_t c_lo = 1u << lg_c_lo;
     const uint32_t c_out = c < c_lo ? c : c_lo;     // surviving extent of the axis
     const uint32_t inner = c_out * gap;             // outputs per outer index
-    const uint32_t total = outer * inner;
-    const uint32_t tid = ((uint32_t)blockIdx.x * IW + iw) * 64 + lane;
+    const uint32_t total = job.outer * inner;
+    const uint32_t tid = (((uint32_t)blockIdx.x - (second ? args.blocks0 : 0u)) * IW + iw) * 64 + lane;
     const bool live = tid < total;
     const uint32_t o = live ? tid / inner : 0;
     const uint32_t p = live ? tid - o * inner : 0;  // i_lo*gap + g
@@ -269,15 +303,6 @@ __global__ void __launch_bounds__(kBlock) fold_pass_kernel(uint32_t* __restrict_
     constexpr int U = I32 ? 8 : 4;
     const uint32_t n_full = c >> lg_c_lo;
     uint32_t h = (uint32_t)part;
-    // an integer x = l0 + 2^26 l1 with 0 <= l0 < 2^26, -32 <= l1 < 32: a column grows by < 2^53 per term
-    auto mac_int = [&](const fr26::Limbs& w, int32_t xv) {
-        const int64_t l0 = (int64_t)(xv & (int32_t)fr26::MASK), l1 = (int64_t)(xv >> fr26::W);
-#pragma unroll
-        for (int j = 0; j < fr26::N; j++) {
-            C.c[j] += (int64_t)w.v[j] * l0;
-            C.c[j + 1] += (int64_t)w.v[j] * l1;
-        }
-    };
     for (; h + (U - 1) * S < n_full; h += U * S) {
         Fr t[I32 ? 1 : U];
         int32_t ti[I32 ? U : 1];
@@ -291,7 +316,7 @@ __global__ void __launch_bounds__(kBlock) fold_pass_kernel(uint32_t* __restrict_
             fr26::Limbs w;
 #pragma unroll
             for (int j = 0; j < fr26::N; j++) w.v[j] = wts[(size_t)fr26::N * (h + k * S) + j];
-            if (I32) mac_int(w, ti[k]);
+            if (I32) fold_mac_int(C, w, ti[k]);
             else fr26::mac(C, w, fr26::pack(t[k]));
         }
     }
@@ -300,7 +325,7 @@ __global__ void __launch_bounds__(kBlock) fold_pass_kernel(uint32_t* __restrict_
             fr26::Limbs w;
 #pragma unroll
             for (int j = 0; j < fr26::N; j++) w.v[j] = wts[(size_t)fr26::N * h + j];
-            if (I32) mac_int(w, isrc[(size_t)h * hi_stride]);
+            if (I32) fold_mac_int(C, w, isrc[(size_t)h * hi_stride]);
             else fr26::mac(C, w, ld_l26(src, (size_t)h * hi_stride));
         }
     }
@@ -325,12 +350,95 @@ __global__ void __launch_bounds__(kBlock) fold_pass_kernel(uint32_t* __restrict_
     if (part == 0 && live) st_fr(out, tid, fr26::unpack(fr26::canon_wide(r)));
 }
 
+// A pass with few outputs: 256 / P of them a workgroup, each summed by P of its threads, P = 16 or 256, so that a chain of
+// terms is a sixteenth as long and the outputs of a short pass still fill the chip.  Two operands' 4096 outputs of 128 terms: 11 us
+// where four waves an output took 2 x 8 for 8 terms each and left the rest to a workgroup per outer index (2 x 13).  P threads' sums of at most 256 / P
+// products each: P = 16, 16 (1 + 16 / 35.3) r = 23.3 r at most; P = 256, 16 (1 + 1 / 35.3) r = 16.5 r in a row of lanes.
+template <int P, bool I32 = false>
+__global__ void __launch_bounds__(kBlock) fold_short_kernel(FoldPassArgs args) {
+    static_assert(P == 16 || P == 256, "parts that meet in LDS resp. in a row of lanes first");
+    constexpr int OW = kBlock / P;
+    const bool second = blockIdx.x >= args.blocks0;
+    const FoldJob& job = args.job[second];
+    const uint32_t c = job.c, lg_c_lo = job.lg_c_lo, gap = job.gap;
+    const uint32_t c_lo = 1u << lg_c_lo, c_out = c < c_lo ? c : c_lo, inner = c_out * gap, total = job.outer * inner;
+    const uint32_t o_in = threadIdx.x % OW, part = threadIdx.x / OW;
+    const uint32_t q = ((uint32_t)blockIdx.x - (second ? args.blocks0 : 0u)) * OW + o_in;
+    const bool live = q < total;
+    const uint32_t o = live ? q / inner : 0, p = live ? q - o * inner : 0, i_lo = p / gap;
+    const size_t first = (size_t)o * c * gap + p, hi_stride = (size_t)c_lo * gap;
+    const uint32_t n_hi = live ? (c - i_lo + c_lo - 1) >> lg_c_lo : 0;
+    const int32_t* in32 = reinterpret_cast<const int32_t*>(job.in);
+    fr26::Acc C;
+    fr26::acc_zero(C);
+    auto terms = [&](uint32_t h, auto count) {      // `count` terms, all their operands asked for before the first is used
+        constexpr int U = decltype(count)::value;
+        Fr t[U];
+        int32_t ti[U];
+        fr26::Limbs w[U];
+#pragma unroll
+        for (int k = 0; k < U; k++) {
+            if (I32) ti[k] = in32[first + (h + k * P) * hi_stride];
+            else t[k] = ld_fr(job.in, first + (h + k * P) * hi_stride);
+            const int2* wp = reinterpret_cast<const int2*>(job.wts + (size_t)fr26::N * (h + k * P));
+#pragma unroll
+            for (int j = 0; j < fr26::N / 2; j++) {
+                const int2 v = wp[j];
+                w[k].v[2 * j] = v.x;
+                w[k].v[2 * j + 1] = v.y;
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);          // the compiler would ask for each where it is used: a round trip a term
+#pragma unroll
+        for (int k = 0; k < U; k++) {
+            if (I32) fold_mac_int(C, w[k], ti[k]);
+            else fr26::mac(C, w[k], fr26::pack(t[k]));
+        }
+    };
+    uint32_t h = part;
+    if (P == 16)
+        for (; h + 3 * P < n_hi; h += 4 * P) terms(h, std::integral_constant<int, 4>());
+    for (; h < n_hi; h += P) terms(h, std::integral_constant<int, 1>());
+    fr26::Limbs r = fr26::reduce(C, 0);
+    if constexpr (P == 16) {
+        __shared__ int32_t lds[fr26::N][kBlock + OW];
+#pragma unroll
+        for (int k = 0; k < fr26::N; k++) lds[k][threadIdx.x] = r.v[k];
+        __syncthreads();
+        if (threadIdx.x < fr26::N * OW) {
+            const uint32_t k = threadIdx.x / OW, oo = threadIdx.x % OW;
+            int32_t sum = 0;
+#pragma unroll
+            for (int i = 0; i < P; i++) sum += lds[k][i * OW + oo];
+            lds[k][kBlock + oo] = sum;
+        }
+        __syncthreads();
+        if (part == 0 && live) {
+#pragma unroll
+            for (int k = 0; k < fr26::N; k++) r.v[k] = lds[k][kBlock + o_in];
+            st_fr(job.out, q, fr26::unpack(fr26::canon_wide(fr26::normalize(r))));
+        }
+    } else {
+        __shared__ Fr rows[kBlock / 16];
+        const Fr f = fr26::limb_sum_to_fr(row_sum(r), 0);
+        if ((threadIdx.x & 15) == 15) rows[threadIdx.x >> 4] = f;
+        __syncthreads();
+        if (threadIdx.x < 64) {
+            const Fr s = fr26::limb_sum_to_fr(row_sum(fr26::pack(rows[threadIdx.x & 15])), 0);
+            if (threadIdx.x == 15 && live) st_fr(job.out, q, s);
+        }
+    }
+}
+
 // Small-tensor finish: one workgroup holds the whole [c][gap] slab of one outer index in LDS
 // and binds the remaining bits top-down with a barrier per level.
 constexpr int kFoldSmallElems = 2048;   // 64 KiB of LDS
 constexpr int kFoldSmallMaxOuter = 256; // one workgroup per outer index: worth it only for few
+// Only the whole of a fold that is short anyway, which needs no weights then: an element a thread, or two variables (one call after
+// another, launches included: 256 elements 11.5 us against 13.3 through a pass, 16 slabs of 16 x 4 12.5 against 17; 2048
+// elements 19 against 16.5, 4096 with a pass before it 33 against 17).
 static bool fold_small_fits(size_t outer, size_t c, size_t gap) {
-    return c * gap <= (size_t)kFoldSmallElems && outer <= (size_t)kFoldSmallMaxOuter;
+    return c * gap <= (size_t)(c <= 4 ? kFoldSmallElems : kBlock) && outer <= (size_t)kFoldSmallMaxOuter;
 }
 
 __global__ void __launch_bounds__(kBlock) fold_small_kernel(uint32_t* out, const uint32_t* in, const uint32_t* x,
@@ -563,185 +671,280 @@ int grape_i32_pad_fill(int32_t* out, const int32_t* in, uint32_t N, uint32_t pad
     return GRAPE_OK;
 }
 
-// Plan of a fold's passes: each binds as many top bits as possible (6, or more when the outputs are
-// too few to fill the chip and S waves share one output), until the slab of one outer index
-// fits the LDS finish kernel.
-struct FoldPass { uint32_t b, S, off; };
-static int plan_fold(size_t outer, uint32_t c, uint32_t gap, uint32_t id, FoldPass* passes, FoldPlan& plan) {
+// Plan of a fold's passes.  While a pass has outputs enough to fill the chip it binds as many top bits as it can stream; behind those
+// the passes are short, bound by the chain of terms of one output, and bind up to eight bits each.
+struct FoldPass { uint32_t b, P; };                // bits, parts that share an output
+struct FoldPlan {
+    uint32_t npass;
+    FoldPass pass[kFoldMaxPasses];
+    uint32_t lo[kFoldMaxPasses];
+};
+// Parts per output of a short pass over n_out outputs and 2^b terms: 125 instructions a term, 350 for the reduction of a part's sum
+// and what the parts take to meet; a lone wave on a SIMD issues one instruction every 6.5 cycles, more of them one every 4.4.
+static uint32_t short_pass_parts(size_t n_out, uint32_t b) {
+    uint32_t best = 0;
+    double best_t = 0;
+    for (uint32_t P : {1u, 2u, 4u, 16u, 256u}) {
+        if (P < 4 && (1u << b) > 64 * P) continue;
+        const uint32_t terms = ((1u << b) + P - 1) / P;
+        const double meet = P == 1 ? 0 : P < 16 ? 80 : P == 16 ? 150 : 300;
+        const double waves = (double)n_out * P / (64 * 4 * kNumCU);
+        const double t = (125.0 * terms + 350 + meet) * (4.4 * waves > 6.5 ? 4.4 * waves : 6.5);
+        if (best == 0 || t < best_t) {
+            best = P;
+            best_t = t;
+        }
+    }
+    return best;
+}
+static int plan_fold(size_t outer, uint32_t c, uint32_t gap, uint32_t id, bool ints, FoldPlan& plan) {
     plan.npass = 0;
-    plan.first_plain = 0;
-    uint32_t l = log2ceil(c), off = 0;
-    size_t cc = c;
-    while (l > 0 && !fold_small_fits(outer, cc, gap)) {
+    uint32_t l = log2ceil(c);
+    if (fold_small_fits(outer, c, gap)) return GRAPE_OK;
+    while (l > 0) {
         // Measured on MI355X: a pass streams fastest with one thread per output, 16 to 64
         // terms per thread and 2^20 threads; 2^19 threads come close.  Failing that, up to
-        // four waves share an output to reach 2^19 threads.
-        uint32_t S = 0, b = 0;
+        // four waves share an output to reach 2^19 threads.  A pass over integers reads an eighth of the bytes and is bound by
+        // instructions, of which a thread's reduction is as many as 16 terms: 2^17 threads of up to 64 terms there (2048 x 4096
+        // integers 30 -> 24 us, 4096 x 4096 45 -> 32, 2048 x 11008 53 -> 39, no size slower; 16 loads in flight instead of 8: no faster).
+        const bool plain = ints && plan.npass == 0;
+        const uint32_t most = plain ? 17 : 20, least = plain ? 17 : 19;
+        uint32_t P = 0, b = 0;
         auto items = [&](uint32_t tb) { return outer * gap * ((size_t)1 << (l - tb)); };
-        for (uint32_t want = 20; want >= 19 && S == 0; want--) {
-            for (uint32_t tb = l < 6 ? l : 6; tb >= 4 && S == 0; tb--) {
-                if (items(tb) >= ((size_t)1 << want)) { S = 1; b = tb; }
+        for (uint32_t want = most; want >= least && P == 0; want--) {
+            for (uint32_t tb = l < 6 ? l : 6; tb >= 4 && P == 0; tb--) {
+                if (items(tb) >= ((size_t)1 << want)) { P = 1; b = tb; }
             }
         }
-        for (uint32_t tb = l < 8 ? l : 8; tb >= 4 && S == 0; tb--) {
+        for (uint32_t tb = l < 8 ? l : 8; tb >= 4 && P == 0; tb--) {
             const uint32_t ts = items(tb) * 2 >= ((size_t)1 << 19) ? 2 : 4;
-            if (items(tb) * ts >= ((size_t)1 << 19) && (1u << tb) <= 64 * ts) { S = ts; b = tb; }
+            if (items(tb) * ts >= ((size_t)1 << 19) && (1u << tb) <= 64 * ts) { P = ts; b = tb; }
         }
-        if (S == 0) {
-            // too few outputs to fill the chip whatever the split: four waves per output and
-            // at most 32 terms per thread keep the pass short
-            S = 4; b = l <= 7 ? l : 6;
-            // few, short slabs: stop as soon as the LDS finish kernel can take over
-            if (outer <= (size_t)kFoldSmallMaxOuter && gap <= (size_t)kFoldSmallElems) {
-                uint32_t keep = 0;      // bits the finish kernel can bind
-                while (keep < l && (((size_t)2 << keep) * gap) <= (size_t)kFoldSmallElems) keep++;
-                if (l > keep && l - keep < b) b = l - keep;
-            }
+        if (P == 0) {
+            // too few outputs to fill the chip whatever the split: as few passes as there can be, of about the same length
+            const uint32_t left = (l + kFoldMaxBits - 1) / kFoldMaxBits;
+            b = (l + left - 1) / left;
+            P = short_pass_parts(items(b), b);
         }
         GRAPE_REQUIRE(plan.npass < (uint32_t)kFoldMaxPasses, "fold: too many passes");
-        passes[plan.npass] = {b, S, off};
+        plan.pass[plan.npass] = {b, P};
         plan.lo[plan.npass] = id + (l - b);
-        plan.b[plan.npass] = b;
-        plan.off[plan.npass] = off;
         plan.npass++;
-        off += 1u << b;
         l -= b;
-        const size_t c_lo = (size_t)1 << l;
-        cc = cc < c_lo ? cc : c_lo;
     }
     return GRAPE_OK;
 }
 
-// grape_fr_fold on t, or the fold of another tensor left in t: of field elements (`from`), which the first pass reads where
-// they are - a caller that keeps them need not copy them first, as much traffic as the fold itself - or of integers
-// (`ints`, 4 bytes per element); the later passes work on what the first one wrote.
-static int fold_impl(uint32_t* t, const uint32_t* from, const int32_t* ints, size_t N, const uint32_t* x, uint32_t c, uint32_t id, uint32_t gap, grape_stream_t st) {
-    if (N == 0) return GRAPE_OK;
-    CHECK_PTR16(t); CHECK_PTR16(x);
-    GRAPE_REQUIRE(c >= 1 && gap >= 1 && N >= (size_t)c * gap && N % ((size_t)c * gap) == 0, "N must be a multiple of c*gap");
-    hipStream_t s = as_stream(st);
-    const size_t outer = N / ((size_t)c * gap);
-    uint32_t L = log2ceil(c);
-    FoldPass passes[kFoldMaxPasses];
+// The fold of one tensor on its way through its passes.
+// With a single outer index a pass can run in place (an output's threads read nothing that another output is left in).
+// Otherwise passes ping-pong through scratch and the last one writes to the front.
+struct FoldRun {
+    const grape_fold_job* j;
     FoldPlan plan;
-    int prc = plan_fold(outer, c, gap, id, passes, plan);
-    if (prc) return prc;
-    if (ints && (L == 0 || plan.npass == 0)) {
-        // nothing to bind, or a tensor small enough for the finish kernel alone: embedded first (N elements of t)
-        from_i32_kernel<<<blocks_for(N), kBlock, 0, s>>>(t, ints, N);
-        GRAPE_LAUNCH_CHECK();
-        ints = nullptr;
+    size_t outer, cur_c;
+    uint32_t L, pi;
+    bool ints, done;
+    const uint32_t* src;
+    size_t each;                       // elements of one scratch buffer, 0: none
+    uint32_t* ws[2];
+    int which;
+    const int32_t* wts;
+};
+static int fold_start(FoldRun& r, const grape_fold_job& j, hipStream_t s) {
+    r = FoldRun{};
+    r.j = &j;
+    r.done = j.N == 0;
+    if (r.done) return GRAPE_OK;
+    CHECK_PTR16(j.t); CHECK_PTR16(j.x);
+    GRAPE_REQUIRE(j.c >= 1 && j.gap >= 1 && j.N >= (size_t)j.c * j.gap && j.N % ((size_t)j.c * j.gap) == 0, "N must be a multiple of c*gap");
+    GRAPE_REQUIRE(!j.from || !j.ints, "one source");
+    if (j.from) {
+        CHECK_PTR16(j.from);
+        GRAPE_REQUIRE(j.from != j.t, "the source is kept: grape_fr_fold folds in place");
     }
-    if (L == 0) {                  // c == 1: nothing to bind, data already compact
-        if (from) GRAPE_HIP_CHECK(hipMemcpyAsync(t, from, N * 32, hipMemcpyDeviceToDevice, s));
+    r.outer = j.N / ((size_t)j.c * j.gap);
+    r.cur_c = j.c;
+    r.L = log2ceil(j.c);
+    int rc = plan_fold(r.outer, j.c, j.gap, j.id, j.ints != nullptr, r.plan);
+    if (rc) return rc;
+    r.ints = j.ints != nullptr;
+    if (r.ints && (r.L == 0 || r.plan.npass == 0)) {
+        // nothing to bind, or a tensor small enough for the finish kernel alone: embedded first (N elements of t)
+        from_i32_kernel<<<blocks_for(j.N), kBlock, 0, s>>>(j.t, j.ints, j.N);
+        GRAPE_LAUNCH_CHECK();
+        r.ints = false;
+    }
+    r.src = r.ints ? reinterpret_cast<const uint32_t*>(j.ints) : j.from ? j.from : j.t;
+    if (r.L == 0) {                // c == 1: nothing to bind, data already compact
+        if (j.from) GRAPE_HIP_CHECK(hipMemcpyAsync(j.t, j.from, j.N * 32, hipMemcpyDeviceToDevice, s));
+        r.done = true;
         return GRAPE_OK;
     }
-    plan.first_plain = ints ? 1u : 0u;
-    const uint32_t* xs = x + 8 * (size_t)id;
-    size_t cur_c = c;
-    const uint32_t* src = ints ? reinterpret_cast<const uint32_t*>(ints) : from ? from : t;
-    // With a single outer index a pass can run in place (thread p reads p + k*stride only).
-    // Otherwise passes ping-pong through scratch and the result is copied to the front.
-    uint32_t* ws[2] = {nullptr, nullptr};
-    int which = 0;
-    const int32_t* wts = nullptr;
-    if (plan.npass) {
+    // a single pass from another tensor writes to the front; with several outer indices the others go through scratch, the largest first
+    if (r.outer > 1) {
+        const uint32_t first = r.plan.npass ? r.L - r.plan.pass[0].b : 0;
+        const size_t c_out = r.cur_c < ((size_t)1 << first) ? r.cur_c : (size_t)1 << first;
+        if (r.plan.npass > 1 || r.src == j.t) r.each = r.outer * c_out * j.gap;
+    }
+    return GRAPE_OK;
+}
+// where the next pass, which leaves `c_out` of the axis, writes
+static uint32_t* fold_target(FoldRun& r, bool last) {
+    if (r.outer == 1 || (last && r.src != r.j->t)) return r.j->t;
+    uint32_t* dst = r.ws[r.which];
+    r.which ^= 1;
+    return dst;
+}
+static int fold_next(FoldRun& r, FoldJob& out, uint32_t& total) {
+    const FoldPass& ps = r.plan.pass[r.pi];
+    const uint32_t lo = r.L - ps.b;
+    const size_t c_lo = (size_t)1 << lo, c_out = r.cur_c < c_lo ? r.cur_c : c_lo, n = r.outer * c_out * r.j->gap;
+    GRAPE_REQUIRE(n < ((size_t)1 << 32) - 256, "fold: more than 2^32 outputs in one pass");
+    total = (uint32_t)n;
+    out.out = fold_target(r, lo == 0);
+    out.in = r.src;
+    out.wts = r.wts + (size_t)fr26::N * ((size_t)r.pi << kFoldMaxBits);
+    out.n_hi_max = (uint32_t)((r.cur_c + c_lo - 1) / c_lo);
+    out.outer = (uint32_t)r.outer;
+    out.c = (uint32_t)r.cur_c;
+    out.lg_c_lo = lo;
+    out.gap = r.j->gap;
+    r.src = out.out;
+    r.cur_c = c_out;
+    r.L = lo;
+    r.pi++;
+    r.ints = false;                    // the first pass of a fold of integers leaves field elements
+    return GRAPE_OK;
+}
+
+extern "C++" {
+template <bool I32>
+static void launch_fold_pass(const FoldPassArgs& a, uint32_t P, unsigned blocks, hipStream_t s) {
+    if (P == 1) fold_pass_kernel<1, I32><<<blocks, kBlock, 0, s>>>(a);
+    else if (P == 2) fold_pass_kernel<2, I32><<<blocks, kBlock, 0, s>>>(a);
+    else if (P == 4) fold_pass_kernel<4, I32><<<blocks, kBlock, 0, s>>>(a);
+    else if (P == 16) fold_short_kernel<16, I32><<<blocks, kBlock, 0, s>>>(a);
+    else fold_short_kernel<256, I32><<<blocks, kBlock, 0, s>>>(a);
+}
+}
+
+// Folds of up to two tensors, pass by pass; passes of one kind that stand at the same place of both share a launch.  Two operands of
+// a matrix product go through the same kinds of passes: 32 heads of 2048 x 128 integers took two chains of four
+// launches, 100 us of kernels, and take one of three, 41 (the proof 172 -> 113 us).
+static int fold_jobs(const grape_fold_job* jobs, uint32_t count, grape_stream_t st) {
+    hipStream_t s = as_stream(st);
+    FoldRun run[kFoldJobs];
+    FoldWeights fw = {};
+    size_t scratch = 0;
+    for (uint32_t k = 0; k < count; k++) {
+        int rc = fold_start(run[k], jobs[k], s);
+        if (rc) return rc;
+        if (run[k].done) continue;
+        scratch += 2 * run[k].each;
+        fw.x[k] = jobs[k].x;
+        if (run[k].ints && run[k].plan.npass) fw.plain |= 1u << fw.npass;
+        for (uint32_t i = 0; i < run[k].plan.npass; i++, fw.npass++) {
+            fw.lo[fw.npass] = run[k].plan.lo[i];
+            fw.b[fw.npass] = run[k].plan.pass[i].b;
+        }
+        if (k == 0) fw.npass0 = fw.npass;
+    }
+    if (scratch) {
         void* p;
-        int rc = scratch_get(kSlotFoldW, ((size_t)kFoldMaxPasses * (1u << kFoldMaxBits) + 64) * fr26::N * 4, &p, s);
+        int rc = scratch_get(kSlotFold, scratch * 32 + 64, &p, s);
+        if (rc) return rc;
+        uint32_t* ws = (uint32_t*)p;
+        for (uint32_t k = 0; k < count; k++) {
+            for (int i = 0; i < 2; i++, ws += 8 * run[k].each) run[k].ws[i] = ws;
+        }
+    }
+    if (fw.npass) {
+        void* p;
+        int rc = scratch_get(kSlotFoldW, ((size_t)kFoldJobs * kFoldMaxPasses * (1u << kFoldMaxBits) + 64) * fr26::N * 4, &p, s);
         if (rc) return rc;
         profile_begin();
         profile_mark(s);
-        fold_weights_kernel<<<plan.npass, kBlock, 0, s>>>((int32_t*)p, x, plan);
+        fold_weights_kernel<<<fw.npass, kBlock, 0, s>>>((int32_t*)p, fw);
         GRAPE_LAUNCH_CHECK();
         profile_mark(s);               // profiled intervals: the weight kernel, then one per pass
-        wts = (const int32_t*)p;
+        run[0].wts = (const int32_t*)p;
+        if (count > 1) run[1].wts = (const int32_t*)p + ((size_t)fr26::N * fw.npass0 << kFoldMaxBits);
     }
-    uint32_t pi = 0;
-    while (L > 0) {
-        if (fold_small_fits(outer, cur_c, gap)) {
-            uint32_t* dst = t;
-            if (outer > 1 && src == t) {
-                // reading slabs o*cur_c*gap while writing o*gap would race across workgroups
-                void* p;
-                int rc = scratch_get(kSlotFold, outer * gap * 32 * 2 + 64, &p, s);
-                if (rc) return rc;
-                dst = (uint32_t*)p;
-            }
-            fold_small_kernel<<<(unsigned)outer, kBlock, 0, s>>>(dst, src, xs, L, cur_c, gap);
-            GRAPE_LAUNCH_CHECK();
-            if (dst != t) GRAPE_HIP_CHECK(hipMemcpyAsync(t, dst, outer * gap * 32, hipMemcpyDeviceToDevice, s));
-            return GRAPE_OK;
+    auto at_pass = [&](uint32_t k) { return !run[k].done && run[k].pi < run[k].plan.npass; };
+    for (;;) {
+        FoldPassArgs a = {};
+        unsigned blocks = 0;
+        uint32_t P = 0, jobs_in = 0;
+        bool plain = false;
+        for (uint32_t k = 0; k < count; k++) {
+            if (!at_pass(k)) continue;
+            const uint32_t pk = run[k].plan.pass[run[k].pi].P;
+            if (jobs_in && (pk != P || run[k].ints != plain)) continue;        // takes the next launch
+            P = pk;
+            plain = run[k].ints;
+            uint32_t total = 0;
+            int rc = fold_next(run[k], a.job[jobs_in++], total);
+            if (rc) return rc;
+            if (jobs_in == 1) a.blocks0 = 0xffffffffu;
+            else a.blocks0 = blocks;
+            blocks += blocks_for(total, kBlock / (int)P);
         }
-        const FoldPass& ps = passes[pi++];
-        const uint32_t b = ps.b;
-        const size_t c_lo = (size_t)1 << (L - b);
-        const size_t c_out = cur_c < c_lo ? cur_c : c_lo;
-        uint32_t* dst;
-        if (outer == 1) {
-            dst = t;   // in place, or from the source of the first pass
-        } else if (L == b && src != t) {
-            dst = t;   // the last pass
-        } else {
-            if (!ws[0]) {
-                void* p;
-                // two buffers, each large enough for the first pass output
-                size_t each = outer * c_out * gap * 32;
-                int rc = scratch_get(kSlotFold, 2 * each + 64, &p, s);
-                if (rc) return rc;
-                ws[0] = (uint32_t*)p;
-                ws[1] = (uint32_t*)((char*)p + each);
-            }
-            dst = ws[which];
-            which ^= 1;
-        }
-        const size_t total = outer * c_out * gap;
-        GRAPE_REQUIRE(total < ((size_t)1 << 32) - 256, "fold: more than 2^32 outputs in one pass");
-        const uint32_t n_hi_max = (uint32_t)((cur_c + c_lo - 1) / c_lo);
-        const int32_t* w = wts + (size_t)fr26::N * ps.off;
-        const bool plain = ints != nullptr && pi == 1;      // the first pass of a fold of integers
-#define GRAPE_FOLD_PASS(SS, PER)                                                                                                    \
-    do {                                                                                                                            \
-        if (plain) fold_pass_kernel<SS, true><<<blocks_for(total, PER), kBlock, 0, s>>>(dst, src, w, n_hi_max, (uint32_t)outer, (uint32_t)cur_c, L - b, gap); \
-        else fold_pass_kernel<SS, false><<<blocks_for(total, PER), kBlock, 0, s>>>(dst, src, w, n_hi_max, (uint32_t)outer, (uint32_t)cur_c, L - b, gap);     \
-    } while (0)
-        if (ps.S == 1) GRAPE_FOLD_PASS(1, 256);
-        else if (ps.S == 2) GRAPE_FOLD_PASS(2, 128);
-        else GRAPE_FOLD_PASS(4, 64);
-#undef GRAPE_FOLD_PASS
+        if (!jobs_in) break;
+        if (plain) launch_fold_pass<true>(a, P, blocks, s);
+        else launch_fold_pass<false>(a, P, blocks, s);
         GRAPE_LAUNCH_CHECK();
         profile_mark(s);
-        src = dst;
-        cur_c = c_out;
-        L -= b;
     }
-    if (src != t) GRAPE_HIP_CHECK(hipMemcpyAsync(t, src, outer * gap * 32, hipMemcpyDeviceToDevice, s));
+    for (uint32_t k = 0; k < count; k++) {
+        FoldRun& r = run[k];
+        if (r.done) continue;
+        if (r.plan.npass == 0) {
+            // reading slabs o*c*gap of t while writing o*gap of it would race across workgroups: through scratch
+            uint32_t* dst = fold_target(r, true);
+            fold_small_kernel<<<(unsigned)r.outer, kBlock, 0, s>>>(dst, r.src, r.j->x + 8 * (size_t)r.j->id, r.L, r.cur_c, r.j->gap);
+            GRAPE_LAUNCH_CHECK();
+            r.src = dst;
+        }
+        if (r.src != r.j->t) GRAPE_HIP_CHECK(hipMemcpyAsync(r.j->t, r.src, r.outer * r.j->gap * 32, hipMemcpyDeviceToDevice, s));
+    }
     return GRAPE_OK;
 }
 
 int grape_fr_fold(uint32_t* t, size_t N, const uint32_t* x, uint32_t c, uint32_t id, uint32_t gap, grape_stream_t st) {
-    return fold_impl(t, nullptr, nullptr, N, x, c, id, gap, st);
+    const grape_fold_job j = {t, nullptr, nullptr, N, x, c, id, gap};
+    return fold_jobs(&j, 1, st);
 }
 int grape_fr_fold_from(uint32_t* out, const uint32_t* in, size_t N, const uint32_t* x, uint32_t c, uint32_t id, uint32_t gap, grape_stream_t st) {
     if (N == 0) return GRAPE_OK;
     CHECK_PTR16(in);
-    GRAPE_REQUIRE(in != out, "the source is kept: grape_fr_fold folds in place");
-    return fold_impl(out, in, nullptr, N, x, c, id, gap, st);
+    const grape_fold_job j = {out, in, nullptr, N, x, c, id, gap};
+    return fold_jobs(&j, 1, st);
 }
 
 size_t grape_fr_fold_i32_elems(size_t N, uint32_t c, uint32_t gap) {
     if (N == 0 || c == 0 || gap == 0 || N % ((size_t)c * gap) != 0) return N;
     const size_t outer = N / ((size_t)c * gap);
-    FoldPass passes[kFoldMaxPasses];
-    FoldPlan plan;
-    if (plan_fold(outer, c, gap, 0, passes, plan) != GRAPE_OK || plan.npass == 0) return N;
-    if (outer > 1) return outer * gap;                 // the passes go through work memory of the library
-    const size_t c_lo = (size_t)1 << (log2ceil(c) - passes[0].b);
-    return (c < c_lo ? c : c_lo) * gap;                // one outer index: the first pass writes into d_out
+    size_t most = 0;
+    for (const bool ints : {false, true}) {            // integers are folded in other steps than field elements
+        FoldPlan plan;
+        if (plan_fold(outer, c, gap, 0, ints, plan) != GRAPE_OK || plan.npass == 0) return N;
+        const size_t c_lo = (size_t)1 << (log2ceil(c) - plan.pass[0].b);
+        // several outer indices: the passes go through work memory of the library; one: the first pass writes into d_out
+        const size_t n = outer > 1 ? outer * gap : (c < c_lo ? c : c_lo) * gap;
+        if (n > most) most = n;
+    }
+    return most;
 }
 
 int grape_fr_fold_i32(uint32_t* out, const int32_t* in, size_t N, const uint32_t* x, uint32_t c, uint32_t id, uint32_t gap, grape_stream_t st) {
     GRAPE_REQUIRE(in != nullptr || N == 0, "null input");
-    return fold_impl(out, nullptr, in, N, x, c, id, gap, st);
+    const grape_fold_job j = {out, nullptr, in, N, x, c, id, gap};
+    return fold_jobs(&j, 1, st);
+}
+
+int grape_fr_fold_pair(const grape_fold_job* jobs, uint32_t count, grape_stream_t st) {
+    GRAPE_REQUIRE(jobs != nullptr && count >= 1 && count <= (uint32_t)kFoldJobs, "one or two folds");
+    return fold_jobs(jobs, count, st);
 }
 
 }  // extern "C"

@@ -79,19 +79,6 @@ struct RoundSums {
     uint32_t rowlen[kShortMaxRounds], rowpad[kShortMaxRounds];
 };
 
-// limb-wise sum over the 16 lanes of a row, valid in its last lane
-__device__ __forceinline__ fr26::Limbs row_sum(fr26::Limbs a) {
-#pragma unroll
-    for (int i = 0; i < fr26::N; i++) {
-        int32_t x = a.v[i];
-        x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);     // row_shr 1, 2, 4, 8
-        x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);
-        x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true);
-        x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true);
-        a.v[i] = x;
-    }
-    return a;
-}
 // sum over the wave of limbs whose 16-lane sums lie in (-add_r r, (32 - add_r) r); the same in every lane
 __device__ __forceinline__ Fr wave_limb_sum(const fr26::Limbs& a, int add_r) {
     const Fr f = fr26::limb_sum_to_fr(row_sum(a), add_r);

@@ -172,15 +172,24 @@ struct Operand {
     const fr_t* kept = nullptr;
     const int* ints = nullptr;
     std::unique_ptr<FrTensor> own;
-    FrTensor& fold(uint size, fr_t* x, uint c, uint id, uint gap) {
-        if (consumed) {
-            consumed->partial_eval(size, x, c, id, gap);
-            return *consumed;
+    // the fold over the row variables, into a tensor of its own where the operand is kept
+    grape_fold_job fold(uint size, fr_t* x, uint c, uint id, uint gap) {
+        if (!consumed) {
+            own.reset(new FrTensor((uint)std::max<size_t>(grape_fr_fold_i32_elems(size, c, gap), 1), OnDefaultStream()));
+            own->set_size(size / (c * gap) * gap);
         }
-        own.reset(kept ? new FrTensor(FrTensor::folded_from(kept, size, x, c, id, gap, OnDefaultStream()))
-                       : new FrTensor(FrTensor::folded_from_ints(ints, size, x, c, id, gap, OnDefaultStream())));
-        return *own;
+        grape_fold_job j{};
+        j.t = W(tensor().gpu_data);
+        if (kept) j.from = W(kept);
+        j.ints = ints;
+        j.N = size;
+        j.x = W(x);
+        j.c = c;
+        j.id = id;
+        j.gap = gap;
+        return j;
     }
+    FrTensor& tensor() { return consumed ? *consumed : *own; }
 };
 // Both phases where the folded operands are short: all rounds in one call, and one copy brings their sums and the two
 // elements that are left.  u, v (host) and U, V (device) point behind the variables of the batch and inner index.
@@ -242,8 +251,12 @@ std::pair<Fr, Fr> prove_matmul_impl(Operand A_op, Operand B_op, int L, int N, in
     fr_t* V = grape_host::upload(v, OnDefaultStream());
     std::pair<Fr, Fr> ret;
     try {
-        FrTensor& A = A_op.fold((uint)(L * N * K), U, N, Log2(M), K);
-        FrTensor& B = B_op.fold((uint)(L * M * K), U, M, 0, K);
+        const grape_fold_job folds[2] = {A_op.fold((uint)(L * N * K), U, N, Log2(M), K), B_op.fold((uint)(L * M * K), U, M, 0, K)};
+        // one tensor as both operands is folded twice, one fold after the other
+        const bool apart = folds[0].t != folds[1].t;
+        check(grape_fr_fold_pair(folds, apart ? 2 : 1, nullptr), "grape_fr_fold_pair");
+        if (!apart) check(grape_fr_fold_pair(folds + 1, 1, nullptr), "grape_fr_fold_pair");
+        FrTensor &A = A_op.tensor(), &B = B_op.tensor();
         Fr eq_accumulate;
         if ((uint)(L * K) >= 2 && (uint)(L * K) <= GRAPE_SHORT_MAX && (L & (L - 1)) == 0) {
             ret = matmul_short_rounds(A, B, L, K, u.data() + Log2(L * N * M), v.data() + Log2(L * K), U + Log2(L * N * M), V + Log2(L * K), claim,

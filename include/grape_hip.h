@@ -136,6 +136,17 @@ int grape_fr_fold_from(uint32_t *d_out, const uint32_t *d_in, size_t N, const ui
                        grape_stream_t stream);
 int grape_fr_fold_i32(uint32_t *d_out, const int32_t *d_in, size_t N, const uint32_t *d_x, uint32_t c, uint32_t id, uint32_t gap,
                       grape_stream_t stream);
+/* One or two folds of tensors that do not overlap, side by side: passes of one kind share a launch.  A job folds t in place, or `from`
+ * or the integers `ints` (at most one of them given) into t, as the three calls above do. */
+typedef struct grape_fold_job {
+    uint32_t *t;
+    const uint32_t *from;
+    const int32_t *ints;
+    size_t N;
+    const uint32_t *x;
+    uint32_t c, id, gap;
+} grape_fold_job;
+int grape_fr_fold_pair(const grape_fold_job *jobs, uint32_t count, grape_stream_t stream);
 
 /* ------------------------------------------------------------------ sumcheck ----------------- */
 /*
