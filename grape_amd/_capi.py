@@ -56,6 +56,7 @@ SIGNATURES = {
     "grape_fr_fold_i32": [c_void_p, c_void_p, c_size_t, c_void_p, c_u32, c_u32, c_u32, c_void_p],
     "grape_fr_fold_from": [c_void_p, c_void_p, c_size_t, c_void_p, c_u32, c_u32, c_u32, c_void_p],
     "grape_fr_fold_pair": [c_void_p, c_u32, c_void_p],
+    "grape_fr_random": [c_void_p, c_size_t, ctypes.POINTER(c_u32), c_void_p],
     "grape_sumcheck_round2": [c_void_p, c_void_p, c_u32, c_u32, c_void_p, c_void_p, c_void_p],
     "grape_sumcheck_round2_claim": [c_void_p, c_void_p, c_u32, c_u32, c_void_p, c_void_p, c_void_p, c_void_p],
     "grape_sumcheck_round2_noalloc": [c_void_p, c_void_p, c_u32, c_u32, c_void_p, c_void_p, c_void_p],

@@ -98,6 +98,16 @@ void Fr::seed_from_os() {
 }
 bool Fr::seeded() { return g_seeded.load(std::memory_order_acquire); }
 
+bool Fr::draw_key(uint32_t key[8]) {
+    if (seeded()) return false;
+    for (int i = 0; i < 4; i++) {
+        const uint64_t w = os_random64();
+        key[2 * i] = (uint32_t)w;
+        key[2 * i + 1] = (uint32_t)(w >> 32);
+    }
+    return true;
+}
+
 Fr Fr::random_element() {
     for (;;) {
         fr_t raw;

@@ -37,6 +37,9 @@ public:
     static void seed(uint64_t s);
     static void seed_from_os();
     static bool seeded();
+    // a key of 256 bits from the system's generator for grape_fr_random, to be used once; false (and no key) while the
+    // process is seeded: then elements come from the reproducible stream, one by one
+    static bool draw_key(uint32_t key[8]);
 
     bool is_zero() const { return v.is_zero(); }
     Fr& invert();                       // in place, 1/0 = 0; returns *this like libff

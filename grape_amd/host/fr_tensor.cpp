@@ -210,11 +210,20 @@ FrTensor& FrTensor::operator*=(fr_t* x) {
 FrTensor& FrTensor::operator*=(const uint x) { return *this *= grape_host::device_scalar(Fr((long)x)); }
 FrTensor& FrTensor::operator*=(Fr& x) { return *this *= grape_host::device_scalar(x); }
 
-FrTensor FrTensor::random(uint size) {
+FrTensor FrTensor::random_new(uint size, Memory memory) {
+    FrTensor out(size, memory);
+    uint32_t key[8];
+    if (Fr::draw_key(key)) {
+        check(grape_fr_random(W(out.gpu_data), size, key, nullptr), "grape_fr_random");
+        return out;
+    }
     std::vector<Fr> tmp(size);
     for (uint i = 0; i < size; i++) tmp[i] = Fr::random_element();
-    return from_host(tmp);
+    check(grape_memcpy_h2d(out.gpu_data, tmp.data(), sizeof(fr_t) * (size_t)size, nullptr), "grape_memcpy_h2d");
+    return out;
 }
+FrTensor FrTensor::random(uint size) { return random_new(size, kOrdinary); }
+FrTensor FrTensor::random(uint size, OnDefaultStream) { return random_new(size, kOnDefaultStream); }
 FrTensor FrTensor::fold_new(const fr_t* field, const int* ints, uint N, fr_t* x, uint c, uint id, uint gap, Memory memory) {
     const size_t elems = grape_fr_fold_i32_elems(N, c, gap);
     FrTensor out((uint)(elems ? elems : 1), memory);

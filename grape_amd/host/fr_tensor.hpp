@@ -84,6 +84,7 @@ public:
     FrTensor& operator*=(Fr& x);
 
     static FrTensor random(uint size);
+    static FrTensor random(uint size, grape_host::OnDefaultStream);
 
     // additions: an integer tensor folded or evaluated as the tensor get_data would make of it, without making
     // it (the first pass reads the integers): partial_eval(N, x, c, id, gap) of that tensor, compacted, and
@@ -102,6 +103,7 @@ public:
 private:
     enum Memory { kOrdinary, kOnDefaultStream };
     FrTensor(uint size, Memory memory);
+    static FrTensor random_new(uint size, Memory memory);
     static FrTensor fold_new(const fr_t* field, const int* ints, uint N, fr_t* x, uint c, uint id, uint gap, Memory memory);
     uint capacity_;
     Memory memory_;

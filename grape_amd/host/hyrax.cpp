@@ -65,6 +65,7 @@ Hyrax::~Hyrax() {
     grape_free(int16x2_table_.d);
     grape_free(int32_table_.d);
     grape_free(fr_table_.d);
+    grape_free(row_table_.d);
     grape_free(fr_strided_.d);
 }
 
@@ -176,7 +177,7 @@ size_t Hyrax::strided_bytes() const {
 // without a strided table that gives way (make_room)
 size_t Hyrax::table_bytes_in_use() const {
     size_t used = scaled_bytes_;
-    for (const WideTable* t : {&int16_table_, &int16x2_table_, &int32_table_, &fr_table_})
+    for (const WideTable* t : {&int16_table_, &int16x2_table_, &int32_table_, &fr_table_, &row_table_})
         if (t->d) used += grape_g1_wide_table_bytes(t->ngen, t->nw, t->K);
     return fr_strided_.spare ? used : used + strided_bytes();
 }
@@ -279,13 +280,29 @@ bool Hyrax::ensure_strided_table(uint rowlen, bool build, const double* worth_ms
     return true;
 }
 
+// A single row (an opening's blinding row, the z of its check) is a short accumulation and a chain: through a per-window table, which
+// leaves no doublings, where there is one.  A strided table leaves (J - 1) c of them and the reference-format table 248, one
+// after the other on four lanes, 4.5 us each (4096 columns, whole openings: 0.4 and 1.5 ms against 0.3).  So once an object's
+// single rows have spent on doublings what a small table takes to make - 8-bit windows, 2 GiB and 3 ms for 4096 generators - it is
+// made; wider rows than 8192 would take more memory than an opening is worth.
+const Hyrax::WideTable* Hyrax::single_row_table(uint rowlen, void* stream) {
+    if (ensure_fr_table(rowlen, false)) return &fr_table_;
+    constexpr uint c = 8, nw = 32, K = 128;
+    if (row_table_.d && row_table_.ngen >= rowlen) return &row_table_;
+    const size_t bytes = grape_g1_wide_table_bytes(rowlen, nw, K);
+    if (rowlen > npoints || bytes > (size_t)4 << 30) return nullptr;
+    const bool strided = fr_strided_.d && fr_strided_.ngen >= rowlen;
+    row_saving_ms_ += 4.5e-3 * (strided ? (fr_strided_.J - 1) * fr_strided_.c : 248);
+    if (row_saving_ms_ < 0.2 + 1.35e-9 * (double)bytes || !ensure_table(row_table_, rowlen, c, nw, K)) return nullptr;
+    row_saving_ms_ = 0;
+    if (stream) check(grape_stream_sync(nullptr), "sync");      // made on the default stream: another may read it only once it is there
+    return &row_table_;
+}
+
 bool Hyrax::commit_fr_rows(affine_t* out, fr_t* scalars, size_t size, uint rowlen, bool may_build, void* stream, int* d_flag) {
-    // one row only (an opening's blinding row): a table that is already there is used, none is built for it,
-    // and the per-window table is preferred - its 20 additions per scalar are nothing for one row, while the
-    // strided table's (J-1)*c doublings per row are a chain (4096 columns: 0.23 against 0.34 ms, the byte windows 1.26)
-    const bool single = size == rowlen;
-    if (single && ensure_fr_table(rowlen, false)) {
-        const WideTable& t = fr_table_;
+    const WideTable* own = size == rowlen ? single_row_table(rowlen, stream) : nullptr;
+    if (own) {
+        const WideTable& t = *own;
         if (d_flag) {
             check(grape_commit_fr_nowait(W(out), W(scalars), size, rowlen, W(t.d), t.ngen, t.c, t.nw, t.K, d_flag, stream), "grape_commit_fr_nowait");
             return true;
@@ -481,6 +498,44 @@ jacob_t* Hyrax::commit(FrTensor& tensor, uint size, uint N) {
     return to_jacobian(a, size / (N * com_scale));
 }
 
+namespace {
+// The commitment of a single row is a short accumulation and then a latency chain, so it runs on a stream of its own beside
+// what the default stream works on.  The row is made or uploaded on the default stream; nothing may write to it until wait().
+struct SideRow {
+    static grape_stream_t stream;                 // lives as long as the process, like the event
+    static void* row_there;
+    struct Result { affine_t p; int flag[4]; };
+    static_assert(sizeof(Result) == sizeof(affine_t) + 16, "point and flag travel together");
+    Result* d = nullptr;
+    bool open = false;
+    SideRow() {
+        if (!stream) {
+            check(grape_stream_create(&stream), "grape_stream_create");
+            check(grape_stream_internal(stream), "grape_stream_internal");
+            check(grape_event_create(&row_there), "grape_event_create");
+        }
+        check(grape_event_record(row_there, nullptr), "grape_event_record");        // a short row travels as a queued launch
+        check(grape_stream_wait_event(stream, row_there), "grape_stream_wait_event");
+        check(grape_malloc((void**)&d, sizeof(Result)), "grape_malloc");
+        open = true;
+        check(grape_memset_zero(d->flag, sizeof(int), stream), "grape_memset_zero");
+    }
+    ~SideRow() {
+        if (open) grape_stream_sync(stream);      // left by an exception: nothing the stream still reads is freed under it
+        grape_free(d);
+    }
+    affine_t wait(bool flag_used) {
+        Result h;
+        check(grape_memcpy_d2h(&h, d, sizeof h, stream), "d2h");
+        open = false;
+        if (flag_used && h.flag[0]) throw std::runtime_error("Hyrax: a scalar of a single row does not fit the table's digit range");
+        return h.p;
+    }
+};
+grape_stream_t SideRow::stream = nullptr;
+void* SideRow::row_there = nullptr;
+}  // namespace
+
 // Hyrax::open, src/Hyrax.cu:237-305: fold the tensor down to one row x of length new_N at the
 // outer variables of the point, blind it as z = c*x + d with a random row d, commit d, and send
 // <a,d>*G where a is the eq-vector of the inner variables.
@@ -500,35 +555,12 @@ Hyrax_proof Hyrax::open_impl(FrTensor* tensor_in, const int* ints, const std::ve
     last_open_point_ = eval_point_;
     fr_t* eval_point = grape_host::upload(eval_point_, OnDefaultStream());
 
-    std::vector<Fr> host_d(new_N);
-    for (uint i = 0; i < new_N; i++) host_d[i] = Fr::random_element();
-    FrTensor d = FrTensor::from_host(host_d, OnDefaultStream());
+    FrTensor d = FrTensor::random(new_N, OnDefaultStream());
 
-    // commitment of d: one row of new_N full-width scalars (single_commit, src/Hyrax.cu:176-185).  A short
-    // accumulation and then a latency chain (the row's reduction), so it runs on a stream of its own beside the folds
-    // of the tensor below; nothing below writes to d.
-    static grape_stream_t open_stream = nullptr;      // lives as long as the process
-    static void* d_uploaded = nullptr;
-    if (!open_stream) {
-        check(grape_stream_create(&open_stream), "grape_stream_create");
-        check(grape_stream_internal(open_stream), "grape_stream_internal");
-        check(grape_event_create(&d_uploaded), "grape_event_create");
-    }
-    // left by an exception: nothing the stream still reads is freed under it
-    struct Join {
-        bool open = true;
-        ~Join() { if (open) grape_stream_sync(open_stream); }
-    } join;
-    check(grape_event_record(d_uploaded, nullptr), "grape_event_record");        // a short d travels as a queued launch
-    check(grape_stream_wait_event(open_stream, d_uploaded), "grape_stream_wait_event");
-    // (the point and, behind it, the digit-range flag of a commitment queued without waiting)
-    affine_t* com_d_dev = nullptr;
-    check(grape_malloc((void**)&com_d_dev, sizeof(affine_t) + 16), "grape_malloc");
-    int* d_flag = reinterpret_cast<int*>(com_d_dev + 1);
-    check(grape_memset_zero(d_flag, sizeof(int), open_stream), "grape_memset_zero");
-    const bool flag_used = commit_fr_rows(com_d_dev, d.gpu_data, new_N, new_N, false, open_stream, d_flag);
+    // commitment of d (single_commit, src/Hyrax.cu:176-185) beside the folds of the tensor below, which do not write to d
+    SideRow com_d;
+    const bool flag_used = commit_fr_rows(&com_d.d->p, d.gpu_data, new_N, new_N, false, SideRow::stream, com_d.d->flag);
 
-    FrTensor x(new_N, OnDefaultStream());
     std::unique_ptr<FrTensor> rows_of_ints;
     if (ints) {
         rows_of_ints.reset(new FrTensor(FrTensor::folded_from_ints(ints, size, eval_point, (size / layer_num) / (N * com_scale),
@@ -538,36 +570,39 @@ Hyrax_proof Hyrax::open_impl(FrTensor* tensor_in, const int* ints, const std::ve
     }
     FrTensor& tensor = ints ? *rows_of_ints : *tensor_in;
     tensor.partial_eval((N * com_scale) * layer_num, eval_point, layer_num, Log2(size / layer_num), N * com_scale);
-    x = tensor;
-    if (pad_N != N) x.pad(tensor, N, pad_N, new_N, Fr::zero());
-
-    tensor.partial_eval(new_N, eval_point, new_N, 0, 1);
-    Fr result = grape_host::download(tensor.gpu_data);
-
-    FrTensor z(new_N, OnDefaultStream());
-    z = x;
-    z *= c;
-    z += d;
-
-    FrTensor d_fold(d, OnDefaultStream());                         // folded in place: a copy, the commitment may still be reading d
-    d_fold.partial_eval(d_fold.size, eval_point, new_N, 0, 1);
-    Fr sum_ad = grape_host::download(d_fold.gpu_data);
-    bn128 commit_ad = multiple_of_G(sum_ad);
-
-    struct { affine_t p; int flag[4]; } com_d_host;
-    static_assert(sizeof(com_d_host) == sizeof(affine_t) + 16, "point and flag travel together");
-    check(grape_memcpy_d2h(&com_d_host, com_d_dev, sizeof(com_d_host), open_stream), "d2h");     // waits for the commitment
-    join.open = false;
-    if (flag_used && com_d_host.flag[0]) {
-        grape_free(com_d_dev);
-        grape_free_on_default(eval_point);
-        throw std::runtime_error("Hyrax::open: a blinding scalar does not fit the table's digit range");
+    // x, the row that is left (padded): a copy where the tensor is the caller's, which is bound to its last element
+    std::unique_ptr<FrTensor> row;
+    if (!ints || pad_N != N) {
+        row.reset(new FrTensor(new_N, OnDefaultStream()));
+        *row = tensor;
+        if (pad_N != N) row->pad(tensor, N, pad_N, new_N, Fr::zero());
     }
-    const affine_t& host_com_d = com_d_host.p;
-    Hyrax_proof proof(result, new_N, bn128(host_com_d), commit_ad);
-    check(grape_memcpy_d2h(proof.z, z.gpu_data, sizeof(fr_t) * (size_t)new_N, nullptr), "d2h");
-    grape_free(com_d_dev);
+    const FrTensor& x = row ? *row : tensor;
+
+    // z = c x + d, and behind it <a, x> and <a, d>: two evaluations at the inner variables side by side, read with z by one copy
+    const size_t behind = grape_fr_fold_i32_elems(new_N, new_N, 1);
+    FrTensor z((uint)(new_N + 2 * behind), OnDefaultStream());
+    const fr_t* const at_x = z.gpu_data + new_N;
+    grape_fold_job folds[2] = {};
+    for (uint k = 0; k < 2; k++) {
+        folds[k].t = W(z.gpu_data + new_N + k * behind);
+        folds[k].from = W(k ? d.gpu_data : x.gpu_data);
+        folds[k].N = folds[k].c = new_N;
+        folds[k].x = W(eval_point);
+        folds[k].gap = 1;
+    }
+    check(grape_fr_fold_pair(folds, 2, nullptr), "grape_fr_fold_pair");
+    check(grape_fr_axpy(W(z.gpu_data), W(d.gpu_data), W(grape_host::device_scalar(c)), W(x.gpu_data), new_N, nullptr), "grape_fr_axpy");
+    if (!ints) check(grape_memcpy_d2d(tensor.gpu_data, at_x, sizeof(fr_t), nullptr), "grape_memcpy_d2d");
+    std::vector<Fr> zs(new_N + behind + 1);
+    check(grape_memcpy_d2h(zs.data(), z.gpu_data, sizeof(fr_t) * zs.size(), nullptr), "d2h");
+    const Fr result = zs[new_N];
+    bn128 commit_ad = multiple_of_G(zs[new_N + behind]);
+
+    const affine_t host_com_d = com_d.wait(flag_used);
     grape_free_on_default(eval_point);
+    Hyrax_proof proof(result, new_N, bn128(host_com_d), commit_ad);
+    std::copy(zs.begin(), zs.begin() + new_N, proof.z);
     return proof;
 }
 
@@ -578,6 +613,11 @@ bool Hyrax::verify(Hyrax_proof& proof, jacob_t* commitment, const std::vector<Fr
     const uint rows = size / rowlen;
     const uint new_N = (uint)proof.z_size;
     const uint inner = Log2(rowlen);
+    // com(z) beside everything else
+    std::vector<Fr> zv(proof.z, proof.z + new_N);
+    FrTensor z = FrTensor::from_host(zv, OnDefaultStream());
+    SideRow com_z_row;
+    const bool flag_used = commit_fr_rows(&com_z_row.d->p, z.gpu_data, new_N, new_N, false, SideRow::stream, com_z_row.d->flag);
     // c * C, C the row commitments folded at the outer variables: sum_i c eq(outer, i) C_i, its window sums on the device
     // and their doubling chain here.  (Folding fewer variables than the rows need leaves the first 2^variables rows; each
     // variable beyond them finds the rows above missing, a factor 1 - u, and needs no table.)
@@ -591,30 +631,31 @@ bool Hyrax::verify(Hyrax_proof& proof, jacob_t* commitment, const std::vector<Fr
     grape_free_on_default(d_outer);
     fr_t* const weights = pyramid.gpu_data + (((size_t)1 << outer.size()) - 1);
     check(grape_fr_bcast_mul(W(weights), W(weights), W(grape_host::device_scalar(scale)), (size_t)1 << outer.size(), nullptr), "grape_fr_bcast_mul");
-    bucket_t* d_windows = nullptr;
-    check(grape_malloc_on_default((void**)&d_windows, sizeof(bucket_t) * GRAPE_MSM_WINDOWS), "grape_malloc");
-    check(grape_g1_msm_windows(W(d_windows), W(commitment), W(weights), used, nullptr), "grape_g1_msm_windows");
-    // com(z) on the device
-    std::vector<Fr> zv(proof.z, proof.z + new_N);
-    FrTensor z = FrTensor::from_host(zv, OnDefaultStream());
-    affine_t* com_z_dev = nullptr;
-    check(grape_malloc_on_default((void**)&com_z_dev, sizeof(affine_t)), "grape_malloc");
-    commit_fr_rows(com_z_dev, z.gpu_data, new_N, new_N, false);
-    std::vector<bucket_t> windows(GRAPE_MSM_WINDOWS);
-    affine_t com_z;
-    check(grape_memcpy_d2h(windows.data(), d_windows, sizeof(bucket_t) * windows.size(), nullptr), "grape_memcpy_d2h");
-    check(grape_memcpy_d2h(&com_z, com_z_dev, sizeof(affine_t), nullptr), "d2h");
-    grape_free_on_default(com_z_dev);
-    grape_free_on_default(d_windows);
-    bucket_t cC = windows[GRAPE_MSM_WINDOWS - 1];
+    // the window sums and behind them <a, z>, read by one copy
+    struct { bucket_t windows[GRAPE_MSM_WINDOWS]; Fr az; } got;
+    static_assert(sizeof(got) == sizeof(bucket_t) * GRAPE_MSM_WINDOWS + sizeof(Fr), "read as it lies there");
+    std::vector<Fr> inner_point(eval_point.begin(), eval_point.begin() + inner);
+    const bool plain = ((uint64_t)1 << inner) == new_N;
+    const size_t behind = plain ? grape_fr_fold_i32_elems(new_N, new_N, 1) : 0;
+    char* d_got = nullptr;
+    check(grape_malloc_on_default((void**)&d_got, sizeof(got.windows) + sizeof(Fr) * (behind + 1)), "grape_malloc");
+    check(grape_g1_msm_windows(W(d_got), W(commitment), W(weights), used, nullptr), "grape_g1_msm_windows");
+    if (plain) {
+        fr_t* d_inner = grape_host::upload(inner_point, OnDefaultStream());
+        check(grape_fr_fold_from(W(d_got + sizeof(got.windows)), W(z.gpu_data), new_N, W(d_inner), new_N, 0, 1, nullptr), "grape_fr_fold_from");
+        grape_free_on_default(d_inner);
+    }
+    check(grape_memcpy_d2h(&got, d_got, plain ? sizeof(got) : sizeof(got.windows), nullptr), "grape_memcpy_d2h");
+    grape_free_on_default(d_got);
+    bucket_t cC = got.windows[GRAPE_MSM_WINDOWS - 1];
     for (int w = GRAPE_MSM_WINDOWS - 2; w >= 0; w--) {
         for (int d = 0; d < 4; d++) grape::xyzz_dbl(cC);
-        grape::xyzz_add(cC, windows[w]);
+        grape::xyzz_add(cC, got.windows[w]);
     }
+    const affine_t com_z = com_z_row.wait(flag_used);
     if (!(bn128(grape::xyzz_to_jac(cC)) + proof.commit_d == bn128(com_z))) return false;
     // (c * result) * G + commit_ad == az * G, with one multiple of G
-    std::vector<Fr> inner_point(eval_point.begin(), eval_point.begin() + inner);
-    Fr az = z(inner_point);
+    const Fr az = plain ? got.az : z(inner_point);
     return proof.commit_ad == multiple_of_G(az - c * proof.result);
 }
 

@@ -118,6 +118,8 @@ private:
     };
     bool ensure_table(WideTable& t, uint rowlen, uint c, uint nw, uint K);
     bool ensure_fr_table(uint rowlen, bool build = true);       // small per-window table (scaled-table builds)
+    const WideTable* single_row_table(uint rowlen, void* stream);
+    double row_saving_ms_ = 0;                                  // what a table for single rows would have saved so far
     bool ensure_strided_table(uint rowlen, bool build = true, const double* worth_ms = nullptr);  // the table full-width commitments go through
     size_t table_bytes_in_use() const;
     size_t strided_bytes() const;
@@ -131,7 +133,7 @@ private:
     void commit_i32_rows(affine_t* out, int* tensor, size_t size, uint rowlen, int* d_flag, void* stream = nullptr);
     void check_shape(uint size, uint N) const;
     bn128 multiple_of_G(const Fr& k);
-    WideTable int16_table_, int16x2_table_, int32_table_, fr_table_;
+    WideTable int16_table_, int16x2_table_, int32_table_, fr_table_, row_table_;
     StridedTable fr_strided_;
     bool int16_ok_ = true;
     size_t scaled_bytes_ = 0;

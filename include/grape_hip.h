@@ -147,6 +147,10 @@ typedef struct grape_fold_job {
     uint32_t c, id, gap;
 } grape_fold_job;
 int grape_fr_fold_pair(const grape_fold_job *jobs, uint32_t count, grape_stream_t stream);
+/* n uniformly random elements, a function of the key (HOST, eight words; the caller draws it from a source fit for blinding and uses
+ * it once): ChaCha20 (RFC 8439) with the element's index as nonce, candidates that are not below the modulus passed over.  What
+ * FrTensor::random (include/fr-tensor.cuh:36-76) is made of. */
+int grape_fr_random(uint32_t *d_out, size_t n, const uint32_t *key, grape_stream_t stream);
 
 /* ------------------------------------------------------------------ sumcheck ----------------- */
 /*
