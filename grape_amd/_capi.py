@@ -96,6 +96,7 @@ SIGNATURES = {
     "grape_carried_halves": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_u32, c_void_p],
     "grape_carried_partial_bytes": [c_void_p],
     "grape_carried_queue": [c_void_p, c_void_p],
+    "grape_carried_queue_pair": [c_void_p, c_void_p, c_void_p],
     "grape_carried_finish": [c_void_p, c_u32, c_void_p, c_u32, c_void_p],
     "grape_carried_end": [c_void_p, c_void_p, c_u32, c_void_p, c_u32, c_void_p, c_void_p],
     "grape_wround_queue_gathered": [c_void_p, c_void_p, c_void_p],

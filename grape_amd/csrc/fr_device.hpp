@@ -100,6 +100,66 @@ __device__ __forceinline__ Fr foldt1(const int32_t* tab, const fr26::Limbs& lo, 
     return fr26::foldt_finish(c);
 }
 
+// foldt1 for a value that is folded again at once: working limbs congruent to lo + v * d, not reduced below r.  The two Montgomery
+// steps take digits in [-2^25, 2^25), so the result lies within r / 2 (and 2^-22 r) of lo; limbs 0..8 normalised, the top one signed.
+__device__ __forceinline__ fr26::Limbs foldt1_limbs(const int32_t* tab, const fr26::Limbs& lo, const fr26::Limbs& d) {
+    constexpr int N = fr26::N, W = fr26::W;
+    int64_t c[N + 2];
+    c[0] = c[1] = 0;
+#pragma unroll
+    for (int k = 0; k < N; k++) c[k + 2] = (int64_t)lo.v[k];
+    FoldTabPtr row[N];
+#pragma unroll
+    for (int j = 0; j < N; j++) row[j] = (FoldTabPtr)(uintptr_t)(tab + j * N);
+    asm volatile("" : "+s"(row[0]), "+s"(row[1]));
+#pragma unroll
+    for (int j = 0; j < N; j++) {
+#pragma unroll
+        for (int k = 0; k < N; k++) c[k] += (int64_t)d.v[j] * (int64_t)row[j][k];
+        if (j + 2 < N) asm volatile("" : "+s"(row[j + 2]) : "v"((uint32_t)c[0]));
+    }
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const int32_t m = (int32_t)((0u - (uint32_t)c[i]) << (32 - W)) >> (32 - W);
+        c[i] += (int64_t)m;
+#pragma unroll
+        for (int j = 1; j < N; j++) c[i + j] += (int64_t)m * (int64_t)fr26::R(j);
+        c[i + 1] += c[i] >> W;
+    }
+    fr26::Limbs r;
+    int64_t carry = 0;
+#pragma unroll
+    for (int k = 0; k < N - 1; k++) {
+        const int64_t t = c[2 + k] + carry;
+        r.v[k] = (int32_t)((uint32_t)t & fr26::MASK);
+        carry = t >> W;
+    }
+    r.v[N - 1] = (int32_t)(c[N + 1] + carry);
+    return r;
+}
+
+// The table fold with a table in LDS, where the lanes of a wave fold by different challenges: ten rows of kFoldLdsRow words, sixteen-byte
+// aligned.  lo may be what foldt1_limbs gave: for lo within (-r / 2, 2 r) the value before the last step is within (r / 2, 4 r).
+constexpr int kFoldLdsRow = 12;
+__device__ __forceinline__ Fr foldt_lds(const int32_t* tab, const fr26::Limbs& lo, const fr26::Limbs& d) {
+    constexpr int N = fr26::N;
+    int64_t c[N + 2];
+    c[0] = c[1] = 0;
+#pragma unroll
+    for (int k = 0; k < N; k++) c[k + 2] = (int64_t)lo.v[k];
+#pragma unroll
+    for (int j = 0; j < N; j++) {
+        const int4* q = reinterpret_cast<const int4*>(tab + j * kFoldLdsRow);
+        const int4 x = q[0], y = q[1];
+        const int2 z = *reinterpret_cast<const int2*>(q + 2);
+        const int32_t w[N] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w, z.x, z.y};
+#pragma unroll
+        for (int k = 0; k < N; k++) c[k] += (int64_t)d.v[j] * (int64_t)w[k];
+
+    }
+    return fr26::foldt_finish(c);
+}
+
 // The ten multiples of a round's challenge that the table fold multiplies by (fr26::fold_table), for
 // `count` <= 64 challenges: thread t writes the table of v[t] at tabs + 100 t.  (static: every
 // source file that launches it gets its own copy)

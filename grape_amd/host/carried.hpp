@@ -12,6 +12,7 @@
 #pragma once
 #include <array>
 #include <vector>
+#include "../../include/grape_hip.h"
 #include "fr.hpp"
 
 struct CarriedFactors {
@@ -84,6 +85,17 @@ struct CarriedFactors {
         const Fr at_v = next0 + un * (next1 - next0);
         const Fr top = (q0 + (q1 - q0) * v - at_v) * inv_v[k] * inv_1v[k];
         return {q0, q1 - q0 - top, top};
+    }
+
+    // The rounds run two to a pass, an odd one's last alone.
+    static uint32_t place_in_pass(unsigned i, unsigned rounds) {
+        return i % 2 ? GRAPE_CARRIED_SECOND : i + 1 < rounds ? GRAPE_CARRIED_FIRST : GRAPE_CARRIED_SINGLE;
+    }
+    static void queue_passes(const grape_carried_args* a, unsigned rounds, grape_stream_t st) {
+        for (unsigned i = 0; i < rounds; i++) {
+            if (a[i].pair == GRAPE_CARRIED_SINGLE) grape_host::check(grape_carried_queue(&a[i], st), "grape_carried_queue");
+            if (a[i].pair == GRAPE_CARRIED_FIRST) grape_host::check(grape_carried_queue_pair(&a[i], &a[i + 1], st), "grape_carried_queue_pair");
+        }
     }
 
 private:

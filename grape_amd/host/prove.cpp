@@ -381,11 +381,14 @@ static Fr eleMul_rounds(fr_t* Aw, fr_t* Bw, const fr_t* A, const fr_t* B, fr_t* 
             a.n_out = out;
             a.tab_a = static_cast<int32_t*>(tabs->p) + (size_t)GRAPE_FOLD_TABLE_WORDS * (rounds - 1 - i);
             a.tab_z = static_cast<int32_t*>(ratio_tabs->p) + (size_t)GRAPE_FOLD_TABLE_WORDS * i;
-            partials.emplace_back(new DeviceBuf(grape_carried_partial_bytes(&a)));
-            a.partial = W(partials.back()->fr());
-            check(grape_carried_queue(&a, nullptr), "grape_carried_queue");
             carried.push_back(a);
         }
+        for (uint i = 0; i < carrying; i++) {
+            carried[i].pair = CarriedFactors::place_in_pass(i, carrying);
+            partials.emplace_back(new DeviceBuf(grape_carried_partial_bytes(&carried[i])));
+            carried[i].partial = W(partials.back()->fr());
+        }
+        CarriedFactors::queue_passes(carried.data(), carrying, nullptr);
         check(grape_carried_finish(W(sums.gpu_data), 3, carried.data(), carrying, nullptr), "grape_carried_finish");
         check(grape_carried_end(W(Bw), W(Bw), in, W(consts->fr() + carrying), period, nullptr, nullptr), "grape_carried_end");
         if (in == second_size) out = 1u << (Log2(in) - 1);     // a row's own variables: those of its padded length

@@ -758,7 +758,10 @@ Fr tLookup::run(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax& hyrax
             carried[0].len = N;
             carried[0].eq_high = plan.high_level(E.gpu_data, nu - 1 - GRAPE_EQ_SPLIT_LOW);
             need = 0;
-            for (const grape_carried_args& b : carried) need += grape_carried_partial_bytes(&b);
+            for (uint i = 0; i < (uint)carried.size(); i++) {
+                carried[i].pair = CarriedFactors::place_in_pass(i, (uint)carried.size());
+                need += grape_carried_partial_bytes(&carried[i]);
+            }
             // the ratios' tables and the two multiples of every table entry
             ratio_tabs.reset(new FrTensor((uint)((sizeof(int32_t) * GRAPE_FOLD_TABLE_WORDS * carried.size() + sizeof(fr_t) - 1) / sizeof(fr_t)), OnDefaultStream()));
             consts.reset(new FrTensor((uint)carried.size() + 1, OnDefaultStream()));
@@ -779,9 +782,9 @@ Fr tLookup::run(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax& hyrax
                 b.tab_z = tabs + GRAPE_FOLD_TABLE_WORDS * i;
                 b.partial = reinterpret_cast<uint32_t*>(long_work + long_used);
                 long_used += grape_carried_partial_bytes(&b);
-                check(grape_carried_queue(&b, nullptr), "grape_carried_queue");
                 cur /= 2;
             }
+            CarriedFactors::queue_passes(carried.data(), (uint)carried.size(), nullptr);
             grape_stream_t fs = nullptr;
             if (overlap) {
                 witness.after(nullptr);

@@ -323,11 +323,19 @@ typedef struct {
     const int32_t *tab_a, *tab_z;
     int plain_sums;
     uint32_t *partial;
+    uint32_t pair;             /* GRAPE_CARRIED_SINGLE, or which round of a pass over two it is */
 } grape_carried_args;
+#define GRAPE_CARRIED_SINGLE 0u
+#define GRAPE_CARRIED_FIRST 1u
+#define GRAPE_CARRIED_SECOND 2u
 int grape_carried_halves(uint32_t *d_halves, const uint32_t *d_B, const uint32_t *d_T, const uint32_t *d_beta, const uint32_t *d_v, uint32_t len,
                          grape_stream_t stream);
 size_t grape_carried_partial_bytes(const grape_carried_args *args);
 int grape_carried_queue(const grape_carried_args *args, grape_stream_t stream);
+/* Two consecutive rounds in one pass: `first` (of any kind) and the later round behind it, whose sums are those that two calls of
+ * grape_carried_queue give.  first->A_out and Z_out and second->A and Z are not used: what the first round folds is not written.
+ * Both have their own partial and are marked in `pair`, also for grape_carried_partial_bytes and grape_carried_finish. */
+int grape_carried_queue_pair(const grape_carried_args *first, const grape_carried_args *second, grape_stream_t stream);
 /* finishes `count` <= 32 rounds of one kind; round i's sums go to element i * stride of d_sums */
 int grape_carried_finish(uint32_t *d_sums, uint32_t stride, const grape_carried_args *rounds, uint32_t count, grape_stream_t stream);
 /* S back from what is left of Z: out[i] = Z[i] factor[i / period] - beta (beta may be NULL; out may be Z) */
