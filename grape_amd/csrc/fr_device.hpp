@@ -160,11 +160,24 @@ __device__ __forceinline__ Fr foldt_lds(const int32_t* tab, const fr26::Limbs& l
     return fr26::foldt_finish(c);
 }
 
-// The ten multiples of a round's challenge that the table fold multiplies by (fr26::fold_table), for
-// `count` <= 64 challenges: thread t writes the table of v[t] at tabs + 100 t.  (static: every
-// source file that launches it gets its own copy)
+// The ten multiples of a round's challenge that the table fold multiplies by (fr26::fold_table), for `count` <= 64 challenges: workgroup
+// t makes the table of v[t] at tabs + 100 t, a thread a row.  A row is two dependent products from v where the rows one after the other
+// are twelve (11 -> 5 us, on the chain before the first long round): up to j = 7 the factor 2^(26 j + 52) is below r as it
+// stands, the last two rows go through row 7.  (static: every source file that launches it gets its own copy)
 static __global__ void __launch_bounds__(64) fold_tables_kernel(int32_t* tabs, const uint32_t* v, uint32_t count) {
-    if (threadIdx.x < count) fr26::fold_table(tabs + (size_t)fr26::kFoldTableWords * threadIdx.x, ld_fr(v, threadIdx.x));
+    const uint32_t j = threadIdx.x;
+    if (blockIdx.x >= count || j >= (uint32_t)fr26::N) return;
+    const uint32_t e = 26 * (j < 7 ? j : 7) + 52, rest = j < 7 ? 0 : 26 * (j - 7);
+    Fr p = Fr::zero(), q = Fr::zero();
+#pragma unroll
+    for (uint32_t i = 0; i < 8; i++) {
+        p.v[i] = e >> 5 == i ? 1u << (e & 31) : 0;
+        q.v[i] = rest >> 5 == i ? 1u << (rest & 31) : 0;
+    }
+    const fr26::Limbs l = fr26::pack(fr26::mulc(fr26::mulc(ld_fr(v, blockIdx.x), p), fr26::to_montc(q)));
+    int32_t* row = tabs + (size_t)fr26::kFoldTableWords * blockIdx.x + j * fr26::N;
+#pragma unroll
+    for (int k = 0; k < fr26::N; k++) row[k] = l.v[k];
 }
 // Rounds of at least this many output indices fold through the table of the challenge's multiples
 // (one more small launch per round); shorter rounds are launch-bound and keep the single product.

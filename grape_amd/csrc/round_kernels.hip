@@ -11,34 +11,62 @@
 namespace grape {
 
 // ---------------------------------------------------------------- eq pyramid
-// Level j (2^j entries) sits at element offset 2^j - 1; level j holds eq(u[0..j-1], i), bit b of i
-// paired with u[b].  Level j+1 from level j: hi = lo * u[j], lo' = lo - hi.
-constexpr uint32_t kPyrHeadLevels = 9;   // levels 0..9 built by one workgroup (512 threads' worth at the top)
+// Level j (2^j entries) sits at element offset 2^j - 1; level j holds eq(u[0..j-1], i), bit b of i paired with u[b].
+// Level by level (hi = lo * u[j], lo' = lo - hi) a pyramid is a chain of launches, one for each level above 9, before a proof's
+// first round.  Here every level is made at once, in one launch: a workgroup takes a head of 2^11 entries of a level that share their
+// high bits, an entry is the product of a factor over bits 0..4, one over bits 5..10 and the head's own, and those are
+// products of at most 6 (3 deep; 19 for the head, a tree over the lanes) factors u or 1 - u, made by different waves side by
+// side.  One product an entry as before.  Bound by its chain of about 14 products below 2^16 entries, by issue above: 2^13 entries
+// 26 -> 13 us and 5 -> 1 launches, 2^16 40 -> 13.5 and 8 -> 1, 2^20 73 -> 42 and 12 -> 1.
+constexpr uint32_t kPyrLow = 5, kPyrHead = 11;
 
-__global__ void __launch_bounds__(kBlock) eq_pyramid_head_kernel(uint32_t* pyr, const uint32_t* u, uint32_t levels) {
-    if (threadIdx.x == 0) st_fr(pyr, 0, Fr::one());
-    __syncthreads();
-    for (uint32_t j = 0; j < levels; j++) {
-        const size_t half = (size_t)1 << j, src = half - 1, dst = 2 * half - 1;
-        const Fr uj = ld_fr(u, j);
-        for (size_t i = threadIdx.x; i < half; i += kBlock) {
-            const Fr lo = ld_fr(pyr, src + i);
-            const Fr hi = fr26::mulc(lo, uj);
-            st_fr(pyr, dst + i + half, hi);
-            st_fr(pyr, dst + i, sub(lo, hi));
-        }
-        __threadfence_block();
-        __syncthreads();
-    }
+// the factor of u[b] for bit `set`; one for a variable that is not there
+__device__ __forceinline__ Fr eq_factor(const uint32_t* u, uint32_t b, bool there, bool set) {
+    if (!there) return Fr::one();
+    const Fr x = ld_fr(u, b);
+    return set ? x : sub(Fr::one(), x);
 }
-__global__ void __launch_bounds__(kBlock) eq_pyramid_level_kernel(uint32_t* pyr, const uint32_t* u, uint32_t j) {
-    const size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x;
-    const size_t half = (size_t)1 << j;
-    if (i >= half) return;
-    const Fr lo = ld_fr(pyr, half - 1 + i);
-    const Fr hi = fr26::mulc(lo, ld_fr(u, j));
-    st_fr(pyr, 2 * half - 1 + i + half, hi);
-    st_fr(pyr, 2 * half - 1 + i, sub(lo, hi));
+// the product of n <= 6 of them from u[b] on for the bits of i, three products deep
+__device__ __forceinline__ Fr eq_factors(const uint32_t* u, uint32_t b, uint32_t n, uint32_t i) {
+    Fr x[3];
+#pragma unroll
+    for (uint32_t k = 0; k < 3; k++)
+        x[k] = fr26::mulc(eq_factor(u, b + 2 * k, 2 * k < n, (i >> 2 * k) & 1), eq_factor(u, b + 2 * k + 1, 2 * k + 1 < n, (i >> (2 * k + 1)) & 1));
+    return fr26::mulc(fr26::mulc(x[0], x[1]), x[2]);
+}
+__global__ void __launch_bounds__(kBlock) eq_pyramid_head_kernel(uint32_t* pyr, const uint32_t* u) {
+    __shared__ Fr low[1 << kPyrLow], mid[1 << (kPyrHead - kPyrLow)], high;
+    // workgroups 0..kPyrHead are the levels up to kPyrHead, 2^(level - kPyrHead) of them each level above
+    uint32_t level = blockIdx.x, h = 0;
+    if (level > kPyrHead) {
+        const uint32_t i = blockIdx.x - kPyrHead + 1, lg = 31 - __clz(i);      // 2, 3 | 4, 5, 6, 7 | ...
+        level = kPyrHead + lg;
+        h = i - (1u << lg);
+    }
+    const uint32_t t = threadIdx.x, wave = t >> 6, lane = t & 63;
+    const uint32_t nlow = level < kPyrLow ? level : kPyrLow, nhead = level < kPyrHead ? level : kPyrHead, nmid = nhead - nlow;
+    if (wave == 0) {
+        if (lane < (1u << nlow)) low[lane] = eq_factors(u, 0, nlow, lane);
+    } else if (wave == 1) {
+        if (lane < (1u << nmid)) mid[lane] = eq_factors(u, nlow, nmid, lane);
+    } else if (wave == 2) {
+        const uint32_t rest = level - nhead;                // at most 19 of 32 lanes
+        Fr x = eq_factor(u, kPyrHead + lane, lane < rest, (h >> (lane & 31)) & 1);
+        for (uint32_t off = 16; off >= 1; off >>= 1) {
+            if (off >= rest) continue;                      // the same for every lane
+            const Fr y = shfl_down_fr(x, off);
+            x = fr26::mulc(x, lane < off ? y : Fr::one());
+        }
+        if (lane == 0) high = x;
+    }
+    __syncthreads();
+    if (wave == 1 && level > kPyrHead) mid[lane] = fr26::mulc(mid[lane], high);
+    __syncthreads();
+    const size_t at = ((size_t)1 << level) - 1 + ((size_t)h << kPyrHead);
+    for (uint32_t i = t; i < (1u << nhead); i += kBlock) {
+        const Fr l = low[i & ((1u << nlow) - 1)];
+        st_fr(pyr, at + i, level > kPyrLow ? fr26::mulc(l, mid[i >> nlow]) : l);
+    }
 }
 
 // ---------------------------------------------------------------- weighted two-tensor round
@@ -335,9 +363,8 @@ int grape_eq_pyramid(uint32_t* pyr, const uint32_t* u, uint32_t nu, grape_stream
     GRAPE_REQUIRE(nu <= 30, "too many variables");
     if (nu) CHECK_PTR16(u);
     hipStream_t s = as_stream(st);
-    const uint32_t head = nu < kPyrHeadLevels ? nu : kPyrHeadLevels;
-    eq_pyramid_head_kernel<<<1, kBlock, 0, s>>>(pyr, u, head);
-    for (uint32_t j = head; j < nu; j++) eq_pyramid_level_kernel<<<blocks_for((size_t)1 << j), kBlock, 0, s>>>(pyr, u, j);
+    const unsigned nb = nu <= kPyrHead ? nu + 1 : kPyrHead - 1 + (1u << (nu - kPyrHead + 1));
+    eq_pyramid_head_kernel<<<nb, kBlock, 0, s>>>(pyr, u);
     GRAPE_LAUNCH_CHECK();
     return GRAPE_OK;
 }
@@ -466,7 +493,7 @@ int grape_fold_tables(int32_t* tabs, const uint32_t* v, uint32_t count, grape_st
     GRAPE_REQUIRE(tabs != nullptr && (reinterpret_cast<uintptr_t>(tabs) & 3) == 0, "tabs must be 4-byte aligned");
     GRAPE_REQUIRE(count >= 1 && count <= 64, "1..64 challenges");
     CHECK_PTR16(v);
-    fold_tables_kernel<<<1, 64, 0, as_stream(st)>>>(tabs, v, count);
+    fold_tables_kernel<<<count, 64, 0, as_stream(st)>>>(tabs, v, count);
     GRAPE_LAUNCH_CHECK();
     return GRAPE_OK;
 }

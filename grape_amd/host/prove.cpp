@@ -336,7 +336,6 @@ static Fr eleMul_rounds(fr_t* Aw, fr_t* Bw, const fr_t* A, const fr_t* B, fr_t* 
     const uint lg_row = Log2(second_size);
     const bool padded = second_size != row_pad;
     const uint low = padded ? lg_row : kSplitLow;
-    const EqWeights eq(u - rounds, rounds - 1, low, padded && lg_row > kLongestPrefix ? rounds : kLongestPrefix);
     FrTensor sums(3 * rounds + 2, OnDefaultStream());
     // the tables of all challenges' multiples, and every long round's partial sums until one launch finishes them all
     std::vector<grape_wround_args> queued;
@@ -358,11 +357,13 @@ static Fr eleMul_rounds(fr_t* Aw, fr_t* Bw, const fr_t* A, const fr_t* B, fr_t* 
     if (Aw != Bw && period >= kCarriedRow && period <= GRAPE_WROUND_MAX_PERIOD && size / 2 >= 1u << 20)
         for (uint n = size; n % 2 == 0 && n / 2 >= kLongRoundPairs && (n / 2) % period == 0; n /= 2) carrying++;
     const CarriedFactors factors(hu - rounds, hv - rounds, rounds, carrying, low);
+    const bool carry = factors.ok && carrying >= 2;
+    // carried rounds read the split tables alone, and the rounds behind them a prefix table of at most 2^kSplitLow entries or a split one;
+    // four rows and more leave variables above both
+    const EqWeights eq(u - rounds, rounds - 1, low, carry ? std::max(low, kSplitLow) : padded && lg_row > kLongestPrefix ? rounds : kLongestPrefix);
     std::vector<grape_carried_args> carried;
     std::unique_ptr<DeviceBuf> consts, ratio_tabs;
-    std::unique_ptr<EqPyramid> own_high;
-    if (factors.ok && carrying >= 2) {
-        if (!eq.high) own_high.reset(new EqPyramid(u - rounds + low, rounds - 1 - low));
+    if (carry) {
         std::vector<Fr> c(factors.ratio);
         c.insert(c.end(), factors.end.begin(), factors.end.end());
         consts.reset(new DeviceBuf(sizeof(fr_t) * c.size()));
@@ -376,7 +377,7 @@ static Fr eleMul_rounds(fr_t* Aw, fr_t* Bw, const fr_t* A, const fr_t* B, fr_t* 
             a.A = W(i ? Aw : A);
             a.Z = W(i ? Bw : B);
             a.eq = W(eq.prefix.level(low));
-            a.eq_high = i == 0 ? W((eq.high ? *eq.high : *own_high).level(rounds - 1 - low)) : nullptr;
+            a.eq_high = i == 0 ? W(eq.high->level(rounds - 1 - low)) : nullptr;
             a.period = period;
             a.n_out = out;
             a.tab_a = static_cast<int32_t*>(tabs->p) + (size_t)GRAPE_FOLD_TABLE_WORDS * (rounds - 1 - i);
@@ -388,8 +389,13 @@ static Fr eleMul_rounds(fr_t* Aw, fr_t* Bw, const fr_t* A, const fr_t* B, fr_t* 
             partials.emplace_back(new DeviceBuf(grape_carried_partial_bytes(&carried[i])));
             carried[i].partial = W(partials.back()->fr());
         }
-        CarriedFactors::queue_passes(carried.data(), carrying, nullptr);
-        check(grape_carried_finish(W(sums.gpu_data), 3, carried.data(), carrying, nullptr), "grape_carried_finish");
+        // a pass's sums are finished behind it, while the caches hold its partial sums; an odd round's with the pass before
+        for (uint i = 0; i < carrying; i += 2) {
+            const uint n = std::min(i + 3 == carrying ? 3u : 2u, carrying - i);
+            CarriedFactors::queue_passes(&carried[i], n, nullptr);
+            check(grape_carried_finish(W(sums.gpu_data + 3 * i), 3, &carried[i], n, nullptr), "grape_carried_finish");
+            if (n == 3) break;
+        }
         check(grape_carried_end(W(Bw), W(Bw), in, W(consts->fr() + carrying), period, nullptr, nullptr), "grape_carried_end");
         if (in == second_size) out = 1u << (Log2(in) - 1);     // a row's own variables: those of its padded length
     }

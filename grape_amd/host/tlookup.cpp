@@ -386,7 +386,8 @@ struct WeightPlan {
     bool split = false;
     WeightPlan(uint nu, uint N, bool carry) {
         const uint all = nu ? nu - 1 : 0;
-        whole = std::min(all, std::max(GRAPE_EQ_LONGEST_PREFIX, Log2(N)));
+        // carried rounds read the split tables alone: what is left for prefix tables are the rounds behind them and the table side
+        whole = std::min(all, std::max(carry ? GRAPE_EQ_SPLIT_LOW : GRAPE_EQ_LONGEST_PREFIX, Log2(N)));
         split = all > whole || carry;
         if (split) high = all - GRAPE_EQ_SPLIT_LOW;
     }
@@ -418,7 +419,8 @@ void tLookup::start_weights(uint D, bool gather) {
     forced_u_.clear();
     E_ready_.reset();
     if (u_ready_.size() != nu) return;          // run() reports the mismatch
-    const WeightPlan plan(nu, T.size, gather && may_carry(D, T.size));
+    carry_weights_ = gather && may_carry(D, T.size);
+    const WeightPlan plan(nu, T.size, carry_weights_);
     E_ready_.reset(new FrTensor((uint)plan.elems()));       // not OnDefaultStream: first written on the second stream
     // the point travels on the second stream too: on the default stream it would queue behind the pass over the
     // witness, and the pyramid with it
@@ -589,7 +591,7 @@ Fr tLookup::run(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax& hyrax
     // D / 2^(k+1) index pairs with those of nu-1-k variables; nothing is halved between rounds
     const uint nu = (uint)u.size();
     const bool may = gather_S && may_carry(D, N);            // then start_weights was told to gather
-    const WeightPlan plan(nu, N, may);
+    const WeightPlan plan(nu, N, E_early ? carry_weights_ : may);     // as they were laid out, whatever became of the witness since
     std::unique_ptr<FrTensor> E_own;
     if (E_early) {
         SideChain early(0);

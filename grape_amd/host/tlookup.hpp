@@ -55,6 +55,7 @@ protected:
     void start_weights(uint D, bool gather = false);
     std::vector<Fr> u_ready_;
     std::unique_ptr<FrTensor> E_ready_;
+    bool carry_weights_ = false;             // E_ready_ is laid out for rounds that carry their weights
     bool indexed_commit_ = true;
     bool index_known_ = false;          // set by tLookupRange: A's index is S - low
     int index_low_ = 0;

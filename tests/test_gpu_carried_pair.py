@@ -3,11 +3,10 @@ period, several workgroups and steps, every kind of first round, and the element
 import ctypes
 import numpy as np
 import pytest
+import bigref as br
 from gpuutil import rand_fr, assert_same
 
 pytestmark = pytest.mark.gpu
-
-_R = 0x73eda753299d7d483339d80809a1d80553bda402fffe5bfeffffffff00000001
 
 
 class Carried(ctypes.Structure):
@@ -27,7 +26,7 @@ def ops():
 def _elements(n, seed, largest):
     x = rand_fr(n, seed)
     if largest:                                              # r - 1 in memory, and zero
-        x[:] = np.frombuffer((_R - 1).to_bytes(32, "little"), dtype=np.uint64)
+        x[:] = np.frombuffer((br.R_MOD - 1).to_bytes(32, "little"), dtype=np.uint64)
         x[seed % 3::5] = 0
     return x
 
