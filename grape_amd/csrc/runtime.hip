@@ -102,6 +102,10 @@ int scratch_get(ScratchSlot slot, size_t bytes, void** out, hipStream_t stream) 
             return GRAPE_ENOMEM;
         }
         pool.bytes[slot] = want;
+        if (slot == kSlotTicket) {
+            const int rc = zero_fill(pool.ptr[slot], want, stream);
+            if (rc) return rc;
+        }
     }
     *out = pool.ptr[slot];
     return GRAPE_OK;
