@@ -498,12 +498,22 @@ __global__ void __launch_bounds__(kBlock) ref_from_wide_kernel(uint32_t* out, co
 // Each wave owns one row segment of `seg` columns; lane l takes columns l, l+64, ...
 // partial[(row*nseg + s)*64 + lane] receives the lane's XYZZ accumulator; full-width scalars of few rows go over split.parts
 // waves per segment (geom::window_split), partial[((row*nseg + s)*parts + part)*64 + lane].
-template <bool FR>
+// BASED (digits that are table indices): elements of index base1 cost nothing, the rows start at `start` instead (see
+// grape_commit_indexed).  Where the rows are uneven the workgroups are one wave, dealt by geom::spread_unit: a row that is all
+// padding is over at once, and beside three full ones in a workgroup, or on the same engine every time, its place would stay
+// empty.  2048 rows of 11008 padded to 16384, a third of 2^25 elements the padding's: a range lookup 6.28 -> 5.40 ms.  (Even
+// rows keep the order of the launch: a mapping lookup of 2^27 takes 25.3 ms that way and 25.8 dealt.)
+struct CommitBase {
+    const uint32_t* start;      // an accumulator: conversions in every wave would cost 1 % of a row of 4096
+    int32_t base1;
+    size_t step;                // of the deal, or 0
+};
+template <bool FR, bool BASED = false>
 __global__ void __launch_bounds__(kBlock) commit_wide_kernel(uint32_t* partial, const void* scalars, uint32_t rowlen, size_t rows,
                                                              uint32_t seg, uint32_t nseg, const uint32_t* table, size_t N,
-                                                             uint32_t c, uint32_t nw, uint32_t K, int* err_flag, geom::WindowSplit split) {
+                                                             uint32_t c, uint32_t nw, uint32_t K, int* err_flag, geom::WindowSplit split, CommitBase base) {
     const int lane = threadIdx.x & 63;
-    const size_t wave = ((size_t)blockIdx.x * kBlock + threadIdx.x) >> 6;
+    const size_t wave = BASED && base.step ? geom::spread_unit(blockIdx.x, gridDim.x, base.step) : ((size_t)blockIdx.x * kBlock + threadIdx.x) >> 6;
     const uint32_t parts = FR ? split.parts : 1;
     if (wave >= rows * nseg * parts) return;
     const size_t unit = FR ? wave / parts : wave;
@@ -513,15 +523,19 @@ __global__ void __launch_bounds__(kBlock) commit_wide_kernel(uint32_t* partial, 
     const uint32_t s = span.s, col_end = span.col_end;
     const uint32_t half = 1u << (c - 1), mask = (c == 32) ? 0xffffffffu : ((1u << c) - 1u);
     Xyzz30 acc = xyzz30_inf();
+    if (BASED && s == 0 && lane == 0) acc = ld_partial30(base.start, 0);
+    auto digits_of = [&](uint32_t col) { return ((const int32_t*)scalars)[geom::scalar_index(row, rowlen, col)]; };
+    // where a digit is used, not where it is loaded: there it would wait for the load
+    auto without_base = [&](int32_t x) { return BASED && x == base.base1 ? 0 : x; };
     // int path: the scalars of the next two columns are kept in flight (the next one addresses
     // the table line to touch, the one after is being loaded)
     int32_t sc1 = 0, sc2 = 0;
     if (!FR) {
         const uint32_t c0 = s * seg + lane;
-        if (c0 + 64 < col_end) sc1 = ((const int32_t*)scalars)[geom::scalar_index(row, rowlen, c0 + 64)];
-        if (c0 + 128 < col_end) sc2 = ((const int32_t*)scalars)[geom::scalar_index(row, rowlen, c0 + 128)];
+        if (c0 + 64 < col_end) sc1 = digits_of(c0 + 64);
+        if (c0 + 128 < col_end) sc2 = digits_of(c0 + 128);
     }
-    int32_t sc0 = (!FR && s * seg + lane < col_end) ? ((const int32_t*)scalars)[geom::scalar_index(row, rowlen, s * seg + lane)] : 0;
+    int32_t sc0 = (!FR && s * seg + lane < col_end) ? digits_of(s * seg + lane) : 0;
     // destination of the look-ahead touches: one register for the whole loop, read only after it.  (Declared
     // inside the loop it is free again at the top of the next iteration, the compiler reuses it for an
     // address there and has to wait for every outstanding load first - 1.5 % of the kernel's time.)
@@ -531,11 +545,11 @@ __global__ void __launch_bounds__(kBlock) commit_wide_kernel(uint32_t* partial, 
             const Fr k = from_mont(ld_fr8((const uint32_t*)scalars, geom::scalar_index(row, rowlen, col)));
             madd_scalar_fr(acc, k, table, N, col, c, nw, K, err_flag, w0, w0 + split.per);
         } else {
-            int64_t v = sc0;
-            const int64_t v_next = sc1;
+            int64_t v = without_base(sc0);
+            const int64_t v_next = without_base(sc1);
             sc0 = sc1;
             sc1 = sc2;
-            sc2 = (col + 192 < col_end) ? ((const int32_t*)scalars)[geom::scalar_index(row, rowlen, col + 192)] : 0;
+            sc2 = (col + 192 < col_end) ? digits_of(col + 192) : 0;
             // The table line of the NEXT column's first digit is touched (one word) right after
             // this column's own entry is requested, so that it is in cache when its turn comes:
             // with two waves per SIMD an exposed HBM round trip per addition costs issue slots.
@@ -578,6 +592,11 @@ __global__ void __launch_bounds__(kBlock) commit_wide_kernel(uint32_t* partial, 
     }
     asm volatile("" ::"v"(touch));                  // keeps the touches alive until here
     st_partial30(partial, wave * 64 + lane, acc);
+}
+
+__global__ void commit_start_kernel(uint32_t* out, const uint32_t* affine) {
+    const G1Affine a = ld_affine(affine, 0);
+    st_partial30(out, 0, a.is_inf() ? xyzz30_inf() : xyzz30_from_canonical(G1Xyzz{a.x, a.y, Fp::one(), Fp::one()}));
 }
 
 // Scaled table: out[t*ncols + i] = s_t * G_i for a short list of scalars s_t (Montgomery Fr).
@@ -1128,7 +1147,7 @@ static void launch_reduce(uint32_t* out, const uint32_t* partial, size_t rows, u
 
 template <bool FR>
 static int commit_wide_impl(uint32_t* out, const void* scalars, size_t size, uint32_t rowlen, const uint32_t* table, size_t N,
-                            uint32_t c, uint32_t nw, uint32_t K, grape_stream_t st, int* caller_flag = nullptr) {
+                            uint32_t c, uint32_t nw, uint32_t K, grape_stream_t st, int* caller_flag = nullptr, const CommitBase* base = nullptr) {
     if (size == 0) return GRAPE_OK;                      // no rows: nothing is read or written
     GRAPE_REQUIRE(size <= kMaxCommitScalars, "more than 2^28 scalars in one call: commit the rows in several calls");
     CHECK_PTR16(out); CHECK_PTR16(scalars); CHECK_PTR16(table);
@@ -1168,7 +1187,12 @@ static int commit_wide_impl(uint32_t* out, const void* scalars, size_t size, uin
         const size_t nr = rows - r0 < slab ? rows - r0 : slab;
         const uint32_t* sc = (const uint32_t*)scalars + r0 * rowlen * elem_words;
         profile_mark(s);
-        commit_wide_kernel<FR><<<blocks_for(nr * nparts), kBlock, 0, s>>>((uint32_t*)ws, sc, rowlen, nr, seg, nseg, table, N, c, nw, K, err, split);
+        if (!FR && base) {
+            const size_t waves = nr * nseg, step = base->step ? geom::spread_step(waves) : 0;
+            commit_wide_kernel<false, true><<<step ? (unsigned)waves : blocks_for(nr * nparts), step ? 64 : kBlock, 0, s>>>(
+                (uint32_t*)ws, sc, rowlen, nr, seg, nseg, table, N, c, nw, K, err, split, CommitBase{base->start, base->base1, step});
+        } else
+            commit_wide_kernel<FR><<<blocks_for(nr * nparts), kBlock, 0, s>>>((uint32_t*)ws, sc, rowlen, nr, seg, nseg, table, N, c, nw, K, err, split, CommitBase{});
         profile_mark(s);
         launch_reduce<true>(out + r0 * (size_t)(2 * FW), (const uint32_t*)ws, nr, nparts, red_tmp, s);
         profile_mark(s);
@@ -1491,6 +1515,23 @@ int grape_commit_i32_nowait(uint32_t* out, const int32_t* scalars, size_t size, 
                             uint32_t c, uint32_t nw, uint32_t K, int32_t* d_flag, grape_stream_t st) {
     GRAPE_REQUIRE(d_flag != nullptr, "the caller's flag is required");
     return commit_wide_impl<false>(out, scalars, size, rowlen, table, N, c, nw, K, st, d_flag);
+}
+int grape_commit_start(uint32_t* out, const uint32_t* affine, grape_stream_t st) {
+    CHECK_PTR16(out); CHECK_PTR16(affine);
+    static_assert(GRAPE_COMMIT_START_WORDS == kPartialWords, "the header's accumulator is the kernels'");
+    commit_start_kernel<<<1, 1, 0, as_stream(st)>>>(out, affine);
+    GRAPE_LAUNCH_CHECK();
+    return GRAPE_OK;
+}
+int grape_commit_indexed(uint32_t* out, const int32_t* idx1, size_t size, uint32_t rowlen, const uint32_t* table, size_t ncols, uint32_t len, int32_t base1,
+                         const uint32_t* start, int uneven, int32_t* d_flag, grape_stream_t st) {
+    GRAPE_REQUIRE(len >= 1 && len < (1u << 23), "between 1 and 2^23 - 1 entries");
+    uint32_t c = 2;                                      // radix 2^c keeps the digits 1..len below the sign threshold
+    while ((1u << (c - 1)) <= len) c++;
+    if (!start) return commit_wide_impl<false>(out, idx1, size, rowlen, table, ncols, c, 1, len, st, d_flag);
+    CHECK_PTR16(start);
+    const CommitBase base{start, base1, (size_t)(uneven ? 1 : 0)};
+    return commit_wide_impl<false>(out, idx1, size, rowlen, table, ncols, c, 1, len, st, d_flag, &base);
 }
 int grape_commit_fr(uint32_t* out, const uint32_t* scalars, size_t size, uint32_t rowlen, const uint32_t* table, size_t N,
                     uint32_t c, uint32_t nw, uint32_t K, grape_stream_t st) {

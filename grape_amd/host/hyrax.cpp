@@ -339,6 +339,14 @@ affine_t* Hyrax::commit_affine(FrTensor& tensor, uint size, uint N) {
     return out;
 }
 
+affine_t* Hyrax::commit_row(FrTensor& row) {
+    if (row.size > npoints) throw std::runtime_error("row longer than the generator set");
+    affine_t* out = nullptr;
+    check(grape_malloc((void**)&out, sizeof(affine_t)), "grape_malloc");
+    commit_fr_rows(out, row.gpu_data, row.size, row.size, false);
+    return out;
+}
+
 bool Hyrax::prepare_scaled_tables(uint ncols) { return ensure_fr_table(ncols); }
 
 affine_t* Hyrax::build_scaled_table(const FrTensor& scalars, uint ncols) {
@@ -408,20 +416,18 @@ bool Hyrax::owns_scaled_table(const affine_t* table) const {
     return it != scaled_registry().end() && it->second.owner == this;
 }
 
-affine_t* Hyrax::commit_indexed_affine(int* idx_plus1, uint size, uint N, affine_t* scaled_table, uint ncols, uint len, int* d_flag) {
+affine_t* Hyrax::commit_indexed_affine(int* idx_plus1, uint size, uint N, affine_t* scaled_table, uint ncols, uint len, int* d_flag, int base1,
+                                       const void* start, bool uneven) {
     check_shape(size, N);
     const uint rowlen = N * com_scale;
     if (rowlen > ncols) throw std::runtime_error("row longer than the scaled table");
     const uint rows = size / rowlen;
     affine_t* out = nullptr;
     check(grape_malloc((void**)&out, sizeof(affine_t) * (size_t)rows), "grape_malloc");
-    // one unsigned "digit" idx+1 in [1, len]: radix 2^(log2(len)+1) keeps it below the sign threshold
-    const uint c = Log2(len) + 1 < 2 ? 2 : Log2(len) + 1;
     check(for_row_chunks(size, rowlen, [&](size_t e0, size_t n, size_t r0) {
-              if (d_flag) return grape_commit_i32_nowait(W(out + r0), idx_plus1 + e0, n, rowlen, W(scaled_table), ncols, c, 1, len, d_flag, nullptr);
-              return grape_commit_i32(W(out + r0), idx_plus1 + e0, n, rowlen, W(scaled_table), ncols, c, 1, len, nullptr);
+              return grape_commit_indexed(W(out + r0), idx_plus1 + e0, n, rowlen, W(scaled_table), ncols, len, base1, static_cast<const uint32_t*>(start), uneven, d_flag, nullptr);
           }),
-          "grape_commit_i32 (indexed)");
+          "grape_commit_indexed");
     return out;
 }
 

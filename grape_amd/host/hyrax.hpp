@@ -70,6 +70,7 @@ public:
     // owned by the caller, freed with grape_free); nullptr when it would not fit the budget.
     // With it, a tensor whose elements are scalars[idx] commits at one addition per element:
     affine_t* build_scaled_table(const FrTensor& scalars, uint ncols);
+    affine_t* commit_row(FrTensor& row);             // one row over the first row.size generators, whatever the layers
     // Builds what build_scaled_table reads (the per-window table over the first ncols generators) if it is
     // not there yet, so that table_bytes_free() afterwards is what a scaled table may really take; false when
     // it does not fit the budget (build_scaled_table would return nullptr).
@@ -88,7 +89,9 @@ public:
     // built it is gone, even if a new object sits at the same address)
     bool owns_scaled_table(const affine_t* table) const;
     // idx_plus1[j] = idx_j + 1 (0 = contributes nothing); rows of N*com_scale, affine output.
-    affine_t* commit_indexed_affine(int* idx_plus1, uint size, uint N, affine_t* scaled_table, uint ncols, uint len, int* d_flag = nullptr);
+    // base1, start, uneven: see grape_commit_indexed
+    affine_t* commit_indexed_affine(int* idx_plus1, uint size, uint N, affine_t* scaled_table, uint ncols, uint len, int* d_flag = nullptr,
+                                    int base1 = 0, const void* start = nullptr, bool uneven = false);
 
     // Row commitments of the elements whose flag skip[j] is zero (`live` of them), the others left out; through the
     // strided table where rows hold many of them, through the per-window table that scaled tables are built with

@@ -25,6 +25,7 @@ tLookup::tLookup(const uint size) : alpha(Fr::random_element()), beta(Fr((long)s
 tLookup::~tLookup() {
     grape_free(com_A);
     grape_free(com_m);
+    grape_free(base_point_);
     Hyrax::release_scaled_table(scaled_table_);
     Hyrax::release_scaled_table(hot_table_);
     grape_free(hot_slot1_);
@@ -131,7 +132,36 @@ void tLookup::gather_by_index(FrTensor& out, const FrTensor& table, uint D) {
     check(grape_fr_gather(W(out.gpu_data), W(table.gpu_data) - 8, reinterpret_cast<const uint32_t*>(d_idx_), D, nullptr), "grape_fr_gather");   // d_idx_ holds index + 1
 }
 
-// com(A) through the entries that occur often (A: nullptr when it has not been written out).  A[i] = B[index_i]; an entry t that occurs n_t times
+FrTensor& tLookup::scaled_by() {
+    if (base_ < 0) return B;
+    if (!B_less_base_) {
+        B_less_base_.reset(new FrTensor(B));
+        const Fr less = Fr::zero() - B((uint)base_);
+        check(grape_fr_bcast_add(W(B_less_base_->gpu_data), W(B.gpu_data), W(grape_host::device_scalar(less)), B.size, nullptr), "grape_fr_bcast_add");
+    }
+    return *B_less_base_;
+}
+const void* tLookup::base_point(Hyrax& hyrax, uint msm_size) {
+    if (base_ < 0) return nullptr;
+    const uint rowlen = msm_size * hyrax.com_scale;
+    if (base_cols_ != rowlen) {
+        FrTensor row(rowlen, OnDefaultStream());
+        check(grape_memset_zero(row.gpu_data, sizeof(fr_t) * (size_t)rowlen, nullptr), "grape_memset_zero");
+        check(grape_fr_bcast_add(W(row.gpu_data), W(row.gpu_data), W(B.gpu_data + base_), rowlen, nullptr), "grape_fr_bcast_add");
+        affine_t* p = hyrax.commit_row(row);
+        if (!base_point_) check(grape_malloc(&base_point_, sizeof(uint32_t) * GRAPE_COMMIT_START_WORDS), "grape_malloc");
+        const int rc = grape_commit_start(static_cast<uint32_t*>(base_point_), reinterpret_cast<uint32_t*>(p), nullptr);
+        grape_free(p);
+        check(rc, "grape_commit_start");
+        base_cols_ = rowlen;
+    }
+    return base_point_;
+}
+namespace {
+constexpr int kBaseMark = 0x7fffffff;            // the slot of the base entry: no row's
+}
+
+// com(A) through the entries that occur often.  A[i] = B[index_i]; an entry t that occurs n_t times
 // costs n_t full-width scalars (16 to 20 additions each) on the plain path, or one row B[t]*G_i of
 // the scaled table (rowlen entries at 20 additions and a normalisation each) plus n_t single additions.  So an entry is worth a row
 // when n_t exceeds rowlen by a factor somewhat above one; 1.8 is taken (the first proof's time is flat from 1.2 to 2.2).  Elements of the
@@ -188,12 +218,14 @@ uint64_t tLookup::grow_hot_rows(Hyrax& hyrax, const uint64_t info[3]) {
         const uint n_new = (uint)given[0];
         if (n_new != 0) {
             FrTensor more(n_new, OnDefaultStream());
-            check(grape_fr_gather(W(more.gpu_data), W(B.gpu_data), d_list, n_new, nullptr), "grape_fr_gather");
+            check(grape_fr_gather(W(more.gpu_data), W(scaled_by().gpu_data), d_list, n_new, nullptr), "grape_fr_gather");
             bool built;
             if (hot_table_) {
                 built = hyrax.extend_scaled_table(hot_table_, hot_rows_, hot_capacity_, more, hot_cols_);
             } else {
                 hot_table_ = hyrax.build_scaled_table(more, hot_cols_);
+                base_cols_ = 0;
+                if (hot_table_ && base_ >= 0) check(grape_memcpy_h2d(slots + base_, &kBaseMark, sizeof(int), nullptr), "grape_memcpy_h2d");
                 built = hot_table_ != nullptr;
                 hot_capacity_ = built ? n_new : 0;
             }
@@ -217,7 +249,7 @@ uint64_t tLookup::grow_hot_rows(Hyrax& hyrax, const uint64_t info[3]) {
     return left;
 }
 
-bool tLookup::commit_A_by_occupancy(FrTensor* A, uint D, uint msm_size, Hyrax& hyrax) {
+bool tLookup::commit_A_by_occupancy(uint D, uint msm_size, Hyrax& hyrax) {
     const uint N = T.size;
     const uint rowlen = msm_size * hyrax.com_scale;
     const uint rows = D / rowlen;
@@ -263,8 +295,10 @@ bool tLookup::commit_A_by_occupancy(FrTensor* A, uint D, uint msm_size, Hyrax& h
             cold = info[1];
             if (n_hot != 0) {
                 FrTensor Bhot(n_hot, OnDefaultStream());
-                check(grape_fr_gather(W(Bhot.gpu_data), W(B.gpu_data), d_list, n_hot, nullptr), "grape_fr_gather");
+                check(grape_fr_gather(W(Bhot.gpu_data), W(scaled_by().gpu_data), d_list, n_hot, nullptr), "grape_fr_gather");
                 hot_table_ = hyrax.build_scaled_table(Bhot, rowlen);
+                base_cols_ = 0;
+                if (hot_table_ && base_ >= 0) check(grape_memcpy_h2d(hot_slot1_ + base_, &kBaseMark, sizeof(int), nullptr), "grape_memcpy_h2d");
                 if (!hot_table_) check(grape_memset_zero(hot_slot1_, sizeof(int) * (size_t)N, nullptr), "grape_memset_zero");
             }
             hot_rows_ = hot_capacity_ = hot_table_ ? n_hot : 0;
@@ -288,14 +322,14 @@ bool tLookup::commit_A_by_occupancy(FrTensor* A, uint D, uint msm_size, Hyrax& h
     try {
         check(grape_malloc_on_default((void**)&d_hot, sizeof(int) * (size_t)D), "grape_malloc");
         check(grape_tlookup_hot_index(d_hot, d_idx_, D, hot_slot1_, N, nullptr), "grape_tlookup_hot_index");
-        com_A = hyrax.commit_indexed_affine(d_hot, D, msm_size, hot_table_, rowlen, hot_rows_);
+        com_A = hyrax.commit_indexed_affine(d_hot, D, msm_size, hot_table_, rowlen, hot_rows_, nullptr, kBaseMark, base_point(hyrax, msm_size), padded_);
         if (cold != 0) {
             // the elements without a table row: queued per row and committed as full-width scalars
-            com_cold = A ? hyrax.commit_sparse_affine(*A, d_hot, D, msm_size, cold) : hyrax.commit_sparse_affine(B, d_hot, D, msm_size, cold, d_idx_);
+            com_cold = hyrax.commit_sparse_affine(scaled_by(), d_hot, D, msm_size, cold, d_idx_);
             if (!com_cold) {
                 FrTensor Acold(D, OnDefaultStream());
-                if (!A) gather_by_index(Acold, B, D);
-                check(grape_fr_mask_cold(W(Acold.gpu_data), W(A ? A->gpu_data : Acold.gpu_data), d_hot, D, nullptr), "grape_fr_mask_cold");
+                gather_by_index(Acold, scaled_by(), D);
+                check(grape_fr_mask_cold(W(Acold.gpu_data), W(Acold.gpu_data), d_hot, D, nullptr), "grape_fr_mask_cold");
                 com_cold = hyrax.commit_affine(Acold, D, msm_size);
             }
             check(grape_g1_affine_add((uint32_t*)com_A, (const uint32_t*)com_A, (const uint32_t*)com_cold, rows, nullptr),
@@ -451,6 +485,7 @@ static void histogram_to_m(FrTensor& m, const FrTensor& vals, int low) {
 tLookupRange::tLookupRange(int low_, uint len) : tLookup(1u << Log2(len)), low(low_) {
     index_known_ = true;
     index_low_ = low_;
+    base_ = low <= 0 && (int64_t)low + (int64_t)T.size > 0 ? -low : -1;
     // the table always covers the whole power-of-two range T.size (the reference initialises
     // only the first len entries and leaves the rest unset)
     check(grape_tlookup_init(W(T.gpu_data), W(B.gpu_data), low, T.size, W(grape_host::device_scalar(beta)), nullptr, nullptr, nullptr),
@@ -508,12 +543,16 @@ Fr tLookup::run(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax& hyrax
         if (indexed_commit_ && index_known_ &&
             (scaled_for_ != &hyrax || scaled_cols_ < rowlen || (scaled_table_ && !hyrax.owns_scaled_table(scaled_table_)))) {
             Hyrax::release_scaled_table(scaled_table_);
-            scaled_table_ = hyrax.build_scaled_table(B, rowlen);   // nullptr when over budget
+            scaled_table_ = hyrax.build_scaled_table(scaled_by(), rowlen);   // nullptr when over budget
+            B_less_base_.reset();                    // every entry has its row
+            base_cols_ = 0;
             scaled_cols_ = scaled_table_ ? rowlen : 0;
             scaled_for_ = &hyrax;
         }
     });
     const bool indexed = indexed_commit_ && index_known_ && scaled_table_;
+    const void* start = nullptr;                 // made here, where the host may wait
+    if (indexed) timed([&] { start = base_point(hyrax, msm_size); });
     const bool overlap = indexed && d_idx_ != nullptr;
     // A = 1/(S + beta): read from B where the witness matches its table entry (every element of
     // a valid witness does), computed by batched inversion otherwise (tlookup_inv_kernel,
@@ -553,11 +592,11 @@ Fr tLookup::run(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax& hyrax
                 check(grape_malloc((void**)&d_idx, sizeof(int) * (size_t)D), "grape_malloc");
                 check(grape_tlookup_index(d_idx, W(S.gpu_data), D, index_low_, N, nullptr), "grape_tlookup_index");
             }
-            com_A = hyrax.commit_indexed_affine(d_idx, D, msm_size, scaled_table_, scaled_cols_, N);
+            com_A = hyrax.commit_indexed_affine(d_idx, D, msm_size, scaled_table_, scaled_cols_, N, nullptr, base_ + 1, start, padded_);
             check(grape_stream_sync(nullptr), "sync");
             if (d_idx != d_idx_) grape_free(d_idx);
         } else if (indexed_commit_ && from_table && d_idx_ && d_hist_ && D / rowlen > 1 &&
-                   commit_A_by_occupancy(gather_first ? nullptr : &A, D, msm_size, hyrax)) {
+                   commit_A_by_occupancy(D, msm_size, hyrax)) {
             // committed through a table of the entries that occur often
         } else {
             if (gather_first) gather_by_index(A, B, D);
@@ -843,7 +882,7 @@ Fr tLookup::run(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax& hyrax
             // commit_time of this mode: what the commitment of A takes on the default stream, between two events
             check(grape_event_record(commit_events().first, nullptr), "grape_event_record");
             timed([&] {
-                com_A = hyrax.commit_indexed_affine(d_idx_, D, msm_size, scaled_table_, scaled_cols_, N, d_flags);
+                com_A = hyrax.commit_indexed_affine(d_idx_, D, msm_size, scaled_table_, scaled_cols_, N, d_flags, base_ + 1, start, padded_);
                 com_A_rows = D / (msm_size * hyrax.com_scale);
                 if (!m_aside) com_m = hyrax.commit_affine(m, N, m_N);
             });
@@ -957,6 +996,15 @@ Fr tLookup::run(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax& hyrax
     return S_last;
 }
 
+namespace {
+// the witness of the proof in flight has been padded by this object
+struct PaddedScope {
+    bool &flag, before;
+    PaddedScope(bool& f, bool now) : flag(f), before(f) { flag = before || now; }
+    ~PaddedScope() { flag = before; }
+};
+}  // namespace
+
 Fr tLookupRange::prove(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax& hyrax, uint msm_size, double& commit_time) {
     uint D = S.size;
     if (D == (1u << Log2(D)) && A.size >= D) {
@@ -976,6 +1024,7 @@ Fr tLookupRange::prove(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax
     } else {
         index_to_m(D, low);
     }
+    PaddedScope padded(padded_, D != (1u << Log2(D)));
     if (D != (1u << Log2(D))) {
         // src/tlookup.cu:299-305: rows of 11008 padded to 16384 with zeros
         Fr pad_value = Fr::zero();
@@ -1006,6 +1055,7 @@ Fr tLookupRange::prove(const int* device_int_S, FrTensor& S, FrTensor& A, const 
         int* padded = nullptr;
         check(grape_malloc_on_default((void**)&padded, sizeof(int) * (size_t)Dp), "grape_malloc");
         Fr ret;
+        PaddedScope scope(padded_, true);
         try {
             check(grape_i32_pad(padded, device_int_S, 11008, 16384, Dp, nullptr), "grape_i32_pad");
             S.set_size(Dp);
@@ -1056,6 +1106,7 @@ void tLookupRangeMapping::init_from_host(const int* host_table, uint len) {
     d_map_int_ = d_int;                   // kept: a witness handed over as integers is checked against it
     have_map_zero_ = low <= 0 && (int64_t)low + (int64_t)len > 0;
     map_zero_ = have_map_zero_ ? host_table[-low] : 0;
+    base_ = have_map_zero_ ? -low : -1;
 }
 tLookupRangeMapping::~tLookupRangeMapping() { grape_free(d_map_int_); }
 
@@ -1093,6 +1144,7 @@ Fr tLookupRangeMapping::prove(FrTensor& S_in, FrTensor& S_out, FrTensor& A, cons
     FrTensor S(1u << Log2(D), OnDefaultStream());
     S.set_size(D);
     check(grape_fr_axpy(W(S.gpu_data), W(S_in.gpu_data), W(grape_host::device_scalar(r)), W(S_out.gpu_data), D, nullptr), "grape_fr_axpy");
+    PaddedScope padded(padded_, D != (1u << Log2(D)));
     if (D != (1u << Log2(D))) {
         Fr pad_value = mapped_vals((uint)(-low)) * r;
         S.pad(A, 11008, 16384, 1u << Log2(D), pad_value);
@@ -1117,6 +1169,7 @@ Fr tLookupRangeMapping::prove(const int* device_int_S_in, const int* device_int_
         // (src/tlookup.cu:411-420) and proved as a witness that needs no padding
         int *pin = nullptr, *pout = nullptr;
         Fr ret;
+        PaddedScope scope(padded_, true);
         try {
             check(grape_malloc_on_default((void**)&pin, sizeof(int) * (size_t)Dp), "grape_malloc");
             check(grape_malloc_on_default((void**)&pout, sizeof(int) * (size_t)Dp), "grape_malloc");

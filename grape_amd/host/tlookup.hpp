@@ -91,7 +91,7 @@ protected:
     uint hot_entries_ = 0;
     uint64_t cold_elements_ = 0;
     bool hot_reused_ = false;
-    bool commit_A_by_occupancy(FrTensor* A, uint D, uint msm_size, Hyrax& hyrax);
+    bool commit_A_by_occupancy(uint D, uint msm_size, Hyrax& hyrax);
     // Rows B[t]*G_i of the entries that were occupied in an earlier witness, with their slot
     // assignment: B is fixed for the object's life (the reference keeps one lookup object for all
     // layers of a model, test/llm.cu:57-64), so the rows serve later proofs as long as they cover
@@ -104,7 +104,17 @@ protected:
     uint32_t* hot_credit_ = nullptr;    // occurrences of entries without a row in the proofs since the rows were made
     double hot_missed_ = 0;             // elements of entries that had earned a row when there was no more room for it
     uint64_t grow_hot_rows(Hyrax& hyrax, const uint64_t info[3]);
-    affine_t* scaled_table_ = nullptr;  // B[t]*G_i, built on first use
+    // The entry a witness is padded with, the key 0 (-1: not in the table).  Its elements - a third of a witness of rows of 11008, the
+    // zeros of any other - take no addition: the rows of both tables hold (B[t] - B[base]) G_i, and every committed row starts at
+    // sum_i B[base] G_i.
+    int base_ = -1;
+    bool padded_ = false;               // the witness of the proof in flight
+    std::unique_ptr<FrTensor> B_less_base_;
+    void* base_point_ = nullptr;
+    uint base_cols_ = 0;                // the row length it was made for (0: not made for the tables at hand)
+    FrTensor& scaled_by();              // what the tables' rows are multiples by
+    const void* base_point(Hyrax& hyrax, uint msm_size);
+    affine_t* scaled_table_ = nullptr;  // (B[t] - B[base])*G_i, built on first use
     uint scaled_cols_ = 0;
     Hyrax* scaled_for_ = nullptr;
 };

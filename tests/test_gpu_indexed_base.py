@@ -1,0 +1,52 @@
+"""Rows committed through their table indices with a base entry that costs nothing, against the oracle's commitment of the values:
+rows of the base entry alone, without it, elements outside the table, one and several column segments, both orders of the rows."""
+import numpy as np
+import pytest
+import orc
+from gpuutil import rand_fr, assert_same
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from grape_amd import ops
+    ops.init(0)
+    return ops
+
+
+@pytest.fixture(scope="module")
+def tables(ops):
+    gens = ops.g1_make_generators(rand_fr(256, 801))
+    return gens, ops.g1_wide_table_gen(gens, 8, 32, 128), orc.g1_table(ops.g1_to_host(gens), 256)
+
+
+@pytest.mark.parametrize("rows,cols,uneven", [(1, 1, 0), (1, 256, 1), (5, 65, 0), (37, 256, 1), (64, 100, 0), (600, 64, 1), (600, 128, 0)])
+def test_base_entry(ops, tables, rows, cols, uneven):
+    import torch
+    from grape_amd import _capi
+    lib = ops.init()
+    gens, wide, ref = tables
+    length, base = 9, 3
+    B = rand_fr(length, 802)
+    rng = np.random.default_rng(rows * cols)
+    idx = rng.integers(0, length + 1, (rows, cols)).astype(np.int32)      # 0 is outside the table
+    idx[0::4] = base + 1
+    idx[1::4, cols // 2:] = base + 1
+    idx[2::4][idx[2::4] == base + 1] = 0
+    less = orc.vec2("orc_fr_vec_sub", B, np.repeat(B[base:base + 1], length, axis=0))
+    scaled = torch.empty(lib.grape_g1_wide_table_bytes(cols, 1, length) // 4, dtype=torch.int32, device="cuda")
+    d_less = ops.to_dev(less)
+    _capi.check(lib.grape_g1_scaled_table_gen(scaled.data_ptr(), d_less.data_ptr(), length, cols, wide.data_ptr(), 256, 8, 32, 128, None))
+    # every row starts at sum_i B_base G_i; elements outside the table then stand for B_base too
+    point = ops.to_dev(orc.commit_fr(np.repeat(B[base:base + 1], cols, axis=0), ref, cols, 256))
+    start = torch.empty(64, dtype=torch.int32, device="cuda")
+    _capi.check(lib.grape_commit_start(start.data_ptr(), point.data_ptr(), None))
+    d_idx, out = torch.from_numpy(idx).cuda(), ops.g1_empty(rows)
+    flag = torch.zeros(1, dtype=torch.int32, device="cuda")
+    _capi.check(lib.grape_commit_indexed(out.data_ptr(), d_idx.data_ptr(), rows * cols, cols, scaled.data_ptr(), cols, length, base + 1,
+                                         start.data_ptr(), uneven, flag.data_ptr(), None))
+    torch.cuda.synchronize()
+    values = B[np.where(idx == 0, base, idx - 1).ravel()]
+    assert int(flag) == 0
+    assert_same(ops.g1_to_host(out), orc.commit_fr(values, ref, cols, 256), "commitments")
