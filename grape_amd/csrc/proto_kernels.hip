@@ -289,14 +289,20 @@ __global__ void __launch_bounds__(kHistThreads) hist_lds_kernel(uint32_t* __rest
         for (int q = 0; q < 4; q++) {
             const uint32_t b = (uint32_t)(vv[q] - 1) - base;      // 0 (out of range) wraps far away
             const bool in = b < (uint32_t)BINS;
-            // lanes that share a bin are counted once: up to four leaders, then plain adds
+            // lanes that share a bin are counted once: up to four leaders, then plain adds.  Two leaders that share theirs with
+            // fewer than three others each tell that the values are spread out, where plain adds are cheaper (2^27 scores on some
+            // 900 entries: 1.08 -> 0.77 ms with the passes around it; half of them one entry: 1.08 -> 0.95).
             unsigned long long todo = __ballot(in);
+            uint32_t shared = 0;
             for (int it = 0; it < 4 && todo != 0ull; it++) {
                 const int leader = __ffsll((long long)todo) - 1;
-                const uint32_t lb = __shfl(b, leader, 64);
+                const uint32_t lb = (uint32_t)__builtin_amdgcn_readlane((int)b, leader);
                 const unsigned long long same = __ballot(in && b == lb) & todo;
-                if (lane == leader) atomicAdd(&bins[lb], (uint32_t)__popcll(same));
+                const uint32_t count = (uint32_t)__popcll(same);
+                if (lane == leader) atomicAdd(&bins[lb], count);
                 todo &= ~same;
+                shared += count;
+                if (it == 1 && shared < 8) break;
             }
             if (in && ((todo >> lane) & 1ull)) atomicAdd(&bins[b], 1u);
         }
