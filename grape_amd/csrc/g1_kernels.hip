@@ -498,13 +498,14 @@ __global__ void __launch_bounds__(kBlock) ref_from_wide_kernel(uint32_t* out, co
 // Each wave owns one row segment of `seg` columns; lane l takes columns l, l+64, ...
 // partial[(row*nseg + s)*64 + lane] receives the lane's XYZZ accumulator; full-width scalars of few rows go over split.parts
 // waves per segment (geom::window_split), partial[((row*nseg + s)*parts + part)*64 + lane].
-// BASED (digits that are table indices): elements of index base1 cost nothing, the rows start at `start` instead (see
-// grape_commit_indexed).  Where the rows are uneven the workgroups are one wave, dealt by geom::spread_unit: a row that is all
+// BASED (digits that are table indices): elements of index base1 cost nothing, the rows' sums are added to `start` instead (see
+// grape_commit_indexed), on their way to affine coordinates: a lane that began with it would make a full addition of its first
+// entry where the others take theirs over, 1.5 % of a row of 4096 and twice the time of one of 256.  Where the rows are uneven the workgroups are one wave, dealt by geom::spread_unit: a row that is all
 // padding is over at once, and beside three full ones in a workgroup, or on the same engine every time, its place would stay
 // empty.  2048 rows of 11008 padded to 16384, a third of 2^25 elements the padding's: a range lookup 6.28 -> 5.40 ms.  (Even
 // rows keep the order of the launch: a mapping lookup of 2^27 takes 25.3 ms that way and 25.8 dealt.)
 struct CommitBase {
-    const uint32_t* start;      // an accumulator: conversions in every wave would cost 1 % of a row of 4096
+    const uint32_t* start;      // an accumulator
     int32_t base1;
     size_t step;                // of the deal, or 0
 };
@@ -523,7 +524,6 @@ __global__ void __launch_bounds__(kBlock) commit_wide_kernel(uint32_t* partial, 
     const uint32_t s = span.s, col_end = span.col_end;
     const uint32_t half = 1u << (c - 1), mask = (c == 32) ? 0xffffffffu : ((1u << c) - 1u);
     Xyzz30 acc = xyzz30_inf();
-    if (BASED && s == 0 && lane == 0) acc = ld_partial30(base.start, 0);
     auto digits_of = [&](uint32_t col) { return ((const int32_t*)scalars)[geom::scalar_index(row, rowlen, col)]; };
     // where a digit is used, not where it is loaded: there it would wait for the load
     auto without_base = [&](int32_t x) { return BASED && x == base.base1 ? 0 : x; };
@@ -925,10 +925,13 @@ __global__ void __launch_bounds__(kBlock) commit_reduce_quad_kernel(uint32_t* ou
     }
     if (have && sub == 0) st_quad_partial(out, row, acc);      // 256 bytes per row: an accumulator
 }
-__global__ void __launch_bounds__(kBlock) quad_affine_kernel(uint32_t* out, const uint32_t* sums, size_t rows) {
+template <bool START>
+__global__ void __launch_bounds__(kBlock) quad_affine_kernel(uint32_t* out, const uint32_t* sums, size_t rows, const uint32_t* start) {
     const size_t row = ((size_t)blockIdx.x * kBlock + threadIdx.x) >> 2;
     if (row >= rows) return;
-    const Fp c = quad::to_affine(ld_quad_partial(sums, row));
+    quad::Acc acc = ld_quad_partial(sums, row);
+    if (START) quad::add(acc, ld_quad_partial(start, 0));
+    const Fp c = quad::to_affine(acc);
     const uint32_t r = threadIdx.x & 3;
     if (r < 2) st_fp(out + 2 * FW * row + FW * r, c);
 }
@@ -1132,7 +1135,7 @@ constexpr size_t kMaxCommitScalars = (size_t)1 << 28;
 // to accumulators of 256 bytes for a later combination.
 static size_t reduce_tmp_bytes(size_t rows, uint32_t nparts) { return geom::reduce_tmp_accumulators(rows, nparts) * (4 * kPartialWords); }
 template <bool AFFINE>
-static void launch_reduce(uint32_t* out, const uint32_t* partial, size_t rows, uint32_t nparts, uint32_t* tmp, hipStream_t s) {
+static void launch_reduce(uint32_t* out, const uint32_t* partial, size_t rows, uint32_t nparts, uint32_t* tmp, hipStream_t s, const uint32_t* start = nullptr) {
     geom::ReduceStage st[geom::kMaxReduceStages];
     const int n = geom::reduce_stages(rows, nparts, st);
     uint32_t* sums = nullptr;
@@ -1142,7 +1145,8 @@ static void launch_reduce(uint32_t* out, const uint32_t* partial, size_t rows, u
         if (st[i].lanes) commit_reduce_lane_kernel<<<blocks_for(st[i].units * st[i].keep), kBlock, 0, s>>>(sums, from, st[i].units, st[i].parts, st[i].keep);
         else commit_reduce_quad_kernel<<<blocks_for(st[i].units << (st[i].lg_qpr + 2)), kBlock, 0, s>>>(sums, from, st[i].units, st[i].parts, st[i].lg_qpr);
     }
-    if (AFFINE) quad_affine_kernel<<<blocks_for(rows * 4), kBlock, 0, s>>>(out, sums, rows);
+    if (AFFINE && start) quad_affine_kernel<true><<<blocks_for(rows * 4), kBlock, 0, s>>>(out, sums, rows, start);
+    else if (AFFINE) quad_affine_kernel<false><<<blocks_for(rows * 4), kBlock, 0, s>>>(out, sums, rows, nullptr);
 }
 
 template <bool FR>
@@ -1194,7 +1198,7 @@ static int commit_wide_impl(uint32_t* out, const void* scalars, size_t size, uin
         } else
             commit_wide_kernel<FR><<<blocks_for(nr * nparts), kBlock, 0, s>>>((uint32_t*)ws, sc, rowlen, nr, seg, nseg, table, N, c, nw, K, err, split, CommitBase{});
         profile_mark(s);
-        launch_reduce<true>(out + r0 * (size_t)(2 * FW), (const uint32_t*)ws, nr, nparts, red_tmp, s);
+        launch_reduce<true>(out + r0 * (size_t)(2 * FW), (const uint32_t*)ws, nr, nparts, red_tmp, s, base ? base->start : nullptr);
         profile_mark(s);
     }
     GRAPE_LAUNCH_CHECK();
