@@ -1529,9 +1529,9 @@ int grape_commit_start(uint32_t* out, const uint32_t* affine, grape_stream_t st)
 }
 int grape_commit_indexed(uint32_t* out, const int32_t* idx1, size_t size, uint32_t rowlen, const uint32_t* table, size_t ncols, uint32_t len, int32_t base1,
                          const uint32_t* start, int uneven, int32_t* d_flag, grape_stream_t st) {
-    GRAPE_REQUIRE(len >= 1 && len < (1u << 23), "between 1 and 2^23 - 1 entries");
-    uint32_t c = 2;                                      // radix 2^c keeps the digits 1..len below the sign threshold
-    while ((1u << (c - 1)) <= len) c++;
+    GRAPE_REQUIRE(len >= 1 && len <= (1u << 23), "between 1 and 2^23 entries");
+    uint32_t c = 2;                                      // radix 2^c: a digit of up to 2^(c-1) with nothing above it stays positive
+    while ((1u << (c - 1)) < len) c++;
     if (!start) return commit_wide_impl<false>(out, idx1, size, rowlen, table, ncols, c, 1, len, st, d_flag);
     CHECK_PTR16(start);
     const CommitBase base{start, base1, (size_t)(uneven ? 1 : 0)};

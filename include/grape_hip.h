@@ -572,7 +572,7 @@ int grape_commit_i32(uint32_t *d_out_affine, const int32_t *d_scalars, size_t si
 int grape_commit_i32_nowait(uint32_t *d_out_affine, const int32_t *d_scalars, size_t size, uint32_t rowlen,
                             const uint32_t *d_wide_table, size_t N, uint32_t c, uint32_t nw, uint32_t K, int32_t *d_flag,
                             grape_stream_t stream);
-/* Rows committed through a scaled table (grape_g1_scaled_table_gen, `len` scalars by `ncols` generators): element (row, i) of index
+/* Rows committed through a scaled table (grape_g1_scaled_table_gen, `len` <= 2^23 scalars by `ncols` generators): element (row, i) of index
  * j = d_idx1 in 1..len adds s_(j - 1) G_i, index 0 nothing.  With d_start (made of an affine point by grape_commit_start) every row starts there and elements of
  * index base1, which need be none of the table's, add nothing: with s_t = B_t - B_b and a start of sum_i B_b G_i over a row,
  * entry b's own elements - the padding of a witness - cost nothing.  uneven: some rows hold many of them,

@@ -121,6 +121,34 @@ static void carried_lookups() {
     expect(carried(8, 18) == 0, "as are short proofs");
 }
 
+// A range of 2^23 entries has a row for each of them where rows are short (64 GiB for 64 columns): its indices, 2^23 among them, are
+// digits of the widest radix there is.
+static void the_longest_indexed_range() {
+    const uint cols = 64, gens = 1u << 12, log_len = 23, D = 1u << log_len;
+    bn128 G = bn128::one();
+    Hyrax hyrax(1, gens, device_points(256 * (size_t)gens), G, 1);
+    tLookupRange lookup(-(int)(D / 2), D);
+    FrTensor S(D), A(D);
+    const std::unique_ptr<FrTensor> ints(new FrTensor(D / 8));
+    double seconds = 0;
+    std::string error;
+    const unsigned long before = fake_launched("scaled_chain");
+    try {
+        lookup.prove(reinterpret_cast<const int*>(ints->gpu_data), S, A, random_vec(log_len), hyrax, cols, seconds);
+    } catch (const std::exception& e) {
+        error = e.what();
+    }
+    expect(fake_launched("scaled_chain") > before, "the table is built");
+    expect(error.find("tLookup_phase2: claim") == 0, "and the proof goes on to its claims, which do not hold here");
+    uint32_t *out = reinterpret_cast<uint32_t*>(device_points(8)), *flag = reinterpret_cast<uint32_t*>(device_points(1));
+    auto committed = [&](uint32_t len) {
+        return grape_commit_indexed(out, reinterpret_cast<const int32_t*>(ints->gpu_data), 2 * cols, cols, out, cols, len, 0, nullptr, 0,
+                                    reinterpret_cast<int32_t*>(flag), nullptr) == GRAPE_OK;
+    };
+    for (uint32_t len : {1u, 2u, 3u, 4u, 5u, 1u << 22, (1u << 23) - 1, 1u << 23}) expect(committed(len), "a table of that length");
+    expect(!committed(0) && !committed((1u << 23) + 1), "none and more are refused");
+}
+
 // A mapping's witness is S_in + r S_out with the r its caller sees: read as T[index] while T was made with it, written out otherwise (the
 // rounds then find that it is not T's).
 static void a_mapping_with_another_r() {
@@ -471,6 +499,7 @@ int main(int argc, char** argv) {
         {"proof_after_a_refused_one", proof_after_a_refused_one},
         {"mapping_objects", mapping_objects},
         {"carried_lookups", carried_lookups},
+        {"the_longest_indexed_range", the_longest_indexed_range},
         {"a_mapping_with_another_r", a_mapping_with_another_r},
         {"lookups_without_a_weighted_term", lookups_without_a_weighted_term},
         {"weights_that_are_read", weights_that_are_read},

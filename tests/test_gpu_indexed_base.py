@@ -21,13 +21,18 @@ def tables(ops):
     return gens, ops.g1_wide_table_gen(gens, 8, 32, 128), orc.g1_table(ops.g1_to_host(gens), 256)
 
 
+@pytest.mark.parametrize("length,base", [(1, 0), (2, 0), (2, 1), (8, 3), (64, 63)])
+def test_tables_of_a_power_of_two(ops, tables, length, base):
+    """the last index is the digit 2^(c-1) of its radix 2^c: it stays positive"""
+    test_base_entry(ops, tables, 7, 65, 0, length, base)
+
+
 @pytest.mark.parametrize("rows,cols,uneven", [(1, 1, 0), (1, 256, 1), (5, 65, 0), (37, 256, 1), (64, 100, 0), (600, 64, 1), (600, 128, 0)])
-def test_base_entry(ops, tables, rows, cols, uneven):
+def test_base_entry(ops, tables, rows, cols, uneven, length=9, base=3):
     import torch
     from grape_amd import _capi
     lib = ops.init()
     gens, wide, ref = tables
-    length, base = 9, 3
     B = rand_fr(length, 802)
     rng = np.random.default_rng(rows * cols)
     idx = rng.integers(0, length + 1, (rows, cols)).astype(np.int32)      # 0 is outside the table
