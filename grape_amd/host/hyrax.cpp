@@ -75,18 +75,29 @@ void Hyrax::check_shape(uint size, uint N) const {
     if (N != (1u << Log2(N))) throw std::runtime_error("N must be a power of 2");
 }
 
-// Builds (once) the wide table over the first `rowlen` generators; false when it exceeds the budget.
-bool Hyrax::ensure_table(WideTable& t, uint rowlen, uint c, uint nw, uint K) {
+// Builds (once) the wide table over the first `rowlen` generators; false when it exceeds the budget.  `optional`: also when there is no
+// device memory for it beside the one it would replace, which then stays.
+bool Hyrax::ensure_table(WideTable& t, uint rowlen, uint c, uint nw, uint K, bool optional) {
     if (t.d && t.ngen >= rowlen && t.c == c && t.nw == nw) return true;
     size_t bytes = grape_g1_wide_table_bytes(rowlen, nw, K);
     // against what every other table of this object holds (the one being replaced gives its bytes back)
-    if (!make_room(bytes, t.d ? grape_g1_wide_table_bytes(t.ngen, t.nw, t.K) : 0)) return false;
+    if (!make_room(bytes, t.d && !optional ? grape_g1_wide_table_bytes(t.ngen, t.nw, t.K) : 0)) return false;
     if (rowlen > npoints) throw std::runtime_error("row longer than the generator set");
-    grape_free(t.d);
-    t = WideTable();
-    check(grape_malloc((void**)&t.d, bytes), "grape_malloc");
+    if (!optional) {
+        grape_free(t.d);
+        t = WideTable();
+    }
+    affine_t* d = nullptr;
+    int rc = grape_malloc((void**)&d, bytes);
     // generators are row k = 1 of the reference-format table
-    check(grape_g1_wide_table_gen(W(t.d), W(g_affine + npoints), rowlen, c, nw, K, nullptr), "grape_g1_wide_table_gen");
+    if (rc == GRAPE_OK) rc = grape_g1_wide_table_gen(W(d), W(g_affine + npoints), rowlen, c, nw, K, nullptr);
+    if (rc != GRAPE_OK) {
+        grape_free(d);
+        if (optional && rc == GRAPE_ENOMEM) return false;
+        check(rc, "a table over the generators");
+    }
+    grape_free(t.d);
+    t.d = d;
     t.ngen = rowlen;
     t.c = c;
     t.nw = nw;
@@ -293,8 +304,9 @@ const Hyrax::WideTable* Hyrax::single_row_table(uint rowlen, void* stream) {
     if (rowlen > npoints || bytes > (size_t)4 << 30) return nullptr;
     const bool strided = fr_strided_.d && fr_strided_.ngen >= rowlen;
     row_saving_ms_ += 4.5e-3 * (strided ? (fr_strided_.J - 1) * fr_strided_.c : 248);
-    if (row_saving_ms_ < 0.2 + 1.35e-9 * (double)bytes || !ensure_table(row_table_, rowlen, c, nw, K)) return nullptr;
-    row_saving_ms_ = 0;
+    if (row_saving_ms_ < 0.2 + 1.35e-9 * (double)bytes) return nullptr;
+    row_saving_ms_ = 0;                                         // where there is no memory for it: tried again after as much
+    if (!ensure_table(row_table_, rowlen, c, nw, K, true)) return nullptr;
     if (stream) check(grape_stream_sync(nullptr), "sync");      // made on the default stream: another may read it only once it is there
     return &row_table_;
 }

@@ -119,7 +119,7 @@ private:
         uint ngen = 0, c = 0, J = 0, nsets = 0;
         bool spare = false;             // gives way to any other table (make_room)
     };
-    bool ensure_table(WideTable& t, uint rowlen, uint c, uint nw, uint K);
+    bool ensure_table(WideTable& t, uint rowlen, uint c, uint nw, uint K, bool optional = false);
     bool ensure_fr_table(uint rowlen, bool build = true);       // small per-window table (scaled-table builds)
     const WideTable* single_row_table(uint rowlen, void* stream);
     double row_saving_ms_ = 0;                                  // what a table for single rows would have saved so far

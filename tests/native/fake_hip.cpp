@@ -31,6 +31,7 @@ std::map<const void*, Kernel>& kernels() {
     return k;
 }
 unsigned long launches = 0, copies = 0, waits = 0;
+unsigned long limit = ~0ul;                              // bytes of the device's memory
 thread_local int device = 0;
 char symbol[1 << 24];
 
@@ -72,6 +73,8 @@ unsigned long fake_bytes() {
     for (auto& a : memory) n += a.second.bytes;
     return n;
 }
+// no more than `bytes` can be allocated together from now on
+void fake_limit(unsigned long bytes) { limit = bytes; }
 unsigned long fake_launches() { return launches; }
 // launches of the kernels whose name holds `part`
 unsigned long fake_launched(const char* part) {
@@ -102,6 +105,7 @@ hipError_t hipGetLastError() { return hipSuccess; }
 hipError_t hipMalloc(void** p, size_t bytes) {
     Lock l(mu);
     bytes = (bytes + 4095) & ~(size_t)4095;
+    if (limit != ~0ul && fake_bytes() + bytes > limit) return hipErrorOutOfMemory;
     void* m = mmap(nullptr, bytes, PROT_NONE, MAP_PRIVATE | MAP_ANONYMOUS | MAP_NORESERVE, -1, 0);
     if (m == MAP_FAILED) return hipErrorOutOfMemory;
     memory[(const char*)m] = Alloc{bytes, device};

@@ -21,6 +21,7 @@ unsigned long fake_copies();
 void fake_queue(const void* stream);
 unsigned long fake_waits();
 unsigned long fake_bytes();
+void fake_limit(unsigned long bytes);
 void fake_set_device(int device);
 }
 
@@ -393,6 +394,40 @@ static void verify_with_more_variables() {
     expect(!hyrax.verify(wrong, commitment, random_vec(6 + 2 + 40), c, rows * cols, cols), "a wrong one does not");
 }
 
+// A check's single row goes without a table of its own where the device has no memory for it, and asks for it again only now and then.
+static void single_rows_without_memory() {
+    const uint cols = 4096, rows = 4;
+    bn128 G = bn128::one();
+    Hyrax hyrax(1, cols, device_points(256 * cols), G, 1);
+    jacob_t* commitment = reinterpret_cast<jacob_t*>(device_points(2 * rows));
+    const Fr c(3);
+    Hyrax_proof proof = trivial_opening(G, c, cols);
+    auto checked = [&] {
+        const unsigned long before = fake_launched("wide_chain_kernel");
+        expect(hyrax.verify(proof, commitment, random_vec(12 + 2), c, rows * cols, cols), "the opening verifies");
+        return fake_launched("wide_chain_kernel") - before;
+    };
+    expect(checked() == 0, "the first row is worth no table");
+    fake_limit(fake_bytes() + (64ul << 20));
+    unsigned long tables = 0;
+    for (int i = 0; i < 20; i++) tables += checked();
+    expect(tables == 0, "without memory for one none is made");
+    fake_limit(fake_bytes() + (3ul << 30));
+    for (int i = 0; i < 20; i++) tables += checked();
+    expect(tables == 1, "with it one");
+    // rows of another length: there is memory for their table or for the one at hand, not for both
+    Hyrax two(1, 2 * cols, device_points(256 * 2 * cols), G, 1);
+    Hyrax_proof longer = trivial_opening(G, c, 2 * cols);
+    auto check_two = [&](Hyrax_proof& p, uint n) { expect(two.verify(p, commitment, random_vec(Log2(n) + 2), c, rows * n, n), "the opening verifies"); };
+    fake_limit(~0ul);
+    for (int i = 0; i < 20; i++) check_two(proof, cols);
+    const unsigned long at_hand = fake_launched("wide_chain_kernel");
+    fake_limit(fake_bytes() + (1ul << 30));
+    for (int i = 0; i < 20; i++) check_two(longer, 2 * cols);
+    for (int i = 0; i < 20; i++) check_two(proof, cols);
+    expect(at_hand == 2 && fake_launched("wide_chain_kernel") == at_hand, "the one at hand stays");
+}
+
 // the generator of an object is replaced between two checks
 static void verify_with_another_generator() {
     const uint cols = 64, rows = 4;
@@ -509,6 +544,7 @@ int main(int argc, char** argv) {
         {"element_products_that_carry", element_products_that_carry},
         {"a_tensor_times_itself", a_tensor_times_itself},
         {"verify_with_more_variables", verify_with_more_variables},
+        {"single_rows_without_memory", single_rows_without_memory},
         {"verify_with_another_generator", verify_with_another_generator},
         {"blocks_of_two_devices", blocks_of_two_devices},
         {"default_order_blocks", default_order_blocks},
