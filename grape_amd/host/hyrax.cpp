@@ -81,7 +81,12 @@ bool Hyrax::ensure_table(WideTable& t, uint rowlen, uint c, uint nw, uint K, boo
     if (t.d && t.ngen >= rowlen && t.c == c && t.nw == nw) return true;
     size_t bytes = grape_g1_wide_table_bytes(rowlen, nw, K);
     // against what every other table of this object holds (the one being replaced gives its bytes back)
-    if (!make_room(bytes, t.d && !optional ? grape_g1_wide_table_bytes(t.ngen, t.nw, t.K) : 0)) return false;
+    if (optional) {
+        // none of the others goes for it, and the one it would replace is there until it is made
+        if (table_bytes_in_use() + (fr_strided_.spare ? strided_bytes() : 0) + bytes_of(t) + bytes > table_budget_) return false;
+    } else if (!make_room(bytes, bytes_of(t))) {
+        return false;
+    }
     if (rowlen > npoints) throw std::runtime_error("row longer than the generator set");
     if (!optional) {
         grape_free(t.d);
@@ -185,20 +190,27 @@ affine_t* Hyrax::commit_affine_i32(int* tensor, uint size, uint N, int* d_flag, 
 size_t Hyrax::strided_bytes() const {
     return fr_strided_.d ? grape_g1_wide_table_bytes(fr_strided_.ngen, fr_strided_.nsets, 1u << (fr_strided_.c - 1)) : 0;
 }
-// without a strided table that gives way (make_room)
+size_t Hyrax::bytes_of(const WideTable& t) { return t.d ? grape_g1_wide_table_bytes(t.ngen, t.nw, t.K) : 0; }
+// without the tables that give way (make_room)
 size_t Hyrax::table_bytes_in_use() const {
     size_t used = scaled_bytes_;
-    for (const WideTable* t : {&int16_table_, &int16x2_table_, &int32_table_, &fr_table_, &row_table_})
-        if (t->d) used += grape_g1_wide_table_bytes(t->ngen, t->nw, t->K);
+    for (const WideTable* t : {&int16_table_, &int16x2_table_, &int32_table_, &fr_table_}) used += bytes_of(*t);
     return fr_strided_.spare ? used : used + strided_bytes();
 }
-// Is there room in the budget for a table of `bytes` that replaces one of `replaced` bytes?  A strided table that only sparse
-// commitments asked for goes if it stands in the way: it saves them a fifth to a half of their additions, while a scaled or int16
+void Hyrax::drop_row_table() {
+    grape_free(row_table_.d);
+    row_table_ = WideTable();
+}
+// Is there room in the budget for a table of `bytes` that replaces one of `replaced` bytes?  Two tables go if they stand in the way:
+// first the one for single rows, which saves a row a millisecond at most, then a strided table that only sparse
+// commitments asked for: it saves them a fifth to a half of their additions, while a scaled or int16
 // table that is not there costs 16 additions instead of one, or 2.
 bool Hyrax::make_room(size_t bytes, size_t replaced) {
     const size_t used = table_bytes_in_use() - replaced;
     if (used + bytes > table_budget_) return false;
-    if (fr_strided_.spare && used + strided_bytes() + bytes > table_budget_) {
+    const size_t spare = fr_strided_.spare ? strided_bytes() : 0;
+    if (used + spare + bytes_of(row_table_) + bytes > table_budget_) drop_row_table();
+    if (spare && used + spare + bytes > table_budget_) {
         grape_free(fr_strided_.d);
         fr_strided_ = StridedTable();
     }
@@ -220,7 +232,11 @@ bool Hyrax::ensure_fr_table(uint rowlen, bool build) {
         const size_t bytes = grape_g1_wide_table_bytes(rowlen, nw, K);
         // wide windows may take 48 GB, narrow ones (which lose to the strided table anyway) 16 GB
         const size_t cap = (size_t)(c >= 12 ? 48 : 16) << 30;
-        if (bytes <= cap && used + bytes <= table_budget_) return ensure_table(fr_table_, rowlen, c, nw, K);
+        if (bytes <= cap && used + bytes <= table_budget_) {
+            if (!ensure_table(fr_table_, rowlen, c, nw, K)) return false;
+            if (row_table_.ngen <= fr_table_.ngen) drop_row_table();     // single rows go through this one now
+            return true;
+        }
     }
     return false;
 }
@@ -279,6 +295,7 @@ bool Hyrax::ensure_strided_table(uint rowlen, bool build, const double* worth_ms
     // 64 GiB in 92 ms, 48 in 72 (4096 generators)
     const double build_ms = 1.35e-9 * (double)grape_g1_wide_table_bytes(ngen, bs, 1u << (bc - 1));
     if (worth_ms && (build_ms > *worth_ms || (fr_strided_.d && !fr_strided_.spare))) return false;
+    if (used + grape_g1_wide_table_bytes(ngen, bs, 1u << (bc - 1)) + bytes_of(row_table_) > table_budget_) drop_row_table();
     grape_free(fr_strided_.d);
     fr_strided_ = StridedTable();
     check(grape_malloc((void**)&fr_strided_.d, grape_g1_wide_table_bytes(ngen, bs, 1u << (bc - 1))), "grape_malloc");
@@ -295,7 +312,8 @@ bool Hyrax::ensure_strided_table(uint rowlen, bool build, const double* worth_ms
 // leaves no doublings, where there is one.  A strided table leaves (J - 1) c of them and the reference-format table 248, one
 // after the other on four lanes, 4.5 us each (4096 columns, whole openings: 0.4 and 1.5 ms against 0.3).  So once an object's
 // single rows have spent on doublings what a small table takes to make - 8-bit windows, 2 GiB and 3 ms for 4096 generators - it is
-// made; wider rows than 8192 would take more memory than an opening is worth.
+// made; wider rows than 8192 would take more memory than an opening is worth.  It gives way to any other table, and to the per-window one
+// over as many generators for good.
 const Hyrax::WideTable* Hyrax::single_row_table(uint rowlen, void* stream) {
     if (ensure_fr_table(rowlen, false)) return &fr_table_;
     constexpr uint c = 8, nw = 32, K = 128;

@@ -122,6 +122,8 @@ private:
     bool ensure_table(WideTable& t, uint rowlen, uint c, uint nw, uint K, bool optional = false);
     bool ensure_fr_table(uint rowlen, bool build = true);       // small per-window table (scaled-table builds)
     const WideTable* single_row_table(uint rowlen, void* stream);
+    void drop_row_table();
+    static size_t bytes_of(const WideTable& t);
     double row_saving_ms_ = 0;                                  // what a table for single rows would have saved so far
     bool ensure_strided_table(uint rowlen, bool build = true, const double* worth_ms = nullptr);  // the table full-width commitments go through
     size_t table_bytes_in_use() const;

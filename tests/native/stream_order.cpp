@@ -428,6 +428,51 @@ static void single_rows_without_memory() {
     expect(at_hand == 2 && fake_launched("wide_chain_kernel") == at_hand, "the one at hand stays");
 }
 
+// The table for single rows is in no other table's way: it goes for one that needs its bytes, and for a per-window table that serves
+// its rows, and it is not made where a table that gives way itself would have to go for it.
+static void single_row_table_gives_way() {
+    const uint cols = 4096, rows = 4;
+    bn128 G = bn128::one();
+    affine_t* gens = device_points(256 * cols);
+    jacob_t* commitment = reinterpret_cast<jacob_t*>(device_points(2 * rows));
+    const Fr c(3);
+    Hyrax_proof proof = trivial_opening(G, c, cols);
+    auto check_rows = [&](Hyrax& hyrax) {
+        const unsigned long before = fake_launched("wide_chain_kernel");
+        for (int i = 0; i < 20; i++) expect(hyrax.verify(proof, commitment, random_vec(12 + 2), c, rows * cols, cols), "the opening verifies");
+        return fake_launched("wide_chain_kernel") - before;
+    };
+    int* ints = reinterpret_cast<int*>(device_points(4 * cols));
+    {
+        Hyrax hyrax(1, cols, gens, G, 1);
+        hyrax.set_table_budget((size_t)16 << 30);
+        expect(check_rows(hyrax) == 1, "single rows have a table");
+        const unsigned long before = fake_bytes();
+        grape_free(hyrax.commit_affine(ints, 2 * cols, cols));
+        expect(fake_bytes() - before > (13ul << 30), "the one for 16-bit integers takes its place");
+        expect(check_rows(hyrax) == 0, "and keeps it");
+    }
+    {
+        Hyrax hyrax(1, cols, gens, G, 1), other(1, cols, gens, G, 1);
+        expect(check_rows(hyrax) == 1 && other.prepare_scaled_tables(cols), "single rows have a table");
+        const unsigned long before = fake_bytes();
+        expect(hyrax.prepare_scaled_tables(cols), "the per-window table fits");
+        expect(fake_bytes() - before < grape_g1_wide_table_bytes(cols, 20, 1u << 12) - (1ul << 30), "and serves them too");
+        expect(check_rows(hyrax) == 0, "so that no other is made");
+    }
+    Hyrax hyrax(1, cols, gens, G, 1);
+    hyrax.set_table_budget((size_t)96 << 30);
+    FrTensor A(1u << 21);
+    int* skip = reinterpret_cast<int*>(device_points(1u << 17));
+    const unsigned long none = fake_bytes();
+    for (int i = 0; i < 40; i++) grape_free(hyrax.commit_sparse_affine(A, skip, A.size, cols, A.size / 2));
+    const unsigned long spare = fake_bytes() - none;
+    expect(spare > (8ul << 30), "sparse commitments have a table");
+    hyrax.set_table_budget(spare + (1ul << 30));
+    const unsigned long before = fake_bytes();
+    expect(check_rows(hyrax) == 0 && fake_bytes() >= before, "single rows do not take its place");
+}
+
 // the generator of an object is replaced between two checks
 static void verify_with_another_generator() {
     const uint cols = 64, rows = 4;
@@ -545,6 +590,7 @@ int main(int argc, char** argv) {
         {"a_tensor_times_itself", a_tensor_times_itself},
         {"verify_with_more_variables", verify_with_more_variables},
         {"single_rows_without_memory", single_rows_without_memory},
+        {"single_row_table_gives_way", single_row_table_gives_way},
         {"verify_with_another_generator", verify_with_another_generator},
         {"blocks_of_two_devices", blocks_of_two_devices},
         {"default_order_blocks", default_order_blocks},
