@@ -455,8 +455,10 @@ static void single_row_table_gives_way() {
     {
         Hyrax hyrax(1, cols, gens, G, 1), other(1, cols, gens, G, 1);
         expect(check_rows(hyrax) == 1 && other.prepare_scaled_tables(cols), "single rows have a table");
+        grape_host::check(grape_alloc_cache_release(nullptr), "grape_alloc_cache_release");
         const unsigned long before = fake_bytes();
         expect(hyrax.prepare_scaled_tables(cols), "the per-window table fits");
+        grape_host::check(grape_alloc_cache_release(nullptr), "grape_alloc_cache_release");
         expect(fake_bytes() - before < grape_g1_wide_table_bytes(cols, 20, 1u << 12) - (1ul << 30), "and serves them too");
         expect(check_rows(hyrax) == 0, "so that no other is made");
     }
