@@ -310,8 +310,8 @@ bool Hyrax::ensure_strided_table(uint rowlen, bool build, const double* worth_ms
 
 // A single row (an opening's blinding row, the z of its check) is a short accumulation and a chain: through a per-window table, which
 // leaves no doublings, where there is one.  A strided table leaves (J - 1) c of them and the reference-format table 248, one
-// after the other on four lanes, 4.5 us each (4096 columns, whole openings: 0.4 and 1.5 ms against 0.3).  So once an object's
-// single rows have spent on doublings what a small table takes to make - 8-bit windows, 2 GiB and 3 ms for 4096 generators - it is
+// after the other on four lanes, 4.5 us each (4096 columns, whole openings: 0.4 and 1.5 ms against 0.3).  So for the first row behind
+// those that have spent on doublings what a small table takes to make - 8-bit windows, 2 GiB and 3 ms for 4096 generators - it is
 // made; wider rows than 8192 would take more memory than an opening is worth.  It gives way to any other table, and to the per-window one
 // over as many generators for good.
 const Hyrax::WideTable* Hyrax::single_row_table(uint rowlen, void* stream) {
@@ -320,9 +320,11 @@ const Hyrax::WideTable* Hyrax::single_row_table(uint rowlen, void* stream) {
     if (row_table_.d && row_table_.ngen >= rowlen) return &row_table_;
     const size_t bytes = grape_g1_wide_table_bytes(rowlen, nw, K);
     if (rowlen > npoints || bytes > (size_t)4 << 30) return nullptr;
-    const bool strided = fr_strided_.d && fr_strided_.ngen >= rowlen;
-    row_saving_ms_ += 4.5e-3 * (strided ? (fr_strided_.J - 1) * fr_strided_.c : 248);
-    if (row_saving_ms_ < 0.2 + 1.35e-9 * (double)bytes) return nullptr;
+    if (row_saving_ms_ < 0.2 + 1.35e-9 * (double)bytes) {
+        const bool strided = fr_strided_.d && fr_strided_.ngen >= rowlen;
+        row_saving_ms_ += 4.5e-3 * (strided ? (fr_strided_.J - 1) * fr_strided_.c : 248);
+        return nullptr;
+    }
     row_saving_ms_ = 0;                                         // where there is no memory for it: tried again after as much
     if (!ensure_table(row_table_, rowlen, c, nw, K, true)) return nullptr;
     if (stream) check(grape_stream_sync(nullptr), "sync");      // made on the default stream: another may read it only once it is there

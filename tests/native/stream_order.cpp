@@ -428,6 +428,33 @@ static void single_rows_without_memory() {
     expect(at_hand == 2 && fake_launched("wide_chain_kernel") == at_hand, "the one at hand stays");
 }
 
+// Which table a single row goes through: the reference-format one until such rows have cost a table, a strided one where there is one (its
+// doublings count too), the row's own from then on.
+static void tables_of_single_rows() {
+    const uint cols = 512, rows = 4;
+    bn128 G = bn128::one();
+    jacob_t* commitment = reinterpret_cast<jacob_t*>(device_points(2 * rows));
+    const Fr c(3);
+    Hyrax_proof proof = trivial_opening(G, c, cols);
+    auto path = [&](Hyrax& hyrax) {
+        const unsigned long ref = fake_launched("commit_ref30_kernel"), strided = fake_launched("commit_strided_kernel"), wide = fake_launched("commit_wide_kernel");
+        expect(hyrax.verify(proof, commitment, random_vec(9 + 2), c, rows * cols, cols), "the opening verifies");
+        return std::string(fake_launched("commit_ref30_kernel") - ref, 'r') + std::string(fake_launched("commit_strided_kernel") - strided, 's') +
+               std::string(fake_launched("commit_wide_kernel") - wide, 'w');
+    };
+    affine_t* gens = device_points(256 * cols);
+    Hyrax first(1, cols, gens, G, 1), none(1, cols, gens, G, 1), second(1, cols, gens, G, 1);
+    expect(path(first) == "r" && path(first) == "w" && path(first) == "w", "the reference-format table, then the row's own");
+    none.set_table_budget(0);
+    for (int i = 0; i < 5; i++) expect(path(none) == "r", "without a budget the reference-format table");
+    // half of the budget for a strided table, the rest too little for the row's own
+    second.set_table_budget((size_t)400 << 20);
+    FrTensor two(2 * cols);
+    grape_free(second.commit_affine(two, 2 * cols, cols));
+    expect(path(second) == "s", "a strided table");
+    for (int i = 0; i < 20; i++) expect(path(second) == "s", "for good where the row's own does not fit beside it");
+}
+
 // The table for single rows is in no other table's way: it goes for one that needs its bytes, and for a per-window table that serves
 // its rows, and it is not made where a table that gives way itself would have to go for it.
 static void single_row_table_gives_way() {
@@ -592,6 +619,7 @@ int main(int argc, char** argv) {
         {"a_tensor_times_itself", a_tensor_times_itself},
         {"verify_with_more_variables", verify_with_more_variables},
         {"single_rows_without_memory", single_rows_without_memory},
+        {"tables_of_single_rows", tables_of_single_rows},
         {"single_row_table_gives_way", single_row_table_gives_way},
         {"verify_with_another_generator", verify_with_another_generator},
         {"blocks_of_two_devices", blocks_of_two_devices},

@@ -1,6 +1,7 @@
 """Random elements from a key against a ChaCha20 written here from RFC 8439 (checked by the RFC's own block), and openings that
 commit their blinding row through every kind of table."""
 import ctypes
+import os
 import numpy as np
 import pytest
 import bigref as br
@@ -8,6 +9,9 @@ import orc
 from gpuutil import rand_fr, assert_same
 
 pytestmark = pytest.mark.gpu
+
+# the host objects are found by their table's address: it stays taken until the process ends
+_TABLES = []
 
 
 @pytest.fixture(scope="module")
@@ -63,15 +67,20 @@ def test_random_elements_of_a_key(ops, n):
     assert bool((out[n:] == -1).all()) and (n < 100 or retried > 10)
 
 
-def test_openings_of_a_single_row_through_every_table(ops):
-    """one row of 512: its commitment, the blinding row and the check all go through the reference-format table until their doublings
-    have cost a table of their own, then through that; two rows later through the strided one that their commitment makes"""
+@pytest.mark.parametrize("n,budget,rows_of", [(512, None, [1, 1, 1, 2, 1, 2]), (512, "0", [1, 1, 2]), (2048, "1", [2, 1, 1])])
+def test_openings_of_a_single_row_through_every_table(ops, monkeypatch, n, budget, rows_of):
+    """commitment, blinding row and check of one row: through the reference-format table and then through the row's own; through the
+    reference-format one alone, without a budget; through the strided table that a commitment of two rows makes of half of a GiB, beside which the
+    row's own does not fit (which path is taken when is counted on the host: tables_of_single_rows in native/stream_order.cpp)"""
     from grape_amd import _host as host
     host.load()
-    n = 512
+    if budget is not None:
+        monkeypatch.setitem(os.environ, "GRAPE_TABLE_BUDGET_GIB", budget)
     table = ops.g1_table_gen(ops.g1_make_generators(rand_fr(n, 920)), 256)
-    for i, rows in enumerate([1, 1, 1, 2, 1, 2]):
-        t, point, c = rand_fr(rows * n, 921 + i), rand_fr(9 + rows - 1, 930 + i), rand_fr(1, 940 + i)
+    _TABLES.append(table)
+    lg = n.bit_length() - 1
+    for i, rows in enumerate(rows_of):
+        t, point, c = rand_fr(rows * n, 921 + i), rand_fr(lg + rows - 1, 930 + i), rand_fr(1, 940 + i)
         res, ok = host.hyrax_open_verify(ops.to_dev(t), rows * n, n, table, n, point, c, com_scale=1)
         assert ok
         assert_same(res, orc.partial_eval(t, rows * n, point, rows * n, 0, 1)[0], "value %d" % i)
