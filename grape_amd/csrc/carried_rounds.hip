@@ -19,7 +19,7 @@
 // wround2_kernel: the gathered first round of 2^26 pairs 2.8 -> 2.1 ms, a round of 2^25 pairs 1.77 -> 1.34 ms, the first
 // round of a 2048 x 11008 element product 0.69 -> 0.61 ms and its second 0.36 -> 0.23 ms.  A thread's next operands are asked
 // for before this pair's arithmetic: two waves a SIMD do not cover the loads (2048 x 11008 proof 1.33 -> 1.29 ms).
-// Proofs run the rounds two to a pass (pair_carried_round_kernel), an odd one's last alone.
+// Proofs run the rounds two to a pass (carried_pair_kernel), an odd one's last alone.
 #include "fr_device.hpp"
 
 namespace grape {
@@ -179,7 +179,7 @@ struct CarriedPair {
     uint32_t *partial, *next_partial;
 };
 template <int MODE, bool PLAIN>
-__device__ __forceinline__ void carried_pair(const CarriedPair& p) {
+__global__ void __launch_bounds__(kBlock, MODE == kGather ? 3 : 2) carried_pair_kernel(CarriedPair p) {
     constexpr bool SUMS = MODE != kGather;                  // the first round has weighted sums
     constexpr int V0 = SUMS ? 2 : 0, NV = V0 + 1 + (PLAIN ? 2 : 0), NW = kBlock / 64;
     __shared__ Fr lds[NV * 2 * NW];
@@ -315,12 +315,6 @@ __device__ __forceinline__ void carried_pair(const CarriedPair& p) {
     }
 }
 
-template <int MODE, bool PLAIN>
-__global__ void __launch_bounds__(kBlock, 2) pair_carried_round_kernel(CarriedPair p) {
-    carried_pair<MODE, PLAIN>(p);
-}
-__global__ void __launch_bounds__(kBlock, 3) pair_carried_gather_kernel(CarriedPair p) { carried_pair<kGather, true>(p); }
-
 constexpr uint32_t kMaxCarried = 32;
 struct CarriedFinish {
     const uint32_t* partial[kMaxCarried];
@@ -329,7 +323,7 @@ struct CarriedFinish {
 };
 // NW weighted sums go to out[0 ..), times the radix factor 16 that they leave their kernel without, NV - NW plain ones to out[3 ..)
 template <int NV, int NW, int BLOCK>
-__global__ void __launch_bounds__(BLOCK) carried_round_kernel_sums(CarriedFinish f) {
+__global__ void __launch_bounds__(BLOCK) carried_final_kernel(CarriedFinish f) {
     __shared__ uint32_t lds9[NV * (BLOCK / 64) * 9];
     Fr tot[NV];
     workgroup_totals<NV, BLOCK>(tot, f.partial[blockIdx.x], f.nblocks[blockIdx.x], lds9);
@@ -463,7 +457,7 @@ int grape_carried_queue_pair(const grape_carried_args* first, const grape_carrie
         CHECK_PTR16(a.halves); CHECK_PTR16(a.eq_high);
         GRAPE_REQUIRE(a.len >= 1, "empty table");
         GRAPE_REQUIRE(b.plain_sums, "a lookup's later rounds have plain sums");
-        pair_carried_gather_kernel<<<nb, kBlock, 0, s>>>(p);
+        carried_pair_kernel<kGather, true><<<nb, kBlock, 0, s>>>(p);
         GRAPE_LAUNCH_CHECK();
         return GRAPE_OK;
     }
@@ -473,11 +467,11 @@ int grape_carried_queue_pair(const grape_carried_args* first, const grape_carrie
     if (a.eq_high) {
         CHECK_PTR16(a.eq_high);
         GRAPE_REQUIRE(!a.plain_sums, "the weights enter in a round without plain sums");
-        pair_carried_round_kernel<kEnter, false><<<nb, kBlock, 0, s>>>(p);
+        carried_pair_kernel<kEnter, false><<<nb, kBlock, 0, s>>>(p);
     } else {
         GRAPE_REQUIRE(a.tab_z != nullptr, "the round needs the carried tensor's table");
-        if (a.plain_sums) pair_carried_round_kernel<kLater, true><<<nb, kBlock, 0, s>>>(p);
-        else pair_carried_round_kernel<kLater, false><<<nb, kBlock, 0, s>>>(p);
+        if (a.plain_sums) carried_pair_kernel<kLater, true><<<nb, kBlock, 0, s>>>(p);
+        else carried_pair_kernel<kLater, false><<<nb, kBlock, 0, s>>>(p);
     }
     GRAPE_LAUNCH_CHECK();
     return GRAPE_OK;
@@ -499,8 +493,8 @@ int grape_carried_finish(uint32_t* sums, uint32_t stride, const grape_carried_ar
     hipStream_t s = as_stream(st);
 #define GRAPE_CFINAL(NV, NW)                                                                                   \
     do {                                                                                                       \
-        if (nb >= kFinalWideMin) carried_round_kernel_sums<NV, NW, kFinalBlock><<<count, kFinalBlock, 0, s>>>(f);   \
-        else carried_round_kernel_sums<NV, NW, kBlock><<<count, kBlock, 0, s>>>(f);                                 \
+        if (nb >= kFinalWideMin) carried_final_kernel<NV, NW, kFinalBlock><<<count, kFinalBlock, 0, s>>>(f);   \
+        else carried_final_kernel<NV, NW, kBlock><<<count, kBlock, 0, s>>>(f);                                 \
     } while (0)
     if (rounds[0].idx1) GRAPE_CFINAL(2, 0);
     else if (rounds[0].plain_sums) GRAPE_CFINAL(4, 2);

@@ -389,13 +389,8 @@ static Fr eleMul_rounds(fr_t* Aw, fr_t* Bw, const fr_t* A, const fr_t* B, fr_t* 
             partials.emplace_back(new DeviceBuf(grape_carried_partial_bytes(&carried[i])));
             carried[i].partial = W(partials.back()->fr());
         }
-        // a pass's sums are finished behind it, while the caches hold its partial sums; an odd round's with the pass before
-        for (uint i = 0; i < carrying; i += 2) {
-            const uint n = std::min(i + 3 == carrying ? 3u : 2u, carrying - i);
-            CarriedFactors::queue_passes(&carried[i], n, nullptr);
-            check(grape_carried_finish(W(sums.gpu_data + 3 * i), 3, &carried[i], n, nullptr), "grape_carried_finish");
-            if (n == 3) break;
-        }
+        CarriedFactors::queue_passes(carried.data(), carrying, nullptr);
+        check(grape_carried_finish(W(sums.gpu_data), 3, carried.data(), carrying, nullptr), "grape_carried_finish");
         check(grape_carried_end(W(Bw), W(Bw), in, W(consts->fr() + carrying), period, nullptr, nullptr), "grape_carried_end");
         if (in == second_size) out = 1u << (Log2(in) - 1);     // a row's own variables: those of its padded length
     }

@@ -110,12 +110,12 @@ static void carried_lookups() {
         tLookupRange lookup(-(int)(1u << (log_len - 1)), 1u << log_len);
         FrTensor S(D), A(D);
         const std::unique_ptr<FrTensor> ints(new FrTensor(D / 8));
-        const unsigned long before = fake_launched("carried_gather_kernel");
+        const unsigned long before = fake_launched("carried_pair_kernelILi2E");          // the kind whose first round gathers
         try {
             lookup.prove(reinterpret_cast<const int*>(ints->gpu_data), S, A, random_vec(log_D), hyrax, cols, seconds);
         } catch (const std::exception&) {                    // nothing is computed here, so its claims do not hold
         }
-        return fake_launched("carried_gather_kernel") - before;
+        return fake_launched("carried_pair_kernelILi2E") - before;
     };
     expect(carried(8, 19) == 1 && carried(19, 19) == 1 && carried(24, 24) == 1, "tables of up to 2^24 entries");
     expect(carried(25, 25) == 0 && carried(30, 30) == 0, "longer ones are left to the weighted rounds");
@@ -337,19 +337,43 @@ static void operands_at_any_address() {
     }
 }
 
+// passes over the long rounds that carry their weights, two rounds each or one, and the launches that finish their sums
+struct CarriedLaunches {
+    unsigned long pairs = 0, singles = 0, finished = 0;
+    static CarriedLaunches now() {
+        CarriedLaunches c;
+        c.pairs = fake_launched("carried_pair_kernel");
+        c.singles = fake_launched("carried_round_kernel");
+        c.finished = fake_launched("carried_final_kernel");
+        return c;
+    }
+    CarriedLaunches since(const CarriedLaunches& before) const {
+        CarriedLaunches c;
+        c.pairs = pairs - before.pairs;
+        c.singles = singles - before.singles;
+        c.finished = finished - before.finished;
+        return c;
+    }
+    unsigned long rounds() const { return 2 * pairs + singles; }
+    bool none() const { return pairs + singles + finished == 0; }
+    // every round but an odd one's last runs in a pass of two, and one launch finishes all sums
+    bool carried(unsigned long n) const { return rounds() == n && singles == n % 2 && finished == 1; }
+};
+
 // An element product carries its weights where few rows are left in the end: each of them costs the host a factor.
 static void element_products_that_carry() {
     uint32_t *a = reinterpret_cast<uint32_t*>(device_points(1u << 20)), claim[8] = {0}, transcript[32 * 32], rounds, at_a[8], at_b[8];
     std::vector<uint32_t> point(8 * 32, 3);
-    auto carried = [&](uint rows, uint cols) {
-        const unsigned long before = fake_launched("carried_round_kernel");
+    auto product = [&](uint rows, uint cols) {
+        const CarriedLaunches before = CarriedLaunches::now();
         const int vars = (int)Log2(rows) + (int)Log2(cols);
         grape_host_prove_elemul(a, a, 1, rows, cols, point.data(), vars, point.data(), vars, claim, transcript, &rounds, at_a, at_b);
-        return fake_launched("carried_round_kernel") - before;
+        return CarriedLaunches::now().since(before);
     };
     grape_host_set_input_format(0);
-    expect(carried(1u << 10, 3000) == 5 && carried(1u << 11, 1u << 10) == 5 && carried(1u << 13, 257) == 5, "from rows of 256 on");
-    expect(carried(1u << 19, 5) == 0 && carried(1u << 15, 65) == 0 && carried(1u << 14, 255) == 0, "not with shorter rows");
+    expect(product(1u << 10, 3000).carried(5) && product(1u << 11, 1u << 10).carried(5) && product(1u << 13, 257).carried(5), "from rows of 256 on");
+    expect(product(1u << 11, 3000).carried(6), "an even number of rounds");
+    expect(product(1u << 19, 5).none() && product(1u << 15, 65).none() && product(1u << 14, 255).none(), "not with shorter rows");
 }
 
 // A tensor times itself, both operands bound in the one buffer: the weighted half would overwrite the plain one, and from the second
@@ -357,15 +381,15 @@ static void element_products_that_carry() {
 static void a_tensor_times_itself() {
     const uint rows = 1u << 10, cols = 1u << 11;
     const std::vector<Fr> point(Log2(rows) + Log2(cols), Fr(3));
-    auto carried = [&](FrTensor& x, FrTensor& y) {
-        const unsigned long before = fake_launched("carried_round_kernel");
+    auto product = [&](FrTensor& x, FrTensor& y) {
+        const CarriedLaunches before = CarriedLaunches::now();
         Fr claim = Fr::zero();
         prove_eleMul(x, y, 1, rows, cols, point, point, claim);
-        return fake_launched("carried_round_kernel") - before;
+        return CarriedLaunches::now().since(before);
     };
     FrTensor x(rows * cols), y(rows * cols);
-    expect(carried(x, y) == 5, "two tensors carry");
-    expect(carried(x, x) == 0, "one tensor does not");
+    expect(product(x, y).carried(5), "two tensors carry");
+    expect(product(x, x).none(), "one tensor does not");
 }
 
 // An opening that verifies here: every commitment is the identity (device memory reads as zero), so its two equations are
