@@ -90,11 +90,14 @@ __global__ void __launch_bounds__(kBlock) pad_i32_kernel(int32_t* out, const int
 // reductions
 // ------------------------------------------------------------------------------------------------
 // Grid-stride partial sums, one for each workgroup.  ONCE: the last workgroup to leave its own adds them up, so that a sum is
-// one launch instead of two (*ticket is zero between launches).  Up to kSumOnce elements, over at most 64 workgroups: 2^16
-// elements behind a product 21.8 -> 18.7 us, most of it calls and launches.  Every workgroup pays for a fence and for its turn
-// at the counter, and where it is one of thousands that is more than a launch (2^20 elements 33 -> 52 us, 2^24 380 -> 473).
+// one launch instead of two (*ticket is zero between launches).  Up to kSumOnce elements, over at most kSumOnceBlocks workgroups, behind
+// a product of as many elements: 2^16 20.5 to 21.6 -> 18.2 to 18.9 us, 190 003 20.8 to 21.9 -> 18.3 to 19.3, 2^19 23.2 -> 20.8, most of it
+// calls and launches (64 workgroups: 21.4 at 2^19, 256: 22.7).  From 2^20 elements on reading them is what takes the time: 32.5 us
+// either way.  Every workgroup pays for a fence and for its turn at the counter, and where it is one of
+// thousands that is more than a launch (2^20 elements 33 -> 52 us, 2^24 380 -> 473).
 constexpr int kSumTerms = 4;               // loads a thread of a short sum has in flight
-constexpr size_t kSumOnce = 1 << 17;
+constexpr size_t kSumOnce = 1 << 19;
+constexpr unsigned kSumOnceBlocks = 128;
 template <bool ONCE>
 __global__ void __launch_bounds__(kBlock) sum_kernel(uint32_t* out, const uint32_t* in, size_t n, uint32_t* partial, uint32_t* ticket) {
     __shared__ Fr lds[kBlock / 64];
@@ -716,7 +719,7 @@ int grape_fr_sum(uint32_t* out, const uint32_t* in, size_t n, grape_stream_t st)
     }
     const bool once = n <= kSumOnce;
     unsigned nb = blocks_for(n, once ? kBlock * kSumTerms : kBlock);
-    const unsigned most = once ? 64 : kNumCU * 8;
+    const unsigned most = once ? kSumOnceBlocks : kNumCU * 8;
     if (nb > most) nb = most;
     void *ws, *ticket;
     int rc = scratch_get(kSlotReduce, (size_t)nb * 32, &ws, s);

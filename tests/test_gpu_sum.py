@@ -15,7 +15,7 @@ def ops():
     return ops
 
 
-@pytest.mark.parametrize("n", [1, 255, 256, 1024, 1025, 2048, 3000, 65536, 65537, 1 << 17, (1 << 17) + 1, (1 << 21) - 1, (1 << 21) + 1, (1 << 22) + 4099])
+@pytest.mark.parametrize("n", [1, 255, 256, 1024, 1025, 2048, 3000, 65536, 65537, 1 << 17, (1 << 17) + 1, 190003, 1 << 19, (1 << 19) + 1, (1 << 21) - 1, (1 << 21) + 1, (1 << 22) + 4099])
 def test_sum(ops, n):
     import torch
     a = rand_fr(min(n, 1 << 16), n & 0xffff)
