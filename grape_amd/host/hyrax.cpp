@@ -388,17 +388,21 @@ affine_t* Hyrax::build_scaled_table(const FrTensor& scalars, uint ncols) {
     if (!ensure_fr_table(ncols)) return nullptr;
     if (!make_room(bytes, 0)) return nullptr;
     affine_t* out = nullptr;
-    check(grape_malloc((void**)&out, bytes), "grape_malloc");
-    gen_scaled(out, scalars, ncols);
+    int rc = grape_malloc((void**)&out, bytes);
+    if (rc == GRAPE_OK) rc = gen_scaled(out, scalars, ncols);
+    if (rc != GRAPE_OK) {
+        grape_free(out);
+        if (rc == GRAPE_ENOMEM) return nullptr;
+        check(rc, "a scaled table");
+    }
     scaled_bytes_ += bytes;
     scaled_registry()[out] = ScaledTable{this, bytes, false};
     return out;
 }
 
-void Hyrax::gen_scaled(affine_t* out, const FrTensor& scalars, uint ncols) {
-    check(grape_g1_scaled_table_gen(W(out), W(scalars.gpu_data), scalars.size, ncols, W(fr_table_.d), fr_table_.ngen, fr_table_.c,
-                                    fr_table_.nw, fr_table_.K, nullptr),
-          "grape_g1_scaled_table_gen");
+int Hyrax::gen_scaled(affine_t* out, const FrTensor& scalars, uint ncols) {
+    return grape_g1_scaled_table_gen(W(out), W(scalars.gpu_data), scalars.size, ncols, W(fr_table_.d), fr_table_.ngen, fr_table_.c, fr_table_.nw,
+                                     fr_table_.K, nullptr);
 }
 
 size_t Hyrax::most_scaled_rows(const affine_t* table, uint ncols) const {
@@ -414,9 +418,14 @@ bool Hyrax::extend_scaled_table(affine_t*& table, uint rows, uint& capacity, con
     const size_t row_bytes = grape_g1_wide_table_bytes(ncols, 1, 1), need = (size_t)rows + more.size, most = most_scaled_rows(table, ncols);
     if (need > most || !ensure_fr_table(ncols)) return false;
     if (need > capacity) {
-        // with room for twice as many where the share allows it: the rows are copied (4.7 TB/s) a bounded number of times
-        const size_t room = std::max(need, std::min(most, 2 * (size_t)capacity)), bytes = room * row_bytes;
-        if (!make_room(bytes, it->second.bytes)) return false;
+        // with room for twice as many where the share allows it: the rows are copied (4.7 TB/s) a bounded number of times.  Both
+        // tables are there while that is done, and the budget holds both; where it does not, room for what is needed has to do.
+        size_t room = std::max(need, std::min(most, 2 * (size_t)capacity));
+        if (!make_room(room * row_bytes, 0)) {
+            room = need;
+            if (!make_room(room * row_bytes, 0)) return false;
+        }
+        const size_t bytes = room * row_bytes;
         affine_t* out = nullptr;
         const int rc = grape_malloc((void**)&out, bytes);
         if (rc == GRAPE_ENOMEM) return false;
@@ -429,7 +438,9 @@ bool Hyrax::extend_scaled_table(affine_t*& table, uint rows, uint& capacity, con
         capacity = (uint)room;
     }
     it->second.extended = true;
-    gen_scaled(reinterpret_cast<affine_t*>(reinterpret_cast<char*>(table) + (size_t)rows * row_bytes), more, ncols);
+    const int rc = gen_scaled(reinterpret_cast<affine_t*>(reinterpret_cast<char*>(table) + (size_t)rows * row_bytes), more, ncols);
+    if (rc == GRAPE_ENOMEM) return false;
+    check(rc, "grape_g1_scaled_table_gen");
     return true;
 }
 

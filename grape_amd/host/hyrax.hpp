@@ -67,7 +67,7 @@ public:
     void verify(Hyrax_proof& proof, jacob_t* commitment, Fr c, uint size, uint N);
 
     // Scaled table out[t*ncols + i] = scalars[t] * G_i over the first ncols generators (device,
-    // owned by the caller, freed with grape_free); nullptr when it would not fit the budget.
+    // owned by the caller, freed with grape_free); nullptr when it would not fit the budget or the device's memory.
     // With it, a tensor whose elements are scalars[idx] commits at one addition per element:
     affine_t* build_scaled_table(const FrTensor& scalars, uint ncols);
     affine_t* commit_row(FrTensor& row);             // one row over the first row.size generators, whatever the layers
@@ -142,7 +142,7 @@ private:
     StridedTable fr_strided_;
     bool int16_ok_ = true;
     size_t scaled_bytes_ = 0;
-    void gen_scaled(affine_t* out, const FrTensor& scalars, uint ncols);
+    int gen_scaled(affine_t* out, const FrTensor& scalars, uint ncols);
     std::vector<Fr> last_open_point_;
     std::unique_ptr<G1FixedBase> G_multiples_;      // built by the first opening or verification
     bn128 G_multiples_of_;

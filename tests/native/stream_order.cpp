@@ -324,6 +324,38 @@ static void sparse_commitment_table() {
     expect(other.table_bytes_free() < (size_t)16 << 30 && other.build_scaled_table(B, cols) == nullptr, "a table in use by others does not give way");
 }
 
+// A scaled table that grows by moving: the budget holds the old and the new one, and where it or the device's memory does not, the
+// table stays as it was.  One that there is no memory for is not made.
+static void scaled_tables_that_grow() {
+    const uint cols = 256, rows = 1u << 16;
+    const unsigned long row_bytes = grape_g1_wide_table_bytes(cols, 1, 1);
+    bn128 G = bn128::one();
+    Hyrax hyrax(1, cols, device_points(256 * cols), G, 1);
+    hyrax.set_table_budget((size_t)64 << 30);
+    expect(hyrax.prepare_scaled_tables(cols), "the per-window table fits");
+    FrTensor B(rows), more(1);
+    affine_t* table = hyrax.build_scaled_table(B, cols);
+    affine_t* const first = table;
+    const size_t used = ((size_t)64 << 30) - hyrax.table_bytes_free();
+    uint capacity = rows;
+    auto unchanged = [&] { return table == first && capacity == rows && hyrax.table_bytes_free() + used <= (size_t)64 << 30; };
+    // the eighth of the budget that tables may grow into holds the new one, the rest of it not the old one beside it
+    FrTensor C((uint)((((size_t)64 << 30) - used - rows * row_bytes) / row_bytes));
+    affine_t* rest = hyrax.build_scaled_table(C, cols);
+    expect(table && rest && hyrax.table_bytes_free() > rows / 2 * row_bytes, "two tables, and room for half of the first");
+    expect(!hyrax.extend_scaled_table(table, rows, capacity, more, cols) && unchanged(), "no room for both");
+    Hyrax::release_scaled_table(rest);
+    grape_host::check(grape_alloc_cache_release(nullptr), "grape_alloc_cache_release");
+    fake_limit(fake_bytes() + (1ul << 30));
+    expect(!hyrax.extend_scaled_table(table, rows, capacity, more, cols) && unchanged(), "no memory for both");
+    expect(hyrax.build_scaled_table(B, cols) == nullptr && unchanged(), "none for another table");
+    fake_limit(~0ul);
+    expect(hyrax.extend_scaled_table(table, rows, capacity, more, cols) && table != first && capacity > rows, "with both it grows");
+    const affine_t* second = table;
+    expect(hyrax.extend_scaled_table(table, rows + 1, capacity, more, cols) && table == second, "and then in place");
+    Hyrax::release_scaled_table(table);
+}
+
 // operands of the C calls at addresses that are multiples of 4 only
 static void operands_at_any_address() {
     uint32_t* at = reinterpret_cast<uint32_t*>(device_points(4096));
@@ -638,6 +670,7 @@ int main(int argc, char** argv) {
         {"weights_that_are_read", weights_that_are_read},
         {"tensor_memory_is_idle", tensor_memory_is_idle},
         {"sparse_commitment_table", sparse_commitment_table},
+        {"scaled_tables_that_grow", scaled_tables_that_grow},
         {"operands_at_any_address", operands_at_any_address},
         {"element_products_that_carry", element_products_that_carry},
         {"a_tensor_times_itself", a_tensor_times_itself},
