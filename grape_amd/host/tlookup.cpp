@@ -132,8 +132,8 @@ void tLookup::gather_by_index(FrTensor& out, const FrTensor& table, uint D) {
     check(grape_fr_gather(W(out.gpu_data), W(table.gpu_data) - 8, reinterpret_cast<const uint32_t*>(d_idx_), D, nullptr), "grape_fr_gather");   // d_idx_ holds index + 1
 }
 
-FrTensor& tLookup::scaled_by() {
-    if (base_ < 0) return B;
+FrTensor& tLookup::scaled_by(bool based) {
+    if (!based) return B;
     if (!B_less_base_) {
         B_less_base_.reset(new FrTensor(B));
         const Fr less = Fr::zero() - B((uint)base_);
@@ -141,8 +141,8 @@ FrTensor& tLookup::scaled_by() {
     }
     return *B_less_base_;
 }
-const void* tLookup::base_point(Hyrax& hyrax, uint msm_size) {
-    if (base_ < 0) return nullptr;
+const void* tLookup::base_point(Hyrax& hyrax, uint msm_size, bool based) {
+    if (!based) return nullptr;
     const uint rowlen = msm_size * hyrax.com_scale;
     if (base_cols_ != rowlen) {
         FrTensor row(rowlen, OnDefaultStream());
@@ -159,6 +159,16 @@ const void* tLookup::base_point(Hyrax& hyrax, uint msm_size) {
 }
 namespace {
 constexpr int kBaseMark = 0x7fffffff;            // the slot of the base entry: no row's
+constexpr uint kBasedElements = 1u << 20;        // a range's table made for a witness this long is less B[base] also where that is not padded
+}
+// the elements of the base entry that had no slot; they take no addition now
+uint64_t tLookup::mark_base(int* slots) {
+    int slot = 0;
+    uint32_t count = 0;
+    check(grape_memcpy_d2h(&slot, slots + base_, sizeof slot, nullptr), "grape_memcpy_d2h");
+    if (!slot) check(grape_memcpy_d2h(&count, d_hist_ + base_, sizeof count, nullptr), "grape_memcpy_d2h");
+    check(grape_memcpy_h2d(slots + base_, &kBaseMark, sizeof kBaseMark, nullptr), "grape_memcpy_h2d");
+    return count;
 }
 
 // com(A) through the entries that occur often.  A[i] = B[index_i]; an entry t that occurs n_t times
@@ -218,14 +228,15 @@ uint64_t tLookup::grow_hot_rows(Hyrax& hyrax, const uint64_t info[3]) {
         const uint n_new = (uint)given[0];
         if (n_new != 0) {
             FrTensor more(n_new, OnDefaultStream());
-            check(grape_fr_gather(W(more.gpu_data), W(scaled_by().gpu_data), d_list, n_new, nullptr), "grape_fr_gather");
+            if (!hot_table_) hot_based_ = padding_is_free();
+            check(grape_fr_gather(W(more.gpu_data), W(scaled_by(hot_based_).gpu_data), d_list, n_new, nullptr), "grape_fr_gather");
             bool built;
             if (hot_table_) {
                 built = hyrax.extend_scaled_table(hot_table_, hot_rows_, hot_capacity_, more, hot_cols_);
             } else {
                 hot_table_ = hyrax.build_scaled_table(more, hot_cols_);
                 base_cols_ = 0;
-                if (hot_table_ && base_ >= 0) check(grape_memcpy_h2d(slots + base_, &kBaseMark, sizeof(int), nullptr), "grape_memcpy_h2d");
+                if (hot_table_ && hot_based_) given[1] -= mark_base(slots);
                 built = hot_table_ != nullptr;
                 hot_capacity_ = built ? n_new : 0;
             }
@@ -295,10 +306,11 @@ bool tLookup::commit_A_by_occupancy(uint D, uint msm_size, Hyrax& hyrax) {
             cold = info[1];
             if (n_hot != 0) {
                 FrTensor Bhot(n_hot, OnDefaultStream());
-                check(grape_fr_gather(W(Bhot.gpu_data), W(scaled_by().gpu_data), d_list, n_hot, nullptr), "grape_fr_gather");
+                hot_based_ = padding_is_free();
+                check(grape_fr_gather(W(Bhot.gpu_data), W(scaled_by(hot_based_).gpu_data), d_list, n_hot, nullptr), "grape_fr_gather");
                 hot_table_ = hyrax.build_scaled_table(Bhot, rowlen);
                 base_cols_ = 0;
-                if (hot_table_ && base_ >= 0) check(grape_memcpy_h2d(hot_slot1_ + base_, &kBaseMark, sizeof(int), nullptr), "grape_memcpy_h2d");
+                if (hot_table_ && hot_based_) cold -= mark_base(hot_slot1_);
                 if (!hot_table_) check(grape_memset_zero(hot_slot1_, sizeof(int) * (size_t)N, nullptr), "grape_memset_zero");
             }
             hot_rows_ = hot_capacity_ = hot_table_ ? n_hot : 0;
@@ -322,13 +334,13 @@ bool tLookup::commit_A_by_occupancy(uint D, uint msm_size, Hyrax& hyrax) {
     try {
         check(grape_malloc_on_default((void**)&d_hot, sizeof(int) * (size_t)D), "grape_malloc");
         check(grape_tlookup_hot_index(d_hot, d_idx_, D, hot_slot1_, N, nullptr), "grape_tlookup_hot_index");
-        com_A = hyrax.commit_indexed_affine(d_hot, D, msm_size, hot_table_, rowlen, hot_rows_, nullptr, kBaseMark, base_point(hyrax, msm_size), padded_);
+        com_A = hyrax.commit_indexed_affine(d_hot, D, msm_size, hot_table_, rowlen, hot_rows_, nullptr, kBaseMark, base_point(hyrax, msm_size, hot_based_), padded_);
         if (cold != 0) {
             // the elements without a table row: queued per row and committed as full-width scalars
-            com_cold = hyrax.commit_sparse_affine(scaled_by(), d_hot, D, msm_size, cold, d_idx_);
+            com_cold = hyrax.commit_sparse_affine(scaled_by(hot_based_), d_hot, D, msm_size, cold, d_idx_);
             if (!com_cold) {
                 FrTensor Acold(D, OnDefaultStream());
-                gather_by_index(Acold, scaled_by(), D);
+                gather_by_index(Acold, scaled_by(hot_based_), D);
                 check(grape_fr_mask_cold(W(Acold.gpu_data), W(Acold.gpu_data), d_hot, D, nullptr), "grape_fr_mask_cold");
                 com_cold = hyrax.commit_affine(Acold, D, msm_size);
             }
@@ -543,7 +555,8 @@ Fr tLookup::run(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax& hyrax
         if (indexed_commit_ && index_known_ &&
             (scaled_for_ != &hyrax || scaled_cols_ < rowlen || (scaled_table_ && !hyrax.owns_scaled_table(scaled_table_)))) {
             Hyrax::release_scaled_table(scaled_table_);
-            scaled_table_ = hyrax.build_scaled_table(scaled_by(), rowlen);   // nullptr when over budget
+            scaled_based_ = padding_is_free() || (base_ >= 0 && D >= kBasedElements);
+            scaled_table_ = hyrax.build_scaled_table(scaled_by(scaled_based_), rowlen);   // nullptr when over budget
             B_less_base_.reset();                    // every entry has its row
             base_cols_ = 0;
             scaled_cols_ = scaled_table_ ? rowlen : 0;
@@ -552,7 +565,7 @@ Fr tLookup::run(FrTensor& S, FrTensor& A, const std::vector<Fr>& v, Hyrax& hyrax
     });
     const bool indexed = indexed_commit_ && index_known_ && scaled_table_;
     const void* start = nullptr;                 // made here, where the host may wait
-    if (indexed) timed([&] { start = base_point(hyrax, msm_size); });
+    if (indexed) timed([&] { start = base_point(hyrax, msm_size, scaled_based_); });
     const bool overlap = indexed && d_idx_ != nullptr;
     // A = 1/(S + beta): read from B where the witness matches its table entry (every element of
     // a valid witness does), computed by batched inversion otherwise (tlookup_inv_kernel,

@@ -104,17 +104,23 @@ protected:
     uint32_t* hot_credit_ = nullptr;    // occurrences of entries without a row in the proofs since the rows were made
     double hot_missed_ = 0;             // elements of entries that had earned a row when there was no more room for it
     uint64_t grow_hot_rows(Hyrax& hyrax, const uint64_t info[3]);
-    // The entry a witness is padded with, the key 0 (-1: not in the table).  Its elements - a third of a witness of rows of 11008, the
-    // zeros of any other - take no addition: the rows of both tables hold (B[t] - B[base]) G_i, and every committed row starts at
-    // sum_i B[base] G_i.
+    // The entry a witness is padded with, the key 0 (-1: not in the table).  Where a table is made for a witness that this object has padded,
+    // the entry's elements - a third of rows of 11008 - take no addition: the table's rows hold (B[t] - B[base]) G_i, and every
+    // committed row starts at sum_i B[base] G_i.  The start is an addition on the chain at a commitment's end, 8 us, which one entry
+    // in 2^bits does not earn: tables made for other witnesses hold B[t] G_i (ranges of 2^12 to 2^16 elements, 0.40 to 0.45 ms, take 1 to
+    // 2 % more with a start), but for a range's of 2^20 elements and more, which may be padded in a later proof and are not measurably
+    // slower.
     int base_ = -1;
     bool padded_ = false;               // the witness of the proof in flight
     std::unique_ptr<FrTensor> B_less_base_;
     void* base_point_ = nullptr;
     uint base_cols_ = 0;                // the row length it was made for (0: not made for the tables at hand)
-    FrTensor& scaled_by();              // what the tables' rows are multiples by
-    const void* base_point(Hyrax& hyrax, uint msm_size);
-    affine_t* scaled_table_ = nullptr;  // (B[t] - B[base])*G_i, built on first use
+    bool hot_based_ = false, scaled_based_ = false;      // whether the table's rows are less B[base]
+    bool padding_is_free() const { return base_ >= 0 && padded_; }
+    FrTensor& scaled_by(bool based);    // what a table's rows are multiples by
+    const void* base_point(Hyrax& hyrax, uint msm_size, bool based);
+    uint64_t mark_base(int* slots);
+    affine_t* scaled_table_ = nullptr;  // B[t]*G_i or (B[t] - B[base])*G_i, built on first use
     uint scaled_cols_ = 0;
     Hyrax* scaled_for_ = nullptr;
 };

@@ -150,6 +150,30 @@ static void the_longest_indexed_range() {
     expect(!committed(0) && !committed((1u << 23) + 1), "none and more are refused");
 }
 
+// Rows start at the entry that witnesses are padded with where their table was made for a padded witness, or for a long one.
+static void where_padding_is_free() {
+    const uint cols = 64, gens = 1u << 12;
+    bn128 G = bn128::one();
+    Hyrax hyrax(1, gens, device_points(256 * (size_t)gens), G, 1);
+    double seconds = 0;
+    auto started = [&](tLookupRange& lookup, uint D) {
+        const uint Dp = 1u << Log2(D);
+        FrTensor S(Dp), A(Dp);
+        S.set_size(D);
+        const std::unique_ptr<FrTensor> ints(new FrTensor(D / 8));
+        const unsigned long before = fake_launched("quad_affine_kernelILb1E");
+        try {
+            lookup.prove(reinterpret_cast<const int*>(ints->gpu_data), S, A, random_vec(Log2(D)), hyrax, cols, seconds);
+        } catch (const std::exception&) {                    // nothing is computed here, so its claims do not hold
+        }
+        return fake_launched("quad_affine_kernelILb1E") - before;
+    };
+    tLookupRange even(-128, 256), padded(-128, 256), large(-128, 256);
+    expect(started(even, 1u << 14) == 0 && started(even, 16 * 11008) == 0, "not for a short witness that is not padded");
+    expect(started(padded, 16 * 11008) == 1 && started(padded, 1u << 14) == 1, "for one that is");
+    expect(started(large, 1u << 20) == 1 && started(large, 16 * 11008) == 1, "for a long one");
+}
+
 // A mapping's witness is S_in + r S_out with the r its caller sees: read as T[index] while T was made with it, written out otherwise (the
 // rounds then find that it is not T's).
 static void a_mapping_with_another_r() {
@@ -665,6 +689,7 @@ int main(int argc, char** argv) {
         {"mapping_objects", mapping_objects},
         {"carried_lookups", carried_lookups},
         {"the_longest_indexed_range", the_longest_indexed_range},
+        {"where_padding_is_free", where_padding_is_free},
         {"a_mapping_with_another_r", a_mapping_with_another_r},
         {"lookups_without_a_weighted_term", lookups_without_a_weighted_term},
         {"weights_that_are_read", weights_that_are_read},

@@ -55,3 +55,38 @@ def test_base_entry(ops, tables, rows, cols, uneven, length=9, base=3):
     values = B[np.where(idx == 0, base, idx - 1).ravel()]
     assert int(flag) == 0
     assert_same(ops.g1_to_host(out), orc.commit_fr(values, ref, cols, 256), "commitments")
+
+
+# the host objects are found by their table's address: it stays taken until the process ends
+_TABLES = []
+
+
+@pytest.mark.parametrize("first", ["padded", "even"])
+def test_ranges_whose_rows_are_the_lowest_key(ops, first):
+    """one lookup object for witnesses that it pads and others, in both orders: its table is made for the first of them.  beta is the
+    table's size, so B[low] = 2 B[0]: a row of nothing but the lowest key adds its start to a sum that is equal to it"""
+    import torch
+    from grape_amd import _host as host
+    host.load()
+    N, low, msm = 16, -8, 64
+    table = ops.g1_table_gen(ops.g1_make_generators(rand_fr(msm, 830 if first == "padded" else 831)), 256)
+    _TABLES.append(table)
+    rng = np.random.default_rng(832)
+    host.set_input_format("i32")
+    try:
+        for turn, kind in enumerate([first, "even" if first == "padded" else "padded", first]):
+            D, lg = (2 * 11008, 15) if kind == "padded" else (1 << 14, 14)
+            x = rng.integers(low, -low, D).astype(np.int32)
+            x[:4 * msm] = low
+            x[5 * msm:6 * msm] = 0
+            x[7 * msm:8 * msm] = -low - 1
+            args = (torch.from_numpy(x).cuda(), D, low, N, rand_fr(1, 833 + turn), rand_fr(lg, 840 + turn), rand_fr(lg, 850 + turn), table, msm, 1, msm)
+            got = host.tlookup_range_prove(*args, want_commitments=True)
+            host.set_indexed_commit(False)
+            want = host.tlookup_range_prove(*args, want_commitments=True)
+            host.set_indexed_commit(True)
+            for k in ("transcript", "S_claim", "com_A", "com_m"):
+                assert_same(got[k], want[k], "%s, %s" % (kind, k))
+    finally:
+        host.set_indexed_commit(True)
+        host.set_input_format("fr")
