@@ -75,6 +75,8 @@ public:
     // not there yet, so that table_bytes_free() afterwards is what a scaled table may really take; false when
     // it does not fit the budget (build_scaled_table would return nullptr).
     bool prepare_scaled_tables(uint ncols);
+    // whether commitments of full-width rows of that length find their table in place
+    bool has_strided_table(uint rowlen) const { return fr_strided_.d && fr_strided_.ngen >= rowlen; }
     // Puts the rows of `more` behind the `rows` rows of a scaled table over ncols generators that has room for `capacity`: in
     // place while they fit, else a copy with room for up to twice as many takes its place first (the old one is freed).
     // False, and the table as it was, where that does not fit the budget, the share of it that tables may grow into

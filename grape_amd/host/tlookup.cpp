@@ -195,23 +195,57 @@ constexpr double kColdAdditions = 19.0, kRowAdditions = 23.0;
 // A growing step costs some 0.3 ms of its own - synchronisations, allocations, at times a copy of the rows.  The entries that
 // are due hold this many elements of a witness when their rows save that in each proof (2.4 to 4.1 ns an element).
 constexpr uint64_t kDueElements = 1u << 17;
+// Elements without a row are committed apart from the others, at some 21 additions each where all elements alike take 16
+// (2^23 elements, nine tenths of them without a row: 24.5 against 20.9 ms).  So where full rows find their table in place, rows of entries are
+// used, and made, if they leave out no more than the share that makes up for it: (16 - 1) / (21 - 1), less what their own launches take.
+constexpr double kApartAdditions = 21.0, kPlainAdditions = 16.0, kColdShare = 0.7;
+// what a growing step may cost: of the commitment without any rows, and of what the rows at hand save it
+constexpr double kStepShare = 0.2, kSavedShare = 0.25;
 uint hot_threshold(uint rowlen) { return (uint)(1.8 * rowlen) + 1; }
+// elements that cost as much without a row as the row does
+uint hot_due(uint rowlen) { return (uint)(kRowAdditions / kColdAdditions * rowlen) + 1; }
 }  // namespace
 
+bool tLookup::rows_are_used(const Hyrax& hyrax, uint rowlen, uint D, uint64_t cold) const {
+    return hot_min_count_ != 0 || (double)cold <= kColdShare * D || !hyrax.has_strided_table(rowlen);
+}
+// Slots from `first` on for at most max_new entries that are due, those that have cost most first (by octaves): `list` holds them in the
+// order of their slots, `left` what the witness has then without one.
+uint tLookup::hot_choice(uint first, size_t max_new, int* slots, uint32_t* list, uint64_t& left) {
+    uint n = 0;
+    for (uint octave = 4; octave-- > 0 && n < max_new;) {
+        uint64_t given[2] = {0, 0};
+        check(grape_tlookup_hot_extend(d_hist_, hot_credit_, T.size, hot_due(hot_cols_) << octave, first + n, (uint32_t)(max_new - n), slots, list + n, given,
+                                       nullptr),
+              "grape_tlookup_hot_extend");
+        n += (uint)given[0];
+        left = given[1];
+    }
+    return n;
+}
+
 // Rows for entries that keep coming back.  Whether a witness repeats is not known in advance, so an entry without a row pays for
-// its elements proof by proof until what it has paid is what its row costs - its occurrences since the object's first proof reach the
-// count that earns a row within one proof - and gets the row then: at most twice what the better choice would have cost, however
-// long the object lives.  A proof builds no more rows than cost what its cold elements cost, so none takes longer than twice its time.
-// SiLU of 2048 x 11008 activations, sigma 4096 (20 000 entries of 200 to 2200 occurrences, 7 of which earn a row in one proof): 56.5 ms a
-// proof; with growing rows the object's proofs take 56 (4th), 94, 62, 43, 37, 29, 31, 28, 26 ... 12 ms (40th).  The exponential of
-// 2^27 scores, sigma 181: 29.5 to 27.5 ms.
-// info: what grape_tlookup_hot_credit has said of this witness.  Returns the elements that the rows leave out.
-uint64_t tLookup::grow_hot_rows(Hyrax& hyrax, const uint64_t info[3]) {
-    const uint N = T.size, due_at = hot_threshold(hot_cols_);
-    const uint64_t cold = info[0];
+// its elements proof by proof until what it has paid is what its row costs, and gets the row then, those that have paid most first.
+// A proof's step costs a fifth of a commitment without rows, and a quarter of what the rows at hand save it (what the new ones save at once
+// taken off): no proof takes more than some 1.3 times what it takes without any, for rows that later ones may never
+// use, and what is due together is made in several steps.
+// info: what grape_tlookup_hot_credit has said of this witness of D elements.  Returns the elements that the rows leave out.
+uint64_t tLookup::grow_hot_rows(Hyrax& hyrax, uint D, const uint64_t info[3]) {
+    const uint N = T.size;
+    uint64_t cold = info[0];
+    auto used = [&](uint64_t without) { return rows_are_used(hyrax, hot_cols_, D, without); };
     const size_t most = hyrax.most_scaled_rows(hot_table_, hot_cols_);
-    const size_t room = most > hot_rows_ ? most - hot_rows_ : 0;
-    const size_t max_new = std::min({room, (size_t)N, (size_t)(cold * kColdAdditions / (kRowAdditions * hot_cols_))});
+    const size_t room = std::min(most > hot_rows_ ? most - hot_rows_ : 0, (size_t)N);
+    const bool padding = hot_table_ ? hot_based_ : padding_is_free();
+    uint32_t of_base = 0;
+    if (padding) check(grape_memcpy_d2h(&of_base, d_hist_ + base_, sizeof of_base, nullptr), "grape_memcpy_d2h");
+    double without = kApartAdditions * (double)(D - of_base), with = used(cold) ? kApartAdditions * (double)cold : without;
+    if (hyrax.has_strided_table(hot_cols_)) without = std::min(without, kPlainAdditions * D);
+    with = std::min(with, without);
+    const double row = kRowAdditions * hot_cols_, share = std::min(kStepShare * without + kSavedShare * (without - with), with);
+    // (entries that earn their row by this witness alone are no risk)
+    const double spend = std::max(share, kColdAdditions * kDueElements) + kColdAdditions * (double)info[2];
+    const size_t max_new = std::min(room, (size_t)(spend / row));
     if (room == 0) hot_missed_ += (double)info[1];
     if (max_new == 0) return cold;
     // the new slots are given on a copy: they count once their rows are there
@@ -221,14 +255,32 @@ uint64_t tLookup::grow_hot_rows(Hyrax& hyrax, const uint64_t info[3]) {
     try {
         check(grape_malloc_on_default((void**)&d_list, sizeof(uint32_t) * (size_t)N), "grape_malloc");
         check(grape_malloc((void**)&slots, sizeof(int) * (size_t)N), "grape_malloc");
-        check(grape_memcpy_d2d(slots, hot_slot1_, sizeof(int) * (size_t)N, nullptr), "grape_memcpy_d2d");
-        uint64_t given[2] = {0, 0};
-        check(grape_tlookup_hot_extend(d_hist_, hot_credit_, N, due_at, hot_rows_, (uint32_t)max_new, slots, d_list, given, nullptr),
-              "grape_tlookup_hot_extend");
-        const uint n_new = (uint)given[0];
+        auto copy_slots = [&] { check(grape_memcpy_d2d(slots, hot_slot1_, sizeof(int) * (size_t)N, nullptr), "grape_memcpy_d2d"); };
+        copy_slots();
+        const bool marked = !hot_table_ && padding;
+        if (marked) left = cold -= mark_base(slots);
+        bool enough = true;
+        if (!used(cold)) {
+            // not made for nothing: there is room for as many as it takes to use them
+            uint64_t all[2] = {0, cold};
+            check(grape_tlookup_hot_extend(d_hist_, hot_credit_, N, hot_due(hot_cols_), hot_rows_, (uint32_t)room, slots, d_list, all, nullptr),
+                  "grape_tlookup_hot_extend");
+            enough = used(all[1]);
+            if (enough) {
+                copy_slots();
+                if (marked) mark_base(slots);
+            }
+        }
+        uint n_new = enough ? hot_choice(hot_rows_, max_new, slots, d_list, left) : 0;
+        // what these rows take in comes off the proof at hand: as many more (as many again at most) as the step may cost then
+        if (n_new != 0 && n_new == max_new && used(left)) {
+            const double saved = std::min(kColdAdditions * (double)(cold - left) / n_new, row / 2);
+            const size_t all = std::min(room, (size_t)(spend / (row - saved)));
+            if (all > n_new) n_new += hot_choice(hot_rows_ + n_new, all - n_new, slots, d_list + n_new, left);
+        }
         if (n_new != 0) {
             FrTensor more(n_new, OnDefaultStream());
-            if (!hot_table_) hot_based_ = padding_is_free();
+            if (!hot_table_) hot_based_ = marked;
             check(grape_fr_gather(W(more.gpu_data), W(scaled_by(hot_based_).gpu_data), d_list, n_new, nullptr), "grape_fr_gather");
             bool built;
             if (hot_table_) {
@@ -236,16 +288,15 @@ uint64_t tLookup::grow_hot_rows(Hyrax& hyrax, const uint64_t info[3]) {
             } else {
                 hot_table_ = hyrax.build_scaled_table(more, hot_cols_);
                 base_cols_ = 0;
-                if (hot_table_ && hot_based_) given[1] -= mark_base(slots);
                 built = hot_table_ != nullptr;
                 hot_capacity_ = built ? n_new : 0;
             }
             if (built) {
                 hot_rows_ += n_new;
                 std::swap(slots, hot_slot1_);
-                left = given[1];
             } else {
-                hot_missed_ += (double)(cold - given[1]);
+                hot_missed_ += (double)(cold - left);
+                left = cold;
             }
         }
     } catch (...) {
@@ -275,15 +326,15 @@ bool tLookup::commit_A_by_occupancy(uint D, uint msm_size, Hyrax& hyrax) {
             check(grape_memset_zero(hot_credit_, sizeof(uint32_t) * (size_t)N, nullptr), "grape_memset_zero");
         }
         uint64_t info[3] = {0, 0, 0};
-        check(grape_tlookup_hot_credit(d_hist_, N, hot_slot1_, hot_credit_, min_count, info, nullptr), "grape_tlookup_hot_credit");
+        check(grape_tlookup_hot_credit(d_hist_, N, hot_slot1_, hot_credit_, hot_due(rowlen), info, nullptr), "grape_tlookup_hot_credit");
         cold = info[0];
         // rows kept from earlier proofs: used again, with more of them where entries are due, unless the elements that new rows would
         // take in (20 additions each instead of one) cost more than building all rows anew (rowlen entries of 20 additions and
         // a normalisation per row).  Where there is no room for more rows, what the entries that were due have missed counts as well.
         const double anew = (double)hot_rows_ * rowlen * kRowAdditions;
-        if (info[1] >= kDueElements && hot_missed_ * kColdAdditions <= anew) {
+        if (info[1] >= kDueElements && rows_are_used(hyrax, rowlen, D, cold - info[1]) && hot_missed_ * kColdAdditions <= anew) {
             hot_reused_ = hot_table_ != nullptr;
-            cold = grow_hot_rows(hyrax, info);
+            cold = grow_hot_rows(hyrax, D, info);
         } else if (hot_table_) {
             hot_reused_ = std::max((double)info[2], hot_missed_) * kColdAdditions <= anew;
             if (!hot_reused_) drop_hot_rows();
@@ -304,13 +355,16 @@ bool tLookup::commit_A_by_occupancy(uint D, uint msm_size, Hyrax& hyrax) {
             check(grape_tlookup_hot_select(d_hist_, N, min_count, (uint32_t)max_hot, hot_slot1_, d_list, info, nullptr), "grape_tlookup_hot_select");
             const uint n_hot = (uint)info[0];
             cold = info[1];
-            if (n_hot != 0) {
+            const bool marked = n_hot != 0 && padding_is_free();
+            if (marked) cold -= mark_base(hot_slot1_);
+            const bool worth = rows_are_used(hyrax, rowlen, D, cold);
+            if (n_hot != 0 && !worth) check(grape_memset_zero(hot_slot1_, sizeof(int) * (size_t)N, nullptr), "grape_memset_zero");
+            if (n_hot != 0 && worth) {
                 FrTensor Bhot(n_hot, OnDefaultStream());
-                hot_based_ = padding_is_free();
+                hot_based_ = marked;
                 check(grape_fr_gather(W(Bhot.gpu_data), W(scaled_by(hot_based_).gpu_data), d_list, n_hot, nullptr), "grape_fr_gather");
                 hot_table_ = hyrax.build_scaled_table(Bhot, rowlen);
                 base_cols_ = 0;
-                if (hot_table_ && hot_based_) cold -= mark_base(hot_slot1_);
                 if (!hot_table_) check(grape_memset_zero(hot_slot1_, sizeof(int) * (size_t)N, nullptr), "grape_memset_zero");
             }
             hot_rows_ = hot_capacity_ = hot_table_ ? n_hot : 0;
@@ -328,6 +382,10 @@ bool tLookup::commit_A_by_occupancy(uint D, uint msm_size, Hyrax& hyrax) {
             if (hot_min_count_ != 0) drop_hot_rows();
             return false;
         }
+    }
+    if (!rows_are_used(hyrax, rowlen, D, cold)) {
+        hot_reused_ = false;
+        return false;
     }
     int* d_hot = nullptr;
     affine_t* com_cold = nullptr;
