@@ -186,14 +186,15 @@ void tLookup::drop_hot_rows() {
     hot_credit_ = nullptr;
     hot_rows_ = hot_cols_ = hot_capacity_ = 0;
     hot_missed_ = 0;
+    hot_due_ = 0;
     hot_for_ = nullptr;
 }
 
 namespace {
 // a full-width scalar's additions beyond the one through a row, and the additions a row's entry takes to build
 constexpr double kColdAdditions = 19.0, kRowAdditions = 23.0;
-// A growing step costs some 0.3 ms of its own - synchronisations, allocations, at times a copy of the rows.  The entries that
-// are due hold this many elements of a witness when their rows save that in each proof (2.4 to 4.1 ns an element).
+// A growing step costs some 0.3 ms of its own - synchronisations, allocations, at times a copy of the rows.  Entries that are due have paid
+// as much since the last one when this many of their elements have been committed without a row (2.4 to 4.1 ns each).
 constexpr uint64_t kDueElements = 1u << 17;
 // Elements without a row are committed apart from the others, at some 21 additions each where all elements alike take 16
 // (2^23 elements, nine tenths of them without a row: 24.5 against 20.9 ms).  So where full rows find their table in place, rows of entries are
@@ -229,10 +230,10 @@ uint tLookup::hot_choice(uint first, size_t max_new, int* slots, uint32_t* list,
 // A proof's step costs a fifth of a commitment without rows, and a quarter of what the rows at hand save it (what the new ones save at once
 // taken off): no proof takes more than some 1.3 times what it takes without any, for rows that later ones may never
 // use, and what is due together is made in several steps.
-// info: what grape_tlookup_hot_credit has said of this witness of D elements.  Returns the elements that the rows leave out.
-uint64_t tLookup::grow_hot_rows(Hyrax& hyrax, uint D, const uint64_t info[3]) {
+// cold: those of the witness's D elements without a row, earned: those of them whose entry it alone earns one.  Returns the elements that
+// the rows leave out even so.
+uint64_t tLookup::grow_hot_rows(Hyrax& hyrax, uint D, uint64_t cold, uint64_t earned) {
     const uint N = T.size;
-    uint64_t cold = info[0];
     auto used = [&](uint64_t without) { return rows_are_used(hyrax, hot_cols_, D, without); };
     const size_t most = hyrax.most_scaled_rows(hot_table_, hot_cols_);
     const size_t room = std::min(most > hot_rows_ ? most - hot_rows_ : 0, (size_t)N);
@@ -244,9 +245,9 @@ uint64_t tLookup::grow_hot_rows(Hyrax& hyrax, uint D, const uint64_t info[3]) {
     with = std::min(with, without);
     const double row = kRowAdditions * hot_cols_, share = std::min(kStepShare * without + kSavedShare * (without - with), with);
     // (entries that earn their row by this witness alone are no risk)
-    const double spend = std::max(share, kColdAdditions * kDueElements) + kColdAdditions * (double)info[2];
+    const double spend = std::max(share, kColdAdditions * kDueElements) + kColdAdditions * (double)earned;
     const size_t max_new = std::min(room, (size_t)(spend / row));
-    if (room == 0) hot_missed_ += (double)info[1];
+    if (room == 0) hot_missed_ += (double)hot_due_;
     if (max_new == 0) return cold;
     // the new slots are given on a copy: they count once their rows are there
     uint32_t* d_list = nullptr;
@@ -321,7 +322,7 @@ bool tLookup::commit_A_by_occupancy(uint D, uint msm_size, Hyrax& hyrax) {
     if (hot_slot1_ && (hot_min_count_ != 0 || hot_for_ != &hyrax || hot_cols_ != rowlen || (hot_table_ && !hyrax.owns_scaled_table(hot_table_))))
         drop_hot_rows();
     if (hot_slot1_) {
-        if (!hot_credit_) {
+        if (!hot_credit_) {                      // rows of a count that the caller has set and taken back
             check(grape_malloc((void**)&hot_credit_, sizeof(uint32_t) * (size_t)N), "grape_malloc");
             check(grape_memset_zero(hot_credit_, sizeof(uint32_t) * (size_t)N, nullptr), "grape_memset_zero");
         }
@@ -332,9 +333,11 @@ bool tLookup::commit_A_by_occupancy(uint D, uint msm_size, Hyrax& hyrax) {
         // take in (20 additions each instead of one) cost more than building all rows anew (rowlen entries of 20 additions and
         // a normalisation per row).  Where there is no room for more rows, what the entries that were due have missed counts as well.
         const double anew = (double)hot_rows_ * rowlen * kRowAdditions;
-        if (info[1] >= kDueElements && rows_are_used(hyrax, rowlen, D, cold - info[1]) && hot_missed_ * kColdAdditions <= anew) {
+        hot_due_ += info[1];
+        if (hot_due_ >= kDueElements && rows_are_used(hyrax, rowlen, D, cold - info[1]) && hot_missed_ * kColdAdditions <= anew) {
             hot_reused_ = hot_table_ != nullptr;
-            cold = grow_hot_rows(hyrax, D, info);
+            cold = grow_hot_rows(hyrax, D, cold, info[2]);
+            hot_due_ = 0;
         } else if (hot_table_) {
             hot_reused_ = std::max((double)info[2], hot_missed_) * kColdAdditions <= anew;
             if (!hot_reused_) drop_hot_rows();
@@ -355,6 +358,11 @@ bool tLookup::commit_A_by_occupancy(uint D, uint msm_size, Hyrax& hyrax) {
             check(grape_tlookup_hot_select(d_hist_, N, min_count, (uint32_t)max_hot, hot_slot1_, d_list, info, nullptr), "grape_tlookup_hot_select");
             const uint n_hot = (uint)info[0];
             cold = info[1];
+            // what this proof's entries cost counts where no proof before it has been counted
+            if (!hot_credit_ && hot_min_count_ == 0) {
+                check(grape_malloc((void**)&hot_credit_, sizeof(uint32_t) * (size_t)N), "grape_malloc");
+                check(grape_memcpy_d2d(hot_credit_, d_hist_, sizeof(uint32_t) * (size_t)N, nullptr), "grape_memcpy_d2d");
+            }
             const bool marked = n_hot != 0 && padding_is_free();
             if (marked) cold -= mark_base(hot_slot1_);
             const bool worth = rows_are_used(hyrax, rowlen, D, cold);

@@ -102,10 +102,11 @@ protected:
     Hyrax* hot_for_ = nullptr;
     void drop_hot_rows();
     uint32_t* hot_credit_ = nullptr;    // occurrences of entries without a row in the proofs since the rows were made
+    uint64_t hot_due_ = 0;              // elements of entries that are due, in the proofs since rows were made last
     double hot_missed_ = 0;             // elements of entries that had earned a row when there was no more room for it
     bool rows_are_used(const Hyrax& hyrax, uint rowlen, uint D, uint64_t cold) const;
     uint hot_choice(uint first, size_t max_new, int* slots, uint32_t* list, uint64_t& left);
-    uint64_t grow_hot_rows(Hyrax& hyrax, uint D, const uint64_t info[3]);
+    uint64_t grow_hot_rows(Hyrax& hyrax, uint D, uint64_t cold, uint64_t earned);
     // The entry a witness is padded with, the key 0 (-1: not in the table).  Where a table is made for a witness that this object has padded,
     // the entry's elements - a third of rows of 11008 - take no addition: the table's rows hold (B[t] - B[base]) G_i, and every
     // committed row starts at sum_i B[base] G_i.  The start is an addition on the chain at a commitment's end, 8 us, which one entry

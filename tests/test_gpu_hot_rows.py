@@ -97,14 +97,17 @@ def _steps(N, D, msm, proofs, room):
     """(rows, elements without one) that proofs of a witness spread evenly over N entries are committed with, (0, 0) where all of
     it goes the plain way: an entry is due once its elements have cost its row (23 additions a generator against 19 an element); a step
     costs a fifth of the commitment without rows (16 additions an element) and a quarter of what it saves by them (21 for each without
-    a row where they are used), or what 2^17 elements without a row do, and twice that where half of a row's price comes back at once; rows are used from 30 % of the elements on"""
+    a row where they are used), or what 2^17 elements without a row do, and twice that where half of a row's price comes back at once; rows are used from 30 % of the elements on; a
+    step is made once due entries have had 2^17 elements since the last one"""
     each, row, due_at = D // N, 23.0 * msm, int(23.0 / 19.0 * msm) + 1
-    held, credit, out = 0, 0, []
+    held, credit, due, out = 0, 0, 0, []
     for i in range(proofs):
         cold = (N - held) * each
-        if i > 0:
-            credit += each
-            if credit >= due_at and cold >= 1 << 17 and held < room:
+        credit += each
+        if i > 0 and credit >= due_at:
+            due += cold
+            if due >= 1 << 17 and held < room:
+                due = 0
                 without = 16.0 * D
                 now = min(21.0 * cold, without) if cold <= 0.7 * D else without
                 spend = max(min(0.2 * without + 0.25 * (without - now), now), 19.0 * (1 << 17))
@@ -120,18 +123,18 @@ def _steps(N, D, msm, proofs, room):
 
 def test_rows_grow_with_what_entries_have_cost(ops, host):
     """a witness spread evenly over 2^14 entries, 64 occurrences of each: no entry is worth a row of 64 in one proof, the object's
-    third proof makes as many rows as a fifth of it pays for, the next ones more, in a table that has to be moved; they are used once
-    they take in 30 %, and what is left in the end is too little for another step"""
+    second proof makes as many rows as a fifth of it pays for, the next ones more, in a table that has to be moved; they are used once
+    they take in 30 %, and what is left is too little for a step of its own until several proofs have paid for it"""
     prove, low, N, D, msm = _prover(ops, host, 136, 14, 20, 900)
     rng = np.random.default_rng(901)
-    even = [low + rng.permutation(np.arange(D, dtype=np.int64) % N) for _ in range(8)]
+    even = [low + rng.permutation(np.arange(D, dtype=np.int64) % N) for _ in range(13)]
     even = [x.astype(np.int32) for x in even]
     want = _steps(N, D, msm, len(even), N)
-    assert [n for n, _ in want[:4]] == [0, 0, 0, 0] and 0 < want[4][0] < want[5][0] < N and want[7] == want[6] == want[5]
+    assert [n for n, _ in want[:3]] == [0, 0, 0] and 0 < want[3][0] < want[4][0] < N and want[10] == want[4] and want[11:] == [(N, 0)] * 2
     plain = [prove(x, indexed=False) for x in even]
     hot = []
     for i, x in enumerate(even):
-        got = prove(x, fmt="i32" if i != 4 else "fr")
+        got = prove(x, fmt="i32" if i != 3 else "fr")
         _same(got, plain[i])
         hot.append(got[3:])
     assert [h[:2] for h in hot] == want
