@@ -373,16 +373,17 @@ __global__ void __launch_bounds__(kBlock) inverse_by_table_kernel(uint32_t* A, c
 // of 1024, an exclusive scan of the tile counts, slots within every tile.
 constexpr int kHotTile = 1024;          // entries per workgroup: 4 per thread
 // EXTEND: more entries for an assignment that exists.  `weight` is what an entry is chosen by (the counts themselves, or what has
-// been counted over several proofs); entries that hold a slot keep it, the new ones follow from first_slot on.
+// been counted over several proofs; then of those that the witness has); entries that hold a slot keep it, the new ones follow from
+// first_slot on.
 // pass 1: hot entries per tile
 template <bool EXTEND>
-__global__ void __launch_bounds__(kBlock) hot_count_kernel(const uint32_t* __restrict__ weight, uint32_t len, uint32_t min_count,
+__global__ void __launch_bounds__(kBlock) hot_count_kernel(const uint32_t* __restrict__ hist, const uint32_t* __restrict__ weight, uint32_t len, uint32_t min_count,
                                                            const int32_t* __restrict__ slot1, uint32_t* __restrict__ tile_count) {
     __shared__ uint32_t wsum[kBlock / 64];
     const uint32_t base = blockIdx.x * kHotTile + threadIdx.x * 4;
     uint32_t mine = 0;
 #pragma unroll
-    for (int k = 0; k < 4; k++) mine += (base + k < len && weight[base + k] >= min_count && !(EXTEND && slot1[base + k] != 0)) ? 1u : 0u;
+    for (int k = 0; k < 4; k++) mine += (base + k < len && weight[base + k] >= min_count && !(EXTEND && (slot1[base + k] != 0 || hist[base + k] == 0))) ? 1u : 0u;
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) mine += __shfl_down(mine, off, 64);
     if ((threadIdx.x & 63) == 0) wsum[threadIdx.x >> 6] = mine;
@@ -431,7 +432,7 @@ __global__ void __launch_bounds__(kBlock) hot_assign_kernel(const uint32_t* __re
     for (int k = 0; k < 4; k++) {
         const bool in = base + k < len;
         held[k] = EXTEND && in && slot1[base + k] != 0;
-        cand[k] = in && !held[k] && weight[base + k] >= min_count;
+        cand[k] = in && !held[k] && weight[base + k] >= min_count && !(EXTEND && hist[base + k] == 0);
         mine += cand[k] ? 1u : 0u;
     }
     // exclusive prefix of `mine` over the workgroup: inclusive scan within the wave, then the waves before
@@ -1203,7 +1204,7 @@ int grape_tlookup_hot_select(const uint32_t* hist, uint32_t len, uint32_t min_co
     if (rc) return rc;
     unsigned long long* d_info = (unsigned long long*)ws;
     uint32_t* tiles = (uint32_t*)((char*)ws + 64);
-    hot_count_kernel<false><<<ntiles, kBlock, 0, s>>>(hist, len, min_count, nullptr, tiles);
+    hot_count_kernel<false><<<ntiles, kBlock, 0, s>>>(hist, hist, len, min_count, nullptr, tiles);
     hot_scan_kernel<<<1, kBlock, 0, s>>>(tiles, ntiles, max_hot, d_info);
     hot_assign_kernel<false><<<ntiles, kBlock, 0, s>>>(hist, hist, len, min_count, 0, max_hot, tiles, slot1, hot_list, d_info);
     GRAPE_LAUNCH_CHECK();
@@ -1223,7 +1224,7 @@ int grape_tlookup_hot_extend(const uint32_t* hist, const uint32_t* credit, uint3
     if (rc) return rc;
     unsigned long long* d_info = (unsigned long long*)ws;
     uint32_t* tiles = (uint32_t*)((char*)ws + 64);
-    hot_count_kernel<true><<<ntiles, kBlock, 0, s>>>(credit, len, min_credit, slot1, tiles);
+    hot_count_kernel<true><<<ntiles, kBlock, 0, s>>>(hist, credit, len, min_credit, slot1, tiles);
     hot_scan_kernel<<<1, kBlock, 0, s>>>(tiles, ntiles, max_new, d_info);
     hot_assign_kernel<true><<<ntiles, kBlock, 0, s>>>(hist, credit, len, min_credit, first_slot, max_new, tiles, slot1, hot_list, d_info);
     GRAPE_LAUNCH_CHECK();

@@ -101,6 +101,8 @@ protected:
     uint hot_rows_ = 0, hot_cols_ = 0, hot_capacity_ = 0;
     Hyrax* hot_for_ = nullptr;
     void drop_hot_rows();
+    void drop_hot_table();
+    bool other_rows_are_better(uint D, uint64_t cold);
     uint32_t* hot_credit_ = nullptr;    // occurrences of entries without a row in the proofs since the rows were made
     uint64_t hot_due_ = 0;              // elements of entries that are due, in the proofs since rows were made last
     double hot_missed_ = 0;             // elements of entries that had earned a row when there was no more room for it

@@ -438,7 +438,7 @@ int grape_tlookup_hot_coverage(const uint32_t *d_hist, uint32_t len, const int32
  * this witness alone.  No counterpart in the reference. */
 int grape_tlookup_hot_credit(const uint32_t *d_hist, uint32_t len, const int32_t *d_slot1, uint32_t *d_credit, uint32_t min_credit,
                              uint64_t *info, grape_stream_t stream);
-/* More entries for a slot assignment: those without a slot and with d_credit[t] >= min_credit get the slots from first_slot on,
+/* More entries for a slot assignment: those without a slot, with d_credit[t] >= min_credit and d_hist[t] > 0 get the slots from first_slot on,
  * in table order, at most max_new of them (d_hot_list[0 ..] = their entries); slots that are given stay.  info (HOST, two words; the
  * call synchronises): info[0] = number of slots given now, info[1] = elements of the witness counted in d_hist whose entry
  * has none even so.  No counterpart in the reference. */
