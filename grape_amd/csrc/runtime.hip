@@ -101,11 +101,11 @@ int scratch_get(ScratchSlot slot, size_t bytes, void** out, hipStream_t stream) 
             set_error("scratch allocation of %zu bytes failed: %s", want, hipGetErrorString(e));
             return GRAPE_ENOMEM;
         }
-        pool.bytes[slot] = want;
-        if (slot == kSlotTicket) {
+        if (slot == kSlotTicket) {                       // not there until it has been cleared
             const int rc = zero_fill(pool.ptr[slot], want, stream);
             if (rc) return rc;
         }
+        pool.bytes[slot] = want;
     }
     *out = pool.ptr[slot];
     return GRAPE_OK;

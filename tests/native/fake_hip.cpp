@@ -31,6 +31,8 @@ std::map<const void*, Kernel>& kernels() {
     return k;
 }
 unsigned long launches = 0, copies = 0, waits = 0;
+unsigned long failing = 0;                               // launches that fail from now on
+thread_local hipError_t last_error = hipSuccess;
 unsigned long limit = ~0ul;                              // bytes of the device's memory
 thread_local int device = 0;
 char symbol[1 << 24];
@@ -75,6 +77,8 @@ unsigned long fake_bytes() {
 }
 // no more than `bytes` can be allocated together from now on
 void fake_limit(unsigned long bytes) { limit = bytes; }
+// the next n launches fail
+void fake_fail_launches(unsigned long n) { failing = n; }
 unsigned long fake_launches() { return launches; }
 // launches of the kernels whose name holds `part`
 unsigned long fake_launched(const char* part) {
@@ -101,7 +105,11 @@ hipError_t hipGetDevicePropertiesR0600(hipDeviceProp_tR0600* p, int) {
     return hipSuccess;
 }
 const char* hipGetErrorString(hipError_t) { return "fake"; }
-hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipGetLastError() {
+    const hipError_t e = last_error;
+    last_error = hipSuccess;
+    return e;
+}
 hipError_t hipMalloc(void** p, size_t bytes) {
     Lock l(mu);
     bytes = (bytes + 4095) & ~(size_t)4095;
@@ -179,6 +187,10 @@ hipError_t __hipPopCallConfiguration(dim3* g, dim3* b, size_t* sh, hipStream_t* 
 }
 hipError_t hipLaunchKernel(const void* stub, dim3, dim3, void**, size_t, hipStream_t s) {
     Lock l(mu);
+    if (failing) {
+        failing--;
+        return last_error = hipErrorLaunchFailure;
+    }
     push(s);
     launches++;
     kernels()[stub].launched++;

@@ -22,6 +22,7 @@ void fake_queue(const void* stream);
 unsigned long fake_waits();
 unsigned long fake_bytes();
 void fake_limit(unsigned long bytes);
+void fake_fail_launches(unsigned long n);
 void fake_set_device(int device);
 }
 
@@ -508,6 +509,18 @@ static void single_rows_without_memory() {
     expect(at_hand == 2 && fake_launched("wide_chain_kernel") == at_hand, "the one at hand stays");
 }
 
+// The counter that a sum's workgroups take turns at is cleared before the first sum that uses it, also when the first attempt at that fails.
+static void a_sum_behind_a_failed_one() {
+    FrTensor x(4096);
+    uint32_t *in = reinterpret_cast<uint32_t*>(x.gpu_data), *out = in + 8 * 2048;
+    fake_fail_launches(1);
+    expect(grape_fr_sum(out, in, 2000, nullptr) != GRAPE_OK, "the launch that clears it fails");
+    const unsigned long cleared = fake_launched("zero_words_kernel"), sums = fake_launched("sum_kernelILb1E");
+    expect(grape_fr_sum(out, in, 2000, nullptr) == GRAPE_OK && fake_launched("zero_words_kernel") == cleared + 1, "the next sum clears it");
+    expect(grape_fr_sum(out, in, 2000, nullptr) == GRAPE_OK && fake_launched("zero_words_kernel") == cleared + 1, "the one behind it does not");
+    expect(fake_launched("sum_kernelILb1E") == sums + 2, "both are sums in one launch");
+}
+
 // Which table a single row goes through: the reference-format one until such rows have cost a table, a strided one where there is one (its
 // doublings count too), the row's own from then on.
 static void tables_of_single_rows() {
@@ -701,6 +714,7 @@ int main(int argc, char** argv) {
         {"a_tensor_times_itself", a_tensor_times_itself},
         {"verify_with_more_variables", verify_with_more_variables},
         {"single_rows_without_memory", single_rows_without_memory},
+        {"a_sum_behind_a_failed_one", a_sum_behind_a_failed_one},
         {"tables_of_single_rows", tables_of_single_rows},
         {"single_row_table_gives_way", single_row_table_gives_way},
         {"verify_with_another_generator", verify_with_another_generator},
