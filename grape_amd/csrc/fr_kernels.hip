@@ -517,15 +517,28 @@ __global__ void __launch_bounds__(kBlock) fold_short_kernel(FoldPassArgs args) {
     }
 }
 
+static uint32_t log2ceil(size_t n) {
+    uint32_t r = 0;
+    while (((size_t)1 << r) < n) r++;
+    return r;
+}
+
 // Small-tensor finish: one workgroup holds the whole [c][gap] slab of one outer index in LDS
 // and binds the remaining bits top-down with a barrier per level.
 constexpr int kFoldSmallElems = 2048;   // 64 KiB of LDS
 constexpr int kFoldSmallMaxOuter = 256; // one workgroup per outer index: worth it only for few
-// Only the whole of a fold that is short anyway, which needs no weights then: an element a thread, or two variables (one call after
-// another, launches included: 256 elements 11.5 us against 13.3 through a pass, 16 slabs of 16 x 4 12.5 against 17; 2048
-// elements 19 against 16.5, 4096 with a pass before it 33 against 17).
-static bool fold_small_fits(size_t outer, size_t c, size_t gap) {
-    return c * gap <= (size_t)(c <= 4 ? kFoldSmallElems : kBlock) && outer <= (size_t)kFoldSmallMaxOuter;
+// Only the whole of a fold that is short anyway, which needs no weights then.  A workgroup's time is 0.9 us a step of 256 outputs; in
+// steps (one call after another, launches included): one slab 16 x 16 4 steps 7.7 us, 32 x 16 5 7.7, 64 x 16 7 9.6, 256 8 10.6, 512 9 12.0,
+// 32 x 64 9 11.6, 1024 11 14.1, 2048 15 18.4, where a pass takes 11.0 and two of them, for more than eight variables, 13.8; 16 slabs
+// of 64 x 16 7 11.8, of 512 9 14.8, of 128 x 16 11 16.1 against 13.7.  Two folds side by side share their passes'
+// launches and keep to slabs of an element a thread, or two variables, as do integers, which would be embedded first.
+static bool fold_small_fits(size_t outer, size_t c, size_t gap, bool alone) {
+    if (c * gap > (size_t)kFoldSmallElems || outer > (size_t)kFoldSmallMaxOuter) return false;
+    if (!alone) return c <= 4 || c * gap <= (size_t)kBlock;
+    const uint32_t L = log2ceil((uint32_t)c);
+    size_t steps = 0;
+    for (uint32_t l = 0; l < L; l++) steps += (gap << l) / kBlock + ((gap << l) % kBlock != 0);
+    return steps <= (outer == 1 && L > (uint32_t)kFoldMaxBits ? 9u : 8u);
 }
 
 __global__ void __launch_bounds__(kBlock) fold_small_kernel(uint32_t* out, const uint32_t* in, const uint32_t* x,
@@ -556,12 +569,6 @@ __global__ void __launch_bounds__(kBlock) fold_small_kernel(uint32_t* out, const
         __syncthreads();
     }
     for (size_t i = threadIdx.x; i < gap; i += kBlock) st_fr(out, o * gap + i, buf[i]);
-}
-
-static uint32_t log2ceil(size_t n) {
-    uint32_t r = 0;
-    while (((size_t)1 << r) < n) r++;
-    return r;
 }
 
 }  // namespace grape
@@ -792,10 +799,10 @@ static uint32_t short_pass_parts(size_t n_out, uint32_t b) {
     }
     return best;
 }
-static int plan_fold(size_t outer, uint32_t c, uint32_t gap, uint32_t id, bool ints, FoldPlan& plan) {
+static int plan_fold(size_t outer, uint32_t c, uint32_t gap, uint32_t id, bool ints, bool alone, FoldPlan& plan) {
     plan.npass = 0;
     uint32_t l = log2ceil(c);
-    if (fold_small_fits(outer, c, gap)) return GRAPE_OK;
+    if (fold_small_fits(outer, c, gap, alone && !ints)) return GRAPE_OK;
     while (l > 0) {
         // Measured on MI355X: a pass streams fastest with one thread per output, 16 to 64
         // terms per thread and 2^20 threads; 2^19 threads come close.  Failing that, up to
@@ -845,7 +852,7 @@ struct FoldRun {
     int which;
     const int32_t* wts;
 };
-static int fold_start(FoldRun& r, const grape_fold_job& j, hipStream_t s) {
+static int fold_start(FoldRun& r, const grape_fold_job& j, bool alone, hipStream_t s) {
     r = FoldRun{};
     r.j = &j;
     r.done = j.N == 0;
@@ -860,7 +867,7 @@ static int fold_start(FoldRun& r, const grape_fold_job& j, hipStream_t s) {
     r.outer = j.N / ((size_t)j.c * j.gap);
     r.cur_c = j.c;
     r.L = log2ceil(j.c);
-    int rc = plan_fold(r.outer, j.c, j.gap, j.id, j.ints != nullptr, r.plan);
+    int rc = plan_fold(r.outer, j.c, j.gap, j.id, j.ints != nullptr, alone, r.plan);
     if (rc) return rc;
     r.ints = j.ints != nullptr;
     if (r.ints && (r.L == 0 || r.plan.npass == 0)) {
@@ -932,7 +939,7 @@ static int fold_jobs(const grape_fold_job* jobs, uint32_t count, grape_stream_t 
     FoldWeights fw = {};
     size_t scratch = 0;
     for (uint32_t k = 0; k < count; k++) {
-        int rc = fold_start(run[k], jobs[k], s);
+        int rc = fold_start(run[k], jobs[k], count == 1, s);
         if (rc) return rc;
         if (run[k].done) continue;
         scratch += 2 * run[k].each;
@@ -1033,7 +1040,7 @@ size_t grape_fr_fold_i32_elems(size_t N, uint32_t c, uint32_t gap) {
     size_t most = 0;
     for (const bool ints : {false, true}) {            // integers are folded in other steps than field elements
         FoldPlan plan;
-        if (plan_fold(outer, c, gap, 0, ints, plan) != GRAPE_OK || plan.npass == 0) return N;
+        if (plan_fold(outer, c, gap, 0, ints, true, plan) != GRAPE_OK || plan.npass == 0) return N;
         const size_t c_lo = (size_t)1 << (log2ceil(c) - plan.pass[0].b);
         // several outer indices: the passes go through work memory of the library; one: the first pass writes into d_out
         const size_t n = outer > 1 ? outer * gap : (c < c_lo ? c : c_lo) * gap;

@@ -40,13 +40,26 @@ SHAPES = {
     "ints_rows": ("ints", 2, 300, 250, 0),
     "nine_variables": ("t", 1, 512, 3, 0),
     "seventeen_variables": ("from", 1, 70001, 1, 0),
+    # one workgroup's steps of 256 outputs: eight and nine, one slab and several, field elements and integers
+    "steps_9_of_512": ("t", 1, 512, 1, 0),
+    "steps_9_of_300": ("from", 1, 300, 1, 1),
+    "steps_10_of_513": ("t", 1, 513, 1, 0),
+    "steps_9_of_several": ("from", 3, 300, 1, 0),
+    "steps_8": ("t", 1, 128, 8, 2),
+    "steps_8_of_several": ("from", 17, 100, 8, 0),
+    "steps_7": ("t", 256, 64, 16, 0),
+    "steps_9_of_2048": ("from", 1, 32, 64, 0),
+    "steps_5_ragged": ("t", 2, 17, 30, 1),
+    "steps_7_of_ints": ("ints", 5, 64, 16, 0),
 }
 
 
 @pytest.mark.parametrize("pair", [("one_thread_an_output", "slab"), ("two_variables", "nothing_to_bind"), ("ragged_16", "ragged_16_rows"),
                                   ("eval", "eval_ragged"), ("rows_256", "eval"), ("ints_16", "ints_256"), ("ints_rows", "ragged_16"),
                                   ("nine_variables", "seventeen_variables"), ("nothing_to_bind", "ints_rows"), ("seventeen_variables",),
-                                  ("ints_256",)], ids="-".join)
+                                  ("ints_256",), ("steps_9_of_512",), ("steps_9_of_300",), ("steps_10_of_513",), ("steps_9_of_several",), ("steps_8",),
+                                  ("steps_8_of_several",), ("steps_7",), ("steps_9_of_2048",), ("steps_5_ragged",), ("steps_7_of_ints",),
+                                  ("steps_9_of_512", "steps_8_of_several")], ids="-".join)
 def test_folds_side_by_side(ops, pair):
     import torch
     from grape_amd import _capi
