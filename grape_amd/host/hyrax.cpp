@@ -623,8 +623,12 @@ Hyrax_proof Hyrax::open_impl(FrTensor* tensor_in, const int* ints, const std::ve
     std::unique_ptr<FrTensor> row;
     if (!ints || pad_N != N) {
         row.reset(new FrTensor(new_N, OnDefaultStream()));
-        *row = tensor;
-        if (pad_N != N) row->pad(tensor, N, pad_N, new_N, Fr::zero());
+        if (pad_N == N) {
+            *row = tensor;
+        } else {
+            // padded from where it lies: neither the folded integers nor a single row hold the padded length, which pad() would write there
+            check(grape_fr_pad(W(row->gpu_data), W(tensor.gpu_data), N, pad_N, new_N, W(grape_host::device_scalar(Fr::zero())), nullptr), "grape_fr_pad");
+        }
     }
     const FrTensor& x = row ? *row : tensor;
 

@@ -136,8 +136,14 @@ hipError_t hipFree(void* p) {
     return hipSuccess;
 }
 hipError_t hipHostMalloc(void** p, size_t bytes, unsigned) { *p = calloc(1, bytes); return *p ? hipSuccess : hipErrorOutOfMemory; }
-hipError_t hipMemcpyAsync(void* dst, const void*, size_t bytes, hipMemcpyKind kind, hipStream_t s) {
+hipError_t hipMemcpyAsync(void* dst, const void* src, size_t bytes, hipMemcpyKind kind, hipStream_t s) {
     Lock l(mu);
+    if (kind == hipMemcpyDeviceToDevice)                     // inside one block at each end
+        for (const void* p : {(const void*)dst, src}) {
+            const char* base;
+            const Alloc* b = block_of(p, &base);
+            if (!b || (const char*)p + bytes > base + b->bytes) return hipErrorInvalidValue;
+        }
     push(s);
     copies++;
     if (kind == hipMemcpyDeviceToHost) memset(dst, 0, bytes);

@@ -458,6 +458,19 @@ static Hyrax_proof trivial_opening(const bn128& G, const Fr& c, uint cols) {
     return proof;
 }
 
+// Openings of rows that are no power of two long: what the folds leave of integers, or a single row, is shorter than the padded row.
+static void padded_openings() {
+    const uint cols = 1100, gens = 2048;
+    bn128 G = bn128::one();
+    Hyrax hyrax(1, gens, device_points(256 * (size_t)gens), G, 1);
+    const int* ints = reinterpret_cast<int*>(device_points(16 * cols));
+    for (uint rows : {1u, 2u, 16u}) {
+        FrTensor x(rows * cols);
+        expect(hyrax.open(ints, random_vec(11 + Log2(rows)), Fr(3), rows * cols, cols).z_size == gens, "of integers");
+        expect(hyrax.open(x, random_vec(11 + Log2(rows)), Fr(3), rows * cols, cols).z_size == gens, "of field elements");
+    }
+}
+
 // a point with more variables than the rows need: the rows that are missing count as the identity
 static void verify_with_more_variables() {
     const uint cols = 64, rows = 4;
@@ -712,6 +725,7 @@ int main(int argc, char** argv) {
         {"operands_at_any_address", operands_at_any_address},
         {"element_products_that_carry", element_products_that_carry},
         {"a_tensor_times_itself", a_tensor_times_itself},
+        {"padded_openings", padded_openings},
         {"verify_with_more_variables", verify_with_more_variables},
         {"single_rows_without_memory", single_rows_without_memory},
         {"a_sum_behind_a_failed_one", a_sum_behind_a_failed_one},

@@ -316,6 +316,26 @@ def test_hyrax_open_and_verify(ops, host, gens):
     assert_same(res, orc.mle_eval(t, pt), "opened value = T(point)")
 
 
+@pytest.mark.parametrize("rows", [1, 2, 16])
+def test_openings_of_padded_rows(ops, host, rows):
+    """rows of 1100 opened as rows of 2048: integers folded directly, embedded ones, against the padded tensor's evaluation"""
+    import torch
+    N, pad_N = 1100, 2048
+    table = ops.g1_table_gen(ops.g1_make_generators(rand_fr(pad_N, 78)), 256)
+    ints = np.random.default_rng(79 + rows).integers(-(1 << 31), 1 << 31, size=(rows, N), dtype=np.int64).astype(np.int32)
+    di = torch.from_numpy(ints.ravel()).cuda()
+    pt, c = rand_fr(11 + br.log2ceil(rows), 80), rand_fr(1, 81)
+    padded = np.zeros((rows, pad_N), dtype=np.int32)
+    padded[:, :N] = ints
+    want = orc.mle_eval(orc.from_i32(padded.ravel()), pt)
+    host.set_input_format("i32")
+    try:
+        assert_same(host.hyrax_open(di, rows * N, N, table, pad_N, pt, c, com_scale=1), want, "integers")
+    finally:
+        host.set_input_format("fr")
+    assert_same(host.hyrax_open(ops.fr_from_i32(di), rows * N, N, table, pad_N, pt, c, com_scale=1), want, "field elements")
+
+
 @pytest.mark.parametrize("rows,N", [(8, 4), (2048, 256)])
 def test_opening_and_evaluation_of_integer_tensors(ops, host, gens, rows, N):
     """Hyrax::open(const int*, ...) and FrTensor::eval_ints (the fold reads the integers) against get_data + open /

@@ -22,7 +22,7 @@ def program():
 
 @pytest.mark.parametrize("scenario", ["refused_lookup", "proof_after_a_refused_one", "mapping_objects", "carried_lookups", "the_longest_indexed_range", "where_padding_is_free", "a_mapping_with_another_r", "lookups_without_a_weighted_term",
                                       "weights_that_are_read", "tensor_memory_is_idle", "sparse_commitment_table",
-                                      "scaled_tables_that_grow", "operands_at_any_address", "element_products_that_carry", "a_tensor_times_itself", "verify_with_more_variables",
+                                      "scaled_tables_that_grow", "operands_at_any_address", "element_products_that_carry", "a_tensor_times_itself", "padded_openings", "verify_with_more_variables",
                                       "single_rows_without_memory", "single_row_table_gives_way", "tables_of_single_rows", "a_sum_behind_a_failed_one", "verify_with_another_generator", "blocks_of_two_devices",
                                       "default_order_blocks", "short_copies"])
 def test_scenario(program, scenario):
