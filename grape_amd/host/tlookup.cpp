@@ -194,6 +194,7 @@ void tLookup::drop_hot_rows() {
     hot_rows_ = hot_cols_ = hot_capacity_ = 0;
     hot_missed_ = 0;
     hot_due_ = 0;
+    hot_counted_ = 0;
     hot_for_ = nullptr;
 }
 
@@ -233,7 +234,8 @@ uint tLookup::hot_choice(uint first, size_t max_new, int* slots, uint32_t* list,
 }
 
 // Rows for entries that keep coming back.  Whether a witness repeats is not known in advance, so an entry without a row pays for
-// its elements proof by proof until what it has paid is what its row costs, and gets the row then, those that have paid most first.
+// its elements proof by proof until what it has paid is what its row costs, in two proofs at least beyond one that has chosen rows by
+// its own witness, and gets the row then, those that have paid most first.
 // A proof's step costs a fifth of a commitment without rows, and a quarter of what the rows at hand save it (what the new ones save at once
 // taken off): no proof takes more than some 1.3 times what it takes without any, for rows that later ones may never
 // use, and what is due together is made in several steps.  Rows end at their share of the tables' budget: entries without one pay on there.
@@ -358,19 +360,20 @@ bool tLookup::commit_A_by_occupancy(uint D, uint msm_size, Hyrax& hyrax) {
     if (hot_slot1_ && (hot_min_count_ != 0 || hot_for_ != &hyrax || hot_cols_ != rowlen || (hot_table_ && !hyrax.owns_scaled_table(hot_table_))))
         drop_hot_rows();
     if (hot_slot1_) {
-        if (!hot_credit_) {                      // rows of a count that the caller has set and taken back
+        if (!hot_credit_) {
             check(grape_malloc((void**)&hot_credit_, sizeof(uint32_t) * (size_t)N), "grape_malloc");
             check(grape_memset_zero(hot_credit_, sizeof(uint32_t) * (size_t)N, nullptr), "grape_memset_zero");
         }
         uint64_t info[3] = {0, 0, 0};
         check(grape_tlookup_hot_credit(d_hist_, N, hot_slot1_, hot_credit_, hot_due(rowlen), info, nullptr), "grape_tlookup_hot_credit");
+        hot_counted_++;
         cold = info[0];
         // Rows kept from earlier proofs are used again, with more of them where entries are due.  They are given up where what they leave out has
         // cost as much as they did - elements of entries that this witness alone earns a row, or of due ones that there was no room for
         // - and others would be better.  What entries have been counted stays, and the new rows are made from it.
         hot_due_ += info[1];
         const double anew = (double)hot_rows_ * rowlen * kRowAdditions;
-        const bool step = hot_due_ >= kDueElements, full = hot_missed_ * kColdAdditions > anew;
+        const bool step = hot_due_ >= kDueElements && hot_counted_ >= 2, full = hot_missed_ * kColdAdditions > anew;
         if (hot_table_ && (full || (!step && (double)info[2] * kColdAdditions > anew))) {
             hot_missed_ = 0;
             if (other_rows_are_better(D, cold)) {
@@ -399,11 +402,6 @@ bool tLookup::commit_A_by_occupancy(uint D, uint msm_size, Hyrax& hyrax) {
             check(grape_tlookup_hot_select(d_hist_, N, min_count, (uint32_t)max_hot, hot_slot1_, d_list, info, nullptr), "grape_tlookup_hot_select");
             const uint n_hot = (uint)info[0];
             cold = info[1];
-            // what this proof's entries cost counts where no proof before it has been counted
-            if (!hot_credit_ && hot_min_count_ == 0) {
-                check(grape_malloc((void**)&hot_credit_, sizeof(uint32_t) * (size_t)N), "grape_malloc");
-                check(grape_memcpy_d2d(hot_credit_, d_hist_, sizeof(uint32_t) * (size_t)N, nullptr), "grape_memcpy_d2d");
-            }
             const bool marked = n_hot != 0 && padding_is_free();
             if (marked) cold -= mark_base(hot_slot1_);
             const bool worth = rows_are_used(hyrax, rowlen, D, cold);
@@ -427,8 +425,14 @@ bool tLookup::commit_A_by_occupancy(uint D, uint msm_size, Hyrax& hyrax) {
         }
         grape_free_on_default(d_list);
         if (!hot_table_) {
-            // nothing has earned a row yet: the slots (none given) and what the entries have paid so far are kept
-            if (hot_min_count_ != 0) drop_hot_rows();
+            // nothing has earned a row yet: the slots (none given) and what the entries have paid so far are kept, in the first proof too
+            if (hot_min_count_ != 0) {
+                drop_hot_rows();
+            } else if (!hot_credit_) {
+                check(grape_malloc((void**)&hot_credit_, sizeof(uint32_t) * (size_t)N), "grape_malloc");
+                check(grape_memcpy_d2d(hot_credit_, d_hist_, sizeof(uint32_t) * (size_t)N, nullptr), "grape_memcpy_d2d");
+                hot_counted_ = 1;
+            }
             return false;
         }
     }

@@ -104,6 +104,7 @@ protected:
     void drop_hot_table();
     bool other_rows_are_better(uint D, uint64_t cold);
     uint32_t* hot_credit_ = nullptr;    // occurrences of entries without a row in the proofs since the rows were made
+    uint hot_counted_ = 0;              // the proofs that have counted them
     uint64_t hot_due_ = 0;              // elements of entries that are due, in the proofs since rows were made last
     double hot_missed_ = 0;             // elements of entries that had earned a row when there was no more room for it
     bool rows_are_used(const Hyrax& hyrax, uint rowlen, uint D, uint64_t cold) const;
