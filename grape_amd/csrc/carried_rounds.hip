@@ -19,7 +19,8 @@
 // wround2_kernel: the gathered first round of 2^26 pairs 2.8 -> 2.1 ms, a round of 2^25 pairs 1.77 -> 1.34 ms, the first
 // round of a 2048 x 11008 element product 0.69 -> 0.61 ms and its second 0.36 -> 0.23 ms.  A thread's next operands are asked
 // for before this pair's arithmetic: two waves a SIMD do not cover the loads (2048 x 11008 proof 1.33 -> 1.29 ms).
-// Proofs run the rounds two to a pass (carried_pair_kernel), an odd one's last alone.
+// Proofs run the rounds two to a pass (carried_pair_kernel), an odd one's last alone; a single first round, gathered or with the weights
+// entering, is there for callers of grape_carried_queue.
 #include "fr_device.hpp"
 
 namespace grape {

@@ -38,9 +38,9 @@ public:
     // Where no table over every entry fits (mapping lookups), A is committed through a table of
     // the entries that occur at least `n` times in the witness (0 = the break-even count, 1.8 times
     // the row length), built by the first proof that needs it and kept: a later proof uses the rows
-    // again unless its elements outside them would cost more than new rows, and entries whose elements have
-    // cost as much as a row over the proofs get theirs.  What the last prove()
-    // did is reported below (hot_rows_reused: it found its rows in place).
+    // again where they leave out few enough of its elements, entries whose elements have cost as much as a row over the proofs get
+    // theirs, and rows are given up for others that would be better.  What the last prove()
+    // did is reported below (no entries where A was committed without rows; hot_rows_reused: it found its rows in place).
     void set_hot_min_count(uint n) { hot_min_count_ = n; }
     uint hot_entries() const { return hot_entries_; }
     uint64_t cold_elements() const { return cold_elements_; }
