@@ -171,12 +171,6 @@ uint64_t tLookup::mark_base(int* slots) {
     return count;
 }
 
-// com(A) through the entries that occur often.  A[i] = B[index_i]; an entry t that occurs n_t times
-// costs n_t full-width scalars (16 to 20 additions each) on the plain path, or one row B[t]*G_i of
-// the scaled table (rowlen entries at 20 additions and a normalisation each) plus n_t single additions.  So an entry is worth a row
-// when n_t exceeds rowlen by a factor somewhat above one; 1.8 is taken (the first proof's time is flat from 1.2 to 2.2).  Elements of the
-// other entries keep their scalars and are committed on the plain path; the two sums are added.
-// Returns false (nothing committed) when no entry qualifies or the table does not fit.
 // the rows alone: the slots are empty, what entries have been counted stays
 void tLookup::drop_hot_table() {
     Hyrax::release_scaled_table(hot_table_);
@@ -350,6 +344,12 @@ bool tLookup::other_rows_are_better(uint D, uint64_t cold) {
     return due * hot_rows_ > 1.25 * held * n;
 }
 
+// com(A) through the entries that occur often.  A[i] = B[index_i]; an entry t that occurs n_t times
+// costs n_t full-width scalars (16 to 20 additions each) on the plain path, or one row B[t]*G_i of
+// the scaled table (rowlen entries at 20 additions and a normalisation each) plus n_t single additions.  So an entry is worth a row
+// when n_t exceeds rowlen by a factor somewhat above one; 1.8 is taken (the first proof's time is flat from 1.2 to 2.2).  Elements of the
+// other entries keep their scalars and are committed on the plain path; the two sums are added.
+// Returns false (nothing committed) when no entry qualifies, the table does not fit or rows are not worth using.
 bool tLookup::commit_A_by_occupancy(uint D, uint msm_size, Hyrax& hyrax) {
     const uint N = T.size;
     const uint rowlen = msm_size * hyrax.com_scale;
