@@ -12,13 +12,17 @@ namespace grape {
 
 // ---------------------------------------------------------------- eq pyramid
 // Level j (2^j entries) sits at element offset 2^j - 1; level j holds eq(u[0..j-1], i), bit b of i paired with u[b].
-// Level by level (hi = lo * u[j], lo' = lo - hi) a pyramid is a chain of launches, one for each level above 9, before a proof's
-// first round.  Here every level is made at once, in one launch: a workgroup takes a head of 2^11 entries of a level that share their
+// Level by level (hi = lo * u[j], lo' = lo - hi) a pyramid is a chain of products, and above level 9 of launches, before a proof's
+// first round.  Here levels up to kPyrTop are made at once, in one launch: a workgroup takes a head of 2^11 entries of a level that share their
 // high bits, an entry is the product of a factor over bits 0..4, one over bits 5..10 and the head's own, and those are
 // products of at most 6 (3 deep; 19 for the head, a tree over the lanes) factors u or 1 - u, made by different waves side by
 // side.  One product an entry as before.  Bound by its chain of about 14 products below 2^16 entries, by issue above: 2^13 entries
-// 26 -> 13 us and 5 -> 1 launches, 2^16 40 -> 13.5 and 8 -> 1, 2^20 73 -> 42 and 12 -> 1.
-constexpr uint32_t kPyrLow = 5, kPyrHead = 11;
+// 26 -> 13 us and 5 -> 1 launches, 2^16 40 -> 13.5 and 8 -> 1.
+// Up to kPyrShort variables an entry is its own product, three deep, and nothing meets anywhere: 3.8 to 6.2 us for 0 to 6 variables
+// against 6.8 to 8.8 (7 variables 8.6 against 8.5 level by level).  Levels above kPyrTop are a launch each that reads the one
+// below, half a product an entry: 21 variables 54 against 66 us, 22 90 against 124; one such level alone is not worth its launch
+// (20 variables 38 against 41).
+constexpr uint32_t kPyrLow = 5, kPyrHead = 11, kPyrShort = 6, kPyrTop = 19;
 
 // the factor of u[b] for bit `set`; one for a variable that is not there
 __device__ __forceinline__ Fr eq_factor(const uint32_t* u, uint32_t b, bool there, bool set) {
@@ -34,7 +38,28 @@ __device__ __forceinline__ Fr eq_factors(const uint32_t* u, uint32_t b, uint32_t
         x[k] = fr26::mulc(eq_factor(u, b + 2 * k, 2 * k < n, (i >> 2 * k) & 1), eq_factor(u, b + 2 * k + 1, 2 * k + 1 < n, (i >> (2 * k + 1)) & 1));
     return fr26::mulc(fr26::mulc(x[0], x[1]), x[2]);
 }
-__global__ void __launch_bounds__(kBlock) eq_pyramid_head_kernel(uint32_t* pyr, const uint32_t* u) {
+template <bool SHORT>
+__global__ void __launch_bounds__(kBlock) eq_pyramid_head_kernel(uint32_t* pyr, const uint32_t* u, uint32_t nu) {
+    if constexpr (SHORT) {
+        // a thread an entry: entry i of a level is thread 2^level + i - 1
+        const uint32_t at = threadIdx.x + 1, level = 31 - __clz(at), i = at - (1u << level);
+        Fr f[kPyrShort];
+#pragma unroll
+        for (uint32_t j = 0; j < kPyrShort; j++)
+            if (j < nu) f[j] = ld_fr(u, j);
+        if (level > nu) return;
+#pragma unroll
+        for (uint32_t j = 0; j < kPyrShort; j++)
+            if (j < nu) f[j] = j >= level ? Fr::one() : (i >> j) & 1 ? f[j] : sub(Fr::one(), f[j]);
+        Fr x = nu > 1 ? fr26::mulc(f[0], f[1]) : nu ? f[0] : Fr::one();
+        if (nu > 2) {
+            Fr y = nu > 3 ? fr26::mulc(f[2], f[3]) : f[2];
+            if (nu > 4) y = fr26::mulc(y, nu > 5 ? fr26::mulc(f[4], f[5]) : f[4]);
+            x = fr26::mulc(x, y);
+        }
+        st_fr(pyr, threadIdx.x, x);
+        return;
+    }
     __shared__ Fr low[1 << kPyrLow], mid[1 << (kPyrHead - kPyrLow)], high;
     // workgroups 0..kPyrHead are the levels up to kPyrHead, 2^(level - kPyrHead) of them each level above
     uint32_t level = blockIdx.x, h = 0;
@@ -67,6 +92,14 @@ __global__ void __launch_bounds__(kBlock) eq_pyramid_head_kernel(uint32_t* pyr, 
         const Fr l = low[i & ((1u << nlow) - 1)];
         st_fr(pyr, at + i, level > kPyrLow ? fr26::mulc(l, mid[i >> nlow]) : l);
     }
+}
+
+__global__ void __launch_bounds__(kBlock) eq_pyramid_level_kernel(uint32_t* pyr, const uint32_t* u, uint32_t j) {
+    const size_t half = (size_t)1 << j, i = (size_t)blockIdx.x * kBlock + threadIdx.x;
+    if (i >= half) return;
+    const Fr lo = ld_fr(pyr, half - 1 + i), hi = fr26::mulc(lo, ld_fr(u, j));
+    st_fr(pyr, 2 * half - 1 + half + i, hi);
+    st_fr(pyr, 2 * half - 1 + i, sub(lo, hi));
 }
 
 // ---------------------------------------------------------------- weighted two-tensor round
@@ -363,8 +396,11 @@ int grape_eq_pyramid(uint32_t* pyr, const uint32_t* u, uint32_t nu, grape_stream
     GRAPE_REQUIRE(nu <= 30, "too many variables");
     if (nu) CHECK_PTR16(u);
     hipStream_t s = as_stream(st);
-    const unsigned nb = nu <= kPyrHead ? nu + 1 : kPyrHead - 1 + (1u << (nu - kPyrHead + 1));
-    eq_pyramid_head_kernel<<<nb, kBlock, 0, s>>>(pyr, u);
+    const uint32_t top = nu <= kPyrTop + 1 ? nu : kPyrTop;
+    const unsigned nb = top <= kPyrHead ? top + 1 : kPyrHead - 1 + (1u << (top - kPyrHead + 1));
+    if (nu <= kPyrShort) eq_pyramid_head_kernel<true><<<1, 2 << kPyrShort, 0, s>>>(pyr, u, nu);
+    else eq_pyramid_head_kernel<false><<<nb, kBlock, 0, s>>>(pyr, u, top);
+    for (uint32_t j = top; j < nu; j++) eq_pyramid_level_kernel<<<blocks_for((size_t)1 << j), kBlock, 0, s>>>(pyr, u, j);
     GRAPE_LAUNCH_CHECK();
     return GRAPE_OK;
 }

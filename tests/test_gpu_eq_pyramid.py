@@ -1,5 +1,5 @@
 """Every entry of the eq tables of all prefixes, at the sizes where an entry's factors change their place (5 low bits, 11 bits a
-workgroup, workgroups of several levels), and the challenge tables' rows: both against their definitions."""
+workgroup, workgroups of several levels), an entry a thread below those and level by level above them, and the challenge tables' rows: both against their definitions."""
 import numpy as np
 import pytest
 import bigref as br
@@ -16,7 +16,7 @@ def ops():
     return ops
 
 
-@pytest.mark.parametrize("nu", [0, 1, 4, 5, 6, 10, 11, 12, 13, 14, 18])
+@pytest.mark.parametrize("nu", [0, 1, 2, 3, 4, 5, 6, 7, 10, 11, 12, 13, 14, 18, 19, 20, 21])
 def test_every_level(ops, nu):
     u = rand_fr(max(nu, 1), 300 + nu)[:nu]
     if nu > 3:
