@@ -261,6 +261,10 @@ __global__ void __launch_bounds__(kHistThreads) hist_ranges_kernel(unsigned long
     if (threadIdx.x == 0) mask[blockIdx.x] = any;
 }
 
+// Lanes of a wave that share a bin are counted once, by a leader; two leaders first, and two more where those have counted this many
+// of the 64, plain adds for the rest.  2^22 entries on one value 39 us, on two 52, three 58, four and more 52, half of them one value 46;
+// four leaders in every case 40, 51, 61, 71 and 56.  Asking for 26: four values 69, five 64.
+constexpr uint32_t kHistShared = 44;
 template <int BINS>
 __global__ void __launch_bounds__(kHistThreads) hist_lds_kernel(uint32_t* __restrict__ partial, const int32_t* __restrict__ idx1,
                                                                 size_t n, size_t per_chunk, uint32_t len,
@@ -289,20 +293,25 @@ __global__ void __launch_bounds__(kHistThreads) hist_lds_kernel(uint32_t* __rest
         for (int q = 0; q < 4; q++) {
             const uint32_t b = (uint32_t)(vv[q] - 1) - base;      // 0 (out of range) wraps far away
             const bool in = b < (uint32_t)BINS;
-            // lanes that share a bin are counted once: up to four leaders, then plain adds.  Two leaders that share theirs with
-            // fewer than three others each tell that the values are spread out, where plain adds are cheaper (2^27 scores on some
-            // 900 entries: 1.08 -> 0.77 ms with the passes around it; half of them one entry: 1.08 -> 0.95).
             unsigned long long todo = __ballot(in);
-            uint32_t shared = 0;
-            for (int it = 0; it < 4 && todo != 0ull; it++) {
+            auto count_leader = [&] {
                 const int leader = __ffsll((long long)todo) - 1;
                 const uint32_t lb = (uint32_t)__builtin_amdgcn_readlane((int)b, leader);
                 const unsigned long long same = __ballot(in && b == lb) & todo;
                 const uint32_t count = (uint32_t)__popcll(same);
                 if (lane == leader) atomicAdd(&bins[lb], count);
                 todo &= ~same;
-                shared += count;
-                if (it == 1 && shared < 8) break;
+                return count;
+            };
+            if (todo != 0ull) {
+                uint32_t counted = count_leader();
+                if (todo != 0ull) {
+                    counted += count_leader();
+                    if (todo != 0ull && counted >= kHistShared) {
+                        count_leader();
+                        if (todo != 0ull) count_leader();
+                    }
+                }
             }
             if (in && ((todo >> lane) & 1ull)) atomicAdd(&bins[b], 1u);
         }

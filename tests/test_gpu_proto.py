@@ -130,6 +130,22 @@ def test_histogram(ops):
     assert h3.sum() == 1 and h3[3] == 1
 
 
+@pytest.mark.parametrize("values", [1, 2, 3, 4, 5, 9, 30, 4000])
+def test_counts_of_few_values(ops, values):
+    """lanes of a wave that share a bin: every one, two, three leaders' worth, some left over after them, none; elements outside the
+    table between them"""
+    import torch
+    rng = np.random.default_rng(40 + values)
+    length = 4096
+    idx = rng.integers(50, 50 + values, (1 << 20) + 4099).astype(np.int32)
+    idx[rng.random(idx.shape[0]) < 0.1] = 50                    # uneven shares
+    idx[::61] = 0
+    idx[::67] = length + 1
+    h = ops.tlookup_hist_index(torch.from_numpy(idx).cuda(), length).cpu().numpy()
+    inside = (idx >= 1) & (idx <= length)
+    assert np.array_equal(h, np.bincount(idx[inside] - 1, minlength=length))
+
+
 def test_histogram_long_witness(ops):
     """witnesses of 2^20 values and more take the LDS-counting path: ragged length, a table that
     is not a multiple of the bins held in LDS, a clipped (heavily repeated) value, values outside
