@@ -228,8 +228,8 @@ uint tLookup::hot_choice(uint first, size_t max_new, int* slots, uint32_t* list,
 }
 
 // Rows for entries that keep coming back.  Whether a witness repeats is not known in advance, so an entry without a row pays for
-// its elements proof by proof until what it has paid is what its row costs, in two proofs at least beyond one that has chosen rows by
-// its own witness, and gets the row then, those that have paid most first.
+// its elements proof by proof until what it has paid is what its row costs, and gets the row then, those that have paid most first -
+// in the second proof at the earliest, or the second behind the one that has chosen rows by its own witness.
 // A proof's step costs a fifth of a commitment without rows, and a quarter of what the rows at hand save it (what the new ones save at once
 // taken off): no proof takes more than some 1.3 times what it takes without any, for rows that later ones may never
 // use, and what is due together is made in several steps.  Rows end at their share of the tables' budget: entries without one pay on there.
@@ -424,15 +424,15 @@ bool tLookup::commit_A_by_occupancy(uint D, uint msm_size, Hyrax& hyrax) {
             throw;
         }
         grape_free_on_default(d_list);
+        // the first proof's entries have paid too
+        if (hot_min_count_ == 0 && !hot_credit_) {
+            check(grape_malloc((void**)&hot_credit_, sizeof(uint32_t) * (size_t)N), "grape_malloc");
+            check(grape_memcpy_d2d(hot_credit_, d_hist_, sizeof(uint32_t) * (size_t)N, nullptr), "grape_memcpy_d2d");
+            hot_counted_ = hot_table_ ? 0 : 1;               // one that has chosen rows has judged its other entries
+        }
         if (!hot_table_) {
-            // nothing has earned a row yet: the slots (none given) and what the entries have paid so far are kept, in the first proof too
-            if (hot_min_count_ != 0) {
-                drop_hot_rows();
-            } else if (!hot_credit_) {
-                check(grape_malloc((void**)&hot_credit_, sizeof(uint32_t) * (size_t)N), "grape_malloc");
-                check(grape_memcpy_d2d(hot_credit_, d_hist_, sizeof(uint32_t) * (size_t)N, nullptr), "grape_memcpy_d2d");
-                hot_counted_ = 1;
-            }
+            // nothing has earned a row yet: the slots (none given) and what the entries have paid so far are kept
+            if (hot_min_count_ != 0) drop_hot_rows();
             return false;
         }
     }
